@@ -8,6 +8,7 @@ import threading
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmlstm_hip.so")
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 F32, BF16 = 0, 1
 F16 = 2
@@ -73,6 +74,21 @@ def get_lib() -> ctypes.CDLL:
                 )
             _lib = lib
     return _lib
+
+
+def get_host():
+    """The extension module with the native host path of the operators; raise RuntimeError if it was not built."""
+    global _host
+    if _host is None:
+        get_lib()  # torch and libmlstm_hip.so come first: the extension binds to both
+        try:
+            from . import _torch_host
+        except ImportError as e:
+            raise RuntimeError(
+                f"mlstm_kernels_amd._torch_host cannot be loaded ({e}). Build it with `python -m mlstm_kernels_amd.build`."
+            ) from e
+        _host = _torch_host
+    return _host
 
 
 _PATH_CODES = {"auto": PATH_AUTO, "split": PATH_SPLIT, "fused": PATH_FUSED, "stream": PATH_STREAM}

@@ -570,8 +570,8 @@ static const char* launch_fused_hv_t(const FusedHvArgs& a, int BH, hipStream_t s
   const size_t smem = (size_t)(128 * DQ + 3 * 128 * 64 + 2 * ND * 512) * 2 + (size_t)((2 + 4 * NWQ) * DQ + 768 + 4) * 4;
   if ((size_t)a.S * (size_t)(a.DHHV > DQ ? a.DHHV : DQ) * 2 >= ((size_t)1 << 32))
     return "fused_hv: one (batch, head) slab of an input exceeds 4 GiB";
-  if (hipFuncSetAttribute((const void*)fused_hv_kernel<DQ, IS_DV, HILO, NWQ>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)fused_hv_kernel<DQ, IS_DV, HILO, NWQ>, smem))
     return "fused_hv: cannot raise the dynamic LDS limit";
   dim3 grid(a.DHHV / 64, BH);
   hipLaunchKernelGGL((fused_hv_kernel<DQ, IS_DV, HILO, NWQ>), grid, dim3(256 * NWQ), smem, stream, a);

@@ -5,9 +5,43 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "layout.h"
 
 namespace mlstm {
+
+// Properties of a device that every launch needs and that cost the host about as much as a launch to ask the runtime
+// for: kept per device after the first question.
+constexpr int kMaxHostDevices = 64;
+inline int current_device() {
+  int dev = -1;
+  return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxHostDevices ? dev : -1;
+}
+inline int device_cu_count() {
+  static std::atomic<int> cached[kMaxHostDevices];
+  const int dev = current_device();
+  if (dev < 0) return 0;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+// The dynamic LDS limit of one kernel (one object per kernel instantiation): raised when a launch needs more than any
+// launch on that device before it.
+struct LdsLimit {
+  std::atomic<int> bytes[kMaxHostDevices];
+  bool allow(const void* kernel, size_t need) {
+    const int dev = current_device();
+    if (dev < 0) return false;
+    if (bytes[dev].load(std::memory_order_relaxed) >= (int)need) return true;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need) != hipSuccess) return false;
+    bytes[dev].store((int)need, std::memory_order_relaxed);
+    return true;
+  }
+};
 
 struct ScanArgs {
   const uint16_t* X;      // (B,NH,S,DHQK) bf16/fp16: K (forward) or Q (backward)

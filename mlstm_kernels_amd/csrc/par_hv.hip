@@ -644,8 +644,8 @@ static const char* launch_par_hv_hn(const ParHvArgs& a, int BH, hipStream_t stre
   if (smem > 160 * 1024) return "par_hv: DHQK too large for the LDS-resident tile";
   if ((size_t)a.S * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32))
     return "par_hv: one (batch, head) slab of an input exceeds 4 GiB";
-  if (hipFuncSetAttribute((const void*)par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>, smem))
     return "par_hv: cannot raise the dynamic LDS limit";
   dim3 grid(2, a.NC, BH);
   hipLaunchKernelGGL((par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>), grid, dim3(64 * (WT / MW)), smem, stream, a);

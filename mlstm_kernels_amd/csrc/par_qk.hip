@@ -508,8 +508,8 @@ static const char* launch_par_qk_pair_f(const ParQkArgs& a, int BH, hipStream_t 
   constexpr int sab = sa > sb ? sa : sb;
   constexpr int stage = sab > sc ? sab : sc;
   const size_t smem = (size_t)(stage + 64 * 136) * 2 + (size_t)(64 * 2 + 128 * 2 + 64 + (MT / 64) * 64) * 4;
-  if (hipFuncSetAttribute((const void*)par_qk_pair_kernel<MT, F16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)par_qk_pair_kernel<MT, F16>, smem))
     return "par_qk: cannot raise the dynamic LDS limit";
   dim3 grid(4 * (a.DHQK / MT), a.NC, BH);
   hipLaunchKernelGGL((par_qk_pair_kernel<MT, F16>), grid, dim3(MT), smem, stream, a);

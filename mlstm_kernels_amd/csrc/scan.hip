@@ -383,8 +383,8 @@ static const char* launch_scan_f(const ScanArgs& a, int BH, hipStream_t stream) 
   constexpr int PS = 128;
   const size_t smem = (size_t)PS * (RT + 32) * 2 + (size_t)PS * (WT + 32) * 2 * (HILO ? 2 : 1) +
                       (size_t)(XROWS * RT + kGBlock + 2 * kChunk) * 4;
-  if (hipFuncSetAttribute((const void*)scan_kernel<RT, WT, HILO, PS, WCOLS, F16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)scan_kernel<RT, WT, HILO, PS, WCOLS, F16>, smem))
     return "scan: cannot raise the dynamic LDS limit";
   dim3 grid(a.DHQK / RT, a.DHHV / WT, BH);
   hipLaunchKernelGGL((scan_kernel<RT, WT, HILO, PS, WCOLS, F16>), grid, dim3(NT), smem, stream, a);
@@ -799,8 +799,8 @@ template <int RT, int WT, bool F16>
 static const char* launch_scan_roles_f(const ScanArgs& a, int BH, hipStream_t stream) {
   constexpr int NW = (RT / 64) * (WT / 32);
   const size_t smem = (size_t)2 * kChunk * (RT + WT) * 2 + (size_t)(kGBlock + 2 * kChunk) * 4 + (size_t)3 * kChunk * 3 * 2;
-  if (hipFuncSetAttribute((const void*)scan_roles_kernel<RT, WT, F16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16>, smem))
     return "scan: cannot raise the dynamic LDS limit";
   dim3 grid(a.DHQK / RT, a.DHHV / WT, BH);
   hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16>), grid, dim3(128 * NW), smem, stream, a);

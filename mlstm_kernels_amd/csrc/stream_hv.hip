@@ -593,18 +593,6 @@ bool stream_hv_supported(const ParHvArgs& a) {
 }
 
 namespace {
-int device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <bool IS_DV, bool F16, bool NORM = false>
 const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
   constexpr int QS = 256 + 8, PSS = 72, SLOT = 64 * QS;
@@ -618,8 +606,8 @@ const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
   int G = (int)(n_items < cus ? n_items : cus);
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
-  if (hipFuncSetAttribute((const void*)stream_hv_kernel<IS_DV, F16, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)stream_hv_kernel<IS_DV, F16, NORM>, smem))
     return "stream_hv: cannot raise the dynamic LDS limit";
   hipLaunchKernelGGL((stream_hv_kernel<IS_DV, F16, NORM>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
   return nullptr;

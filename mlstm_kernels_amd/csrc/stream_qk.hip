@@ -441,18 +441,6 @@ __global__ __launch_bounds__(768) void stream_qk_kernel(ParQkArgs a, int n_items
 bool stream_qk_supported(const ParQkArgs& a) { return a.DHQK == 256 && a.DHHV % 128 == 0 && a.S % kChunk == 0; }
 
 namespace {
-int qk_device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <bool F16>
 const char* launch_stream_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   constexpr int ZS = 256 + 32, PS = 128 + 8, SLOT = 64 * ZS;
@@ -461,12 +449,13 @@ const char* launch_stream_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   if (n_items >= (1ll << 31)) return "stream_qk: too many work items";
   if ((size_t)a.S * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32))
     return "stream_qk: one (batch, head) slab of an input exceeds 4 GiB";
-  const int cus = qk_device_cu_count();
+  const int cus = device_cu_count();
   if (cus <= 0) return "stream_qk: cannot read the number of compute units";
   int G = (int)(n_items < cus ? n_items : cus);
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
-  if (hipFuncSetAttribute((const void*)stream_qk_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)stream_qk_kernel<F16>, smem))
     return "stream_qk: cannot raise the dynamic LDS limit";
   hipLaunchKernelGGL((stream_qk_kernel<F16>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
   return nullptr;

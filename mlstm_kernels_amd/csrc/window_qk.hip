@@ -528,30 +528,19 @@ bool window_qk_supported(const ParQkArgs& a) {
 }
 
 namespace {
-int wq_device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <bool F16>
 const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   const long long n_items = (long long)BH * (a.NC / 2);
   if (n_items >= (1ll << 31)) return "window_qk: too many work items";
   if ((size_t)a.S * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32))
     return "window_qk: one (batch, head) slab of an input exceeds 4 GiB";
-  const int cus = wq_device_cu_count();
+  const int cus = device_cu_count();
   if (cus <= 0) return "window_qk: cannot read the number of compute units";
   int G = (int)(n_items < cus ? n_items : cus);
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
-  if (hipFuncSetAttribute((const void*)window_qk_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, kWqSmem) != hipSuccess)
+  static LdsLimit lds;
+  if (!lds.allow((const void*)window_qk_kernel<F16>, kWqSmem))
     return "window_qk: cannot raise the dynamic LDS limit";
   hipLaunchKernelGGL((window_qk_kernel<F16>), dim3(G), dim3(768), kWqSmem, stream, a, (int)n_items, n_rounds);
   return nullptr;

@@ -22,10 +22,9 @@ from __future__ import annotations
 import warnings
 
 import torch
-from torch.amp import custom_bwd, custom_fwd
 
 from ... import _lib
-from ..utils import current_stream_ptr, dtype_code, ptr, require_gpu
+from ..utils import require_gpu
 
 _IGNORED_TUNING_KWARGS = (
     "siz_b_L_parallel", "siz_b_L_loop", "siz_b_DH_parallel", "siz_b_DH_loop", "num_warps_intra", "num_warps_inter",
@@ -109,46 +108,8 @@ def _fw_launch(q, k, v, i, f, c0, n0, m0, eps, siging, normalize, want_last, kee
     """One forward launch.  n_out / m_out: optional fp32 (B,NH,S) tensors that receive the row normaliser
     max(|den|, floor) and the combined stabiliser (vecN_out / vecM_out of the reference's mlstm_chunkwise_fw,
     mlstm_kernels/torch/chunkwise/triton_xl_chunk/fw.py:150-170)."""
-    B, NH, S, DHQK = q.shape
-    DHHV = v.shape[-1]
-    dev = q.device
-    lib = _lib.get_lib()
-    if path == _lib.PATH_FUSED and q.dtype != torch.bfloat16:
-        raise RuntimeError(f"the fused kernel path supports bfloat16 operands only, got {q.dtype}")
-    ws_bytes = lib.mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DHQK, DHHV, int(keep), path, stride)
-    if ws_bytes == 0:
-        if DHQK % 64 == 0 and DHQK > 896:
-            raise RuntimeError(f"DHQK too large for the HIP chunkwise kernels: {DHQK} (at most 896)")
-        if path == _lib.PATH_FUSED and DHQK not in (128, 256) and DHQK % 64 == 0 and DHHV % 64 == 0:
-            raise RuntimeError(f"the fused kernel path supports DHQK = 128 or 256 only, got {DHQK}")
-        raise ValueError(
-            f"unsupported shape for the HIP chunkwise kernels: B={B}, NH={NH}, S={S}, DHQK={DHQK}, DHHV={DHHV} "
-            "(head dimensions must be multiples of 64, DHQK <= 896, B*NH <= 65535)"
-        )
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    H = torch.empty(B, NH, S, DHHV, dtype=q.dtype, device=dev)
-    if norm != _lib.NORM_NONE:
-        if DHHV not in (64, 128, 256, 512):
-            raise ValueError(f"the fused head norm needs DHHV = 64, 128, 256 or 512, got {DHHV}")
-        norm_mean = torch.empty(B, NH, S, dtype=torch.float32, device=dev)
-        norm_rstd = torch.empty(B, NH, S, dtype=torch.float32, device=dev)
-    else:
-        norm_mean = norm_rstd = None
-    if want_last:
-        c_last = torch.empty(B, NH, DHQK, DHHV, dtype=torch.float32, device=dev)
-        n_last = torch.empty(B, NH, DHQK, dtype=torch.float32, device=dev)
-        m_last = torch.empty(B, NH, 1, dtype=torch.float32, device=dev)
-    else:
-        c_last = n_last = m_last = None
-    rc = lib.mlstm_hip_chunkwise_fw(
-        ptr(q), ptr(k), ptr(v), ptr(i), ptr(f), ptr(c0), ptr(n0), ptr(m0),
-        ptr(H), ptr(n_out), ptr(m_out), ptr(c_last), ptr(n_last), ptr(m_last),
-        ptr(ws), ws_bytes, int(keep), B, NH, S, DHQK, DHHV, float(eps),
-        dtype_code(q), dtype_code(i), _lib.GATE_SIG if siging else _lib.GATE_EXP, int(normalize), path, stride,
-        norm, float(norm_eps), ptr(norm_mean), ptr(norm_rstd), current_stream_ptr(dev),
-    )
-    _lib.check(rc, "mlstm_hip_chunkwise_fw")
-    return H, c_last, n_last, m_last, ws, norm_rstd
+    return _lib.get_host().forward(q, k, v, i, f, c0, n0, m0, float(eps), siging, normalize, want_last, keep, path, stride,
+                                   norm, float(norm_eps), n_out, m_out)
 
 
 def _prep_inputs(q, k, v, i, f, c0, n0, m0, siging, f32_as_f16=False):
@@ -178,100 +139,50 @@ def _prep_inputs(q, k, v, i, f, c0, n0, m0, siging, f32_as_f16=False):
     return dev, qb, kb, vb, ib, fb, c0, n0, m0
 
 
-def _make_fwbw(autocast_kernel_dtype, siging: bool, normalize: bool, path: int, stride: int, norm: int, norm_eps: float,
-               recompute: bool, f32_as_f16: bool = False):
-    class _HipChunkwiseFwBw(torch.autograd.Function):
-        @staticmethod
-        @custom_fwd(device_type="cuda", cast_inputs=autocast_kernel_dtype)
-        def forward(ctx, q, k, v, i, f, c0, n0, m0, return_last_states, eps):
-            # outputs nobody differentiates (the last states in most losses) arrive as None in backward instead of as
-            # freshly allocated zero tensors the size of the state
-            ctx.set_materialize_grads(False)
-            out_dtype = q.dtype
-            dev, qb, kb, vb, ib, fb, c0f, n0f, m0f = _prep_inputs(q, k, v, i, f, c0, n0, m0, siging, f32_as_f16)
-            needs_bw = any(ctx.needs_input_grad[:6])
-            H, c_last, n_last, m_last, ws, norm_rstd = _fw_launch(
-                qb, kb, vb, ib, fb, c0f, n0f, m0f, eps, siging, normalize, return_last_states, needs_bw, path, stride,
-                norm, norm_eps
-            )
-            c0s = None
-            if recompute and needs_bw:
-                # keep only what lies in front of the chunk states (gate vectors, normaliser states, row normalisers);
-                # the backward runs the state scan again, from the initial state when there is one
-                B_, NH_, S_, DHQK_ = qb.shape
-                saved_bytes = _lib.get_lib().mlstm_hip_chunkwise_fw_saved_bytes(B_, NH_, S_, DHQK_, vb.shape[-1])
-                if ws.numel() > saved_bytes:
-                    ws = ws[:saved_bytes].clone()
-                c0s = c0f
-            if norm != _lib.NORM_NONE and needs_bw:
-                ctx.save_for_backward(qb, kb, vb, ib, fb, ws, c0s, H, norm_rstd)   # H holds the normalised rows
+class _Operator:
+    """The chunkwise operator with its options fixed: forward, and backward through a native autograd node."""
+
+    def __init__(self, autocast_kernel_dtype, siging: bool, normalize: bool, path: int, stride: int, norm: int, norm_eps: float,
+                 recompute: bool, f32_as_f16: bool):
+        self._autocast_code = _DTYPE_CODES[autocast_kernel_dtype]
+        self._options = (siging, normalize, path, stride, norm, norm_eps, recompute, f32_as_f16)
+        # float32 operands are rounded to bfloat16 in the kernels: those of the call or, under autocast, those it makes
+        self._warn = not f32_as_f16
+        self._autocast_to_float32 = autocast_kernel_dtype == torch.float32
+
+    def apply(self, q, k, v, i, f, c0, n0, m0, return_last_states, eps):
+        if self._warn and torch.float32 not in _warned_rounding:
+            if torch.is_autocast_enabled("cuda"):
+                rounds = self._autocast_to_float32
             else:
-                ctx.save_for_backward(qb, kb, vb, ib, fb, ws, c0s)
-            ctx.cfg = (eps, q.dtype, k.dtype, v.dtype, i.dtype, f.dtype,
-                       None if c0 is None else c0.dtype, n0 is not None, m0 is not None)
-            H = H if out_dtype == H.dtype else H.to(out_dtype)
-            return H, c_last, n_last, m_last
-
-        @staticmethod
-        @custom_bwd(device_type="cuda")
-        def backward(ctx, dH, dC_last, dn_last, dm_last):
-            qb, kb, vb, ib, fb, ws, c0s, *normed = ctx.saved_tensors
-            eps, qdt, kdt, vdt, idt, fdt, c0dt, has_n0, has_m0 = ctx.cfg
-            B, NH, S, DHQK = qb.shape
-            DHHV = vb.shape[-1]
-            dev = qb.device
-            lib = _lib.get_lib()
-            bw_bytes = lib.mlstm_hip_chunkwise_bw_workspace_bytes(B, NH, S, DHQK, DHHV, stride)
-            bws = torch.empty(bw_bytes, dtype=torch.uint8, device=dev)
-            if recompute:
-                full_bytes = lib.mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DHQK, DHHV, 1, path, stride)
-                full = torch.empty(full_bytes, dtype=torch.uint8, device=dev)
-                full[:ws.numel()].copy_(ws)
-                rc = lib.mlstm_hip_chunkwise_recompute_states(
-                    ptr(kb), ptr(vb), ptr(c0s), ptr(full), full_bytes, B, NH, S, DHQK, DHHV, dtype_code(qb), stride,
-                    current_stream_ptr(dev),
-                )
-                _lib.check(rc, "mlstm_hip_chunkwise_recompute_states")
-                ws = full
-            if dH is None:  # only the last states are differentiated
-                dH = torch.zeros(B, NH, S, DHHV, dtype=qb.dtype, device=dev)
-            dHb = dH.to(qb.dtype).contiguous()
-            if normed:
-                # gradient of the normalised rows -> gradient of H (the un-normalised rows were never stored)
-                Hn, rstd = normed
-                dHraw = torch.empty_like(dHb)
-                rc = lib.mlstm_hip_head_norm_bw(ptr(dHb), ptr(Hn), ptr(rstd), ptr(dHraw), B * NH * S, DHHV, norm,
-                                                dtype_code(dHb), current_stream_ptr(dev))
-                _lib.check(rc, "mlstm_hip_head_norm_bw")
-                dHb = dHraw
-            dCl = None if dC_last is None else dC_last.to(torch.float32).contiguous()
-            dQ, dK, dV = torch.empty_like(qb), torch.empty_like(kb), torch.empty_like(vb)
-            dI = torch.empty(B, NH, S, dtype=torch.float32, device=dev)
-            dF = torch.empty(B, NH, S, dtype=torch.float32, device=dev)
-            dC0 = torch.empty(B, NH, DHQK, DHHV, dtype=torch.float32, device=dev) if c0dt is not None else None
-            rc = lib.mlstm_hip_chunkwise_bw(
-                ptr(qb), ptr(kb), ptr(vb), ptr(ib), ptr(fb), ptr(dHb), ptr(dCl),
-                ptr(dQ), ptr(dK), ptr(dV), ptr(dI), ptr(dF), ptr(dC0),
-                ptr(ws), ws.numel(), ptr(bws), bw_bytes, B, NH, S, DHQK, DHHV, float(eps),
-                dtype_code(qb), dtype_code(ib), _lib.GATE_SIG if siging else _lib.GATE_EXP, int(normalize), path, stride,
-                current_stream_ptr(dev),
-            )
-            _lib.check(rc, "mlstm_hip_chunkwise_bw")
-            dn0 = torch.zeros(B, NH, DHQK, dtype=torch.float32, device=dev) if has_n0 else None
-            dm0 = torch.zeros(B, NH, 1, dtype=torch.float32, device=dev) if has_m0 else None
-            return (dQ.to(qdt), dK.to(kdt), dV.to(vdt), dI.to(idt), dF.to(fdt),
-                    None if dC0 is None else dC0.to(c0dt), dn0, dm0, None, None)
-
-    return _HipChunkwiseFwBw
+                rounds = q.dtype == torch.float32 or k.dtype == torch.float32 or v.dtype == torch.float32
+            if rounds and q.is_cuda:
+                _warn_rounding_once(torch.float32)
+        return (_host or _get_host()).chunkwise(q, k, v, i, f, c0, n0, m0, return_last_states, eps, self._autocast_code,
+                                                *self._options)
 
 
+_host = None
+
+
+def _get_host():
+    global _host
+    _host = _lib.get_host()
+    return _host
+
+
+_DTYPE_CODES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 _FWBW_CACHE: dict = {}
 
 
 def _get_fwbw(autocast_kernel_dtype: torch.dtype, siging: bool, normalize: bool, kernel_path: str, stride: int,
               head_norm: str = "none", head_norm_eps: float = 1e-6, recompute: bool = False,
               float32_operands: str = "bfloat16"):
-    if autocast_kernel_dtype not in (torch.float32, torch.float16, torch.bfloat16):
+    key = (autocast_kernel_dtype, siging, normalize, kernel_path, stride, head_norm, head_norm_eps, recompute, float32_operands)
+    op = _FWBW_CACHE.get(key)
+    if op is not None:
+        return op
+    if autocast_kernel_dtype not in _DTYPE_CODES:
         raise ValueError(f"Unsupported kernel dtype {autocast_kernel_dtype}.")
     path = _lib.path_code(kernel_path)
     norm = _lib.norm_code(head_norm)
@@ -282,11 +193,9 @@ def _get_fwbw(autocast_kernel_dtype: torch.dtype, siging: bool, normalize: bool,
     f32_as_f16 = float32_operands == "float16"
     if f32_as_f16 and path == _lib.PATH_FUSED:
         raise ValueError("the fused kernel path multiplies bfloat16 operands only")
-    key = (autocast_kernel_dtype, siging, normalize, path, stride, norm, float(head_norm_eps), bool(recompute), f32_as_f16)
-    if key not in _FWBW_CACHE:
-        _FWBW_CACHE[key] = _make_fwbw(autocast_kernel_dtype, siging, normalize, path, stride, norm, float(head_norm_eps),
-                                      bool(recompute), f32_as_f16)
-    return _FWBW_CACHE[key]
+    op = _Operator(autocast_kernel_dtype, siging, normalize, path, stride, norm, float(head_norm_eps), bool(recompute), f32_as_f16)
+    _FWBW_CACHE[key] = op
+    return op
 
 
 def mlstm_chunkwise__hip_xl_chunk(

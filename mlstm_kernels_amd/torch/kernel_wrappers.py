@@ -32,20 +32,30 @@ def wrap_chunkwise__arbitrary_sequence_length(
 
     A chunkwise kernel that masks a ragged tail itself announces it with the function attribute
     ``supports_any_sequence_length``; it then gets the whole sequence in ONE call (keyword
-    ``any_sequence_length=True``) instead of the chunk-halving loop plus the per-token loop."""
+    ``any_sequence_length=True``) instead of the chunk-halving loop plus the per-token loop.  A step kernel with the
+    attribute ``takes_sequences_of_one`` gets q, k, v as (B, NH, 1, D) and returns h in that shape."""
     B, NH, S, DHQK = k.shape
     DHHV = v.shape[-1]
     dev = k.device
-    c_state = c_initial if c_initial is not None else torch.zeros(B, NH, DHQK, DHHV, device=dev, dtype=dtype_state)
-    n_state = n_initial if n_initial is not None else torch.zeros(B, NH, DHQK, device=dev, dtype=dtype_state)
-    m_state = m_initial if m_initial is not None else torch.zeros(B, NH, 1, device=dev, dtype=dtype_state)
+    one_call = S > 1 and getattr(mlstm_chunkwise_kernel, "supports_any_sequence_length", False)
+    c_state, n_state, m_state = c_initial, n_initial, m_initial
+    if not (one_call and c_state is None and n_state is None and m_state is None):  # such a kernel starts from zeros by itself
+        if c_state is None:
+            c_state = torch.zeros(B, NH, DHQK, DHHV, device=dev, dtype=dtype_state)
+        if n_state is None:
+            n_state = torch.zeros(B, NH, DHQK, device=dev, dtype=dtype_state)
+        if m_state is None:
+            m_state = torch.zeros(B, NH, 1, device=dev, dtype=dtype_state)
 
     if S == 1:
-        h_out, (c_state, n_state, m_state) = mlstm_step_kernel(
-            q=q.squeeze(2), k=k.squeeze(2), v=v.squeeze(2), i=i, f=f, c=c_state, n=n_state, m=m_state, eps=eps
-        )
-        h_out = h_out[:, :, None, :]
-    elif getattr(mlstm_chunkwise_kernel, "supports_any_sequence_length", False):
+        if getattr(getattr(mlstm_step_kernel, "func", mlstm_step_kernel), "takes_sequences_of_one", False):
+            h_out, (c_state, n_state, m_state) = mlstm_step_kernel(q=q, k=k, v=v, i=i, f=f, c=c_state, n=n_state, m=m_state, eps=eps)
+        else:
+            h_out, (c_state, n_state, m_state) = mlstm_step_kernel(
+                q=q.squeeze(2), k=k.squeeze(2), v=v.squeeze(2), i=i, f=f, c=c_state, n=n_state, m=m_state, eps=eps
+            )
+            h_out = h_out[:, :, None, :]
+    elif one_call:
         h_out, (c_state, n_state, m_state) = mlstm_chunkwise_kernel(
             q=q.contiguous(), k=k.contiguous(), v=v.contiguous(), f=f.contiguous(), i=i.contiguous(),
             c_initial=c_state, n_initial=n_state, m_initial=m_state,

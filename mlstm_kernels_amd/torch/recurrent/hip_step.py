@@ -8,7 +8,18 @@ from __future__ import annotations
 import torch
 
 from ... import _lib
-from ..utils import current_stream_ptr, dtype_code, ptr, require_gpu, state_dtype_code
+from ..utils import dtype_code, require_gpu
+
+_STATE_CODES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
+
+
+_host = None
+
+
+def _get_host():
+    global _host
+    _host = _lib.get_host()
+    return _host
 
 
 def _check_state_dtype(dtype_state: torch.dtype) -> torch.dtype:
@@ -38,6 +49,17 @@ def mlstm_recurrent_step__hip_fw(
 ):
     """One step.  ``matC_new`` may be ``matC_old`` itself (in-place state update, the step then moves the
     state through HBM exactly once each way); ``vecN_new``/``scaM_new`` must be distinct buffers."""
+    if qk_scale is None and dtype_state in _STATE_CODES:
+        # everything as the kernel needs it (the usual case): checked, allocated and launched in native code
+        out = (_host or _get_host()).step(matC_old, vecN_old, scaM_old, vecQ, vecK, vecV, scaI, scaF, matC_new, vecN_new,
+                                          scaM_new, eps, _STATE_CODES[dtype_state])
+        if out is not None:
+            return out
+    # something has to be converted, or is wrong
+    if vecQ.dim() == 4:   # a sequence of one
+        out = mlstm_recurrent_step__hip_fw(matC_old, vecN_old, scaM_old, vecQ.squeeze(2), vecK.squeeze(2), vecV.squeeze(2), scaI,
+                                           scaF, matC_new, vecN_new, scaM_new, qk_scale, eps, dtype_state)
+        return out[0][:, :, None, :], out[1]
     B, NH, DHQK = vecQ.shape
     DHHV = vecV.shape[-1]
     assert vecQ.shape == vecK.shape, "q and k must have the same shape"
@@ -49,31 +71,22 @@ def mlstm_recurrent_step__hip_fw(
     if qk_scale is not None and abs(qk_scale - DHQK ** -0.5) > 1e-12:
         raise NotImplementedError("the HIP step kernel uses qk_scale = DHQK**-0.5")
     dtype_state = _check_state_dtype(dtype_state)
-    dev = require_gpu(vecQ, vecK, vecV, scaI, scaF, matC_old, vecN_old, scaM_old)
+    require_gpu(vecQ, vecK, vecV, scaI, scaF, matC_old, vecN_old, scaM_old)
     qdt, gdt = vecQ.dtype, scaI.dtype   # float32, bfloat16 or float16 each; the arithmetic is float32
+    dtype_code(vecQ), dtype_code(scaI)
     q, k, v = vecQ.contiguous(), vecK.to(qdt).contiguous(), vecV.to(qdt).contiguous()
     i, f = scaI.to(gdt).contiguous(), scaF.to(gdt).contiguous()
-    c_old = matC_old.to(dtype_state).contiguous()
-    n_old = vecN_old.to(dtype_state).contiguous()
-    m_old = scaM_old.to(dtype_state).contiguous()
+    c_old, n_old, m_old = (t.to(dtype_state).contiguous() for t in (matC_old, vecN_old, scaM_old))
     if matC_new is None:
         assert vecN_new is None and scaM_new is None, "Initial states must be provided together."
-        matC_new = torch.empty_like(c_old)
-        vecN_new = torch.empty_like(n_old)
-        scaM_new = torch.empty_like(m_old)
     else:
         assert vecN_new is not None and scaM_new is not None, "Initial states must be provided together."
         for t in (matC_new, vecN_new, scaM_new):
             assert t.dtype == dtype_state and t.is_contiguous(), f"state outputs must be contiguous {dtype_state}"
-    h = torch.empty_like(v)
-    lib = _lib.get_lib()
-    rc = lib.mlstm_hip_step(
-        ptr(q), ptr(k), ptr(v), ptr(i), ptr(f), ptr(c_old), ptr(n_old), ptr(m_old),
-        ptr(h), ptr(matC_new), ptr(vecN_new), ptr(scaM_new),
-        B, NH, DHQK, DHHV, float(eps), dtype_code(q), dtype_code(i), state_dtype_code(c_old), current_stream_ptr(dev),
-    )
-    _lib.check(rc, "mlstm_hip_step")
-    return h, (matC_new, vecN_new, scaM_new)
+    out = _get_host().step(c_old, n_old, m_old, q, k, v, i, f, matC_new, vecN_new, scaM_new, eps, _STATE_CODES[dtype_state])
+    if out is None:
+        raise RuntimeError("mlstm_recurrent_step__hip: v and the state outputs must match the shapes of q and the old states")
+    return out
 
 
 def mlstm_recurrent_step__hip(
@@ -89,12 +102,15 @@ def mlstm_recurrent_step__hip(
     dtype_state: torch.dtype = torch.float32,
     **kwargs,
 ):
-    """Single mLSTM step: returns ``h (B,NH,DHHV)`` in q's dtype and ``(C', n', m')`` in ``dtype_state`` (float32 unless
+    """Single mLSTM step (q, k, v may also be sequences of one, (B, NH, 1, D)): returns ``h (B,NH,DHHV)`` in q's dtype and ``(C', n', m')`` in ``dtype_state`` (float32 unless
     asked otherwise; the arithmetic is float32 either way and h is formed from the unrounded new state)."""
     return mlstm_recurrent_step__hip_fw(
         matC_old=c, vecN_old=n, scaM_old=m, vecQ=q, vecK=k, vecV=v, scaI=i, scaF=f,
         eps=eps, dtype_state=dtype_state, **kwargs,
     )
+
+
+mlstm_recurrent_step__hip.takes_sequences_of_one = True
 
 
 def mlstm_recurrent_sequence__hip(
@@ -124,6 +140,12 @@ def mlstm_recurrent_sequence__hip(
                                   "(return_all_states=True); loop over mlstm_recurrent_step__hip for that")
     if kwargs:
         raise TypeError(f"mlstm_recurrent_sequence__hip() got unexpected keyword arguments {sorted(kwargs)}")
+    if c_initial is not None and dtype_state in _STATE_CODES:
+        # everything as the kernel needs it (the usual case): checked, allocated and launched in native code
+        out = (_host or _get_host()).sequence(q, k, v, i, f, c_initial, n_initial, m_initial, eps, _STATE_CODES[dtype_state])
+        if out is not None:
+            return out if return_last_states else out[0]
+    # something has to be made or converted, or is wrong
     B, NH, S, DHQK = q.shape
     DHHV = v.shape[-1]
     assert k.shape == q.shape, "q and k must have the same shape"
@@ -146,17 +168,10 @@ def mlstm_recurrent_sequence__hip(
         H = torch.empty(B, NH, 0, DHHV, dtype=q.dtype, device=dev)
         return (H, (c.clone(), n.clone(), m.clone())) if return_last_states else H
     qdt, gdt = q.dtype, i.dtype
-    qc, kc, vc = q.contiguous(), k.to(qdt).contiguous(), v.to(qdt).contiguous()
-    ic, fc = i.to(gdt).contiguous(), f.to(gdt).contiguous()
-    H = torch.empty(B, NH, S, DHHV, dtype=qdt, device=dev)
-    c_out, n_out, m_out = torch.empty_like(c), torch.empty_like(n), torch.empty_like(m)
-    lib = _lib.get_lib()
-    rc = lib.mlstm_hip_recurrent_sequence(
-        ptr(qc), ptr(kc), ptr(vc), ptr(ic), ptr(fc), ptr(c), ptr(n), ptr(m),
-        ptr(H), ptr(c_out), ptr(n_out), ptr(m_out),
-        B, NH, S, DHQK, DHHV, float(eps), dtype_code(qc), dtype_code(ic), state_dtype_code(c), current_stream_ptr(dev),
-    )
-    _lib.check(rc, "mlstm_hip_recurrent_sequence")
-    if return_last_states:
-        return H, (c_out, n_out, m_out)
-    return H
+    dtype_code(q), dtype_code(i)
+    out = _get_host().sequence(
+        q.contiguous(), k.to(qdt).contiguous(), v.to(qdt).contiguous(), i.to(gdt).contiguous(), f.to(gdt).contiguous(),
+        c, n, m, eps, _STATE_CODES[dtype_state])
+    if out is None:
+        raise RuntimeError("mlstm_recurrent_sequence__hip: all tensors must be on the same device")
+    return out if return_last_states else out[0]
