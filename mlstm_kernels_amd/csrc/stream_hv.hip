@@ -26,7 +26,7 @@
 //   in the same step), 2 slabs of 32 rows x 512 value columns (output product)
 // Register set and ring slot alternate from step to step and every source chunk has an even number of steps, so both
 // are compile-time constants everywhere.
-// Supported: DHQK = 256, DHHV a multiple of 512, S a multiple of 128, no head norm; everything else runs par_hv.hip.
+// Supported: DHQK = 256, DHHV a multiple of 512 (exactly 512 with a head norm); everything else runs par_hv.hip.
 #include "common.h"
 #include "kernels.h"
 
@@ -151,14 +151,16 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     }                                                                                                                \
     if (__builtin_amdgcn_readfirstlane((int)((w_ >> 22) & 1)) && p < 64) {                                           \
       ovec[p] = fa##E[0];                                                                                   \
-      if (IS_DV) orho[p] = a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f;                                              \
+      if (IS_DV) orho[p] = ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
     }                                                                                                                \
   }
     // base_: (batch, head) base of the operand; g0_: byte offset of the thread's first piece, gs_: distance between
     // its pieces; gi_: index of the gate-vector entry that rides along (stored only with the flag set; the other
     // slabs request an entry all the same so that every step issues the same loads); NP_: pieces per thread (8, or 4
-    // for the half-size slabs of the resident rows, flagged by bit 23 of the destination word)
-#define HV_PROC(E, NP_, base_, g0_, gs_, dstw_, gi_)                                                                 \
+    // for the half-size slabs of the resident rows, flagged by bit 23 of the destination word); lim_: largest byte
+    // offset of a piece.  Rows past the end of the sequence re-read its last row: as keys their gate factor is zero
+    // (their w is infinite), as query rows of dV their rho is stored as zero (bit 24), as output rows they are not stored
+#define HV_PROC(E, NP_, base_, g0_, gs_, lim_, dstw_, gi_)                                                                 \
   {                                                                                                                  \
     if (L >= 4) __syncthreads();                                                                                           \
     /* piece by piece: the old content of a register goes to LDS, then the register is requested anew, so that the */ \
@@ -172,7 +174,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     const bool st_ = L >= 3;                                                                                         \
     if (st_ && __builtin_amdgcn_readfirstlane((int)((w_ >> 22) & 1)) && p < 64) {                                    \
       ovec[p] = fa##E[0];                                                                                   \
-      if (IS_DV) orho[p] = a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f;                                              \
+      if (IS_DV) orho[p] = ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
     }                                                                                                                \
     fa##E[0] = ov_src[gi_];                                                                                          \
     fa##E[1] = rho_src[gi_];                                                                                         \
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         *(uint2*)(smem_raw + d0_ + i_ * step_) = make_uint2(fd##E[i_][0], fd##E[i_][1]);                             \
         *(uint2*)(smem_raw + d0_ + i_ * step_ + half_) = make_uint2(fd##E[i_][2], fd##E[i_][3]);                     \
       }                                                                                                              \
-      if (i_ < (NP_)) fd##E[i_] = *(const u32x4*)((base_) + ((g0_) + i_ * (gs_)));                                             \
+      if (i_ < (NP_)) fd##E[i_] = *(const u32x4*)((base_) + min((g0_) + i_ * (gs_), (lim_)));                         \
     }                                                                                                                \
     fw##E = (dstw_) | ((NP_) == 4 ? 1u << 23 : 0u);                                                                  \
     ++L;                                                                                                             \
@@ -195,16 +197,17 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const size_t gown = (size_t)it.bh * Sp + (size_t)it.c * kChunk + (pl & 63);
       // fragment-order destination of piece pc inside a row (see store_perm16)
       const uint32_t permo = (pc >> 1) * 32 + 8 * (pc & 1);
+      const uint32_t klim = (uint32_t)(S - 1) * (DHQK * 2) + pc * 16;  // this thread's piece of the last row
       {
         // ---- resident rows, 32 per step (half-size slabs: four steps for the consumers' epilogue of the previous
         // item, and a step count per item that is a multiple of three)
         const char* const base = Xn_b + (size_t)it.bh * S * DHQK * 2;
         const uint32_t g0 = ((uint32_t)(it.c * kChunk) + row) * (DHQK * 2) + pc * 16;
         const uint32_t d0 = row * (QS * 2) + permo;
-        HV_PROC(0, 4, base, g0, 8 * DHQK * 2, d0, gown)
-        HV_PROC(1, 4, base, g0 + 32 * DHQK * 2, 8 * DHQK * 2, d0 + 32 * QS * 2, gown)
-        HV_PROC(2, 4, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, d0 + 64 * QS * 2, gown)
-        HV_PROC(0, 4, base, g0 + 96 * DHQK * 2, 8 * DHQK * 2, d0 + 96 * QS * 2, gown)
+        HV_PROC(0, 4, base, g0, 8 * DHQK * 2, klim, d0, gown)
+        HV_PROC(1, 4, base, g0 + 32 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 32 * QS * 2, gown)
+        HV_PROC(2, 4, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 64 * QS * 2, gown)
+        HV_PROC(0, 4, base, g0 + 96 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 96 * QS * 2, gown)
       }
       {
         // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks
@@ -212,14 +215,14 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         const uint32_t f0 = pl >> 6;  // fragment of the first piece inside the slab: block f0 / 2, contraction step f0 % 2
         const uint32_t g0 = (((uint32_t)it.ch * 16 + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
         const uint32_t r0 = (kRing0Off + pl * 16) | (1u << 20), r1 = (kRing1Off + pl * 16) | (1u << 20);
-        HV_PROC(1, 8, base, g0, 2 * ND * 1024, r0, gown)
-        HV_PROC(2, 8, base, g0 + 1 * 2048, 2 * ND * 1024, r1, gown)
-        HV_PROC(0, 8, base, g0 + 2 * 2048, 2 * ND * 1024, r0, gown)
-        HV_PROC(1, 8, base, g0 + 3 * 2048, 2 * ND * 1024, r1, gown)
-        HV_PROC(2, 8, base, g0 + 4 * 2048, 2 * ND * 1024, r0, gown)
-        HV_PROC(0, 8, base, g0 + 5 * 2048, 2 * ND * 1024, r1, gown)
-        HV_PROC(1, 8, base, g0 + 6 * 2048, 2 * ND * 1024, r0, gown)
-        HV_PROC(2, 8, base, g0 + 7 * 2048, 2 * ND * 1024, r1, gown)
+        HV_PROC(1, 8, base, g0, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(2, 8, base, g0 + 1 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(0, 8, base, g0 + 2 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(1, 8, base, g0 + 3 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(2, 8, base, g0 + 4 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(0, 8, base, g0 + 5 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(1, 8, base, g0 + 6 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(2, 8, base, g0 + 7 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
       }
       {
         const char* const kbase = Xo_b + (size_t)it.bh * S * DHQK * 2;
@@ -227,20 +230,23 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         const uint32_t kd = row * (QS * 2) + permo;
         const uint32_t vrow = pl >> 6, vpc = pl & 63;  // rows of 1024 bytes: 64 pieces per row, 4 rows per sweep
         const uint32_t vd = (vrow * (VS * 2) + vpc * 16) | (3u << 20);
+        const uint32_t vlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * 1024 + vpc * 16;
         for (int sci = 0; sci < it.nsc; ++sci) {
           const int sc = it.sc_first + sci * it.sc_step;
           const uint32_t t0 = (uint32_t)(sc * kChunk);
           const size_t gi = (size_t)it.bh * Sp + (size_t)sc * kChunk + (pl & 63);
           const uint32_t vg = (t0 + vrow) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * 1024 + vpc * 16;
+          // (bit 24: the gate-vector entry this thread carries lies past the end of the sequence)
+          const uint32_t past0 = t0 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24, past1 = t0 + 64 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24;
           const uint32_t vgs = 4 * (uint32_t)DHHV * 2, vg32 = 32 * (uint32_t)DHHV * 2;
           // first half: scores -> slot 0, value rows -> slot 1 and slot 0
-          HV_PROC(0, 8, kbase, (t0 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, (kRing0Off + kd) | (1u << 22), gi)
-          HV_PROC(1, 8, vbase, vg, vgs, kRing1Off + vd, gown)
-          HV_PROC(2, 8, vbase, vg + vg32, vgs, kRing0Off + vd, gown)
+          HV_PROC(0, 8, kbase, (t0 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, klim, (kRing0Off + kd) | (1u << 22) | past0, gi)
+          HV_PROC(1, 8, vbase, vg, vgs, vlim, kRing1Off + vd, gown)
+          HV_PROC(2, 8, vbase, vg + vg32, vgs, vlim, kRing0Off + vd, gown)
           // second half: the other way round
-          HV_PROC(0, 8, kbase, (t0 + 64 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, (kRing1Off + kd) | (1u << 22), gi + 64)
-          HV_PROC(1, 8, vbase, vg + 2 * vg32, vgs, kRing0Off + vd, gown)
-          HV_PROC(2, 8, vbase, vg + 3 * vg32, vgs, kRing1Off + vd, gown)
+          HV_PROC(0, 8, kbase, (t0 + 64 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, klim, (kRing1Off + kd) | (1u << 22) | past1, gi + 64)
+          HV_PROC(1, 8, vbase, vg + 2 * vg32, vgs, vlim, kRing0Off + vd, gown)
+          HV_PROC(2, 8, vbase, vg + 3 * vg32, vgs, vlim, kRing1Off + vd, gown)
         }
       }
     }
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const float ex_ = t1_ * iv * (1.f / 512.f), ex2_ = t2_ * iv * iv * (1.f / 512.f);                              \
       const float mean_ = a.head_norm == 1 ? ex_ : 0.f;                                                              \
       const float rstd_ = rsqrtf(fmaxf(ex2_ - mean_ * mean_, 0.f) + a.norm_eps);                                     \
-      if (ci == 0 && h == 0) {                                                                                       \
+      if (ci == 0 && h == 0 && prev.c * kChunk + t_ < S) {                                                           \
         const size_t tg_ = (size_t)prev.bh * S + (size_t)prev.c * kChunk + t_;                                       \
         a.norm_mean[tg_] = mean_;                                                                                    \
         a.norm_rstd[tg_] = rstd_;                                                                                    \
@@ -315,9 +321,11 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     uint16_t* const Og = a.Out + ((size_t)prev.bh * S + (size_t)prev.c * kChunk + 64 * pi + 32 * NB) * DHHV +        \
                          prev.ch * 512 + 128 * ci + 32 * (MB0_);                                                     \
     constexpr int VPR = 4 * (NMB_); /* 16-byte vectors per row */                                                    \
+    const int rows_left_ = S - (prev.c * kChunk + 64 * pi + 32 * NB);                                                \
     _Pragma("unroll") for (int k = 0; k < 32 * VPR / 64; ++k) {                                                      \
       const int row = le / VPR + (64 / VPR) * k, pc = le % VPR;                                                      \
-      __builtin_nontemporal_store(*(const u32x4*)(stg + row * SR + pc * 8), (u32x4*)(Og + (size_t)row * DHHV + pc * 8)); \
+      if (row < rows_left_)                                                                                          \
+        __builtin_nontemporal_store(*(const u32x4*)(stg + row * SR + pc * 8), (u32x4*)(Og + (size_t)row * DHHV + pc * 8)); \
     }                                                                                                                \
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                                           \
     __builtin_amdgcn_wave_barrier();                                                                                 \
@@ -565,8 +573,10 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
                 if (it.ch == 0) {
                   a.nrow_out[gofs + t] = nmax;
                   const size_t tg = (size_t)bh * S + (size_t)c * kChunk + t;
-                  if (a.n_out != nullptr) a.n_out[tg] = nmax;
-                  if (a.m_out != nullptr) a.m_out[tg] = mcr;
+                  if (c * kChunk + t < S) {
+                    if (a.n_out != nullptr) a.n_out[tg] = nmax;
+                    if (a.m_out != nullptr) a.m_out[tg] = mcr;
+                  }
                 }
               }
             }
@@ -589,7 +599,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
 bool stream_hv_supported(const ParHvArgs& a) {
   // with the fused head norm a work item must hold complete rows: one group of 512 value columns
   const bool norm_ok = a.head_norm == 0 || (a.DHHV == 512 && a.norm_mean != nullptr && a.norm_rstd != nullptr);
-  return a.DHQK == 256 && a.DHHV % 512 == 0 && a.S % kChunk == 0 && norm_ok;
+  return a.DHQK == 256 && a.DHHV % 512 == 0 && norm_ok;
 }
 
 namespace {
@@ -616,7 +626,7 @@ const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
 
 const char* launch_stream_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
   if (!stream_hv_supported(a))
-    return "stream_hv: unsupported shape (needs DHQK = 256, DHHV % 512 == 0, S % 128 == 0; with a head norm DHHV = 512)";
+    return "stream_hv: unsupported shape (needs DHQK = 256, DHHV % 512 == 0; with a head norm DHHV = 512)";
   if (a.stride < 1 || a.stride > kMaxStateStride) return "stream_hv: state stride out of range";
   if (is_dv) return a.f16 ? launch_stream_hv_t<true, true>(a, BH, stream) : launch_stream_hv_t<true, false>(a, BH, stream);
   if (a.head_norm != 0)

@@ -20,14 +20,14 @@
 //           4 steps  [64 Q rows]                                                   row dots q . dQ; dQ rows leave
 //       K  NV steps  [dC fragments | V rows],  4 steps [64 Q rows], 4 steps [64 K rows]   the same for dK (P read
 //                                                                                  transposed)
-//     A window moves 3 * DHHV + 512 KB through the CU (2048 KB at DHHV = 512) where its four chunk-and-gradient items
-//     take 2944 KB in stream_qk.hip, and multiplies every score block once instead of twice.
+//     A window moves 3 * DHHV + 512 KB through the CU (2048 KB at DHHV = 512) where the same arrangement for
+//     single chunks and gradients took 2944 KB, and multiplies every score block once instead of twice.
 //   * A consumer wave owns 64 head-dim rows x four 32-position blocks of alternating parity (128 accumulator
 //     registers); the causal structure then loads both parities nearly alike.  The q (k) rows of the gate-gradient
 //     row dots come through the ring like every other operand (fetched by the consumers themselves they cost a
 //     memory latency per handful of positions); the rounded results pass through a private 2 KB staging tile per
 //     wave into row order and are stored as full 128-byte lines.
-// Supported: state stride 2, DHQK = 256, DHHV a multiple of 64, S a multiple of 256.
+// Supported: state stride 2, DHQK = 256, DHHV a multiple of 64.
 #include <type_traits>
 
 #include "common.h"
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   if (G % 8 == 0) vid = (vid % 8) * (G / 8) + vid / 8;  // consecutive ids share an XCD (and its L2)
   const int NC = a.NC, S = a.S, DHHV = a.DHHV;
   const int NV = DHHV / 32;   // steps of 32 value columns (even)
-  const int NWIN = NC / 2;
+  const int NWIN = (NC + 1) / 2;  // the last window may hold one chunk only: the other half of it is past the end
   const size_t Sp = (size_t)NC * kChunk;
 
   if (wave_all >= 8) {
@@ -124,8 +124,9 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) *(u32x4*)(smem_raw + dB_ + i_ * 4096) = fd##E[4 + i_];          \
   }
     // one step: bA_/gA_/sA_ base, first byte offset and piece distance of pieces 0..3, bB_/gB_/sB_ of pieces 4..7;
-    // dA_ / dB_ destination units of the two halves inside the slot
-#define WQ_PROC(E, bA_, gA_, sA_, bB_, gB_, sB_, dAu_, dBu_)                                                         \
+    // lA_, lB_ largest byte offset of a piece (rows past the end of the sequence re-read its last row: their score
+    // factors are zero and their results are not stored), dAu_ / dBu_ destination units of the two halves inside the slot
+#define WQ_PROC(E, bA_, gA_, sA_, lA_, bB_, gB_, sB_, lB_, dAu_, dBu_)                                                         \
   {                                                                                                                  \
     if (L >= 3) __syncthreads();                                                                                     \
     /* piece by piece: the old content of a register goes to LDS, then the register is requested anew, so that the */ \
@@ -135,11 +136,11 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     const bool st_ = L >= 2;                                                                                         \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oA_ + i_ * 4096) = fd##E[i_];                                                    \
-      fd##E[i_] = *(const u32x4*)((bA_) + ((gA_) + i_ * (sA_)));                                                     \
+      fd##E[i_] = *(const u32x4*)((bA_) + min((gA_) + i_ * (sA_), (lA_)));                                                     \
     }                                                                                                                \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oB_ + i_ * 4096) = fd##E[4 + i_];                                                \
-      fd##E[4 + i_] = *(const u32x4*)((bB_) + ((gB_) + i_ * (sB_)));                                                 \
+      fd##E[4 + i_] = *(const u32x4*)((bB_) + min((gB_) + i_ * (sB_), (lB_)));                                                 \
     }                                                                                                                \
     fw##E = ((dAu_) + (E) * (kWqSlot / 16)) | (((dBu_) + (E) * (kWqSlot / 16)) << 16);                               \
     ++L;                                                                                                             \
@@ -161,6 +162,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const uint32_t xdu = xrow * 4 + (xun ^ (uint32_t)wq_f64((int)xrow));
       const uint32_t xg = (t0 + xrow) * (uint32_t)(DHHV * 2) + xun * 16;
       const uint32_t xstep = 64 * (uint32_t)DHHV * 2;
+      const uint32_t xlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + xun * 16;  // this thread's unit of the last row
       // state fragments of 32 value columns: 16 KB contiguous in memory; lanes 32..63 of every fragment are stored 4
       // slots off so that the two lane halves a transposing read touches together fall on different LDS banks
       const uint32_t cdu = pl ^ (((pl >> 5) & 1) << 2);
@@ -168,40 +170,41 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const uint32_t zrow = pl >> 5, zun = pl & 31;
       const uint32_t zdu = zrow * 32 + (zun ^ (2 * (zrow & 3)));
       const uint32_t zg = (t0 + zrow) * (DHQK * 2) + zun * 16;
+      const uint32_t zlim = (uint32_t)(S - 1) * (DHQK * 2) + zun * 16;
       // (every loop works on its own opaque copy of the offsets: addresses shared between two loops would otherwise be
       // kept, and spilled, across everything in between)
 #define WQ_ROWS(bA_, bB_)                                                                                            \
   {                                                                                                                  \
     const uint32_t zz = (uint32_t)opaque((int)zg);                                                                   \
     for (int z = 0; z < 4; z += 2) {                                                                                 \
-      WQ_PROC(0, bA_, zz + z * 32768, 4096, bB_, zz + z * 32768 + 16384, 4096, zdu, 1024 + zdu)                      \
-      WQ_PROC(1, bA_, zz + (z + 1) * 32768, 4096, bB_, zz + (z + 1) * 32768 + 16384, 4096, zdu, 1024 + zdu)          \
+      WQ_PROC(0, bA_, zz + z * 32768, 4096, zlim, bB_, zz + z * 32768 + 16384, 4096, zlim, zdu, 1024 + zdu)                      \
+      WQ_PROC(1, bA_, zz + (z + 1) * 32768, 4096, zlim, bB_, zz + (z + 1) * 32768 + 16384, 4096, zlim, zdu, 1024 + zdu)          \
     }                                                                                                                \
   }
       // ---- phase S: dH rows | V rows
       {
-        const uint32_t xx = (uint32_t)opaque((int)xg);
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim);
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, dH_b, xx + w * 64, xstep, V_b, xx + w * 64, xstep, xdu, 1024 + xdu)
-          WQ_PROC(1, dH_b, xx + (w + 1) * 64, xstep, V_b, xx + (w + 1) * 64, xstep, xdu, 1024 + xdu)
+          WQ_PROC(0, dH_b, xx + w * 64, xstep, xl + w * 64, V_b, xx + w * 64, xstep, xl + w * 64, xdu, 1024 + xdu)
+          WQ_PROC(1, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, xdu, 1024 + xdu)
         }
       }
       // ---- phase Q: C fragments | dH rows, then the K rows (products) and the Q rows (row dots)
       {
-        const uint32_t xx = (uint32_t)opaque((int)xg), cc = (uint32_t)opaque((int)(pl * 16));
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16));
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, C_b, (uint32_t)w * 16384 + cc, 4096, dH_b, xx + w * 64, xstep, cdu, 1024 + xdu)
-          WQ_PROC(1, C_b, (uint32_t)(w + 1) * 16384 + cc, 4096, dH_b, xx + (w + 1) * 64, xstep, cdu, 1024 + xdu)
+          WQ_PROC(0, C_b, (uint32_t)w * 16384 + cc, 4096, 0xffffffffu, dH_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
+          WQ_PROC(1, C_b, (uint32_t)(w + 1) * 16384 + cc, 4096, 0xffffffffu, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
       }
       WQ_ROWS(K_b, K_b)
       WQ_ROWS(Q_b, Q_b)
       // ---- phase K: dC fragments | V rows, then the Q rows (products) and the K rows (row dots)
       {
-        const uint32_t xx = (uint32_t)opaque((int)xg), cc = (uint32_t)opaque((int)(pl * 16));
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16));
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, dC_b, (uint32_t)w * 16384 + cc, 4096, V_b, xx + w * 64, xstep, cdu, 1024 + xdu)
-          WQ_PROC(1, dC_b, (uint32_t)(w + 1) * 16384 + cc, 4096, V_b, xx + (w + 1) * 64, xstep, cdu, 1024 + xdu)
+          WQ_PROC(0, dC_b, (uint32_t)w * 16384 + cc, 4096, 0xffffffffu, V_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
+          WQ_PROC(1, dC_b, (uint32_t)(w + 1) * 16384 + cc, 4096, 0xffffffffu, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
       }
       WQ_ROWS(Q_b, Q_b)
@@ -241,7 +244,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     auto finish_rowdots = [&]() {
       if (pending && tid < 256) {
         const float dot = (red[tid] + red[256 + tid]) + (red[512 + tid] + red[768 + tid]);
-        (pending == 2 ? a.rowdot2 : a.rowdot)[(size_t)prev.bh * Sp + (size_t)prev.win * 256 + tid] = dot;
+        if (prev.win * 256 + tid < S)
+          (pending == 2 ? a.rowdot2 : a.rowdot)[(size_t)prev.bh * Sp + (size_t)prev.win * 256 + tid] = dot;
       }
       pending = 0;
     };
@@ -253,15 +257,17 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const float* graw = a.g.graw + (size_t)bh * NC;
       const float* mst = a.g.mstates + (size_t)bh * (NC + 1);
       const float g01 = graw[c0];   // decay over chunk c0: what separates a position of c1 from the keys of c0
+      const int n_pos = S - 256 * it.win;   // positions of the window inside the sequence (256 or more: all)
 
       // ================================================================================= phase S: the score blocks
       {
         // gate vectors of the window, requested now, written to LDS after the first step
         float pu = 0.f, pw = 0.f, pr = 1.f;
         if (tid < 256) {
-          pu = a.g.u[gofs + tid];
-          pw = a.g.w[gofs + tid];
-          if (a.use_nrow) pr = a.nrow[gofs + tid];
+          const int tv = min(tid, n_pos - 1);
+          pu = a.g.u[gofs + tv];
+          pw = a.g.w[gofs + tv];
+          if (a.use_nrow) pr = a.nrow[gofs + tv];
         }
         f32x16 sacc[5];
 #pragma unroll
@@ -277,9 +283,10 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           }
           if (w == (NV > 2 ? 1 : 0)) {
             if (tid < 256) {
+              // past the end: no key (w = infinity), no query (factor 0)
               uvec[tid] = pu;
-              wvec[tid] = pw;
-              lqr[tid] = __log2f(a.qk_scale * (a.use_nrow ? 1.f / (pr + a.eps) : 1.f));
+              wvec[tid] = tid < n_pos ? pw : __builtin_inff();
+              lqr[tid] = tid < n_pos ? __log2f(a.qk_scale * (a.use_nrow ? 1.f / (pr + a.eps) : 1.f)) : -__builtin_inff();
             }
           }
           const int le = opaque(lane);
@@ -337,9 +344,10 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         // step of the value pass, used after its last one (registers are what this kernel is short of)
         float csn = 0.f;
         if (tid < 256) {
-          const size_t gi = gofs + tid;
+          const size_t gi = gofs + min(tid, n_pos - 1);
           if (dk) {
-            const float xs = __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]);   // keys of c0 see dC through chunk c1
+            // keys of c0 see dC through chunk c1, where there is one (the gradient kept is that after the last chunk)
+            const float xs = c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
             csn = a.g.abar[gi] * (tid < 128 ? xs : 1.f);
           } else {
             const float xs = __expf(g01 + mst[c0] - mst[c0 + 1]);                // positions of c1 see C through chunk c0
@@ -507,8 +515,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
             const u32x4 o1 = *(const u32x4*)(stg + (row8 + 8) * 128 + ((un ^ row8) * 16));
             __builtin_amdgcn_wave_barrier();
             const uint32_t n0 = (uint32_t)(64 * z + 32 * par + 16 * q);
-            __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (DHQK * 2))));
-            __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (DHQK * 2))));
+            if ((int)n0 + row8 < n_pos) __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (DHQK * 2))));
+            if ((int)n0 + 8 + row8 < n_pos) __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (DHQK * 2))));
           }
         }
         pending = dk ? 2 : 1;
@@ -524,13 +532,13 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 }
 
 bool window_qk_supported(const ParQkArgs& a) {
-  return a.stride == 2 && a.DHQK == 256 && a.DHHV % 64 == 0 && a.S % (2 * kChunk) == 0;
+  return a.stride == 2 && a.DHQK == 256 && a.DHHV % 64 == 0;
 }
 
 namespace {
 template <bool F16>
 const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
-  const long long n_items = (long long)BH * (a.NC / 2);
+  const long long n_items = (long long)BH * ((a.NC + 1) / 2);
   if (n_items >= (1ll << 31)) return "window_qk: too many work items";
   if ((size_t)a.S * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32))
     return "window_qk: one (batch, head) slab of an input exceeds 4 GiB";
@@ -548,7 +556,7 @@ const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
 }  // namespace
 
 const char* launch_window_qk(const ParQkArgs& a, int BH, hipStream_t stream) {
-  if (!window_qk_supported(a)) return "window_qk: unsupported shape (needs state stride 2, DHQK = 256, DHHV % 64 == 0, S % 256 == 0)";
+  if (!window_qk_supported(a)) return "window_qk: unsupported shape (needs state stride 2, DHQK = 256, DHHV % 64 == 0)";
   if (a.states2 == nullptr || a.Out2 == nullptr || a.rowdot2 == nullptr) return "window_qk: the dK operands are missing";
   return a.f16 ? launch_window_qk_t<true>(a, BH, stream) : launch_window_qk_t<false>(a, BH, stream);
 }
