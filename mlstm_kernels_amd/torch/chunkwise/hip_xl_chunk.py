@@ -291,3 +291,6 @@ def mlstm_siging_chunkwise__hip_xl_chunk(
 # the kernels mask a ragged last chunk themselves: sequence-length adapters may hand over any S >= 1 in one call
 mlstm_chunkwise__hip_xl_chunk.supports_any_sequence_length = True
 mlstm_siging_chunkwise__hip_xl_chunk.supports_any_sequence_length = True
+# the rules they check otherwise, for an adapter that skips the padding but keeps the rules
+mlstm_chunkwise__hip_xl_chunk.check_sequence_length = validate_xl_chunk_shapes
+mlstm_siging_chunkwise__hip_xl_chunk.check_sequence_length = validate_xl_chunk_shapes

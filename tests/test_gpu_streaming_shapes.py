@@ -1,0 +1,77 @@
+"""The streaming kernels at the lengths where they can go wrong (one position, either side of a chunk and of a window of
+two chunks, several windows with a ragged last one), forward and backward, against the fp64 oracle; and the padding
+adapter, which hands such a length over as it is, against explicit padding.  Tolerances are norm-relative as in the
+randomised sweep: H 6e-3, gradients 8e-3, gate gradients 5e-2 of their scale."""
+import pytest
+import torch
+
+import oracle as O
+from helpers import make_qkvif, rel_norm
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(S, DQ, DV, *, B=1, NH=2, sig=False, norm="none", init=False, seed=0, dtype=torch.bfloat16, path="auto"):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    q, k, v, i, f = make_qkvif(B, NH, S, DQ, DV, seed=seed, dtype=dtype)
+    g = torch.Generator().manual_seed(seed + 1)
+    dH = torch.randn(B, NH, S, DV, generator=g).to(dtype)
+    st = (None, None, None)
+    if init:
+        st = (0.1 * torch.randn(B, NH, DQ, DV, generator=g), 0.1 * torch.randn(B, NH, DQ, generator=g), 0.3 * torch.randn(B, NH, 1, generator=g))
+    d = lambda t: None if t is None else t.double()
+    L = next(x for x in (64, 32, 16, 8, 4, 2, 1) if S % x == 0)
+    m0 = None if sig else d(st[2])
+    fw = O.chunkwise_fw(d(q), d(k), d(v), d(i), d(f), d(st[0]), d(st[1]), m0, chunk_size=L, siging=sig)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v, i, f)]
+    cu = lambda t: None if t is None else t.cuda()
+    print(f"S={S} {DQ}/{DV} sig={sig} norm={norm} init={init} {dtype} {path}", flush=True)
+    H, last = op(*leaves, c_initial=cu(st[0]), n_initial=cu(st[1]), m_initial=cu(st[2]), return_last_states=True, chunk_size=128,
+                 any_sequence_length=True, kernel_path=path, head_norm=norm)
+    H.backward(dH.cuda())
+    if norm == "none":
+        H_ref, dH_ref = fw["H"], d(dH)
+    else:
+        raw = fw["H"].detach().requires_grad_(True)
+        x = raw - raw.mean(-1, keepdim=True) if norm == "layer" else raw
+        H_ref = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6)
+        (dH_ref,) = torch.autograd.grad(H_ref, raw, d(dH))
+    bw = O.chunkwise_bw(d(q), d(k), d(v), d(i), d(f), dH_ref, d(st[0]), d(st[1]), m0, None, chunk_size=L, siging=sig)
+    tol = 2.0 if norm != "none" else 1.0   # the norm divides by the spread of a row, which may be small
+    assert rel_norm(H, H_ref) <= 6e-3 * tol
+    # (the norm of the only row of a sequence removes its scale, which is all q and k change: their gradients vanish)
+    grads = list(zip(("dQ", "dK", "dV"), leaves, bw[:3]))[2 if norm != "none" and S == 1 else 0:]
+    for name, leaf, ref in grads:
+        assert rel_norm(leaf.grad, ref) <= 8e-3 * tol, name
+    for name, leaf, ref in zip(("dI", "dF"), leaves[3:], bw[3:5]) if len(grads) == 3 else ():
+        # (a sequence of one has dF = 0: the oracle's own rounding is no scale)
+        scale = max(float(ref.abs().max()), 1e-3 * float(bw[3].abs().max()))
+        assert float((leaf.grad.double().cpu() - ref).abs().max()) <= 5e-2 * tol * scale, name
+    assert rel_norm(last[0], fw["C_last"]) <= 1e-3
+
+
+@pytest.mark.parametrize("S", [1, 63, 127, 129, 255, 257, 384, 385, 1001])
+@pytest.mark.parametrize("opt", [dict(), dict(sig=True, init=True), dict(norm="layer"), dict(dtype=torch.float16, init=True)],
+                         ids=["exp", "sig-init", "norm", "fp16-init"])
+def test_ragged_lengths(S, opt):
+    _run(S, 256, 512, seed=S, **opt)
+
+
+@pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
+def test_padding_adapter_without_padding(S, chunk):
+    from mlstm_kernels_amd.torch.backend_module import mLSTMBackend, mLSTMBackendConfig
+
+    backend = mLSTMBackend(mLSTMBackendConfig(mode="train_with_padding", chunk_size=chunk, return_last_states=False))
+    q, k, v, i, f = make_qkvif(2, 2, S, 256, 512, seed=S)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v, i, f)]
+    dH = torch.randn(2, 2, S, 512, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    grads = torch.autograd.grad(backend(*leaves), leaves, dH)
+    S_pad = -(-S // chunk) * chunk
+    padded = [torch.cat([t.cuda(), t.new_zeros(*t.shape[:2], S_pad - S, *t.shape[3:]).cuda()], dim=2).requires_grad_(True)
+              for t in (q, k, v, i, f)]
+    ref = torch.autograd.grad(mLSTMBackend(mLSTMBackendConfig(mode="train", chunk_size=chunk, return_last_states=False))(*padded)[:, :, :S],
+                              padded, dH)
+    for name, x, y in zip(("dQ", "dK", "dV", "dI", "dF"), grads, ref):
+        assert rel_norm(x, y[:, :, :S]) <= 2e-3, name
