@@ -78,18 +78,19 @@ const char* check_options(int path, int state_stride, int DHQK, int DHHV) {
   return nullptr;
 }
 // H / dV kernel of the split form: the streaming kernel where the path asks for it (or leaves the choice open) and the
-// shape is one it supports, otherwise the tiled kernel
+// shape is one it supports; MLSTM_PATH_AUTO: the window kernel where it is faster; otherwise the tiled kernel
 const char* launch_hv(int path, const mlstm::ParHvArgs& a, int BH, bool is_dv, hipStream_t st) {
   if (path == MLSTM_PATH_STREAM && !mlstm::stream_hv_supported(a))
     return "the stream kernel path supports DHQK = 256, DHHV % 512 == 0 only (with a head norm: DHHV = 512)";
   if ((path == MLSTM_PATH_STREAM || path == MLSTM_PATH_AUTO) && mlstm::stream_hv_supported(a))
     return mlstm::launch_stream_hv(a, BH, is_dv, st);
+  if (path == MLSTM_PATH_AUTO && mlstm::window_hv_preferred(a, BH)) return mlstm::launch_window_hv(a, BH, is_dv, st);
   return mlstm::launch_par_hv(a, BH, is_dv, st);
 }
-// dQ / dK launch.  MLSTM_PATH_STREAM and MLSTM_PATH_AUTO: the window kernel where stride and shape allow, else the tiled
-// pair kernel; MLSTM_PATH_SPLIT: the tiled pair kernel
+// dQ / dK launch.  MLSTM_PATH_STREAM: the window kernel where the stride allows; MLSTM_PATH_AUTO: where it is faster;
+// else the tiled pair kernel; MLSTM_PATH_SPLIT: the tiled pair kernel
 const char* launch_qk(int path, const mlstm::ParQkArgs& a, int BH, hipStream_t st) {
-  if ((path == MLSTM_PATH_STREAM || path == MLSTM_PATH_AUTO) && mlstm::window_qk_supported(a))
+  if (path == MLSTM_PATH_STREAM ? mlstm::window_qk_supported(a) : path == MLSTM_PATH_AUTO && mlstm::window_qk_preferred(a, BH))
     return mlstm::launch_window_qk(a, BH, st);
   return mlstm::launch_par_qk_pair(a, BH, st);
 }

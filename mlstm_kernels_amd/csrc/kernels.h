@@ -160,12 +160,17 @@ bool par_hv_head_norm_supported(int DHHV);
 // streaming (persistent, producer / consumer waves) form of the same two kernels for the shapes it supports
 bool stream_hv_supported(const ParHvArgs& a);
 const char* launch_stream_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
+// form of the same two kernels for windows of two chunks (state stride 2), any head dimensions
+bool window_hv_supported(const ParHvArgs& a);
+bool window_hv_preferred(const ParHvArgs& a, int BH);  // supported, and faster than the tiled kernel at this size
+const char* launch_window_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 const char* launch_head_norm_bw(const HeadNormBwArgs& a, hipStream_t stream);
 bool fused_hv_supported(int DHQK, int DHHV);
 const char* launch_fused_hv(const FusedHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 const char* launch_par_qk_pair(const ParQkArgs& a, int BH, hipStream_t stream);
 // streaming (persistent, producer / consumer waves) form of the same launch for windows of two chunks
 bool window_qk_supported(const ParQkArgs& a);
+bool window_qk_preferred(const ParQkArgs& a, int BH);
 const char* launch_window_qk(const ParQkArgs& a, int BH, hipStream_t stream);
 int par_qk_head_tile(int DHQK);  // head-dimension rows per workgroup of the dQ/dK kernel
 const char* launch_gate_grads(const GateGradArgs& a, int BH, hipStream_t stream);

@@ -1,0 +1,53 @@
+// What the two window kernels (window_hv.hip, window_qk.hip) share: a WINDOW is the pair of chunks (256 positions) that
+// share a kept state at state stride 2; its causal score matrix is a lower triangle of 8 x 8 blocks of 32 x 32, 36
+// blocks, which eight consumer waves compute together and keep in LDS as 16-bit values.
+#pragma once
+#include "common.h"
+
+namespace mlstm {
+
+struct WinItem {
+  int bh, win;  // (batch * head), window
+};
+
+// Work item of workgroup `vid` in round `round`: consecutive workgroups take consecutive windows (neighbours share rows
+// through the L2 of their XCD); the assignment rotates by one per round.
+__device__ __forceinline__ bool win_decode(WinItem& it, int round, int vid, int G, int n_items, int NWIN) {
+  const int rot = (vid + round) % G;
+  const long long idx = (long long)round * G + rot;
+  if (idx >= n_items) return false;
+  it.win = (int)idx % NWIN;
+  it.bh = (int)idx / NWIN;
+  return true;
+}
+
+constexpr float kWinLog2e = 1.4426950408889634f;
+constexpr int kWinSlot = 32768;          // bytes per ring slot (the largest slab)
+constexpr int kWinPOfs = 2 * kWinSlot;   // P behind the two slots: 36 blocks of 32 x 32 (2 KB each, 64-byte rows, swizzled)
+constexpr int kWinPBytes = 36 * 2048;
+
+// 16-byte-unit swizzle of tiles with 64-byte rows (operand rows of 32 columns, blocks of P): eight consecutive rows read
+// at one unit, and the 4 rows x 2 units patch of a transposing read, both fall on distinct LDS banks
+__device__ __forceinline__ int win_f64(int row) { return (((row >> 1) & 1) << 1) | ((row >> 2) & 1); }
+
+// The blocks (tb, jb) of the lower triangle that a consumer wave computes: three blocks of row ta (keys ja, ja + 1, ja + 2)
+// and up to two of row tc (keys jc, jc + 1).  With at most two rows per wave and the split between them fixed, the
+// operand of a row is read once for all its blocks: seven fragments feed five matrix instructions instead of ten.
+// A wave computes a missing fifth (fourth) block all the same and drops it (nc = how many of the last two count).
+struct WinBlocks {
+  int ta, ja, tc, jc, nc;
+};
+__device__ __forceinline__ WinBlocks win_blocks(int wave) {
+  switch (wave) {
+    case 0: return {7, 0, 7, 6, 2};
+    case 1: return {7, 3, 6, 3, 2};
+    case 2: return {6, 0, 6, 5, 2};
+    case 3: return {5, 0, 4, 3, 2};
+    case 4: return {5, 3, 1, 0, 2};
+    case 5: return {4, 0, 3, 3, 1};
+    case 6: return {3, 0, 0, 0, 1};
+    default: return {2, 0, 2, 1, 0};
+  }
+}
+
+}  // namespace mlstm

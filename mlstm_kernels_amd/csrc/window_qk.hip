@@ -13,7 +13,8 @@
 //   * One PERSISTENT workgroup per CU (twelve waves) walks its share of the windows.  Four PRODUCER waves move data
 //     only, in slabs of 32 KB through a FIFO of two register sets into a ring of two LDS slots; eight CONSUMER waves
 //     read operand fragments from LDS, multiply, gate and write the results.  One barrier per slab.
-//   * Three phases per window, all with a static step structure (NV = DHHV / 32):
+//   * Three phases per window, all with a static step structure (NV = DHHV / 32; written for head-dim tiles of 256: with
+//     tiles of 128 and 64 a slab of rows holds 128 and 256 positions, two steps and one instead of four):
 //       S  NV steps  [dH rows x 32 value columns | V rows x 32 value columns]      scores of all 36 blocks, then gating
 //       Q  NV steps  [C fragments of 32 value columns | dH rows x 32 columns]      Out^T += C dH^T  (256 x 256 tile)
 //           4 steps  [64 K rows x 256 head-dim entries]                            Out^T += K^T P^T
@@ -27,68 +28,32 @@
 //     row dots come through the ring like every other operand (fetched by the consumers themselves they cost a
 //     memory latency per handful of positions); the rounded results pass through a private 2 KB staging tile per
 //     wave into row order and are stored as full 128-byte lines.
-// Supported: state stride 2, DHQK = 256, DHHV a multiple of 64.
+// Supported: state stride 2, any head dimensions (multiples of 64; DHQK in tiles of 256, 128 or 64, whichever divides it).
+// Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 357 -> 182, 128/128 264 -> 124,
+// 64/128 250 -> 87, 64/64 with 524288 419 -> 129, 512/1024 with 32768 238 -> 209; 256/512 with 524288 1060 -> 810.
 #include <type_traits>
 
-#include "common.h"
 #include "kernels.h"
+#include "window.h"
 
 namespace mlstm {
 namespace {
-
-struct WqItem {
-  int bh, win;   // (batch * head), window of two chunks
-};
-
-__device__ __forceinline__ bool wq_decode(WqItem& it, int round, int vid, int G, int n_items, int NWIN) {
-  const int rot = (vid + round) % G;
-  const long long idx = (long long)round * G + rot;
-  if (idx >= n_items) return false;
-  it.win = (int)idx % NWIN;
-  it.bh = (int)idx / NWIN;
-  return true;
-}
-
-constexpr float kWqLog2e = 1.4426950408889634f;
-constexpr int kWqSlot = 32768;                    // bytes per ring slot = per slab
-constexpr int kWqPOfs = 2 * kWqSlot;              // P: 36 blocks of 32 x 32 (2 KB each, 64-byte rows, swizzled)
-constexpr int kWqVecOfs = kWqPOfs + 36 * 2048;    // u[256], w[256], lqr[256] (fp32)
+constexpr int kWqVecOfs = kWinPOfs + kWinPBytes;  // u[256], w[256], lqr[256] (fp32)
 constexpr int kWqRedOfs = kWqVecOfs + 3 * 1024;   // [4][256] row-dot partials per 64-row block of the head dimension
 constexpr int kWqStgOfs = kWqRedOfs + 4 * 1024;   // [8 waves][16 rows][64 elements] staging tiles
 constexpr int kWqCsOfs = kWqStgOfs + 8 * 2048;    // [256] column scale of the inter-chunk part of the running phase
 constexpr int kWqSmem = kWqCsOfs + 1024;
 static_assert(kWqSmem <= 160 * 1024, "LDS budget of one CU");
-
-// the blocks (tb, jb) of the lower triangle a consumer wave computes in phase S: up to five, at most two distinct tb
-// (packed: 3 bits tb, 3 bits jb per entry, count in bits 30..32)
-__device__ __forceinline__ uint64_t wq_score_blocks(int wave) {
-#define E5(t0, j0, t1, j1, t2, j2, t3, j3, t4, j4, n)                                                                \
-  ((uint64_t)(t0) | ((uint64_t)(j0) << 3) | ((uint64_t)(t1) << 6) | ((uint64_t)(j1) << 9) | ((uint64_t)(t2) << 12) | \
-   ((uint64_t)(j2) << 15) | ((uint64_t)(t3) << 18) | ((uint64_t)(j3) << 21) | ((uint64_t)(t4) << 24) |               \
-   ((uint64_t)(j4) << 27) | ((uint64_t)(n) << 30))
-  switch (wave) {
-    case 0: return E5(7, 0, 7, 1, 7, 2, 7, 3, 0, 0, 5);
-    case 1: return E5(7, 4, 7, 5, 7, 6, 7, 7, 7, 7, 4);
-    case 2: return E5(6, 0, 6, 1, 6, 2, 6, 3, 6, 3, 4);
-    case 3: return E5(6, 4, 6, 5, 6, 6, 1, 0, 1, 1, 5);
-    case 4: return E5(5, 0, 5, 1, 5, 2, 5, 3, 5, 3, 4);
-    case 5: return E5(5, 4, 5, 5, 2, 0, 2, 1, 2, 2, 5);
-    case 6: return E5(4, 0, 4, 1, 4, 2, 4, 3, 4, 4, 5);
-    default: return E5(3, 0, 3, 1, 3, 2, 3, 3, 3, 3, 4);
-  }
-#undef E5
-}
-
-// 16-byte-unit swizzle of tiles with 64-byte rows (operand rows of 32 value columns, blocks of P): eight consecutive
-// rows read at one unit, and the 4 rows x 2 units patch of a transposing read, both fall on distinct LDS banks
-__device__ __forceinline__ int wq_f64(int row) { return (((row >> 1) & 1) << 1) | ((row >> 2) & 1); }
-
 }  // namespace
 
-template <bool F16>
-__global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items, int n_rounds) {
-  constexpr int DHQK = 256;
-  constexpr int ND = DHQK / 16;
+// DT = head-dim rows of a tile: 256, 128 or 64.  MULTI: the head dimension is several tiles, walked one after the other
+// with the same scores (otherwise it is a compile-time constant).
+template <int DT, bool MULTI, bool F16>
+__global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items, int n_rounds, int n_bh) {
+  constexpr int NDI = DT / 64;           // consumer waves over the head-dim rows of a tile
+  constexpr int NPG = 8 / NDI;           // consumer waves over the positions: blocks NPG * nb + pg of 32 positions
+  constexpr int NNB = NDI;               // position blocks per wave
+  constexpr int ZROWS = 16384 / DT;      // positions per slab of K / Q rows
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float* const uvec = (float*)(smem_raw + kWqVecOfs);  // [256] u_t of the window's positions
   float* const wvec = uvec + 256;                      // [256] w_j
@@ -101,7 +66,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   const int G = gridDim.x;
   int vid = blockIdx.x;
   if (G % 8 == 0) vid = (vid % 8) * (G / 8) + vid / 8;  // consecutive ids share an XCD (and its L2)
-  const int NC = a.NC, S = a.S, DHHV = a.DHHV;
+  const int NC = a.NC, S = a.S, DHHV = a.DHHV, DHQK = MULTI ? a.DHQK : DT;
+  const int ND = DHQK / 16, NDG = DHQK / DT;
   const int NV = DHHV / 32;   // steps of 32 value columns (even)
   const int NWIN = (NC + 1) / 2;  // the last window may hold one chunk only: the other half of it is past the end
   const size_t Sp = (size_t)NC * kChunk;
@@ -124,9 +90,10 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) *(u32x4*)(smem_raw + dB_ + i_ * 4096) = fd##E[4 + i_];          \
   }
     // one step: bA_/gA_/sA_ base, first byte offset and piece distance of pieces 0..3, bB_/gB_/sB_ of pieces 4..7;
+    // nA_ pieces of the first half that carry something (small state slabs; the rest lands where nobody reads);
     // lA_, lB_ largest byte offset of a piece (rows past the end of the sequence re-read its last row: their score
     // factors are zero and their results are not stored), dAu_ / dBu_ destination units of the two halves inside the slot
-#define WQ_PROC(E, bA_, gA_, sA_, lA_, bB_, gB_, sB_, lB_, dAu_, dBu_)                                                         \
+#define WQ_PROC(E, bA_, gA_, sA_, lA_, nA_, bB_, gB_, sB_, lB_, dAu_, dBu_)                                                         \
   {                                                                                                                  \
     if (L >= 3) __syncthreads();                                                                                     \
     /* piece by piece: the old content of a register goes to LDS, then the register is requested anew, so that the */ \
@@ -136,18 +103,18 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     const bool st_ = L >= 2;                                                                                         \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oA_ + i_ * 4096) = fd##E[i_];                                                    \
-      fd##E[i_] = *(const u32x4*)((bA_) + min((gA_) + i_ * (sA_), (lA_)));                                                     \
+      if (i_ < (nA_)) fd##E[i_] = *(const u32x4*)((bA_) + min((gA_) + i_ * (sA_), (lA_)));                                                     \
     }                                                                                                                \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oB_ + i_ * 4096) = fd##E[4 + i_];                                                \
       fd##E[4 + i_] = *(const u32x4*)((bB_) + min((gB_) + i_ * (sB_), (lB_)));                                                 \
     }                                                                                                                \
-    fw##E = ((dAu_) + (E) * (kWqSlot / 16)) | (((dBu_) + (E) * (kWqSlot / 16)) << 16);                               \
+    fw##E = ((dAu_) + (E) * (kWinSlot / 16)) | (((dBu_) + (E) * (kWinSlot / 16)) << 16);                               \
     ++L;                                                                                                             \
   }
-    WqItem it;
+    WinItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!wq_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const uint32_t pl = (uint32_t)opaque(p);
       const char* const dH_b = (const char*)a.dH + (size_t)it.bh * S * DHHV * 2;
       const char* const V_b = (const char*)a.V + (size_t)it.bh * S * DHHV * 2;
@@ -159,57 +126,76 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const uint32_t t0 = (uint32_t)it.win * 256;  // first position of the window
       // operand rows x 32 value columns: piece (row, unit) = (pl / 4 + 64 i, pl % 4), 64 bytes per row and slab
       const uint32_t xrow = pl >> 2, xun = pl & 3;
-      const uint32_t xdu = xrow * 4 + (xun ^ (uint32_t)wq_f64((int)xrow));
+      const uint32_t xdu = xrow * 4 + (xun ^ (uint32_t)win_f64((int)xrow));
       const uint32_t xg = (t0 + xrow) * (uint32_t)(DHHV * 2) + xun * 16;
       const uint32_t xstep = 64 * (uint32_t)DHHV * 2;
       const uint32_t xlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + xun * 16;  // this thread's unit of the last row
-      // state fragments of 32 value columns: 16 KB contiguous in memory; lanes 32..63 of every fragment are stored 4
+      // state fragments of 32 value columns: DT / 16 KB contiguous in memory; lanes 32..63 of every fragment are stored 4
       // slots off so that the two lane halves a transposing read touches together fall on different LDS banks
       const uint32_t cdu = pl ^ (((pl >> 5) & 1) << 2);
-      // 64 rows x 256 head-dim entries: piece (row, unit) = (pl / 32 + 8 i, pl % 32), 512 bytes per row
-      const uint32_t zrow = pl >> 5, zun = pl & 31;
-      const uint32_t zdu = zrow * 32 + (zun ^ (2 * (zrow & 3)));
-      const uint32_t zg = (t0 + zrow) * (DHQK * 2) + zun * 16;
-      const uint32_t zlim = (uint32_t)(S - 1) * (DHQK * 2) + zun * 16;
+      // ZROWS rows x DT head-dim entries: piece (row, unit) = (pl / UPR + 256 / UPR i, pl % UPR)
+      constexpr int UPR = DT / 8;  // 16-byte units per row of a tile
+      const uint32_t zpitch = (uint32_t)DHQK * 2;
+      const uint32_t zrow = pl / UPR, zun = pl % UPR;
+      const uint32_t zdu = zrow * UPR + (zun ^ (2 * (zrow & 3)));
+      const uint32_t zg0 = (t0 + zrow) * zpitch + zun * 16;
+      const uint32_t zlim0 = (uint32_t)(S - 1) * zpitch + zun * 16;
+      const uint32_t zstep = (256 / UPR) * zpitch;
       // (every loop works on its own opaque copy of the offsets: addresses shared between two loops would otherwise be
       // kept, and spilled, across everything in between)
+#define WQ_ROW_SLAB(E, b_, z_)                                                                                       \
+  WQ_PROC(E, b_, zz + (uint32_t)((z_) * ZROWS) * zpitch, zstep, zlim, 4, b_,                                         \
+          zz + (uint32_t)((z_) * ZROWS) * zpitch + 4 * zstep, zstep, zlim, zdu, 1024 + zdu)
+    // the rows of the products (first) and those of the row dots
 #define WQ_ROWS(bA_, bB_)                                                                                            \
   {                                                                                                                  \
-    const uint32_t zz = (uint32_t)opaque((int)zg);                                                                   \
-    for (int z = 0; z < 4; z += 2) {                                                                                 \
-      WQ_PROC(0, bA_, zz + z * 32768, 4096, zlim, bB_, zz + z * 32768 + 16384, 4096, zlim, zdu, 1024 + zdu)                      \
-      WQ_PROC(1, bA_, zz + (z + 1) * 32768, 4096, zlim, bB_, zz + (z + 1) * 32768 + 16384, 4096, zlim, zdu, 1024 + zdu)          \
+    const uint32_t zz = (uint32_t)opaque((int)zg), zlim = (uint32_t)opaque((int)zl);                                 \
+    if constexpr (NDI == 1) {                                                                                        \
+      WQ_ROW_SLAB(0, bA_, 0)                                                                                         \
+      WQ_ROW_SLAB(1, bB_, 0)                                                                                         \
+    } else {                                                                                                         \
+      for (int z = 0; z < NDI; z += 2) {                                                                             \
+        WQ_ROW_SLAB(0, bA_, z)                                                                                       \
+        WQ_ROW_SLAB(1, bA_, z + 1)                                                                                   \
+      }                                                                                                              \
+      for (int z = 0; z < NDI; z += 2) {                                                                             \
+        WQ_ROW_SLAB(0, bB_, z)                                                                                       \
+        WQ_ROW_SLAB(1, bB_, z + 1)                                                                                   \
+      }                                                                                                              \
     }                                                                                                                \
   }
       // ---- phase S: dH rows | V rows
       {
         const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim);
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, dH_b, xx + w * 64, xstep, xl + w * 64, V_b, xx + w * 64, xstep, xl + w * 64, xdu, 1024 + xdu)
-          WQ_PROC(1, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, xdu, 1024 + xdu)
+          WQ_PROC(0, dH_b, xx + w * 64, xstep, xl + w * 64, 4, V_b, xx + w * 64, xstep, xl + w * 64, xdu, 1024 + xdu)
+          WQ_PROC(1, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, 4, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, xdu, 1024 + xdu)
         }
       }
+      for (int dg = 0; dg < NDG; ++dg) {
+      const uint32_t cstep = (uint32_t)ND * 1024;  // fragments of 32 value columns, all head-dim tiles
+      const uint32_t zg = zg0 + dg * (DT * 2), zl = zlim0 + dg * (DT * 2);
       // ---- phase Q: C fragments | dH rows, then the K rows (products) and the Q rows (row dots)
       {
-        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16));
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16 + dg * (DT / 16) * 1024));
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, C_b, (uint32_t)w * 16384 + cc, 4096, 0xffffffffu, dH_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
-          WQ_PROC(1, C_b, (uint32_t)(w + 1) * 16384 + cc, 4096, 0xffffffffu, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
+          WQ_PROC(0, C_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
+          WQ_PROC(1, C_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
       }
-      WQ_ROWS(K_b, K_b)
-      WQ_ROWS(Q_b, Q_b)
+      WQ_ROWS(K_b, Q_b)
       // ---- phase K: dC fragments | V rows, then the Q rows (products) and the K rows (row dots)
       {
-        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16));
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16 + dg * (DT / 16) * 1024));
         for (int w = 0; w < NV; w += 2) {
-          WQ_PROC(0, dC_b, (uint32_t)w * 16384 + cc, 4096, 0xffffffffu, V_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
-          WQ_PROC(1, dC_b, (uint32_t)(w + 1) * 16384 + cc, 4096, 0xffffffffu, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
+          WQ_PROC(0, dC_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
+          WQ_PROC(1, dC_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
       }
-      WQ_ROWS(Q_b, Q_b)
-      WQ_ROWS(K_b, K_b)
+      WQ_ROWS(Q_b, K_b)
+      }
 #undef WQ_ROWS
+#undef WQ_ROW_SLAB
     }
     // ---- drain: the last two slabs go to LDS, then the barriers of the consumers' last steps and of the final row dots
     if (L > 0) {
@@ -226,32 +212,35 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     // =========================================================================================== consumer waves
     const int wave = wave_all;
     const int tid = wave * 64 + lane;
-    const int di = wave & 3, par = wave >> 2;  // head-dim rows 64 di .., position blocks 2 nb + par (nb = 0 .. 3)
+    const int di = wave % NDI, pg = wave / NDI;  // head-dim rows 64 di .. of a tile, position blocks NPG * nb + pg
     unsigned char* const stg = smem_raw + kWqStgOfs + wave * 2048;
-    const uint64_t sblk = wq_score_blocks(wave);
-    const int n_sblk = (int)((sblk >> 30) & 7);
-    f32x16 acc[2][4];
-    WqItem it, prev;
-    prev = WqItem{0, 0};
+    const WinBlocks blk = win_blocks(wave);
+    f32x16 acc[2][NNB];
+    WinItem it, prev;
+    prev = WinItem{0, 0};
     int pending = 0;       // row dots waiting in `red`: 1 dQ of `prev`, 2 dK of `prev`
+    int prev_dg = 0;       // ... of this head-dim tile
     uint32_t slot = 0;     // ring slot of the next slab
     auto next_slab = [&]() {
-      const unsigned char* s = smem_raw + slot * kWqSlot;
+      const unsigned char* s = smem_raw + slot * kWinSlot;
       slot ^= 1;
       return s;
     };
     // row dots of the last finished phase: the four 64-row blocks' partials meet in LDS, 256 threads add them up
     auto finish_rowdots = [&]() {
       if (pending && tid < 256) {
-        const float dot = (red[tid] + red[256 + tid]) + (red[512 + tid] + red[768 + tid]);
+        float dot = red[tid];
+        if constexpr (NDI == 2) dot += red[256 + tid];
+        if constexpr (NDI == 4) dot = (dot + red[256 + tid]) + (red[512 + tid] + red[768 + tid]);
+        // one slot per head-dim tile: [tile][batch * head][position]
         if (prev.win * 256 + tid < S)
-          (pending == 2 ? a.rowdot2 : a.rowdot)[(size_t)prev.bh * Sp + (size_t)prev.win * 256 + tid] = dot;
+          (pending == 2 ? a.rowdot2 : a.rowdot)[((size_t)prev_dg * n_bh + prev.bh) * Sp + (size_t)prev.win * 256 + tid] = dot;
       }
       pending = 0;
     };
 
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!wq_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const size_t hofs = (size_t)bh * Sp, gofs = hofs + (size_t)c0 * kChunk;
       const float* graw = a.g.graw + (size_t)bh * NC;
@@ -291,16 +280,18 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           }
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
+          const int ra = 32 * blk.ta + r, rc = 32 * blk.tc + r;
 #pragma unroll
           for (int ks = 0; ks < 2; ++ks) {
+            Frag Ba, Bc;
+            Ba.u = *(const uint4*)(slab + ra * 64 + (((2 * ks + h) ^ win_f64(ra)) * 16));
+            Bc.u = *(const uint4*)(slab + rc * 64 + (((2 * ks + h) ^ win_f64(rc)) * 16));
 #pragma unroll
             for (int e = 0; e < 5; ++e) {
-              const int tb = (int)((sblk >> (6 * e)) & 7), jb = (int)((sblk >> (6 * e + 3)) & 7);
-              const int trow = 32 * tb + r, jrow = 32 * jb + r;
-              Frag A, B;
-              B.u = *(const uint4*)(slab + trow * 64 + (((2 * ks + h) ^ wq_f64(trow)) * 16));
-              A.u = *(const uint4*)(slab + 16384 + jrow * 64 + (((2 * ks + h) ^ wq_f64(jrow)) * 16));
-              mfma32<F16>(sacc[e], A, B);   // rows: keys j, columns: positions t
+              const int jrow = 32 * (e < 3 ? blk.ja + e : blk.jc + e - 3) + r;
+              Frag A;
+              A.u = *(const uint4*)(slab + 16384 + jrow * 64 + (((2 * ks + h) ^ win_f64(jrow)) * 16));
+              mfma32<F16>(sacc[e], A, e < 3 ? Ba : Bc);   // rows: keys j, columns: positions t
             }
           }
         }
@@ -311,13 +302,13 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           const int r = le & 31, h = le >> 5;
 #pragma unroll
           for (int e = 0; e < 5; ++e) {
-            if (e < n_sblk) {
-              const int tb = (int)((sblk >> (6 * e)) & 7), jb = (int)((sblk >> (6 * e + 3)) & 7);
+            if (e < 3 + blk.nc) {
+              const int tb = e < 3 ? blk.ta : blk.tc, jb = e < 3 ? blk.ja + e : blk.jc + e - 3;
               const float gg = (tb >= 4 && jb < 4) ? g01 : 0.f;
               const float un = uvec[32 * tb + r] + gg;
               const float lq = lqr[32 * tb + r];
-              unsigned char* const pb = smem_raw + kWqPOfs + (tb * (tb + 1) / 2 + jb) * 2048 + r * 64;
-              const int fr = wq_f64(r);
+              unsigned char* const pb = smem_raw + kWinPOfs + (tb * (tb + 1) / 2 + jb) * 2048 + r * 64;
+              const int fr = win_f64(r);
 #pragma unroll
               for (int g4 = 0; g4 < 4; ++g4) {
                 const int j0 = 8 * g4 + 4 * h;
@@ -326,7 +317,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 float pv[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                  const float e2 = __builtin_amdgcn_exp2f(__builtin_fmaf(un - wv[q], kWqLog2e, lq));
+                  const float e2 = __builtin_amdgcn_exp2f(__builtin_fmaf(un - wv[q], kWinLog2e, lq));
                   const bool keep = tb != jb || j0 + q <= r;
                   pv[q] = keep ? sacc[e][4 * g4 + q] * e2 : 0.f;
                 }
@@ -338,7 +329,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       }
 
       // ============================================================================ phases Q (dQ) and K (dK)
-      auto run_phase = [&](auto DKT) {
+      auto run_phase = [&](auto DKT, int dg) {
         constexpr bool dk = decltype(DKT)::value;
         // column scale of the inter-chunk part: requested now by one thread per position, parked in LDS after the first
         // step of the value pass, used after its last one (registers are what this kernel is short of)
@@ -358,7 +349,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int nb = 0; nb < 4; ++nb)
+          for (int nb = 0; nb < NNB; ++nb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
 
@@ -380,11 +371,11 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           const int h_src = d_grp & 1, a_src = d_grp >> 1;
 #pragma unroll
           for (int ks = 0; ks < 2; ++ks) {
-            Frag A[2], B[4];
+            Frag A[2], B[NNB];
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-              const int row = 32 * (2 * nb + par) + r;
-              B[nb].u = *(const uint4*)(Xn + row * 64 + (((2 * ks + h) ^ wq_f64(row)) * 16));
+            for (int nb = 0; nb < NNB; ++nb) {
+              const int row = 32 * (NPG * nb + pg) + r;
+              B[nb].u = *(const uint4*)(Xn + row * 64 + (((2 * ks + h) ^ win_f64(row)) * 16));
             }
             const int wrow = 16 * ks + 8 * h + (i16 >> 2);  // value column inside the 32-column slab (first read)
 #pragma unroll
@@ -400,22 +391,22 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-              for (int nb = 0; nb < 4; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
+              for (int nb = 0; nb < NNB; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
           }
         }
         // column scale of the inter-chunk part (kept apart from the matrix instructions around it)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-          const float cs = csv[32 * (2 * nb + par) + (opaque(lane) & 31)];
+        for (int nb = 0; nb < NNB; ++nb) {
+          const float cs = csv[32 * (NPG * nb + pg) + (opaque(lane) & 31)];
 #pragma unroll
           for (int mb = 0; mb < 2; ++mb) acc[mb][nb] *= cs;
         }
         __builtin_amdgcn_sched_barrier(0);
 
-        // ---- Out^T += Z^T P'^T over the 256 positions of the window, 64 rows of Z per slab (Z = K for dQ with
+        // ---- Out^T += Z^T P'^T over the 256 positions of the window, ZROWS rows of Z per slab (Z = K for dQ with
         // P' = P: contraction over the keys j; Z = Q for dK with P' = P^T: contraction over the positions t)
-        for (int z = 0; z < 4; ++z) {
+        for (int z = 0; z < NDI; ++z) {
           __syncthreads();
           const unsigned char* const Zs = next_slab();
           const int le = opaque(lane);
@@ -424,8 +415,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           const int krow = 8 * h + (i16 >> 2);
           const int zun = 2 * q16 + ((i16 & 3) >> 1), zin = 8 * (i16 & 1);   // 16-byte unit and byte inside it
 #pragma unroll
-          for (int zh = 0; zh < 2; ++zh) {
-            const int ob = 2 * z + zh;  // 32-position block of the contraction index
+          for (int zh = 0; zh < ZROWS / 32; ++zh) {
+            const int ob = z * (ZROWS / 32) + zh;  // 32-position block of the contraction index
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
               Frag A[2];
@@ -435,11 +426,11 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 for (int half = 0; half < 2; ++half) {
                   const int row = 32 * zh + 16 * kk + krow + 4 * half;
                   const int un = 8 * di + 4 * mb + zun;
-                  A[mb].d[half] = lds_read_tr16(Zs + row * 512 + ((un ^ (2 * (row & 3))) * 16) + zin);
+                  A[mb].d[half] = lds_read_tr16(Zs + row * (DT * 2) + ((un ^ (2 * (row & 3))) * 16) + zin);
                 }
 #pragma unroll
-              for (int nb = 0; nb < 4; ++nb) {
-                const int nbk = 2 * nb + par;   // the wave's position block (dQ: t, dK: j)
+              for (int nb = 0; nb < NNB; ++nb) {
+                const int nbk = NPG * nb + pg;   // the wave's position block (dQ: t, dK: j)
                 const bool live = dk ? ob >= nbk : ob <= nbk;
                 // (the matrix instructions stay unconditional: accumulators that pass through a branch get copied;
                 // a block above the diagonal contributes an operand of zeros instead)
@@ -448,15 +439,15 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 if (live) {
                   if (dk) {
                     // P^T: rows t of block (ob, nbk) are the contraction index -> transposing read
-                    const unsigned char* const pb = smem_raw + kWqPOfs + (ob * (ob + 1) / 2 + nbk) * 2048;
+                    const unsigned char* const pb = smem_raw + kWinPOfs + (ob * (ob + 1) / 2 + nbk) * 2048;
 #pragma unroll
                     for (int half = 0; half < 2; ++half) {
                       const int row = 16 * kk + krow + 4 * half;
-                      B.d[half] = lds_read_tr16(pb + row * 64 + ((zun ^ wq_f64(row)) * 16) + zin);
+                      B.d[half] = lds_read_tr16(pb + row * 64 + ((zun ^ win_f64(row)) * 16) + zin);
                     }
                   } else {
-                    const unsigned char* const pb = smem_raw + kWqPOfs + (nbk * (nbk + 1) / 2 + ob) * 2048;
-                    B.u = *(const uint4*)(pb + r * 64 + (((2 * kk + h) ^ wq_f64(r)) * 16));
+                    const unsigned char* const pb = smem_raw + kWinPOfs + (nbk * (nbk + 1) / 2 + ob) * 2048;
+                    B.u = *(const uint4*)(pb + r * 64 + (((2 * kk + h) ^ win_f64(r)) * 16));
                   }
                 }
 #pragma unroll
@@ -466,21 +457,21 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           }
         }
 
-        // ---- results, 64 positions per step: the x rows (q for dQ, k for dK) of those positions arrive as one more
+        // ---- results, ZROWS positions per step: the x rows (q for dQ, k for dK) of those positions arrive as one more
         // slab; every wave owns one 32-position block of them.  Row dots sum_d x Out from the fp32 accumulators (they
         // feed a suffix sum over the whole sequence, where the rounding noise of 16-bit outputs would add up); then
         // the rounded values pass, 16 positions at a time, through the wave's private staging tile into row order and
         // leave as full 128-byte lines.
-        char* const Ob = (char*)(dk ? a.Out2 : a.Out) + ((size_t)bh * S + (size_t)c0 * kChunk) * (DHQK * 2);
+        char* const Ob = (char*)(dk ? a.Out2 : a.Out) + ((size_t)bh * S + (size_t)c0 * kChunk) * (DHQK * 2) + dg * (DT * 2);
 #pragma unroll
-        for (int z = 0; z < 4; ++z) {
+        for (int z = 0; z < NDI; ++z) {
           __syncthreads();
           const unsigned char* const Xs = next_slab();
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
           {
-            const int row = 32 * par + r;
-            const unsigned char* const xrow = Xs + row * 512 + 8 * h;
+            const int row = 32 * pg + r;
+            const unsigned char* const xrow = Xs + row * (DT * 2) + 8 * h;
             const int sw = 2 * (row & 3);
             float part = 0.f;
 #pragma unroll
@@ -494,9 +485,9 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 part += acc[mb][z][4 * g4 + 3] * hi2<F16>(xv.y);
               }
             part += __shfl_xor(part, 32);
-            if (h == 0) red[di * 256 + 64 * z + row] = part;
+            if (h == 0) red[di * 256 + ZROWS * z + row] = part;
           }
-          const uint32_t lofs = (uint32_t)((le >> 3) * (DHQK * 2) + 128 * di + 16 * (le & 7));
+          const uint32_t lofs = (uint32_t)(le >> 3) * (uint32_t)(DHQK * 2) + (uint32_t)(128 * di + 16 * (le & 7));
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
             if ((r >> 4) == q) {
@@ -514,15 +505,18 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
             const u32x4 o0 = *(const u32x4*)(stg + row8 * 128 + ((un ^ row8) * 16));
             const u32x4 o1 = *(const u32x4*)(stg + (row8 + 8) * 128 + ((un ^ row8) * 16));
             __builtin_amdgcn_wave_barrier();
-            const uint32_t n0 = (uint32_t)(64 * z + 32 * par + 16 * q);
-            if ((int)n0 + row8 < n_pos) __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (DHQK * 2))));
-            if ((int)n0 + 8 + row8 < n_pos) __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (DHQK * 2))));
+            const uint32_t n0 = (uint32_t)(ZROWS * z + 32 * pg + 16 * q);
+            if ((int)n0 + row8 < n_pos) __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (uint32_t)(DHQK * 2))));
+            if ((int)n0 + 8 + row8 < n_pos) __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (uint32_t)(DHQK * 2))));
           }
         }
         pending = dk ? 2 : 1;
+        prev_dg = dg;
       };
-      run_phase(std::false_type{});
-      run_phase(std::true_type{});
+      for (int dg = 0; dg < NDG; ++dg) {
+        run_phase(std::false_type{}, dg);
+        run_phase(std::true_type{}, dg);
+      }
     }
     if (pending) {   // (a workgroup without a window passes no barrier at all, like its producers)
       __syncthreads();
@@ -532,11 +526,11 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 }
 
 bool window_qk_supported(const ParQkArgs& a) {
-  return a.stride == 2 && a.DHQK == 256 && a.DHHV % 64 == 0;
+  return a.stride == 2 && a.DHQK % 64 == 0 && a.DHHV % 64 == 0;
 }
 
 namespace {
-template <bool F16>
+template <int DT, bool MULTI, bool F16>
 const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   const long long n_items = (long long)BH * ((a.NC + 1) / 2);
   if (n_items >= (1ll << 31)) return "window_qk: too many work items";
@@ -548,17 +542,37 @@ const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
-  if (!lds.allow((const void*)window_qk_kernel<F16>, kWqSmem))
+  if (!lds.allow((const void*)window_qk_kernel<DT, MULTI, F16>, kWqSmem))
     return "window_qk: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((window_qk_kernel<F16>), dim3(G), dim3(768), kWqSmem, stream, a, (int)n_items, n_rounds);
+  hipLaunchKernelGGL((window_qk_kernel<DT, MULTI, F16>), dim3(G), dim3(768), kWqSmem, stream, a, (int)n_items, n_rounds, BH);
   return nullptr;
+}
+template <int DT, bool MULTI>
+const char* launch_window_qk_d(const ParQkArgs& a, int BH, hipStream_t stream) {
+  return a.f16 ? launch_window_qk_t<DT, MULTI, true>(a, BH, stream) : launch_window_qk_t<DT, MULTI, false>(a, BH, stream);
 }
 }  // namespace
 
+// Where the window kernel is the faster one: a window is one workgroup's 26 to 64 steps, so with few windows the tiled
+// kernel's eight or more workgroups per window finish first.  They meet at half a window per CU with tiles of 256 rows
+// (256/512, us, window / tiled: 65 / 39 at 64 windows, 67 / 69 at 128, 100 / 133 at 256), at three eighths with 128
+// (128/256: 34 / 29 at 64, 35 / 50 at 128), and with 64 the window kernel wins from one window on (17 / 25).
+bool window_qk_preferred(const ParQkArgs& a, int BH) {
+  if (!window_qk_supported(a)) return false;
+  const long long windows = (long long)BH * ((a.NC + 1) / 2), cus = device_cu_count();
+  const int DT = par_qk_head_tile(a.DHQK);
+  return DT == 64 || (DT == 128 ? 8 * windows >= 3 * cus : 2 * windows >= cus);
+}
+
 const char* launch_window_qk(const ParQkArgs& a, int BH, hipStream_t stream) {
-  if (!window_qk_supported(a)) return "window_qk: unsupported shape (needs state stride 2, DHQK = 256, DHHV % 64 == 0)";
+  if (!window_qk_supported(a)) return "window_qk: unsupported shape (needs state stride 2, head dimensions that are multiples of 64)";
   if (a.states2 == nullptr || a.Out2 == nullptr || a.rowdot2 == nullptr) return "window_qk: the dK operands are missing";
-  return a.f16 ? launch_window_qk_t<true>(a, BH, stream) : launch_window_qk_t<false>(a, BH, stream);
+  // (the tile decides the layout of the row-dot slots, as for the tiled kernel)
+  const int DT = par_qk_head_tile(a.DHQK);
+  const bool multi = a.DHQK > DT;
+  if (DT == 256) return multi ? launch_window_qk_d<256, true>(a, BH, stream) : launch_window_qk_d<256, false>(a, BH, stream);
+  if (DT == 128) return multi ? launch_window_qk_d<128, true>(a, BH, stream) : launch_window_qk_d<128, false>(a, BH, stream);
+  return multi ? launch_window_qk_d<64, true>(a, BH, stream) : launch_window_qk_d<64, false>(a, BH, stream);
 }
 
 }  // namespace mlstm

@@ -39,7 +39,7 @@ def _run(S, DQ, DV, *, B=1, NH=2, sig=False, norm="none", init=False, seed=0, dt
         H_ref = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6)
         (dH_ref,) = torch.autograd.grad(H_ref, raw, d(dH))
     bw = O.chunkwise_bw(d(q), d(k), d(v), d(i), d(f), dH_ref, d(st[0]), d(st[1]), m0, None, chunk_size=L, siging=sig)
-    tol = 2.0 if norm != "none" else 1.0   # the norm divides by the spread of a row, which may be small
+    tol = 4.0 if norm != "none" else 1.0   # the norm removes the scale of a row: what is left of dQ and dK cancels in part
     assert rel_norm(H, H_ref) <= 6e-3 * tol
     # (the norm of the only row of a sequence removes its scale, which is all q and k change: their gradients vanish)
     grads = list(zip(("dQ", "dK", "dV"), leaves, bw[:3]))[2 if norm != "none" and S == 1 else 0:]
@@ -57,6 +57,17 @@ def _run(S, DQ, DV, *, B=1, NH=2, sig=False, norm="none", init=False, seed=0, dt
                          ids=["exp", "sig-init", "norm", "fp16-init"])
 def test_ragged_lengths(S, opt):
     _run(S, 256, 512, seed=S, **opt)
+
+
+@pytest.mark.parametrize("DQ,DV", [(64, 64), (64, 128), (128, 128), (128, 256), (256, 256), (512, 1024), (192, 320), (256, 192),
+                                   (128, 384), (64, 512), (512, 64)])
+@pytest.mark.parametrize("S", [40, 256, 390])
+@pytest.mark.parametrize("opt", [dict(), dict(sig=True, init=True), dict(norm="rms"), dict(dtype=torch.float16)],
+                         ids=["exp", "sig-init", "norm", "fp16"])
+def test_head_dimensions(DQ, DV, S, opt):
+    if "norm" in opt and DV not in (64, 128, 256, 512):
+        pytest.skip("the fused head norm needs DHHV = 64, 128, 256 or 512")
+    _run(S, DQ, DV, seed=S + DQ + DV, **opt)
 
 
 @pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
