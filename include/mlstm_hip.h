@@ -152,6 +152,7 @@ size_t mlstm_hip_chunkwise_fw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   c0,n0,m0: initial states or NULL (all three NULL together; m0 ignored for the sig gate).
  *   H (B,NH,S,DHHV) in dtype_qkv.  n_out, m_out: optional fp32 (B,NH,S) per-row normaliser max(|den|,floor)
  *   and stabiliser (NULL to skip).  c_last,n_last,m_last: optional fp32 last states (NULL to skip).
+ *   H serves the state scan as scratch before it is written (dV likewise in the backward).
  *   With c_last given, the state scan carries the gated values as a 16-bit head plus a 16-bit remainder in every
  *   chunk that still weighs at least 2^-8 in the last state, so c_last is accurate to ~1e-5 relative; with c_last
  *   NULL it rounds them once (as the replaced kernels do), which is up to a fifth faster and changes H only within
@@ -177,7 +178,8 @@ int mlstm_hip_chunkwise_fw(const void* q, const void* k, const void* v, const vo
  * of a full-size workspace and calls mlstm_hip_chunkwise_recompute_states, which runs the forward state scan again
  * and writes the chunk states behind them (k, v, c0, dtype_qkv, state_stride as in the forward call; c0 NULL = zero
  * initial state).  The workspace is then what mlstm_hip_chunkwise_bw expects.  The recomputed states equal the
- * forward's bit for bit when the forward returned no last state (c_last NULL); a forward that returned it carried a
+ * forward's bit for bit when the forward returned no last state (c_last NULL) and its scan ran in one piece (it is cut into
+ * segments where few heads meet a long sequence; the fp32 states before the rounding then differ in the order of a sum); a forward that returned it carried a
  * remainder of the value operand in its late chunks, and the recomputed states of those chunks differ from the
  * forward's by one 16-bit rounding of that operand.
  */

@@ -299,6 +299,8 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   // scale in every chunk: true for the exponential gate (its stabiliser rescales them), not for the sigmoid gate,
   // whose late positions may all be closed while early chunks dominate the state.
   sa.all_remainder = sig;
+  sa.seg = (float*)H;  // H is written after the scan
+  sa.seg_bytes = (size_t)BH * S * DHHV * 2;
   {
     ProfileScope ps("scan_fw", st);
     // The head + remainder split of the value operand only serves the fp32 last state (1e-5 instead of 1.5e-3
@@ -470,6 +472,8 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     sa.S = S; sa.NC = NC; sa.DHQK = DHQK; sa.DHHV = DHHV;
     sa.qk_scale = qk_scale; sa.eps = eps;
     sa.backward = 1;
+    sa.seg = (float*)dV;  // dV is written after the scan
+    sa.seg_bytes = (size_t)BH * S * DHHV * 2;
     sa.stride = stride;
     sa.f16 = f16;
     {

@@ -63,8 +63,13 @@ struct ScanArgs {
   int all_remainder;      // forward, last state returned: every chunk carries the remainder of the value operand (the
                           // sigmoid input gate has no stabiliser, so the decay factors alone do not say which chunks
                           // still weigh in the last state)
-  int part;               // set by the launcher: 0 whole sequence; 1 / 2 the two launches of a forward scan that
-                          // returns the last state (before / from the first chunk that carries the remainder)
+  float* seg;             // scratch for the states between segments, of seg_bytes (an output that is written later), or nullptr
+  size_t seg_bytes;
+  // set by the launcher:
+  int part;               // 0 whole sequence; 1 / 2 the two launches of a forward scan that returns the last state
+  int n_bh;               // batch * heads
+  int nseg, seg_len;      // segments of the sequence, chunks in each (the last one may be shorter)
+  int seg_phase;          // 0 one piece; 1 every segment but the last from zero, 2 all segments from their states
 };
 
 struct ParHvArgs {

@@ -16,10 +16,15 @@
 // state keeps ~16 mantissa bits: a single bf16 rounding of abar*V leaves a relative error of about 1.5e-3
 // in C, above the 1e-3 the state is specified to.
 //
-// Two kernels: scan_roles_kernel (below, second) without the remainder -- the training forward, every backward scan,
-// and of a forward that returns the fp32 last state the chunks whose rounding no longer shows in it -- and scan_kernel
-// with the head + remainder split for the rest of such a forward (two launches; the state passes from one to the
-// other in the caller's last-state buffers).  Same tiling, same arithmetic, same results.
+// Two kernels: scan_roles_kernel (below, second) -- every scan -- and scan_kernel with the head + remainder split for
+// forwards that return the last state and in which many chunks still weigh in it (it continues where the first one
+// stopped; the state passes through the caller's last-state buffers).  Where only a few do, scan_roles_kernel runs those
+// chunks twice, once with the heads and once with the remainders.  Same tiling, same arithmetic, same results.
+//
+// A scan of few (batch, head) pairs has too few state tiles to fill the chip and walks the sequence chunk by chunk at
+// 1.9 us, whatever the memory could deliver.  It is cut into segments of the sequence that run side by side: a first
+// launch accumulates every segment but the last from zero, a second one runs all segments from the state before them,
+// which is the decayed sum of the first launch's results (the decay factors depend on the gates only).
 //
 // Workgroups are renumbered so that all tiles of one (batch, head) run on the same XCD (the hardware deals
 // consecutive workgroup ids round-robin to the 8 XCDs): the K/V rows every tile of a head re-reads then hit
@@ -68,6 +73,13 @@ __device__ __forceinline__ int first_remainder_chunk(const float* gbar_bh, int N
   }
   return __builtin_amdgcn_readfirstlane(NC - cnt);
 }
+
+// Whether the chunks that carry the remainder run twice in scan_roles_kernel (once with the 16-bit heads, once with the
+// remainders) or go to scan_kernel in a launch of its own.  A second run costs a chunk's time again (2.3 us at B = 4,
+// S = 16384, against 3.6 us for both operands at once in scan_kernel), the launch and its tail a fixed 12 us per round
+// of workgroups: worth it while the late chunks are at most a quarter of all, and for sequences of four chunks at most.
+constexpr int kScanShort = 4;
+__device__ __forceinline__ bool scan_repeats_late(int NC, int c_lo) { return NC <= kScanShort || 4 * (NC - c_lo) <= NC; }
 
 #define SCAN_WPE(HILO_, WCOLS_) ((WCOLS_) == 64 && (HILO_) ? 1 : 2)
 // WCOLS = value columns per wave (64 or 32): with 32 a 128 x 128 tile takes eight waves, two per SIMD, each with
@@ -119,6 +131,12 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
   const int d_wave = d_tile + wr * 64, w_wave = w_tile + wc * WCOLS;
   const int DHQK = a.DHQK, DHHV = a.DHHV, S = a.S, NC = a.NC;
   const size_t Sp = (size_t)NC * kChunk;
+  // c_lo = first chunk that carries the remainder of the value operand
+  int c_lo = 0;
+  if constexpr (HILO) {
+    if (!a.backward) c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
+    if (a.part == 2 && scan_repeats_late(NC, c_lo)) return;  // the first launch ran everything
+  }
 
   f32x16 acc[2][NBW];
 #pragma unroll
@@ -182,11 +200,6 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
   };
 
   const int c_first_all = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
-  // c_lo = first chunk that carries the remainder of the value operand
-  int c_lo = 0;
-  if constexpr (HILO) {
-    if (!a.backward) c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
-  }
   // part 2 of a forward scan in two launches: the chunks from c_lo on, continuing from the state the first launch left
   // in final_out / n_final (loaded above)
   const int c_first = a.part == 2 ? c_lo : c_first_all;
@@ -434,25 +447,56 @@ __device__ __forceinline__ Frag scan_tr_frag(const uint16_t* tile, int k0, const
 }
 }  // namespace
 
+// What a workgroup of scan_roles_kernel runs: chunks it_lo .. it_hi - 1 in scan order (forward: the chunk index, backward
+// counted from the end), those from it_rep on twice in a row (heads, then remainders of the value rows).  Everything
+// below is counted in runs p = 0 .. total - 1.
+struct ScanRuns {
+  int it_lo, it_hi, it_rep, total;
+  __device__ __forceinline__ ScanRuns(int lo, int hi, int rep) : it_lo(lo), it_hi(hi), it_rep(max(rep, lo)) {
+    total = max(hi - lo, 0) + max(hi - it_rep, 0);
+  }
+  __device__ __forceinline__ int it(int p) const {  // scan index of run p
+    const int q = p - (it_rep - it_lo);
+    return q < 0 ? it_lo + p : it_rep + (q >> 1);
+  }
+  __device__ __forceinline__ bool rest(int p) const {  // whether run p is the second run of its chunk
+    const int q = p - (it_rep - it_lo);
+    return q >= 0 && (q & 1);
+  }
+  __device__ __forceinline__ bool last(int p) const {  // whether run p is the last one of its chunk
+    const int q = p - (it_rep - it_lo);
+    return q < 0 || (q & 1);
+  }
+  // the decay table in LDS holds kGBlock chunks: refilled before the first run of every kGBlock-th chunk of the workgroup
+  __device__ __forceinline__ bool refill(int p) const { return p > 0 && !rest(p) && ((it(p) - it_lo) & (kGBlock - 1)) == 0; }
+};
+
+// Segment states between the two launches of a segmented scan, in the register order of the consumer waves:
+// [(batch * head * (segments - 1) + segment)][tile][consumer wave][8][64 lanes][4], behind them n [..][DHQK].
+struct ScanSeg {
+  float* c;
+  float* n;
+};
+__device__ __forceinline__ ScanSeg scan_seg(const ScanArgs& a, int bh, int seg) {
+  const size_t per_c = (size_t)a.DHQK * a.DHHV, count = (size_t)a.n_bh * (a.nseg - 1), idx = (size_t)bh * (a.nseg - 1) + seg;
+  return {a.seg + idx * per_c, a.seg + count * per_c + idx * a.DHQK};
+}
+
 // The consumer role of the scan kernel (see there).  NDB = 0 or 1: this wave also carries the normaliser vector of the
 // first or second 32 of its 64 state rows, NDB = -1: it does not (copies of the role rather than a branch around matrix
 // instructions, which would make the compiler keep those accumulators in scratch memory).
 template <int RT, int WT, bool F16, int NDB>
 __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t* bufs, const float* gl, const uint16_t* nB,
-                                              int wave, int lane, int bh, int d_tile, int w_tile, int n_run) {
-  constexpr int c_lo = 0;  // (no remainder operand in this kernel)
-  constexpr bool HILO = false;
+                                              int wave, int lane, int bh, int seg, int tile, int d_tile, int w_tile,
+                                              const ScanRuns runs, bool is_end) {
   constexpr int WC = WT / 32;
-  constexpr int PS = HILO ? 64 : 128;
-  constexpr int NP = kChunk / PS;
-  constexpr int XELEMS = PS * RT, YELEMS = PS * WT;
-  constexpr int BUF = XELEMS + YELEMS * (HILO ? 2 : 1);
+  constexpr int NWC = (RT / 64) * WC;
+  constexpr int XELEMS = kChunk * RT, YELEMS = kChunk * WT;
+  constexpr int BUF = XELEMS + YELEMS;
   const int DHQK = a.DHQK, DHHV = a.DHHV, NC = a.NC;
-  const int total = n_run * NP;  // n_run: chunks this launch runs
-  const int c_first = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
+  const int total = runs.total;
   constexpr bool WITH_N = NDB >= 0;
   constexpr int DB = WITH_N ? NDB : 0;
-  auto refill_due = [&](int p) { return p % NP == 0 && p / NP > 0 && ((p / NP) & (kGBlock - 1)) == 0; };
   const int wr = wave / WC, wc = wave % WC;
   const int r = lane & 31, h = lane >> 5;
   const int d_wave = d_tile + wr * 64, w_wave = w_tile + wc * 32;
@@ -462,7 +506,7 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float v0 = 0.f;
-      if (a.init != nullptr) {
+      if (a.init != nullptr && a.seg_phase != 1) {
         const int d = d_wave + 32 * db + 8 * (i / 4) + 4 * h + (i % 4);
         v0 = a.init[((size_t)bh * DHQK + d) * DHHV + w_wave + r];
       }
@@ -474,23 +518,54 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     float v0 = 0.f;
-    if (WITH_N && a.n_init != nullptr && r == 0) v0 = a.n_init[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)];
+    if (WITH_N && a.n_init != nullptr && a.seg_phase != 1 && r == 0)
+      v0 = a.n_init[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)];
     accn[i] = v0;
+  }
+  const size_t seg_ofs = ((size_t)tile * NWC + wave) * 2048 + lane * 4;
+  if (a.seg_phase == 2) {
+    // the state before this segment: the segments in front of it, each decayed over what lies between
+    for (int x = 0; x < seg; ++x) {
+      float dec = 1.f;
+      for (int k = lane; k < a.seg_len; k += kWave) {
+        const int itx = x * a.seg_len + k;
+        dec *= a.gbar[(size_t)bh * NC + (a.backward ? NC - 1 - itx : itx)];
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) dec *= __shfl_xor(dec, o);
+      const ScanSeg ss = scan_seg(a, bh, x);
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 v = *(const f32x4*)(ss.c + seg_ofs + (db * 4 + g4) * 256);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[db][4 * g4 + e] = acc[db][4 * g4 + e] * dec + v[e];
+        }
+      if (WITH_N) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float v = r == 0 ? ss.n[d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)] : 0.f;
+          accn[i] = accn[i] * dec + v;
+        }
+      }
+    }
   }
   const ScanTrOff offA0 = scan_tr_offsets<RT>(wr * 64, lane);
   const ScanTrOff offA1 = scan_tr_offsets<RT>(wr * 64 + 32, lane);
   const ScanTrOff offB = scan_tr_offsets<WT>(wc * 32, lane);
   __syncthreads();  // the producers' prologue barrier
   for (int p = 0; p < total; ++p) {
-    const int it = p / NP, piece = p % NP;
-    const int c = c_first + it * c_step;
-    if (refill_due(p)) __syncthreads();
-    __syncthreads();  // piece p staged by the producers
-    if (piece == 0) {
+    const int it = runs.it(p);
+    const bool rest = runs.rest(p);
+    const int c = a.backward ? NC - 1 - it : it;
+    if (runs.refill(p)) __syncthreads();
+    __syncthreads();  // run p staged by the producers
+    if (!rest) {
       // ---- the state before this chunk's update as operand fragments, at the kept boundaries only: forward the
       // state before every stride-th chunk, backward the gradient of the state after the last chunk of every group
       // of `stride` chunks (and after the last chunk of the sequence); slot c / stride either way
-      const bool keep = a.backward ? (c == NC - 1 || (c + 1) % a.stride == 0) : (c % a.stride == 0);
+      const bool keep = a.seg_phase != 1 && (a.backward ? (c == NC - 1 || (c + 1) % a.stride == 0) : (c % a.stride == 0));
       if (keep) {
         const size_t ND = DHQK / 16, NWB = DHHV / 32;
         const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
@@ -509,12 +584,12 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
           }
         }
       }
-      const float g = gl[it & (kGBlock - 1)];
+      const float g = gl[(it - runs.it_lo) & (kGBlock - 1)];
       acc[0] *= g;
       acc[1] *= g;
       if (WITH_N) {
         // n before this chunk, as its three partial vectors [3][DHQK] (the consumer of the states adds them up)
-        if (r < 3) {
+        if (r < 3 && a.seg_phase != 1) {
           float* dst = a.nstates + (((size_t)bh * NC + c) * 3 + r) * DHQK + d_wave + 32 * DB + 4 * h;
 #pragma unroll
           for (int g4 = 0; g4 < 4; ++g4)
@@ -523,14 +598,12 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
         accn *= g;
       }
     }
-    // ---- accumulate X^T (scale . Y) over the positions of this piece; two copies of the loop (with and without
-    // the remainder) rather than a branch inside it: the accumulators stay where they are either way
+    // ---- accumulate X^T (scale . Y) over the positions of the chunk
     const uint16_t* Xs = bufs + (p & 1) * BUF;
     const uint16_t* Yh = Xs + XELEMS;
-    const uint16_t* Yl = Yh + YELEMS;
-    const uint16_t* nBp = nB + (it % 3) * (kChunk * 3) + (piece * (PS / 8) + h) * 24 + min(r, 2) * 8;
-    auto multiply_step = [&](auto lo_tag, int js) {
-      constexpr bool LO = decltype(lo_tag)::value;
+    const uint16_t* nBp = nB + (it % 3) * (kChunk * 3) + h * 24 + min(r, 2) * 8;
+#pragma unroll
+    for (int js = 0; js < kChunk / 16; ++js) {
       const Frag A0 = scan_tr_frag<RT>(Xs, 16 * js, offA0), A1 = scan_tr_frag<RT>(Xs, 16 * js, offA1);
       const Frag Bh = scan_tr_frag<WT>(Yh, 16 * js, offB);
       mfma32<F16>(acc[0], A0, Bh);
@@ -538,29 +611,22 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
       if (WITH_N) {
         Frag Bn;
         Bn.u = *(const uint4*)(nBp + js * 48);
-        if (r >= 3) Bn.u = make_uint4(0, 0, 0, 0);
+        // (a second run adds nothing: the three parts carry the whole scale)
+        if (r >= 3 || rest) Bn.u = make_uint4(0, 0, 0, 0);
         mfma32<F16>(accn, DB == 0 ? A0 : A1, Bn);
       }
-      if (LO) {
-        const Frag Bl = scan_tr_frag<WT>(Yl, 16 * js, offB);
-        mfma32<F16>(acc[0], A0, Bl);
-        mfma32<F16>(acc[1], A1, Bl);
-      }
-    };
-    auto multiply = [&](auto lo_tag) {
-      if constexpr (decltype(lo_tag)::value) {
-        // with the remainder operand a step holds four fragments: two steps in flight fit the 128 registers of a wave
-#pragma unroll 2
-        for (int js = 0; js < PS / 16; ++js) multiply_step(lo_tag, js);
-      } else {
-#pragma unroll
-        for (int js = 0; js < PS / 16; ++js) multiply_step(lo_tag, js);
-      }
-    };
-    if (HILO && c >= c_lo) multiply(BoolTag<HILO>{});
-    else multiply(BoolTag<false>{});
+    }
   }
-  if (a.final_out != nullptr) {
+  if (a.seg_phase == 1) {
+    const ScanSeg ss = scan_seg(a, bh, seg);
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const f32x4 v = {acc[db][4 * g4], acc[db][4 * g4 + 1], acc[db][4 * g4 + 2], acc[db][4 * g4 + 3]};
+        *(f32x4*)(ss.c + seg_ofs + (db * 4 + g4) * 256) = v;
+      }
+  } else if (a.final_out != nullptr && is_end) {
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
@@ -569,44 +635,41 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
         a.final_out[((size_t)bh * DHQK + d) * DHHV + w_wave + r] = acc[db][i];
       }
   }
-  if (WITH_N && a.n_final != nullptr) {
+  if (WITH_N && (a.seg_phase == 1 || (a.n_final != nullptr && is_end))) {
+    float* const dst = a.seg_phase == 1 ? scan_seg(a, bh, seg).n : a.n_final + (size_t)bh * DHQK;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       // the three partial columns live in lanes r = 0, 1, 2 of either half wave
       const float x = accn[i];
       const float sum = __shfl(x, 32 * h) + __shfl(x, 32 * h + 1) + __shfl(x, 32 * h + 2);
-      if (r == 0) a.n_final[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)] = sum;
+      if (r == 0) dst[d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)] = sum;
     }
   }
 }
 
-// RT x WT state tile.  HILO: the scaled value rows are split into a 16-bit head and a 16-bit remainder (pieces of 64
-// positions), otherwise rounded once (pieces of 128 positions).
+// RT x WT state tile, one chunk of 128 positions per run.
 //
 // The workgroup has two kinds of waves, NWC of each: CONSUMER waves own a 64 x 32 block of the state tile in their
 // accumulators and do nothing but fragment reads, matrix instructions, the decay and the emission of the state;
-// PRODUCER waves fetch the rows, scale / round / split them and write them into the LDS buffer the consumers will read
-// next, keep the normaliser vector and the scale table.  The two instruction streams of a SIMD that limit each other
+// PRODUCER waves fetch the rows, scale and round them and write them into the LDS buffer the consumers will read
+// next, keep the normaliser operand and the scale table.  The two instruction streams of a SIMD that limit each other
 // when every wave does everything (conversion arithmetic against matrix instructions) then belong to different waves
 // and overlap; four waves per SIMD instead of two.
 template <int RT, int WT, bool F16>
 __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel(ScanArgs a) {
-  constexpr bool HILO = false;  // the remainder split of the value operand is the other kernel's
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;     // consumer waves (and as many producer waves)
   constexpr int NTP = 64 * NWC;           // producer threads
-  constexpr int PS = HILO ? 64 : 128;     // positions per piece
-  constexpr int NP = kChunk / PS;         // pieces per chunk
   constexpr int XU = RT / 8, YU = WT / 8; // 16-byte units per row
-  constexpr int XV = PS * XU / NTP;       // 16-byte vectors per producer thread per piece
-  constexpr int YV = PS * YU / NTP;
+  constexpr int XV = kChunk * XU / NTP;   // 16-byte vectors per producer thread per chunk
+  constexpr int YV = kChunk * YU / NTP;
   constexpr int XRG = NTP / XU;           // rows one sweep of the producers covers (X); a thread's rows are XRG apart
   constexpr int YRG = NTP / YU;
-  constexpr int XELEMS = PS * RT, YELEMS = PS * WT;
-  constexpr int BUF = XELEMS + YELEMS * (HILO ? 2 : 1);  // elements per LDS buffer
+  constexpr int XELEMS = kChunk * RT, YELEMS = kChunk * WT;
+  constexpr int BUF = XELEMS + YELEMS;    // elements per LDS buffer
   static_assert(XV >= 1 && YV >= 1 && XRG % 4 == 0 && YRG % 4 == 0, "tile shape does not fit the staging pattern");
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  uint16_t* bufs = (uint16_t*)smem_raw;                 // [2][X | Yh | Yl]
+  uint16_t* bufs = (uint16_t*)smem_raw;                 // [2][X | Y]
   float* gl = (float*)(bufs + 2 * BUF);                 // [kGBlock] decay factors of the next chunks, in scan order
   float* scl = gl + kGBlock;                            // [2][128] row scales, by chunk parity
   uint16_t* nB = (uint16_t*)(scl + 2 * kChunk);         // [3][128 / 8][3][8] the row scales as a matrix operand (below)
@@ -617,31 +680,36 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
   const int wave = producer ? wave_all : wave_all - NWC;
   const int tid = wave * 64 + lane;                     // index inside the own group of waves
   const BlockId blk = xcd_block_id();  // all tiles of one (batch, head) on one XCD: they share its K/V rows in the L2
-  const int bh = blk.z;
+  const int nrun = a.seg_phase == 1 ? a.nseg - 1 : a.nseg;  // segments this launch runs
+  const int bh = blk.z / nrun, seg = blk.z % nrun;
   const int d_tile = blk.x * RT, w_tile = blk.y * WT;
   const int DHQK = a.DHQK, DHHV = a.DHHV, S = a.S, NC = a.NC;
   const size_t Sp = (size_t)NC * kChunk;
-  // part 1 of a forward scan in two launches: only the chunks before the first one that carries the remainder of the
-  // value operand; the state reached there is handed over in final_out / n_final
-  const int n_run = a.part == 1 ? (a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane)) : NC;
-  const int total = n_run * NP;
-  const int c_first = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
-
-  constexpr int c_lo = 0;  // (no remainder operand in this kernel)
-  // Both kinds of waves pass the same barriers: one after the prologue, one per piece, and one more before every
-  // refill of the decay table (every kGBlock chunks).
-  auto refill_due = [&](int p) { return p % NP == 0 && p / NP > 0 && ((p / NP) & (kGBlock - 1)) == 0; };
+  // forward that returns the last state: the chunks from c_lo on carry the remainder of the value operand and either run
+  // twice here or are left to scan_kernel (the state reached before them is then handed over in final_out / n_final)
+  int n_all = NC, c_lo = NC;
+  if (a.part == 1) {
+    c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
+    if (!scan_repeats_late(NC, c_lo)) n_all = c_lo;
+  }
+  const int it_lo = seg * a.seg_len;
+  const ScanRuns runs(it_lo, min(it_lo + a.seg_len, n_all), min(c_lo, n_all));
+  // the segment whose state is the last one
+  const bool is_end = n_all == 0 ? seg == 0 : (it_lo < n_all && it_lo + a.seg_len >= n_all);
+  if (a.seg_phase == 2 && it_lo >= n_all && !is_end) return;
+  const int total = runs.total;
+  const int c_step = a.backward ? -1 : 1;
+  auto chunk_of = [&](int it) { return a.backward ? NC - 1 - it : it; };
 
   if (producer) {
     // ======================================================================================= producer waves
     const bool do_n = (a.nstates != nullptr) && blk.y == 0;
     const uint16_t* Xg = a.X + (size_t)bh * S * DHQK + d_tile + (tid % XU) * 8;
     const uint16_t* Yg = a.Y + (size_t)bh * S * DHHV + w_tile + (tid % YU) * 8;
-    const int xrow = tid / XU, yrow = tid / YU;  // first row of this thread inside a piece; further rows XRG / YRG apart
+    const int xrow = tid / XU, yrow = tid / YU;  // first row of this thread inside a chunk; further rows XRG / YRG apart
     // LDS store offsets of the first row (elements); the rows of a thread are a multiple of 4 apart: same swizzle
     const int xst = xrow * RT + (((tid % XU) ^ scan_swz<XU>(xrow)) << 3);
     const int yst = yrow * WT + (((tid % YU) ^ scan_swz<YU>(yrow)) << 3);
-    auto piece_t0 = [&](int p) { return (c_first + (p / NP) * c_step) * kChunk + (p % NP) * PS; };
 
     // ---- row scales (forward: abar_j; backward: bbar_t / sqrt(DHQK) / (nrow_t + eps)) go through a table in LDS:
     // every thread fetches the factor of ONE row of a chunk three chunks before that chunk is staged (first in its
@@ -667,7 +735,7 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     // The normaliser recurrence n_c = gbar_c n_{c-1} + sum_j abar_j k_j rides on the matrix pipe of the consumers: the
     // row scale of every position, split exactly into three 16-bit parts, forms three columns of a B operand
     // (position 8b + e of a chunk, part r, at [b][r][e]); K^T times it gives sum_j abar_j k_j in three partial columns
-    // whose sum carries 24 bits of every abar_j.  Slot c % 3: written two chunks before chunk c is multiplied.
+    // whose sum carries 24 bits of every abar_j.  Slot it % 3: written two chunks before chunk `it` is multiplied.
     auto write_n_operand = [&](int it_of_chunk, float sn) {
       uint16_t* dst = nB + (it_of_chunk % 3) * (kChunk * 3) + (srow >> 3) * 24 + (srow & 7);
       const uint16_t p0 = f32_to_elem<F16>(sn);
@@ -679,13 +747,13 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
       dst[16] = p2;
     };
 
-    // two register sets, by piece parity (macros, not lambdas: with the arrays captured by reference the compiler keeps
+    // two register sets, by run parity (macros, not lambdas: with the arrays captured by reference the compiler keeps
     // them in scratch memory)
     u32x4 xr0[XV], yr0[YV], xr1[XV], yr1[YV];
     // The prefetch only LOADS: any arithmetic on a loaded value here would make the wave wait for the whole batch.
 #define MLSTM_SCAN_PREFETCH(SET, p_)                                                                             \
   {                                                                                                              \
-    const int t0_ = piece_t0(p_);                                                                                \
+    const int t0_ = chunk_of(runs.it(p_)) * kChunk;                                                              \
     _Pragma("unroll") for (int v = 0; v < XV; ++v) {                                                             \
       /* rows past the end re-read the last row; their scale is 0 */                                             \
       const int t = min(t0_ + xrow + v * XRG, S - 1);                                                            \
@@ -696,74 +764,71 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
       yr##SET[v] = *(const u32x4*)(Yg + (size_t)t * DHHV);                                                       \
     }                                                                                                            \
   }
-    // registers -> LDS buffer `bi_` (Y rows scaled in fp32, then rounded / split)
+    // registers -> LDS buffer `bi_` (Y rows scaled in fp32, then rounded; second runs: the remainder of that rounding)
 #define MLSTM_SCAN_STAGE(SET, p_, bi_)                                                                           \
   {                                                                                                              \
-    const int c_ = c_first + ((p_) / NP) * c_step, piece_ = (p_) % NP;                                           \
     uint16_t* Xs = bufs + (bi_) * BUF;                                                                           \
     uint16_t* Yh = Xs + XELEMS;                                                                                  \
-    uint16_t* Yl = Yh + YELEMS;                                                                                  \
-    const float* scur = scl + (((p_) / NP) & 1) * kChunk + piece_ * PS;                                          \
-    const bool with_lo = HILO && c_ >= c_lo; /* uniform over the workgroup */                                    \
+    const float* scur = scl + (runs.it(p_) & 1) * kChunk;                                                        \
+    const bool rest_ = runs.rest(p_);                                                                            \
     _Pragma("unroll") for (int v = 0; v < XV; ++v) *(u32x4*)(Xs + xst + v * XRG * RT) = xr##SET[v];              \
     _Pragma("unroll") for (int v = 0; v < YV; ++v) {                                                             \
       const uint32_t in[4] = {yr##SET[v][0], yr##SET[v][1], yr##SET[v][2], yr##SET[v][3]};                       \
-      uint32_t hi[4], lo[4];                                                                                     \
+      uint32_t hi[4];                                                                                            \
       const float sc = scur[yrow + v * YRG];                                                                     \
       _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                                            \
         const float e0 = lo2<F16>(in[e]) * sc;                                                                   \
         const float e1 = hi2<F16>(in[e]) * sc;                                                                   \
         hi[e] = pack2<F16>(e0, e1);                                                                              \
-        if (HILO) lo[e] = pack2<F16>(e0 - lo2<F16>(hi[e]), e1 - hi2<F16>(hi[e]));                                \
+        if (rest_) hi[e] = pack2<F16>(e0 - lo2<F16>(hi[e]), e1 - hi2<F16>(hi[e]));                               \
       }                                                                                                          \
       *(uint4*)(Yh + yst + v * YRG * WT) = make_uint4(hi[0], hi[1], hi[2], hi[3]);                               \
-      if (HILO) {                                                                                                \
-        if (with_lo) *(uint4*)(Yl + yst + v * YRG * WT) = make_uint4(lo[0], lo[1], lo[2], lo[3]);                \
-      }                                                                                                          \
     }                                                                                                            \
   }
 
-    // ---- prologue: scales of the first two chunks, pieces 0 and 1 in registers, piece 0 staged, piece 2 requested
+    // ---- prologue: scales of the first two chunks, runs 0 and 1 in registers, run 0 staged, run 2 requested
+    const int c_first = chunk_of(it_lo);
     {
       load_scales(c_first);
       const float sc0 = scale_value(c_first);
       load_scales(c_first + c_step);
-      const float sc1 = scale_value(NC > 1 ? c_first + c_step : -1);
+      const float sc1 = scale_value(it_lo + 1 < NC ? c_first + c_step : -1);
       if (tid < kChunk) {
-        scl[srow] = sc0;
-        scl[kChunk + srow] = sc1;
+        scl[(it_lo & 1) * kChunk + srow] = sc0;
+        scl[((it_lo + 1) & 1) * kChunk + srow] = sc1;
         if (do_n) {
-          write_n_operand(0, sc0);
-          write_n_operand(1, sc1);
+          write_n_operand(it_lo, sc0);
+          write_n_operand(it_lo + 1, sc1);
         }
       }
-      for (int k = tid; k < kGBlock && k < NC; k += NTP) gl[k] = a.gbar[(size_t)bh * NC + c_first + k * c_step];
+      for (int k = tid; k < kGBlock && it_lo + k < NC; k += NTP) gl[k] = a.gbar[(size_t)bh * NC + c_first + k * c_step];
     }
-    load_scales(c_first + 2 * c_step);  // consumed (table write) at the last piece of the first chunk
-    // (the prefetches are unconditional, past the end the last piece is fetched again: a conditional prefetch makes
+    load_scales(c_first + 2 * c_step);  // consumed (table write) at the last run of the first chunk
+    // (the prefetches are unconditional, past the end the last run is fetched again: a conditional prefetch makes
     // the compiler keep the register sets in scratch memory across the loop back-edge)
+    const int p_max = max(total - 1, 0);
     MLSTM_SCAN_PREFETCH(0, 0)
-    MLSTM_SCAN_PREFETCH(1, max(min(1, total - 1), 0))
+    MLSTM_SCAN_PREFETCH(1, min(1, p_max))
     __syncthreads();  // scale table visible
     MLSTM_SCAN_STAGE(0, 0, 0)
-    MLSTM_SCAN_PREFETCH(0, max(min(2, total - 1), 0))
+    MLSTM_SCAN_PREFETCH(0, min(2, p_max))
 
-    // one piece p of parity PAR (its LDS buffer); the pieces p+1 and p+3 use the other buffer and register set
+    // one run p of parity PAR (its LDS buffer); the runs p+1 and p+3 use the other buffer and register set
 #define MLSTM_SCAN_BODY(PAR, OTHER, p_)                                                                          \
   {                                                                                                              \
-    const int it = (p_) / NP, piece = (p_) % NP;                                                                 \
-    const int c = c_first + it * c_step;                                                                         \
+    const int it = runs.it(p_);                                                                                  \
+    const int c = chunk_of(it);                                                                                  \
     /* The decay factors come from LDS, a block of chunks at a time. */                                          \
-    if (refill_due(p_)) {                                                                                        \
+    if (runs.refill(p_)) {                                                                                       \
       __syncthreads();                                                                                           \
       for (int k = tid; k < kGBlock && it + k < NC; k += NTP) gl[k] = a.gbar[(size_t)bh * NC + c + k * c_step];  \
     }                                                                                                            \
-    /* piece p staged; the consumers are done with piece p-1, whose buffer is staged into next */                \
+    /* run p staged; the consumers are done with run p-1, whose buffer is staged into next */                    \
     __syncthreads();                                                                                             \
-    if (piece == NP - 1) {                                                                                       \
+    if (runs.last(p_)) {                                                                                         \
       /* Table entry of chunk it+2 (its factors were fetched one chunk ago) into the slot of chunk it, all of */ \
-      /* whose pieces have been staged; it is read from the next piece on.  Then the factors of chunk it+3 are */\
-      /* requested, first in this piece's batch of loads. */                                                     \
+      /* whose runs have been staged; it is read from the next run on.  Then the factors of chunk it+3 are */    \
+      /* requested, first in this run's batch of loads. */                                                       \
       if (tid < kChunk) {                                                                                        \
         const float sn = scale_value(it + 2 < NC ? c + 2 * c_step : -1);                                         \
         scl[(it & 1) * kChunk + srow] = sn;                                                                      \
@@ -772,7 +837,7 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
       load_scales(c + 3 * c_step);                                                                               \
     }                                                                                                            \
     if ((p_) + 1 < total) MLSTM_SCAN_STAGE(OTHER, (p_) + 1, OTHER)                                               \
-    MLSTM_SCAN_PREFETCH(OTHER, min((p_) + 3, total - 1))                                                         \
+    MLSTM_SCAN_PREFETCH(OTHER, min((p_) + 3, p_max))                                                             \
   }
     for (int p = 0; p < total; p += 2) {
       MLSTM_SCAN_BODY(0, 1, p)
@@ -786,12 +851,13 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     // the normaliser vector rides with two waves of every 64 state rows in the first column tile: value-column blocks
     // 0 and 1 carry it for the first and the second 32 rows
     const bool with_n = (a.nstates != nullptr) && blk.y == 0;
+    const int tile = blk.x + (int)gridDim.x * blk.y;
     if (with_n && wave % WC == 0)
-      scan_consumer<RT, WT, F16, 0>(a, bufs, gl, nB, wave, lane, bh, d_tile, w_tile, n_run);
+      scan_consumer<RT, WT, F16, 0>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
     else if (with_n && wave % WC == 1)
-      scan_consumer<RT, WT, F16, 1>(a, bufs, gl, nB, wave, lane, bh, d_tile, w_tile, n_run);
+      scan_consumer<RT, WT, F16, 1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
     else
-      scan_consumer<RT, WT, F16, -1>(a, bufs, gl, nB, wave, lane, bh, d_tile, w_tile, n_run);
+      scan_consumer<RT, WT, F16, -1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
   }
 }
 
@@ -802,7 +868,7 @@ static const char* launch_scan_roles_f(const ScanArgs& a, int BH, hipStream_t st
   static LdsLimit lds;
   if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16>, smem))
     return "scan: cannot raise the dynamic LDS limit";
-  dim3 grid(a.DHQK / RT, a.DHHV / WT, BH);
+  dim3 grid(a.DHQK / RT, a.DHHV / WT, BH * (a.seg_phase == 1 ? a.nseg - 1 : a.nseg));
   hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16>), grid, dim3(128 * NW), smem, stream, a);
   return nullptr;
 }
@@ -814,24 +880,53 @@ static const char* launch_scan_roles_t(const ScanArgs& a, int BH, hipStream_t st
 const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t stream) {
   ScanArgs a = a_in;
   a.part = 0;
+  a.n_bh = BH;
+  a.nseg = 1;
+  a.seg_len = a.NC;
+  a.seg_phase = 0;
   if (a.DHQK % 64 != 0 || a.DHHV % 64 != 0) return "scan: DHQK and DHHV must be multiples of 64";
   if (a.stride < 1 || a.stride > kMaxStateStride) return "scan: state stride out of range";
   const bool r128 = a.DHQK % 128 == 0, w128 = a.DHHV % 128 == 0;
+  // Segments (see the top of the file): as many as fit the chip beside each other, at most eight, of eight chunks or more;
+  // with fewer than three the second reading of the sequence costs what the segments gain.  Their states go through the
+  // caller's scratch (an output that is written later), which has to hold them.  B = 1, NH = 8, S = 10000, 256/512: one
+  // scan 151 us in one piece, 45 + 57 us in four.
+  {
+    const int tiles = (a.DHQK / (r128 ? 128 : 64)) * (a.DHHV / (w128 ? 128 : 64));
+    const int fit = device_cu_count() / (BH * tiles);
+    const int nseg = fit < 8 ? fit : 8;
+    const size_t need = (size_t)BH * (nseg - 1) * ((size_t)a.DHQK * a.DHHV + a.DHQK) * sizeof(float);
+    if (nseg >= 3 && a.NC >= 8 * nseg && a.seg != nullptr && need <= a.seg_bytes) {
+      a.seg_len = (a.NC + nseg - 1) / nseg;
+      a.nseg = (a.NC + a.seg_len - 1) / a.seg_len;
+    }
+  }
   auto roles = [&]() -> const char* {
-    if (r128 && w128) return launch_scan_roles_t<128, 128>(a, BH, stream);
-    if (r128) return launch_scan_roles_t<128, 64>(a, BH, stream);
-    if (w128) return launch_scan_roles_t<64, 128>(a, BH, stream);
-    return launch_scan_roles_t<64, 64>(a, BH, stream);
+    auto one = [&]() -> const char* {
+      if (r128 && w128) return launch_scan_roles_t<128, 128>(a, BH, stream);
+      if (r128) return launch_scan_roles_t<128, 64>(a, BH, stream);
+      if (w128) return launch_scan_roles_t<64, 128>(a, BH, stream);
+      return launch_scan_roles_t<64, 64>(a, BH, stream);
+    };
+    if (a.nseg > 1) {
+      a.seg_phase = 1;
+      if (const char* e = one()) return e;
+      a.seg_phase = 2;
+    }
+    return one();
   };
   if (hilo) {
-    // Two launches (forward only): the chunks whose rounding no longer shows in the last state go through the faster
-    // kernel without the remainder operand, which leaves its state in final_out / n_final; the kernel with the
-    // remainder continues from there.  Both find the chunk where they meet from the decay factors alone.
+    // Forward that returns the last state: the chunks whose rounding no longer shows in it need no remainder operand.
+    // Where the rest are few they run twice in the same kernel; otherwise it leaves its state in final_out / n_final and
+    // the kernel with both operands continues from there.  The number is known on the device only (it follows from the
+    // decay factors): the second launch is made in any case and ends at once where it has nothing to do, except for short
+    // sequences, which do not need it, and for the sigmoid gate, where all chunks carry the remainder.
     if (a.final_out == nullptr || a.backward) return "scan: the remainder split serves the forward last state only";
     const bool two = a.nstates == nullptr || a.n_final != nullptr;  // n needs its hand-over buffer too
-    if (two) {
+    if (a.NC <= kScanShort || (two && !a.all_remainder)) {
       a.part = 1;
       if (const char* e = roles()) return e;
+      if (a.NC <= kScanShort) return nullptr;
       a.part = 2;
     }
     if (r128 && w128) return launch_scan_t<128, 128, true>(a, BH, stream);

@@ -11,11 +11,12 @@ from helpers import make_qkvif, rel_norm
 pytestmark = pytest.mark.gpu
 
 
-def _run(S, DQ, DV, *, B=1, NH=2, sig=False, norm="none", init=False, seed=0, dtype=torch.bfloat16, path="auto"):
+def _run(S, DQ, DV, *, B=1, NH=2, sig=False, norm="none", init=False, seed=0, dtype=torch.bfloat16, path="auto",
+         f_offset=3.0):
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
 
     op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
-    q, k, v, i, f = make_qkvif(B, NH, S, DQ, DV, seed=seed, dtype=dtype)
+    q, k, v, i, f = make_qkvif(B, NH, S, DQ, DV, seed=seed, dtype=dtype, f_offset=f_offset)
     g = torch.Generator().manual_seed(seed + 1)
     dH = torch.randn(B, NH, S, DV, generator=g).to(dtype)
     st = (None, None, None)
@@ -68,6 +69,17 @@ def test_head_dimensions(DQ, DV, S, opt):
     if "norm" in opt and DV not in (64, 128, 256, 512):
         pytest.skip("the fused head norm needs DHHV = 64, 128, 256 or 512")
     _run(S, DQ, DV, seed=S + DQ + DV, **opt)
+
+
+@pytest.mark.parametrize("B,NH,S,DQ,DV,opt", [
+    (1, 2, 8 * 128, 256, 512, dict()),                 # one segment per chunk group: the shortest that is cut
+    (1, 2, 65 * 128 - 5, 128, 128, dict(init=True)),   # eight segments, the last one shorter and ragged
+    (1, 1, 67 * 128 + 3, 64, 64, dict(sig=True, init=True)),
+    (1, 4, 4100, 256, 512, dict(dtype=torch.float16)),
+])
+@pytest.mark.parametrize("f_offset", [3.0, 9.0])       # only the last chunks / all chunks weigh in the last state
+def test_segmented_scan(B, NH, S, DQ, DV, opt, f_offset):
+    _run(S, DQ, DV, B=B, NH=NH, seed=S, f_offset=f_offset, **opt)
 
 
 @pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
