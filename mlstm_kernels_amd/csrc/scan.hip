@@ -449,7 +449,8 @@ __device__ __forceinline__ Frag scan_tr_frag(const uint16_t* tile, int k0, const
 
 // What a workgroup of scan_roles_kernel runs: chunks it_lo .. it_hi - 1 in scan order (forward: the chunk index, backward
 // counted from the end), those from it_rep on twice in a row (heads, then remainders of the value rows).  Everything
-// below is counted in runs p = 0 .. total - 1.
+// below is counted in runs p = 0 .. total - 1.  REP = false: nothing runs twice (no last state returned).
+template <bool REP>
 struct ScanRuns {
   int it_lo, it_hi, it_rep, total;
   __device__ __forceinline__ ScanRuns(int lo, int hi, int rep) : it_lo(lo), it_hi(hi), it_rep(max(rep, lo)) {
@@ -457,15 +458,15 @@ struct ScanRuns {
   }
   __device__ __forceinline__ int it(int p) const {  // scan index of run p
     const int q = p - (it_rep - it_lo);
-    return q < 0 ? it_lo + p : it_rep + (q >> 1);
+    return !REP || q < 0 ? it_lo + p : it_rep + (q >> 1);
   }
   __device__ __forceinline__ bool rest(int p) const {  // whether run p is the second run of its chunk
     const int q = p - (it_rep - it_lo);
-    return q >= 0 && (q & 1);
+    return REP && q >= 0 && (q & 1);
   }
   __device__ __forceinline__ bool last(int p) const {  // whether run p is the last one of its chunk
     const int q = p - (it_rep - it_lo);
-    return q < 0 || (q & 1);
+    return !REP || q < 0 || (q & 1);
   }
   // the decay table in LDS holds kGBlock chunks: refilled before the first run of every kGBlock-th chunk of the workgroup
   __device__ __forceinline__ bool refill(int p) const { return p > 0 && !rest(p) && ((it(p) - it_lo) & (kGBlock - 1)) == 0; }
@@ -485,17 +486,22 @@ __device__ __forceinline__ ScanSeg scan_seg(const ScanArgs& a, int bh, int seg) 
 // The consumer role of the scan kernel (see there).  NDB = 0 or 1: this wave also carries the normaliser vector of the
 // first or second 32 of its 64 state rows, NDB = -1: it does not (copies of the role rather than a branch around matrix
 // instructions, which would make the compiler keep those accumulators in scratch memory).
-template <int RT, int WT, bool F16, int NDB>
+template <int RT, int WT, bool F16, bool REP, bool SEG, int NDB>
 __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t* bufs, const float* gl, const uint16_t* nB,
                                               int wave, int lane, int bh, int seg, int tile, int d_tile, int w_tile,
-                                              const ScanRuns runs, bool is_end) {
+                                              const ScanRuns<REP> runs, bool is_end) {
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;
   constexpr int XELEMS = kChunk * RT, YELEMS = kChunk * WT;
   constexpr int BUF = XELEMS + YELEMS;
   const int DHQK = a.DHQK, DHHV = a.DHHV, NC = a.NC;
   const int total = runs.total;
-  constexpr bool WITH_N = NDB >= 0;
+  constexpr bool WITH_N = NDB >= 0;  // (forward only)
+  const bool backward = !WITH_N && a.backward;
+  const int c_base = backward ? NC - 1 : 0, c_step = backward ? -1 : 1;
+  // slot and position of the running chunk among the kept states, carried along: divisions by the stride in the loop
+  // take as long as half its matrix instructions
+  int st_slot = (c_base + runs.it_lo * c_step) / a.stride, st_pos = (c_base + runs.it_lo * c_step) % a.stride;
   constexpr int DB = WITH_N ? NDB : 0;
   const int wr = wave / WC, wc = wave % WC;
   const int r = lane & 31, h = lane >> 5;
@@ -506,7 +512,7 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float v0 = 0.f;
-      if (a.init != nullptr && a.seg_phase != 1) {
+      if (a.init != nullptr && (!SEG || a.seg_phase != 1)) {
         const int d = d_wave + 32 * db + 8 * (i / 4) + 4 * h + (i % 4);
         v0 = a.init[((size_t)bh * DHQK + d) * DHHV + w_wave + r];
       }
@@ -518,12 +524,12 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     float v0 = 0.f;
-    if (WITH_N && a.n_init != nullptr && a.seg_phase != 1 && r == 0)
+    if (WITH_N && a.n_init != nullptr && (!SEG || a.seg_phase != 1) && r == 0)
       v0 = a.n_init[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)];
     accn[i] = v0;
   }
   const size_t seg_ofs = ((size_t)tile * NWC + wave) * 2048 + lane * 4;
-  if (a.seg_phase == 2) {
+  if (SEG && a.seg_phase == 2) {
     // the state before this segment: the segments in front of it, each decayed over what lies between
     for (int x = 0; x < seg; ++x) {
       float dec = 1.f;
@@ -558,18 +564,18 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
   for (int p = 0; p < total; ++p) {
     const int it = runs.it(p);
     const bool rest = runs.rest(p);
-    const int c = a.backward ? NC - 1 - it : it;
+    const int c = c_base + it * c_step;
     if (runs.refill(p)) __syncthreads();
     __syncthreads();  // run p staged by the producers
     if (!rest) {
       // ---- the state before this chunk's update as operand fragments, at the kept boundaries only: forward the
       // state before every stride-th chunk, backward the gradient of the state after the last chunk of every group
       // of `stride` chunks (and after the last chunk of the sequence); slot c / stride either way
-      const bool keep = a.seg_phase != 1 && (a.backward ? (c == NC - 1 || (c + 1) % a.stride == 0) : (c % a.stride == 0));
+      const bool keep = (!SEG || a.seg_phase != 1) && (backward ? (c == NC - 1 || st_pos == a.stride - 1) : st_pos == 0);
       if (keep) {
         const size_t ND = DHQK / 16, NWB = DHHV / 32;
         const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
-        u32x4* st = (u32x4*)a.states + ((size_t)bh * NCS + c / a.stride) * NWB * ND * 64;
+        u32x4* st = (u32x4*)a.states + ((size_t)bh * NCS + st_slot) * NWB * ND * 64;
 #pragma unroll
         for (int db = 0; db < 2; ++db) {
           const size_t W32 = w_wave / 32, D16 = (d_wave + 32 * db) / 16;
@@ -584,12 +590,20 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
           }
         }
       }
+      st_pos += c_step;
+      if (st_pos == a.stride) {
+        st_pos = 0;
+        ++st_slot;
+      } else if (st_pos < 0) {
+        st_pos = a.stride - 1;
+        --st_slot;
+      }
       const float g = gl[(it - runs.it_lo) & (kGBlock - 1)];
       acc[0] *= g;
       acc[1] *= g;
       if (WITH_N) {
         // n before this chunk, as its three partial vectors [3][DHQK] (the consumer of the states adds them up)
-        if (r < 3 && a.seg_phase != 1) {
+        if (r < 3 && (!SEG || a.seg_phase != 1)) {
           float* dst = a.nstates + (((size_t)bh * NC + c) * 3 + r) * DHQK + d_wave + 32 * DB + 4 * h;
 #pragma unroll
           for (int g4 = 0; g4 < 4; ++g4)
@@ -617,7 +631,7 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
       }
     }
   }
-  if (a.seg_phase == 1) {
+  if (SEG && a.seg_phase == 1) {
     const ScanSeg ss = scan_seg(a, bh, seg);
 #pragma unroll
     for (int db = 0; db < 2; ++db)
@@ -635,8 +649,8 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
         a.final_out[((size_t)bh * DHQK + d) * DHHV + w_wave + r] = acc[db][i];
       }
   }
-  if (WITH_N && (a.seg_phase == 1 || (a.n_final != nullptr && is_end))) {
-    float* const dst = a.seg_phase == 1 ? scan_seg(a, bh, seg).n : a.n_final + (size_t)bh * DHQK;
+  if (WITH_N && (SEG && a.seg_phase == 1 || (a.n_final != nullptr && is_end))) {
+    float* const dst = SEG && a.seg_phase == 1 ? scan_seg(a, bh, seg).n : a.n_final + (size_t)bh * DHQK;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       // the three partial columns live in lanes r = 0, 1, 2 of either half wave
@@ -647,7 +661,8 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
   }
 }
 
-// RT x WT state tile, one chunk of 128 positions per run.
+// RT x WT state tile, one chunk of 128 positions per run.  REP: the late chunks run twice; SEG: the sequence is cut into
+// segments (both compile-time: tested per run they cost the plain scan 6 %, 331 against 311 us at B = 4, S = 16384).
 //
 // The workgroup has two kinds of waves, NWC of each: CONSUMER waves own a 64 x 32 block of the state tile in their
 // accumulators and do nothing but fragment reads, matrix instructions, the decay and the emission of the state;
@@ -655,7 +670,7 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 // next, keep the normaliser operand and the scale table.  The two instruction streams of a SIMD that limit each other
 // when every wave does everything (conversion arithmetic against matrix instructions) then belong to different waves
 // and overlap; four waves per SIMD instead of two.
-template <int RT, int WT, bool F16>
+template <int RT, int WT, bool F16, bool REP, bool SEG>
 __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel(ScanArgs a) {
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;     // consumer waves (and as many producer waves)
@@ -680,26 +695,26 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
   const int wave = producer ? wave_all : wave_all - NWC;
   const int tid = wave * 64 + lane;                     // index inside the own group of waves
   const BlockId blk = xcd_block_id();  // all tiles of one (batch, head) on one XCD: they share its K/V rows in the L2
-  const int nrun = a.seg_phase == 1 ? a.nseg - 1 : a.nseg;  // segments this launch runs
-  const int bh = blk.z / nrun, seg = blk.z % nrun;
+  const int nrun = !SEG ? 1 : (a.seg_phase == 1 ? a.nseg - 1 : a.nseg);  // segments this launch runs
+  const int bh = SEG ? blk.z / nrun : blk.z, seg = SEG ? blk.z % nrun : 0;
   const int d_tile = blk.x * RT, w_tile = blk.y * WT;
   const int DHQK = a.DHQK, DHHV = a.DHHV, S = a.S, NC = a.NC;
   const size_t Sp = (size_t)NC * kChunk;
   // forward that returns the last state: the chunks from c_lo on carry the remainder of the value operand and either run
   // twice here or are left to scan_kernel (the state reached before them is then handed over in final_out / n_final)
   int n_all = NC, c_lo = NC;
-  if (a.part == 1) {
+  if (REP) {
     c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
     if (!scan_repeats_late(NC, c_lo)) n_all = c_lo;
   }
-  const int it_lo = seg * a.seg_len;
-  const ScanRuns runs(it_lo, min(it_lo + a.seg_len, n_all), min(c_lo, n_all));
+  const int it_lo = SEG ? seg * a.seg_len : 0;
+  const ScanRuns<REP> runs(it_lo, SEG ? min(it_lo + a.seg_len, n_all) : n_all, min(c_lo, n_all));
   // the segment whose state is the last one
-  const bool is_end = n_all == 0 ? seg == 0 : (it_lo < n_all && it_lo + a.seg_len >= n_all);
-  if (a.seg_phase == 2 && it_lo >= n_all && !is_end) return;
+  const bool is_end = !SEG || (n_all == 0 ? seg == 0 : (it_lo < n_all && it_lo + a.seg_len >= n_all));
+  if (SEG && a.seg_phase == 2 && it_lo >= n_all && !is_end) return;
   const int total = runs.total;
-  const int c_step = a.backward ? -1 : 1;
-  auto chunk_of = [&](int it) { return a.backward ? NC - 1 - it : it; };
+  const int c_base = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
+  auto chunk_of = [&](int it) { return c_base + it * c_step; };
 
   if (producer) {
     // ======================================================================================= producer waves
@@ -853,28 +868,34 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     const bool with_n = (a.nstates != nullptr) && blk.y == 0;
     const int tile = blk.x + (int)gridDim.x * blk.y;
     if (with_n && wave % WC == 0)
-      scan_consumer<RT, WT, F16, 0>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
+      scan_consumer<RT, WT, F16, REP, SEG, 0>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
     else if (with_n && wave % WC == 1)
-      scan_consumer<RT, WT, F16, 1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
+      scan_consumer<RT, WT, F16, REP, SEG, 1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
     else
-      scan_consumer<RT, WT, F16, -1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
+      scan_consumer<RT, WT, F16, REP, SEG, -1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
   }
 }
 
-template <int RT, int WT, bool F16>
+template <int RT, int WT, bool F16, bool REP, bool SEG>
 static const char* launch_scan_roles_f(const ScanArgs& a, int BH, hipStream_t stream) {
   constexpr int NW = (RT / 64) * (WT / 32);
   const size_t smem = (size_t)2 * kChunk * (RT + WT) * 2 + (size_t)(kGBlock + 2 * kChunk) * 4 + (size_t)3 * kChunk * 3 * 2;
   static LdsLimit lds;
-  if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16>, smem))
+  if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16, REP, SEG>, smem))
     return "scan: cannot raise the dynamic LDS limit";
   dim3 grid(a.DHQK / RT, a.DHHV / WT, BH * (a.seg_phase == 1 ? a.nseg - 1 : a.nseg));
-  hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16>), grid, dim3(128 * NW), smem, stream, a);
+  hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16, REP, SEG>), grid, dim3(128 * NW), smem, stream, a);
   return nullptr;
+}
+template <int RT, int WT, bool F16>
+static const char* launch_scan_roles_s(const ScanArgs& a, int BH, hipStream_t stream) {
+  if (a.nseg > 1)
+    return a.part == 1 ? launch_scan_roles_f<RT, WT, F16, true, true>(a, BH, stream) : launch_scan_roles_f<RT, WT, F16, false, true>(a, BH, stream);
+  return a.part == 1 ? launch_scan_roles_f<RT, WT, F16, true, false>(a, BH, stream) : launch_scan_roles_f<RT, WT, F16, false, false>(a, BH, stream);
 }
 template <int RT, int WT>
 static const char* launch_scan_roles_t(const ScanArgs& a, int BH, hipStream_t stream) {
-  return a.f16 ? launch_scan_roles_f<RT, WT, true>(a, BH, stream) : launch_scan_roles_f<RT, WT, false>(a, BH, stream);
+  return a.f16 ? launch_scan_roles_s<RT, WT, true>(a, BH, stream) : launch_scan_roles_s<RT, WT, false>(a, BH, stream);
 }
 
 const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t stream) {

@@ -72,7 +72,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 // NORM (forward, DHHV = 512: a work item then holds complete rows of H): the multi-head layer / rms norm over the value
 // columns is applied when the rows are rounded, as an affine map of the accumulators.
-template <bool IS_DV, bool F16, bool NORM = false>
+// RAGGED: S is not a multiple of 128 (at compile time: the clamps and predicated stores cost full chunks 2 %).
+template <bool IS_DV, bool F16, bool NORM, bool RAGGED>
 __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items, int n_rounds) {
   static_assert(!(IS_DV && NORM), "the head norm belongs to the forward");
   constexpr int DHQK = 256;
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     }                                                                                                                \
     if (__builtin_amdgcn_readfirstlane((int)((w_ >> 22) & 1)) && p < 64) {                                           \
       ovec[p] = fa##E[0];                                                                                   \
-      if (IS_DV) orho[p] = ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
+      if (IS_DV) orho[p] = RAGGED && ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
     }                                                                                                                \
   }
     // base_: (batch, head) base of the operand; g0_: byte offset of the thread's first piece, gs_: distance between
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     const bool st_ = L >= 3;                                                                                         \
     if (st_ && __builtin_amdgcn_readfirstlane((int)((w_ >> 22) & 1)) && p < 64) {                                    \
       ovec[p] = fa##E[0];                                                                                   \
-      if (IS_DV) orho[p] = ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
+      if (IS_DV) orho[p] = RAGGED && ((w_ >> 24) & 1) ? 0.f : (a.use_nrow ? 1.f / (fa##E[1] + a.eps) : 1.f);                   \
     }                                                                                                                \
     fa##E[0] = ov_src[gi_];                                                                                          \
     fa##E[1] = rho_src[gi_];                                                                                         \
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         *(uint2*)(smem_raw + d0_ + i_ * step_) = make_uint2(fd##E[i_][0], fd##E[i_][1]);                             \
         *(uint2*)(smem_raw + d0_ + i_ * step_ + half_) = make_uint2(fd##E[i_][2], fd##E[i_][3]);                     \
       }                                                                                                              \
-      if (i_ < (NP_)) fd##E[i_] = *(const u32x4*)((base_) + min((g0_) + i_ * (gs_), (lim_)));                         \
+      if (i_ < (NP_)) fd##E[i_] = *(const u32x4*)((base_) + (RAGGED ? min((g0_) + i_ * (gs_), (lim_)) : (g0_) + i_ * (gs_)));                         \
     }                                                                                                                \
     fw##E = (dstw_) | ((NP_) == 4 ? 1u << 23 : 0u);                                                                  \
     ++L;                                                                                                             \
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
           const size_t gi = (size_t)it.bh * Sp + (size_t)sc * kChunk + (pl & 63);
           const uint32_t vg = (t0 + vrow) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * 1024 + vpc * 16;
           // (bit 24: the gate-vector entry this thread carries lies past the end of the sequence)
-          const uint32_t past0 = t0 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24, past1 = t0 + 64 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24;
+          const uint32_t past0 = !RAGGED || t0 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24, past1 = !RAGGED || t0 + 64 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24;
           const uint32_t vgs = 4 * (uint32_t)DHHV * 2, vg32 = 32 * (uint32_t)DHHV * 2;
           // first half: scores -> slot 0, value rows -> slot 1 and slot 0
           HV_PROC(0, 8, kbase, (t0 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, klim, (kRing0Off + kd) | (1u << 22) | past0, gi)
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const float ex_ = t1_ * iv * (1.f / 512.f), ex2_ = t2_ * iv * iv * (1.f / 512.f);                              \
       const float mean_ = a.head_norm == 1 ? ex_ : 0.f;                                                              \
       const float rstd_ = rsqrtf(fmaxf(ex2_ - mean_ * mean_, 0.f) + a.norm_eps);                                     \
-      if (ci == 0 && h == 0 && prev.c * kChunk + t_ < S) {                                                           \
+      if (ci == 0 && h == 0 && (!RAGGED || prev.c * kChunk + t_ < S)) {                                                           \
         const size_t tg_ = (size_t)prev.bh * S + (size_t)prev.c * kChunk + t_;                                       \
         a.norm_mean[tg_] = mean_;                                                                                    \
         a.norm_rstd[tg_] = rstd_;                                                                                    \
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     const int rows_left_ = S - (prev.c * kChunk + 64 * pi + 32 * NB);                                                \
     _Pragma("unroll") for (int k = 0; k < 32 * VPR / 64; ++k) {                                                      \
       const int row = le / VPR + (64 / VPR) * k, pc = le % VPR;                                                      \
-      if (row < rows_left_)                                                                                          \
+      if (!RAGGED || row < rows_left_)                                                                                          \
         __builtin_nontemporal_store(*(const u32x4*)(stg + row * SR + pc * 8), (u32x4*)(Og + (size_t)row * DHHV + pc * 8)); \
     }                                                                                                                \
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                                           \
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
                 if (it.ch == 0) {
                   a.nrow_out[gofs + t] = nmax;
                   const size_t tg = (size_t)bh * S + (size_t)c * kChunk + t;
-                  if (c * kChunk + t < S) {
+                  if (!RAGGED || c * kChunk + t < S) {
                     if (a.n_out != nullptr) a.n_out[tg] = nmax;
                     if (a.m_out != nullptr) a.m_out[tg] = mcr;
                   }
@@ -603,8 +604,8 @@ bool stream_hv_supported(const ParHvArgs& a) {
 }
 
 namespace {
-template <bool IS_DV, bool F16, bool NORM = false>
-const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
+template <bool IS_DV, bool F16, bool NORM, bool RAGGED>
+const char* launch_stream_hv_r(const ParHvArgs& a, int BH, hipStream_t stream) {
   constexpr int QS = 256 + 8, PSS = 72, SLOT = 64 * QS;
   const size_t smem = (size_t)(128 * QS + 128 * PSS + 2 * SLOT) * 2 +
                       (size_t)(4 * 128 + 128 + 256 + 64 + 64 + 128 + 128 + (NORM ? 8 * 128 : 0)) * 4;
@@ -617,10 +618,15 @@ const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
-  if (!lds.allow((const void*)stream_hv_kernel<IS_DV, F16, NORM>, smem))
+  if (!lds.allow((const void*)stream_hv_kernel<IS_DV, F16, NORM, RAGGED>, smem))
     return "stream_hv: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((stream_hv_kernel<IS_DV, F16, NORM>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
+  hipLaunchKernelGGL((stream_hv_kernel<IS_DV, F16, NORM, RAGGED>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
   return nullptr;
+}
+template <bool IS_DV, bool F16, bool NORM = false>
+const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
+  return a.S % kChunk != 0 ? launch_stream_hv_r<IS_DV, F16, NORM, true>(a, BH, stream)
+                           : launch_stream_hv_r<IS_DV, F16, NORM, false>(a, BH, stream);
 }
 }  // namespace
 

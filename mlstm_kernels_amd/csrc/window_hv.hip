@@ -39,7 +39,8 @@ static_assert(kHvSmem <= 160 * 1024, "LDS budget of one CU");
 
 // MULTI: DHHV is several groups of CW columns (P then has to outlive the epilogue of a group, which otherwise stages its
 // rows in it).  NORM (forward, one group): the multi-head layer / rms norm is applied to the rows as they are rounded.
-template <int CW, bool MULTI, bool IS_DV, bool NORM, bool F16>
+// RAGGED: S is not a multiple of 256.
+template <int CW, bool MULTI, bool IS_DV, bool NORM, bool RAGGED, bool F16>
 __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items, int n_rounds) {
   static_assert(!(IS_DV && NORM) && !(MULTI && NORM), "the head norm belongs to the forward and needs complete rows");
   constexpr int NCI = CW / 64;                     // 64-column groups = consumer waves side by side over the columns
@@ -110,11 +111,11 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     const bool st_ = L >= 2;                                                                                         \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oA_ + i_ * 4096) = fd##E[i_];                                                    \
-      if (i_ < (nA_)) fd##E[i_] = *(const u32x4*)((bA_) + min((gA_) + i_ * (sA_), (lA_)));                           \
+      if (i_ < (nA_)) fd##E[i_] = *(const u32x4*)((bA_) + (RAGGED ? min((gA_) + i_ * (sA_), (lA_)) : (gA_) + i_ * (sA_)));                           \
     }                                                                                                                \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) WH_PUT_B(E, i_, perm_)                                                                                \
-      if (i_ < (nB_)) fd##E[4 + i_] = *(const u32x4*)((bB_) + min((gB_) + i_ * (sB_), (lB_)));                       \
+      if (i_ < (nB_)) fd##E[4 + i_] = *(const u32x4*)((bB_) + (RAGGED ? min((gB_) + i_ * (sB_), (lB_)) : (gB_) + i_ * (sB_)));                       \
     }                                                                                                                \
     fa##E = (dA_) + (E) * kWinSlot;                                                                                  \
     fb##E = (dB_) + (E) * kWinSlot;                                                                                  \
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     // gate vectors and normaliser state of a window, requested ahead of its first step
     float pu = 0.f, pw = 0.f, pr = 1.f, pc = 0.f, pb = 0.f, pm = 0.f, np0 = 0.f, np1 = 0.f, np2 = 0.f;
     auto request = [&](const WinItem& x) {
-      const int c0 = 2 * x.win, n_pos = S - 256 * x.win;
+      const int c0 = 2 * x.win, n_pos = RAGGED ? S - 256 * x.win : 256;
       const size_t gofs = (size_t)x.bh * Sp + (size_t)c0 * kChunk;
       if (tid < 256) {
         const size_t gi = gofs + min(tid, n_pos - 1);
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         if (IS_DV) {
           if (a.use_nrow) pr = a.nrow[gi];
           // keys of c0 see dC through chunk c1, where there is one
-          const float xs = c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
+          const float xs = !RAGGED || c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
           pc = a.g.abar[gi] * (tid < 128 ? xs : 1.f);
         } else {
           const float xs = __expf(graw[c0] + mst[c0] - mst[c0 + 1]);  // positions of c1 see C through chunk c0
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       }
     };
     auto publish = [&](const WinItem& x) {
-      const int n_pos = S - 256 * x.win;
+      const int n_pos = RAGGED ? S - 256 * x.win : 256;
       if (tid < 256) {
         // past the end: no key (w = infinity), no query (factor 0)
         uvec[tid] = pu;
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   {                                                                                                                  \
     const int le = opaque(lane);                                                                                     \
     const int r = le & 31, h = le >> 5;                                                                              \
-    const int n_pos_ = S - 256 * prev.win;                                                                           \
+    const int n_pos_ = RAGGED ? S - 256 * prev.win : 256;                                                                           \
     char* const Ob_ = (char*)a.Out + ((size_t)prev.bh * S + (size_t)prev.win * 256) * (DHHV * 2);                    \
     const uint32_t lofs_ = (uint32_t)(le >> 3) * (uint32_t)(DHHV * 2) + (uint32_t)(prev_cg * CW * 2 + 128 * ci + 16 * (le & 7)); \
     _Pragma("unroll") for (int nb = 0; nb < NNB; ++nb) {                                                             \
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         _Pragma("unroll") for (int k = 0; k < SROWS / 8; ++k) {                                                      \
           const int row_ = (le >> 3) + 8 * k, n0_ = 32 * (NPG * nb + pg) + sr + 8 * k;                               \
           const u32x4 o_ = *(const u32x4*)(stg + row_ * 128 + (((le & 7) ^ (row_ & 7)) * 16));                       \
-          if (n0_ + (le >> 3) < n_pos_)                                                                              \
+          if (!RAGGED || n0_ + (le >> 3) < n_pos_)                                                                              \
             __builtin_nontemporal_store(o_, (u32x4*)(Ob_ + ((uint32_t)n0_ * (uint32_t)(DHHV * 2) + lofs_)));         \
         }                                                                                                            \
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                                       \
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     for (int rd = 0; rd < n_rounds; ++rd) {
       if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
-      const int n_pos = S - 256 * it.win;
+      const int n_pos = RAGGED ? S - 256 * it.win : 256;
       const float g01 = a.g.graw[(size_t)bh * NC + c0];
 
       if (first) request(it);
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
               iv = 1.f / (nmax + a.eps);
             }
             inv[t] = iv;
-            if (c0 * kChunk + t < (int)Sp) a.nrow_out[(size_t)bh * Sp + (size_t)c0 * kChunk + t] = nmax;
+            if (!RAGGED || c0 * kChunk + t < (int)Sp) a.nrow_out[(size_t)bh * Sp + (size_t)c0 * kChunk + t] = nmax;
             if (t < n_pos) {
               const size_t tg = (size_t)bh * S + (size_t)c0 * kChunk + t;
               if (a.n_out != nullptr) a.n_out[tg] = nmax;
@@ -574,8 +575,8 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
 }
 
 namespace {
-template <int CW, bool MULTI, bool IS_DV, bool NORM, bool F16>
-const char* launch_window_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
+template <int CW, bool MULTI, bool IS_DV, bool NORM, bool RAGGED, bool F16>
+const char* launch_window_hv_r(const ParHvArgs& a, int BH, hipStream_t stream) {
   const long long n_items = (long long)BH * ((a.NC + 1) / 2);
   if (n_items >= (1ll << 31)) return "window_hv: too many work items";
   if ((size_t)a.S * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32))
@@ -586,20 +587,26 @@ const char* launch_window_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
-  if (!lds.allow((const void*)window_hv_kernel<CW, MULTI, IS_DV, NORM, F16>, kHvSmem))
+  if (!lds.allow((const void*)window_hv_kernel<CW, MULTI, IS_DV, NORM, RAGGED, F16>, kHvSmem))
     return "window_hv: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((window_hv_kernel<CW, MULTI, IS_DV, NORM, F16>), dim3(G), dim3(768), kHvSmem, stream, a, (int)n_items, n_rounds);
+  hipLaunchKernelGGL((window_hv_kernel<CW, MULTI, IS_DV, NORM, RAGGED, F16>), dim3(G), dim3(768), kHvSmem, stream, a, (int)n_items, n_rounds);
   return nullptr;
+}
+template <int CW, bool MULTI, bool IS_DV, bool NORM>
+const char* launch_window_hv_n(const ParHvArgs& a, int BH, hipStream_t stream) {
+  if (a.S % (2 * kChunk) != 0)
+    return a.f16 ? launch_window_hv_r<CW, MULTI, IS_DV, NORM, true, true>(a, BH, stream)
+                 : launch_window_hv_r<CW, MULTI, IS_DV, NORM, true, false>(a, BH, stream);
+  return a.f16 ? launch_window_hv_r<CW, MULTI, IS_DV, NORM, false, true>(a, BH, stream)
+               : launch_window_hv_r<CW, MULTI, IS_DV, NORM, false, false>(a, BH, stream);
 }
 template <int CW, bool MULTI>
 const char* launch_window_hv_c(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
-  if (is_dv)
-    return a.f16 ? launch_window_hv_t<CW, MULTI, true, false, true>(a, BH, stream) : launch_window_hv_t<CW, MULTI, true, false, false>(a, BH, stream);
+  if (is_dv) return launch_window_hv_n<CW, MULTI, true, false>(a, BH, stream);
   if constexpr (!MULTI) {
-    if (a.head_norm != 0)
-      return a.f16 ? launch_window_hv_t<CW, MULTI, false, true, true>(a, BH, stream) : launch_window_hv_t<CW, MULTI, false, true, false>(a, BH, stream);
+    if (a.head_norm != 0) return launch_window_hv_n<CW, MULTI, false, true>(a, BH, stream);
   }
-  return a.f16 ? launch_window_hv_t<CW, MULTI, false, false, true>(a, BH, stream) : launch_window_hv_t<CW, MULTI, false, false, false>(a, BH, stream);
+  return launch_window_hv_n<CW, MULTI, false, false>(a, BH, stream);
 }
 }  // namespace
 

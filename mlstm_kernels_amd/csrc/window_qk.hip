@@ -48,7 +48,8 @@ static_assert(kWqSmem <= 160 * 1024, "LDS budget of one CU");
 
 // DT = head-dim rows of a tile: 256, 128 or 64.  MULTI: the head dimension is several tiles, walked one after the other
 // with the same scores (otherwise it is a compile-time constant).
-template <int DT, bool MULTI, bool F16>
+// RAGGED: S is not a multiple of 256 (at compile time: the clamps and predicated stores cost full windows 1 %).
+template <int DT, bool MULTI, bool RAGGED, bool F16>
 __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items, int n_rounds, int n_bh) {
   constexpr int NDI = DT / 64;           // consumer waves over the head-dim rows of a tile
   constexpr int NPG = 8 / NDI;           // consumer waves over the positions: blocks NPG * nb + pg of 32 positions
@@ -103,11 +104,11 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     const bool st_ = L >= 2;                                                                                         \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oA_ + i_ * 4096) = fd##E[i_];                                                    \
-      if (i_ < (nA_)) fd##E[i_] = *(const u32x4*)((bA_) + min((gA_) + i_ * (sA_), (lA_)));                                                     \
+      if (i_ < (nA_)) fd##E[i_] = *(const u32x4*)((bA_) + (RAGGED ? min((gA_) + i_ * (sA_), (lA_)) : (gA_) + i_ * (sA_)));                                                     \
     }                                                                                                                \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       if (st_) *(u32x4*)(smem_raw + oB_ + i_ * 4096) = fd##E[4 + i_];                                                \
-      fd##E[4 + i_] = *(const u32x4*)((bB_) + min((gB_) + i_ * (sB_), (lB_)));                                                 \
+      fd##E[4 + i_] = *(const u32x4*)((bB_) + (RAGGED ? min((gB_) + i_ * (sB_), (lB_)) : (gB_) + i_ * (sB_)));                                                 \
     }                                                                                                                \
     fw##E = ((dAu_) + (E) * (kWinSlot / 16)) | (((dBu_) + (E) * (kWinSlot / 16)) << 16);                               \
     ++L;                                                                                                             \
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         if constexpr (NDI == 2) dot += red[256 + tid];
         if constexpr (NDI == 4) dot = (dot + red[256 + tid]) + (red[512 + tid] + red[768 + tid]);
         // one slot per head-dim tile: [tile][batch * head][position]
-        if (prev.win * 256 + tid < S)
+        if (!RAGGED || prev.win * 256 + tid < S)
           (pending == 2 ? a.rowdot2 : a.rowdot)[((size_t)prev_dg * n_bh + prev.bh) * Sp + (size_t)prev.win * 256 + tid] = dot;
       }
       pending = 0;
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const float* graw = a.g.graw + (size_t)bh * NC;
       const float* mst = a.g.mstates + (size_t)bh * (NC + 1);
       const float g01 = graw[c0];   // decay over chunk c0: what separates a position of c1 from the keys of c0
-      const int n_pos = S - 256 * it.win;   // positions of the window inside the sequence (256 or more: all)
+      const int n_pos = RAGGED ? S - 256 * it.win : 256;   // positions of the window inside the sequence (256 or more: all)
 
       // ================================================================================= phase S: the score blocks
       {
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           const size_t gi = gofs + min(tid, n_pos - 1);
           if (dk) {
             // keys of c0 see dC through chunk c1, where there is one (the gradient kept is that after the last chunk)
-            const float xs = c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
+            const float xs = !RAGGED || c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
             csn = a.g.abar[gi] * (tid < 128 ? xs : 1.f);
           } else {
             const float xs = __expf(g01 + mst[c0] - mst[c0 + 1]);                // positions of c1 see C through chunk c0
@@ -506,8 +507,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
             const u32x4 o1 = *(const u32x4*)(stg + (row8 + 8) * 128 + ((un ^ row8) * 16));
             __builtin_amdgcn_wave_barrier();
             const uint32_t n0 = (uint32_t)(ZROWS * z + 32 * pg + 16 * q);
-            if ((int)n0 + row8 < n_pos) __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (uint32_t)(DHQK * 2))));
-            if ((int)n0 + 8 + row8 < n_pos) __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (uint32_t)(DHQK * 2))));
+            if (!RAGGED || (int)n0 + row8 < n_pos) __builtin_nontemporal_store(o0, (u32x4*)(Ob + (lofs + n0 * (uint32_t)(DHQK * 2))));
+            if (!RAGGED || (int)n0 + 8 + row8 < n_pos) __builtin_nontemporal_store(o1, (u32x4*)(Ob + (lofs + (n0 + 8) * (uint32_t)(DHQK * 2))));
           }
         }
         pending = dk ? 2 : 1;
@@ -530,7 +531,7 @@ bool window_qk_supported(const ParQkArgs& a) {
 }
 
 namespace {
-template <int DT, bool MULTI, bool F16>
+template <int DT, bool MULTI, bool RAGGED, bool F16>
 const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   const long long n_items = (long long)BH * ((a.NC + 1) / 2);
   if (n_items >= (1ll << 31)) return "window_qk: too many work items";
@@ -542,14 +543,16 @@ const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
-  if (!lds.allow((const void*)window_qk_kernel<DT, MULTI, F16>, kWqSmem))
+  if (!lds.allow((const void*)window_qk_kernel<DT, MULTI, RAGGED, F16>, kWqSmem))
     return "window_qk: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((window_qk_kernel<DT, MULTI, F16>), dim3(G), dim3(768), kWqSmem, stream, a, (int)n_items, n_rounds, BH);
+  hipLaunchKernelGGL((window_qk_kernel<DT, MULTI, RAGGED, F16>), dim3(G), dim3(768), kWqSmem, stream, a, (int)n_items, n_rounds, BH);
   return nullptr;
 }
 template <int DT, bool MULTI>
 const char* launch_window_qk_d(const ParQkArgs& a, int BH, hipStream_t stream) {
-  return a.f16 ? launch_window_qk_t<DT, MULTI, true>(a, BH, stream) : launch_window_qk_t<DT, MULTI, false>(a, BH, stream);
+  if (a.S % (2 * kChunk) != 0)
+    return a.f16 ? launch_window_qk_t<DT, MULTI, true, true>(a, BH, stream) : launch_window_qk_t<DT, MULTI, true, false>(a, BH, stream);
+  return a.f16 ? launch_window_qk_t<DT, MULTI, false, true>(a, BH, stream) : launch_window_qk_t<DT, MULTI, false, false>(a, BH, stream);
 }
 }  // namespace
 
