@@ -157,6 +157,16 @@ const char* launch_step_seq(const void* q, const void* k, const void* v, const v
                             const void* c_in, const void* n_in, const void* m_in, void* h, void* c_out,
                             void* n_out, void* m_out, int B, int NH, int T, int DHQK, int DHHV, float eps,
                             int dtype_qkv, int dtype_gates, int dtype_state, hipStream_t stream);
+// the same recurrence on the matrix cores, tokens in blocks, for the types and shapes it supports
+struct StepBlockArgs {
+  const void *q, *k, *v, *i, *f, *c_in, *n_in, *m_in;
+  void *h, *c_out, *n_out, *m_out;
+  int BH, T, DHQK, DHHV;
+  float eps;
+  int dtype_qkv, dtype_gates, dtype_state;
+};
+bool step_block_supported(int DHQK, int DHHV, int dtype_qkv);
+const char* launch_step_block(const StepBlockArgs& a, hipStream_t stream);
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
                          int B, int NH, int S, int dtype_gates, int sig_gate, hipStream_t stream);
 const char* launch_scan(const ScanArgs& a, int BH, bool hilo, hipStream_t stream);

@@ -1,4 +1,5 @@
-// Recurrent mLSTM over T tokens in ONE launch: the step of step.hip repeated with the state held on chip.
+// Recurrent mLSTM over T tokens in ONE launch: the step of step.hip repeated with the state held on chip (fp32 inputs and
+// dimensions that step_block.hip does not take).
 //
 //   for t = 0 .. T-1:   m' = max(logsig(f_t) + m, i_t)      f' = exp(logsig(f_t) + m - m')     i' = exp(i_t - m')
 //                       C  = f' C + i' k_t v_t^T             n  = f' n + i' k_t
@@ -360,6 +361,10 @@ const char* launch_step_seq(const void* q, const void* k, const void* v, const v
   if (B <= 0 || NH <= 0 || T <= 0 || DHQK <= 0 || DHHV <= 0) return "mlstm_hip_recurrent_sequence: non-positive dimension";
   if ((long long)B * NH > 65535) return "mlstm_hip_recurrent_sequence: B*NH exceeds 65535";
   if (DHQK > 1024) return "mlstm_hip_recurrent_sequence: DHQK above 1024 does not fit the register-resident state slice";
+  // on the matrix cores where the types and dimensions allow it (step_block.hip), at any token count
+  if (step_block_supported(DHQK, DHHV, dtype_qkv))
+    return launch_step_block({q, k, v, i, f, c_in, n_in, m_in, h, c_out, n_out, m_out, B * NH, T, DHQK, DHHV, eps, dtype_qkv,
+                              dtype_gates, dtype_state}, stream);
 #define MLSTM_SEQ_ARGS q, k, v, i, f, c_in, n_in, m_in, h, c_out, n_out, m_out, B, NH, T, DHQK, DHHV, eps, dtype_qkv, dtype_gates, dtype_state, stream
   // rows per lane x columns per lane: at most 128 state registers per lane
   const bool vec = DHHV % 4 == 0;

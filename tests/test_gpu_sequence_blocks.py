@@ -1,0 +1,36 @@
+"""The recurrence over several tokens on the matrix cores, at the token counts where its blocks of 32 begin and end and at
+the head dimensions where its split changes, against the fp64 oracle.  The sums are fp32-exact, so with fp16 inputs and
+fp32 states the tolerances are those of fp32 arithmetic (the outputs h are rounded once)."""
+import pytest
+import torch
+
+import oracle as O
+from helpers import make_qkvif, rel_norm
+
+pytestmark = pytest.mark.gpu
+
+_DIMS = [(64, 64), (64, 192), (128, 128), (128, 320), (256, 64), (512, 128)]
+
+
+@pytest.mark.parametrize("T", [1, 2, 16, 17, 31, 32, 33, 64, 97])
+@pytest.mark.parametrize("dims", _DIMS, ids=str)
+@pytest.mark.parametrize("dtype,state", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32),
+                                         (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16)], ids=str)
+def test_blocks_of_tokens(T, dims, dtype, state):
+    from mlstm_kernels_amd.torch.recurrent import mlstm_recurrent_sequence__hip
+
+    DQ, DV = dims
+    B, NH = 2, 3
+    print(f"T={T} {DQ}/{DV} {dtype} {state}", flush=True)
+    q, k, v, i, f = make_qkvif(B, NH, T, DQ, DV, seed=T + DQ, dtype=dtype, f_offset=2.0)
+    g = torch.Generator().manual_seed(T)
+    rn = lambda *s: torch.randn(*s, generator=g).to(state)
+    c, n, m = rn(B, NH, DQ, DV), rn(B, NH, DQ), rn(B, NH, 1)
+    d = lambda t: t.double()
+    H_ref, (C_r, n_r, m_r) = O.recurrent_sequence(d(q), d(k), d(v), d(i), d(f), d(c), d(n), d(m))
+    cu = lambda t: t.cuda()
+    H, (C, nn, mm) = mlstm_recurrent_sequence__hip(*map(cu, (q, k, v, i, f, c, n, m)), return_last_states=True, dtype_state=state)
+    out = {torch.bfloat16: 3e-3, torch.float16: 4e-4, torch.float32: 2e-6}
+    assert rel_norm(H, H_ref) < out[dtype]
+    for a, b in ((C, C_r), (nn, n_r), (mm, m_r)):
+        assert rel_norm(a.reshape(b.shape), b) < out[state]
