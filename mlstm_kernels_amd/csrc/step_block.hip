@@ -7,11 +7,11 @@
 //   C'  = b_T C + sum_j k_j (D[T][j] v_j)^T,     n' = b_T n + sum_j D[T][j] k_j
 //
 // What bounded the token-by-token kernel is vector arithmetic: three operations per state element and token.  As products
-// of blocks the same work is a few dozen matrix instructions, and what is left is one pass over the state: measured in bf16
-with fp32 states against the token-by-token kernel (us): B = 16, NH = 8, 256/512: 2 tokens 37 -> 32, 16 tokens 63 -> 34
-(3.9 TB/s of state), 32 tokens 89 -> 38, 128 tokens 250 -> 103; B = 1, 16 tokens: 32 -> 10; 16 x 4 heads of 512/1024, 16
-tokens: 208 -> 62; 64 x 8 heads of 64/128, 128 tokens: 155 -> 50.  Register budgets for three waves a SIMD spill: 32 tokens
-38 -> 47.
+// of blocks the same work is a few dozen matrix instructions, and what is left is one pass over the state: measured in
+// bf16 with fp32 states against the token-by-token kernel (us): B = 16, NH = 8, 256/512: 2 tokens 37 -> 32, 16 tokens
+// 63 -> 34 (3.9 TB/s of state), 32 tokens 89 -> 38, 128 tokens 250 -> 103; B = 1, 16 tokens: 32 -> 10; 16 x 4 heads of
+// 512/1024, 16 tokens: 208 -> 62; 64 x 8 heads of 64/128, 128 tokens: 155 -> 50.  Register budgets for three waves a SIMD
+// spill: 32 tokens 38 -> 47.
 //
 // Arithmetic: as exact as the fp32 recurrence.  q, k and v are exact in bf16 (an fp16 value is the exact sum of two bf16
 // values); the other operand of every product -- the state, the gated scores, the weighted values, all fp32 -- is split
