@@ -416,13 +416,17 @@ PyObject* py_chunkwise(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     for (const Tensor* t : {&q, &k, &v, &i, &f, (const Tensor*)&c0}) grad = grad || (t->defined() && t->requires_grad());
   }
   cfg->needs_bw = grad;
+  // forward-mode tangents go through the node as well, which refuses them: they would be dropped without a word otherwise
+  bool tangents = false;
+  for (const Tensor* t : {&q, &k, &v, &i, &f, (const Tensor*)&c0, (const Tensor*)&n0, (const Tensor*)&m0})
+    tangents = tangents || (t->defined() && t->_fw_grad(/*level=*/0).defined());
   const auto opt = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
   torch::autograd::variable_list out;
   {
     pybind11::gil_scoped_release no_gil;
     // without a gradient to keep anything for there is no node to build
-    out = grad ? ChunkwiseFunction::apply(q, k, v, i, f, opt(c0), opt(n0), opt(m0), cfg)
-               : ChunkwiseFunction::forward(nullptr, q, k, v, i, f, opt(c0), opt(n0), opt(m0), cfg);
+    out = grad || tangents ? ChunkwiseFunction::apply(q, k, v, i, f, opt(c0), opt(n0), opt(m0), cfg)
+                           : ChunkwiseFunction::forward(nullptr, q, k, v, i, f, opt(c0), opt(n0), opt(m0), cfg);
   }
   PyObject* tup = PyTuple_New(4);
   for (size_t x = 0; x < 4; ++x) PyTuple_SET_ITEM(tup, x, x < out.size() ? wrap_or_none(out[x]) : wrap_or_none(Tensor()));
