@@ -16,7 +16,9 @@
 // Arithmetic: as exact as the fp32 recurrence.  q, k and v are exact in bf16 (an fp16 value is the exact sum of two bf16
 // values); the other operand of every product -- the state, the gated scores, the weighted values, all fp32 -- is split
 // into three bf16 parts whose sum carries 24 bits, one matrix instruction each; sums are fp32.  The gate products are
-// formed by successive multiplication like in the recurrence, not from differences of prefix sums.
+// formed by successive multiplication like in the recurrence, not from differences of prefix sums.  A NaN or infinity in a
+// row of k or v would reach the earlier tokens of its block (0 times it is NaN): such a block is taken a token at a time.
+// What it reaches is what it reaches in the recurrence, but an infinity may come out as NaN.
 //
 // Split: a wave owns 64 rows x 64 value columns of the state of one (batch, head), in registers from the first token to
 // the last (64 per lane; lane r of a half holds columns 2 r and 2 r + 1, so rows move in 8-byte pieces of whole 256-byte
@@ -73,6 +75,14 @@ __device__ __forceinline__ void mfma_exact(f32x16& acc, const float* x, const Fr
     mfma32(acc, a, u);
   }
 }
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+// the larger magnitudes, as bit patterns, of two 16-bit values each
+__device__ __forceinline__ u16x2 max_magnitude(u16x2 a, uint4 w) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    a = __builtin_elementwise_max(a, __builtin_bit_cast(u16x2, (&w.x)[e] & 0x7fff7fffu));
+  return a;
+}
 __device__ __forceinline__ float lane_value(float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); }
 }  // namespace
 
@@ -92,7 +102,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* const et = bt + kBlk;                      // [32] exp(-m_t)
   float* const den = et + kBlk;                     // [nw][32] partial denominators
   float* const nvec = den + nw * kBlk;              // [nw][64] n of the wave's rows
-  uint16_t* const Vs = (uint16_t*)(nvec + nw * 64); // [CG][32][kRowS] v rows, even columns first
+  int* const odd = (int*)(nvec + nw * 64);          // [nw] whether the wave's rows hold a value that is not finite
+  uint16_t* const Vs = (uint16_t*)(odd + 8);        // [CG][32][kRowS] v rows, even columns first
   unsigned char* const wave_mem = (unsigned char*)(Vs + CG * kBlk * kRowS);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -112,8 +123,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const size_t c_base = ((size_t)bh * DHQK + row0) * DHHV + col;   // uniform; plus a 32-bit offset per lane
   const uint32_t c_lane = 4 * hh * DHHV + 2 * r;
 
-  auto block = [&](int t0, bool first) __attribute__((always_inline)) {
-    const int nb = min(kBlk, T - t0);
+  // tokens t0 to t0 + nb; false, with nothing done, if they have to be taken one by one (the same in all waves)
+  auto block = [&](int t0, int nb, bool first) __attribute__((always_inline)) {
     const size_t tok = (size_t)bh * T + t0;
     // ---- the block's rows (zeros past the last token): k and v through LDS, q straight into operands
     uint4 kraw[4];
@@ -166,7 +177,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (MULTI && !first) __syncthreads();  // the previous block's tables, rows and sums are no longer read
+    if (!first) __syncthreads();  // the previous block's tables, rows and sums are no longer read
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       uint16_t* const p = Ks + (8 * x + (lane >> 3)) * kRowS + 8 * (lane & 7);
@@ -184,6 +195,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     nw_v[lane] = nreg;
+    {
+      u16x2 big = {0, 0};
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        big = max_magnitude(big, kraw[x]);
+        if (x < max(vn, 1)) big = max_magnitude(big, vraw[x]);
+      }
+      const bool any_odd = __any(max(big.x, big.y) >= (F16 ? 0x7c00 : 0x7f80));
+      if (lane == 0) odd[wave] = any_odd;
+    }
+    float m_next = m;
     // ---- gate tables, by the first wave: lane t holds the gates of token t (past the last token: keep everything, add
     // nothing), then lane j the column j of D
     if (wave == 0) {
@@ -206,9 +228,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (lane < kBlk) Dt[t * kDS + lane] = x;
       }
       if (lane < kBlk) bt[lane] = b_keep;
-      m = mm;
+      m_next = mm;
     }
     __syncthreads();
+    if (nb > 1 && __any(lane < nw && odd[lane < nw ? lane : 0])) return false;
+    m = m_next;
     // Everything below works on columns t = r; those past the last token hold rubbish and are not stored.
     const float* const Dlast = Dt + (nb - 1) * kDS;
     // ---- this wave's part of the scores (rows j, columns t), gated
@@ -343,7 +367,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     // ---- n: lane d of the wave's 64
-    if (MULTI || (id.x == 0 && cg == 0)) {
+    if (MULTI || !first || (id.x == 0 && cg == 0)) {
       float s = 0.f;
       for (int j = 0; j < nb; ++j) s = __builtin_fmaf(Dlast[j], elem_to_f32<F16>(Ks[j * kRowS + lane]), s);
       nreg = __builtin_fmaf(bt[nb - 1], nreg, s);
@@ -358,9 +382,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         *(float4*)(p + 16 * g4 + 4) = make_float4(out[0][4 * g4 + 2], out[1][4 * g4 + 2], out[0][4 * g4 + 3], out[1][4 * g4 + 3]);
       }
     }
+    return true;
   };
-  auto finish = [&](int t0) __attribute__((always_inline)) {  // h of the block: sum over the row groups, divide
-    const int nb = min(kBlk, T - t0);
+  auto finish = [&](int t0, int nb) __attribute__((always_inline)) {  // h of the block: sum over the row groups, divide
     __syncthreads();
     for (int x = rg * 64 + lane; x < nb * 16; x += RG * 64) {
       const int t = x >> 4, c4 = 4 * (x & 15);
@@ -377,13 +401,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
 
-  block(0, true);
-  if constexpr (MULTI) {
-    finish(0);
+  const int nb0 = min(kBlk, T);
+  const bool whole = block(0, nb0, true);
+  if (MULTI || !whole) {
+    if (whole) finish(0, nb0);
+    int singles = whole ? 0 : nb0;  // the token up to which they are taken one by one
 #pragma unroll 1
-    for (int t0 = kBlk; t0 < T; t0 += kBlk) {
-      block(t0, false);
-      finish(t0);
+    for (int t0 = whole ? nb0 : 0; t0 < T;) {
+      const int nb = t0 < singles ? 1 : min(kBlk, T - t0);
+      if (block(t0, nb, false)) {
+        finish(t0, nb);
+        t0 += nb;
+      } else {
+        singles = t0 + nb;
+      }
     }
   }
   // ---- state out (C may be updated in place: this wave read its whole part before)
@@ -397,7 +428,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   if (id.x == 0 && cg == 0) store_state_scalar(n_out, (size_t)bh * DHQK + row0 + lane, SDT, nreg);
   if (id.x == 0 && tid == 0) store_state_scalar(m_out, bh, SDT, m);
-  if constexpr (!MULTI) finish(0);
+  if (!MULTI && whole) finish(0, nb0);
 }
 
 template <bool F16, int SDT, int MODE>
@@ -405,7 +436,7 @@ static const char* launch_step_block_t(const StepBlockArgs& a, hipStream_t strea
   const int RG = a.DHQK / 64, CG = a.DHHV % 128 == 0 && RG <= 2 ? 2 : 1, nw = RG * CG;
   const int rows = a.T < kBlk ? a.T : kBlk;
   const int wave_bytes = kBlk * kRowS * 2 > rows * kOutS * 4 ? kBlk * kRowS * 2 : rows * kOutS * 4;
-  const size_t smem = (size_t)(kBlk * kDS + 2 * kBlk + nw * (kBlk + 64)) * 4 + (size_t)CG * kBlk * kRowS * 2 + (size_t)nw * wave_bytes;
+  const size_t smem = (size_t)(kBlk * kDS + 2 * kBlk + nw * (kBlk + 64) + 8) * 4 + (size_t)CG * kBlk * kRowS * 2 + (size_t)nw * wave_bytes;
   static LdsLimit lds;
   if (!lds.allow((const void*)step_block_kernel<F16, SDT, MODE>, smem)) return "step_block: cannot raise the dynamic LDS limit";
   hipLaunchKernelGGL((step_block_kernel<F16, SDT, MODE>), dim3(a.DHHV / (64 * CG), a.BH), dim3(64 * nw), smem, stream,

@@ -34,3 +34,31 @@ def test_blocks_of_tokens(T, dims, dtype, state):
     assert rel_norm(H, H_ref) < out[dtype]
     for a, b in ((C, C_r), (nn, n_r), (mm, m_r)):
         assert rel_norm(a.reshape(b.shape), b) < out[state]
+
+
+@pytest.mark.parametrize("T", [7, 23, 70])
+@pytest.mark.parametrize("dims", [(64, 128), (256, 64)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_values_that_are_not_finite_reach_no_earlier_token(T, dims, dtype):
+    from mlstm_kernels_amd.torch.recurrent import mlstm_recurrent_sequence__hip
+
+    DQ, DV = dims
+    B, NH = 1, 4
+    print(f"T={T} {DQ}/{DV} {dtype}", flush=True)
+    q, k, v, i, f = make_qkvif(B, NH, T, DQ, DV, seed=T + DQ, dtype=dtype, f_offset=2.0)
+    v[0, 0, T // 2, 3] = float("nan")
+    v[0, 1, T - 2, 5] = float("inf")
+    k[0, 2, T // 3, 7] = float("nan")
+    g = torch.Generator().manual_seed(T)
+    c, n, m = torch.randn(B, NH, DQ, DV, generator=g), torch.randn(B, NH, DQ, generator=g), torch.randn(B, NH, 1, generator=g)
+    d = lambda t: t.double()
+    H_ref, (C_r, n_r, m_r) = O.recurrent_sequence(*map(d, (q, k, v, i, f, c, n, m)))
+    cu = lambda t: t.cuda()
+    H, (C, nn, mm) = mlstm_recurrent_sequence__hip(*map(cu, (q, k, v, i, f, c, n, m)), return_last_states=True)
+    out = {torch.bfloat16: 3e-3, torch.float16: 4e-4}[dtype]
+    for a, b, tol in ((H, H_ref, out), (C, C_r, 2e-6), (nn, n_r, 2e-6), (mm, m_r, 2e-6)):
+        a, b = a.cpu().reshape(b.shape), b
+        fin = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), fin)
+        assert rel_norm(a[fin], b[fin]) < tol
+    assert torch.isfinite(H_ref[0, 0, : T // 2]).all() and not torch.isfinite(H_ref[0, 0, T // 2:]).all()
