@@ -16,7 +16,9 @@
 // the sequence end inside the last chunk get logsig(f) = 0 and it = -inf, i.e. they neither decay nor feed
 // the state, so any sequence length is handled.
 //
-// Two launches, each with one workgroup per (batch, head, group of 16 chunks) so that a small batch still fills
+// Up to 16 chunks (2048 positions) one workgroup takes a head and both halves are one launch: its time is a chain of scans
+// and of memory latencies, and a launch (8 heads of 317 positions 4.0 + 3.4 -> 4.6 us, 128 of 2048 7.6 + 6.7 -> 9.4, and
+// the gap between the two).  Longer sequences take two launches, each with one workgroup per (batch, head, group of 16 chunks) so that a small batch still fills
 // the chip: the first does the within-chunk scans (one wave per chunk); the second scans the (max,+) recurrence of m
 // over ALL chunks of its head with one wave (the recurrence is associative and only NC scalars long, so every
 // workgroup of a head repeats it rather than waiting for a neighbour) and finishes its own chunks elementwise.
@@ -51,23 +53,16 @@ __device__ __forceinline__ float wave_rev_incl_scan(float x, Op op) {
 
 constexpr int kGateChunks = kGateThreads / kWave;  // chunks per workgroup: one wave each
 
-__global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
-    const void* __restrict__ ig, const void* __restrict__ fg, GateBufs gb, int S, int NC, int dtype_gates,
-    int sig_gate) {
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int c = blockIdx.x * kGateChunks + wave;
-  if (c >= NC) return;
-  const size_t Sp = (size_t)NC * kChunk;
-  float* u = gb.u + bh * Sp;          // here: b
-  float* wv = gb.w + bh * Sp;
-  float* abar = gb.abar + bh * Sp;    // here: a
-  float* mcomb = gb.mcomb + bh * Sp;  // here: b + cummax(it - b)
+// Within-chunk scans of one chunk by one wave, two positions per lane.
+struct ChunkScan {
+  float b[2], a[2], cm[2], w[2];  // b; a; b + cummax(it - b); b - it
+  float g, amax;                  // of the whole chunk
+};
+__device__ __forceinline__ ChunkScan scan_chunk(const void* ig, const void* fg, int bh, int c, int lane, int S,
+                                                int dtype_gates, int sig_gate) {
   const float NEG_INF = -__builtin_inff();
   auto add = [](float a, float b) { return a + b; };
   auto mx = [](float a, float b) { return fmaxf(a, b); };
-
-  // within-chunk scans, one wave per chunk, two positions per lane
   const int t0 = c * kChunk + 2 * lane;
   float lf[2], it[2];
 #pragma unroll
@@ -86,7 +81,6 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
   const float pair = lf[0] + lf[1];
   const float incl = wave_incl_scan(pair, add, 0.f);
   const float b1 = incl, b0 = (incl - pair) + lf[0];
-  const float g = __shfl(incl, 63);
   const float rincl = wave_rev_incl_scan(pair, add);
   const float suf1 = rincl - pair, suf0 = suf1 + lf[1];
   const float a0 = suf0 + it[0], a1 = suf1 + it[1];
@@ -95,14 +89,84 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
   float pm_excl = __shfl_up(pm, 1);
   if (lane == 0) pm_excl = NEG_INF;
   const float cm0 = fmaxf(pm_excl, x0), cm1 = pm;
-  const float am = wave_max(fmaxf(a0, a1));
-  *(float2*)(u + t0) = make_float2(b0, b1);
-  *(float2*)(mcomb + t0) = make_float2(b0 + cm0, b1 + cm1);
-  *(float2*)(abar + t0) = make_float2(a0, a1);
-  *(float2*)(wv + t0) = make_float2(b0 - it[0], b1 - it[1]);
+  return {{b0, b1}, {a0, a1}, {b0 + cm0, b1 + cm1}, {b0 - it[0], b1 - it[1]}, __shfl(incl, 63), wave_max(fmaxf(a0, a1))};
+}
+
+__global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
+    const void* __restrict__ ig, const void* __restrict__ fg, GateBufs gb, int S, int NC, int dtype_gates,
+    int sig_gate) {
+  const int bh = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = blockIdx.x * kGateChunks + wave;
+  if (c >= NC) return;
+  const size_t o = bh * ((size_t)NC * kChunk) + c * kChunk + 2 * lane;
+  const ChunkScan x = scan_chunk(ig, fg, bh, c, lane, S, dtype_gates, sig_gate);
+  *(float2*)(gb.u + o) = make_float2(x.b[0], x.b[1]);  // b, a and b + cummax(it - b) for the moment
+  *(float2*)(gb.mcomb + o) = make_float2(x.cm[0], x.cm[1]);
+  *(float2*)(gb.abar + o) = make_float2(x.a[0], x.a[1]);
+  *(float2*)(gb.w + o) = make_float2(x.w[0], x.w[1]);
   if (lane == 0) {
-    gb.graw[(size_t)bh * NC + c] = g;
-    gb.amax[(size_t)bh * NC + c] = am;
+    gb.graw[(size_t)bh * NC + c] = x.g;
+    gb.amax[(size_t)bh * NC + c] = x.amax;
+  }
+}
+
+// Both halves in one launch where one workgroup holds a head (NC <= kGateChunks): a wave keeps the scans of its chunk in
+// registers, the chunks meet in LDS, and every wave repeats the recurrence of m over them (a lane per chunk, the order of
+// gates_finish_kernel).
+__global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
+    const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb,
+    float* __restrict__ m_last, int S, int NC, int dtype_gates, int sig_gate) {
+  __shared__ float gs[kGateChunks], as[kGateChunks];
+  const int bh = blockIdx.y;
+  const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;  // one wave per chunk
+  const float NEG_INF = -__builtin_inff();
+  const float m_init = !sig_gate && m0 != nullptr ? m0[bh] : 0.f;
+  const ChunkScan x = scan_chunk(ig, fg, bh, c, lane, S, dtype_gates, sig_gate);
+  if (lane == 0) {
+    gs[c] = x.g;
+    as[c] = x.amax;
+  }
+  __syncthreads();
+  float mp = 0.f, mn = 0.f;  // m before and after this chunk
+  if (!sig_gate) {
+    float G = lane < NC ? gs[lane < NC ? lane : 0] : 0.f, A = lane < NC ? as[lane < NC ? lane : 0] : NEG_INF;
+#pragma unroll
+    for (int o = 1; o < kGateChunks; o <<= 1) {
+      const float Gp = __shfl_up(G, o), Ap = __shfl_up(A, o);
+      if (lane >= o) {
+        A = fmaxf(Ap + G, A);
+        G = Gp + G;
+      }
+    }
+    const float Gex = c > 0 ? __shfl(G, c - 1) : 0.f, Aex = c > 0 ? __shfl(A, c - 1) : NEG_INF;
+    mp = fmaxf(m_init + Gex, Aex);
+    mn = fmaxf(mp + x.g, x.amax);
+  }
+  const size_t o = bh * ((size_t)NC * kChunk) + c * kChunk + 2 * lane;
+  float u[2], bbar[2], abar[2], mc[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    mc[e] = sig_gate ? 0.f : fmaxf(x.b[e] + mp, x.cm[e]);
+    u[e] = x.b[e] - mc[e];
+    bbar[e] = expf(x.b[e] + mp - mc[e]);
+    abar[e] = expf(x.a[e] - mn);
+  }
+  *(float2*)(gb.u + o) = make_float2(u[0], u[1]);
+  *(float2*)(gb.w + o) = make_float2(x.w[0], x.w[1]);
+  *(float2*)(gb.bbar + o) = make_float2(bbar[0], bbar[1]);
+  *(float2*)(gb.abar + o) = make_float2(abar[0], abar[1]);
+  *(float2*)(gb.mcomb + o) = make_float2(mc[0], mc[1]);
+  if (lane == 0) {
+    const size_t h = (size_t)bh * NC + c;
+    gb.graw[h] = x.g;
+    gb.amax[h] = x.amax;
+    gb.gbar[h] = expf(x.g + mp - mn);
+    gb.mstates[h + bh] = mp;  // NC + 1 of them per head
+    if (c == NC - 1) {
+      gb.mstates[h + bh + 1] = mn;
+      if (m_last != nullptr) m_last[bh] = mn;
+    }
   }
 }
 
@@ -197,6 +261,11 @@ __global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(const float*
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
                          int B, int NH, int S, int dtype_gates, int sig_gate, hipStream_t stream) {
   const int NC = (S + kChunk - 1) / kChunk;
+  if (NC <= kGateChunks) {
+    hipLaunchKernelGGL(gates_whole_kernel, dim3(1, B * NH), dim3(kWave * NC), 0, stream, i, f, m0, gb, m_last, S, NC, dtype_gates,
+                       sig_gate);
+    return nullptr;
+  }
   const dim3 grid((NC + kGateChunks - 1) / kGateChunks, B * NH);
   hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, gb, S, NC, dtype_gates, sig_gate);
   hipLaunchKernelGGL(gates_finish_kernel, grid, dim3(kGateThreads), 0, stream, m0, gb, m_last, NC, sig_gate);

@@ -82,6 +82,12 @@ def test_segmented_scan(B, NH, S, DQ, DV, opt, f_offset):
     _run(S, DQ, DV, B=B, NH=NH, seed=S, f_offset=f_offset, **opt)
 
 
+@pytest.mark.parametrize("S", [2047, 2048, 2049])      # a head's gates in one workgroup up to 2048 positions
+@pytest.mark.parametrize("opt", [dict(), dict(init=True), dict(sig=True, init=True)], ids=["exp", "init", "sig-init"])
+def test_gates_in_one_or_two_launches(S, opt):
+    _run(S, 64, 64, seed=S, **opt)
+
+
 @pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
 def test_padding_adapter_without_padding(S, chunk):
     from mlstm_kernels_amd.torch.backend_module import mLSTMBackend, mLSTMBackendConfig
