@@ -907,7 +907,8 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
   a.seg_phase = 0;
   if (a.DHQK % 64 != 0 || a.DHHV % 64 != 0) return "scan: DHQK and DHHV must be multiples of 64";
   if (a.stride < 1 || a.stride > kMaxStateStride) return "scan: state stride out of range";
-  const bool r128 = a.DHQK % 128 == 0, w128 = a.DHHV % 128 == 0;
+  const bool r128 = a.DHQK % 128 == 0;
+  bool w128 = a.DHHV % 128 == 0;
   // Segments (see the top of the file): as many as fit the chip beside each other, at most eight, of eight chunks or more;
   // with fewer than three the second reading of the sequence costs what the segments gain.  Their states go through the
   // caller's scratch (an output that is written later), which has to hold them.  B = 1, NH = 8, S = 10000, 256/512: one
@@ -922,6 +923,12 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
       a.nseg = (a.NC + a.seg_len - 1) / a.seg_len;
     }
   }
+  // Tiles of half the width where those of both halves still have a CU each: the walk over the chunks is what the launch
+  // takes then, and half the columns make a chunk a quarter shorter (256/512, us, 128 / 64 columns: 8 heads of 317 positions
+  // with the last state 20.5 / 16.1, of 2048 without 33.6 / 26.2; 16 heads of 10000 157 / 118).  With more tiles than CUs
+  // the rows are read twice for nothing (32 heads of 2048: 37.6 / 44.9); half the rows instead gain less (17.5, 26.3, 128).
+  const int ncol = a.DHHV / 128 * (a.DHQK / (r128 ? 128 : 64));
+  if (w128 && a.nseg == 1 && 2ll * BH * ncol <= device_cu_count()) w128 = false;
   auto roles = [&]() -> const char* {
     auto one = [&]() -> const char* {
       if (r128 && w128) return launch_scan_roles_t<128, 128>(a, BH, stream);

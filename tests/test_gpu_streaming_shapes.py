@@ -88,6 +88,25 @@ def test_gates_in_one_or_two_launches(S, opt):
     _run(S, 64, 64, seed=S, **opt)
 
 
+@pytest.mark.parametrize("DQ,DV,BH", [(256, 512, 16), (128, 256, 64), (192, 128, 42)])  # the most heads with half tiles
+@pytest.mark.parametrize("S", [129, 1100])
+def test_width_of_the_scan_tiles(DQ, DV, BH, S):
+    """The tiles of a scan split the state: their width changes no bit of the results."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    print(f"S={S} {DQ}/{DV} {BH}", flush=True)
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(BH + 1, 1, S, DQ, DV, seed=S))
+    dH = torch.randn(BH + 1, 1, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    out = []
+    for n in (BH, BH + 1):
+        leaves = [t[:n].clone().requires_grad_(True) for t in (q, k, v, i, f)]
+        H, last = mlstm_chunkwise__hip_xl_chunk(*leaves, return_last_states=True, any_sequence_length=True)
+        grads = torch.autograd.grad(H, leaves, dH[:n])
+        out.append([t.detach()[:BH] for t in (H, *last, *grads)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
 def test_padding_adapter_without_padding(S, chunk):
     from mlstm_kernels_amd.torch.backend_module import mLSTMBackend, mLSTMBackendConfig
