@@ -792,8 +792,11 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
       uint32_t hi[4];                                                                                            \
       const float sc = scur[yrow + v * YRG];                                                                     \
       _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                                            \
-        const float e0 = lo2<F16>(in[e]) * sc;                                                                   \
-        const float e1 = hi2<F16>(in[e]) * sc;                                                                   \
+        float e0 = lo2<F16>(in[e]) * sc;                                                                         \
+        float e1 = hi2<F16>(in[e]) * sc;                                                                         \
+        /* both runs round the same fp32 products: the product and its conversion to float16 may be fused in */  \
+        /* one of them, and the remainder would then belong to another head */                                   \
+        if constexpr (F16) asm("" : "+v"(e0), "+v"(e1));                                                         \
         hi[e] = pack2<F16>(e0, e1);                                                                              \
         if (rest_) hi[e] = pack2<F16>(e0 - lo2<F16>(hi[e]), e1 - hi2<F16>(hi[e]));                               \
       }                                                                                                          \

@@ -88,15 +88,19 @@ def test_gates_in_one_or_two_launches(S, opt):
     _run(S, 64, 64, seed=S, **opt)
 
 
-@pytest.mark.parametrize("DQ,DV,BH", [(256, 512, 16), (128, 256, 64), (192, 128, 42)])  # the most heads with half tiles
-@pytest.mark.parametrize("S", [129, 1100])
-def test_width_of_the_scan_tiles(DQ, DV, BH, S):
-    """The tiles of a scan split the state: their width changes no bit of the results."""
+# the most heads with half tiles (scan: 16, 42, 64), half items or one column group a workgroup (the others, at one length)
+@pytest.mark.parametrize("DQ,DV,BH", [(256, 512, 16), (192, 128, 42), (128, 256, 64), (256, 512, 14), (256, 512, 64), (256, 1024, 32),
+                                      (512, 1024, 32)])
+@pytest.mark.parametrize("S", [129, 1024, 1100])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
+    """The tiles of the scans and the items of the H / dV kernels split the value columns: their width changes no bit of the
+    results."""
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
 
     print(f"S={S} {DQ}/{DV} {BH}", flush=True)
-    q, k, v, i, f = (t.cuda() for t in make_qkvif(BH + 1, 1, S, DQ, DV, seed=S))
-    dH = torch.randn(BH + 1, 1, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(BH + 1, 1, S, DQ, DV, seed=S, dtype=dtype))
+    dH = torch.randn(BH + 1, 1, S, DV, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
     out = []
     for n in (BH, BH + 1):
         leaves = [t[:n].clone().requires_grad_(True) for t in (q, k, v, i, f)]
