@@ -111,6 +111,12 @@ def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("S", [64, 200])
+def test_stream_path_takes_whole_chunks(S):
+    with pytest.raises(RuntimeError, match="S % 128 == 0"):
+        _run(S, 256, 512, path="stream")
+
+
 @pytest.mark.parametrize("S,chunk", [(1, 64), (65, 64), (200, 128), (1000, 64)])
 def test_padding_adapter_without_padding(S, chunk):
     from mlstm_kernels_amd.torch.backend_module import mLSTMBackend, mLSTMBackendConfig
