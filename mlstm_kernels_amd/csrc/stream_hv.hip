@@ -73,12 +73,17 @@ constexpr float kLog2e = 1.4426950408889634f;
 // NORM (forward, DHHV = 512: a work item then holds complete rows of H): the multi-head layer / rms norm over the value
 // columns is applied when the rows are rounded, as an affine map of the accumulators.
 // RAGGED: S is not a multiple of 128 (at compile time: the clamps and predicated stores cost full chunks 2 %).
-template <bool IS_DV, bool F16, bool NORM, bool RAGGED>
+// CW: value columns of an item, 512 or 256.
+template <bool IS_DV, bool F16, bool NORM, bool RAGGED, int CW>
 __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items, int n_rounds) {
   static_assert(!(IS_DV && NORM), "the head norm belongs to the forward");
+  static_assert(CW == 512 || (CW == 256 && !NORM), "the head norm needs complete rows");
   constexpr int DHQK = 256;
   constexpr int QS = DHQK + 8;   // resident rows [128][DHQK] and score-operand slabs [64][DHQK], fragment order
-  constexpr int VS = 512 + 16;   // value-operand slab: 32 rows x 512 value columns, row-major
+  constexpr int VS = CW + 16;    // value-operand slab: 32 rows x CW value columns, row-major
+  constexpr int MB = CW / 128;   // 32-column blocks of a consumer wave
+  constexpr int NPC = CW / 64;   // 16-byte pieces a producer thread moves of a slab that spans the columns
+  constexpr int VRS = 2048 / CW; // rows of a value-operand slab that the producers move at a time
   constexpr int PSS = 64 + 8;    // gated score block P[n][o]: 128 positions x 64 source positions
   constexpr int SLOT = 64 * QS;  // elements per ring slot (the largest slab kind)
   constexpr int ND = DHQK / 16;
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
   const int G = gridDim.x;
   int vid = blockIdx.x;
   if (G % 8 == 0) vid = (vid % 8) * (G / 8) + vid / 8;  // consecutive ids share an XCD (and its L2)
-  const int NC = a.NC, S = a.S, DHHV = a.DHHV, NCH = DHHV / 512, stride = a.stride;
+  const int NC = a.NC, S = a.S, DHHV = a.DHHV, NCH = DHHV / CW, stride = a.stride;
   const size_t Sp = (size_t)NC * kChunk;
   const int NCS = (NC + stride - 1) / stride;
 
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     const bool whole_ = __builtin_amdgcn_readfirstlane((int)((w_ >> 23) & 1)) == 0;                                  \
     const uint32_t d0_ = w_ & 0xFFFFFu;                                                                              \
     const uint32_t half_ = kind_ == 0 ? 16u : 8u;                                                                    \
-    const uint32_t step_ = kind_ == 0 ? 8 * QS * 2 : (kind_ == 1 ? 4096 : 4 * VS * 2);                               \
+    const uint32_t step_ = kind_ == 0 ? 8 * QS * 2 : (kind_ == 1 ? 4096 : VRS * VS * 2);                               \
     _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) {                                                               \
       *(uint2*)(smem_raw + d0_ + i_ * step_) = make_uint2(fd##E[i_][0], fd##E[i_][1]);                               \
       *(uint2*)(smem_raw + d0_ + i_ * step_ + half_) = make_uint2(fd##E[i_][2], fd##E[i_][3]);                       \
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     const bool whole_ = __builtin_amdgcn_readfirstlane((int)((w_ >> 23) & 1)) == 0;                                  \
     const uint32_t d0_ = w_ & 0xFFFFFu;                                                                              \
     const uint32_t half_ = kind_ == 0 ? 16u : 8u;                                                                    \
-    const uint32_t step_ = kind_ == 0 ? 8 * QS * 2 : (kind_ == 1 ? 4096 : 4 * VS * 2);                               \
+    const uint32_t step_ = kind_ == 0 ? 8 * QS * 2 : (kind_ == 1 ? 4096 : VRS * VS * 2);                               \
     const bool st_ = L >= 3;                                                                                         \
     if (st_ && __builtin_amdgcn_readfirstlane((int)((w_ >> 22) & 1)) && p < 64) {                                    \
       ovec[p] = fa##E[0];                                                                                   \
@@ -214,40 +219,40 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks
         const char* const base = St_b + ((size_t)it.bh * NCS + it.slot) * (size_t)(DHHV / 32) * ND * 1024;
         const uint32_t f0 = pl >> 6;  // fragment of the first piece inside the slab: block f0 / 2, contraction step f0 % 2
-        const uint32_t g0 = (((uint32_t)it.ch * 16 + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
+        const uint32_t g0 = (((uint32_t)it.ch * (CW / 32) + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
         const uint32_t r0 = (kRing0Off + pl * 16) | (1u << 20), r1 = (kRing1Off + pl * 16) | (1u << 20);
-        HV_PROC(1, 8, base, g0, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(2, 8, base, g0 + 1 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(0, 8, base, g0 + 2 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(1, 8, base, g0 + 3 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(2, 8, base, g0 + 4 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(0, 8, base, g0 + 5 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(1, 8, base, g0 + 6 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(2, 8, base, g0 + 7 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(1, NPC, base, g0, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(2, NPC, base, g0 + 1 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(0, NPC, base, g0 + 2 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(1, NPC, base, g0 + 3 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(2, NPC, base, g0 + 4 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(0, NPC, base, g0 + 5 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        HV_PROC(1, NPC, base, g0 + 6 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
+        HV_PROC(2, NPC, base, g0 + 7 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
       }
       {
         const char* const kbase = Xo_b + (size_t)it.bh * S * DHQK * 2;
         const char* const vbase = Xw_b + (size_t)it.bh * S * DHHV * 2;
         const uint32_t kd = row * (QS * 2) + permo;
-        const uint32_t vrow = pl >> 6, vpc = pl & 63;  // rows of 1024 bytes: 64 pieces per row, 4 rows per sweep
+        const uint32_t vrow = pl / (CW / 8), vpc = pl % (CW / 8);  // pieces of 16 bytes: CW / 8 per row, VRS rows per sweep
         const uint32_t vd = (vrow * (VS * 2) + vpc * 16) | (3u << 20);
-        const uint32_t vlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * 1024 + vpc * 16;
+        const uint32_t vlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * (CW * 2) + vpc * 16;
         for (int sci = 0; sci < it.nsc; ++sci) {
           const int sc = it.sc_first + sci * it.sc_step;
           const uint32_t t0 = (uint32_t)(sc * kChunk);
           const size_t gi = (size_t)it.bh * Sp + (size_t)sc * kChunk + (pl & 63);
-          const uint32_t vg = (t0 + vrow) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * 1024 + vpc * 16;
+          const uint32_t vg = (t0 + vrow) * (uint32_t)(DHHV * 2) + (uint32_t)it.ch * (CW * 2) + vpc * 16;
           // (bit 24: the gate-vector entry this thread carries lies past the end of the sequence)
           const uint32_t past0 = !RAGGED || t0 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24, past1 = !RAGGED || t0 + 64 + (pl & 63) < (uint32_t)S ? 0u : 1u << 24;
-          const uint32_t vgs = 4 * (uint32_t)DHHV * 2, vg32 = 32 * (uint32_t)DHHV * 2;
+          const uint32_t vgs = VRS * (uint32_t)DHHV * 2, vg32 = 32 * (uint32_t)DHHV * 2;
           // first half: scores -> slot 0, value rows -> slot 1 and slot 0
           HV_PROC(0, 8, kbase, (t0 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, klim, (kRing0Off + kd) | (1u << 22) | past0, gi)
-          HV_PROC(1, 8, vbase, vg, vgs, vlim, kRing1Off + vd, gown)
-          HV_PROC(2, 8, vbase, vg + vg32, vgs, vlim, kRing0Off + vd, gown)
+          HV_PROC(1, NPC, vbase, vg, vgs, vlim, kRing1Off + vd, gown)
+          HV_PROC(2, NPC, vbase, vg + vg32, vgs, vlim, kRing0Off + vd, gown)
           // second half: the other way round
           HV_PROC(0, 8, kbase, (t0 + 64 + row) * (DHQK * 2) + pc * 16, 8 * DHQK * 2, klim, (kRing1Off + kd) | (1u << 22) | past1, gi + 64)
-          HV_PROC(1, 8, vbase, vg + 2 * vg32, vgs, vlim, kRing0Off + vd, gown)
-          HV_PROC(2, 8, vbase, vg + 3 * vg32, vgs, vlim, kRing1Off + vd, gown)
+          HV_PROC(1, NPC, vbase, vg + 2 * vg32, vgs, vlim, kRing0Off + vd, gown)
+          HV_PROC(2, NPC, vbase, vg + 3 * vg32, vgs, vlim, kRing1Off + vd, gown)
         }
       }
     }
@@ -269,11 +274,11 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     // =========================================================================================== consumer waves
     const int wave = wave_all;
     const int tid = wave * 64 + lane;
-    const int pi = wave & 1, ci = wave >> 1;  // output role: positions 64 pi .., value columns 128 ci .. of the item
+    const int pi = wave & 1, ci = wave >> 1;  // output role: positions 64 pi .., value columns CW / 4 ci .. of the item
     const int pb = wave & 3, kb = wave >> 2;  // score role: position block pb, source block kb of a 64-position half
-    f32x16 acc[4][2], sacc;
+    f32x16 acc[MB][2], sacc;
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -320,7 +325,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                                           \
     __builtin_amdgcn_wave_barrier();                                                                                 \
     uint16_t* const Og = a.Out + ((size_t)prev.bh * S + (size_t)prev.c * kChunk + 64 * pi + 32 * NB) * DHHV +        \
-                         prev.ch * 512 + 128 * ci + 32 * (MB0_);                                                     \
+                         prev.ch * CW + 32 * MB * ci + 32 * (MB0_);                                                     \
     constexpr int VPR = 4 * (NMB_); /* 16-byte vectors per row */                                                    \
     const int rows_left_ = S - (prev.c * kChunk + 64 * pi + 32 * NB);                                                \
     _Pragma("unroll") for (int k = 0; k < 32 * VPR / 64; ++k) {                                                      \
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       // per-item vectors are requested
       float csr[2], nv, cs0r = 0.f, mcr = 0.f, np0 = 0.f, np1 = 0.f, np2 = 0.f;
       __syncthreads();
-      if (have_prev) HV_EPILOGUE(0, 0, 4, Ring0 + wave * (32 * 136))
+      if (have_prev) HV_EPILOGUE(0, 0, MB, Ring0 + wave * (32 * (32 * MB + 8)))
       {
         const int r = opaque(lane) & 31;
         float gsum = 0.f, xs = 1.f;
@@ -375,7 +380,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         }
       }
       __syncthreads();
-      if (have_prev) HV_EPILOGUE(1, 0, 4, Ring0 + wave * (32 * 136))
+      if (have_prev) HV_EPILOGUE(1, 0, MB, Ring0 + wave * (32 * (32 * MB + 8)))
       __syncthreads();
       if (!IS_DV && tid < DHQK) nperm[perm16(tid)] = (np0 + np1) + np2;
       __syncthreads();
@@ -411,7 +416,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         if (si == 0) {
           // (after the dot product above, which runs while no accumulator is live)
 #pragma unroll
-          for (int mb = 0; mb < 4; ++mb)
+          for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -422,14 +427,14 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         const uint16_t* const slab = (si & 1) ? Ring1 : Ring0;
 #pragma unroll
         for (int dsl = 0; dsl < 2; ++dsl) {
-          Frag A[4], B[2];
+          Frag A[MB], B[2];
 #pragma unroll
-          for (int mb = 0; mb < 4; ++mb) A[mb].u = *(const uint4*)(slab + ((4 * ci + mb) * 2 + dsl) * 512 + le * 8);
+          for (int mb = 0; mb < MB; ++mb) A[mb].u = *(const uint4*)(slab + ((MB * ci + mb) * 2 + dsl) * 512 + le * 8);
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb)
             B[nb].u = *(const uint4*)(Ns + (64 * pi + 32 * nb + r) * QS + 16 * (2 * si + dsl) + 8 * h);
 #pragma unroll
-          for (int mb = 0; mb < 4; ++mb)
+          for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
         }
@@ -440,7 +445,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) acc[mb][nb] *= csr[nb];
+        for (int mb = 0; mb < MB; ++mb) acc[mb][nb] *= csr[nb];
       __builtin_amdgcn_sched_barrier(0);
 
       // ---- source chunks (the own chunk last), 64 source positions at a time
@@ -517,10 +522,10 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
             const uint16_t* const slab = ((kh + vi) & 1) ? Ring0 : Ring1;
 #pragma unroll
             for (int k16 = 0; k16 < 2; ++k16) {
-              Frag A[4], B[2];
+              Frag A[MB], B[2];
 #pragma unroll
-              for (int mb = 0; mb < 4; ++mb) {
-                const uint16_t* pp = slab + (16 * k16 + krow) * VS + (128 * ci + 32 * mb + ncol);
+              for (int mb = 0; mb < MB; ++mb) {
+                const uint16_t* pp = slab + (16 * k16 + krow) * VS + (32 * MB * ci + 32 * mb + ncol);
                 A[mb].d[0] = lds_read_tr16(pp);
                 A[mb].d[1] = lds_read_tr16(pp + 4 * VS);
               }
@@ -528,7 +533,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
               for (int nb = 0; nb < 2; ++nb)
                 B[nb].u = *(const uint4*)(Ps + (64 * pi + 32 * nb + r) * PSS + 32 * vi + 16 * k16 + 8 * h);
 #pragma unroll
-              for (int mb = 0; mb < 4; ++mb)
+              for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
             }
@@ -539,7 +544,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
                 for (int nb = 0; nb < 2; ++nb) {
                   float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-                  for (int mb = 0; mb < 4; ++mb)
+                  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                       const float x = acc[mb][nb][i];
@@ -589,9 +594,9 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     }
     if (have_prev) {
       __syncthreads();
-      HV_EPILOGUE(0, 0, 4, Ring0 + wave * (32 * 136))
+      HV_EPILOGUE(0, 0, MB, Ring0 + wave * (32 * (32 * MB + 8)))
       __syncthreads();
-      HV_EPILOGUE(1, 0, 4, Ring0 + wave * (32 * 136))
+      HV_EPILOGUE(1, 0, MB, Ring0 + wave * (32 * (32 * MB + 8)))
     }
 #undef HV_EPILOGUE
   }
@@ -604,12 +609,12 @@ bool stream_hv_supported(const ParHvArgs& a) {
 }
 
 namespace {
-template <bool IS_DV, bool F16, bool NORM, bool RAGGED>
-const char* launch_stream_hv_r(const ParHvArgs& a, int BH, hipStream_t stream) {
+template <bool IS_DV, bool F16, bool NORM, bool RAGGED, int CW>
+const char* launch_stream_hv_c(const ParHvArgs& a, int BH, hipStream_t stream) {
   constexpr int QS = 256 + 8, PSS = 72, SLOT = 64 * QS;
   const size_t smem = (size_t)(128 * QS + 128 * PSS + 2 * SLOT) * 2 +
                       (size_t)(4 * 128 + 128 + 256 + 64 + 64 + 128 + 128 + (NORM ? 8 * 128 : 0)) * 4;
-  const long long n_items = (long long)BH * a.NC * (a.DHHV / 512);
+  const long long n_items = (long long)BH * a.NC * (a.DHHV / CW);
   if (n_items >= (1ll << 31)) return "stream_hv: too many work items";
   if ((size_t)a.S * (size_t)a.DHHV * 2 >= ((size_t)1 << 32)) return "stream_hv: one (batch, head) slab of an input exceeds 4 GiB";
   const int cus = device_cu_count();
@@ -618,10 +623,21 @@ const char* launch_stream_hv_r(const ParHvArgs& a, int BH, hipStream_t stream) {
   if (G >= 8) G -= G % 8;
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
-  if (!lds.allow((const void*)stream_hv_kernel<IS_DV, F16, NORM, RAGGED>, smem))
+  if (!lds.allow((const void*)stream_hv_kernel<IS_DV, F16, NORM, RAGGED, CW>, smem))
     return "stream_hv: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((stream_hv_kernel<IS_DV, F16, NORM, RAGGED>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
+  hipLaunchKernelGGL((stream_hv_kernel<IS_DV, F16, NORM, RAGGED, CW>), dim3(G), dim3(768), smem, stream, a, (int)n_items, n_rounds);
   return nullptr;
+}
+// Items of 256 columns where all of them still have a CU each: an item is then all that a CU does, and with half the columns
+// twelve of its steps (sixteen with two source chunks) move half a slab, for the price of computing the scores twice.
+// Us, 512 / 256 columns: 8 heads of 317 positions H 27.6 / 22.1, dV 25.8 / 20.6, of 2048 30.3 / 24.3 and 27.9 / 23.5 (a CU
+// each to the last one).  Beyond that a CU would take two items of 22 for one of 28.
+template <bool IS_DV, bool F16, bool NORM, bool RAGGED>
+const char* launch_stream_hv_r(const ParHvArgs& a, int BH, hipStream_t stream) {
+  if constexpr (!NORM) {
+    if ((long long)BH * a.NC * (a.DHHV / 256) <= device_cu_count()) return launch_stream_hv_c<IS_DV, F16, NORM, RAGGED, 256>(a, BH, stream);
+  }
+  return launch_stream_hv_c<IS_DV, F16, NORM, RAGGED, 512>(a, BH, stream);
 }
 template <bool IS_DV, bool F16, bool NORM = false>
 const char* launch_stream_hv_t(const ParHvArgs& a, int BH, hipStream_t stream) {
