@@ -540,7 +540,7 @@ const char* launch_window_qk_t(const ParQkArgs& a, int BH, hipStream_t stream) {
   const int cus = device_cu_count();
   if (cus <= 0) return "window_qk: cannot read the number of compute units";
   int G = (int)(n_items < cus ? n_items : cus);
-  if (G >= 8) G -= G % 8;
+  if (n_items > G && G >= 8) G -= G % 8;  // (fewer items than CUs: one each, two rounds otherwise)
   const int n_rounds = (int)((n_items + G - 1) / G);
   static LdsLimit lds;
   if (!lds.allow((const void*)window_qk_kernel<DT, MULTI, RAGGED, F16>, kWqSmem))

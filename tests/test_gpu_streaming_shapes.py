@@ -111,6 +111,11 @@ def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("S,DQ,DV,NH", [(1100, 64, 64, 4), (1100, 128, 128, 2), (300, 256, 512, 5), (700, 256, 512, 26)])
+def test_items_that_are_no_multiple_of_eight(S, DQ, DV, NH):
+    _run(S, DQ, DV, NH=NH, seed=S + NH)
+
+
 @pytest.mark.parametrize("S", [64, 200])
 def test_stream_path_takes_whole_chunks(S):
     with pytest.raises(RuntimeError, match="S % 128 == 0"):
