@@ -77,8 +77,9 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
   const int bh = blk.z, c = blk.y;
-  const int nh = blk.x;                // which half of the chunk's positions
-  const int NG = DHHV / GW;            // column groups, handled one after the other by this workgroup
+  const int nh = blk.x & 1;            // which half of the chunk's positions
+  // column groups, handled one after the other by this workgroup: all of them, or one (launch_par_hv_hn)
+  const int grp_lo = blk.x >> 1, grp_hi = gridDim.x == 2 ? DHHV / GW : grp_lo + 1;
   const size_t Sp = (size_t)NC * kChunk;
   const size_t hofs = bh * Sp;
   const size_t gofs = hofs + (size_t)c * kChunk;
@@ -192,8 +193,8 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
       OR_[e] = (IS_DV && a.use_nrow) ? a.nrow[hofs + (size_t)nx_.sc * kChunk + idx_] : 1.f;                          \
     }                                                                                                                \
   }
-  MLSTM_LOAD_AT(sA, ovA, orA, 0, (Target{sc_first, 0, 0, true}))
-  MLSTM_LOAD_AT(sB, ovB, orB, 0, (Target{sc_first, 0, nslab > 1 ? 1 : 0, nslab > 1}))
+  MLSTM_LOAD_AT(sA, ovA, orA, grp_lo, (Target{sc_first, 0, 0, true}))
+  MLSTM_LOAD_AT(sB, ovB, orB, grp_lo, (Target{sc_first, 0, nslab > 1 ? 1 : 0, nslab > 1}))
   // state fragments of the first contraction steps of the first column tile: requested up front, together with
   // everything else this workgroup needs first, so that all of it costs ONE trip to memory
   const int m_wave = wave * MW;  // first value column of this wave inside a column tile
@@ -211,7 +212,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
       _Pragma("unroll") for (int mb = 0; mb < MB; ++mb)                                                    \
         ring[p][mb].u = MLSTM_STATE_FRAG((col0_) + m_wave + 32 * mb, p);                                   \
   }
-  MLSTM_LOAD_RING(0)
+  MLSTM_LOAD_RING(grp_lo * GW)
   {
     // resident rows: all loads of a batch are issued before the first LDS store (a load-store-load-store loop
     // would pay the memory latency once per iteration)
@@ -349,7 +350,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
     }                                                                                                                \
   }
 
-  for (int grp = 0; grp < NG; ++grp) {
+  for (int grp = grp_lo; grp < grp_hi; ++grp) {
     f32x16 acc[NTG][MB][2];
 #pragma unroll
     for (int tl = 0; tl < NTG; ++tl)
@@ -360,7 +361,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[tl][mb][nb][i] = 0.f;
     // later groups request their first two slabs only now (the first group's travel since the kernel started)
-    if (grp > 0) {
+    if (grp > grp_lo) {
       MLSTM_LOAD_AT(sA, ovA, orA, grp, (Target{sc_first, 0, 0, true}))
       MLSTM_LOAD_AT(sB, ovB, orB, grp, (Target{sc_first, 0, nslab > 1 ? 1 : 0, nslab > 1}))
     }
@@ -465,7 +466,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
               *(uint2*)(Ps + nl * PS + o0) = make_uint2(pack2<F16>(pv[0], pv[1]), pack2<F16>(pv[2], pv[3]));
             }
           }
-          if (!IS_DV && own && grp == 0) {
+          if (!IS_DV && own && grp == grp_lo) {
             const float tot = rsum + __shfl_xor(rsum, 32);
             if (h == 0) rows[u * 32 + r] = tot;  // units above the diagonal publish zero
           }
@@ -473,7 +474,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
       }
 
       // ---- denominators (forward, own chunk = last source chunk, first group only); NTH/64 threads share a row
-      if (!IS_DV && own && grp == 0) {
+      if (!IS_DV && own && grp == grp_lo) {
         __syncthreads();  // row sums visible
         constexpr int TPR = NTH / 64;  // threads per row: 8, 4, 2 or 1
         const int td = opaque(tid);
@@ -505,9 +506,9 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
             iv = 1.f / (nmax + a.eps);
           }
           inv[t] = iv;
-          a.nrow_out[gofs + n0 + t] = nmax;
           const int tg = t_base + n0 + t;
-          if (tg < S) {
+          if (grp == 0) a.nrow_out[gofs + n0 + t] = nmax;
+          if (grp == 0 && tg < S) {
             if (a.n_out != nullptr) a.n_out[(size_t)bh * S + tg] = nmax;
             if (a.m_out != nullptr) a.m_out[(size_t)bh * S + tg] = mcs[t];
           }
@@ -525,7 +526,7 @@ __device__ __forceinline__ void par_hv_body(const ParHvArgs& a, const BlockId bl
     // The next group's first state fragments travel during the epilogue (held across the score and value phases they
     // would cost the registers those need).  Unconditional: after the last group the fragments of that group are
     // requested once more, cache hits nobody waits for; a conditional load would be parked in scratch memory.
-    MLSTM_LOAD_RING(min(grp + 1, NG - 1) * GW)
+    MLSTM_LOAD_RING(min(grp + 1, grp_hi - 1) * GW)
     // ---- optional head norm (forward only; the launcher admits it only when one group spans the whole value
     // dimension, so that this workgroup holds complete rows of H): with x = H_t, y = (x - mean) * rsqrt(var + eps) over
     // the DHHV columns ("layer"), or y = x * rsqrt(mean(x^2) + eps) ("rms").  Statistics in fp32 from the fp32
@@ -647,7 +648,11 @@ static const char* launch_par_hv_hn(const ParHvArgs& a, int BH, hipStream_t stre
   static LdsLimit lds;
   if (!lds.allow((const void*)par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>, smem))
     return "par_hv: cannot raise the dynamic LDS limit";
-  dim3 grid(2, a.NC, BH);
+  // Several column groups go to a workgroup each where those fill no more than the CUs: nothing but the resident rows is
+  // shared between the groups, and the launch takes as long as one workgroup (512/1024, two groups, us, H and
+  // dV: 4 heads of 300 positions 71 / 42 and 69 / 39, of 1100 73 / 45 and 71 / 42).
+  const int NG = a.DHHV / GW;
+  dim3 grid(2ll * NG * a.NC * BH <= device_cu_count() ? 2 * NG : 2, a.NC, BH);
   hipLaunchKernelGGL((par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>), grid, dim3(64 * (WT / MW)), smem, stream, a);
   return nullptr;
 }
