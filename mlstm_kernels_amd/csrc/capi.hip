@@ -81,7 +81,7 @@ const char* check_options(int path, int state_stride, int DHQK, int DHHV) {
 // shape is one it supports; MLSTM_PATH_AUTO: the window kernel where it is faster; otherwise the tiled kernel
 const char* launch_hv(int path, const mlstm::ParHvArgs& a, int BH, bool is_dv, hipStream_t st) {
   // (by request the stream kernels take whole chunks only; MLSTM_PATH_AUTO uses them for ragged lengths as well)
-  if (path == MLSTM_PATH_STREAM && !(mlstm::stream_hv_supported(a) && a.S % mlstm::kChunk == 0))
+  if (path == MLSTM_PATH_STREAM && !(mlstm::stream_hv_supported(a) && a.S % 128 == 0))
     return "the stream kernel path supports DHQK = 256, DHHV % 512 == 0, S % 128 == 0 only (with a head norm: DHHV = 512)";
   if ((path == MLSTM_PATH_STREAM || path == MLSTM_PATH_AUTO) && mlstm::stream_hv_supported(a))
     return mlstm::launch_stream_hv(a, BH, is_dv, st);
