@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 
 #include "layout.h"
 
@@ -30,15 +31,19 @@ inline int device_cu_count() {
   return n;
 }
 // The dynamic LDS limit of one kernel (one object per kernel instantiation): raised when a launch needs more than any
-// launch on that device before it.
+// launch on that device before it.  Raising it is one step with recording it: of two threads with different needs the
+// one with the smaller could otherwise set the limit last and the larger be recorded as allowed for good.
 struct LdsLimit {
   std::atomic<int> bytes[kMaxHostDevices];
+  std::mutex raise;
   bool allow(const void* kernel, size_t need) {
     const int dev = current_device();
     if (dev < 0) return false;
+    if (bytes[dev].load(std::memory_order_acquire) >= (int)need) return true;
+    std::lock_guard<std::mutex> lock(raise);
     if (bytes[dev].load(std::memory_order_relaxed) >= (int)need) return true;
     if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need) != hipSuccess) return false;
-    bytes[dev].store((int)need, std::memory_order_relaxed);
+    bytes[dev].store((int)need, std::memory_order_release);
     return true;
   }
 };
