@@ -520,18 +520,29 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
             const int q16 = (le >> 4) & 1, i16 = le & 15;
             const int krow = 8 * h + (i16 >> 2), ncol = 16 * q16 + 4 * (i16 & 3);
             const uint16_t* const slab = ((kh + vi) & 1) ? Ring0 : Ring1;
+            // The half of the own chunk that the causal mask removes for this wave's positions: P is zero there, and the
+            // rows are taken as zeros too, for zero times a NaN or infinity in one of them would be NaN.  The reads are
+            // left out with them (32 heads of 16384, us, H 448 without the branch, 453 with it, dV 424 either way; zeros
+            // put in after the reads cost another 1 %).
+            const bool dead = own && (IS_DV ? kh == 0 && pi == 1 : kh == 1 && pi == 0);
 #pragma unroll
             for (int k16 = 0; k16 < 2; ++k16) {
               Frag A[MB], B[2];
 #pragma unroll
-              for (int mb = 0; mb < MB; ++mb) {
-                const uint16_t* pp = slab + (16 * k16 + krow) * VS + (32 * MB * ci + 32 * mb + ncol);
-                A[mb].d[0] = lds_read_tr16(pp);
-                A[mb].d[1] = lds_read_tr16(pp + 4 * VS);
-              }
+              for (int mb = 0; mb < MB; ++mb) A[mb].u = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-              for (int nb = 0; nb < 2; ++nb)
-                B[nb].u = *(const uint4*)(Ps + (64 * pi + 32 * nb + r) * PSS + 32 * vi + 16 * k16 + 8 * h);
+              for (int nb = 0; nb < 2; ++nb) B[nb].u = make_uint4(0u, 0u, 0u, 0u);
+              if (!dead) {
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) {
+                  const uint16_t* pp = slab + (16 * k16 + krow) * VS + (32 * MB * ci + 32 * mb + ncol);
+                  A[mb].d[0] = lds_read_tr16(pp);
+                  A[mb].d[1] = lds_read_tr16(pp + 4 * VS);
+                }
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb)
+                  B[nb].u = *(const uint4*)(Ps + (64 * pi + 32 * nb + r) * PSS + 32 * vi + 16 * k16 + 8 * h);
+              }
 #pragma unroll
               for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

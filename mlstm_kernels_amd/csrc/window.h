@@ -50,4 +50,18 @@ __device__ __forceinline__ WinBlocks win_blocks(int wave) {
   }
 }
 
+// Which blocks of P a wave multiplies: those of its position blocks NPG * nb + pg (pg < NPG) that lie on the causal side of
+// the contraction block ob (ahead: contraction over later positions).  Known at compile time except for which waves have it.
+// A block on the other side is left out, operands and all: P holds nothing there, and as an operand of zeros it would turn a
+// NaN or infinity in the rows of block ob into NaN at every position of the window (now: at those of its own 32 at most).
+// Without their matrix instructions and with the loop over the blocks unrolled (us, before / after): H at 128/256 with 262144
+// token-heads 116 / 114, dQ / dK at 256/256 with 131072 135 / 130, at 512/1024 with 32768 199 / 192, at 256/512 with 64 heads of
+// 1000 98 / 94; dV and the small tiles the same.
+enum WinSide { kWinOff, kWinSome, kWinOn };
+constexpr WinSide win_side(bool ahead, int ob, int nb, int NPG) {
+  const int lo = NPG * nb, hi = lo + NPG - 1;
+  if (ahead) return ob >= hi ? kWinOn : (ob < lo ? kWinOff : kWinSome);
+  return ob <= lo ? kWinOn : (ob > hi ? kWinOff : kWinSome);
+}
+
 }  // namespace mlstm

@@ -484,6 +484,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         __builtin_amdgcn_sched_barrier(0);
 
         // ================================================== phase V: Out^T += Xw^T P over the positions of the window
+#pragma unroll
         for (int z = 0; z < NVS; ++z) {
           __syncthreads();
           const unsigned char* const Zs = next_slab();
@@ -508,12 +509,16 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
                 }
 #pragma unroll
               for (int nb = 0; nb < NNB; ++nb) {
+                const WinSide side = win_side(IS_DV, ob, nb, NPG);
+                if (side == kWinOff) continue;
                 const int nbk = NPG * nb + pg;
-                const bool live = IS_DV ? ob >= nbk : ob <= nbk;
-                // (unconditional matrix instructions; a block above the diagonal contributes an operand of zeros)
-                Frag B;
-                B.u = make_uint4(0u, 0u, 0u, 0u);
+                const bool live = side == kWinOn || (IS_DV ? ob >= nbk : ob <= nbk);
+                // (the matrix instructions stay unconditional: accumulators that pass through a branch get copied)
+                Frag Ax[2], B;
+                B.u = Ax[0].u = Ax[1].u = make_uint4(0u, 0u, 0u, 0u);
                 if (live) {
+                  Ax[0] = A[0];
+                  Ax[1] = A[1];
                   if (IS_DV) {
                     const unsigned char* const pbk = smem_raw + kWinPOfs + (ob * (ob + 1) / 2 + nbk) * 2048;
 #pragma unroll
@@ -527,7 +532,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
                   }
                 }
 #pragma unroll
-                for (int mb = 0; mb < 2; ++mb) mfma32<F16>(acc[mb][nb], A[mb], B);
+                for (int mb = 0; mb < 2; ++mb) mfma32<F16>(acc[mb][nb], Ax[mb], B);
               }
             }
           }

@@ -407,6 +407,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 
         // ---- Out^T += Z^T P'^T over the 256 positions of the window, ZROWS rows of Z per slab (Z = K for dQ with
         // P' = P: contraction over the keys j; Z = Q for dK with P' = P^T: contraction over the positions t)
+#pragma unroll
         for (int z = 0; z < NDI; ++z) {
           __syncthreads();
           const unsigned char* const Zs = next_slab();
@@ -431,13 +432,16 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 }
 #pragma unroll
               for (int nb = 0; nb < NNB; ++nb) {
+                const WinSide side = win_side(dk, ob, nb, NPG);
+                if (side == kWinOff) continue;
                 const int nbk = NPG * nb + pg;   // the wave's position block (dQ: t, dK: j)
-                const bool live = dk ? ob >= nbk : ob <= nbk;
-                // (the matrix instructions stay unconditional: accumulators that pass through a branch get copied;
-                // a block above the diagonal contributes an operand of zeros instead)
-                Frag B;
-                B.u = make_uint4(0u, 0u, 0u, 0u);
+                const bool live = side == kWinOn || (dk ? ob >= nbk : ob <= nbk);
+                // (the matrix instructions stay unconditional: accumulators that pass through a branch get copied)
+                Frag Ax[2], B;
+                B.u = Ax[0].u = Ax[1].u = make_uint4(0u, 0u, 0u, 0u);
                 if (live) {
+                  Ax[0] = A[0];
+                  Ax[1] = A[1];
                   if (dk) {
                     // P^T: rows t of block (ob, nbk) are the contraction index -> transposing read
                     const unsigned char* const pb = smem_raw + kWinPOfs + (ob * (ob + 1) / 2 + nbk) * 2048;
@@ -452,7 +456,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                   }
                 }
 #pragma unroll
-                for (int mb = 0; mb < 2; ++mb) mfma32<F16>(acc[mb][nb], A[mb], B);
+                for (int mb = 0; mb < 2; ++mb) mfma32<F16>(acc[mb][nb], Ax[mb], B);
               }
             }
           }
