@@ -9,16 +9,20 @@
 // What bounded the token-by-token kernel is vector arithmetic: three operations per state element and token.  As products
 // of blocks the same work is a few dozen matrix instructions, and what is left is one pass over the state: measured in
 // bf16 with fp32 states against the token-by-token kernel (us): B = 16, NH = 8, 256/512: 2 tokens 37 -> 32, 16 tokens
-// 63 -> 34 (3.9 TB/s of state), 32 tokens 89 -> 38, 128 tokens 250 -> 103; B = 1, 16 tokens: 32 -> 10; 16 x 4 heads of
+// 63 -> 35 (3.8 TB/s of state), 32 tokens 89 -> 39, 128 tokens 250 -> 105; B = 1, 16 tokens: 32 -> 10; 16 x 4 heads of
 // 512/1024, 16 tokens: 208 -> 62; 64 x 8 heads of 64/128, 128 tokens: 155 -> 50.  Register budgets for three waves a SIMD
 // spill: 32 tokens 38 -> 47.
 //
 // Arithmetic: as exact as the fp32 recurrence.  q, k and v are exact in bf16 (an fp16 value is the exact sum of two bf16
 // values); the other operand of every product -- the state, the gated scores, the weighted values, all fp32 -- is split
 // into three bf16 parts whose sum carries 24 bits, one matrix instruction each; sums are fp32.  The gate products are
-// formed by successive multiplication like in the recurrence, not from differences of prefix sums.  A NaN or infinity in a
-// row of k or v would reach the earlier tokens of its block (0 times it is NaN): such a block is taken a token at a time.
-// What it reaches is what it reaches in the recurrence, but an infinity may come out as NaN.
+// formed by successive multiplication like in the recurrence, not from differences of prefix sums.
+// Values that are not finite, or so large that a product or sum of the block form could overflow where the recurrence does
+// not (kHugeRow, kHugeState), do not go through it: zero times them is NaN at the earlier tokens of the block, and the parts
+// of a split infinity are an infinity and a NaN.  Such a block is taken a token at a time in the recurrence's own fp32
+// arithmetic (one_token), whose results are those of step_seq.hip, infinities and NaN included.  Looking costs 1 us of 33 at
+// 16 x 8 heads of 256/512 and 16 tokens (the waves wait for the state before the scores instead of behind them; a barrier
+// of its own behind them costs 2) and 2 of 57 at 64 tokens.
 //
 // Split: a wave owns 64 rows x 64 value columns of the state of one (batch, head), in registers from the first token to
 // the last (64 per lane; lane r of a half holds columns 2 r and 2 r + 1, so rows move in 8-byte pieces of whole 256-byte
@@ -37,6 +41,11 @@ constexpr int kBlk = 32;     // tokens per block
 constexpr int kDS = 36;      // row stride of the table D (floats)
 constexpr int kRowS = 100;   // row stride of the 64-entry K and V rows: plain and transposing reads fall on distinct banks
 constexpr int kOutS = 68;    // row stride of the partial sums (floats)
+// With q, k, v below 2^30 (fp16: finite) and C, n below 2^80 before the first block no sum of their products overflows: a
+// token adds less than 2^60 to the state, so that it needs no second look in later blocks, a score of 64 rows stays below
+// 2^66 and a block's share of h below 2^128 for any number of tokens that memory can hold.
+constexpr uint16_t kHugeRow = 0x4e80;                 // 2^30 in bf16
+constexpr float kHugeState = 1.2089258196146292e24f;  // 2^80
 
 // eight fp32 values -> three bf16 fragments whose sum is the value to 24 bits
 __device__ __forceinline__ void split3(const float* x, Frag& a, Frag& b, Frag& c) {
@@ -102,7 +111,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* const et = bt + kBlk;                      // [32] exp(-m_t)
   float* const den = et + kBlk;                     // [nw][32] partial denominators
   float* const nvec = den + nw * kBlk;              // [nw][64] n of the wave's rows
-  int* const odd = (int*)(nvec + nw * 64);          // [nw] whether the wave's rows hold a value that is not finite
+  int* const odd = (int*)(nvec + nw * 64);          // [nw] whether the wave's rows or state hold a value that is too large or NaN
   uint16_t* const Vs = (uint16_t*)(odd + 8);        // [CG][32][kRowS] v rows, even columns first
   unsigned char* const wave_mem = (unsigned char*)(Vs + CG * kBlk * kRowS);
 
@@ -123,8 +132,42 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const size_t c_base = ((size_t)bh * DHQK + row0) * DHHV + col;   // uniform; plus a 32-bit offset per lane
   const uint32_t c_lane = 4 * hh * DHHV + 2 * r;
 
-  // tokens t0 to t0 + nb; false, with nothing done, if they have to be taken one by one (the same in all waves)
-  auto block = [&](int t0, int nb, bool first) __attribute__((always_inline)) {
+  // the token whose rows and gates stand in the first rows of the tables, as step_seq.hip computes it: vector arithmetic in
+  // fp32 on the state where it lies, this wave's sums over its rows to Ps and den
+  auto one_token = [&](size_t tok, const Frag (&Q)[4]) __attribute__((always_inline)) {
+    const float fa = bt[0], ia = Dt[0];
+    const float v0 = elem_to_f32<F16>(Vs[cg * kBlk * kRowS + r]), v1 = elem_to_f32<F16>(Vs[cg * kBlk * kRowS + 32 + r]);
+    nreg = fa * nreg + ia * elem_to_f32<F16>(Ks[lane]);
+    const float qn = wave_sum(elem_to_f32<F16>(q[tok * DHQK + row0 + lane]) * scale * nreg);
+    float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const uint2 kw = *(const uint2*)(Ks + 32 * b + 8 * g4 + 4 * hh), qw = Q[2 * b + g4 / 2].d[g4 % 2];
+        const float kk[4] = {lo2<F16>(kw.x), hi2<F16>(kw.x), lo2<F16>(kw.y), hi2<F16>(kw.y)};
+        const float qq[4] = {lo2<F16>(qw.x), hi2<F16>(qw.x), lo2<F16>(qw.y), hi2<F16>(qw.y)};
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          float c0 = C[b][0][4 * g4 + x] * fa, c1 = C[b][1][4 * g4 + x] * fa;
+          c0 = __builtin_fmaf(ia * kk[x], v0, c0);
+          c1 = __builtin_fmaf(ia * kk[x], v1, c1);
+          a0 = __builtin_fmaf(qq[x] * scale, c0, a0);
+          a1 = __builtin_fmaf(qq[x] * scale, c1, a1);
+          C[b][0][4 * g4 + x] = c0;
+          C[b][1][4 * g4 + x] = c1;
+        }
+      }
+    a0 += __shfl_xor(a0, 32);
+    a1 += __shfl_xor(a1, 32);
+    asm volatile("" ::: "memory");  // (Ps lies over the K row)
+    if (hh == 0) *(float2*)(Ps + 2 * r) = make_float2(a0, a1);
+    if (lane == 0) den[wave * kBlk] = qn;
+  };
+
+  // tokens t0 to t0 + nb; false, with nothing done, if they have to be taken one by one (the same in all waves).  look: the
+  // state has not been found small yet
+  auto block = [&](int t0, int nb, bool first, bool look) __attribute__((always_inline)) {
     const size_t tok = (size_t)bh * T + t0;
     // ---- the block's rows (zeros past the last token): k and v through LDS, q straight into operands
     uint4 kraw[4];
@@ -195,15 +238,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     nw_v[lane] = nreg;
-    {
+    bool huge;
+    {  // (in front of the tables: the barrier behind them waits for the wave that makes them)
       u16x2 big = {0, 0};
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         big = max_magnitude(big, kraw[x]);
+        big = max_magnitude(big, Q[x].u);
         if (x < max(vn, 1)) big = max_magnitude(big, vraw[x]);
       }
-      const bool any_odd = __any(max(big.x, big.y) >= (F16 ? 0x7c00 : 0x7f80));
-      if (lane == 0) odd[wave] = any_odd;
+      huge = max(big.x, big.y) >= (F16 ? 0x7c00 : kHugeRow);
     }
     float m_next = m;
     // ---- gate tables, by the first wave: lane t holds the gates of token t (past the last token: keep everything, add
@@ -230,8 +274,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (lane < kBlk) bt[lane] = b_keep;
       m_next = mm;
     }
+    if (look) {  // (behind the tables: the state may still be on its way)
+      float top = fabsf(nreg);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          top = __builtin_elementwise_maximum(__builtin_elementwise_maximum(top, fabsf(C[b][0][i])), fabsf(C[b][1][i]));
+      huge |= !(top < kHugeState);
+    }
+    {
+      const bool any_huge = __any(huge);
+      if (lane == 0) odd[wave] = any_huge;
+    }
     __syncthreads();
-    if (nb > 1 && __any(lane < nw && odd[lane < nw ? lane : 0])) return false;
+    if (__any(lane < nw && odd[lane < nw ? lane : 0])) {
+      if (first || nb > 1) return false;
+      m = m_next;
+      one_token(tok, Q);
+      return true;
+    }
     m = m_next;
     // Everything below works on columns t = r; those past the last token hold rubbish and are not stored.
     const float* const Dlast = Dt + (nb - 1) * kDS;
@@ -402,14 +464,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   const int nb0 = min(kBlk, T);
-  const bool whole = block(0, nb0, true);
+  const bool whole = block(0, nb0, true, true);
   if (MULTI || !whole) {
     if (whole) finish(0, nb0);
-    int singles = whole ? 0 : nb0;  // the token up to which they are taken one by one
+    int singles = whole ? 0 : nb0;  // the token up to which they are taken one by one (and the state looked at until then)
 #pragma unroll 1
     for (int t0 = whole ? nb0 : 0; t0 < T;) {
       const int nb = t0 < singles ? 1 : min(kBlk, T - t0);
-      if (block(t0, nb, false)) {
+      if (block(t0, nb, false, singles > 0 && t0 <= singles)) {
         finish(t0, nb);
         t0 += nb;
       } else {

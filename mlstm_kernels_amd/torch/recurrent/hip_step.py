@@ -134,7 +134,8 @@ def mlstm_recurrent_sequence__hip(
     two differences that are stated here rather than hidden: ``return_all_states=True`` (the state after every token,
     native_sequence.py:20,64-83) is not implemented and raises; with a 16-bit ``dtype_state`` the state is rounded
     once per call -- it stays float32 in registers between the tokens -- where the reference's token loop rounds it
-    after every step (the results of that mode are therefore closer to the float32 recurrence, not bit-equal)."""
+    after every step (the results of that mode are therefore closer to the float32 recurrence, not bit-equal).  Infinities,
+    NaN and values that overflow give what the token loop gives: tokens that hold any are computed one by one."""
     if kwargs.pop("return_all_states", False):
         raise NotImplementedError("mlstm_recurrent_sequence__hip does not return the state after every token "
                                   "(return_all_states=True); loop over mlstm_recurrent_step__hip for that")
