@@ -63,7 +63,9 @@ const char* mlstm_hip_last_error(void);
  *   MLSTM_PATH_AUTO  : the fastest one for the shape as measured on MI355X: the streaming H / dV kernels where the
  *                      conditions of MLSTM_PATH_STREAM hold; at state_stride 2 the kernels over windows of two chunks
  *                      that share a kept state (H / dV of the other shapes, dQ / dK of all) where the launch has enough
- *                      windows for them; the kernels of MLSTM_PATH_SPLIT for everything else
+ *                      windows for them; the kernels of MLSTM_PATH_SPLIT for everything else.  The number of windows
+ *                      and heads (batch included) has a part in the choice, and so has the number of CUs: the last bits
+ *                      of a sequence's results may depend on what it is batched with.  With the other paths they do not.
  *   MLSTM_PATH_SPLIT : state scan + chunk-parallel kernel over materialised chunk states
  *   MLSTM_PATH_STREAM: the split form with the chunk-parallel kernels as persistent workgroups whose waves are split
  *                      into producers (global memory -> LDS, several slabs in flight) and consumers (matrix
@@ -178,8 +180,8 @@ int mlstm_hip_chunkwise_fw(const void* q, const void* k, const void* v, const vo
  * of a full-size workspace and calls mlstm_hip_chunkwise_recompute_states, which runs the forward state scan again
  * and writes the chunk states behind them (k, v, c0, dtype_qkv, state_stride as in the forward call; c0 NULL = zero
  * initial state).  The workspace is then what mlstm_hip_chunkwise_bw expects.  The recomputed states equal the
- * forward's bit for bit when the forward returned no last state (c_last NULL) and its scan ran in one piece (it is cut into
- * segments where few heads meet a long sequence; the fp32 states before the rounding then differ in the order of a sum); a forward that returned it carried a
+ * forward's bit for bit when the forward returned no last state (c_last NULL) and its scan ran in one piece (with
+ * MLSTM_PATH_AUTO it is cut into segments where few heads meet a long sequence; the fp32 states before the rounding then differ in the order of a sum); a forward that returned it carried a
  * remainder of the value operand in its late chunks, and the recomputed states of those chunks differ from the
  * forward's by one 16-bit rounding of that operand.
  */

@@ -300,7 +300,9 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   // scale in every chunk: true for the exponential gate (its stabiliser rescales them), not for the sigmoid gate,
   // whose late positions may all be closed while early chunks dominate the state.
   sa.all_remainder = sig;
-  sa.seg = (float*)H;  // H is written after the scan
+  // H is written after the scan.  (Where the caller names the path, the same kernels run whatever a sequence is batched
+  // with, and its results do not depend on the batch: no segments there.)
+  sa.seg = path == MLSTM_PATH_AUTO ? (float*)H : nullptr;
   sa.seg_bytes = (size_t)BH * S * DHHV * 2;
   {
     ProfileScope ps("scan_fw", st);
@@ -473,7 +475,7 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     sa.S = S; sa.NC = NC; sa.DHQK = DHQK; sa.DHHV = DHHV;
     sa.qk_scale = qk_scale; sa.eps = eps;
     sa.backward = 1;
-    sa.seg = (float*)dV;  // dV is written after the scan
+    sa.seg = path == MLSTM_PATH_AUTO ? (float*)dV : nullptr;  // as in the forward; dV is written after the scan
     sa.seg_bytes = (size_t)BH * S * DHHV * 2;
     sa.stride = stride;
     sa.f16 = f16;

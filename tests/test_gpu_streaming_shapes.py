@@ -95,7 +95,8 @@ def test_gates_in_one_or_two_launches(S, opt):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
 def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
     """The tiles of the scans and the items of the H / dV kernels split the value columns: their width changes no bit of the
-    results."""
+    results.  (Window or tiled kernel, and segments of the scan, are chosen by the number of heads too, and do change some:
+    the shapes here are those at which only the widths differ between the two batches.)"""
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
 
     print(f"S={S} {DQ}/{DV} {BH}", flush=True)
@@ -107,6 +108,25 @@ def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
         H, last = mlstm_chunkwise__hip_xl_chunk(*leaves, return_last_states=True, any_sequence_length=True)
         grads = torch.autograd.grad(H, leaves, dH[:n])
         out.append([t.detach()[:BH] for t in (H, *last, *grads)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("path,S,DQ,DV", [("split", 8192, 128, 128), ("stream", 8192, 256, 512), ("split", 8200, 64, 64), ("stream", 256, 256, 512)])
+def test_named_paths_do_not_depend_on_the_batch(path, S, DQ, DV):
+    """With the path named a sequence gets the same bits alone (where the scan of "auto" runs in segments and fewer windows
+    change the kernels it takes) and in a batch."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    n = 100 if DQ < 256 else 40
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(n + 1, 1, S, DQ, DV, seed=S))
+    dH = torch.randn(n + 1, 1, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    out = []
+    for rows in (slice(n, n + 1), slice(0, n + 1)):
+        leaves = [t[rows].clone().requires_grad_(True) for t in (q, k, v, i, f)]
+        H, last = mlstm_chunkwise__hip_xl_chunk(*leaves, return_last_states=True, any_sequence_length=True, kernel_path=path)
+        grads = torch.autograd.grad(H, leaves, dH[rows])
+        out.append([t.detach()[-1] for t in (H, *last, *grads)])
     for a, b in zip(*out):
         assert torch.equal(a, b)
 
