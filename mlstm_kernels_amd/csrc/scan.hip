@@ -101,7 +101,11 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
   constexpr int YV = PS * WT / 8 / NT;
   constexpr int NP = kChunk / PS;        // pieces per chunk
   constexpr int XROWS = NT / (RT / 8);   // rows covered by one sweep of the workgroup over X
+  // The n update is summed in one order whatever the tile's width, so that the width changes no bit: rows j, j + 32, ... first,
+  // then the sums of j and j + 16, then those.  A sweep covers 32 rows (a wave's two sums meet behind LDS) or 16 (in front).
+  constexpr int NSET = 32 / XROWS;
   static_assert(XV >= 1 && YV >= 1 && PS % 16 == 0, "piece too small for this tile");
+  static_assert((XROWS == 32 || XROWS == 16) && XV % NSET == 0, "the sums of n");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* Xs = (uint16_t*)smem_raw;
   uint16_t* Yh = Xs + PS * XS;
@@ -240,7 +244,7 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
       }
       scl[((it + 1) & 1) * kChunk + srow] = sn;
     }
-    float np[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float np[NSET][8] = {};
 #pragma unroll
     for (int v = 0; v < XV; ++v) {
       const int idx = tid + v * NT;
@@ -251,16 +255,20 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
         const float xsc = scur[j];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-          np[2 * p] += xsc * lo2<F16>(in[p]);
-          np[2 * p + 1] += xsc * hi2<F16>(in[p]);
+          np[v % NSET][2 * p] += xsc * lo2<F16>(in[p]);
+          np[v % NSET][2 * p + 1] += xsc * hi2<F16>(in[p]);
         }
       }
     }
     if (do_n) {
-      // thread (row group tid/(RT/8), column vector tid%(RT/8)) holds the sum over its XV rows
+      // thread (row group tid/(RT/8), column vector tid%(RT/8)) holds the sums over its XV rows
+      if constexpr (NSET == 2) {
+#pragma unroll
+        for (int p = 0; p < 8; ++p) np[0][p] += np[1][p];
+      }
       float* dst = npart + (tid / (RT / 8)) * RT + (tid % (RT / 8)) * 8;
-      *(float4*)dst = make_float4(np[0], np[1], np[2], np[3]);
-      *(float4*)(dst + 4) = make_float4(np[4], np[5], np[6], np[7]);
+      *(float4*)dst = make_float4(np[0][0], np[0][1], np[0][2], np[0][3]);
+      *(float4*)(dst + 4) = make_float4(np[0][4], np[0][5], np[0][6], np[0][7]);
     }
 #pragma unroll
     for (int v = 0; v < YV; ++v) {
@@ -368,7 +376,7 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
       }
       float s = 0.f;
 #pragma unroll
-      for (int g2 = 0; g2 < XROWS; ++g2) s += npart[g2 * RT + tid];
+      for (int g2 = 0; g2 < 16; ++g2) s += NSET == 2 ? npart[g2 * RT + tid] : npart[g2 * RT + tid] + npart[(g2 + 16) * RT + tid];
       nval = g * nval + s;
     }
     __syncthreads();

@@ -112,14 +112,15 @@ def test_width_of_the_tiles(DQ, DV, BH, S, dtype):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("path,S,DQ,DV", [("split", 8192, 128, 128), ("stream", 8192, 256, 512), ("split", 8200, 64, 64), ("stream", 256, 256, 512)])
+@pytest.mark.parametrize("path,S,DQ,DV", [("split", 8192, 128, 128), ("stream", 8192, 256, 512), ("split", 8200, 64, 64), ("stream", 256, 256, 512),
+                                          ("split", 1024, 64, 128), ("split", 1100, 192, 256)])
 def test_named_paths_do_not_depend_on_the_batch(path, S, DQ, DV):
     """With the path named a sequence gets the same bits alone (where the scan of "auto" runs in segments and fewer windows
     change the kernels it takes) and in a batch."""
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
 
     n = 100 if DQ < 256 else 40
-    q, k, v, i, f = (t.cuda() for t in make_qkvif(n + 1, 1, S, DQ, DV, seed=S))
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(n + 1, 1, S, DQ, DV, seed=S, f_offset=9.0))
     dH = torch.randn(n + 1, 1, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
     out = []
     for rows in (slice(n, n + 1), slice(0, n + 1)):
