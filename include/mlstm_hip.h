@@ -180,16 +180,24 @@ int mlstm_hip_chunkwise_fw(const void* q, const void* k, const void* v, const vo
  * of a full-size workspace and calls mlstm_hip_chunkwise_recompute_states, which runs the forward state scan again
  * and writes the chunk states behind them (k, v, c0, dtype_qkv, state_stride as in the forward call; c0 NULL = zero
  * initial state).  The workspace is then what mlstm_hip_chunkwise_bw expects.  The recomputed states equal the
- * forward's bit for bit when the forward returned no last state (c_last NULL) and its scan ran in one piece (with
- * MLSTM_PATH_AUTO it is cut into segments where few heads meet a long sequence; the fp32 states before the rounding then differ in the order of a sum); a forward that returned it carried a
+ * forward's bit for bit when the forward returned no last state (c_last NULL); a forward that returned it carried a
  * remainder of the value operand in its late chunks, and the recomputed states of those chunks differ from the
  * forward's by one 16-bit rounding of that operand.
+ * A forward with MLSTM_PATH_AUTO cuts its scan into segments where few heads meet a long sequence, and keeps their fp32
+ * states in H meanwhile.  For equal bits its recomputation takes a scratch buffer of H's size
+ * (mlstm_hip_chunkwise_recompute_states_scratch; the dV that the backward writes next serves), that of a forward with
+ * another path takes none (scratch NULL, or the first form).  Without the scratch the scan runs in one piece, and the fp32
+ * states in front of the rounding differ in the order of a sum.
  */
 size_t mlstm_hip_chunkwise_fw_saved_bytes(int B, int NH, int S, int DHQK, int DHHV);
 int mlstm_hip_chunkwise_recompute_states(const void* k, const void* v, const float* c0,
                                          void* workspace, size_t workspace_bytes,
                                          int B, int NH, int S, int DHQK, int DHHV,
                                          int dtype_qkv, int state_stride, void* stream);
+int mlstm_hip_chunkwise_recompute_states_scratch(const void* k, const void* v, const float* c0,
+                                                 void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes,
+                                                 int B, int NH, int S, int DHQK, int DHHV,
+                                                 int dtype_qkv, int state_stride, void* stream);
 
 /*
  * Backward of the fused head norm: dX = rstd * (dY - mean_D(dY) - Y * mean_D(dY * Y)) for MLSTM_NORM_LAYER,

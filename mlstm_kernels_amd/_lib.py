@@ -31,6 +31,7 @@ _SIGNATURES = {
     "mlstm_hip_chunkwise_fw": (_i, [_vp] * 15 + [_sz, _i] + [_i] * 5 + [_f] + [_i] * 7 + [_f, _vp, _vp] + [_vp]),
     "mlstm_hip_chunkwise_fw_saved_bytes": (_sz, [_i] * 5),
     "mlstm_hip_chunkwise_recompute_states": (_i, [_vp] * 4 + [_sz] + [_i] * 7 + [_vp]),
+    "mlstm_hip_chunkwise_recompute_states_scratch": (_i, [_vp] * 4 + [_sz, _vp, _sz] + [_i] * 7 + [_vp]),
     "mlstm_hip_head_norm_bw": (_i, [_vp] * 4 + [_sz, _i, _i, _i, _vp]),
     "mlstm_hip_chunkwise_fw_noalloc": (_i, [_vp] * 14 + [_i] * 5 + [_f] + [_i] * 4 + [_vp]),
     "mlstm_hip_chunkwise_bw_workspace_bytes": (_sz, [_i] * 6),

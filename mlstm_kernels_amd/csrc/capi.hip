@@ -363,6 +363,13 @@ size_t mlstm_hip_chunkwise_fw_saved_bytes(int B, int NH, int S, int DHQK, int DH
 int mlstm_hip_chunkwise_recompute_states(const void* k, const void* v, const float* c0, void* workspace,
                                          size_t workspace_bytes, int B, int NH, int S, int DHQK, int DHHV,
                                          int dtype_qkv, int state_stride, void* stream) {
+  return mlstm_hip_chunkwise_recompute_states_scratch(k, v, c0, workspace, workspace_bytes, nullptr, 0, B, NH, S, DHQK, DHHV,
+                                                      dtype_qkv, state_stride, stream);
+}
+
+int mlstm_hip_chunkwise_recompute_states_scratch(const void* k, const void* v, const float* c0, void* workspace,
+                                                 size_t workspace_bytes, void* scratch, size_t scratch_bytes, int B, int NH,
+                                                 int S, int DHQK, int DHHV, int dtype_qkv, int state_stride, void* stream) {
   if (!k || !v || !workspace) return fail("mlstm_hip_chunkwise_recompute_states: null pointer argument");
   if (const char* e = check_dims(B, NH, S, DHQK, DHHV)) return fail(e);
   if (const char* e = check_options(MLSTM_PATH_AUTO, state_stride, DHQK, DHHV)) return fail(e);
@@ -386,6 +393,8 @@ int mlstm_hip_chunkwise_recompute_states(const void* k, const void* v, const flo
   sa.backward = 0;
   sa.stride = stride;
   sa.f16 = dtype_qkv == MLSTM_F16;
+  sa.seg = (float*)scratch;
+  sa.seg_bytes = scratch_bytes;
   {
     ProfileScope ps("scan_fw_recompute", st);
     if (const char* e = mlstm::launch_scan(sa, B * NH, /*hilo=*/false, st)) return fail(e);

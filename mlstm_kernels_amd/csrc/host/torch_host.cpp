@@ -328,13 +328,16 @@ class ChunkwiseFunction : public torch::autograd::Function<ChunkwiseFunction> {
     const at::ScalarType kd = q.scalar_type();
     void* const stream = stream_of(dev);
     const size_t bw_bytes = mlstm_hip_chunkwise_bw_workspace_bytes(B, NH, S, DQ, DV, cfg->stride);
-    const Tensor bws = empty({(int64_t)bw_bytes}, at::kByte, dev);
+    const Tensor bws = empty({(int64_t)bw_bytes}, at::kByte, dev), dV = empty(v.sizes(), kd, dev);
     if (cfg->recompute) {
       const size_t full_bytes = mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DQ, DV, 1, cfg->path, cfg->stride);
       Tensor full = empty({(int64_t)full_bytes}, at::kByte, dev);
       full.slice(0, 0, ws.numel()).copy_(ws);
-      check_rc(mlstm_hip_chunkwise_recompute_states(ptr(k), ptr(v), fptr(c0s), ptr(full), full_bytes, B, NH, S, DQ, DV,
-                                                    dtype_code(kd), cfg->stride, stream),
+      // dV is not written yet: it holds the states between the segments, as H did in the forward (on that path)
+      const bool segments = cfg->path == MLSTM_PATH_AUTO;
+      check_rc(mlstm_hip_chunkwise_recompute_states_scratch(ptr(k), ptr(v), fptr(c0s), ptr(full), full_bytes,
+                                                            segments ? ptr(dV) : nullptr, segments ? dV.nbytes() : 0, B, NH, S,
+                                                            DQ, DV, dtype_code(kd), cfg->stride, stream),
                "mlstm_hip_chunkwise_recompute_states");
       ws = full;
     }
@@ -351,7 +354,7 @@ class ChunkwiseFunction : public torch::autograd::Function<ChunkwiseFunction> {
     }
     Tensor dCl;
     if (grads.size() > 1 && grads[1].defined()) dCl = as_dense(grads[1], at::kFloat);
-    const Tensor dQ = empty(q.sizes(), kd, dev), dK = empty(k.sizes(), kd, dev), dV = empty(v.sizes(), kd, dev);
+    const Tensor dQ = empty(q.sizes(), kd, dev), dK = empty(k.sizes(), kd, dev);
     const Tensor dI = empty({B, NH, S}, at::kFloat, dev), dF = empty({B, NH, S}, at::kFloat, dev);
     Tensor dC0;
     if (cfg->has_c0) dC0 = empty({B, NH, DQ, DV}, at::kFloat, dev);

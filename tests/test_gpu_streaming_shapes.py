@@ -82,6 +82,24 @@ def test_segmented_scan(B, NH, S, DQ, DV, opt, f_offset):
     _run(S, DQ, DV, B=B, NH=NH, seed=S, f_offset=f_offset, **opt)
 
 
+@pytest.mark.parametrize("NH,S,DQ,DV", [(1, 8200, 128, 128), (2, 8192, 256, 512), (8, 4100, 256, 512)])
+@pytest.mark.parametrize("path", ["auto", "split"])
+def test_segmented_scan_is_recomputed_in_segments(NH, S, DQ, DV, path):
+    """recompute_states_in_bw: the gradients are bit for bit those of the kept states where no last state is returned, also
+    where the forward's scan ran in segments."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(1, NH, S, DQ, DV, seed=S, f_offset=9.0))   # (states that remember)
+    dH = torch.randn(1, NH, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    grads = []
+    for recompute in (False, True):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v, i, f)]
+        H = mlstm_chunkwise__hip_xl_chunk(*leaves, any_sequence_length=True, kernel_path=path, recompute_states_in_bw=recompute)
+        grads.append((H.detach(), *torch.autograd.grad(H, leaves, dH)))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("S", [2047, 2048, 2049])      # a head's gates in one workgroup up to 2048 positions
 @pytest.mark.parametrize("opt", [dict(), dict(init=True), dict(sig=True, init=True)], ids=["exp", "init", "sig-init"])
 def test_gates_in_one_or_two_launches(S, opt):
