@@ -177,6 +177,7 @@ const char* launch_gates(const void* i, const void* f, const float* m0, const Ga
 const char* launch_scan(const ScanArgs& a, int BH, bool hilo, hipStream_t stream);
 const char* launch_par_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 bool par_hv_head_norm_supported(int DHHV);
+bool par_hv_group_each(const ParHvArgs& a, int BH);  // whether launch_par_hv has a workgroup and a CU for every column group
 // streaming (persistent, producer / consumer waves) form of the same two kernels for the shapes it supports
 bool stream_hv_supported(const ParHvArgs& a);
 const char* launch_stream_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);

@@ -634,6 +634,15 @@ __global__ __launch_bounds__(64 * (WT / MW))
   par_hv_body<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>(a, xcd_block_id());  // the workgroups that share a kept state run on one XCD
 }
 
+// value columns that a workgroup holds at a time
+static int par_hv_group(int DHHV) { return DHHV % 512 == 0 ? 512 : (DHHV % 256 == 0 ? 256 : (DHHV % 128 == 0 ? 128 : 64)); }
+// Several column groups go to a workgroup each where those fill no more than the CUs: nothing but the resident rows is
+// shared between the groups, and the launch takes as long as one workgroup (512/1024, two groups, us, H and
+// dV: 4 heads of 300 positions 71 / 42 and 69 / 39, of 1100 73 / 45 and 71 / 42).
+bool par_hv_group_each(const ParHvArgs& a, int BH) {
+  return 2ll * (a.DHHV / par_hv_group(a.DHHV)) * a.NC * BH <= device_cu_count();
+}
+
 template <int WT, int NTG, bool IS_DV, int PD, int MW, bool HEAD_NORM, bool F16>
 static const char* launch_par_hv_hn(const ParHvArgs& a, int BH, hipStream_t stream) {
   constexpr int GW = WT * NTG;
@@ -648,11 +657,7 @@ static const char* launch_par_hv_hn(const ParHvArgs& a, int BH, hipStream_t stre
   static LdsLimit lds;
   if (!lds.allow((const void*)par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>, smem))
     return "par_hv: cannot raise the dynamic LDS limit";
-  // Several column groups go to a workgroup each where those fill no more than the CUs: nothing but the resident rows is
-  // shared between the groups, and the launch takes as long as one workgroup (512/1024, two groups, us, H and
-  // dV: 4 heads of 300 positions 71 / 42 and 69 / 39, of 1100 73 / 45 and 71 / 42).
-  const int NG = a.DHHV / GW;
-  dim3 grid(2ll * NG * a.NC * BH <= device_cu_count() ? 2 * NG : 2, a.NC, BH);
+  dim3 grid(par_hv_group_each(a, BH) ? 2 * (a.DHHV / GW) : 2, a.NC, BH);
   hipLaunchKernelGGL((par_hv_kernel<WT, NTG, IS_DV, PD, MW, HEAD_NORM, F16>), grid, dim3(64 * (WT / MW)), smem, stream, a);
   return nullptr;
 }
@@ -678,10 +683,12 @@ static const char* launch_par_hv_t(const ParHvArgs& a, int BH, hipStream_t strea
 
 template <bool IS_DV>
 static const char* launch_par_hv_d(const ParHvArgs& a, int BH, hipStream_t stream) {
-  if (a.DHHV % 512 == 0) return launch_par_hv_t<256, 2, IS_DV>(a, BH, stream);
-  if (a.DHHV % 256 == 0) return launch_par_hv_t<256, 1, IS_DV>(a, BH, stream);
-  if (a.DHHV % 128 == 0) return launch_par_hv_t<128, 1, IS_DV>(a, BH, stream);
-  return launch_par_hv_t<64, 1, IS_DV>(a, BH, stream);
+  switch (par_hv_group(a.DHHV)) {
+    case 512: return launch_par_hv_t<256, 2, IS_DV>(a, BH, stream);
+    case 256: return launch_par_hv_t<256, 1, IS_DV>(a, BH, stream);
+    case 128: return launch_par_hv_t<128, 1, IS_DV>(a, BH, stream);
+    default: return launch_par_hv_t<64, 1, IS_DV>(a, BH, stream);
+  }
 }
 
 // one workgroup holds complete rows of H only when a single group of column tiles spans the value dimension

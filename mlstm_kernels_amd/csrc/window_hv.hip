@@ -617,12 +617,17 @@ const char* launch_window_hv_c(const ParHvArgs& a, int BH, bool is_dv, hipStream
 
 // Where the window kernel is the faster one.  Its workgroups are one per CU and walk a window in 10 to 30 steps of one
 // slab, so a launch of few windows leaves CUs idle that the tiled kernel (two workgroups per chunk of 128 positions, all
-// value columns) fills: with groups of 256 columns the two meet at half a window per CU (128/256, us, window / tiled: 23 / 18
-// at 16 windows, 28 / 27 at 128, 34 / 47 at 256).  With groups of 64 and 128 columns the window kernel wins from one
-// window on (64/64: 14 / 27 at 8 windows, 17 / 56 at 256): the tiled kernel has one or two waves per workgroup there.
+// value columns) fills: with groups of 256 columns the two meet at half a window per CU (H, us, window / tiled: 256/256 31 / 25
+// at 64 windows, 32 / 34 at 128, 43 / 65 at 256).  With groups of 64 and 128 columns the window kernel wins from one window on
+// (64/64: 14 / 27 at 8 windows, 17 / 55 at 256; 128/128 18 / 23, 23 / 49): the tiled kernel has one or two waves per workgroup
+// there.  So it does with three groups of 64 (128/192: 26 / 33 at 8, 31 / 160 at 256); with five and more one workgroup's
+// walk through the groups takes longer than the tiled kernel as long as that has a workgroup and a CU for every group of its
+// own (128/384: 39 / 24 at 16 windows, 128/320 35 / 32 at 8, 256/640 76 / 30), and far less once it has not (128/384: 40 / 53
+// at 64, 128/320 35 / 123 at 16).
 bool window_hv_preferred(const ParHvArgs& a, int BH) {
   if (!window_hv_supported(a)) return false;
-  return a.DHHV % 256 != 0 || 2ll * BH * ((a.NC + 1) / 2) >= device_cu_count();
+  if (a.DHHV % 256 == 0) return 2ll * BH * ((a.NC + 1) / 2) >= device_cu_count();
+  return a.DHHV < 320 || !par_hv_group_each(a, BH);
 }
 
 bool window_hv_supported(const ParHvArgs& a) {

@@ -155,6 +155,13 @@ def test_items_that_are_no_multiple_of_eight(S, DQ, DV, NH):
     _run(S, DQ, DV, NH=NH, seed=S + NH)
 
 
+# the tiled kernel with a workgroup for every column group of the most heads that fit the CUs, the window kernel with one more
+@pytest.mark.parametrize("DQ,DV,S,NH", [(128, 384, 200, 21), (64, 320, 390, 6), (64, 448, 129, 9)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_several_column_groups(DQ, DV, S, NH, more):
+    _run(S, DQ, DV, NH=NH + more, seed=S + NH)
+
+
 @pytest.mark.parametrize("S", [64, 200])
 def test_stream_path_takes_whole_chunks(S):
     with pytest.raises(RuntimeError, match="S % 128 == 0"):
