@@ -113,6 +113,7 @@ def _fw_launch(q, k, v, i, f, c0, n0, m0, eps, siging, normalize, want_last, kee
 
 
 def _prep_inputs(q, k, v, i, f, c0, n0, m0, siging, f32_as_f16=False):
+    """Arguments of ``_fw_launch`` from those of the operators (which convert and check in native code themselves)."""
     dev = require_gpu(q, k, v, i, f)
     B, NH, S, DHQK = q.shape
     assert k.shape == (B, NH, S, DHQK), f"k has wrong shape {tuple(k.shape)}"

@@ -48,7 +48,8 @@ def mlstm_recurrent_step__hip_fw(
     **kwargs,
 ):
     """One step.  ``matC_new`` may be ``matC_old`` itself (in-place state update, the step then moves the
-    state through HBM exactly once each way); ``vecN_new``/``scaM_new`` must be distinct buffers."""
+    state through HBM exactly once each way); ``vecN_new``/``scaM_new`` must be distinct buffers.  State outputs have the
+    shapes of the old states: (B, NH, DHQK, DHHV), (B, NH, DHQK), (B, NH, 1); others of the same size are refused."""
     if qk_scale is None and dtype_state in _STATE_CODES:
         # everything as the kernel needs it (the usual case): checked, allocated and launched in native code
         out = (_host or _get_host()).step(matC_old, vecN_old, scaM_old, vecQ, vecK, vecV, scaI, scaF, matC_new, vecN_new,
