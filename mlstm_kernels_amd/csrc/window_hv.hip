@@ -18,9 +18,9 @@
 //   * What bounds it: HBM.  Everything a window needs passes through the CU once, only the rows of O a second time: at
 //     128/256 384 KB in and 128 KB out per window where the tiled kernel moved 285 KB per 64 positions; a score block is
 //     computed once for all value columns of its group's window.
-// Measured on MI355X, H / dV in us, tiled kernel -> this one: 128/256 with 262144 token-heads 190 / 182 -> 134 / 106
-// (3.5 / 4.5 TB/s on operands and results counted once), 128/128 187 / 172 -> 77 / 72, 64/128 119 / 108 -> 63 / 56, 64/64
-// with 524288 417 / 386 -> 95 / 87, 256/256 with 131072 134 / 123 -> 85 / 73, 512/1024 with 32768 167 / 163 -> 117 / 106.
+// Measured on MI355X, H / dV in us, tiled kernel -> this one: 128/256 with 262144 token-heads 170 / 165 -> 119 / 104
+// (3.9 / 4.5 TB/s on operands and results counted once), 128/128 180 / 163 -> 71 / 67, 64/128 113 / 102 -> 57 / 51, 64/64
+// with 524288 404 / 367 -> 88 / 77, 256/256 with 131072 119 / 108 -> 80 / 73, 512/1024 with 32768 142 / 141 -> 108 / 101.
 // At 256/512 the streaming kernel (stream_hv.hip, Q resident: no second reading) is as fast: 137 / 128 against 147 / 131.
 #include "kernels.h"
 #include "window.h"

@@ -29,8 +29,8 @@
 //     memory latency per handful of positions); the rounded results pass through a private 2 KB staging tile per
 //     wave into row order and are stored as full 128-byte lines.
 // Supported: state stride 2, any head dimensions (multiples of 64; DHQK in tiles of 256, 128 or 64, whichever divides it).
-// Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 357 -> 182, 128/128 264 -> 124,
-// 64/128 250 -> 87, 64/64 with 524288 419 -> 129, 512/1024 with 32768 238 -> 209; 256/512 with 524288 1060 -> 810.
+// Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 326 -> 170, 128/128 259 -> 119,
+// 64/128 244 -> 82, 64/64 with 524288 419 -> 119, 512/1024 with 32768 210 -> 191; 256/512 with 524288 1042 -> 780.
 #include <type_traits>
 
 #include "kernels.h"
@@ -562,8 +562,8 @@ const char* launch_window_qk_d(const ParQkArgs& a, int BH, hipStream_t stream) {
 
 // Where the window kernel is the faster one: a window is one workgroup's 26 to 64 steps, so with few windows the tiled
 // kernel's eight or more workgroups per window finish first.  They meet at half a window per CU with tiles of 256 rows
-// (256/512, us, window / tiled: 65 / 39 at 64 windows, 67 / 69 at 128, 100 / 133 at 256), at three eighths with 128
-// (128/256: 34 / 29 at 64, 35 / 50 at 128), and with 64 the window kernel wins from one window on (17 / 25).
+// (256/512, us, window / tiled: 63 / 39 at 64 windows, 65 / 73 at 128, 109 / 135 at 256), at three eighths with 128
+// (128/256: 34 / 29 at 64, 33 / 50 at 128), and with 64 the window kernel wins from one window on (17 / 25).
 bool window_qk_preferred(const ParQkArgs& a, int BH) {
   if (!window_qk_supported(a)) return false;
   const long long windows = (long long)BH * ((a.NC + 1) / 2), cus = device_cu_count();
