@@ -27,6 +27,8 @@
 // Register set and ring slot alternate from step to step and every source chunk has an even number of steps, so both
 // are compile-time constants everywhere.
 // Supported: DHQK = 256, DHHV a multiple of 512 (exactly 512 with a head norm); everything else runs par_hv.hip.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -448,10 +450,10 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         for (int mb = 0; mb < MB; ++mb) acc[mb][nb] *= csr[nb];
       __builtin_amdgcn_sched_barrier(0);
 
-      // ---- source chunks (the own chunk last), 64 source positions at a time
-      for (int sci = 0; sci < it.nsc; ++sci) {
-        const int sc = it.sc_first + sci * it.sc_step;
-        const bool own = sc == c;
+      // ---- source chunks (the own chunk last), 64 source positions at a time.  The own chunk in a copy of its own: the mask,
+      // the row sums and the half that is left out are there only (32 heads of 16384, us, H 454 -> 438, dV 425 -> 416)
+      auto source_chunk = [&](int sc, auto own_tag) __attribute__((always_inline)) {
+        constexpr bool own = decltype(own_tag)::value;
         float gs = 0.f;  // decay between the source chunk and this chunk
         for (int x = (IS_DV ? c : sc); x < (IS_DV ? sc : c); ++x) gs += graw[x];
         // gate exponent of this lane's position; the 1/sqrt(d) of the scores rides in the exponent (lq)
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
             // The half of the own chunk that the causal mask removes for this wave's positions: P is zero there, and the
             // rows are taken as zeros too, for zero times a NaN or infinity in one of them would be NaN.  The reads are
             // left out with them (32 heads of 16384, us, H 448 without the branch, 453 with it, dV 424 either way; zeros
-            // put in after the reads cost another 1 %).
+            // put in after the reads cost another 1 %; both before the own chunk had its copy of the code).
             const bool dead = own && (IS_DV ? kh == 0 && pi == 1 : kh == 1 && pi == 0);
 #pragma unroll
             for (int k16 = 0; k16 < 2; ++k16) {
@@ -599,7 +601,9 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
             }
           }
         }
-      }
+      };
+      for (int sci = 0; sci + 1 < it.nsc; ++sci) source_chunk(it.sc_first + sci * it.sc_step, std::false_type{});
+      source_chunk(c, std::true_type{});
       prev = it;
       have_prev = true;
     }
