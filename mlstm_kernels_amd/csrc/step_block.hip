@@ -19,10 +19,10 @@
 // formed by successive multiplication like in the recurrence, not from differences of prefix sums.
 // Values that are not finite, or so large that a product or sum of the block form could overflow where the recurrence does
 // not (kHugeRow, kHugeState), do not go through it: zero times them is NaN at the earlier tokens of the block, and the parts
-// of a split infinity are an infinity and a NaN.  Such a block is taken a token at a time in the recurrence's own fp32
-// arithmetic (one_token), whose results are those of step_seq.hip, infinities and NaN included.  Looking costs 1 us of 33 at
-// 16 x 8 heads of 256/512 and 16 tokens (the waves wait for the state before the scores instead of behind them; a barrier
-// of its own behind them costs 2) and 2 of 57 at 64 tokens.
+// of a split infinity are an infinity and a NaN.  From such a block on tokens are taken one at a time in the
+// recurrence's own fp32 arithmetic (one_by_one), whose results are those of step_seq.hip, infinities and NaN included.
+// Looking costs 0.4 us of 32 at 16 x 8 heads of 256/512 and 16 tokens and 2 of 98 at 128 (the waves wait for the state in front
+// of the gating instead of behind it; a barrier of its own behind it costs 2 of 32).
 //
 // Split: a wave owns 64 rows x 64 value columns of the state of one (batch, head), in registers from the first token to
 // the last (64 per lane; lane r of a half holds columns 2 r and 2 r + 1, so rows move in 8-byte pieces of whole 256-byte
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* const et = bt + kBlk;                      // [32] exp(-m_t)
   float* const den = et + kBlk;                     // [nw][32] partial denominators
   float* const nvec = den + nw * kBlk;              // [nw][64] n of the wave's rows
-  int* const odd = (int*)(nvec + nw * 64);          // [nw] whether the wave's rows or state hold a value that is too large or NaN
+  int* const odd = (int*)(nvec + nw * 64);          // [nw] whether the wave's rows or its state hold a value that is too large
   uint16_t* const Vs = (uint16_t*)(odd + 8);        // [CG][32][kRowS] v rows, even columns first
   unsigned char* const wave_mem = (unsigned char*)(Vs + CG * kBlk * kRowS);
 
@@ -132,42 +132,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const size_t c_base = ((size_t)bh * DHQK + row0) * DHHV + col;   // uniform; plus a 32-bit offset per lane
   const uint32_t c_lane = 4 * hh * DHHV + 2 * r;
 
-  // the token whose rows and gates stand in the first rows of the tables, as step_seq.hip computes it: vector arithmetic in
-  // fp32 on the state where it lies, this wave's sums over its rows to Ps and den
-  auto one_token = [&](size_t tok, const Frag (&Q)[4]) __attribute__((always_inline)) {
-    const float fa = bt[0], ia = Dt[0];
-    const float v0 = elem_to_f32<F16>(Vs[cg * kBlk * kRowS + r]), v1 = elem_to_f32<F16>(Vs[cg * kBlk * kRowS + 32 + r]);
-    nreg = fa * nreg + ia * elem_to_f32<F16>(Ks[lane]);
-    const float qn = wave_sum(elem_to_f32<F16>(q[tok * DHQK + row0 + lane]) * scale * nreg);
-    float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const uint2 kw = *(const uint2*)(Ks + 32 * b + 8 * g4 + 4 * hh), qw = Q[2 * b + g4 / 2].d[g4 % 2];
-        const float kk[4] = {lo2<F16>(kw.x), hi2<F16>(kw.x), lo2<F16>(kw.y), hi2<F16>(kw.y)};
-        const float qq[4] = {lo2<F16>(qw.x), hi2<F16>(qw.x), lo2<F16>(qw.y), hi2<F16>(qw.y)};
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          float c0 = C[b][0][4 * g4 + x] * fa, c1 = C[b][1][4 * g4 + x] * fa;
-          c0 = __builtin_fmaf(ia * kk[x], v0, c0);
-          c1 = __builtin_fmaf(ia * kk[x], v1, c1);
-          a0 = __builtin_fmaf(qq[x] * scale, c0, a0);
-          a1 = __builtin_fmaf(qq[x] * scale, c1, a1);
-          C[b][0][4 * g4 + x] = c0;
-          C[b][1][4 * g4 + x] = c1;
-        }
-      }
-    a0 += __shfl_xor(a0, 32);
-    a1 += __shfl_xor(a1, 32);
-    asm volatile("" ::: "memory");  // (Ps lies over the K row)
-    if (hh == 0) *(float2*)(Ps + 2 * r) = make_float2(a0, a1);
-    if (lane == 0) den[wave * kBlk] = qn;
-  };
-
-  // tokens t0 to t0 + nb; false, with nothing done, if they have to be taken one by one (the same in all waves).  look: the
-  // state has not been found small yet
-  auto block = [&](int t0, int nb, bool first, bool look) __attribute__((always_inline)) {
+  // tokens t0 to t0 + nb; false, with nothing done, if they have to be taken one by one (the same in all waves)
+  auto block = [&](int t0, int nb, bool first) __attribute__((always_inline)) {
     const size_t tok = (size_t)bh * T + t0;
     // ---- the block's rows (zeros past the last token): k and v through LDS, q straight into operands
     uint4 kraw[4];
@@ -244,7 +210,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         big = max_magnitude(big, kraw[x]);
-        big = max_magnitude(big, Q[x].u);
         if (x < max(vn, 1)) big = max_magnitude(big, vraw[x]);
       }
       huge = max(big.x, big.y) >= (F16 ? 0x7c00 : kHugeRow);
@@ -274,7 +239,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (lane < kBlk) bt[lane] = b_keep;
       m_next = mm;
     }
-    if (look) {  // (behind the tables: the state may still be on its way)
+    // ---- this wave's part of the scores (rows j, columns t) and of q . n, from its own rows alone.  Everything works on
+    // columns t = r; those past the last token hold rubbish and are not stored.
+    f32x16 sc;
+    float qn = 0.f;
+    asm volatile("" ::: "memory");  // (the rows and n were written by this wave)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      Frag A;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        A.d[half] = *(const uint2*)(Ks + r * kRowS + 16 * ks + 8 * half + 4 * hh);
+        const float4 nv = *(const float4*)(nw_v + 16 * ks + 8 * half + 4 * hh);
+        const uint2 w = Q[ks].d[half];
+        qn += lo2<F16>(w.x) * nv.x + hi2<F16>(w.x) * nv.y + lo2<F16>(w.y) * nv.z + hi2<F16>(w.y) * nv.w;
+      }
+      mfma32<F16>(sc, A, Q[ks]);
+    }
+    {  // (q here, where it is needed anyway)
+      u16x2 bq = {0, 0};
+#pragma unroll
+      for (int x = 0; x < 4; ++x) bq = max_magnitude(bq, Q[x].u);
+      huge |= max(bq.x, bq.y) >= (F16 ? 0x7c00 : kHugeRow);
+    }
+    if (first) {  // (behind all that does not need it: the state may still be on its way)
       float top = fabsf(nreg);
 #pragma unroll
       for (int b = 0; b < 2; ++b)
@@ -288,47 +278,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (lane == 0) odd[wave] = any_huge;
     }
     __syncthreads();
-    if (__any(lane < nw && odd[lane < nw ? lane : 0])) {
-      if (first || nb > 1) return false;
-      m = m_next;
-      one_token(tok, Q);
-      return true;
-    }
+    if (__builtin_expect(__any(lane < nw && odd[lane < nw ? lane : 0]), 0)) return false;
     m = m_next;
-    // Everything below works on columns t = r; those past the last token hold rubbish and are not stored.
     const float* const Dlast = Dt + (nb - 1) * kDS;
-    // ---- this wave's part of the scores (rows j, columns t), gated
+    // ---- the scores gated, the wave's part of the denominators
     float P[16];
     {
-      f32x16 s;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        Frag A;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) A.d[half] = *(const uint2*)(Ks + r * kRowS + 16 * ks + 8 * half + 4 * hh);
-        mfma32<F16>(s, A, Q[ks]);
-      }
-      float rsum = 0.f, qn = 0.f;
+      float rsum = 0.f;
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
         const float4 dv = *(const float4*)(Dt + r * kDS + 8 * g4 + 4 * hh);
         const float dd[4] = {dv.x, dv.y, dv.z, dv.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          P[4 * g4 + e] = s[4 * g4 + e] * scale * dd[e];
+          P[4 * g4 + e] = sc[4 * g4 + e] * scale * dd[e];
           rsum += P[4 * g4 + e];
         }
       }
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const float4 nv = *(const float4*)(nw_v + 16 * ks + 8 * half + 4 * hh);
-          const uint2 w = Q[ks].d[half];
-          qn += lo2<F16>(w.x) * nv.x + hi2<F16>(w.x) * nv.y + lo2<F16>(w.y) * nv.z + hi2<F16>(w.y) * nv.w;
-        }
       float dp = __builtin_fmaf(bt[r] * scale, qn, rsum);
       dp += __shfl_xor(dp, 32);
       den[wave * kBlk + r] = dp;
@@ -463,22 +429,67 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
 
-  const int nb0 = min(kBlk, T);
-  const bool whole = block(0, nb0, true, true);
-  if (MULTI || !whole) {
-    if (whole) finish(0, nb0);
-    int singles = whole ? 0 : nb0;  // the token up to which they are taken one by one (and the state looked at until then)
+  // tokens t0 to T one by one, as step_seq.hip computes them: vector arithmetic in fp32 on the state where it lies
+  auto one_by_one = [&](int t0) __attribute__((always_inline)) {
+    if (wave == 0) et[1] = m;  // (the other waves have not followed it)
+    __syncthreads();
+    m = et[1];
 #pragma unroll 1
-    for (int t0 = whole ? nb0 : 0; t0 < T;) {
-      const int nb = t0 < singles ? 1 : min(kBlk, T - t0);
-      if (block(t0, nb, false, singles > 0 && t0 <= singles)) {
-        finish(t0, nb);
-        t0 += nb;
-      } else {
-        singles = t0 + nb;
-      }
+    for (int t = t0; t < T; ++t) {
+      const size_t tok = (size_t)bh * T + t;
+      const float lf = log_sigmoid(load_scalar(fg, tok, dtype_gates)), ii = load_scalar(ig, tok, dtype_gates);
+      const float m_new = fmaxf(lf + m, ii);
+      const float fa = expf(lf + m - m_new), ia = expf(ii - m_new);
+      m = m_new;
+      const uint32_t vw = *(const uint32_t*)(v + tok * DHHV + col + 2 * r);
+      const float v0 = lo2<F16>(vw), v1 = hi2<F16>(vw);
+      const uint16_t* const qt = q + tok * DHQK + row0;
+      const uint16_t* const kt = k + tok * DHQK + row0;
+      nreg = fa * nreg + ia * elem_to_f32<F16>(kt[lane]);
+      const float qn = wave_sum(elem_to_f32<F16>(qt[lane]) * scale * nreg);
+      float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const uint2 kw = *(const uint2*)(kt + 32 * b + 8 * g4 + 4 * hh), qw = *(const uint2*)(qt + 32 * b + 8 * g4 + 4 * hh);
+          const float kk[4] = {lo2<F16>(kw.x), hi2<F16>(kw.x), lo2<F16>(kw.y), hi2<F16>(kw.y)};
+          const float qq[4] = {lo2<F16>(qw.x), hi2<F16>(qw.x), lo2<F16>(qw.y), hi2<F16>(qw.y)};
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            float c0 = C[b][0][4 * g4 + x] * fa, c1 = C[b][1][4 * g4 + x] * fa;
+            c0 = __builtin_fmaf(ia * kk[x], v0, c0);
+            c1 = __builtin_fmaf(ia * kk[x], v1, c1);
+            a0 = __builtin_fmaf(qq[x] * scale, c0, a0);
+            a1 = __builtin_fmaf(qq[x] * scale, c1, a1);
+            C[b][0][4 * g4 + x] = c0;
+            C[b][1][4 * g4 + x] = c1;
+          }
+        }
+      a0 += __shfl_xor(a0, 32);
+      a1 += __shfl_xor(a1, 32);
+      __syncthreads();  // the sums of the token before are no longer read
+      if (hh == 0) *(float2*)(Ps + 2 * r) = make_float2(a0, a1);
+      if (lane == 0) den[wave * kBlk] = qn;
+      if (tid == 0) et[0] = expf(-m_new);
+      finish(t, 1);
+    }
+  };
+
+  const int nb0 = min(kBlk, T);
+  const bool whole = block(0, nb0, true);
+  int t0 = whole ? nb0 : 0;
+  if (MULTI && whole) {
+    finish(0, nb0);
+#pragma unroll 1
+    while (t0 < T) {
+      const int nb = min(kBlk, T - t0);
+      if (!block(t0, nb, false)) break;
+      finish(t0, nb);
+      t0 += nb;
     }
   }
+  if (__builtin_expect(t0 < T, 0)) one_by_one(t0);  // (out of the way of the blocks)
   // ---- state out (C may be updated in place: this wave read its whole part before)
 #pragma unroll
   for (int b = 0; b < 2; ++b)
