@@ -70,7 +70,10 @@ struct ScanArgs {
                           // still weigh in the last state)
   float* seg;             // scratch for the states between segments, of seg_bytes (an output that is written later), or nullptr
   size_t seg_bytes;
+  int skip_zero;          // the readers of `states` know that the one at the start is zero (init = nullptr): it is not written
   // set by the launcher:
+  int n_jobs;             // state tiles * batch * heads * segments
+  int end_c, end_n;       // chunks run for the state (in scan order) and for n
   int part;               // 0 whole sequence; 1 / 2 the two launches of a forward scan that returns the last state
   int n_bh;               // batch * heads
   int nseg, seg_len;      // segments of the sequence, chunks in each (the last one may be shorter)

@@ -455,14 +455,16 @@ __device__ __forceinline__ Frag scan_tr_frag(const uint16_t* tile, int k0, const
 }
 }  // namespace
 
-// What a workgroup of scan_roles_kernel runs: chunks it_lo .. it_hi - 1 in scan order (forward: the chunk index, backward
-// counted from the end), those from it_rep on twice in a row (heads, then remainders of the value rows).  Everything
+// What a workgroup of scan_roles_kernel runs of one job: chunks it_lo .. it_hi - 1 in scan order (forward: the chunk index,
+// backward counted from the end), those from it_rep on twice in a row (heads, then remainders of the value rows).  Everything
 // below is counted in runs p = 0 .. total - 1.  REP = false: nothing runs twice (no last state returned).
 template <bool REP>
 struct ScanRuns {
-  int it_lo, it_hi, it_rep, total;
-  __device__ __forceinline__ ScanRuns(int lo, int hi, int rep) : it_lo(lo), it_hi(hi), it_rep(max(rep, lo)) {
-    total = max(hi - lo, 0) + max(hi - it_rep, 0);
+  int it_lo, it_rep, total;
+  __device__ __forceinline__ void set(int lo, int hi, int rep) {
+    it_lo = lo;
+    it_rep = rep;
+    total = hi - lo + (REP ? hi - rep : 0);
   }
   __device__ __forceinline__ int it(int p) const {  // scan index of run p
     const int q = p - (it_rep - it_lo);
@@ -476,9 +478,50 @@ struct ScanRuns {
     const int q = p - (it_rep - it_lo);
     return !REP || q < 0 || (q & 1);
   }
-  // the decay table in LDS holds kGBlock chunks: refilled before the first run of every kGBlock-th chunk of the workgroup
-  __device__ __forceinline__ bool refill(int p) const { return p > 0 && !rest(p) && ((it(p) - it_lo) & (kGBlock - 1)) == 0; }
 };
+
+// One job of scan_roles_kernel: a state tile of one (batch, head), of one segment of the sequence.  The jobs of a workgroup
+// are worked out once, at its start, and lie in LDS: worked out where they are needed, their divisions and their prefix
+// products would stand five times in the producers' loop and cost it its scalar registers.
+constexpr int kScanRounds = 32;  // jobs of a workgroup at most
+struct ScanJob {
+  int bh, seg, bx, by;
+  int it_lo, it_hi, it_rep;  // see ScanRuns
+  int end;                   // bit 0: the state after this job is the last one; bits 1..: 1 + scan index of the chunk in front
+};                           // of which the state is wanted although the chunk is not run, or 0
+
+// Job of workgroup `vid` in round `round`.  Consecutive workgroups of an XCD take consecutive jobs: all tiles of one (batch,
+// head), which share its K / V rows in the L2.  The assignment rotates by one column of tiles per round, so that the first
+// column's tiles, which carry n and may run a chunk more, do not all fall to the same workgroups.
+template <int RT, int WT, bool REP, bool SEG>
+__device__ __forceinline__ ScanJob scan_decode(const ScanArgs& a, int round, int vid, int lane) {
+  ScanJob job = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int G = (int)gridDim.x, nx = a.DHQK / RT, ny = a.DHHV / WT;
+  const int rot = (int)((vid + (unsigned)round * nx) % (unsigned)G);
+  const long long idx = (long long)round * G + rot;
+  if (idx >= a.n_jobs) return job;
+  job.bx = (int)idx % nx;
+  job.by = ((int)idx / nx) % ny;
+  const int z = (int)idx / (nx * ny);
+  const int nrun = !SEG ? 1 : (a.seg_phase == 1 ? a.nseg - 1 : a.nseg);  // segments this launch runs
+  job.bh = SEG ? z / nrun : z;
+  job.seg = SEG ? z % nrun : 0;
+  // chunks of the whole sequence that this tile runs; forward that returns the last state: the chunks from c_lo on carry the
+  // remainder of the value operand and either run twice here or are left to scan_kernel (the state reached before them is
+  // then handed over in final_out / n_final)
+  int n_all = a.nstates != nullptr && job.by == 0 ? a.end_n : a.end_c, c_lo = a.NC;
+  if (REP) {
+    c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)job.bh * a.NC, a.NC, lane);
+    if (!scan_repeats_late(a.NC, c_lo)) n_all = c_lo;
+  }
+  job.it_lo = SEG ? job.seg * a.seg_len : 0;
+  job.it_hi = max(SEG ? min(job.it_lo + a.seg_len, n_all) : n_all, job.it_lo);
+  job.it_rep = max(min(c_lo, job.it_hi), job.it_lo);
+  const bool is_end = !SEG || (n_all == 0 ? job.seg == 0 : (job.it_lo < n_all && job.it_lo + a.seg_len >= n_all));
+  const bool emit = !REP && n_all < a.NC && (!SEG || (a.seg_phase == 2 && job.it_lo <= n_all && n_all < job.it_lo + a.seg_len));
+  job.end = (is_end ? 1 : 0) | (emit ? (n_all + 1) << 1 : 0);
+  return job;
+}
 
 // Segment states between the two launches of a segmented scan, in the register order of the consumer waves:
 // [(batch * head * (segments - 1) + segment)][tile][consumer wave][8][64 lanes][4], behind them n [..][DHQK].
@@ -494,16 +537,20 @@ __device__ __forceinline__ ScanSeg scan_seg(const ScanArgs& a, int bh, int seg) 
 // The consumer role of the scan kernel (see there).  NDB = 0 or 1: this wave also carries the normaliser vector of the
 // first or second 32 of its 64 state rows, NDB = -1: it does not (copies of the role rather than a branch around matrix
 // instructions, which would make the compiler keep those accumulators in scratch memory).
+// `run`: runs this workgroup has made, `chunk`: chunks it has finished; they select the LDS buffer and the slots of the tables.
 template <int RT, int WT, bool F16, bool REP, bool SEG, int NDB>
 __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t* bufs, const float* gl, const uint16_t* nB,
-                                              int wave, int lane, int bh, int seg, int tile, int d_tile, int w_tile,
-                                              const ScanRuns<REP> runs, bool is_end) {
+                                              int wave, int lane, const ScanJob& job, int& run, int& chunk) {
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;
   constexpr int XELEMS = kChunk * RT, YELEMS = kChunk * WT;
   constexpr int BUF = XELEMS + YELEMS;
   const int DHQK = a.DHQK, DHHV = a.DHHV, NC = a.NC;
-  const int total = runs.total;
+  ScanRuns<REP> runs;
+  runs.set(job.it_lo, job.it_hi, job.it_rep);
+  const int bh = job.bh, seg = job.seg, total = runs.total;
+  const int tile = job.bx + (DHQK / RT) * job.by, d_tile = job.bx * RT, w_tile = job.by * WT;
+  const bool is_end = job.end & 1;
   constexpr bool WITH_N = NDB >= 0;  // (forward only)
   const bool backward = !WITH_N && a.backward;
   const int c_base = backward ? NC - 1 : 0, c_step = backward ? -1 : 1;
@@ -514,27 +561,21 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
   const int wr = wave / WC, wc = wave % WC;
   const int r = lane & 31, h = lane >> 5;
   const int d_wave = d_tile + wr * 64, w_wave = w_tile + wc * 32;
-  f32x16 acc[2];
+  f32x16 acc[2], accn;
 #pragma unroll
-  for (int db = 0; db < 2; ++db)
+  for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = accn[i] = 0.f;
+  if (a.init != nullptr && (!SEG || a.seg_phase != 1)) {
+    const float* const src = a.init + ((size_t)bh * DHQK + d_wave + 4 * h) * DHHV + w_wave + r;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float v0 = 0.f;
-      if (a.init != nullptr && (!SEG || a.seg_phase != 1)) {
-        const int d = d_wave + 32 * db + 8 * (i / 4) + 4 * h + (i % 4);
-        v0 = a.init[((size_t)bh * DHQK + d) * DHHV + w_wave + r];
-      }
-      acc[db][i] = v0;
-    }
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[db][i] = src[(size_t)(32 * db + 8 * (i / 4) + (i % 4)) * DHHV];
+  }
   // normaliser vector: the waves of the first 32 value columns of the first column tile carry it as three partial
-  // columns (lanes r = 0, 1, 2) of one more accumulator pair, see write_n_operand
-  f32x16 accn;
+  // columns (lanes r = 0, 1, 2) of one more accumulator pair, see write_tables
+  if (WITH_N && a.n_init != nullptr && (!SEG || a.seg_phase != 1) && r == 0) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float v0 = 0.f;
-    if (WITH_N && a.n_init != nullptr && (!SEG || a.seg_phase != 1) && r == 0)
-      v0 = a.n_init[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)];
-    accn[i] = v0;
+    for (int i = 0; i < 16; ++i) accn[i] = a.n_init[(size_t)bh * DHQK + d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)];
   }
   const size_t seg_ofs = ((size_t)tile * NWC + wave) * 2048 + lane * 4;
   if (SEG && a.seg_phase == 2) {
@@ -557,10 +598,13 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
           for (int e = 0; e < 4; ++e) acc[db][4 * g4 + e] = acc[db][4 * g4 + e] * dec + v[e];
         }
       if (WITH_N) {
+        // (four values a load, of all lanes: one at a time under r == 0 they were sixteen trips to memory in a row)
+        const float* const nsrc = ss.n + d_wave + 32 * DB + 4 * h;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float v = r == 0 ? ss.n[d_wave + 32 * DB + 8 * (i / 4) + 4 * h + (i % 4)] : 0.f;
-          accn[i] = accn[i] * dec + v;
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 v = *(const f32x4*)(nsrc + 8 * g4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) accn[4 * g4 + e] = accn[4 * g4 + e] * dec + (r == 0 ? v[e] : 0.f);
         }
       }
     }
@@ -568,36 +612,47 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
   const ScanTrOff offA0 = scan_tr_offsets<RT>(wr * 64, lane);
   const ScanTrOff offA1 = scan_tr_offsets<RT>(wr * 64 + 32, lane);
   const ScanTrOff offB = scan_tr_offsets<WT>(wc * 32, lane);
-  __syncthreads();  // the producers' prologue barrier
+  // ---- the state before chunk `it` as operand fragments, at the kept boundaries only: forward the state before every
+  // stride-th chunk, backward the gradient of the state after the last chunk of every group of `stride` chunks (and after
+  // the last chunk of the sequence); slot c / stride either way.  A state known to be zero is not written if nobody reads it.
+  auto emit_state = [&](int it) __attribute__((always_inline)) {
+    const int c = c_base + it * c_step;
+    const bool keep = (!SEG || a.seg_phase != 1) && (backward ? (c == NC - 1 || st_pos == a.stride - 1) : st_pos == 0) &&
+                      !(it == 0 && a.skip_zero && a.init == nullptr);
+    if (keep) {
+      const size_t ND = DHQK / 16, NWB = DHHV / 32;
+      const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
+      u32x4* st = (u32x4*)a.states + ((size_t)bh * NCS + st_slot) * NWB * ND * 64;
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        const size_t W32 = w_wave / 32, D16 = (d_wave + 32 * db) / 16;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          u32x4 f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f[e] = pack2<F16>(acc[db][8 * half + 2 * e], acc[db][8 * half + 2 * e + 1]);
+          // non-temporal: the fragments are read by a later kernel; kept out of the L2 they do not evict the K/V
+          // rows the tiles of a head share
+          __builtin_nontemporal_store(f, st + (W32 * ND + D16 + half) * 64 + lane);
+        }
+      }
+    }
+  };
+  // ---- n before chunk `it`, as its three partial vectors [3][DHQK] (the consumer of the states adds them up)
+  auto emit_n = [&](int it) __attribute__((always_inline)) {
+    if (r < 3 && (!SEG || a.seg_phase != 1)) {
+      float* dst = a.nstates + (((size_t)bh * NC + it) * 3 + r) * DHQK + d_wave + 32 * DB + 4 * h;
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *(float4*)(dst + 8 * g4) = make_float4(accn[4 * g4], accn[4 * g4 + 1], accn[4 * g4 + 2], accn[4 * g4 + 3]);
+    }
+  };
   for (int p = 0; p < total; ++p) {
     const int it = runs.it(p);
     const bool rest = runs.rest(p);
-    const int c = c_base + it * c_step;
-    if (runs.refill(p)) __syncthreads();
     __syncthreads();  // run p staged by the producers
     if (!rest) {
-      // ---- the state before this chunk's update as operand fragments, at the kept boundaries only: forward the
-      // state before every stride-th chunk, backward the gradient of the state after the last chunk of every group
-      // of `stride` chunks (and after the last chunk of the sequence); slot c / stride either way
-      const bool keep = (!SEG || a.seg_phase != 1) && (backward ? (c == NC - 1 || st_pos == a.stride - 1) : st_pos == 0);
-      if (keep) {
-        const size_t ND = DHQK / 16, NWB = DHHV / 32;
-        const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
-        u32x4* st = (u32x4*)a.states + ((size_t)bh * NCS + st_slot) * NWB * ND * 64;
-#pragma unroll
-        for (int db = 0; db < 2; ++db) {
-          const size_t W32 = w_wave / 32, D16 = (d_wave + 32 * db) / 16;
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            u32x4 f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = pack2<F16>(acc[db][8 * half + 2 * e], acc[db][8 * half + 2 * e + 1]);
-            // non-temporal: the fragments are read by a later kernel; kept out of the L2 they do not evict the K/V
-            // rows the tiles of a head share
-            __builtin_nontemporal_store(f, st + (W32 * ND + D16 + half) * 64 + lane);
-          }
-        }
-      }
+      emit_state(it);
       st_pos += c_step;
       if (st_pos == a.stride) {
         st_pos = 0;
@@ -606,24 +661,18 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
         st_pos = a.stride - 1;
         --st_slot;
       }
-      const float g = gl[(it - runs.it_lo) & (kGBlock - 1)];
+      const float g = gl[chunk & 3];
       acc[0] *= g;
       acc[1] *= g;
       if (WITH_N) {
-        // n before this chunk, as its three partial vectors [3][DHQK] (the consumer of the states adds them up)
-        if (r < 3 && (!SEG || a.seg_phase != 1)) {
-          float* dst = a.nstates + (((size_t)bh * NC + c) * 3 + r) * DHQK + d_wave + 32 * DB + 4 * h;
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4)
-            *(float4*)(dst + 8 * g4) = make_float4(accn[4 * g4], accn[4 * g4 + 1], accn[4 * g4 + 2], accn[4 * g4 + 3]);
-        }
+        emit_n(it);
         accn *= g;
       }
     }
     // ---- accumulate X^T (scale . Y) over the positions of the chunk
-    const uint16_t* Xs = bufs + (p & 1) * BUF;
+    const uint16_t* Xs = bufs + (run & 1) * BUF;
     const uint16_t* Yh = Xs + XELEMS;
-    const uint16_t* nBp = nB + (it % 3) * (kChunk * 3) + h * 24 + min(r, 2) * 8;
+    const uint16_t* nBp = nB + (chunk % 3) * (kChunk * 3) + h * 24 + min(r, 2) * 8;
 #pragma unroll
     for (int js = 0; js < kChunk / 16; ++js) {
       const Frag A0 = scan_tr_frag<RT>(Xs, 16 * js, offA0), A1 = scan_tr_frag<RT>(Xs, 16 * js, offA1);
@@ -638,6 +687,12 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
         mfma32<F16>(accn, DB == 0 ? A0 : A1, Bn);
       }
     }
+    ++run;
+    if (runs.last(p)) ++chunk;
+  }
+  if (job.end >> 1) {
+    emit_state((job.end >> 1) - 1);
+    if (WITH_N) emit_n((job.end >> 1) - 1);
   }
   if (SEG && a.seg_phase == 1) {
     const ScanSeg ss = scan_seg(a, bh, seg);
@@ -678,8 +733,15 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 // next, keep the normaliser operand and the scale table.  The two instruction streams of a SIMD that limit each other
 // when every wave does everything (conversion arithmetic against matrix instructions) then belong to different waves
 // and overlap; four waves per SIMD instead of two.
-template <int RT, int WT, bool F16, bool REP, bool SEG>
-__global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel(ScanArgs a) {
+//
+// The workgroups are persistent (MANY; a launch of no more jobs than fit the chip keeps the plain form, whose loop has no
+// cursors): one workgroup fills a CU, and a tile of eight chunks spent a third of its time on filling the pipeline and on
+// its last stores with the CU otherwise idle.  Now the next tile's rows are on their way meanwhile.  Without a last state the
+// chunks behind the last kept boundary (in front of the first one) are not run: only n, for its own tiles, is wanted there.
+// Both together, us for a forward and backward call: 128 heads of 1024, 256/512, with layer norm 729 -> 665, 64 heads of 1000
+// 330 -> 302, 128 heads of 2048, 128/256 500 -> 487; 128 heads of 2048 with the last state, forward 418 -> 416.
+template <int RT, int WT, bool F16, bool REP, bool SEG, bool MANY>
+__global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel(ScanArgs a, int n_rounds) {
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;     // consumer waves (and as many producer waves)
   constexpr int NTP = 64 * NWC;           // producer threads
@@ -693,61 +755,116 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
   static_assert(XV >= 1 && YV >= 1 && XRG % 4 == 0 && YRG % 4 == 0, "tile shape does not fit the staging pattern");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   uint16_t* bufs = (uint16_t*)smem_raw;                 // [2][X | Y]
-  float* gl = (float*)(bufs + 2 * BUF);                 // [kGBlock] decay factors of the next chunks, in scan order
-  float* scl = gl + kGBlock;                            // [2][128] row scales, by chunk parity
+  float* gl = (float*)(bufs + 2 * BUF);                 // [4] decay factors, by chunk of this workgroup
+  float* scl = gl + 4;                                  // [2][128] row scales, likewise
   uint16_t* nB = (uint16_t*)(scl + 2 * kChunk);         // [3][128 / 8][3][8] the row scales as a matrix operand (below)
+  ScanJob* jobs = (ScanJob*)(nB + 3 * kChunk * 3);      // [kScanRounds]
 
   // the wave index is made scalar so that branches on it are scalar branches
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const bool producer = wave_all < NWC;
   const int wave = producer ? wave_all : wave_all - NWC;
   const int tid = wave * 64 + lane;                     // index inside the own group of waves
-  const BlockId blk = xcd_block_id();  // all tiles of one (batch, head) on one XCD: they share its K/V rows in the L2
-  const int nrun = !SEG ? 1 : (a.seg_phase == 1 ? a.nseg - 1 : a.nseg);  // segments this launch runs
-  const int bh = SEG ? blk.z / nrun : blk.z, seg = SEG ? blk.z % nrun : 0;
-  const int d_tile = blk.x * RT, w_tile = blk.y * WT;
-  const int DHQK = a.DHQK, DHHV = a.DHHV, S = a.S, NC = a.NC;
-  const size_t Sp = (size_t)NC * kChunk;
-  // forward that returns the last state: the chunks from c_lo on carry the remainder of the value operand and either run
-  // twice here or are left to scan_kernel (the state reached before them is then handed over in final_out / n_final)
-  int n_all = NC, c_lo = NC;
-  if (REP) {
-    c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
-    if (!scan_repeats_late(NC, c_lo)) n_all = c_lo;
+  const int G = gridDim.x;
+  int vid = blockIdx.x;
+  if (G % 8 == 0) vid = (vid % 8) * (G / 8) + vid / 8;  // consecutive ids share an XCD (and its L2)
+  ScanJob job0 = {0, 0, 0, 0, 0, 0, 0, 0};  // !MANY: the only one
+  if constexpr (MANY) {
+    for (int rd = wave_all; rd < n_rounds; rd += 2 * NWC) {
+      const ScanJob job = scan_decode<RT, WT, REP, SEG>(a, rd, vid, lane);
+      if (lane == 0) jobs[rd] = job;
+    }
+    __syncthreads();
+  } else {
+    job0 = scan_decode<RT, WT, REP, SEG>(a, 0, vid, lane);
   }
-  const int it_lo = SEG ? seg * a.seg_len : 0;
-  const ScanRuns<REP> runs(it_lo, SEG ? min(it_lo + a.seg_len, n_all) : n_all, min(c_lo, n_all));
-  // the segment whose state is the last one
-  const bool is_end = !SEG || (n_all == 0 ? seg == 0 : (it_lo < n_all && it_lo + a.seg_len >= n_all));
-  if (SEG && a.seg_phase == 2 && it_lo >= n_all && !is_end) return;
-  const int total = runs.total;
-  const int c_base = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
-  auto chunk_of = [&](int it) { return c_base + it * c_step; };
 
   if (producer) {
     // ======================================================================================= producer waves
-    const bool do_n = (a.nstates != nullptr) && blk.y == 0;
-    const uint16_t* Xg = a.X + (size_t)bh * S * DHQK + d_tile + (tid % XU) * 8;
-    const uint16_t* Yg = a.Y + (size_t)bh * S * DHHV + w_tile + (tid % YU) * 8;
+    const int DHQK = a.DHQK, DHHV = a.DHHV, S = a.S, NC = a.NC;
+    const size_t Sp = (size_t)NC * kChunk;
+    const int c_base = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
     const int xrow = tid / XU, yrow = tid / YU;  // first row of this thread inside a chunk; further rows XRG / YRG apart
+    const int xcol = (tid % XU) * 8, ycol = (tid % YU) * 8;
     // LDS store offsets of the first row (elements); the rows of a thread are a multiple of 4 apart: same swizzle
     const int xst = xrow * RT + (((tid % XU) ^ scan_swz<XU>(xrow)) << 3);
     const int yst = yrow * WT + (((tid % YU) ^ scan_swz<YU>(yrow)) << 3);
+
+    // The runs of all jobs of this workgroup form one sequence, and the producers work ahead of it without regard to where a
+    // job ends: run P + 3 is requested and run P + 1 staged while run P is multiplied, the scales of the chunk three ahead
+    // are requested.  Two cursors walk the jobs, one over runs and one over chunks; past the last job they stay where they
+    // are (the requests are unconditional: a conditional one makes the compiler keep the registers in scratch memory).
+    int r_rd = -1, r_p = -1, r_bh = job0.bh, r_bx = job0.bx, r_by = job0.by, r_par = 0;  // run cursor
+    ScanRuns<REP> rr;
+    rr.set(job0.it_lo, job0.it_hi, job0.it_rep);
+    int k_rd = -1, k_bh = job0.bh, k_by = job0.by, k_it = job0.it_lo - 1, k_hi = job0.it_hi;  // chunk cursor
+    // a run's properties travel with it: bit 0 there is one, 1 second run of its chunk, 2 last run of its chunk, 3 its slot in
+    // the scale table
+    auto next_run = [&]() -> int {
+      if (r_p + 1 < rr.total) {
+        ++r_p;
+      } else {
+        if constexpr (!MANY) return 0;
+        int lo, hi, rep;
+        do {
+          if (r_rd + 1 >= n_rounds) return 0;
+          ++r_rd;
+          lo = __builtin_amdgcn_readfirstlane(jobs[r_rd].it_lo);
+          hi = __builtin_amdgcn_readfirstlane(jobs[r_rd].it_hi);
+          rep = __builtin_amdgcn_readfirstlane(jobs[r_rd].it_rep);
+        } while (lo == hi);
+        r_bh = __builtin_amdgcn_readfirstlane(jobs[r_rd].bh);
+        r_bx = __builtin_amdgcn_readfirstlane(jobs[r_rd].bx);
+        r_by = __builtin_amdgcn_readfirstlane(jobs[r_rd].by);
+        rr.set(lo, hi, rep);
+        r_p = 0;
+      }
+      const bool last = rr.last(r_p);
+      const int m = 1 | (rr.rest(r_p) ? 2 : 0) | (last ? 4 : 0) | (r_par << 3);
+      if (last) r_par ^= 1;
+      return m;
+    };
+    auto next_chunk = [&]() -> bool {
+      if (k_it + 1 < k_hi) {
+        ++k_it;
+        return true;
+      }
+      if constexpr (!MANY) return false;
+      int lo, hi;
+      do {
+        if (k_rd + 1 >= n_rounds) return false;
+        ++k_rd;
+        lo = __builtin_amdgcn_readfirstlane(jobs[k_rd].it_lo);
+        hi = __builtin_amdgcn_readfirstlane(jobs[k_rd].it_hi);
+      } while (lo == hi);
+      k_bh = __builtin_amdgcn_readfirstlane(jobs[k_rd].bh);
+      k_by = __builtin_amdgcn_readfirstlane(jobs[k_rd].by);
+      k_it = lo;
+      k_hi = hi;
+      return true;
+    };
 
     // ---- row scales (forward: abar_j; backward: bbar_t / sqrt(DHQK) / (nrow_t + eps)) go through a table in LDS:
     // every thread fetches the factor of ONE row of a chunk three chunks before that chunk is staged (first in its
     // batch of loads, so that waiting for it does not wait for the rows requested with it) and writes the table entry
     // one chunk later; positions past the end of the sequence get 0 and so neither feed the state nor the normaliser.
+    // The decay factor of the chunk rides along.
     const int srow = tid & (kChunk - 1);
     const float* const nrow_or_dummy = a.nrow != nullptr ? a.nrow : a.scale_a;
-    float s_raw = 0.f, s_nrm = 1.f;
-    auto load_scales = [&](int c) {  // c: chunk index in memory order, clamped
-      const int cc = min(max(c, 0), NC - 1);
-      s_raw = a.scale_a[bh * Sp + cc * kChunk + srow];
-      s_nrm = nrow_or_dummy[bh * Sp + cc * kChunk + srow];
+    float s_raw = 0.f, s_nrm = 1.f, s_g = 0.f;
+    int s_lim = 0;       // rows of the chunk that lie inside the sequence
+    bool s_n = false;    // whether the chunk's tile carries n
+    auto load_scales = [&](bool there) {  // of the chunk cursor's chunk
+      const int c = c_base + max(k_it, 0) * c_step;
+      const size_t o = (size_t)k_bh * Sp + c * kChunk + srow;
+      s_raw = a.scale_a[o];
+      s_nrm = nrow_or_dummy[o];
+      s_g = a.gbar[(size_t)k_bh * NC + c + opaque(0)];
+      s_lim = there ? S - c * kChunk : 0;
+      s_n = there && a.nstates != nullptr && k_by == 0;
     };
-    auto scale_value = [&](int c) {  // the table entry of row srow of chunk c from the fetched values
-      float sn = (c >= 0 && c < NC && c * kChunk + srow < S) ? s_raw : 0.f;
+    auto scale_value = [&]() {  // the table entry of row srow from the fetched values
+      float sn = srow < s_lim ? s_raw : 0.f;
       if (a.backward) {
         sn *= a.qk_scale;
         if (a.nrow != nullptr) sn /= (s_nrm + a.eps);
@@ -758,25 +875,34 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     // The normaliser recurrence n_c = gbar_c n_{c-1} + sum_j abar_j k_j rides on the matrix pipe of the consumers: the
     // row scale of every position, split exactly into three 16-bit parts, forms three columns of a B operand
     // (position 8b + e of a chunk, part r, at [b][r][e]); K^T times it gives sum_j abar_j k_j in three partial columns
-    // whose sum carries 24 bits of every abar_j.  Slot it % 3: written two chunks before chunk `it` is multiplied.
-    auto write_n_operand = [&](int it_of_chunk, float sn) {
-      uint16_t* dst = nB + (it_of_chunk % 3) * (kChunk * 3) + (srow >> 3) * 24 + (srow & 7);
-      const uint16_t p0 = f32_to_elem<F16>(sn);
-      const float r1 = sn - elem_to_f32<F16>(p0);
-      const uint16_t p1 = f32_to_elem<F16>(r1);
-      const uint16_t p2 = f32_to_elem<F16>(r1 - elem_to_f32<F16>(p1));
-      dst[0] = p0;
-      dst[8] = p1;
-      dst[16] = p2;
+    // whose sum carries 24 bits of every abar_j.  Written two chunks before the chunk is multiplied, three slots.
+    auto write_tables = [&](int chunk) {
+      const float sn = scale_value();
+      if (tid < kChunk) {
+        scl[(chunk & 1) * kChunk + srow] = sn;
+        if (tid == 0) gl[chunk & 3] = s_g;
+        if (s_n) {
+          uint16_t* dst = nB + (chunk % 3) * (kChunk * 3) + (srow >> 3) * 24 + (srow & 7);
+          const uint16_t p0 = f32_to_elem<F16>(sn);
+          const float r1 = sn - elem_to_f32<F16>(p0);
+          const uint16_t p1 = f32_to_elem<F16>(r1);
+          const uint16_t p2 = f32_to_elem<F16>(r1 - elem_to_f32<F16>(p1));
+          dst[0] = p0;
+          dst[8] = p1;
+          dst[16] = p2;
+        }
+      }
     };
 
     // two register sets, by run parity (macros, not lambdas: with the arrays captured by reference the compiler keeps
     // them in scratch memory)
     u32x4 xr0[XV], yr0[YV], xr1[XV], yr1[YV];
     // The prefetch only LOADS: any arithmetic on a loaded value here would make the wave wait for the whole batch.
-#define MLSTM_SCAN_PREFETCH(SET, p_)                                                                             \
+#define MLSTM_SCAN_PREFETCH(SET)                                                                                 \
   {                                                                                                              \
-    const int t0_ = chunk_of(runs.it(p_)) * kChunk;                                                              \
+    const int t0_ = (c_base + rr.it(max(r_p, 0)) * c_step) * kChunk;                                                \
+    const uint16_t* const Xg = a.X + (size_t)r_bh * S * DHQK + r_bx * RT + xcol;                               \
+    const uint16_t* const Yg = a.Y + (size_t)r_bh * S * DHHV + r_by * WT + ycol;                               \
     _Pragma("unroll") for (int v = 0; v < XV; ++v) {                                                             \
       /* rows past the end re-read the last row; their scale is 0 */                                             \
       const int t = min(t0_ + xrow + v * XRG, S - 1);                                                            \
@@ -787,13 +913,13 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
       yr##SET[v] = *(const u32x4*)(Yg + (size_t)t * DHHV);                                                       \
     }                                                                                                            \
   }
-    // registers -> LDS buffer `bi_` (Y rows scaled in fp32, then rounded; second runs: the remainder of that rounding)
-#define MLSTM_SCAN_STAGE(SET, p_, bi_)                                                                           \
+    // registers -> LDS buffer SET (Y rows scaled in fp32, then rounded; second runs: the remainder of that rounding)
+#define MLSTM_SCAN_STAGE(SET, meta_)                                                                             \
   {                                                                                                              \
-    uint16_t* Xs = bufs + (bi_) * BUF;                                                                           \
+    uint16_t* Xs = bufs + (SET) * BUF;                                                                           \
     uint16_t* Yh = Xs + XELEMS;                                                                                  \
-    const float* scur = scl + (runs.it(p_) & 1) * kChunk;                                                        \
-    const bool rest_ = runs.rest(p_);                                                                            \
+    const float* scur = scl + (((meta_) >> 3) & 1) * kChunk;                                                     \
+    const bool rest_ = REP && ((meta_) & 2);                                                                     \
     _Pragma("unroll") for (int v = 0; v < XV; ++v) *(u32x4*)(Xs + xst + v * XRG * RT) = xr##SET[v];              \
     _Pragma("unroll") for (int v = 0; v < YV; ++v) {                                                             \
       const uint32_t in[4] = {yr##SET[v][0], yr##SET[v][1], yr##SET[v][2], yr##SET[v][3]};                       \
@@ -812,91 +938,109 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     }                                                                                                            \
   }
 
-    // ---- prologue: scales of the first two chunks, runs 0 and 1 in registers, run 0 staged, run 2 requested
-    const int c_first = chunk_of(it_lo);
-    {
-      load_scales(c_first);
-      const float sc0 = scale_value(c_first);
-      load_scales(c_first + c_step);
-      const float sc1 = scale_value(it_lo + 1 < NC ? c_first + c_step : -1);
-      if (tid < kChunk) {
-        scl[(it_lo & 1) * kChunk + srow] = sc0;
-        scl[((it_lo + 1) & 1) * kChunk + srow] = sc1;
-        if (do_n) {
-          write_n_operand(it_lo, sc0);
-          write_n_operand(it_lo + 1, sc1);
-        }
-      }
-      for (int k = tid; k < kGBlock && it_lo + k < NC; k += NTP) gl[k] = a.gbar[(size_t)bh * NC + c_first + k * c_step];
-    }
-    load_scales(c_first + 2 * c_step);  // consumed (table write) at the last run of the first chunk
-    // (the prefetches are unconditional, past the end the last run is fetched again: a conditional prefetch makes
-    // the compiler keep the register sets in scratch memory across the loop back-edge)
-    const int p_max = max(total - 1, 0);
-    MLSTM_SCAN_PREFETCH(0, 0)
-    MLSTM_SCAN_PREFETCH(1, min(1, p_max))
-    __syncthreads();  // scale table visible
-    MLSTM_SCAN_STAGE(0, 0, 0)
-    MLSTM_SCAN_PREFETCH(0, min(2, p_max))
+    // ---- prologue: tables of the first two chunks, runs 0 and 1 in registers, run 0 staged, run 2 requested
+    int chunk = 0;
+    load_scales(next_chunk());
+    write_tables(0);
+    load_scales(next_chunk());
+    write_tables(1);
+    load_scales(next_chunk());  // written at the last run of the first chunk
+    bool more = next_chunk();
+    int m0 = next_run();
+    MLSTM_SCAN_PREFETCH(0)
+    int m1 = next_run();
+    MLSTM_SCAN_PREFETCH(1)
+    __syncthreads();  // tables visible
+    MLSTM_SCAN_STAGE(0, m0)
+    int m2 = next_run();
+    MLSTM_SCAN_PREFETCH(0)
+    int m3 = next_run();
 
-    // one run p of parity PAR (its LDS buffer); the runs p+1 and p+3 use the other buffer and register set
-#define MLSTM_SCAN_BODY(PAR, OTHER, p_)                                                                          \
+    // one run, of properties m0; the next one and the one two after that use LDS buffer and register set OTHER
+#define MLSTM_SCAN_BODY(OTHER)                                                                                   \
   {                                                                                                              \
-    const int it = runs.it(p_);                                                                                  \
-    const int c = chunk_of(it);                                                                                  \
-    /* The decay factors come from LDS, a block of chunks at a time. */                                          \
-    if (runs.refill(p_)) {                                                                                       \
-      __syncthreads();                                                                                           \
-      for (int k = tid; k < kGBlock && it + k < NC; k += NTP) gl[k] = a.gbar[(size_t)bh * NC + c + k * c_step];  \
-    }                                                                                                            \
-    /* run p staged; the consumers are done with run p-1, whose buffer is staged into next */                    \
+    /* this run is staged; the consumers are done with the one before it, whose buffer is staged into next */    \
     __syncthreads();                                                                                             \
-    if (runs.last(p_)) {                                                                                         \
-      /* Table entry of chunk it+2 (its factors were fetched one chunk ago) into the slot of chunk it, all of */ \
-      /* whose runs have been staged; it is read from the next run on.  Then the factors of chunk it+3 are */    \
-      /* requested, first in this run's batch of loads. */                                                       \
-      if (tid < kChunk) {                                                                                        \
-        const float sn = scale_value(it + 2 < NC ? c + 2 * c_step : -1);                                         \
-        scl[(it & 1) * kChunk + srow] = sn;                                                                      \
-        if (do_n) write_n_operand(it + 2, sn);                                                                   \
-      }                                                                                                          \
-      load_scales(c + 3 * c_step);                                                                               \
+    if (m0 & 4) {                                                                                                \
+      /* Table entry of the chunk after the next (its factors were fetched one chunk ago) into the slot of the */ \
+      /* present one, all of whose runs have been staged; it is read from the next run on.  Then the factors */  \
+      /* of the chunk after that are requested, first in this run's batch of loads. */                           \
+      write_tables(chunk + 2);                                                                                   \
+      load_scales(more);                                                                                         \
     }                                                                                                            \
-    if ((p_) + 1 < total) MLSTM_SCAN_STAGE(OTHER, (p_) + 1, OTHER)                                               \
-    MLSTM_SCAN_PREFETCH(OTHER, min((p_) + 3, p_max))                                                             \
+    if (m1 & 1) MLSTM_SCAN_STAGE(OTHER, m1)                                                                      \
+    MLSTM_SCAN_PREFETCH(OTHER)                                                                                   \
+    /* the cursors move on when everything is on its way */                                                      \
+    if (m0 & 4) {                                                                                                \
+      more = next_chunk();                                                                                       \
+      ++chunk;                                                                                                   \
+    }                                                                                                            \
+    m0 = m1;                                                                                                     \
+    m1 = m2;                                                                                                     \
+    m2 = m3;                                                                                                     \
+    m3 = next_run();                                                                                             \
   }
-    for (int p = 0; p < total; p += 2) {
-      MLSTM_SCAN_BODY(0, 1, p)
-      if (p + 1 < total) MLSTM_SCAN_BODY(1, 0, p + 1)
+    while (m0 & 1) {
+      MLSTM_SCAN_BODY(1)
+      if (m0 & 1) MLSTM_SCAN_BODY(0)
     }
 #undef MLSTM_SCAN_BODY
 #undef MLSTM_SCAN_STAGE
 #undef MLSTM_SCAN_PREFETCH
   } else {
     // ======================================================================================= consumer waves
-    // the normaliser vector rides with two waves of every 64 state rows in the first column tile: value-column blocks
-    // 0 and 1 carry it for the first and the second 32 rows
-    const bool with_n = (a.nstates != nullptr) && blk.y == 0;
-    const int tile = blk.x + (int)gridDim.x * blk.y;
-    if (with_n && wave % WC == 0)
-      scan_consumer<RT, WT, F16, REP, SEG, 0>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
-    else if (with_n && wave % WC == 1)
-      scan_consumer<RT, WT, F16, REP, SEG, 1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
-    else
-      scan_consumer<RT, WT, F16, REP, SEG, -1>(a, bufs, gl, nB, wave, lane, bh, seg, tile, d_tile, w_tile, runs, is_end);
+    int run = 0, chunk = 0;
+    __syncthreads();  // the producers' prologue barrier
+    for (int rd = 0; rd < (MANY ? n_rounds : 1); ++rd) {
+      ScanJob job = job0;
+      if constexpr (MANY) {
+        int* const w = (int*)&job;
+#pragma unroll
+        for (int x = 0; x < (int)(sizeof(ScanJob) / sizeof(int)); ++x) w[x] = __builtin_amdgcn_readfirstlane(((const int*)(jobs + rd))[x]);
+      }
+      if (job.it_lo == job.it_hi && job.end == 0) continue;
+      // the normaliser vector rides with two waves of every 64 state rows in the first column tile: value-column blocks
+      // 0 and 1 carry it for the first and the second 32 rows
+      const bool with_n = (a.nstates != nullptr) && job.by == 0;
+      if (with_n && wave % WC == 0)
+        scan_consumer<RT, WT, F16, REP, SEG, 0>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);
+      else if (with_n && wave % WC == 1)
+        scan_consumer<RT, WT, F16, REP, SEG, 1>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);
+      else
+        scan_consumer<RT, WT, F16, REP, SEG, -1>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);
+    }
   }
 }
 
-template <int RT, int WT, bool F16, bool REP, bool SEG>
-static const char* launch_scan_roles_f(const ScanArgs& a, int BH, hipStream_t stream) {
+static size_t scan_roles_smem(int RT, int WT) {
+  return (size_t)2 * kChunk * (RT + WT) * 2 + (size_t)(4 + 2 * kChunk) * 4 + (size_t)3 * kChunk * 3 * 2 + kScanRounds * sizeof(ScanJob);
+}
+template <int RT, int WT, bool F16, bool REP, bool SEG, bool MANY>
+static const char* launch_scan_roles_m(const ScanArgs& a, int G, int n_rounds, hipStream_t stream) {
   constexpr int NW = (RT / 64) * (WT / 32);
-  const size_t smem = (size_t)2 * kChunk * (RT + WT) * 2 + (size_t)(kGBlock + 2 * kChunk) * 4 + (size_t)3 * kChunk * 3 * 2;
   static LdsLimit lds;
-  if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16, REP, SEG>, smem))
+  if (!lds.allow((const void*)scan_roles_kernel<RT, WT, F16, REP, SEG, MANY>, scan_roles_smem(RT, WT)))
     return "scan: cannot raise the dynamic LDS limit";
-  dim3 grid(a.DHQK / RT, a.DHHV / WT, BH * (a.seg_phase == 1 ? a.nseg - 1 : a.nseg));
-  hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16, REP, SEG>), grid, dim3(128 * NW), smem, stream, a);
+  hipLaunchKernelGGL((scan_roles_kernel<RT, WT, F16, REP, SEG, MANY>), dim3(G), dim3(128 * NW), scan_roles_smem(RT, WT), stream, a, n_rounds);
   return nullptr;
+}
+template <int RT, int WT, bool F16, bool REP, bool SEG>
+static const char* launch_scan_roles_f(ScanArgs a, int BH, hipStream_t stream) {
+  const long long n_jobs = (long long)(a.DHQK / RT) * (a.DHHV / WT) * BH * (a.seg_phase == 1 ? a.nseg - 1 : a.nseg);
+  if (n_jobs >= (1ll << 30)) return "scan: too many state tiles";
+  const int cus = device_cu_count();
+  if (cus <= 0) return "scan: cannot read the number of compute units";
+  a.n_jobs = (int)n_jobs;
+  const int fit = cus * (int)(160 * 1024 / scan_roles_smem(RT, WT));
+  if (a.n_jobs <= fit) return launch_scan_roles_m<RT, WT, F16, REP, SEG, false>(a, a.n_jobs, 1, stream);
+  if constexpr (SEG) {
+    return "scan: more segments than the chip holds";
+  } else {
+    const int least = (a.n_jobs + kScanRounds - 1) / kScanRounds;
+    int G = fit > least + 7 ? fit : least + 7;
+    if (G >= 8) G -= G % 8;
+    return launch_scan_roles_m<RT, WT, F16, REP, SEG, true>(a, G, (a.n_jobs + G - 1) / G, stream);
+  }
 }
 template <int RT, int WT, bool F16>
 static const char* launch_scan_roles_s(const ScanArgs& a, int BH, hipStream_t stream) {
@@ -916,6 +1060,13 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
   a.nseg = 1;
   a.seg_len = a.NC;
   a.seg_phase = 0;
+  // Chunks that are run at all: without a last state those up to the last kept boundary (forward), down to the first one
+  // (backward), and for n, which is kept at every chunk, up to the last chunk.
+  a.end_c = a.end_n = a.NC;
+  if (a.final_out == nullptr && a.stride >= 1) {
+    a.end_c = a.backward ? (a.NC > a.stride ? a.NC - a.stride : 0) : (a.NC - 1) / a.stride * a.stride;
+    if (a.n_final == nullptr) a.end_n = a.NC - 1;
+  }
   if (a.DHQK % 64 != 0 || a.DHHV % 64 != 0) return "scan: DHQK and DHHV must be multiples of 64";
   if (a.stride < 1 || a.stride > kMaxStateStride) return "scan: state stride out of range";
   const bool r128 = a.DHQK % 128 == 0;

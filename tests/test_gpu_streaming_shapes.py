@@ -150,6 +150,34 @@ def test_named_paths_do_not_depend_on_the_batch(path, S, DQ, DV):
         assert torch.equal(a, b)
 
 
+# State tiles on persistent workgroups: fewer, as many and many more than the CUs hold (the last: more than 32 for each); the
+# chunks behind the last kept state are not run, with and without a last state, with strides that divide the chunks and not.
+# With the path named a head's bits do not depend on how the tiles fall to the workgroups.
+@pytest.mark.parametrize("DQ,DV,BH,S", [(256, 512, 33, 129), (256, 512, 80, 640), (64, 64, 514, 385), (128, 64, 300, 257), (64, 128, 300, 640),
+                                        (64, 64, 16500, 130)])
+@pytest.mark.parametrize("last,stride,init", [(False, 1, False), (False, 2, True), (False, 3, False), (True, 2, False), (True, 3, True)])
+def test_state_tiles_on_persistent_workgroups(DQ, DV, BH, S, last, stride, init):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    if BH > 1000 and (stride, init) != (2, False) and stride != 1:
+        pytest.skip("the most workgroups: two options only")
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(BH, 1, S, DQ, DV, seed=S, f_offset=3.0))
+    dH = torch.randn(BH, 1, S, DV, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    g = torch.Generator().manual_seed(2)
+    c0 = [torch.randn(BH, 1, *d, generator=g).cuda() for d in ((DQ, DV), (DQ,))] + [torch.zeros(BH, 1, 1).cuda()] if init else [None] * 3
+    out = []
+    pick = [0, BH // 3, BH - 1]
+    for rows in (pick, slice(0, BH)):
+        leaves = [t[rows].clone().requires_grad_(True) for t in (q, k, v, i, f)]
+        H = mlstm_chunkwise__hip_xl_chunk(*leaves, *(None if t is None else t[rows] for t in c0), return_last_states=last,
+                                          any_sequence_length=True, kernel_path="split", chunk_size_intra=128 * stride)
+        H, state = H if last else (H, ())
+        grads = torch.autograd.grad(H, leaves, dH[rows])
+        out.append([t.detach() if rows is pick else t.detach()[pick] for t in (H, *state, *grads)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("S,DQ,DV,NH", [(1100, 64, 64, 4), (1100, 128, 128, 2), (300, 256, 512, 5), (700, 256, 512, 26)])
 def test_items_that_are_no_multiple_of_eight(S, DQ, DV, NH):
     _run(S, DQ, DV, NH=NH, seed=S + NH)
