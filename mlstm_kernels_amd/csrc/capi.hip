@@ -79,20 +79,29 @@ const char* check_options(int path, int state_stride, int DHQK, int DHHV) {
 }
 // H / dV kernel of the split form: the streaming kernel where the path asks for it (or leaves the choice open) and the
 // shape is one it supports; MLSTM_PATH_AUTO: the window kernel where it is faster; otherwise the tiled kernel
+enum HvKernel { kHvStream, kHvWindow, kHvTiled };
+HvKernel choose_hv(int path, const mlstm::ParHvArgs& a, int BH) {
+  if ((path == MLSTM_PATH_STREAM || path == MLSTM_PATH_AUTO) && mlstm::stream_hv_supported(a)) return kHvStream;
+  if (path == MLSTM_PATH_AUTO && mlstm::window_hv_preferred(a, BH)) return kHvWindow;
+  return kHvTiled;
+}
 const char* launch_hv(int path, const mlstm::ParHvArgs& a, int BH, bool is_dv, hipStream_t st) {
   // (by request the stream kernels take whole chunks only; MLSTM_PATH_AUTO uses them for ragged lengths as well)
   if (path == MLSTM_PATH_STREAM && !(mlstm::stream_hv_supported(a) && a.S % 128 == 0))
     return "the stream kernel path supports DHQK = 256, DHHV % 512 == 0, S % 128 == 0 only (with a head norm: DHHV = 512)";
-  if ((path == MLSTM_PATH_STREAM || path == MLSTM_PATH_AUTO) && mlstm::stream_hv_supported(a))
-    return mlstm::launch_stream_hv(a, BH, is_dv, st);
-  if (path == MLSTM_PATH_AUTO && mlstm::window_hv_preferred(a, BH)) return mlstm::launch_window_hv(a, BH, is_dv, st);
-  return mlstm::launch_par_hv(a, BH, is_dv, st);
+  switch (choose_hv(path, a, BH)) {
+    case kHvStream: return mlstm::launch_stream_hv(a, BH, is_dv, st);
+    case kHvWindow: return mlstm::launch_window_hv(a, BH, is_dv, st);
+    default: return mlstm::launch_par_hv(a, BH, is_dv, st);
+  }
 }
 // dQ / dK launch.  MLSTM_PATH_STREAM: the window kernel where the stride allows; MLSTM_PATH_AUTO: where it is faster;
 // else the tiled pair kernel; MLSTM_PATH_SPLIT: the tiled pair kernel
+bool choose_window_qk(int path, const mlstm::ParQkArgs& a, int BH) {
+  return path == MLSTM_PATH_STREAM ? mlstm::window_qk_supported(a) : path == MLSTM_PATH_AUTO && mlstm::window_qk_preferred(a, BH);
+}
 const char* launch_qk(int path, const mlstm::ParQkArgs& a, int BH, hipStream_t st) {
-  if (path == MLSTM_PATH_STREAM ? mlstm::window_qk_supported(a) : path == MLSTM_PATH_AUTO && mlstm::window_qk_preferred(a, BH))
-    return mlstm::launch_window_qk(a, BH, st);
+  if (choose_window_qk(path, a, BH)) return mlstm::launch_window_qk(a, BH, st);
   return mlstm::launch_par_qk_pair(a, BH, st);
 }
 const char* check_dims(int B, int NH, int S, int DHQK, int DHHV) {
@@ -239,7 +248,7 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   const int sig = gate == MLSTM_GATE_SIG;
   {
     ProfileScope ps("gates", st);
-    if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, st)) return fail(e);
+    if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, !has_c0, st)) return fail(e);
   }
   if (check_launch("gates")) return 1;
 
@@ -278,6 +287,26 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     return check_launch("fused_hv forward");
   }
 
+  mlstm::ParHvArgs pa;
+  memset(&pa, 0, sizeof(pa));
+  pa.Q = (const uint16_t*)q; pa.K = (const uint16_t*)k; pa.V = (const uint16_t*)v;
+  pa.g = ws.g;
+  pa.nstates = ws.nstates;
+  pa.states = ws.cstates;
+  pa.nrow_out = ws.nrow;
+  pa.Out = (uint16_t*)H;
+  pa.n_out = n_out; pa.m_out = m_out;
+  pa.S = S; pa.NC = NC; pa.DHQK = DHQK; pa.DHHV = DHHV;
+  pa.qk_scale = 1.0f / sqrtf((float)DHQK); pa.eps = eps;
+  pa.sig_gate = sig;
+  pa.use_nrow = !(sig && !normalize);
+  pa.stride = stride;
+  pa.head_norm = head_norm;
+  pa.f16 = f16;
+  pa.norm_eps = norm_eps;
+  pa.norm_mean = norm_mean;
+  pa.norm_rstd = norm_rstd;
+  pa.zero_state = !has_c0;
   mlstm::ScanArgs sa;
   memset(&sa, 0, sizeof(sa));
   sa.X = (const uint16_t*)k;
@@ -291,11 +320,12 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   sa.nstates = track_n ? ws.nstates : nullptr;
   sa.n_final = track_n ? n_last : nullptr;
   sa.S = S; sa.NC = NC; sa.DHQK = DHQK; sa.DHHV = DHHV;
-  sa.qk_scale = 1.0f / sqrtf((float)DHQK);
+  sa.qk_scale = pa.qk_scale;
   sa.eps = eps;
   sa.backward = 0;
   sa.stride = stride;
   sa.f16 = f16;
+  sa.skip_zero = choose_hv(path, pa, BH) != kHvTiled;  // (in the backward both dQ / dK kernels know, from g.zero_c)
   // Which chunks still weigh in the last state is read off the decay factors, which presumes inputs of comparable
   // scale in every chunk: true for the exponential gate (its stabiliser rescales them), not for the sigmoid gate,
   // whose late positions may all be closed while early chunks dominate the state.
@@ -312,25 +342,6 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   }
   if (check_launch("scan_fw")) return 1;
 
-  mlstm::ParHvArgs pa;
-  memset(&pa, 0, sizeof(pa));
-  pa.Q = (const uint16_t*)q; pa.K = (const uint16_t*)k; pa.V = (const uint16_t*)v;
-  pa.g = ws.g;
-  pa.nstates = ws.nstates;
-  pa.states = ws.cstates;
-  pa.nrow_out = ws.nrow;
-  pa.Out = (uint16_t*)H;
-  pa.n_out = n_out; pa.m_out = m_out;
-  pa.S = S; pa.NC = NC; pa.DHQK = DHQK; pa.DHHV = DHHV;
-  pa.qk_scale = sa.qk_scale; pa.eps = eps;
-  pa.sig_gate = sig;
-  pa.use_nrow = !(sig && !normalize);
-  pa.stride = stride;
-  pa.head_norm = head_norm;
-  pa.f16 = f16;
-  pa.norm_eps = norm_eps;
-  pa.norm_mean = norm_mean;
-  pa.norm_rstd = norm_rstd;
   {
     ProfileScope ps("par_h", st);
     if (const char* e = launch_hv(path, pa, BH, /*is_dv=*/false, st)) return fail(e);
@@ -450,6 +461,20 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
   const int use_nrow = !(sig && !normalize);
   const float qk_scale = 1.0f / sqrtf((float)DHQK);
 
+  mlstm::ParQkArgs pq;
+  memset(&pq, 0, sizeof(pq));
+  pq.Q = (const uint16_t*)q; pq.K = (const uint16_t*)k; pq.V = (const uint16_t*)v; pq.dH = (const uint16_t*)dH;
+  pq.g = ws.g;
+  pq.nrow = ws.nrow;
+  pq.S = S; pq.NC = NC; pq.DHQK = DHQK; pq.DHHV = DHHV;
+  pq.qk_scale = qk_scale; pq.eps = eps;
+  pq.use_nrow = use_nrow;
+  pq.stride = stride;
+  pq.f16 = f16;
+  pq.zero_dc = dC_last == nullptr;
+  // dQ and dK in one launch: the workgroups of a chunk run side by side and share the Q, K, V and dH rows they stream
+  pq.states = ws.cstates; pq.Out = (uint16_t*)dQ; pq.rowdot = bws.qdq;
+  pq.states2 = bws.dcstates; pq.Out2 = (uint16_t*)dK; pq.rowdot2 = bws.kdk;
   if (use_fused(path, DHQK, DHHV)) {
     if (f16) return fail("mlstm_hip_chunkwise_bw: the fused kernel path multiplies bf16 operands only");
     mlstm::FusedHvArgs fa;
@@ -471,29 +496,6 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     }
     if (check_launch("fused_hv dV")) return 1;
   } else {
-    mlstm::ScanArgs sa;
-    memset(&sa, 0, sizeof(sa));
-    sa.X = (const uint16_t*)q;
-    sa.Y = (const uint16_t*)dH;
-    sa.scale_a = ws.g.bbar;
-    sa.nrow = use_nrow ? ws.nrow : nullptr;
-    sa.gbar = ws.g.gbar;
-    sa.init = dC_last;
-    sa.states = bws.dcstates;
-    sa.final_out = dC0;
-    sa.S = S; sa.NC = NC; sa.DHQK = DHQK; sa.DHHV = DHHV;
-    sa.qk_scale = qk_scale; sa.eps = eps;
-    sa.backward = 1;
-    sa.seg = path == MLSTM_PATH_AUTO ? (float*)dV : nullptr;  // as in the forward; dV is written after the scan
-    sa.seg_bytes = (size_t)BH * S * DHHV * 2;
-    sa.stride = stride;
-    sa.f16 = f16;
-    {
-      ProfileScope ps("scan_bw", st);
-      if (const char* e = mlstm::launch_scan(sa, BH, /*hilo=*/false, st)) return fail(e);
-    }
-    if (check_launch("scan_bw")) return 1;
-
     mlstm::ParHvArgs pv;
     memset(&pv, 0, sizeof(pv));
     pv.Q = (const uint16_t*)q; pv.K = (const uint16_t*)k; pv.V = (const uint16_t*)v; pv.dH = (const uint16_t*)dH;
@@ -506,6 +508,31 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     pv.sig_gate = sig; pv.use_nrow = use_nrow;
     pv.stride = stride;
     pv.f16 = f16;
+    pv.zero_state = dC_last == nullptr;
+    mlstm::ScanArgs sa;
+    memset(&sa, 0, sizeof(sa));
+    sa.X = (const uint16_t*)q;
+    sa.Y = (const uint16_t*)dH;
+    sa.scale_a = ws.g.bbar;
+    sa.nrow = use_nrow ? ws.nrow : nullptr;
+    sa.gbar = ws.g.gbar;
+    sa.init = dC_last;
+    sa.states = bws.dcstates;
+    sa.final_out = dC0;
+    sa.S = S; sa.NC = NC; sa.DHQK = DHQK; sa.DHHV = DHHV;
+    sa.qk_scale = qk_scale; sa.eps = eps;
+    sa.skip_zero = choose_hv(path, pv, BH) != kHvTiled && choose_window_qk(path, pq, BH);
+    sa.backward = 1;
+    sa.seg = path == MLSTM_PATH_AUTO ? (float*)dV : nullptr;  // as in the forward; dV is written after the scan
+    sa.seg_bytes = (size_t)BH * S * DHHV * 2;
+    sa.stride = stride;
+    sa.f16 = f16;
+    {
+      ProfileScope ps("scan_bw", st);
+      if (const char* e = mlstm::launch_scan(sa, BH, /*hilo=*/false, st)) return fail(e);
+    }
+    if (check_launch("scan_bw")) return 1;
+
     {
       ProfileScope ps("par_dv", st);
       if (const char* e = launch_hv(path, pv, BH, /*is_dv=*/true, st)) return fail(e);
@@ -513,19 +540,6 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     if (check_launch("par_hv dV")) return 1;
   }
 
-  mlstm::ParQkArgs pq;
-  memset(&pq, 0, sizeof(pq));
-  pq.Q = (const uint16_t*)q; pq.K = (const uint16_t*)k; pq.V = (const uint16_t*)v; pq.dH = (const uint16_t*)dH;
-  pq.g = ws.g;
-  pq.nrow = ws.nrow;
-  pq.S = S; pq.NC = NC; pq.DHQK = DHQK; pq.DHHV = DHHV;
-  pq.qk_scale = qk_scale; pq.eps = eps;
-  pq.use_nrow = use_nrow;
-  pq.stride = stride;
-  pq.f16 = f16;
-  // dQ and dK in one launch: the workgroups of a chunk run side by side and share the Q, K, V and dH rows they stream
-  pq.states = ws.cstates; pq.Out = (uint16_t*)dQ; pq.rowdot = bws.qdq;
-  pq.states2 = bws.dcstates; pq.Out2 = (uint16_t*)dK; pq.rowdot2 = bws.kdk;
   {
     ProfileScope ps("par_dqdk", st);
     if (const char* e = launch_qk(path, pq, BH, st)) return fail(e);

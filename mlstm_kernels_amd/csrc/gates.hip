@@ -94,8 +94,9 @@ __device__ __forceinline__ ChunkScan scan_chunk(const void* ig, const void* fg, 
 
 __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
     const void* __restrict__ ig, const void* __restrict__ fg, GateBufs gb, int S, int NC, int dtype_gates,
-    int sig_gate) {
+    int sig_gate, int zero_c) {
   const int bh = blockIdx.y;
+  if (bh == 0 && blockIdx.x == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = blockIdx.x * kGateChunks + wave;
   if (c >= NC) return;
@@ -116,9 +117,10 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
 // gates_finish_kernel).
 __global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
     const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb,
-    float* __restrict__ m_last, int S, int NC, int dtype_gates, int sig_gate) {
+    float* __restrict__ m_last, int S, int NC, int dtype_gates, int sig_gate, int zero_c) {
   __shared__ float gs[kGateChunks], as[kGateChunks];
   const int bh = blockIdx.y;
+  if (bh == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;  // one wave per chunk
   const float NEG_INF = -__builtin_inff();
   const float m_init = !sig_gate && m0 != nullptr ? m0[bh] : 0.f;
@@ -259,15 +261,15 @@ __global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(const float*
 }
 
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
-                         int B, int NH, int S, int dtype_gates, int sig_gate, hipStream_t stream) {
+                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, hipStream_t stream) {
   const int NC = (S + kChunk - 1) / kChunk;
   if (NC <= kGateChunks) {
     hipLaunchKernelGGL(gates_whole_kernel, dim3(1, B * NH), dim3(kWave * NC), 0, stream, i, f, m0, gb, m_last, S, NC, dtype_gates,
-                       sig_gate);
+                       sig_gate, zero_c);
     return nullptr;
   }
   const dim3 grid((NC + kGateChunks - 1) / kGateChunks, B * NH);
-  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, gb, S, NC, dtype_gates, sig_gate);
+  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, gb, S, NC, dtype_gates, sig_gate, zero_c);
   hipLaunchKernelGGL(gates_finish_kernel, grid, dim3(kGateThreads), 0, stream, m0, gb, m_last, NC, sig_gate);
   return nullptr;
 }

@@ -99,6 +99,7 @@ struct ParHvArgs {
   float norm_eps;
   float* norm_mean;         // forward with head_norm: (B,NH,S) row means (0 for rms)
   float* norm_rstd;         // forward with head_norm: (B,NH,S) reciprocal standard deviations
+  int zero_state;           // the state that the first (forward) / last (dV) group of `stride` chunks uses is known to be zero
   int f16;                  // inputs, state fragments and Out are float16 instead of bfloat16
 };
 
@@ -146,6 +147,7 @@ struct ParQkArgs {
   float qk_scale, eps;
   int use_nrow;
   int stride;               // a chunk state is kept every `stride` chunks
+  int zero_dc;              // the gradient of the state after the last chunk is known to be zero (of the initial state: g.zero_c)
   int f16;                  // inputs, state fragments and outputs are float16 instead of bfloat16
 };
 
@@ -176,7 +178,7 @@ struct StepBlockArgs {
 bool step_block_supported(int DHQK, int DHHV, int dtype_qkv);
 const char* launch_step_block(const StepBlockArgs& a, hipStream_t stream);
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
-                         int B, int NH, int S, int dtype_gates, int sig_gate, hipStream_t stream);
+                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, hipStream_t stream);
 const char* launch_scan(const ScanArgs& a, int BH, bool hilo, hipStream_t stream);
 const char* launch_par_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 bool par_hv_head_norm_supported(int DHHV);

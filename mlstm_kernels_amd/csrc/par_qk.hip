@@ -184,13 +184,16 @@ __device__ __forceinline__ void par_qk_body(const ParQkArgs& a, const BlockId bl
     _Pragma("unroll") for (int v = 0; v < CV; ++v)                                                                   \
         creg[v] = st[((size_t)(slab_) * ND + d_tile / 16) * 64 + tid + v * NTH];                                     \
   }
+    // (an initial state that is zero has no fragments; the gradient after the last chunk always has them where this kernel runs)
+    const bool no_state = IS_DQ && slot == 0 && *a.g.zero_c != 0;
     // lanes 32..63 of every state fragment are stored 4 slots off so that the two lane halves a transposing read
     // touches together fall on different LDS banks
 #define MLSTM_STORE_C(creg)                                                                                          \
   {                                                                                                                  \
     _Pragma("unroll") for (int v = 0; v < CV; ++v) {                                                                 \
       const int idx = tid + v * NTH;                                                                                 \
-      ((u32x4*)Cf)[idx ^ (((idx >> 5) & 1) << 2)] = creg[v];                                                         \
+      const u32x4 none = {0u, 0u, 0u, 0u};                                                                           \
+      ((u32x4*)Cf)[idx ^ (((idx >> 5) & 1) << 2)] = no_state ? none : creg[v];                                       \
     }                                                                                                                \
   }
     // transposing read of the staged fragments: lane i16 of a 16-lane block addresses value column

@@ -1069,6 +1069,8 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
   }
   if (a.DHQK % 64 != 0 || a.DHHV % 64 != 0) return "scan: DHQK and DHHV must be multiples of 64";
   if (a.stride < 1 || a.stride > kMaxStateStride) return "scan: state stride out of range";
+  // (up to one group of chunks and no state from outside: nothing to run and nothing to write)
+  if (a.skip_zero && a.init == nullptr && a.final_out == nullptr && a.nstates == nullptr && a.end_c == 0) return nullptr;
   const bool r128 = a.DHQK % 128 == 0;
   bool w128 = a.DHHV % 128 == 0;
   // Segments (see the top of the file): as many as fit the chip beside each other, at most eight, of eight chunks or more;

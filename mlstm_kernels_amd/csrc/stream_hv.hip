@@ -24,6 +24,8 @@
 //   8 x state slab: 2 contraction steps x 16 fragment blocks of 32 value columns
 //   per source chunk, per half of 64 source positions: 1 slab of 64 rows x DHQK (scores, gated into the score block
 //   in the same step), 2 slabs of 32 rows x 512 value columns (output product)
+// An item whose kept state is known to be zero has two state steps instead of eight (see the producers): 128 heads of 1024
+// positions with layer norm and no initial state, forward and backward, 665 -> 625 us with the same in window_qk.hip.
 // Register set and ring slot alternate from step to step and every source chunk has an even number of steps, so both
 // are compile-time constants everywhere.
 // Supported: DHQK = 256, DHHV a multiple of 512 (exactly 512 with a head norm); everything else runs par_hv.hip.
@@ -39,21 +41,25 @@ struct HvItem {
   int bh, c, ch;               // (batch * head), chunk, group of 512 value columns
   int slot;                    // kept boundary state the chunk uses
   int sc_first, sc_step, nsc;  // source chunks: sc_first, sc_first + sc_step, ... (nsc of them, the own chunk last)
+  bool no_state;               // the kept state is known to be zero
 };
 
 // Work item of workgroup `vid` in round `round`.  Consecutive workgroups take consecutive items (neighbouring chunks
 // share rows and kept states through the L2 of their XCD); the assignment rotates by one item per round so that a
-// workgroup does not always get the chunks with the same number of source chunks.
+// workgroup does not always get the chunks with the same number of source chunks.  The nz chunks of a head whose state is
+// known to be zero (forward the first ones, dV the last ones) have less to do and are dealt out last.
 template <bool IS_DV>
-__device__ __forceinline__ bool hv_decode(HvItem& it, int round, int vid, int G, int n_items, int NC, int NCH, int stride) {
+__device__ __forceinline__ bool hv_decode(HvItem& it, int round, int vid, int G, int n_items, int NC, int NCH, int stride, int nz) {
   const int rot = (vid + round) % G;
   const long long idx = (long long)round * G + rot;
   if (idx >= n_items) return false;
-  const int i = (int)idx;
-  it.ch = i % NCH;
-  const int rest = i / NCH;
-  it.c = rest % NC;
-  it.bh = rest / NC;
+  const int i = (int)idx, full = NC - nz, n_full = n_items / NC * full;
+  it.no_state = i >= n_full;
+  const int per = it.no_state ? nz : full, j = it.no_state ? i - n_full : i;
+  it.ch = j % NCH;
+  const int rest = j / NCH;
+  it.c = rest % per + (it.no_state ? (IS_DV ? full : 0) : (IS_DV ? 0 : nz));
+  it.bh = rest / per;
   it.slot = it.c / stride;
   if (IS_DV) {
     const int hi = min(it.slot * stride + stride - 1, NC - 1);
@@ -116,6 +122,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
   const int NC = a.NC, S = a.S, DHHV = a.DHHV, NCH = DHHV / CW, stride = a.stride;
   const size_t Sp = (size_t)NC * kChunk;
   const int NCS = (NC + stride - 1) / stride;
+  const int nz = !a.zero_state ? 0 : (IS_DV ? NC - (NCS - 1) * stride : min(stride, NC));
 
   if (wave_all >= 8) {
     // =========================================================================================== producer waves
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
   }
     HvItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!hv_decode<IS_DV>(it, rd, vid, G, n_items, NC, NCH, stride)) continue;
+      if (!hv_decode<IS_DV>(it, rd, vid, G, n_items, NC, NCH, stride, nz)) continue;
       // An item has 12 + 6 s steps, a multiple of three: the register set of every step is a literal.
       const uint32_t pl = (uint32_t)opaque(p);
       const uint32_t row = pl >> 5, pc = pl & 31;  // rows of 512 bytes: 32 pieces per row, 8 rows per sweep
@@ -218,19 +225,22 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
         HV_PROC(0, 4, base, g0 + 96 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 96 * QS * 2, gown)
       }
       {
-        // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks
+        // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks.  Without a
+        // state the first two only (a state of another chunk, which nobody looks at): one step the consumers need for the
+        // denominators, one that makes the number of steps a multiple of three.  (Two steps and then threes, so that the
+        // loads behind every register set are as many whether the loop runs or not: the compiler's waits stay partial.)
         const char* const base = St_b + ((size_t)it.bh * NCS + it.slot) * (size_t)(DHHV / 32) * ND * 1024;
         const uint32_t f0 = pl >> 6;  // fragment of the first piece inside the slab: block f0 / 2, contraction step f0 % 2
         const uint32_t g0 = (((uint32_t)it.ch * (CW / 32) + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
         const uint32_t r0 = (kRing0Off + pl * 16) | (1u << 20), r1 = (kRing1Off + pl * 16) | (1u << 20);
         HV_PROC(1, NPC, base, g0, 2 * ND * 1024, 0xffffffffu, r0, gown)
         HV_PROC(2, NPC, base, g0 + 1 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(0, NPC, base, g0 + 2 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(1, NPC, base, g0 + 3 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(2, NPC, base, g0 + 4 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(0, NPC, base, g0 + 5 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
-        HV_PROC(1, NPC, base, g0 + 6 * 2048, 2 * ND * 1024, 0xffffffffu, r0, gown)
-        HV_PROC(2, NPC, base, g0 + 7 * 2048, 2 * ND * 1024, 0xffffffffu, r1, gown)
+        for (int si = it.no_state ? 8 : 2; si < 8; si += 3) {
+          const uint32_t ra = si & 1 ? r1 : r0, rb = si & 1 ? r0 : r1;
+          HV_PROC(0, NPC, base, g0 + si * 2048, 2 * ND * 1024, 0xffffffffu, ra, gown)
+          HV_PROC(1, NPC, base, g0 + (si + 1) * 2048, 2 * ND * 1024, 0xffffffffu, rb, gown)
+          HV_PROC(2, NPC, base, g0 + (si + 2) * 2048, 2 * ND * 1024, 0xffffffffu, ra, gown)
+        }
       }
       {
         const char* const kbase = Xo_b + (size_t)it.bh * S * DHQK * 2;
@@ -286,7 +296,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
     HvItem it, prev;
-    prev = HvItem{0, 0, 0, 0, 0, 1, 1};
+    prev = HvItem{0, 0, 0, 0, 0, 1, 1, false};
     bool have_prev = false;
     // The accumulators are only ever touched in straight-line code between barriers: no matrix instruction that
     // updates them sits under a condition (dead score blocks of the own chunk are masked to zero by the gating), so
@@ -339,7 +349,7 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
     __builtin_amdgcn_wave_barrier();                                                                                 \
   }
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!hv_decode<IS_DV>(it, rd, vid, G, n_items, NC, NCH, stride)) continue;
+      if (!hv_decode<IS_DV>(it, rd, vid, G, n_items, NC, NCH, stride, nz)) continue;
       const int bh = it.bh, c = it.c;
       const size_t hofs = (size_t)bh * Sp, gofs = hofs + (size_t)c * kChunk;
       const float* graw = a.g.graw + (size_t)bh * NC;
@@ -386,59 +396,63 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       __syncthreads();
       if (!IS_DV && tid < DHQK) nperm[perm16(tid)] = (np0 + np1) + np2;
       __syncthreads();
-      // ---- inter-chunk product: Out^T = State^T Xn^T, two contraction steps per slab
-#pragma unroll
-      for (int si = 0; si < 8; ++si) {
-        __syncthreads();
-        if (!IS_DV) {
-          if (si == 0) {
-            // forward: q_t . n_prev for the denominators (four threads per position), while the resident rows are
-            // all there -- the next item's rows start to arrive during this item's last step
-            const int td = opaque(tid);
-            const int t = td >> 2, part = td & 3;
-            const uint16_t* qrow = Ns + t * QS + part * (DHQK / 4);
-            const float* np = nperm + part * (DHQK / 4);
-            float dot = 0.f;
+      // forward: q_t . n_prev for the denominators (four threads per position), while the resident rows are all there -- the
+      // next item's rows start to arrive during this item's last step
+      auto query_dot_n = [&]() __attribute__((always_inline)) {
+        const int td = opaque(tid);
+        const int t = td >> 2, part = td & 3;
+        const uint16_t* qrow = Ns + t * QS + part * (DHQK / 4);
+        const float* np = nperm + part * (DHQK / 4);
+        float dot = 0.f;
 #pragma unroll 1
-            for (int d = 0; d < DHQK / 4; d += 8) {
-              const uint4 qv = *(const uint4*)(qrow + d);
-              const float4 na = *(const float4*)(np + d), nb4 = *(const float4*)(np + d + 4);
-              dot += lo2<F16>(qv.x) * na.x + hi2<F16>(qv.x) * na.y + lo2<F16>(qv.y) * na.z + hi2<F16>(qv.y) * na.w;
-              dot += lo2<F16>(qv.z) * nb4.x + hi2<F16>(qv.z) * nb4.y + lo2<F16>(qv.w) * nb4.z + hi2<F16>(qv.w) * nb4.w;
-            }
-            dot += __shfl_xor(dot, 1);
-            dot += __shfl_xor(dot, 2);
-            // parked in LDS until the row sums of the own chunk are complete: registers are what this kernel is short of
-            if (part == 0) {
-              denq[t] = cs0r * dot;
-              mcv[t] = mcr;
-            }
-          }
+        for (int d = 0; d < DHQK / 4; d += 8) {
+          const uint4 qv = *(const uint4*)(qrow + d);
+          const float4 na = *(const float4*)(np + d), nb4 = *(const float4*)(np + d + 4);
+          dot += lo2<F16>(qv.x) * na.x + hi2<F16>(qv.x) * na.y + lo2<F16>(qv.y) * na.z + hi2<F16>(qv.y) * na.w;
+          dot += lo2<F16>(qv.z) * nb4.x + hi2<F16>(qv.z) * nb4.y + lo2<F16>(qv.w) * nb4.z + hi2<F16>(qv.w) * nb4.w;
         }
-        if (si == 0) {
-          // (after the dot product above, which runs while no accumulator is live)
-#pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-              for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+        dot += __shfl_xor(dot, 1);
+        dot += __shfl_xor(dot, 2);
+        // parked in LDS until the row sums of the own chunk are complete: registers are what this kernel is short of
+        if (part == 0) {
+          denq[t] = cs0r * dot;
+          mcv[t] = mcr;
         }
-        const int le = opaque(lane);
-        const int r = le & 31, h = le >> 5;
-        const uint16_t* const slab = (si & 1) ? Ring1 : Ring0;
+      };
+      auto clear_acc = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int dsl = 0; dsl < 2; ++dsl) {
-          Frag A[MB], B[2];
-#pragma unroll
-          for (int mb = 0; mb < MB; ++mb) A[mb].u = *(const uint4*)(slab + ((MB * ci + mb) * 2 + dsl) * 512 + le * 8);
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb)
-            B[nb].u = *(const uint4*)(Ns + (64 * pi + 32 * nb + r) * QS + 16 * (2 * si + dsl) + 8 * h);
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
+            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+      };
+      // ---- inter-chunk product: Out^T = State^T Xn^T, two contraction steps per slab
+      __syncthreads();
+      if (!IS_DV) query_dot_n();
+      clear_acc();
+      if (it.no_state) {
+        __syncthreads();
+      } else {
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
+        for (int si = 0; si < 8; ++si) {
+          if (si > 0) __syncthreads();
+          const int le = opaque(lane);
+          const int r = le & 31, h = le >> 5;
+          const uint16_t* const slab = (si & 1) ? Ring1 : Ring0;
+#pragma unroll
+          for (int dsl = 0; dsl < 2; ++dsl) {
+            Frag A[MB], B[2];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) A[mb].u = *(const uint4*)(slab + ((MB * ci + mb) * 2 + dsl) * 512 + le * 8);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+              B[nb].u = *(const uint4*)(Ns + (64 * pi + 32 * nb + r) * QS + 16 * (2 * si + dsl) + 8 * h);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+              for (int nb = 0; nb < 2; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
+          }
         }
       }
       // (kept apart from the matrix instructions around it: interleaved with them the products land in fresh

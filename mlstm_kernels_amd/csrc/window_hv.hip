@@ -15,6 +15,8 @@
 //       O        NS steps [state fragments of 32 entries x CW | Q (K for dV) rows x 32]    Out^T  = State^T Xn^T
 //       V  max(2, CW / 64) steps [V (dH) rows x CW]                                        Out^T += Xw^T P
 //     A finished tile leaves during the first step of the next window's S (of several groups: each at its end).
+//   * A window whose state is known to be zero has no phase O (128 heads of 2048, 128/256: the call, forward and backward,
+//     487 -> 479 us with the same in window_qk.hip).
 //   * What bounds it: HBM.  Everything a window needs passes through the CU once, only the rows of O a second time: at
 //     128/256 384 KB in and 128 KB out per window where the tiled kernel moved 285 KB per 64 positions; a score block is
 //     computed once for all value columns of its group's window.
@@ -72,6 +74,10 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   const int NS = DHQK / 32, ND = DHQK / 16, NG = MULTI ? DHHV / CW : 1;
   const int NWIN = (NC + 1) / 2;  // the last window may hold one chunk only
   const size_t Sp = (size_t)NC * kChunk;
+  // without a state in front of the first window (behind the last one) phase O has nothing to add there and falls away; its
+  // q . n moves to the rows of phase S
+  const int zero_win = a.zero_state ? (IS_DV ? NWIN - 1 : 0) : -1;
+  const WinLight light(zero_win == 0 && !IS_DV, zero_win >= 0 && IS_DV, NWIN, n_items);
 
   if (wave_all >= 8) {
     // =========================================================================================== producer waves
@@ -123,7 +129,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   }
     WinItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
       const uint32_t pl = (uint32_t)opaque(p);
       const char* const Q_b = (const char*)a.Q + (size_t)it.bh * S * DHQK * 2;
       const char* const K_b = (const char*)a.K + (size_t)it.bh * S * DHQK * 2;
@@ -152,7 +158,8 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
           const uint32_t f0 = pl >> 6;
           const uint32_t sg = (((uint32_t)cg * (CW / 32) + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
           const uint32_t ss = 2 * (uint32_t)ND * 1024;
-          for (int w = 0; w < NS; w += 2) {
+          const int ns = it.win == zero_win ? 0 : NS;
+          for (int w = 0; w < ns; w += 2) {
             WH_PROC(0, St_b, sg + w * 2048, ss, 0xffffffffu, SP, Xn_b, xx + w * 64, xstep, xl + w * 64, 4, pl * 16, 16384 + xdp)
             WH_PROC(1, St_b, sg + (w + 1) * 2048, ss, 0xffffffffu, SP, Xn_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, 4,
                     pl * 16, 16384 + xdp)
@@ -315,10 +322,11 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   }
     bool first = true;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const int n_pos = RAGGED ? S - 256 * it.win : 256;
       const float g01 = a.g.graw[(size_t)bh * NC + c0];
+      const bool no_state = it.win == zero_win;
 
       if (first) request(it);
 
@@ -344,6 +352,22 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
             }
           }
         };
+        // q_t . n before the second chunk (before the first it is zero), as phase O does it with a state: two threads per
+        // position, 16 of the slab's 32 entries each, in the order of the fragments.  n4(e): entries e .. e + 3 of the sixteen
+        auto s_dot = [&](const unsigned char* slab, auto n4) __attribute__((always_inline)) {
+          const int td = opaque(tid);
+          const int t = td >> 1, part = td & 1;
+          const uint4 q0 = *(const uint4*)(slab + t * 64 + (((2 * part) ^ win_f64(t)) * 16));
+          const uint4 q1 = *(const uint4*)(slab + t * 64 + (((2 * part + 1) ^ win_f64(t)) * 16));
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const uint4 qv = x == 0 ? make_uint4(q0.x, q0.y, q1.x, q1.y) : make_uint4(q0.z, q0.w, q1.z, q1.w);
+            const float4 na = n4(4 * x), nb4 = n4(8 + 4 * x);
+            dot += lo2<F16>(qv.x) * na.x + hi2<F16>(qv.x) * na.y + lo2<F16>(qv.y) * na.z + hi2<F16>(qv.y) * na.w;
+            dot += lo2<F16>(qv.z) * nb4.x + hi2<F16>(qv.z) * nb4.y + lo2<F16>(qv.w) * nb4.z + hi2<F16>(qv.w) * nb4.w;
+          }
+        };
+        const bool with_dot = !IS_DV && no_state && a.use_nrow && tid >= 256;
         // (the first step stands before the loop: the finished tile that leaves in it must not be live around the loop)
         __syncthreads();
         const unsigned char* const first_slab = next_slab();
@@ -353,10 +377,22 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         for (int e = 0; e < 5; ++e)
 #pragma unroll
           for (int i = 0; i < 16; ++i) sacc[e][i] = 0.f;
+        if (with_dot) {  // n from memory: what was published in this step is not visible yet
+          const float* const np3 = a.nstates + ((size_t)bh * NC + min(c0 + 1, NC - 1)) * 3 * DHQK + 16 * (tid & 1);
+          s_dot(first_slab, [&](int e) {
+            const float4 x = *(const float4*)(np3 + e), y = *(const float4*)(np3 + DHQK + e), z = *(const float4*)(np3 + 2 * DHQK + e);
+            return make_float4((x.x + y.x) + z.x, (x.y + y.y) + z.y, (x.z + y.z) + z.z, (x.w + y.w) + z.w);
+          });
+        }
         s_step(first_slab);
         for (int w = 1; w < NS; ++w) {
           __syncthreads();
-          s_step(next_slab());
+          const unsigned char* const slab = next_slab();
+          if (with_dot) {
+            const float* const np = nvec + DHQK + 32 * w + 16 * (tid & 1);
+            s_dot(slab, [&](int e) { return *(const float4*)(np + e); });
+          }
+          s_step(slab);
         }
         // ---- gating: P = scores * exp(u_t - w_j + G) / sqrt(DHQK) (* rho_t), zero above the diagonal; forward: fp32 row
         // sums over the keys of the own chunk (the vectors were written at least one barrier ago)
@@ -433,23 +469,19 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
               for (int nb = 0; nb < NNB; ++nb) mfma32<F16>(acc[mb][nb], A[mb], B[nb]);
           }
         };
-        __syncthreads();
-        {
-          const unsigned char* const slab = next_slab();
 #pragma unroll
-          for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-            for (int nb = 0; nb < NNB; ++nb)
+          for (int nb = 0; nb < NNB; ++nb)
 #pragma unroll
-              for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
-          o_step(slab, 0);
-        }
-        for (int w = 1; w < NS; ++w) {
+            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
+        const int ns = no_state ? 0 : NS;
+        for (int w = 0; w < ns; ++w) {
           __syncthreads();
           o_step(next_slab(), w);
         }
-        if (!IS_DV && cg == 0) {
-          // ---- denominators (the row sums were written before this phase's first barrier)
+        // ---- denominators (the row sums were written before the barrier passed last)
+        auto denominators = [&]() __attribute__((always_inline)) {
           const int td = opaque(tid);
           const int t = td >> 1;
           dot += __shfl_xor(dot, 1);
@@ -473,7 +505,8 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
               if (a.m_out != nullptr) a.m_out[tg] = mc;
             }
           }
-        }
+        };
+        if (!IS_DV && cg == 0 && !no_state) denominators();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int nb = 0; nb < NNB; ++nb) {
@@ -488,6 +521,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         for (int z = 0; z < NVS; ++z) {
           __syncthreads();
           const unsigned char* const Zs = next_slab();
+          if (!IS_DV && z == 0 && cg == 0 && no_state) denominators();
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
           const int q16 = (le >> 4) & 1, i16 = le & 15;
@@ -568,7 +602,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       // the next window's vectors travel while this one's tile leaves (requested with that tile's successor they would
       // cost a trip to memory per window: dV 5 % slower)
       WinItem nx;
-      first = !(rd + 1 < n_rounds && win_decode(nx, rd + 1, vid, G, n_items, NWIN));
+      first = !(rd + 1 < n_rounds && win_decode(nx, rd + 1, vid, G, n_items, NWIN, light));
       if (!first) request(nx);
     }
     if (pending) {  // (a workgroup without a window passes no barrier at all, like its producers)

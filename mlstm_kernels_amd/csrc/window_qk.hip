@@ -28,6 +28,8 @@
 //     row dots come through the ring like every other operand (fetched by the consumers themselves they cost a
 //     memory latency per handful of positions); the rounded results pass through a private 2 KB staging tile per
 //     wave into row order and are stored as full 128-byte lines.
+//   * A window without a state on one side (no initial state, no gradient after the end) leaves out that phase's NV steps:
+//     the state and the second reading of dH (V), a quarter of a 256/512 window.
 // Supported: state stride 2, any head dimensions (multiples of 64; DHQK in tiles of 256, 128 or 64, whichever divides it).
 // Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 326 -> 170, 128/128 259 -> 119,
 // 64/128 244 -> 82, 64/64 with 524288 419 -> 119, 512/1024 with 32768 210 -> 191; 256/512 with 524288 1042 -> 780.
@@ -72,6 +74,9 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   const int NV = DHHV / 32;   // steps of 32 value columns (even)
   const int NWIN = (NC + 1) / 2;  // the last window may hold one chunk only: the other half of it is past the end
   const size_t Sp = (size_t)NC * kChunk;
+  // no initial state, no gradient after the last chunk: the steps that would multiply them fall away
+  const bool zero_c = __builtin_amdgcn_readfirstlane(*a.g.zero_c) != 0, zero_dc = a.zero_dc != 0;
+  const WinLight light(zero_c, zero_dc, NWIN, n_items);
 
   if (wave_all >= 8) {
     // =========================================================================================== producer waves
@@ -115,7 +120,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   }
     WinItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
       const uint32_t pl = (uint32_t)opaque(p);
       const char* const dH_b = (const char*)a.dH + (size_t)it.bh * S * DHHV * 2;
       const char* const V_b = (const char*)a.V + (size_t)it.bh * S * DHHV * 2;
@@ -179,7 +184,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       // ---- phase Q: C fragments | dH rows, then the K rows (products) and the Q rows (row dots)
       {
         const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16 + dg * (DT / 16) * 1024));
-        for (int w = 0; w < NV; w += 2) {
+        const int nv = zero_c && it.win == 0 ? 0 : NV;
+        for (int w = 0; w < nv; w += 2) {
           WQ_PROC(0, C_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
           WQ_PROC(1, C_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
@@ -188,7 +194,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       // ---- phase K: dC fragments | V rows, then the Q rows (products) and the K rows (row dots)
       {
         const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim), cc = (uint32_t)opaque((int)(pl * 16 + dg * (DT / 16) * 1024));
-        for (int w = 0; w < NV; w += 2) {
+        const int nv = zero_dc && it.win == NWIN - 1 ? 0 : NV;
+        for (int w = 0; w < nv; w += 2) {
           WQ_PROC(0, dC_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
           WQ_PROC(1, dC_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
         }
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     };
 
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const size_t hofs = (size_t)bh * Sp, gofs = hofs + (size_t)c0 * kChunk;
       const float* graw = a.g.graw + (size_t)bh * NC;
@@ -354,10 +361,12 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.f;
 
+        const bool no_state = dk ? zero_dc && it.win == NWIN - 1 : zero_c && it.win == 0;
         // ---- Out^T += State Xn^T over the value columns, 32 at a time.  The stored fragments (made for a contraction
         // over the head dimension) are read with the transposing LDS read: lane i16 of a 16-lane block addresses
         // value column k0 + i16 / 4 and the 4 consecutive head-dim rows n0 + 4 (i16 % 4) .. + 3
-        for (int w = 0; w < NV; ++w) {
+        const int nv = no_state ? 0 : NV;
+        for (int w = 0; w < nv; ++w) {
           __syncthreads();
           const unsigned char* const Cf = next_slab();
           if (w == 0) finish_rowdots();
@@ -399,7 +408,8 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int nb = 0; nb < NNB; ++nb) {
-          const float cs = csv[32 * (NPG * nb + pg) + (opaque(lane) & 31)];
+          // (without a state nothing was written there, and the accumulators are zero)
+          const float cs = no_state ? 0.f : csv[32 * (NPG * nb + pg) + (opaque(lane) & 31)];
 #pragma unroll
           for (int mb = 0; mb < 2; ++mb) acc[mb][nb] *= cs;
         }
@@ -411,6 +421,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         for (int z = 0; z < NDI; ++z) {
           __syncthreads();
           const unsigned char* const Zs = next_slab();
+          if (z == 0 && no_state) finish_rowdots();
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
           const int q16 = (le >> 4) & 1, i16 = le & 15;

@@ -178,6 +178,39 @@ def test_state_tiles_on_persistent_workgroups(DQ, DV, BH, S, last, stride, init)
         assert torch.equal(a, b)
 
 
+# States that are known to be zero are neither written nor multiplied: the same bits as with zeros handed over, whatever the
+# workspace holds (it is taken from memory full of NaN), for one window, several, and a ragged last one of either length.
+@pytest.mark.parametrize("DQ,DV,path", [(256, 512, "auto"), (256, 512, "stream"), (256, 512, "split"), (64, 64, "auto"), (128, 256, "auto"),
+                                        (512, 512, "auto"), (128, 128, "split")])
+@pytest.mark.parametrize("NH,S", [(1, 64), (2, 256), (3, 384), (2, 600), (96, 700), (40, 1300)])
+@pytest.mark.parametrize("stride,sig,dtype", [(2, False, torch.bfloat16), (2, True, torch.float16), (3, False, torch.bfloat16)], ids=str)
+def test_zero_states_that_are_left_out(DQ, DV, path, NH, S, stride, sig, dtype):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    if path == "stream":
+        S = (S + 127) // 128 * 128
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(1, NH, S, DQ, DV, seed=S, dtype=dtype, f_offset=3.0))
+    dH = torch.randn(1, NH, S, DV, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    zeros = [torch.zeros(1, NH, *d, device="cuda") for d in ((DQ, DV), (DQ,), (1,))]
+    out = []
+    for init, d_last in ((None, False), (zeros, True)):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v, i, f)]
+        st = dict(zip(("c_initial", "n_initial", "m_initial"), init)) if init else {}
+        torch.cuda.empty_cache()
+        full = torch.full((1 << 28,), float("nan"), device="cuda")
+        del full
+        H, last = op(*leaves, **st, return_last_states=True, any_sequence_length=True, kernel_path=path, chunk_size_intra=128 * stride)
+        if d_last:
+            grads = torch.autograd.grad((H, last[0]), leaves, (dH, torch.zeros_like(last[0])))
+        else:
+            grads = torch.autograd.grad(H, leaves, dH)
+        out.append([H.detach(), *(t.detach() for t in last), *grads])
+    for name, a, b in zip(("H", "C", "n", "m", "dQ", "dK", "dV", "dI", "dF"), *out):
+        assert torch.equal(a, b), name
+        assert bool(torch.isfinite(a).all()), name
+
+
 @pytest.mark.parametrize("S,DQ,DV,NH", [(1100, 64, 64, 4), (1100, 128, 128, 2), (300, 256, 512, 5), (700, 256, 512, 26)])
 def test_items_that_are_no_multiple_of_eight(S, DQ, DV, NH):
     _run(S, DQ, DV, NH=NH, seed=S + NH)
