@@ -287,6 +287,31 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     return check_launch("fused_hv forward");
   }
 
+  if (path == MLSTM_PATH_AUTO && !keep_for_backward && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr)) {
+    mlstm::ShortFwArgs fa;
+    memset(&fa, 0, sizeof(fa));
+    fa.Q = (const uint16_t*)q; fa.K = (const uint16_t*)k; fa.V = (const uint16_t*)v;
+    fa.g = ws.g;
+    fa.Out = (uint16_t*)H;
+    fa.n_out = n_out; fa.m_out = m_out;
+    fa.init = c0;
+    fa.n_init = n0;
+    fa.final_out = c_last;
+    fa.n_final = track_n ? n_last : nullptr;
+    fa.S = S; fa.NC = NC; fa.DHQK = DHQK; fa.DHHV = DHHV;
+    fa.qk_scale = 1.0f / sqrtf((float)DHQK); fa.eps = eps;
+    fa.sig_gate = sig;
+    fa.use_nrow = track_n;
+    fa.f16 = f16;
+    if (mlstm::short_fw_preferred(fa, BH)) {
+      {
+        ProfileScope ps("short_fw", st);
+        if (const char* e = mlstm::launch_short_fw(fa, BH, st)) return fail(e);
+      }
+      return check_launch("short_fw");
+    }
+  }
+
   mlstm::ParHvArgs pa;
   memset(&pa, 0, sizeof(pa));
   pa.Q = (const uint16_t*)q; pa.K = (const uint16_t*)k; pa.V = (const uint16_t*)v;

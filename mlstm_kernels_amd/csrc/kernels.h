@@ -133,6 +133,23 @@ struct FusedHvArgs {
   int stride;               // a chunk state is emitted every `stride` chunks
 };
 
+constexpr int kShortMax = 512;  // longest sequence of the short forward
+struct ShortFwArgs {
+  const uint16_t *Q, *K, *V;
+  GateBufs g;
+  uint16_t* Out;            // (B,NH,S,DHHV)
+  float* n_out;             // optional (B,NH,S)
+  float* m_out;             // optional (B,NH,S)
+  const float* init;        // (B,NH,DHQK,DHHV) or nullptr
+  const float* n_init;      // (B,NH,DHQK), with init
+  float* final_out;         // (B,NH,DHQK,DHHV) fp32 or nullptr
+  float* n_final;           // (B,NH,DHQK) or nullptr (also: n is not tracked)
+  int S, NC, DHQK, DHHV;
+  float qk_scale, eps;
+  int sig_gate, use_nrow;
+  int f16;
+};
+
 struct ParQkArgs {
   const uint16_t *Q, *K, *V, *dH;
   GateBufs g;
@@ -190,6 +207,9 @@ const char* launch_stream_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t
 bool window_hv_supported(const ParHvArgs& a);
 bool window_hv_preferred(const ParHvArgs& a, int BH);  // supported, and faster than the tiled kernel at this size
 const char* launch_window_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
+// forward without backward of a short sequence: H and the last state in one launch
+bool short_fw_preferred(const ShortFwArgs& a, int BH);
+const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream);
 const char* launch_head_norm_bw(const HeadNormBwArgs& a, hipStream_t stream);
 bool fused_hv_supported(int DHQK, int DHHV);
 const char* launch_fused_hv(const FusedHvArgs& a, int BH, bool is_dv, hipStream_t stream);

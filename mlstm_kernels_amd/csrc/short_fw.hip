@@ -1,0 +1,540 @@
+// Forward of short sequences (up to 512 positions) without a backward: prompts.
+//
+//   H[t]    = (cs_t C0^T q_t + sum_{j <= t} P[t][j] v_j) / (normaliser_t + eps),
+//   P[t][j] = (q_t . k_j) / sqrt(DHQK) * exp(u_t - w_j + G)
+//   C_c     = gbar_c C_{c-1} + sum_{j in c} abar_j k_j v_j^T,   n_c = gbar_c n_{c-1} + sum_{j in c} abar_j k_j
+//
+// with the gate vectors of gates.hip (G: the decay of the chunks between those of j and t; cs_t: bbar_t / sqrt(DHQK) and the
+// decay of the chunks in front of t's).  Where the whole sequence is one
+// group of source chunks no chunk state is needed: H takes all keys as score blocks, and the last state is one product over all
+// positions.  Neither waits for the other, so ONE launch holds the workgroups of both:
+//   * H: 64 positions x CW value columns of a (batch, head).  Its eight waves take the blocks of 32 keys in turn, fetch their
+//     K rows straight into operand registers (a whole block at once: one trip to memory), multiply them with the Q rows in LDS
+//     and write the gated block to LDS as 16-bit values; then V goes through two LDS slabs of 64 keys, all of it requested at
+//     the start.  An initial state (INIT) goes through the same slabs first, 64 of its rows at a time, with the Q rows in the
+//     place of P.
+//   * C: a tile of RT x WT of the state.  All rows are requested at the start as well; V is scaled in fp32 and split into a 16-bit
+//     head and a 16-bit remainder, two products per block, as in the scan.
+// What bounds it: latency, four trips to memory or LDS in a row and the matrix work of one workgroup.  The streaming kernels
+// take this in three launches (gates, a scan of up to four chunks that run twice, H from the chunk states), each with most of
+// the chip idle.
+#include "common.h"
+#include "kernels.h"
+
+namespace mlstm {
+namespace {
+constexpr int kShortThreads = 512;
+constexpr int kShortSlabs = kShortMax / 64;  // slabs of 64 positions at most
+
+template <int DQ, int CW, bool INIT>
+struct ShortLds {
+  // H: [Q rows, then (INIT: behind them) two slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs]
+  static constexpr int QS = DQ + 8, VS = CW + 32;
+  static constexpr int kFront = INIT ? 64 * QS + 2 * 64 * VS : (64 * QS > 2 * 64 * VS ? 64 * QS : 2 * 64 * VS);
+  static constexpr int RT = DQ % 128 == 0 ? 128 : 64, WT = CW;  // state tile
+  static constexpr int XS = RT + 32, YS = WT + 32;
+  static size_t bytes(int nt, bool with_c) {
+    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 17 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 64) * 4 : 0);
+    // C: [K slab | head of V | remainder of V | abar | abar as an operand]
+    const size_t c = (size_t)64 * (XS + 2 * YS) * 2 + kShortMax * 4 + kShortMax * 3 * 2;
+    return with_c && c > h ? c : h;
+  }
+};
+
+template <int DQ, int CW, bool F16, bool INIT>
+__device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned char* smem) {
+  using L = ShortLds<DQ, CW, INIT>;
+  constexpr int QS = L::QS, VS = L::VS;
+  constexpr int NF = DQ / 16 < 16 ? DQ / 16 : 16;  // fragments of a K block that are fetched at once
+  constexpr int NGK = DQ / 16 / NF;                // ... so many times
+  constexpr int QV = DQ / 64, VV = CW / 64;        // 16-byte pieces per thread: Q rows, a slab of V
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int S = a.S, DHHV = a.DHHV, NC = a.NC, nt = (S + 63) / 64, ng = DHHV / CW;
+  const int g = item % ng, tq = nt - 1 - (item / ng) % nt, bh = item / (ng * nt);  // the longest first
+  const int t0 = 64 * tq, c = t0 / kChunk;
+  const int PSS = 64 * nt + 8;
+  uint16_t* const Qs = (uint16_t*)smem;
+  uint16_t* const Vs = INIT ? Qs + 64 * QS : Qs;  // (without a state Q is done with before V comes)
+  uint16_t* const Ps = Qs + L::kFront;
+  float* const wv = (float*)(Ps + 64 * PSS);
+  float* const rows = wv + kShortMax;  // [16 key blocks][64]
+  float* const inv = rows + 17 * 64;
+  float* const nv = inv + 64;    // INIT: n0
+  float* const csv = nv + DQ;    // INIT: cs_t
+  const size_t Sp = (size_t)NC * kChunk, gofs = (size_t)bh * Sp;
+  const uint16_t* const Qg = a.Q + (size_t)bh * S * DQ;
+  const uint16_t* const Kg = a.K + (size_t)bh * S * DQ;
+  const uint16_t* const Vg = a.V + (size_t)bh * S * DHHV + g * CW;
+  const int n_kb = min(2 * tq + 2, (S + 31) / 32);  // blocks of 32 keys
+  const int n_sl = tq + 1;                          // slabs of 64 keys
+
+  // ---- everything this workgroup needs is requested here, in the order of its use
+  u32x4 qr[QV];
+#pragma unroll
+  for (int x = 0; x < QV; ++x) {
+    const int idx = tid + x * kShortThreads, row = idx / (DQ / 8), u = idx % (DQ / 8);
+    qr[x] = *(const u32x4*)(Qg + (size_t)min(t0 + row, S - 1) * DQ + u * 8);
+  }
+  // (the gate vectors cover whole chunks: positions past the end have w = infinity, a factor of zero)
+  const float w_own = tid < 64 * n_sl ? a.g.w[gofs + tid] : 0.f;
+  float un[2];
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb) un[tb] = a.g.u[gofs + t0 + 32 * tb + r];
+  const float mc = tid < 64 ? a.g.mcomb[gofs + t0 + tid] : 0.f;
+  Frag k0[NF], k1[NF];
+  // unit x of a wave: key block wave + 8 (x / NGK), fragments NF (x % NGK) ..
+  const int n_units = NGK * ((wave < n_kb ? 1 : 0) + (wave + 8 < n_kb ? 1 : 0));
+  auto fetch = [&](Frag (&f)[NF], int x) __attribute__((always_inline)) {
+    const int j = min(32 * (wave + 8 * (x / NGK)) + r, S - 1);
+    const uint16_t* const p = Kg + (size_t)j * DQ + (x % NGK) * (NF * 16) + 8 * h;
+#pragma unroll
+    for (int ks = 0; ks < NF; ++ks) f[ks].u = *(const uint4*)(p + 16 * ks);
+  };
+  if (n_units > 0) fetch(k0, 0);
+  u32x4 vr[kShortSlabs][VV];
+#pragma unroll
+  for (int s = 0; s < kShortSlabs; ++s)
+    if (s < n_sl) {
+#pragma unroll
+      for (int x = 0; x < VV; ++x) {
+        const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+        vr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
+      }
+    }
+
+#pragma unroll
+  for (int x = 0; x < QV; ++x) {
+    const int idx = tid + x * kShortThreads, row = idx / (DQ / 8), u = idx % (DQ / 8);
+    *(u32x4*)(Qs + row * QS + u * 8) = qr[x];
+  }
+  if (tid < 64 * n_sl) wv[tid] = w_own;
+  if constexpr (INIT) {
+    if (tid < DQ) nv[tid] = a.use_nrow ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
+    if (tid < 64) {
+      float gsum = 0.f;
+      for (int y = 0; y < c; ++y) gsum += a.g.graw[(size_t)bh * NC + y];
+      const float* const mst = a.g.mstates + (size_t)bh * (NC + 1);
+      csv[tid] = a.g.bbar[gofs + t0 + tid] * a.qk_scale * (c > 0 ? __expf(gsum + mst[0] - mst[c]) : 1.f);
+    }
+  }
+  __syncthreads();
+
+  if constexpr (INIT) {
+    // q_t . n0, eight threads per position
+    const int t = tid >> 3, part = tid & 7;
+    float dot = 0.f;
+#pragma unroll
+    for (int d = 0; d < DQ / 8; d += 4) {
+      const uint2 qv = *(const uint2*)(Qs + t * QS + part * (DQ / 8) + d);
+      const float4 n4 = *(const float4*)(nv + part * (DQ / 8) + d);
+      dot += lo2<F16>(qv.x) * n4.x + hi2<F16>(qv.x) * n4.y + lo2<F16>(qv.y) * n4.z + hi2<F16>(qv.y) * n4.w;
+    }
+    dot += __shfl_xor(dot, 1);
+    dot += __shfl_xor(dot, 2);
+    dot += __shfl_xor(dot, 4);
+    if (part == 0) rows[16 * 64 + t] = csv[t] * dot;
+  }
+  // ---- scores of this wave's key blocks, gated into P
+  {
+    const float lq = __log2f(a.qk_scale);
+    f32x16 sacc[2];
+    auto unit = [&](const Frag (&f)[NF], int x) __attribute__((always_inline)) {
+      const int kb = wave + 8 * (x / NGK), gk = x % NGK;
+      if (gk == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sacc[0][i] = sacc[1][i] = 0.f;
+      }
+#pragma unroll
+      for (int ks = 0; ks < NF; ++ks)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+          Frag B;
+          B.u = *(const uint4*)(Qs + (32 * tb + r) * QS + (gk * NF + ks) * 16 + 8 * h);
+          mfma32<F16>(sacc[tb], f[ks], B);  // rows: keys, columns: positions
+        }
+      if (gk == NGK - 1) {
+        float G = 0.f;  // decay of the chunks between the keys' and the positions'
+        for (int y = kb / 4; y < c; ++y) G += a.g.graw[(size_t)bh * NC + y];
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+          const int diag = 2 * tq + tb;  // key block of the positions themselves
+          if (kb <= diag) {
+            float rsum = 0.f;
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+              const int j0 = 8 * g4 + 4 * h;
+              const float4 wj = *(const float4*)(wv + 32 * kb + j0);
+              const float w4[4] = {wj.x, wj.y, wj.z, wj.w};
+              float p[4];
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const float e2 = __builtin_amdgcn_exp2f(__builtin_fmaf(un[tb] + G - w4[q], 1.4426950408889634f, lq));
+                p[q] = kb < diag || j0 + q <= r ? sacc[tb][4 * g4 + q] * e2 : 0.f;
+                rsum += p[q];
+              }
+              *(uint2*)(Ps + (32 * tb + r) * PSS + 32 * kb + j0) = make_uint2(pack2<F16>(p[0], p[1]), pack2<F16>(p[2], p[3]));
+            }
+            const float tot = rsum + __shfl_xor(rsum, 32);
+            if (h == 0) rows[kb * 64 + 32 * tb + r] = tot;
+          }
+        }
+      }
+    };
+    for (int x = 0; x < n_units; x += 2) {
+      if (x + 1 < n_units) fetch(k1, x + 1);
+      unit(k0, x);
+      if (x + 1 < n_units) {
+        if (x + 2 < n_units) fetch(k0, x + 2);
+        unit(k1, x + 1);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- denominators; Out^T += V^T P over the keys, 64 at a time
+  if (tid < 64) {
+    float iv = 1.f, nmax = 1.f;
+    if (a.use_nrow) {
+      float den = INIT ? rows[16 * 64 + tid] : 0.f;
+      for (int kb = 0; kb <= 2 * tq + tid / 32 && kb < n_kb; ++kb) den += rows[kb * 64 + tid];
+      nmax = fmaxf(fabsf(den), a.sig_gate ? 1.f : __expf(-mc));
+      iv = 1.f / (nmax + a.eps);
+    }
+    inv[tid] = iv;
+    if (g == 0 && t0 + tid < S) {
+      const size_t tg = (size_t)bh * S + t0 + tid;
+      if (a.n_out != nullptr) a.n_out[tg] = nmax;
+      if (a.m_out != nullptr) a.m_out[tg] = mc;
+    }
+  }
+  constexpr int NCB = CW / 32;  // column blocks of 32: one and 32 positions for each wave (CW = 64: for four of them)
+  const int cb = wave % NCB, tb = wave / NCB;
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  constexpr int kOdd = INIT ? (DQ / 64) & 1 : 0;  // the first slab of V does not go where the last one of C0 is read
+  auto store_slab = [&](int s, const u32x4 (&v)[VV]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < VV; ++x) {
+      const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+      const u32x4 none = {0u, 0u, 0u, 0u};
+      *(u32x4*)(Vs + ((s + kOdd) & 1) * (64 * VS) + row * VS + u * 8) = 64 * s + row < S ? v[x] : none;
+    }
+  };
+  const int q16 = (lane >> 4) & 1, i16 = lane & 15;
+  const int krow = 8 * h + (i16 >> 2), ncol = 16 * q16 + 4 * (i16 & 3);
+  if constexpr (INIT) {
+    // Out^T = C0^T Q^T over the head dimension, 64 rows of C0 at a time, rounded like every state that is multiplied
+    const float* const Cg = a.init + (size_t)bh * DQ * DHHV + g * CW;
+    f32x4 cr[2][VV][2];
+    auto fetch_c = [&](f32x4 (&x)[VV][2], int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int y = 0; y < VV; ++y) {
+        const int idx = tid + y * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+        const float* const p = Cg + (size_t)(64 * s + row) * DHHV + u * 8;
+        x[y][0] = *(const f32x4*)p;
+        x[y][1] = *(const f32x4*)(p + 4);
+      }
+    };
+    fetch_c(cr[0], 0);
+#pragma unroll
+    for (int s = 0; s < DQ / 64; ++s) {
+      if (s + 1 < DQ / 64) fetch_c(cr[(s + 1) & 1], s + 1);
+      uint16_t* const slab = Vs + (s & 1) * (64 * VS);
+#pragma unroll
+      for (int y = 0; y < VV; ++y) {
+        const int idx = tid + y * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+        const f32x4 lo = cr[s & 1][y][0], hi = cr[s & 1][y][1];
+        *(uint4*)(slab + row * VS + u * 8) = make_uint4(pack2<F16>(lo[0], lo[1]), pack2<F16>(lo[2], lo[3]), pack2<F16>(hi[0], hi[1]), pack2<F16>(hi[2], hi[3]));
+      }
+      __syncthreads();
+      if (tb < 2) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          Frag A, B;
+          const uint16_t* const p = slab + (16 * kk + krow) * VS + 32 * cb + ncol;
+          A.d[0] = lds_read_tr16(p);
+          A.d[1] = lds_read_tr16(p + 4 * VS);
+          B.u = *(const uint4*)(Qs + (32 * tb + r) * QS + 64 * s + 16 * kk + 8 * h);
+          mfma32<F16>(acc, A, B);
+        }
+      }
+    }
+    if (tb < 2) acc *= csv[32 * tb + r];
+  }
+  store_slab(0, vr[0]);
+#pragma unroll
+  for (int s = 0; s < kShortSlabs; ++s)
+    if (s < n_sl) {
+      __syncthreads();
+      if (s + 1 < kShortSlabs && s + 1 < n_sl) store_slab(s + 1, vr[s + 1 < kShortSlabs ? s + 1 : s]);
+      // key blocks above the diagonal are left out: zero times a NaN or infinity in V would be NaN
+      const uint16_t* const slab = Vs + ((s + kOdd) & 1) * (64 * VS);
+      if (tb < 2) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+          if (2 * s + kk / 2 <= 2 * tq + tb) {
+            Frag A, B;
+            const uint16_t* const p = slab + (16 * kk + krow) * VS + 32 * cb + ncol;
+            A.d[0] = lds_read_tr16(p);
+            A.d[1] = lds_read_tr16(p + 4 * VS);
+            B.u = *(const uint4*)(Ps + (32 * tb + r) * PSS + 64 * s + 16 * kk + 8 * h);
+            mfma32<F16>(acc, A, B);  // rows: value columns, columns: positions
+          }
+      }
+    }
+  __syncthreads();
+  // ---- rows out through LDS
+  constexpr int OS = CW + 8;
+  uint16_t* const Os = Vs;
+  if (tb < 2) {
+    const float iv = inv[32 * tb + r];
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4)
+      *(uint2*)(Os + (32 * tb + r) * OS + 32 * cb + 8 * g4 + 4 * h) =
+          make_uint2(pack2<F16>(acc[4 * g4] * iv, acc[4 * g4 + 1] * iv), pack2<F16>(acc[4 * g4 + 2] * iv, acc[4 * g4 + 3] * iv));
+  }
+  __syncthreads();
+  uint16_t* const Og = a.Out + ((size_t)bh * S + t0) * DHHV + g * CW;
+#pragma unroll
+  for (int x = 0; x < VV; ++x) {
+    const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+    if (t0 + row < S) *(u32x4*)(Og + (size_t)row * DHHV + u * 8) = *(const u32x4*)(Os + row * OS + u * 8);
+  }
+}
+
+template <int DQ, int CW, bool F16, bool INIT>
+__device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned char* smem) {
+  using L = ShortLds<DQ, CW, INIT>;
+  constexpr int RT = L::RT, WT = L::WT, XS = L::XS, YS = L::YS;
+  constexpr int XV = RT / 64, YV = WT / 64;          // 16-byte pieces per thread and slab
+  constexpr int NRB = RT / 32, NCB = WT / 32;        // blocks of 32 x 32
+  constexpr int NBW = NRB * NCB > 8 ? NRB * NCB / 8 : 1;  // blocks per wave, side by side
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  const int S = a.S, DHHV = a.DHHV, NC = a.NC;
+  constexpr int nx = DQ / RT;
+  const int ny = DHHV / WT;
+  const int bx = item % nx, by = (item / nx) % ny, bh = item / (nx * ny);
+  uint16_t* const Xs = (uint16_t*)smem;
+  uint16_t* const Yh = Xs + 64 * XS;
+  uint16_t* const Yl = Yh + 64 * YS;
+  float* const wt = (float*)(Yl + 64 * YS);
+  uint16_t* const nB = (uint16_t*)(wt + kShortMax);  // [position / 8][3][8]
+  const size_t Sp = (size_t)NC * kChunk;
+  const uint16_t* const Kg = a.K + (size_t)bh * S * DQ + bx * RT;
+  const uint16_t* const Vg = a.V + (size_t)bh * S * DHHV + by * WT;
+  const int n_sl = (S + 63) / 64;
+  {
+    // (the decay of later chunks is left to the sums: the largest weight of a chunk is one, and one times v has no remainder)
+    const float w = tid < S ? a.g.abar[(size_t)bh * Sp + tid] : 0.f;
+    wt[tid] = w;
+    // n as in the scan: the weights, split exactly into three 16-bit parts, are three columns of one more operand
+    uint16_t* const dst = nB + (tid >> 3) * 24 + (tid & 7);
+    const uint16_t p0 = f32_to_elem<F16>(w);
+    const float r1 = w - elem_to_f32<F16>(p0);
+    const uint16_t p1 = f32_to_elem<F16>(r1);
+    dst[0] = p0;
+    dst[8] = p1;
+    dst[16] = f32_to_elem<F16>(r1 - elem_to_f32<F16>(p1));
+  }
+  float gb[kShortMax / kChunk];
+#pragma unroll
+  for (int y = 0; y < kShortMax / kChunk; ++y) gb[y] = a.g.gbar[(size_t)bh * NC + min(y, NC - 1)];
+  u32x4 xr[kShortSlabs][XV], yr[kShortSlabs][YV];
+#pragma unroll
+  for (int s = 0; s < kShortSlabs; ++s)
+    if (s < n_sl) {
+#pragma unroll
+      for (int x = 0; x < XV; ++x) {
+        const int idx = tid + x * kShortThreads, row = idx / (RT / 8), u = idx % (RT / 8);
+        xr[s][x] = *(const u32x4*)(Kg + (size_t)min(64 * s + row, S - 1) * DQ + u * 8);
+      }
+#pragma unroll
+      for (int x = 0; x < YV; ++x) {
+        const int idx = tid + x * kShortThreads, row = idx / (WT / 8), u = idx % (WT / 8);
+        yr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
+      }
+    }
+  const int rb = wave % NRB, cb0 = wave / NRB * NBW;
+  const bool busy = cb0 < NCB;
+  f32x16 acc[NBW], rest[NBW];  // sums of the heads and of the remainders: a remainder does not cost the large sum a rounding
+#pragma unroll
+  for (int b = 0; b < NBW; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[b][i] = rest[b][i] = 0.f;
+  const bool with_n = a.n_final != nullptr && by == 0 && cb0 == 0;  // this wave carries n of its 32 rows
+  f32x16 accn;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) accn[i] = 0.f;
+  if constexpr (INIT) {
+    if (busy) {
+#pragma unroll
+      for (int b = 0; b < NBW; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int d = bx * RT + 32 * rb + 8 * (i / 4) + 4 * h + (i % 4);
+          acc[b][i] = a.init[((size_t)bh * DQ + d) * DHHV + by * WT + 32 * (cb0 + b) + r];
+        }
+    }
+    if (with_n && r == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) accn[i] = a.n_init[(size_t)bh * DQ + bx * RT + 32 * rb + 8 * (i / 4) + 4 * h + (i % 4)];
+    }
+  }
+  const int q16 = (lane >> 4) & 1, i16 = lane & 15;
+  const int krow = 8 * h + (i16 >> 2), ncol = 16 * q16 + 4 * (i16 & 3);
+#pragma unroll
+  for (int s = 0; s < kShortSlabs; ++s)
+    if (s < n_sl) {
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < XV; ++x) {
+        const int idx = tid + x * kShortThreads, row = idx / (RT / 8), u = idx % (RT / 8);
+        *(u32x4*)(Xs + row * XS + u * 8) = xr[s][x];
+      }
+#pragma unroll
+      for (int x = 0; x < YV; ++x) {
+        const int idx = tid + x * kShortThreads, row = idx / (WT / 8), u = idx % (WT / 8);
+        const float w = wt[64 * s + row];
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float e0 = lo2<F16>(yr[s][x][e]) * w, e1 = hi2<F16>(yr[s][x][e]) * w;
+          // (head and remainder of the same fp32 product: to float16 it may be converted and multiplied in one step)
+          if constexpr (F16) asm("" : "+v"(e0), "+v"(e1));
+          hi[e] = pack2<F16>(e0, e1);
+          lo[e] = pack2<F16>(e0 - lo2<F16>(hi[e]), e1 - hi2<F16>(hi[e]));
+        }
+        *(uint4*)(Yh + row * YS + u * 8) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *(uint4*)(Yl + row * YS + u * 8) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      }
+      __syncthreads();
+      if (s % 2 == 0 && (INIT || s > 0)) {
+#pragma unroll
+        for (int b = 0; b < NBW; ++b) {
+          acc[b] *= gb[s / 2];
+          rest[b] *= gb[s / 2];
+        }
+        accn *= gb[s / 2];
+      }
+      if (busy) {
+#pragma unroll
+        for (int js = 0; js < 4; ++js) {
+          Frag A;
+          const uint16_t* const p = Xs + (16 * js + krow) * XS + 32 * rb + ncol;
+          A.d[0] = lds_read_tr16(p);
+          A.d[1] = lds_read_tr16(p + 4 * XS);
+#pragma unroll
+          for (int b = 0; b < NBW; ++b) {
+            const int o = (16 * js + krow) * YS + 32 * (cb0 + b) + ncol;
+            Frag Bh, Bl;
+            Bh.d[0] = lds_read_tr16(Yh + o);
+            Bh.d[1] = lds_read_tr16(Yh + o + 4 * YS);
+            Bl.d[0] = lds_read_tr16(Yl + o);
+            Bl.d[1] = lds_read_tr16(Yl + o + 4 * YS);
+            mfma32<F16>(acc[b], A, Bh);
+            mfma32<F16>(rest[b], A, Bl);
+          }
+          if (with_n) {
+            Frag Bn;
+            Bn.u = *(const uint4*)(nB + (8 * s + 2 * js + h) * 24 + min(r, 2) * 8);
+            if (r >= 3) Bn.u = make_uint4(0u, 0u, 0u, 0u);
+            mfma32<F16>(accn, A, Bn);
+          }
+        }
+      }
+    }
+  if (busy) {
+#pragma unroll
+    for (int b = 0; b < NBW; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int d = bx * RT + 32 * rb + 8 * (i / 4) + 4 * h + (i % 4);
+        a.final_out[((size_t)bh * DQ + d) * DHHV + by * WT + 32 * (cb0 + b) + r] = acc[b][i] + rest[b][i];
+      }
+  }
+  if (with_n) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float x = accn[i];
+      const float sum = __shfl(x, 32 * h) + __shfl(x, 32 * h + 1) + __shfl(x, 32 * h + 2);
+      if (r == 0) a.n_final[(size_t)bh * DQ + bx * RT + 32 * rb + 8 * (i / 4) + 4 * h + (i % 4)] = sum;
+    }
+  }
+}
+
+}  // namespace
+
+template <int DQ, int CW, bool F16, bool INIT>
+__global__ __launch_bounds__(kShortThreads) void short_fw_kernel(ShortFwArgs a, int n_h, int n_c) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  // consecutive items (of one head) share an XCD and the head's rows in its L2
+  int b = blockIdx.x;
+  const bool is_h = b < n_h;
+  if (!is_h) b -= n_h;
+  const int n = is_h ? n_h : n_c;
+  if (n_h % 8 == 0 && n % 8 == 0) b = (b % 8) * (n / 8) + b / 8;
+  if (is_h) short_h<DQ, CW, F16, INIT>(a, b, smem_raw);
+  else short_c<DQ, CW, F16, INIT>(a, b, smem_raw);
+}
+
+namespace {
+template <int DQ, int CW, bool F16, bool INIT>
+const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  using L = ShortLds<DQ, CW, INIT>;
+  const int nt = (a.S + 63) / 64;
+  const long long n_h = (long long)BH * nt * (a.DHHV / CW);
+  const long long n_c = a.final_out == nullptr ? 0 : (long long)BH * (DQ / L::RT) * (a.DHHV / L::WT);
+  if (n_h + n_c >= (1ll << 31)) return "short_fw: too many workgroups";
+  const size_t smem = L::bytes(nt, n_c > 0);
+  if (smem > 160 * 1024) return "short_fw: too long for one CU's LDS";
+  static LdsLimit lds;
+  if (!lds.allow((const void*)short_fw_kernel<DQ, CW, F16, INIT>, smem)) return "short_fw: cannot raise the dynamic LDS limit";
+  hipLaunchKernelGGL((short_fw_kernel<DQ, CW, F16, INIT>), dim3((unsigned)(n_h + n_c)), dim3(kShortThreads), smem, stream, a, (int)n_h, (int)n_c);
+  return nullptr;
+}
+template <int DQ, int CW>
+const char* launch_short_c(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  if (a.init != nullptr)
+    return a.f16 ? launch_short_t<DQ, CW, true, true>(a, BH, stream) : launch_short_t<DQ, CW, false, true>(a, BH, stream);
+  return a.f16 ? launch_short_t<DQ, CW, true, false>(a, BH, stream) : launch_short_t<DQ, CW, false, false>(a, BH, stream);
+}
+template <int DQ>
+const char* launch_short_d(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  return a.DHHV % 128 == 0 ? launch_short_c<DQ, 128>(a, BH, stream) : launch_short_c<DQ, 64>(a, BH, stream);
+}
+}  // namespace
+
+// Where this kernel is the faster one: a workgroup of H takes 5 to 13 us by its number of keys and a CU one at a time, so with
+// many heads the streaming kernels, which keep the memory system busy, overtake it -- the sooner the longer the sequence.  The
+// line (positions in 64s times workgroups of H, per CU) from gates + scan + H against gates + this, us, at 256/512, 8 heads a
+// sequence: 200 positions B=4 48.1 / 36.6, B=8 63.5 / 60.0, B=16 95 / 103; 317: B=1 42.9 / 22.9, B=4 50.8 / 46.4, B=8 73 / 77;
+// 512: B=1 42.8 / 29.1, B=2 45.1 / 47.5, B=4 52 / 74.  At 128/256, 16 heads: 200 B=8 52.9 / 48.1, B=16 71.5 / 81.4; 512 B=2
+// 40.6 / 39.5, B=4 49 / 63; 64/64, 8 heads: 512 B=8 36.7 / 31.5, B=16 39.4 / 50.7; 512/1024, 4 heads: 512 B=2 70 / 57, B=4
+// 86 / 102.  An initial state counts as two more slabs: 256/512, 200 positions B=4 49.9 / 43.6, B=8 66.0 / 72.7, 512 positions
+// B=1 44.5 / 34.9, B=2 47.4 / 55.1.  Up to 128 positions it wins at every size (256/512, B=64: 264 / 206, with 64 positions 236 / 120).
+bool short_fw_preferred(const ShortFwArgs& a, int BH) {
+  if (a.S > kShortMax || a.DHHV % 64 != 0) return false;
+  if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256 && a.DHQK != 512) return false;
+  if (a.DHQK == 512 && a.init != nullptr && a.S > 320) return false;  // LDS
+  if ((uintptr_t)a.init % 16 != 0) return false;                      // (read by fours; the scan reads it one by one)
+  const long long nt = (a.S + 63) / 64;
+  return nt <= 2 || BH * nt * (a.DHHV / (a.DHHV % 128 == 0 ? 128 : 64)) * (nt + (a.init != nullptr ? 2 : 0)) <= 16ll * device_cu_count();
+}
+
+const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  if (a.S < 1 || a.S > kShortMax || a.NC != (a.S + kChunk - 1) / kChunk || a.DHHV % 64 != 0) return "short_fw: unsupported shape";
+  if (a.n_final != nullptr && a.final_out == nullptr) return "short_fw: n_last without c_last";
+  if ((uintptr_t)a.init % 16 != 0) return "short_fw: the initial state must lie at a multiple of 16 bytes";
+  switch (a.DHQK) {
+    case 64: return launch_short_d<64>(a, BH, stream);
+    case 128: return launch_short_d<128>(a, BH, stream);
+    case 256: return launch_short_d<256>(a, BH, stream);
+    case 512: return launch_short_d<512>(a, BH, stream);
+    default: return "short_fw: unsupported head dimension";
+  }
+}
+
+}  // namespace mlstm

@@ -178,6 +178,58 @@ def test_state_tiles_on_persistent_workgroups(DQ, DV, BH, S, last, stride, init)
         assert torch.equal(a, b)
 
 
+# The forward of short prompts (H and the last state in one launch) at either side of its blocks of 32, of its slabs of 64, of a
+# chunk and of its longest sequence; every head dimension it is built for and two it leaves to the other kernels.  H as above (the
+# gated scores and the products are rounded once each); the last state carries 16 bits of every value and 24 of every weight:
+# 2^-16 of the terms, whose sums are a few times smaller than their terms.
+@pytest.mark.parametrize("S", [1, 31, 33, 63, 64, 65, 127, 128, 129, 257, 320, 321, 449, 512, 513])
+@pytest.mark.parametrize("DQ,DV", [(64, 64), (64, 128), (128, 192), (128, 256), (256, 64), (256, 512), (512, 64), (512, 128), (192, 128)])
+@pytest.mark.parametrize("opt", [dict(), dict(init=True), dict(sig=True, dtype=torch.float16), dict(sig=True, init=True, normalize=False)], ids=str)
+def test_short_prompts(S, DQ, DV, opt):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    sig, init, dtype, normalize = opt.get("sig", False), opt.get("init", False), opt.get("dtype", torch.bfloat16), opt.get("normalize", True)
+    NH = 3
+    q, k, v, i, f = make_qkvif(1, NH, S, DQ, DV, seed=S + DQ, dtype=dtype, f_offset=3.0)
+    g = torch.Generator().manual_seed(S)
+    st = [None] * 3
+    if init:
+        st = [torch.randn(1, NH, DQ, DV, generator=g), torch.randn(1, NH, DQ, generator=g), None if sig else torch.randn(1, NH, 1, generator=g)]
+    d = lambda t: None if t is None else t.double()
+    L = next(x for x in (64, 32, 16, 8, 4, 2, 1) if S % x == 0)
+    okw = dict(normalize=normalize) if sig else {}
+    ref = O.chunkwise_fw(d(q), d(k), d(v), d(i), d(f), *(d(t) for t in st), chunk_size=L, siging=sig, **okw)
+    cu = lambda t: None if t is None else t.cuda()
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    for last in (True, False):
+        with torch.no_grad():
+            out = op(*(t.cuda() for t in (q, k, v, i, f)), *(cu(t) for t in st), return_last_states=last, any_sequence_length=True, **okw)
+        H = out[0] if last else out
+        assert rel_norm(H, ref["H"]) <= 6e-3
+        if last:
+            assert rel_norm(out[1][0], ref["C_last"]) <= 5e-5
+            if normalize:
+                assert rel_norm(out[1][1], ref["n_last"]) <= 5e-6
+            if not sig:
+                assert float((out[1][2].double().cpu() - ref["m_last"].reshape(out[1][2].shape)).abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("S,pos", [(40, 0), (200, 63), (317, 130), (512, 511)])
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_short_prompts_values_not_finite(S, pos, which, bad):
+    """A NaN or infinity at one position reaches no row more than 31 positions in front of it (its own block of 32 keys)."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    x = dict(zip("qkvif", (t.cuda() for t in make_qkvif(1, 2, S, 128, 128, seed=S, f_offset=3.0))))
+    x[which][0, 0, pos, 5] = bad
+    with torch.no_grad():
+        H, _ = mlstm_chunkwise__hip_xl_chunk(*x.values(), return_last_states=True, any_sequence_length=True)
+    assert bool(torch.isfinite(H[0, 1]).all()) and bool(torch.isfinite(H[0, 0, :pos // 32 * 32]).all())
+    if which == "q":
+        assert bool(torch.isfinite(H[0, 0, pos + 1:]).all())
+
+
 # States that are known to be zero are neither written nor multiplied: the same bits as with zeros handed over, whatever the
 # workspace holds (it is taken from memory full of NaN), for one window, several, and a ragged last one of either length.
 @pytest.mark.parametrize("DQ,DV,path", [(256, 512, "auto"), (256, 512, "stream"), (256, 512, "split"), (64, 64, "auto"), (128, 256, "auto"),
