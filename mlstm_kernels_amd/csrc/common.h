@@ -94,6 +94,14 @@ __device__ __forceinline__ void mfma32(f32x16& acc, const Frag& a, const Frag& b
   else acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, acc, 0, 0, 0);
 }
 
+// D(16x16) += A(16x32) * B(32x16).  lane l: A frag: A[l % 16][8 (l / 16) ..]; B frag: B[8 (l / 16) ..][l % 16];
+// acc[i] = D[4 (l / 16) + i][l % 16].
+template <bool F16>
+__device__ __forceinline__ void mfma16(f32x4& acc, const Frag& a, const Frag& b) {
+  if constexpr (F16) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hv, b.hv, acc, 0, 0, 0);
+  else acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc, 0, 0, 0);
+}
+
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 // Transposing 64-bit LDS read.  Within each block of 16 lanes, lane i must pass the address of the 4

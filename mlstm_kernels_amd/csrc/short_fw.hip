@@ -8,11 +8,14 @@
 // decay of the chunks in front of t's).  Where the whole sequence is one
 // group of source chunks no chunk state is needed: H takes all keys as score blocks, and the last state is one product over all
 // positions.  Neither waits for the other, so ONE launch holds the workgroups of both:
-//   * H: 64 positions x CW value columns of a (batch, head).  Its eight waves take the blocks of 32 keys in turn, fetch their
-//     K rows straight into operand registers (a whole block at once: one trip to memory), multiply them with the Q rows in LDS
-//     and write the gated block to LDS as 16-bit values; then V goes through two LDS slabs of 64 keys, all of it requested at
-//     the start.  An initial state (INIT) goes through the same slabs first, 64 of its rows at a time, with the Q rows in the
-//     place of P.
+//   * H: 64 positions x CW value columns of a (batch, head).  Its eight waves take tiles of 16 keys in turn, two at a time, fetch
+//     their K rows straight into operand registers (whole rows: one trip to memory), multiply them with the Q rows in LDS and
+//     write the gated tiles to LDS as 16-bit values; then V goes through LDS in batches of 256 keys, all of it requested at the
+//     start.  An initial state (INIT) goes through LDS before it, 64 of its rows at a time, with the Q rows in the place of P.
+//     Everything is requested as early as its registers allow and in the order of its use, Q by all waves before any K (the
+//     requests of a CU are served in order), and unconditionally (NSL slabs of 64 positions, past the end the last row again: a
+//     request under a branch makes the compiler wait for all of them at the first use of any).  K in operands of 16 x 32: four
+//     lanes a row, 64 bytes of it in one request; of 32 x 16 two lanes and 32 bytes, at half the rate.
 //   * C: a tile of RT x WT of the state.  All rows are requested at the start as well; V is scaled in fp32 and split into a 16-bit
 //     head and a 16-bit remainder, two products per block, as in the scan.
 // What bounds it: latency, four trips to memory or LDS in a row and the matrix work of one workgroup.  The streaming kernels
@@ -24,29 +27,29 @@
 namespace mlstm {
 namespace {
 constexpr int kShortThreads = 512;
-constexpr int kShortSlabs = kShortMax / 64;  // slabs of 64 positions at most
 
 template <int DQ, int CW, bool INIT>
 struct ShortLds {
-  // H: [Q rows, then (INIT: behind them) two slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs]
+  // H: [Q rows, then (INIT: behind them) slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs]
   static constexpr int QS = DQ + 8, VS = CW + 32;
-  static constexpr int kFront = INIT ? 64 * QS + 2 * 64 * VS : (64 * QS > 2 * 64 * VS ? 64 * QS : 2 * 64 * VS);
+  static constexpr int NBT = INIT ? 2 : 4;  // slabs of V at a time
+  static constexpr int kFront = INIT ? 64 * QS + NBT * 64 * VS : (64 * QS > NBT * 64 * VS ? 64 * QS : NBT * 64 * VS);
   static constexpr int RT = DQ % 128 == 0 ? 128 : 64, WT = CW;  // state tile
   static constexpr int XS = RT + 32, YS = WT + 32;
   static size_t bytes(int nt, bool with_c) {
-    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 17 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 64) * 4 : 0);
+    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 9 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 64) * 4 : 0);
     // C: [K slab | head of V | remainder of V | abar | abar as an operand]
     const size_t c = (size_t)64 * (XS + 2 * YS) * 2 + kShortMax * 4 + kShortMax * 3 * 2;
     return with_c && c > h ? c : h;
   }
 };
 
-template <int DQ, int CW, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT>
 __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned char* smem) {
   using L = ShortLds<DQ, CW, INIT>;
   constexpr int QS = L::QS, VS = L::VS;
-  constexpr int NF = DQ / 16 < 16 ? DQ / 16 : 16;  // fragments of a K block that are fetched at once
-  constexpr int NGK = DQ / 16 / NF;                // ... so many times
+  constexpr int NF = DQ / 32 < 8 ? DQ / 32 : 8;  // operands of a tile of K that are fetched at once
+  constexpr int NGK = DQ / 32 / NF;              // ... so many times
   constexpr int QV = DQ / 64, VV = CW / 64;        // 16-byte pieces per thread: Q rows, a slab of V
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
@@ -58,18 +61,18 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   uint16_t* const Vs = INIT ? Qs + 64 * QS : Qs;  // (without a state Q is done with before V comes)
   uint16_t* const Ps = Qs + L::kFront;
   float* const wv = (float*)(Ps + 64 * PSS);
-  float* const rows = wv + kShortMax;  // [16 key blocks][64]
-  float* const inv = rows + 17 * 64;
+  float* const rows = wv + kShortMax;  // [8 waves][64], INIT: q . n0 [64]
+  float* const inv = rows + 9 * 64;
   float* const nv = inv + 64;    // INIT: n0
   float* const csv = nv + DQ;    // INIT: cs_t
   const size_t Sp = (size_t)NC * kChunk, gofs = (size_t)bh * Sp;
   const uint16_t* const Qg = a.Q + (size_t)bh * S * DQ;
   const uint16_t* const Kg = a.K + (size_t)bh * S * DQ;
   const uint16_t* const Vg = a.V + (size_t)bh * S * DHHV + g * CW;
-  const int n_kb = min(2 * tq + 2, (S + 31) / 32);  // blocks of 32 keys
+  const int n_kt = min(4 * tq + 4, (S + 15) / 16);  // tiles of 16 keys
   const int n_sl = tq + 1;                          // slabs of 64 keys
 
-  // ---- everything this workgroup needs is requested here, in the order of its use
+  // ---- everything this workgroup needs is requested here
   u32x4 qr[QV];
 #pragma unroll
   for (int x = 0; x < QV; ++x) {
@@ -77,38 +80,36 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     qr[x] = *(const u32x4*)(Qg + (size_t)min(t0 + row, S - 1) * DQ + u * 8);
   }
   // (the gate vectors cover whole chunks: positions past the end have w = infinity, a factor of zero)
-  const float w_own = tid < 64 * n_sl ? a.g.w[gofs + tid] : 0.f;
-  float un[2];
+  const float w_own = a.g.w[gofs + min(tid, (int)Sp - 1)];
+  const int l16 = lane & 15, lq = lane >> 4;
+  float un[4];
 #pragma unroll
-  for (int tb = 0; tb < 2; ++tb) un[tb] = a.g.u[gofs + t0 + 32 * tb + r];
-  const float mc = tid < 64 ? a.g.mcomb[gofs + t0 + tid] : 0.f;
-  Frag k0[NF], k1[NF];
-  // unit x of a wave: key block wave + 8 (x / NGK), fragments NF (x % NGK) ..
-  const int n_units = NGK * ((wave < n_kb ? 1 : 0) + (wave + 8 < n_kb ? 1 : 0));
-  auto fetch = [&](Frag (&f)[NF], int x) __attribute__((always_inline)) {
-    const int j = min(32 * (wave + 8 * (x / NGK)) + r, S - 1);
-    const uint16_t* const p = Kg + (size_t)j * DQ + (x % NGK) * (NF * 16) + 8 * h;
+  for (int tc = 0; tc < 4; ++tc) un[tc] = a.g.u[gofs + t0 + 16 * tc + l16];
+  const float mc = a.g.mcomb[gofs + t0 + (tid & 63)];
+  float gr[kShortMax / kChunk];
 #pragma unroll
-    for (int ks = 0; ks < NF; ++ks) f[ks].u = *(const uint4*)(p + 16 * ks);
-  };
-  if (n_units > 0) fetch(k0, 0);
-  u32x4 vr[kShortSlabs][VV];
+  for (int y = 0; y < kShortMax / kChunk; ++y) gr[y] = a.g.graw[(size_t)bh * NC + min(y, NC - 1)];
+  __syncthreads();
+  // unit x of a wave: tiles wave + 16 y and wave + 16 y + 8 (y = x / NGK), operands NF (x % NGK) .. of their rows
+  Frag k0[2][NF], k1[2][NF];
+  const int n_units = NGK * ((wave < n_kt ? 1 : 0) + (wave + 16 < n_kt ? 1 : 0));
+  auto fetch = [&](Frag (&f)[2][NF], int x) __attribute__((always_inline)) {
 #pragma unroll
-  for (int s = 0; s < kShortSlabs; ++s)
-    if (s < n_sl) {
+    for (int e = 0; e < 2; ++e) {
+      const int kt = wave + 16 * (x / NGK) + 8 * e;
+      const uint16_t* const p = Kg + (size_t)min(16 * kt + l16, S - 1) * DQ + (x % NGK) * (NF * 32) + 8 * lq;
 #pragma unroll
-      for (int x = 0; x < VV; ++x) {
-        const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
-        vr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
-      }
+      for (int ks = 0; ks < NF; ++ks) f[e][ks].u = *(const uint4*)(p + 32 * ks);
     }
+  };
+  fetch(k0, 0);
 
 #pragma unroll
   for (int x = 0; x < QV; ++x) {
     const int idx = tid + x * kShortThreads, row = idx / (DQ / 8), u = idx % (DQ / 8);
     *(u32x4*)(Qs + row * QS + u * 8) = qr[x];
   }
-  if (tid < 64 * n_sl) wv[tid] = w_own;
+  wv[tid] = w_own;
   if constexpr (INIT) {
     if (tid < DQ) nv[tid] = a.use_nrow ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
     if (tid < 64) {
@@ -119,6 +120,14 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     }
   }
   __syncthreads();
+  u32x4 vr[NSL][VV];
+#pragma unroll
+  for (int s = 0; s < NSL; ++s)
+#pragma unroll
+    for (int x = 0; x < VV; ++x) {
+      const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
+      vr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
+    }
 
   if constexpr (INIT) {
     // q_t . n0, eight threads per position
@@ -133,50 +142,54 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     dot += __shfl_xor(dot, 1);
     dot += __shfl_xor(dot, 2);
     dot += __shfl_xor(dot, 4);
-    if (part == 0) rows[16 * 64 + t] = csv[t] * dot;
+    if (part == 0) rows[8 * 64 + t] = csv[t] * dot;
   }
-  // ---- scores of this wave's key blocks, gated into P
+  // ---- scores of this wave's tiles, gated into P
   {
-    const float lq = __log2f(a.qk_scale);
-    f32x16 sacc[2];
-    auto unit = [&](const Frag (&f)[NF], int x) __attribute__((always_inline)) {
-      const int kb = wave + 8 * (x / NGK), gk = x % NGK;
+    const float lsc = __log2f(a.qk_scale);
+    float rsum[4] = {0.f, 0.f, 0.f, 0.f};
+    f32x4 sacc[2][4];
+    auto unit = [&](const Frag (&f)[2][NF], int x) __attribute__((always_inline)) {
+      const int gk = x % NGK;
       if (gk == 0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[0][i] = sacc[1][i] = 0.f;
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int tc = 0; tc < 4; ++tc) sacc[e][tc] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
       for (int ks = 0; ks < NF; ++ks)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
+        for (int tc = 0; tc < 4; ++tc) {
           Frag B;
-          B.u = *(const uint4*)(Qs + (32 * tb + r) * QS + (gk * NF + ks) * 16 + 8 * h);
-          mfma32<F16>(sacc[tb], f[ks], B);  // rows: keys, columns: positions
+          B.u = *(const uint4*)(Qs + (16 * tc + l16) * QS + (gk * NF + ks) * 32 + 8 * lq);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) mfma16<F16>(sacc[e][tc], f[e][ks], B);  // rows: keys, columns: positions
         }
       if (gk == NGK - 1) {
-        float G = 0.f;  // decay of the chunks between the keys' and the positions'
-        for (int y = kb / 4; y < c; ++y) G += a.g.graw[(size_t)bh * NC + y];
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
-          const int diag = 2 * tq + tb;  // key block of the positions themselves
-          if (kb <= diag) {
-            float rsum = 0.f;
+        for (int e = 0; e < 2; ++e) {
+          const int kt = wave + 16 * (x / NGK) + 8 * e;
+          if (kt < n_kt) {
+            float G = 0.f;  // decay of the chunks between the keys' and the positions'
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-              const int j0 = 8 * g4 + 4 * h;
-              const float4 wj = *(const float4*)(wv + 32 * kb + j0);
-              const float w4[4] = {wj.x, wj.y, wj.z, wj.w};
-              float p[4];
+            for (int y = 0; y < kShortMax / kChunk; ++y) G += y >= kt / 8 && y < c ? gr[y] : 0.f;
+            const float4 wj = *(const float4*)(wv + 16 * kt + 4 * lq);
+            const float w4[4] = {wj.x, wj.y, wj.z, wj.w};
 #pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                const float e2 = __builtin_amdgcn_exp2f(__builtin_fmaf(un[tb] + G - w4[q], 1.4426950408889634f, lq));
-                p[q] = kb < diag || j0 + q <= r ? sacc[tb][4 * g4 + q] * e2 : 0.f;
-                rsum += p[q];
+            for (int tc = 0; tc < 4; ++tc) {
+              const int diag = 4 * tq + tc;  // tile of the positions themselves
+              if (kt <= (diag | 1)) {        // (P is read in blocks of 32 positions)
+                float p[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  const float e2 = __builtin_amdgcn_exp2f(__builtin_fmaf(un[tc] + G - w4[q], 1.4426950408889634f, lsc));
+                  p[q] = kt < diag || (kt == diag && 4 * lq + q <= l16) ? sacc[e][tc][q] * e2 : 0.f;
+                  rsum[tc] += p[q];
+                }
+                *(uint2*)(Ps + (16 * tc + l16) * PSS + 16 * kt + 4 * lq) = make_uint2(pack2<F16>(p[0], p[1]), pack2<F16>(p[2], p[3]));
               }
-              *(uint2*)(Ps + (32 * tb + r) * PSS + 32 * kb + j0) = make_uint2(pack2<F16>(p[0], p[1]), pack2<F16>(p[2], p[3]));
             }
-            const float tot = rsum + __shfl_xor(rsum, 32);
-            if (h == 0) rows[kb * 64 + 32 * tb + r] = tot;
           }
         }
       }
@@ -189,15 +202,22 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
         unit(k1, x + 1);
       }
     }
+#pragma unroll
+    for (int tc = 0; tc < 4; ++tc) {
+      float tot = rsum[tc] + __shfl_xor(rsum[tc], 16);
+      tot += __shfl_xor(tot, 32);
+      if (lq == 0) rows[wave * 64 + 16 * tc + l16] = tot;
+    }
   }
   __syncthreads();
 
-  // ---- denominators; Out^T += V^T P over the keys, 64 at a time
+  // ---- denominators; Out^T += V^T P over the keys
   if (tid < 64) {
     float iv = 1.f, nmax = 1.f;
     if (a.use_nrow) {
-      float den = INIT ? rows[16 * 64 + tid] : 0.f;
-      for (int kb = 0; kb <= 2 * tq + tid / 32 && kb < n_kb; ++kb) den += rows[kb * 64 + tid];
+      float den = INIT ? rows[8 * 64 + tid] : 0.f;
+#pragma unroll
+      for (int y = 0; y < 8; ++y) den += rows[y * 64 + tid];
       nmax = fmaxf(fabsf(den), a.sig_gate ? 1.f : __expf(-mc));
       iv = 1.f / (nmax + a.eps);
     }
@@ -213,13 +233,12 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  constexpr int kOdd = INIT ? (DQ / 64) & 1 : 0;  // the first slab of V does not go where the last one of C0 is read
   auto store_slab = [&](int s, const u32x4 (&v)[VV]) __attribute__((always_inline)) {
 #pragma unroll
     for (int x = 0; x < VV; ++x) {
       const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
       const u32x4 none = {0u, 0u, 0u, 0u};
-      *(u32x4*)(Vs + ((s + kOdd) & 1) * (64 * VS) + row * VS + u * 8) = 64 * s + row < S ? v[x] : none;
+      *(u32x4*)(Vs + (s % L::NBT) * (64 * VS) + row * VS + u * 8) = 64 * s + row < S ? v[x] : none;
     }
   };
   const int q16 = (lane >> 4) & 1, i16 = lane & 15;
@@ -263,25 +282,26 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     }
     if (tb < 2) acc *= csv[32 * tb + r];
   }
-  store_slab(0, vr[0]);
 #pragma unroll
-  for (int s = 0; s < kShortSlabs; ++s)
-    if (s < n_sl) {
+  for (int s0 = 0; s0 < NSL; s0 += L::NBT)
+    if (s0 < n_sl) {
+      if (INIT || s0 > 0) __syncthreads();  // (what lies there has been read)
+#pragma unroll
+      for (int s = s0; s < s0 + L::NBT && s < NSL; ++s)
+        if (s < n_sl) store_slab(s, vr[s]);
       __syncthreads();
-      if (s + 1 < kShortSlabs && s + 1 < n_sl) store_slab(s + 1, vr[s + 1 < kShortSlabs ? s + 1 : s]);
-      // key blocks above the diagonal are left out: zero times a NaN or infinity in V would be NaN
-      const uint16_t* const slab = Vs + ((s + kOdd) & 1) * (64 * VS);
       if (tb < 2) {
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-          if (2 * s + kk / 2 <= 2 * tq + tb) {
-            Frag A, B;
-            const uint16_t* const p = slab + (16 * kk + krow) * VS + 32 * cb + ncol;
-            A.d[0] = lds_read_tr16(p);
-            A.d[1] = lds_read_tr16(p + 4 * VS);
-            B.u = *(const uint4*)(Ps + (32 * tb + r) * PSS + 64 * s + 16 * kk + 8 * h);
-            mfma32<F16>(acc, A, B);  // rows: value columns, columns: positions
-          }
+        // key blocks above the diagonal are left out: zero times a NaN or infinity in V would be NaN
+        const int kk_end = min(4 * (s0 + L::NBT), 4 * tq + 2 * tb + 2);
+#pragma unroll 4
+        for (int kk = 4 * s0; kk < kk_end; ++kk) {
+          Frag A, B;
+          const uint16_t* const p = Vs + (16 * (kk - 4 * s0) + krow) * VS + 32 * cb + ncol;
+          A.d[0] = lds_read_tr16(p);
+          A.d[1] = lds_read_tr16(p + 4 * VS);
+          B.u = *(const uint4*)(Ps + (32 * tb + r) * PSS + 16 * kk + 8 * h);
+          mfma32<F16>(acc, A, B);  // rows: value columns, columns: positions
+        }
       }
     }
   __syncthreads();
@@ -304,7 +324,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   }
 }
 
-template <int DQ, int CW, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT>
 __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned char* smem) {
   using L = ShortLds<DQ, CW, INIT>;
   constexpr int RT = L::RT, WT = L::WT, XS = L::XS, YS = L::YS;
@@ -328,7 +348,8 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
   const int n_sl = (S + 63) / 64;
   {
     // (the decay of later chunks is left to the sums: the largest weight of a chunk is one, and one times v has no remainder)
-    const float w = tid < S ? a.g.abar[(size_t)bh * Sp + tid] : 0.f;
+    const float ab = a.g.abar[(size_t)bh * Sp + min(tid, (int)Sp - 1)];
+    const float w = tid < S ? ab : 0.f;
     wt[tid] = w;
     // n as in the scan: the weights, split exactly into three 16-bit parts, are three columns of one more operand
     uint16_t* const dst = nB + (tid >> 3) * 24 + (tid & 7);
@@ -342,21 +363,20 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
   float gb[kShortMax / kChunk];
 #pragma unroll
   for (int y = 0; y < kShortMax / kChunk; ++y) gb[y] = a.g.gbar[(size_t)bh * NC + min(y, NC - 1)];
-  u32x4 xr[kShortSlabs][XV], yr[kShortSlabs][YV];
+  u32x4 xr[NSL][XV], yr[NSL][YV];
 #pragma unroll
-  for (int s = 0; s < kShortSlabs; ++s)
-    if (s < n_sl) {
+  for (int s = 0; s < NSL; ++s) {
 #pragma unroll
-      for (int x = 0; x < XV; ++x) {
-        const int idx = tid + x * kShortThreads, row = idx / (RT / 8), u = idx % (RT / 8);
-        xr[s][x] = *(const u32x4*)(Kg + (size_t)min(64 * s + row, S - 1) * DQ + u * 8);
-      }
-#pragma unroll
-      for (int x = 0; x < YV; ++x) {
-        const int idx = tid + x * kShortThreads, row = idx / (WT / 8), u = idx % (WT / 8);
-        yr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
-      }
+    for (int x = 0; x < XV; ++x) {
+      const int idx = tid + x * kShortThreads, row = idx / (RT / 8), u = idx % (RT / 8);
+      xr[s][x] = *(const u32x4*)(Kg + (size_t)min(64 * s + row, S - 1) * DQ + u * 8);
     }
+#pragma unroll
+    for (int x = 0; x < YV; ++x) {
+      const int idx = tid + x * kShortThreads, row = idx / (WT / 8), u = idx % (WT / 8);
+      yr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
+    }
+  }
   const int rb = wave % NRB, cb0 = wave / NRB * NBW;
   const bool busy = cb0 < NCB;
   f32x16 acc[NBW], rest[NBW];  // sums of the heads and of the remainders: a remainder does not cost the large sum a rounding
@@ -386,7 +406,7 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
   const int q16 = (lane >> 4) & 1, i16 = lane & 15;
   const int krow = 8 * h + (i16 >> 2), ncol = 16 * q16 + 4 * (i16 & 3);
 #pragma unroll
-  for (int s = 0; s < kShortSlabs; ++s)
+  for (int s = 0; s < NSL; ++s)
     if (s < n_sl) {
       __syncthreads();
 #pragma unroll
@@ -467,7 +487,7 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
 
 }  // namespace
 
-template <int DQ, int CW, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT>
 __global__ __launch_bounds__(kShortThreads) void short_fw_kernel(ShortFwArgs a, int n_h, int n_c) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   // consecutive items (of one head) share an XCD and the head's rows in its L2
@@ -476,12 +496,12 @@ __global__ __launch_bounds__(kShortThreads) void short_fw_kernel(ShortFwArgs a, 
   if (!is_h) b -= n_h;
   const int n = is_h ? n_h : n_c;
   if (n_h % 8 == 0 && n % 8 == 0) b = (b % 8) * (n / 8) + b / 8;
-  if (is_h) short_h<DQ, CW, F16, INIT>(a, b, smem_raw);
-  else short_c<DQ, CW, F16, INIT>(a, b, smem_raw);
+  if (is_h) short_h<DQ, CW, NSL, F16, INIT>(a, b, smem_raw);
+  else short_c<DQ, CW, NSL, F16, INIT>(a, b, smem_raw);
 }
 
 namespace {
-template <int DQ, int CW, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT>
 const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
   using L = ShortLds<DQ, CW, INIT>;
   const int nt = (a.S + 63) / 64;
@@ -491,30 +511,36 @@ const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
   const size_t smem = L::bytes(nt, n_c > 0);
   if (smem > 160 * 1024) return "short_fw: too long for one CU's LDS";
   static LdsLimit lds;
-  if (!lds.allow((const void*)short_fw_kernel<DQ, CW, F16, INIT>, smem)) return "short_fw: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((short_fw_kernel<DQ, CW, F16, INIT>), dim3((unsigned)(n_h + n_c)), dim3(kShortThreads), smem, stream, a, (int)n_h, (int)n_c);
+  if (!lds.allow((const void*)short_fw_kernel<DQ, CW, NSL, F16, INIT>, smem)) return "short_fw: cannot raise the dynamic LDS limit";
+  hipLaunchKernelGGL((short_fw_kernel<DQ, CW, NSL, F16, INIT>), dim3((unsigned)(n_h + n_c)), dim3(kShortThreads), smem, stream, a, (int)n_h, (int)n_c);
   return nullptr;
 }
-template <int DQ, int CW>
+template <int DQ, int CW, int NSL>
 const char* launch_short_c(const ShortFwArgs& a, int BH, hipStream_t stream) {
   if (a.init != nullptr)
-    return a.f16 ? launch_short_t<DQ, CW, true, true>(a, BH, stream) : launch_short_t<DQ, CW, false, true>(a, BH, stream);
-  return a.f16 ? launch_short_t<DQ, CW, true, false>(a, BH, stream) : launch_short_t<DQ, CW, false, false>(a, BH, stream);
+    return a.f16 ? launch_short_t<DQ, CW, NSL, true, true>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, true>(a, BH, stream);
+  return a.f16 ? launch_short_t<DQ, CW, NSL, true, false>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, false>(a, BH, stream);
+}
+template <int DQ, int CW>
+const char* launch_short_s(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  // (registers and requests for as many slabs as there are, in three steps)
+  if (a.S <= 128) return launch_short_c<DQ, CW, 2>(a, BH, stream);
+  return a.S <= 320 ? launch_short_c<DQ, CW, 5>(a, BH, stream) : launch_short_c<DQ, CW, 8>(a, BH, stream);
 }
 template <int DQ>
 const char* launch_short_d(const ShortFwArgs& a, int BH, hipStream_t stream) {
-  return a.DHHV % 128 == 0 ? launch_short_c<DQ, 128>(a, BH, stream) : launch_short_c<DQ, 64>(a, BH, stream);
+  return a.DHHV % 128 == 0 ? launch_short_s<DQ, 128>(a, BH, stream) : launch_short_s<DQ, 64>(a, BH, stream);
 }
 }  // namespace
 
-// Where this kernel is the faster one: a workgroup of H takes 5 to 13 us by its number of keys and a CU one at a time, so with
+// Where this kernel is the faster one: a workgroup of H takes 5 to 12 us by its number of keys and a CU one at a time, so with
 // many heads the streaming kernels, which keep the memory system busy, overtake it -- the sooner the longer the sequence.  The
 // line (positions in 64s times workgroups of H, per CU) from gates + scan + H against gates + this, us, at 256/512, 8 heads a
-// sequence: 200 positions B=4 48.1 / 36.6, B=8 63.5 / 60.0, B=16 95 / 103; 317: B=1 42.9 / 22.9, B=4 50.8 / 46.4, B=8 73 / 77;
-// 512: B=1 42.8 / 29.1, B=2 45.1 / 47.5, B=4 52 / 74.  At 128/256, 16 heads: 200 B=8 52.9 / 48.1, B=16 71.5 / 81.4; 512 B=2
-// 40.6 / 39.5, B=4 49 / 63; 64/64, 8 heads: 512 B=8 36.7 / 31.5, B=16 39.4 / 50.7; 512/1024, 4 heads: 512 B=2 70 / 57, B=4
-// 86 / 102.  An initial state counts as two more slabs: 256/512, 200 positions B=4 49.9 / 43.6, B=8 66.0 / 72.7, 512 positions
-// B=1 44.5 / 34.9, B=2 47.4 / 55.1.  Up to 128 positions it wins at every size (256/512, B=64: 264 / 206, with 64 positions 236 / 120).
+// sequence: 200 positions B=4 48 / 37, B=8 64 / 60, B=16 95 / 106; 317: B=1 42.9 / 21.5, B=4 51 / 46, B=8 73 / 79; 512: B=1 42.8 /
+// 33.1, B=2 45 / 48, B=4 52 / 74.  At 128/256, 16 heads: 200 B=8 53 / 46, B=16 72 / 79; 512 B=2 40.6 / 39.4, B=4 49 / 60; 64/64, 8
+// heads: 512 B=8 37 / 30, B=16 39 / 45; 512/1024, 4 heads: 512 B=2 70 / 64, B=4 86 / 114.  An initial state counts as two more
+// slabs: 256/512, 200 positions B=4 50 / 44, B=8 66 / 77, 512 positions B=1 44 / 37, B=2 47 / 55.  Up to 128 positions it wins at
+// every size (256/512, B=64: 264 / 206, with 64 positions 236 / 120).
 bool short_fw_preferred(const ShortFwArgs& a, int BH) {
   if (a.S > kShortMax || a.DHHV % 64 != 0) return false;
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256 && a.DHQK != 512) return false;
