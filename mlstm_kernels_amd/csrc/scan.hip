@@ -999,12 +999,13 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
         for (int x = 0; x < (int)(sizeof(ScanJob) / sizeof(int)); ++x) w[x] = __builtin_amdgcn_readfirstlane(((const int*)(jobs + rd))[x]);
       }
       if (job.it_lo == job.it_hi && job.end == 0) continue;
-      // the normaliser vector rides with two waves of every 64 state rows in the first column tile: value-column blocks
-      // 0 and 1 carry it for the first and the second 32 rows
+      // the normaliser vector rides with two waves of every 64 state rows in the first column tile: one for the first and one for
+      // the second 32 rows, a SIMD each (with both row groups on the same two SIMDs 128 chunks of the forward took 1.5 % longer)
       const bool with_n = (a.nstates != nullptr) && job.by == 0;
-      if (with_n && wave % WC == 0)
+      const int nd = wave % WC - (NWC == 8 ? 2 * (wave / WC) : 0);
+      if (with_n && nd == 0)
         scan_consumer<RT, WT, F16, REP, SEG, 0>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);
-      else if (with_n && wave % WC == 1)
+      else if (with_n && nd == 1)
         scan_consumer<RT, WT, F16, REP, SEG, 1>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);
       else
         scan_consumer<RT, WT, F16, REP, SEG, -1>(a, bufs, gl, nB, wave, opaque(lane), job, run, chunk);

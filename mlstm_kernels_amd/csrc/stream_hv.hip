@@ -46,20 +46,20 @@ struct HvItem {
 
 // Work item of workgroup `vid` in round `round`.  Consecutive workgroups take consecutive items (neighbouring chunks
 // share rows and kept states through the L2 of their XCD); the assignment rotates by one item per round so that a
-// workgroup does not always get the chunks with the same number of source chunks.  The nz chunks of a head whose state is
-// known to be zero (forward the first ones, dV the last ones) have less to do and are dealt out last.
+// workgroup does not always get the chunks with the same number of source chunks.  The nz chunks of a head whose state is known to
+// be zero (forward the first ones, dV the last ones) stay where they are: dealt out last, so that the rounds end together, they
+// cost more than they save (64 heads of 1000 positions, H 57 -> 60 us, dV 55 -> 60; 128 heads of 1024 109 -> 112, 107 -> 109).
 template <bool IS_DV>
 __device__ __forceinline__ bool hv_decode(HvItem& it, int round, int vid, int G, int n_items, int NC, int NCH, int stride, int nz) {
   const int rot = (vid + round) % G;
   const long long idx = (long long)round * G + rot;
   if (idx >= n_items) return false;
-  const int i = (int)idx, full = NC - nz, n_full = n_items / NC * full;
-  it.no_state = i >= n_full;
-  const int per = it.no_state ? nz : full, j = it.no_state ? i - n_full : i;
-  it.ch = j % NCH;
-  const int rest = j / NCH;
-  it.c = rest % per + (it.no_state ? (IS_DV ? full : 0) : (IS_DV ? 0 : nz));
-  it.bh = rest / per;
+  const int i = (int)idx;
+  it.ch = i % NCH;
+  const int rest = i / NCH;
+  it.c = rest % NC;
+  it.bh = rest / NC;
+  it.no_state = IS_DV ? it.c >= NC - nz : it.c < nz;
   it.slot = it.c / stride;
   if (IS_DV) {
     const int hi = min(it.slot * stride + stride - 1, NC - 1);
@@ -214,15 +214,18 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const uint32_t permo = (pc >> 1) * 32 + 8 * (pc & 1);
       const uint32_t klim = (uint32_t)(S - 1) * (DHQK * 2) + pc * 16;  // this thread's piece of the last row
       {
-        // ---- resident rows, 32 per step (half-size slabs: four steps for the consumers' epilogue of the previous
-        // item, and a step count per item that is a multiple of three)
+        // ---- resident rows in four steps (for the consumers' epilogue of the previous item, and a step count per item that is
+        // a multiple of three): 32, 32, none and 64 rows.  The last one is a whole slab so that as many requests lie behind its
+        // register set as behind any other when the source chunks are reached without the state's steps: the compiler waits
+        // for the fewest there can be, and four fewer cost every item 2 to 5 %.  (The step without rows stores what its
+        // registers held where the rows of the last one go.)
         const char* const base = Xn_b + (size_t)it.bh * S * DHQK * 2;
         const uint32_t g0 = ((uint32_t)(it.c * kChunk) + row) * (DHQK * 2) + pc * 16;
         const uint32_t d0 = row * (QS * 2) + permo;
         HV_PROC(0, 4, base, g0, 8 * DHQK * 2, klim, d0, gown)
         HV_PROC(1, 4, base, g0 + 32 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 32 * QS * 2, gown)
-        HV_PROC(2, 4, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 64 * QS * 2, gown)
-        HV_PROC(0, 4, base, g0 + 96 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 96 * QS * 2, gown)
+        HV_PROC(2, 0, base, g0, 0, klim, (d0 + 64 * QS * 2) | 1u << 23, gown)
+        HV_PROC(0, 8, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 64 * QS * 2, gown)
       }
       {
         // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks.  Without a

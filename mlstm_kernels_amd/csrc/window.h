@@ -10,32 +10,14 @@ struct WinItem {
   int bh, win;  // (batch * head), window
 };
 
-// Which windows of a head have less to do, because a state they would use is known to be zero: those in front of `lo` and
-// those from `hi` on.  They are dealt out last, so that the rounds of the workgroups end together.
-struct WinLight {
-  int lo, hi, n_heavy;  // n_heavy: windows of all heads with everything to do
-  __device__ __forceinline__ WinLight(bool first, bool last, int NWIN, int n_items) {
-    lo = first ? 1 : 0;
-    hi = last ? NWIN - 1 : NWIN;
-    n_heavy = hi > lo ? n_items / NWIN * (hi - lo) : 0;
-  }
-};
-
 // Work item of workgroup `vid` in round `round`: consecutive workgroups take consecutive windows (neighbours share rows
 // through the L2 of their XCD); the assignment rotates by one per round.
-__device__ __forceinline__ bool win_decode(WinItem& it, int round, int vid, int G, int n_items, int NWIN, const WinLight& light) {
+__device__ __forceinline__ bool win_decode(WinItem& it, int round, int vid, int G, int n_items, int NWIN) {
   const int rot = (vid + round) % G;
   const long long idx = (long long)round * G + rot;
   if (idx >= n_items) return false;
-  const int i = (int)idx, heavy = light.hi - light.lo;
-  if (i < light.n_heavy) {
-    it.win = light.lo + i % heavy;
-    it.bh = i / heavy;
-  } else {
-    const int per = light.n_heavy > 0 ? NWIN - heavy : NWIN, j = (i - light.n_heavy) % per;
-    it.win = light.n_heavy == 0 || j < light.lo ? j : light.hi + j - light.lo;
-    it.bh = (i - light.n_heavy) / per;
-  }
+  it.win = (int)idx % NWIN;
+  it.bh = (int)idx / NWIN;
   return true;
 }
 

@@ -75,9 +75,9 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   const int NWIN = (NC + 1) / 2;  // the last window may hold one chunk only
   const size_t Sp = (size_t)NC * kChunk;
   // without a state in front of the first window (behind the last one) phase O has nothing to add there and falls away; its
-  // q . n moves to the rows of phase S
+  // q . n moves to the rows of phase S.  (Such windows are not dealt out last: 128 heads of 2048, 128/256, H 116 -> 119 us, dV
+  // 92 -> 99.)
   const int zero_win = a.zero_state ? (IS_DV ? NWIN - 1 : 0) : -1;
-  const WinLight light(zero_win == 0 && !IS_DV, zero_win >= 0 && IS_DV, NWIN, n_items);
 
   if (wave_all >= 8) {
     // =========================================================================================== producer waves
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   }
     WinItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const uint32_t pl = (uint32_t)opaque(p);
       const char* const Q_b = (const char*)a.Q + (size_t)it.bh * S * DHQK * 2;
       const char* const K_b = (const char*)a.K + (size_t)it.bh * S * DHQK * 2;
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
   }
     bool first = true;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
+      if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const int n_pos = RAGGED ? S - 256 * it.win : 256;
       const float g01 = a.g.graw[(size_t)bh * NC + c0];
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       // the next window's vectors travel while this one's tile leaves (requested with that tile's successor they would
       // cost a trip to memory per window: dV 5 % slower)
       WinItem nx;
-      first = !(rd + 1 < n_rounds && win_decode(nx, rd + 1, vid, G, n_items, NWIN, light));
+      first = !(rd + 1 < n_rounds && win_decode(nx, rd + 1, vid, G, n_items, NWIN));
       if (!first) request(nx);
     }
     if (pending) {  // (a workgroup without a window passes no barrier at all, like its producers)

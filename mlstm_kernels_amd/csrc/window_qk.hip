@@ -46,6 +46,39 @@ constexpr int kWqStgOfs = kWqRedOfs + 4 * 1024;   // [8 waves][16 rows][64 eleme
 constexpr int kWqCsOfs = kWqStgOfs + 8 * 2048;    // [256] column scale of the inter-chunk part of the running phase
 constexpr int kWqSmem = kWqCsOfs + 1024;
 static_assert(kWqSmem <= 160 * 1024, "LDS budget of one CU");
+
+// The order of the windows.  Those of a head that have a phase less, because the state in front of the first or behind the last
+// one is known to be zero, come last, so that the rounds of the workgroups end together.  In the round in which they begin
+// neighbours lie on different XCDs: every XCD having a range of its own, as in the other rounds, they would all fall to the last
+// ones.  Us, as they come / last / last and dealt: 32 heads of 16384 positions, 256/512, 791 / 774 / 777, 128 of 1024 196 / - / 190,
+// 64 of 1000 95 / 102 / 94; tiles of 128 rows gain nothing (128/256, 128 of 2048, 164 / - / 166) and keep the order.
+struct QkOrder {
+  int G, n_items, NWIN, own, dealt;
+  int lo, hi, n_full;  // windows lo .. hi - 1 of a head have everything to do; how many of all heads
+  __device__ __forceinline__ QkOrder(int b, int G_, int n, int w, bool first, bool last) : G(G_), n_items(n), NWIN(w) {
+    own = G % 8 == 0 ? (b % 8) * (G / 8) + b / 8 : b;  // consecutive places share an XCD (and its L2)
+    dealt = b;
+    lo = first ? 1 : 0;
+    hi = max(last ? NWIN - 1 : NWIN, lo);
+    n_full = n_items / NWIN * (hi - lo);
+  }
+  // the item of this workgroup in round `round`; the assignment rotates by one per round
+  __device__ __forceinline__ bool item(WinItem& it, int round) const {
+    const bool mixed = n_full < n_items && round == n_full / G && n_full % G != 0;
+    const long long idx = (long long)round * G + (mixed ? dealt : (own + round) % G);
+    if (idx >= n_items) return false;
+    const int i = (int)idx, full = hi - lo;
+    if (i < n_full) {
+      it.win = lo + i % full;
+      it.bh = i / full;
+    } else {
+      const int per = NWIN - full, j = (i - n_full) % per;
+      it.win = j < lo ? j : hi + j - lo;
+      it.bh = (i - n_full) / per;
+    }
+    return true;
+  }
+};
 }  // namespace
 
 // DT = head-dim rows of a tile: 256, 128 or 64.  MULTI: the head dimension is several tiles, walked one after the other
@@ -67,8 +100,6 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int G = gridDim.x;
-  int vid = blockIdx.x;
-  if (G % 8 == 0) vid = (vid % 8) * (G / 8) + vid / 8;  // consecutive ids share an XCD (and its L2)
   const int NC = a.NC, S = a.S, DHHV = a.DHHV, DHQK = MULTI ? a.DHQK : DT;
   const int ND = DHQK / 16, NDG = DHQK / DT;
   const int NV = DHHV / 32;   // steps of 32 value columns (even)
@@ -76,7 +107,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   const size_t Sp = (size_t)NC * kChunk;
   // no initial state, no gradient after the last chunk: the steps that would multiply them fall away
   const bool zero_c = __builtin_amdgcn_readfirstlane(*a.g.zero_c) != 0, zero_dc = a.zero_dc != 0;
-  const WinLight light(zero_c, zero_dc, NWIN, n_items);
+  const QkOrder order(blockIdx.x, G, n_items, NWIN, DT == 256 && zero_c, DT == 256 && zero_dc);
 
   if (wave_all >= 8) {
     // =========================================================================================== producer waves
@@ -120,7 +151,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
   }
     WinItem it;
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
+      if (!order.item(it, rd)) continue;
       const uint32_t pl = (uint32_t)opaque(p);
       const char* const dH_b = (const char*)a.dH + (size_t)it.bh * S * DHHV * 2;
       const char* const V_b = (const char*)a.V + (size_t)it.bh * S * DHHV * 2;
@@ -248,7 +279,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     };
 
     for (int rd = 0; rd < n_rounds; ++rd) {
-      if (!win_decode(it, rd, vid, G, n_items, NWIN, light)) continue;
+      if (!order.item(it, rd)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const size_t hofs = (size_t)bh * Sp, gofs = hofs + (size_t)c0 * kChunk;
       const float* graw = a.g.graw + (size_t)bh * NC;
