@@ -122,3 +122,34 @@ def test_infinities_stay_infinities(T, dims, dtype, state):
             fin = torch.isfinite(y)
             if fin.any() and y[fin].abs().max() > 0:
                 assert rel_norm(x[fin], y[fin]) < tol[kind], (name, head)
+
+
+@pytest.mark.parametrize("dtype,state", [("bfloat16", "float32"), ("float16", "bfloat16"), ("float32", "float32")])
+@pytest.mark.parametrize("form", ["dense", "strided", "mixed", "other state type"])
+def test_one_token_through_the_backend(dtype, state, form):
+    """One token from given states (in native code where nothing has to be converted) against the step function, and the shapes
+    that the backend refuses."""
+    from mlstm_kernels_amd.torch.backend_module import mLSTMBackend, mLSTMBackendConfig
+    from mlstm_kernels_amd.torch.recurrent import mlstm_recurrent_step__hip
+
+    B, NH, DQ, DV = 2, 3, 64, 128
+    dt, sdt = getattr(torch, dtype), getattr(torch, state)
+    g = torch.Generator().manual_seed(1)
+    rn = lambda *s: torch.randn(*s, generator=g).cuda()
+    q, k, v = rn(B, NH, 1, DQ).to(dt), rn(B, NH, 1, DQ).to(dt), rn(B, NH, 1, DV).to(dt)
+    i, f = rn(B, NH, 1).to(dt), rn(B, NH, 1).to(dt)
+    st = [rn(B, NH, DQ, DV).to(sdt), rn(B, NH, DQ).to(sdt), rn(B, NH, 1).to(sdt)]
+    if form == "strided":
+        q = rn(B, NH, 1, 2 * DQ).to(dt)[..., ::2]
+    elif form == "mixed":
+        f = f.double().to(torch.float32 if dt != torch.float32 else torch.bfloat16)
+    elif form == "other state type":
+        st = [t.half() for t in st]
+    backend = mLSTMBackend(mLSTMBackendConfig(mode="inference", autocast_kernel_dtype=dtype, inference_state_dtype=state))
+    h, new = backend(q, k, v, i, f, *st)
+    h_ref, new_ref = mlstm_recurrent_step__hip(q.squeeze(2), k.squeeze(2), v.squeeze(2), i, f, *st, dtype_state=sdt)
+    assert h.shape == v.shape and torch.equal(h[:, :, 0], h_ref)
+    for a, b in zip(new, new_ref):
+        assert a.dtype == sdt and torch.equal(a, b)
+    with pytest.raises(ValueError):
+        backend(q.squeeze(2), k.squeeze(2), v.squeeze(2), i, f, *st)
