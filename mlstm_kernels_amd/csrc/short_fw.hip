@@ -291,8 +291,9 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
         if (s < n_sl) store_slab(s, vr[s]);
       __syncthreads();
       if (tb < 2) {
-        // key blocks above the diagonal are left out: zero times a NaN or infinity in V would be NaN
-        const int kk_end = min(4 * (s0 + L::NBT), 4 * tq + 2 * tb + 2);
+        // key blocks above the diagonal are left out: zero times a NaN or infinity in V would be NaN.  So are those past the last
+        // tile of keys, where P holds what LDS held before (V is zero there, but that may be a NaN)
+        const int kk_end = min(min(4 * (s0 + L::NBT), n_kt), 4 * tq + 2 * tb + 2);
 #pragma unroll 4
         for (int kk = 4 * s0; kk < kk_end; ++kk) {
           Frag A, B;

@@ -230,6 +230,26 @@ def test_short_prompts_values_not_finite(S, pos, which, bad):
         assert bool(torch.isfinite(H[0, 0, pos + 1:]).all())
 
 
+@pytest.mark.parametrize("S", [1, 33, 65, 129, 257, 321, 496, 497])
+@pytest.mark.parametrize("DQ,DV", [(64, 64), (128, 192), (256, 512), (512, 128)])
+def test_short_prompts_in_used_memory(S, DQ, DV):
+    """What the launches before left in the memory of the compute units does not matter: the same bits after launches full of NaN
+    as after launches full of zeros, also where the last tile of 16 keys is the first of its block of 32."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    x = [t.cuda() for t in make_qkvif(1, 3, S, DQ, DV, seed=S + DQ, f_offset=3.0)]
+    out = []
+    for value in (0.0, float("nan")):
+        fill = [torch.full((1, 128, 512, d), value, device="cuda", dtype=torch.bfloat16) for d in (DQ, DQ, DV)]
+        gates = [torch.zeros(1, 128, 512, device="cuda")] * 2
+        with torch.no_grad():
+            mlstm_chunkwise__hip_xl_chunk(*fill, *gates, return_last_states=True, any_sequence_length=True)
+            H, state = mlstm_chunkwise__hip_xl_chunk(*x, return_last_states=True, any_sequence_length=True)
+        out.append((H, *state))
+    for a, b in zip(*out):
+        assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
+
+
 # States that are known to be zero are neither written nor multiplied: the same bits as with zeros handed over, whatever the
 # workspace holds (it is taken from memory full of NaN), for one window, several, and a ragged last one of either length.
 @pytest.mark.parametrize("DQ,DV,path", [(256, 512, "auto"), (256, 512, "stream"), (256, 512, "split"), (64, 64, "auto"), (128, 256, "auto"),
