@@ -16,13 +16,13 @@
 //       V  max(2, CW / 64) steps [V (dH) rows x CW]                                        Out^T += Xw^T P
 //     A finished tile leaves during the first step of the next window's S (of several groups: each at its end).
 //   * A window whose state is known to be zero has no phase O (128 heads of 2048, 128/256: the call, forward and backward,
-//     487 -> 479 us with the same in window_qk.hip).
+//     487 -> 479 us with the same in window_qk.hip, before the gate vectors went to the producers).
 //   * What bounds it: HBM.  Everything a window needs passes through the CU once, only the rows of O a second time: at
 //     128/256 384 KB in and 128 KB out per window where the tiled kernel moved 285 KB per 64 positions; a score block is
 //     computed once for all value columns of its group's window.
-// Measured on MI355X, H / dV in us, tiled kernel -> this one: 128/256 with 262144 token-heads 170 / 165 -> 119 / 104
-// (3.9 / 4.5 TB/s on operands and results counted once), 128/128 180 / 163 -> 71 / 67, 64/128 113 / 102 -> 57 / 51, 64/64
-// with 524288 404 / 367 -> 88 / 77, 256/256 with 131072 119 / 108 -> 80 / 73, 512/1024 with 32768 142 / 141 -> 108 / 101.
+// Measured on MI355X, H / dV in us, tiled kernel -> this one: 128/256 with 262144 token-heads 170 / 165 -> 99 / 94
+// (4.7 / 4.9 TB/s on operands and results counted once), 128/128 180 / 163 -> 72 / 67, 64/128 113 / 102 -> 56 / 51, 64/64
+// with 524288 404 / 367 -> 84 / 74, 256/256 with 131072 119 / 108 -> 78 / 73, 512/1024 with 32768 142 / 141 -> 105 / 101.
 // At 256/512 the streaming kernel (stream_hv.hip, Q resident: no second reading) is as fast: 137 / 128 against 147 / 131.
 #include "kernels.h"
 #include "window.h"
@@ -89,7 +89,12 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     const int p = (wave_all - 8) * 64 + lane;
     u32x4 fd0[8], fd1[8];
     uint32_t fa0 = 0, fb0 = 0, fa1 = 0, fb1 = 0;
-    int L = 0;
+    int L = 0, passed = 0;  // load steps; barriers passed
+#define WH_BARRIER                                                                                                   \
+  if (L - 2 > passed) {                                                                                              \
+    __syncthreads();                                                                                                 \
+    ++passed;                                                                                                        \
+  }
 #define WH_PUT_B(E, i_, perm_)                                                                                       \
   {                                                                                                                  \
     if (perm_) {                                                                                                     \
@@ -110,7 +115,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     // lands where nobody reads); lA_, lB_: largest byte offset (rows past the end re-read the last row)
 #define WH_PROC(E, bA_, gA_, sA_, lA_, nA_, bB_, gB_, sB_, lB_, nB_, dA_, dB_)                                       \
   {                                                                                                                  \
-    if (L >= 3) __syncthreads();                                                                                     \
+    WH_BARRIER                                                                                                       \
     /* piece by piece: the old content of a register goes to LDS, then the register is requested anew */             \
     const bool perm_ = __builtin_amdgcn_readfirstlane((int)(fb##E & 1)) != 0;                                        \
     const uint32_t oA_ = fa##E, oB_ = fb##E & ~1u;                                                                   \
@@ -143,9 +148,68 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       const uint32_t xg = (t0 + xrow) * pitch + xun * 16, xstep = 64 * pitch, xlim = (uint32_t)(S - 1) * pitch + xun * 16;
       const uint32_t xd = (xrow * 4 + (xun ^ (uint32_t)win_f64((int)xrow))) * 16;
       const uint32_t xdp = ((xrow * 4 + ((xun & 2) ^ (uint32_t)win_f64((int)xrow))) * 16 + 8 * (xun & 1)) | 1u;
+      // ---- gate vectors and normaliser state of the window: requested in front of its first slab, in LDS two steps later, when
+      // the consumers are in the last step of the window before, which reads none of them any more.  These waves have the
+      // registers for it.  Held by the consumers until the window began they were spilled, and reading them back waited for
+      // the stores of the tile that leaves there (128 heads of 2048, 128/256: H 120 -> 99 us, dV 106 -> 94; 256 heads of 2048,
+      // 64/64: 92 -> 84, 81 -> 74; 64 heads of 2048, 256/256: 87 -> 78, 81 -> 74).
+      const int n_pos = RAGGED ? S - 256 * it.win : 256, c0 = 2 * it.win;
+      float pu, pw, pr, pc, pm = 0.f, pg, m0, m1, np[4][3];
+      {
+        const size_t gi = (size_t)it.bh * Sp + (size_t)c0 * kChunk + (RAGGED ? min((int)pl, n_pos - 1) : (int)pl);
+        // dV: keys of the first chunk see dC through the second, where there is one; H: positions of the second see C through the
+        // first
+        const int cx = IS_DV && (!RAGGED || c0 + 1 < NC) ? c0 + 1 : c0;
+        pg = a.g.graw[(size_t)it.bh * NC + cx];
+        m0 = a.g.mstates[(size_t)it.bh * (NC + 1) + cx];
+        m1 = a.g.mstates[(size_t)it.bh * (NC + 1) + cx + 1];
+        pu = a.g.u[gi];
+        pw = a.g.w[gi];
+        if (IS_DV) {
+          pr = (a.use_nrow ? a.nrow : a.g.u)[gi];
+          pc = a.g.abar[gi];
+        } else {
+          pc = a.g.bbar[gi];
+          pm = a.g.mcomb[gi];
+          // n before either chunk as three partial vectors (their sum carries the full fp32 precision); entries past the end repeat
+          // the last one, without a normaliser any readable word does
+          const float* const n_b = a.use_nrow ? a.nstates + ((size_t)it.bh * NC + c0) * 3 * DHQK : a.g.graw;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int e = min((int)pl + 256 * i, 2 * DHQK - 1), ch = e >= DHQK ? 1 : 0;
+            const int o = a.use_nrow ? (c0 + ch < NC ? ch * 3 * DHQK : 0) + e - ch * DHQK : 0, st = a.use_nrow ? DHQK : 0;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) np[i][x] = n_b[o + x * st];
+          }
+        }
+      }
+      const uint32_t xx0 = (uint32_t)opaque((int)xg), xl0 = (uint32_t)opaque((int)xlim);
+      WH_PROC(0, Q_b, xx0, xstep, xl0, 4, K_b, xx0, xstep, xl0, 4, xd, 16384 + xd)
+      WH_PROC(1, Q_b, xx0 + 64, xstep, xl0 + 64, 4, K_b, xx0 + 64, xstep, xl0 + 64, 4, xd, 16384 + xd)
+      WH_BARRIER
+      {
+        // past the end: no key (w = infinity), no query (factor 0)
+        const int t = (int)pl;
+        const bool in = !RAGGED || t < n_pos;
+        const float f = IS_DV && a.use_nrow ? 1.f / (pr + a.eps) : 1.f, xs = __expf(pg + m0 - m1);
+        uvec[t] = pu;
+        wvec[t] = in ? pw : __builtin_inff();
+        lqr[t] = in ? __log2f(a.qk_scale * f) : -__builtin_inff();
+        if (IS_DV) {
+          csv[t] = pc * (t < 128 && (!RAGGED || c0 + 1 < NC) ? xs : 1.f);
+        } else {
+          const float pb = pc * a.qk_scale;
+          csv[t] = pb * (t >= 128 ? xs : 1.f);
+          cs0v[t] = pb;
+          mcv[t] = pm;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (t + 256 * i < 2 * DHQK) nvec[t + 256 * i] = (np[i][0] + np[i][1]) + np[i][2];
+        }
+      }
       {
         const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim);
-        for (int w = 0; w < NS; w += 2) {
+        for (int w = 2; w < NS; w += 2) {
           WH_PROC(0, Q_b, xx + w * 64, xstep, xl + w * 64, 4, K_b, xx + w * 64, xstep, xl + w * 64, 4, xd, 16384 + xd)
           WH_PROC(1, Q_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, 4, K_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, 4,
                   xd, 16384 + xd)
@@ -182,7 +246,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
     }
     // ---- drain: the last two slabs go to LDS, then the barriers of the consumers' last steps and of the last epilogue
     if (L > 0) {
-      if (L >= 3) __syncthreads();
+      WH_BARRIER
       WH_STORE(0)
       __syncthreads();
       WH_STORE(1)
@@ -190,6 +254,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       __syncthreads();
     }
 #undef WH_PROC
+#undef WH_BARRIER
 #undef WH_STORE
 #undef WH_PUT_B
   } else {
@@ -210,63 +275,6 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       const unsigned char* s = smem_raw + slot * kWinSlot;
       slot ^= 1;
       return s;
-    };
-    // gate vectors and normaliser state of a window, requested ahead of its first step
-    float pu = 0.f, pw = 0.f, pr = 1.f, pc = 0.f, pb = 0.f, pm = 0.f, np0 = 0.f, np1 = 0.f, np2 = 0.f;
-    auto request = [&](const WinItem& x) {
-      const int c0 = 2 * x.win, n_pos = RAGGED ? S - 256 * x.win : 256;
-      const size_t gofs = (size_t)x.bh * Sp + (size_t)c0 * kChunk;
-      if (tid < 256) {
-        const size_t gi = gofs + min(tid, n_pos - 1);
-        const float* graw = a.g.graw + (size_t)x.bh * NC;
-        const float* mst = a.g.mstates + (size_t)x.bh * (NC + 1);
-        pu = a.g.u[gi];
-        pw = a.g.w[gi];
-        if (IS_DV) {
-          if (a.use_nrow) pr = a.nrow[gi];
-          // keys of c0 see dC through chunk c1, where there is one
-          const float xs = !RAGGED || c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
-          pc = a.g.abar[gi] * (tid < 128 ? xs : 1.f);
-        } else {
-          const float xs = __expf(graw[c0] + mst[c0] - mst[c0 + 1]);  // positions of c1 see C through chunk c0
-          pb = a.g.bbar[gi] * a.qk_scale;
-          pc = pb * (tid >= 128 ? xs : 1.f);
-          pm = a.g.mcomb[gi];
-        }
-      }
-      if (!IS_DV) {
-        // n before either chunk as three partial vectors (their sum carries the full fp32 precision)
-        const int ch = tid >> 8, d = tid & 255;
-        if (d < DHQK && a.use_nrow) {
-          const float* np3 = a.nstates + ((size_t)x.bh * NC + min(c0 + ch, NC - 1)) * 3 * DHQK + d;
-          np0 = np3[0];
-          np1 = np3[DHQK];
-          np2 = np3[2 * DHQK];
-        }
-      }
-    };
-    auto publish = [&](const WinItem& x) {
-      const int n_pos = RAGGED ? S - 256 * x.win : 256;
-      if (tid < 256) {
-        // past the end: no key (w = infinity), no query (factor 0)
-        uvec[tid] = pu;
-        wvec[tid] = tid < n_pos ? pw : __builtin_inff();
-        const float f = IS_DV && a.use_nrow ? 1.f / (pr + a.eps) : 1.f;
-        lqr[tid] = tid < n_pos ? __log2f(a.qk_scale * f) : -__builtin_inff();
-        csv[tid] = pc;
-        if (!IS_DV) {
-          cs0v[tid] = pb;
-          mcv[tid] = pm;
-        }
-      }
-      if (!IS_DV && a.use_nrow) {
-        const int ch = tid >> 8, d = tid & 255;
-        if (d < DHQK) nvec[ch * DHQK + d] = (np0 + np1) + np2;
-        for (int dd = d + 256; dd < DHQK; dd += 256) {
-          const float* np3 = a.nstates + ((size_t)x.bh * NC + min(2 * x.win + ch, NC - 1)) * 3 * DHQK + dd;
-          nvec[ch * DHQK + dd] = (np3[0] + np3[DHQK]) + np3[2 * DHQK];
-        }
-      }
     };
     // (normalise,) round and store the tile: 32 positions x 64 columns at a time through the wave's private staging tile
     // into row order, full 128-byte lines.  A macro: the accumulator indices stay literal.
@@ -320,15 +328,12 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
       }                                                                                                              \
     }                                                                                                                \
   }
-    bool first = true;
     for (int rd = 0; rd < n_rounds; ++rd) {
       if (!win_decode(it, rd, vid, G, n_items, NWIN)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
       const int n_pos = RAGGED ? S - 256 * it.win : 256;
       const float g01 = a.g.graw[(size_t)bh * NC + c0];
       const bool no_state = it.win == zero_win;
-
-      if (first) request(it);
 
       // ================================================================================= phase S: the score blocks
       float dot = 0.f;
@@ -353,16 +358,17 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
           }
         };
         // q_t . n before the second chunk (before the first it is zero), as phase O does it with a state: two threads per
-        // position, 16 of the slab's 32 entries each, in the order of the fragments.  n4(e): entries e .. e + 3 of the sixteen
-        auto s_dot = [&](const unsigned char* slab, auto n4) __attribute__((always_inline)) {
+        // position, 16 of the slab's 32 entries each, in the order of the fragments
+        auto s_dot = [&](const unsigned char* slab, int w) __attribute__((always_inline)) {
           const int td = opaque(tid);
           const int t = td >> 1, part = td & 1;
+          const float* const np = nvec + DHQK + 32 * w + 16 * part;
           const uint4 q0 = *(const uint4*)(slab + t * 64 + (((2 * part) ^ win_f64(t)) * 16));
           const uint4 q1 = *(const uint4*)(slab + t * 64 + (((2 * part + 1) ^ win_f64(t)) * 16));
 #pragma unroll
           for (int x = 0; x < 2; ++x) {
             const uint4 qv = x == 0 ? make_uint4(q0.x, q0.y, q1.x, q1.y) : make_uint4(q0.z, q0.w, q1.z, q1.w);
-            const float4 na = n4(4 * x), nb4 = n4(8 + 4 * x);
+            const float4 na = *(const float4*)(np + 4 * x), nb4 = *(const float4*)(np + 8 + 4 * x);
             dot += lo2<F16>(qv.x) * na.x + hi2<F16>(qv.x) * na.y + lo2<F16>(qv.y) * na.z + hi2<F16>(qv.y) * na.w;
             dot += lo2<F16>(qv.z) * nb4.x + hi2<F16>(qv.z) * nb4.y + lo2<F16>(qv.w) * nb4.z + hi2<F16>(qv.w) * nb4.w;
           }
@@ -372,26 +378,16 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         __syncthreads();
         const unsigned char* const first_slab = next_slab();
         if (!MULTI && pending) WH_EPILOGUE
-        publish(it);
 #pragma unroll
         for (int e = 0; e < 5; ++e)
 #pragma unroll
           for (int i = 0; i < 16; ++i) sacc[e][i] = 0.f;
-        if (with_dot) {  // n from memory: what was published in this step is not visible yet
-          const float* const np3 = a.nstates + ((size_t)bh * NC + min(c0 + 1, NC - 1)) * 3 * DHQK + 16 * (tid & 1);
-          s_dot(first_slab, [&](int e) {
-            const float4 x = *(const float4*)(np3 + e), y = *(const float4*)(np3 + DHQK + e), z = *(const float4*)(np3 + 2 * DHQK + e);
-            return make_float4((x.x + y.x) + z.x, (x.y + y.y) + z.y, (x.z + y.z) + z.z, (x.w + y.w) + z.w);
-          });
-        }
+        if (with_dot) s_dot(first_slab, 0);
         s_step(first_slab);
         for (int w = 1; w < NS; ++w) {
           __syncthreads();
           const unsigned char* const slab = next_slab();
-          if (with_dot) {
-            const float* const np = nvec + DHQK + 32 * w + 16 * (tid & 1);
-            s_dot(slab, [&](int e) { return *(const float4*)(np + e); });
-          }
+          if (with_dot) s_dot(slab, w);
           s_step(slab);
         }
         // ---- gating: P = scores * exp(u_t - w_j + G) / sqrt(DHQK) (* rho_t), zero above the diagonal; forward: fp32 row
@@ -599,11 +595,6 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
         prev_cg = cg;
         if constexpr (MULTI) WH_EPILOGUE
       }
-      // the next window's vectors travel while this one's tile leaves (requested with that tile's successor they would
-      // cost a trip to memory per window: dV 5 % slower)
-      WinItem nx;
-      first = !(rd + 1 < n_rounds && win_decode(nx, rd + 1, vid, G, n_items, NWIN));
-      if (!first) request(nx);
     }
     if (pending) {  // (a workgroup without a window passes no barrier at all, like its producers)
       __syncthreads();
