@@ -31,8 +31,8 @@
 //   * A window without a state on one side (no initial state, no gradient after the end) leaves out that phase's NV steps:
 //     the state and the second reading of dH (V), a quarter of a 256/512 window.
 // Supported: state stride 2, any head dimensions (multiples of 64; DHQK in tiles of 256, 128 or 64, whichever divides it).
-// Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 326 -> 170, 128/128 259 -> 119,
-// 64/128 244 -> 82, 64/64 with 524288 419 -> 119, 512/1024 with 32768 210 -> 191; 256/512 with 524288 1042 -> 780.
+// Measured on MI355X, us, tiled pair kernel -> this one: 128/256 with 262144 token-heads 326 -> 162, 128/128 259 -> 112,
+// 64/128 244 -> 77, 64/64 with 524288 419 -> 110, 512/1024 with 32768 210 -> 180; 256/512 with 524288 1042 -> 770.
 #include <type_traits>
 
 #include "kernels.h"
@@ -118,7 +118,12 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     const int p = (wave_all - 8) * 64 + lane;  // 0 .. 255: every thread moves eight 16-byte pieces of every slab
     u32x4 fd0[8], fd1[8];
     uint32_t fw0 = 0, fw1 = 0;
-    int L = 0;
+    int L = 0, passed = 0;  // load steps; barriers passed
+#define WQ_BARRIER                                                                                                   \
+  if (L - 2 > passed) {                                                                                              \
+    __syncthreads();                                                                                                 \
+    ++passed;                                                                                                        \
+  }
 #define WQ_STORE(E)                                                                                                  \
   {                                                                                                                  \
     const uint32_t w_ = fw##E;                                                                                       \
@@ -132,7 +137,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     // factors are zero and their results are not stored), dAu_ / dBu_ destination units of the two halves inside the slot
 #define WQ_PROC(E, bA_, gA_, sA_, lA_, nA_, bB_, gB_, sB_, lB_, dAu_, dBu_)                                                         \
   {                                                                                                                  \
-    if (L >= 3) __syncthreads();                                                                                     \
+    WQ_BARRIER                                                                                                       \
     /* piece by piece: the old content of a register goes to LDS, then the register is requested anew, so that the */ \
     /* LDS port and the vector-memory path of the CU work side by side instead of one after the other */             \
     const uint32_t w_ = fw##E;                                                                                       \
@@ -201,10 +206,51 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       }                                                                                                              \
     }                                                                                                                \
   }
+      // ---- gate vectors of the window: requested in front of its first slab, in LDS two steps later, when the consumers are in the
+      // last step of the window before, which reads none of them any more.  (As requests of the consumer waves each phase
+      // waited for them, and with them for the stores of the phase before.  256 heads of 2048, 64/64: 123 -> 111 us; 128 heads,
+      // 128/256: 164.6 -> 161.5; 32 heads of 16384, 256/512: 783 -> 774; with two windows per workgroup of 256/256 1 % more.)
+      const int n_pos = RAGGED ? S - 256 * it.win : 256, c0 = 2 * it.win;
+      // keys of c0 see dC through chunk c1, where there is one (the gradient kept is that after the last chunk); positions of c1 see
+      // C through chunk c0
+      const bool two = !RAGGED || c0 + 1 < NC;
+      float pu, pw, pr, pb, pa, pg0, pg1, pm0, pm1, pm2, csq, csk;
+      {
+        const size_t gi = (size_t)it.bh * Sp + (size_t)c0 * kChunk + (RAGGED ? min((int)pl, n_pos - 1) : (int)pl);
+        const float* const graw = a.g.graw + (size_t)it.bh * NC + c0;
+        const float* const mst = a.g.mstates + (size_t)it.bh * (NC + 1) + c0;
+        pg0 = graw[0];
+        pg1 = graw[two ? 1 : 0];
+        pm0 = mst[0];
+        pm1 = mst[1];
+        pm2 = mst[two ? 2 : 1];
+        pu = a.g.u[gi];
+        pw = a.g.w[gi];
+        pr = (a.use_nrow ? a.nrow : a.g.u)[gi];
+        pb = a.g.bbar[gi];
+        pa = a.g.abar[gi];
+      }
       // ---- phase S: dH rows | V rows
       {
         const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim);
-        for (int w = 0; w < NV; w += 2) {
+        WQ_PROC(0, dH_b, xx, xstep, xl, 4, V_b, xx, xstep, xl, xdu, 1024 + xdu)
+        WQ_PROC(1, dH_b, xx + 64, xstep, xl + 64, 4, V_b, xx + 64, xstep, xl + 64, xdu, 1024 + xdu)
+      }
+      WQ_BARRIER
+      {
+        // past the end: no key (w = infinity), no query (factor 0)
+        const int t = (int)pl;
+        const bool in = !RAGGED || t < n_pos;
+        const float rh = a.use_nrow ? 1.f / (pr + a.eps) : 1.f;
+        uvec[t] = pu;
+        wvec[t] = in ? pw : __builtin_inff();
+        lqr[t] = in ? __log2f(a.qk_scale * rh) : -__builtin_inff();
+        csq = pb * a.qk_scale * rh * (t >= 128 ? __expf(pg0 + pm0 - pm1) : 1.f);
+        csk = pa * (t < 128 && two ? __expf(pg1 + pm1 - pm2) : 1.f);
+      }
+      {
+        const uint32_t xx = (uint32_t)opaque((int)xg), xl = (uint32_t)opaque((int)xlim);
+        for (int w = 2; w < NV; w += 2) {
           WQ_PROC(0, dH_b, xx + w * 64, xstep, xl + w * 64, 4, V_b, xx + w * 64, xstep, xl + w * 64, xdu, 1024 + xdu)
           WQ_PROC(1, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, 4, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, xdu, 1024 + xdu)
         }
@@ -219,6 +265,10 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         for (int w = 0; w < nv; w += 2) {
           WQ_PROC(0, C_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
           WQ_PROC(1, C_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, dH_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
+          if (w == 0) {
+            WQ_BARRIER  // the consumers are done with the factors of the phase before
+            csv[pl] = csq;
+          }
         }
       }
       WQ_ROWS(K_b, Q_b)
@@ -229,6 +279,10 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
         for (int w = 0; w < nv; w += 2) {
           WQ_PROC(0, dC_b, (uint32_t)w * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + w * 64, xstep, xl + w * 64, cdu, 1024 + xdu)
           WQ_PROC(1, dC_b, (uint32_t)(w + 1) * cstep + cc, 4096, 0xffffffffu, NDI, V_b, xx + (w + 1) * 64, xstep, xl + (w + 1) * 64, cdu, 1024 + xdu)
+          if (w == 0) {
+            WQ_BARRIER  // the consumers are done with the factors of the phase before
+            csv[pl] = csk;
+          }
         }
       }
       WQ_ROWS(Q_b, K_b)
@@ -238,7 +292,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     }
     // ---- drain: the last two slabs go to LDS, then the barriers of the consumers' last steps and of the final row dots
     if (L > 0) {
-      if (L >= 3) __syncthreads();
+      WQ_BARRIER
       WQ_STORE(0)
       __syncthreads();
       WQ_STORE(1)
@@ -246,6 +300,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       __syncthreads();
     }
 #undef WQ_PROC
+#undef WQ_BARRIER
 #undef WQ_STORE
   } else {
     // =========================================================================================== consumer waves
@@ -281,22 +336,12 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
     for (int rd = 0; rd < n_rounds; ++rd) {
       if (!order.item(it, rd)) continue;
       const int bh = it.bh, c0 = 2 * it.win;
-      const size_t hofs = (size_t)bh * Sp, gofs = hofs + (size_t)c0 * kChunk;
       const float* graw = a.g.graw + (size_t)bh * NC;
-      const float* mst = a.g.mstates + (size_t)bh * (NC + 1);
       const float g01 = graw[c0];   // decay over chunk c0: what separates a position of c1 from the keys of c0
       const int n_pos = RAGGED ? S - 256 * it.win : 256;   // positions of the window inside the sequence (256 or more: all)
 
       // ================================================================================= phase S: the score blocks
       {
-        // gate vectors of the window, requested now, written to LDS after the first step
-        float pu = 0.f, pw = 0.f, pr = 1.f;
-        if (tid < 256) {
-          const int tv = min(tid, n_pos - 1);
-          pu = a.g.u[gofs + tv];
-          pw = a.g.w[gofs + tv];
-          if (a.use_nrow) pr = a.nrow[gofs + tv];
-        }
         f32x16 sacc[5];
 #pragma unroll
         for (int e = 0; e < 5; ++e)
@@ -308,14 +353,6 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           if (w == 0) {
             finish_rowdots();
             prev = it;
-          }
-          if (w == (NV > 2 ? 1 : 0)) {
-            if (tid < 256) {
-              // past the end: no key (w = infinity), no query (factor 0)
-              uvec[tid] = pu;
-              wvec[tid] = tid < n_pos ? pw : __builtin_inff();
-              lqr[tid] = tid < n_pos ? __log2f(a.qk_scale * (a.use_nrow ? 1.f / (pr + a.eps) : 1.f)) : -__builtin_inff();
-            }
           }
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
@@ -334,8 +371,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
             }
           }
         }
-        // ---- gating: P[t][j] = scores * exp(u_t - w_j + G) / sqrt(DHQK) * rho_t, zero above the diagonal.  The
-        // vectors were written after the first barrier of this phase and NV - 1 >= 1 barriers have passed since.
+        // ---- gating: P[t][j] = scores * exp(u_t - w_j + G) / sqrt(DHQK) * rho_t, zero above the diagonal
         {
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
@@ -370,21 +406,6 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       // ============================================================================ phases Q (dQ) and K (dK)
       auto run_phase = [&](auto DKT, int dg) {
         constexpr bool dk = decltype(DKT)::value;
-        // column scale of the inter-chunk part: requested now by one thread per position, parked in LDS after the first
-        // step of the value pass, used after its last one (registers are what this kernel is short of)
-        float csn = 0.f;
-        if (tid < 256) {
-          const size_t gi = gofs + min(tid, n_pos - 1);
-          if (dk) {
-            // keys of c0 see dC through chunk c1, where there is one (the gradient kept is that after the last chunk)
-            const float xs = !RAGGED || c0 + 1 < NC ? __expf(graw[c0 + 1] + mst[c0 + 1] - mst[c0 + 2]) : 1.f;
-            csn = a.g.abar[gi] * (tid < 128 ? xs : 1.f);
-          } else {
-            const float xs = __expf(g01 + mst[c0] - mst[c0 + 1]);                // positions of c1 see C through chunk c0
-            const float rh = a.use_nrow ? 1.f / (a.nrow[gi] + a.eps) : 1.f;
-            csn = a.g.bbar[gi] * a.qk_scale * rh * (tid >= 128 ? xs : 1.f);
-          }
-        }
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -401,9 +422,6 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           __syncthreads();
           const unsigned char* const Cf = next_slab();
           if (w == 0) finish_rowdots();
-          // (one step after the request, so that its latency hides behind the first step; read after the last step of
-          // this loop, at least one barrier later)
-          if (w == (NV > 2 ? 1 : 0) && tid < 256) csv[tid] = csn;
           const unsigned char* const Xn = Cf + 16384;
           const int le = opaque(lane);
           const int r = le & 31, h = le >> 5;
