@@ -215,10 +215,8 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const uint32_t klim = (uint32_t)(S - 1) * (DHQK * 2) + pc * 16;  // this thread's piece of the last row
       {
         // ---- resident rows in four steps (for the consumers' epilogue of the previous item, and a step count per item that is
-        // a multiple of three): 32, 32, none and 64 rows.  The last one is a whole slab so that as many requests lie behind its
-        // register set as behind any other when the source chunks are reached without the state's steps: the compiler waits
-        // for the fewest there can be, and four fewer cost every item 2 to 5 %.  (The step without rows stores what its
-        // registers held where the rows of the last one go.)
+        // a multiple of three): 32, 32, none and 64 rows.  (The step without rows stores what its registers held where the rows of
+        // the last one go.  Four steps of 32 rows, or 32, 32, 32 and the rest in a whole slab, measure the same.)
         const char* const base = Xn_b + (size_t)it.bh * S * DHQK * 2;
         const uint32_t g0 = ((uint32_t)(it.c * kChunk) + row) * (DHQK * 2) + pc * 16;
         const uint32_t d0 = row * (QS * 2) + permo;
