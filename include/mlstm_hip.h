@@ -214,7 +214,7 @@ int mlstm_hip_head_norm_bw(const void* dY, const void* Y, const float* rstd, voi
  * No counterpart in the reference.  For callers that cannot allocate device memory around the call -- code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc: same arguments and results as
  * mlstm_hip_chunkwise_fw with keep_for_backward = 0, path = MLSTM_PATH_AUTO, state_stride = 0 and no head norm, but the workspace is
- * a static device array of MLSTM_NOALLOC_SCRATCH_BYTES inside the library (one copy per GPU, held until the process
+ * a static device array of MLSTM_NOALLOC_SCRATCH_BYTES (and 256 more for a flag) inside the library (one copy per GPU, held until the process
  * ends) instead of a caller-provided buffer.  The call allocates and frees nothing.  Shapes whose workspace
  * (mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DHQK, DHHV, 0, MLSTM_PATH_AUTO, 0)) exceeds the static scratch are
  * rejected.  All calls on one GPU share that GPU's scratch: calls that overlap in time on one GPU race.

@@ -18,7 +18,9 @@
 #include "kernels.h"
 
 namespace {
-static __device__ __align__(256) unsigned char scratch[MLSTM_NOALLOC_SCRATCH_BYTES];
+// (and 256 bytes for the word in which the forward notes that its initial state is zero: it takes no room from the rest)
+constexpr size_t kScratchBytes = (size_t)MLSTM_NOALLOC_SCRATCH_BYTES + 256;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
@@ -59,19 +61,19 @@ extern "C" int mlstm_hip_chunkwise_fw_noalloc(const void* q, const void* k, cons
   const size_t need = mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DHQK, DHHV, /*keep_for_backward=*/0,
                                                              MLSTM_PATH_AUTO, /*state_stride=*/0);
   if (need == 0) return fail_noalloc("unsupported shape (head dimensions must be multiples of 64, DHQK <= 896, B*NH <= 65535)");
-  if (need > (size_t)MLSTM_NOALLOC_SCRATCH_BYTES) {
+  if (need > kScratchBytes) {
     char msg[200];
     snprintf(msg, sizeof(msg),
              "this shape needs %zu bytes of scratch, the static scratch holds %zu; use mlstm_hip_chunkwise_fw with a "
              "caller-provided workspace",
-             need, (size_t)MLSTM_NOALLOC_SCRATCH_BYTES);
+             need, kScratchBytes);
     return fail_noalloc(msg);
   }
   const char* err = nullptr;
   void* ws = scratch_on_current_device(&err);
   if (ws == nullptr) return fail_noalloc(err);
   return mlstm_hip_chunkwise_fw(q, k, v, i, f, c0, n0, m0, H, n_out, m_out, c_last, n_last, m_last, ws,
-                                (size_t)MLSTM_NOALLOC_SCRATCH_BYTES, /*keep_for_backward=*/0, B, NH, S, DHQK, DHHV, eps,
+                                kScratchBytes, /*keep_for_backward=*/0, B, NH, S, DHQK, DHHV, eps,
                                 dtype_qkv, dtype_gates, gate, normalize, MLSTM_PATH_AUTO, /*state_stride=*/0,
                                 MLSTM_NORM_NONE, 0.f, nullptr, nullptr, stream);
 }

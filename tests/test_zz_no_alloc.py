@@ -119,3 +119,33 @@ def test_noalloc_forward_rejects_shapes_beyond_the_static_scratch():
     assert rc != 0
     msg = lib.mlstm_hip_last_error().decode()
     assert "static scratch" in msg and "caller-provided workspace" in msg
+
+
+def test_noalloc_forward_takes_a_shape_that_fills_the_static_scratch():
+    """64 MiB are there for what such a forward has always needed; the word for a zero initial state comes on top."""
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.utils import current_stream_ptr, ptr
+
+    lib = _lib.get_lib()
+    dev = torch.device("cuda")
+    B, NH, S, DHQK, DHHV = 1, 55, 19 * 128, 64, 896
+    need = lib.mlstm_hip_chunkwise_fw_workspace_bytes(B, NH, S, DHQK, DHHV, 0, _lib.PATH_AUTO, 0)
+    assert _lib.NOALLOC_SCRATCH_BYTES < need <= _lib.NOALLOC_SCRATCH_BYTES + 256
+    g = torch.Generator(device=dev).manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device=dev, generator=g)
+    q, k, v = rn(B, NH, S, DHQK).bfloat16(), rn(B, NH, S, DHQK).bfloat16(), rn(B, NH, S, DHHV).bfloat16()
+    i, f = rn(B, NH, S), 3 + rn(B, NH, S)
+    out = []
+    for noalloc in (True, False):
+        H = torch.empty_like(v)
+        head = [ptr(q), ptr(k), ptr(v), ptr(i), ptr(f), None, None, None, ptr(H), None, None, None, None, None]
+        tail = [B, NH, S, DHQK, DHHV, 1e-6, _lib.BF16, _lib.F32, _lib.GATE_EXP, 1]
+        if noalloc:
+            rc = lib.mlstm_hip_chunkwise_fw_noalloc(*head, *tail, current_stream_ptr(dev))
+        else:
+            ws = torch.empty(need, dtype=torch.uint8, device=dev)
+            rc = lib.mlstm_hip_chunkwise_fw(*head, ptr(ws), need, 0, *tail, _lib.PATH_AUTO, 0, _lib.NORM_NONE, 0.0, None, None, current_stream_ptr(dev))
+        _lib.check(rc, "forward")
+        torch.cuda.synchronize()
+        out.append(H)
+    assert torch.equal(*out)
