@@ -104,6 +104,9 @@ const char* launch_qk(int path, const mlstm::ParQkArgs& a, int BH, hipStream_t s
   if (choose_window_qk(path, a, BH)) return mlstm::launch_window_qk(a, BH, st);
   return mlstm::launch_par_qk_pair(a, BH, st);
 }
+bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  return a != nullptr && b != nullptr && (const char*)a < (const char*)b + b_bytes && (const char*)b < (const char*)a + a_bytes;
+}
 const char* check_dims(int B, int NH, int S, int DHQK, int DHHV) {
   if (B <= 0 || NH <= 0 || S <= 0) return "B, NH and S must be positive";
   if (DHQK <= 0 || DHHV <= 0 || DHQK % 64 != 0 || DHHV % 64 != 0) return "DHQK and DHHV must be positive multiples of 64";
@@ -287,7 +290,14 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     return check_launch("fused_hv forward");
   }
 
-  if (path == MLSTM_PATH_AUTO && !keep_for_backward && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr)) {
+  // States updated where they lie: the short kernel's workgroups of H read all of the initial state while others of the same
+  // launch write the last one.  Scan + H take these calls: a state tile is read and written by the same waves, and H reads the
+  // kept chunk states only.
+  const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float), n_bytes = (size_t)BH * DHQK * sizeof(float);
+  const bool in_place = overlap(c0, c_bytes, c_last, c_bytes) || overlap(n0, n_bytes, n_last, n_bytes) ||
+                        overlap(c0, c_bytes, n_last, n_bytes) || overlap(n0, n_bytes, c_last, c_bytes);
+  if (path == MLSTM_PATH_AUTO && !keep_for_backward && !in_place && head_norm == MLSTM_NORM_NONE &&
+      (n_last == nullptr || c_last != nullptr)) {
     mlstm::ShortFwArgs fa;
     memset(&fa, 0, sizeof(fa));
     fa.Q = (const uint16_t*)q; fa.K = (const uint16_t*)k; fa.V = (const uint16_t*)v;
