@@ -155,8 +155,8 @@ size_t mlstm_hip_chunkwise_fw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   H (B,NH,S,DHHV) in dtype_qkv.  n_out, m_out: optional fp32 (B,NH,S) per-row normaliser max(|den|,floor)
  *   and stabiliser (NULL to skip).  c_last,n_last,m_last: optional fp32 last states (NULL to skip).
  *   c_last, n_last, m_last may be c0, n0, m0 themselves (states updated in place; any other overlap is undefined).  Such a call
- *   does not take the kernel for short sequences: within the tolerance of the 16-bit operands, but not bit for bit, what
- *   separate buffers give.
+ *   does not take the kernel for short sequences and does not cut its scan into segments: within the tolerance of the 16-bit
+ *   operands, but not bit for bit, what separate buffers give.
  *   H serves the state scan as scratch before it is written (dV likewise in the backward).
  *   With c_last given, the state scan carries the gated values as a 16-bit head plus a 16-bit remainder in every
  *   chunk that still weighs at least 2^-8 in the last state, so c_last is accurate to ~1e-5 relative; with c_last
@@ -243,7 +243,7 @@ size_t mlstm_hip_chunkwise_bw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   fw_workspace: the forward's workspace, produced with keep_for_backward != 0 for the same inputs.
  *   dH (B,NH,S,DHHV) in dtype_qkv; dC_last optional fp32 gradient of the last C state (NULL = zero).
  *   dQ,dK (B,NH,S,DHQK), dV (B,NH,S,DHHV) in dtype_qkv; dI,dF fp32 (B,NH,S);
- *   dC0 optional fp32 (B,NH,DHQK,DHHV) gradient of the initial C state (NULL to skip).
+ *   dC0 optional fp32 (B,NH,DHQK,DHHV) gradient of the initial C state (NULL to skip); it may be dC_last itself.
  */
 int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const void* i, const void* f,
                            const void* dH, const float* dC_last,

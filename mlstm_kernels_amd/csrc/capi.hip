@@ -366,8 +366,9 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   // whose late positions may all be closed while early chunks dominate the state.
   sa.all_remainder = sig;
   // H is written after the scan.  (Where the caller names the path, the same kernels run whatever a sequence is batched
-  // with, and its results do not depend on the batch: no segments there.)
-  sa.seg = path == MLSTM_PATH_AUTO ? (float*)H : nullptr;
+  // with, and its results do not depend on the batch: no segments there.  Nor in place: every segment reads the initial state in
+  // the launch in which the last one writes the last state.)
+  sa.seg = path == MLSTM_PATH_AUTO && !in_place ? (float*)H : nullptr;
   sa.seg_bytes = (size_t)BH * S * DHHV * 2;
   {
     ProfileScope ps("scan_fw", st);
@@ -558,7 +559,9 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     sa.qk_scale = qk_scale; sa.eps = eps;
     sa.skip_zero = choose_hv(path, pv, BH) != kHvTiled && choose_window_qk(path, pq, BH);
     sa.backward = 1;
-    sa.seg = path == MLSTM_PATH_AUTO ? (float*)dV : nullptr;  // as in the forward; dV is written after the scan
+    // as in the forward; dV is written after the scan
+    const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float);
+    sa.seg = path == MLSTM_PATH_AUTO && !overlap(dC_last, c_bytes, dC0, c_bytes) ? (float*)dV : nullptr;
     sa.seg_bytes = (size_t)BH * S * DHHV * 2;
     sa.stride = stride;
     sa.f16 = f16;
