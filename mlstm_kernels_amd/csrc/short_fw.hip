@@ -535,20 +535,34 @@ const char* launch_short_d(const ShortFwArgs& a, int BH, hipStream_t stream) {
 }  // namespace
 
 // Where this kernel is the faster one: a workgroup of H takes 5 to 12 us by its number of keys and a CU one at a time, so with
-// many heads the streaming kernels, which keep the memory system busy, overtake it -- the sooner the longer the sequence.  The
-// line (positions in 64s times workgroups of H, per CU) from gates + scan + H against gates + this, us, at 256/512, 8 heads a
-// sequence: 200 positions B=4 48 / 37, B=8 64 / 60, B=16 95 / 106; 317: B=1 42.9 / 21.5, B=4 51 / 46, B=8 73 / 79; 512: B=1 42.8 /
-// 33.1, B=2 45 / 48, B=4 52 / 74.  At 128/256, 16 heads: 200 B=8 53 / 46, B=16 72 / 79; 512 B=2 40.6 / 39.4, B=4 49 / 60; 64/64, 8
-// heads: 512 B=8 37 / 30, B=16 39 / 45; 512/1024, 4 heads: 512 B=2 70 / 64, B=4 86 / 114.  An initial state counts as two more
-// slabs: 256/512, 200 positions B=4 50 / 44, B=8 66 / 77, 512 positions B=1 44 / 37, B=2 47 / 55.  Up to 128 positions it wins at
-// every size (256/512, B=64: 264 / 206, with 64 positions 236 / 120).
+// many heads scan + H, which keep the memory system busy, overtake it -- the sooner the longer the sequence and the larger the
+// head.  The line is drawn in positions in 64s times workgroups of H, per CU; an initial state counts as two more slabs.  us,
+// gates + scan + H / gates + this, B sequences (rows no cache holds up to 128 positions, repeated calls beyond):
+//  * more than 128 positions, 16.  256/512, 8 heads a sequence: 200 positions B=4 48 / 37, B=8 64 / 60, B=16 95 / 106; 317: B=1 42.9
+//    / 21.5, B=4 51 / 46, B=8 73 / 79; 512: B=1 42.8 / 33.1, B=2 45 / 48, B=4 52 / 74.  128/256, 16 heads: 200 B=8 53 / 46, B=16 72 /
+//    79; 512 B=2 40.6 / 39.4, B=4 49 / 60; 64/64, 8 heads: 512 B=8 37 / 30, B=16 39 / 45; 512/1024, 4 heads: 512 B=2 70 / 64, B=4 86 /
+//    114.  With a state, 256/512: 200 B=4 50 / 44, B=8 66 / 77, 512 B=1 44 / 37, B=2 47 / 55.
+//  * up to 128 positions in relation to the head: a head of 64 or 128 rows counts a quarter or a half, groups of 64 columns half.
+//    65 to 128 positions, 12, of 128: 128/256, 16 heads, B=32 72 / 74, B=48 104 / 109; 256/256, 8 heads, B=48 88 / 82, B=64 107 /
+//    115; 512/1024, 4 heads, B=24 165 / 135, B=32 145 / 162; 64/64, 8 heads, B=128 63 / 38; with a state 128/256 B=24 88 / 81, B=32
+//    97 / 107, 256/256 B=24 72 / 69, B=32 85 / 92.  7 where the other side is the streaming H / dV kernel: 256/512, 8 heads, B=8 35 /
+//    30, B=12 41 / 41, B=16 48.5 / 51, B=64 157 / 207; with a state B=4 34 / 24, B=8 49 / 48, B=12 59 / 67.
+//    Up to 64 positions without a state there is no line (256/512 B=64 138 / 116, 512/1024 B=32 142 / 105, 256/256 B=128 174 / 125);
+//    with one, 24 (256/256 B=128 269 / 240, 128/256 B=64 164 / 125) and 18 with the streaming kernel (256/512 B=48 170 / 168, B=64
+//    213 / 222).
 bool short_fw_preferred(const ShortFwArgs& a, int BH) {
   if (a.S > kShortMax || a.DHHV % 64 != 0) return false;
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256 && a.DHQK != 512) return false;
   if (a.DHQK == 512 && a.init != nullptr && a.S > 320) return false;  // LDS
   if ((uintptr_t)a.init % 16 != 0) return false;                      // (read by fours; the scan reads it one by one)
   const long long nt = (a.S + 63) / 64;
-  return nt <= 2 || BH * nt * (a.DHHV / (a.DHHV % 128 == 0 ? 128 : 64)) * (nt + (a.init != nullptr ? 2 : 0)) <= 16ll * device_cu_count();
+  const bool init = a.init != nullptr, wide = a.DHHV % 128 == 0;
+  long long cost = BH * nt * (a.DHHV / (wide ? 128 : 64)) * (nt + (init ? 2 : 0));
+  if (nt > 2) return cost <= 16ll * device_cu_count();
+  if (nt == 1 && !init) return true;
+  cost = cost * (a.DHQK < 256 ? a.DHQK : 256) / (wide ? 256 : 512);
+  const bool streaming = a.DHQK == 256 && a.DHHV % 512 == 0;
+  return cost <= (nt == 1 ? (streaming ? 18ll : 24ll) : (streaming ? 7ll : 12ll)) * device_cu_count();
 }
 
 const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream) {

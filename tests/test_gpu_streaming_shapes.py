@@ -250,6 +250,28 @@ def test_short_prompts_in_used_memory(S, DQ, DV):
         assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
 
 
+# Up to 128 positions many heads take scan + H as well: the most heads that the short kernel takes, and one more.
+@pytest.mark.parametrize("S,DQ,DV,init,most", [(128, 256, 512, False, 112), (65, 256, 512, True, 56), (64, 256, 512, True, 384),
+                                               (100, 128, 256, False, 768), (128, 64, 192, True, 1024)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_short_prompts_of_many_heads(S, DQ, DV, init, most, more):
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    NH = most + more
+    x = [torch.randn(1, NH, *d, device="cuda").bfloat16() for d in ((S, DQ), (S, DQ), (S, DV))]
+    gates = [torch.randn(1, NH, S, device="cuda"), 3 + torch.randn(1, NH, S, device="cuda")]
+    state = [torch.randn(1, NH, *d, device="cuda") for d in ((DQ, DV), (DQ,), (1,))] if init else [None] * 3
+    _lib.profile_read()
+    _lib.profile_enable(True)
+    try:
+        with torch.no_grad():
+            mlstm_chunkwise__hip_xl_chunk(*x, *gates, *state, return_last_states=True, any_sequence_length=True)
+    finally:
+        _lib.profile_enable(False)
+    assert ("short_fw" in _lib.profile_read()) == (more == 0)
+
+
 # States that are known to be zero are neither written nor multiplied: the same bits as with zeros handed over, whatever the
 # workspace holds (it is taken from memory full of NaN), for one window, several, and a ragged last one of either length.
 @pytest.mark.parametrize("DQ,DV,path", [(256, 512, "auto"), (256, 512, "stream"), (256, 512, "split"), (64, 64, "auto"), (128, 256, "auto"),
