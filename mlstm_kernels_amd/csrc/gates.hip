@@ -93,10 +93,13 @@ __device__ __forceinline__ ChunkScan scan_chunk(const void* ig, const void* fg, 
 }
 
 __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
-    const void* __restrict__ ig, const void* __restrict__ fg, GateBufs gb, int S, int NC, int dtype_gates,
-    int sig_gate, int zero_c) {
+    const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb, int S, int NC,
+    int dtype_gates, int sig_gate, int zero_c) {
   const int bh = blockIdx.y;
   if (bh == 0 && blockIdx.x == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
+  // m before the first chunk, for all workgroups of gates_finish_kernel: one of them writes m_last, which may be m0
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    gb.mstates[(size_t)bh * (NC + 1)] = !sig_gate && m0 != nullptr ? fmaxf(m0[bh], -__builtin_inff()) : 0.f;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = blockIdx.x * kGateChunks + wave;
   if (c >= NC) return;
@@ -116,8 +119,8 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
 // registers, the chunks meet in LDS, and every wave repeats the recurrence of m over them (a lane per chunk, the order of
 // gates_finish_kernel).
 __global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
-    const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb,
-    float* __restrict__ m_last, int S, int NC, int dtype_gates, int sig_gate, int zero_c) {
+    const void* __restrict__ ig, const void* __restrict__ fg, const float* m0, GateBufs gb, float* m_last, int S, int NC,
+    int dtype_gates, int sig_gate, int zero_c) {
   __shared__ float gs[kGateChunks], as[kGateChunks];
   const int bh = blockIdx.y;
   if (bh == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
@@ -172,8 +175,8 @@ __global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
   }
 }
 
-__global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(const float* __restrict__ m0, GateBufs gb,
-                                                                    float* __restrict__ m_last, int NC, int sig_gate) {
+__global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(GateBufs gb, float* __restrict__ m_last, int NC,
+                                                                    int sig_gate) {
   __shared__ float msh[kGateChunks + 1];  // m before the chunks of this workgroup, and after its last one
   const int bh = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(const float*
         if (m_last != nullptr) m_last[bh] = 0.f;
       }
     } else {
-      const float m_init = m0 != nullptr ? m0[bh] : 0.f;
+      const float m_init = mst[0];
       const int R = (NC + 63) / 64;
       const int c_lo = min(lane * R, NC), c_hi = min(c_lo + R, NC);
       float G = 0.f, A = NEG_INF;
@@ -231,7 +234,7 @@ __global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(const float*
         const float gc = graw[c];
         const float mn = fmaxf(m + gc, amax[c]);
         if (c >= c_first && c < c_end) {  // this workgroup's chunks: publish
-          mst[c] = m;
+          if (c > 0) mst[c] = m;
           gbar[c] = expf(gc + m - mn);
           msh[c - c_first] = m;
           msh[c - c_first + 1] = mn;
@@ -269,8 +272,8 @@ const char* launch_gates(const void* i, const void* f, const float* m0, const Ga
     return nullptr;
   }
   const dim3 grid((NC + kGateChunks - 1) / kGateChunks, B * NH);
-  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, gb, S, NC, dtype_gates, sig_gate, zero_c);
-  hipLaunchKernelGGL(gates_finish_kernel, grid, dim3(kGateThreads), 0, stream, m0, gb, m_last, NC, sig_gate);
+  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, m0, gb, S, NC, dtype_gates, sig_gate, zero_c);
+  hipLaunchKernelGGL(gates_finish_kernel, grid, dim3(kGateThreads), 0, stream, gb, m_last, NC, sig_gate);
   return nullptr;
 }
 

@@ -43,6 +43,15 @@ def test_short_sequences(S, DQ, DV, sig, noalloc):
         assert torch.equal(a, b), name
 
 
+# a head's gates in several workgroups, all of which need the first m, and scan + H (not in segments) either way: the same bits
+@pytest.mark.parametrize("S", [2048, 2049, 4100])
+@pytest.mark.parametrize("DQ,DV", [(64, 64), (256, 512)])
+def test_gates_of_several_workgroups(S, DQ, DV):
+    got, ref = (_forward(S, DQ, DV, in_place=p, NH=12, seed=S, f_offset=12.0) for p in (True, False))
+    for name, a, b in zip(("H", "C", "n", "m"), got, ref):
+        assert torch.equal(a, b), name
+
+
 # Few heads and a long sequence: the scan in segments, which all read the initial state, is not taken in place.  The states are
 # those of the scan in one piece (which a named path takes), H that of separate buffers but for the order of a sum in fp32.  Gates
 # near one: the initial state still weighs at the end.
