@@ -255,10 +255,11 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   }
   if (check_launch("gates")) return 1;
 
+  const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float), n_bytes = (size_t)BH * DHQK * sizeof(float);
   const bool track_n = !(sig && !normalize);  // the un-normalised sigmoid-gate variant leaves n untouched
-  if (!track_n && n_last != nullptr) {
+  if (!track_n && n_last != nullptr && n_last != n0) {
     if (n0 != nullptr) {
-      if (hipMemcpyAsync(n_last, n0, (size_t)BH * DHQK * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess)
+      if (hipMemcpyAsync(n_last, n0, n_bytes, hipMemcpyDeviceToDevice, st) != hipSuccess)
         return failw("copying n0 to n_last failed");
     } else if (const char* e = mlstm::launch_fill_zero(n_last, (size_t)BH * DHQK, st)) {
       return fail(e);
@@ -271,6 +272,12 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     fa.g = ws.g;
     fa.init = c0;
     fa.n_init = n0;
+    if (overlap(n0, n_bytes, n_last, n_bytes)) {
+      // every workgroup of a head reads n0 and the first one writes n_last: read from a copy, in a part of the workspace that this
+      // path does not use
+      if (hipMemcpyAsync(ws.nstates, n0, n_bytes, hipMemcpyDeviceToDevice, st) != hipSuccess) return failw("copying n0 failed");
+      fa.n_init = ws.nstates;
+    }
     fa.states = keep_for_backward ? ws.cstates : nullptr;
     fa.Out = (uint16_t*)H;
     fa.nrow_out = ws.nrow;
@@ -293,7 +300,6 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   // States updated where they lie: the short kernel's workgroups of H read all of the initial state while others of the same
   // launch write the last one.  Scan + H take these calls: a state tile is read and written by the same waves, and H reads the
   // kept chunk states only.
-  const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float), n_bytes = (size_t)BH * DHQK * sizeof(float);
   const bool in_place = overlap(c0, c_bytes, c_last, c_bytes) || overlap(n0, n_bytes, n_last, n_bytes) ||
                         overlap(c0, c_bytes, n_last, n_bytes) || overlap(n0, n_bytes, c_last, c_bytes);
   if (path == MLSTM_PATH_AUTO && !keep_for_backward && !in_place && head_norm == MLSTM_NORM_NONE &&

@@ -7,7 +7,7 @@ from helpers import rel_norm
 pytestmark = pytest.mark.gpu
 
 
-def _forward(S, DQ, DV, *, in_place, keep=0, path=0, NH=2, sig=False, noalloc=False, seed=0, f_offset=3.0, share="Cnm"):
+def _forward(S, DQ, DV, *, in_place, keep=0, path=0, NH=2, sig=False, normalize=1, noalloc=False, seed=0, f_offset=3.0, share="Cnm"):
     from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.utils import current_stream_ptr, ptr
 
@@ -20,7 +20,7 @@ def _forward(S, DQ, DV, *, in_place, keep=0, path=0, NH=2, sig=False, noalloc=Fa
     last = [t if in_place and x in share else torch.empty_like(t) for t, x in zip(first, "Cnm")]
     H = torch.empty_like(v)
     head = [ptr(t) for t in (q, k, v, i, f, *first, H)] + [None, None] + [ptr(t) for t in last]
-    tail = [1, NH, S, DQ, DV, 1e-6, _lib.BF16, _lib.F32, _lib.GATE_SIG if sig else _lib.GATE_EXP, 1]
+    tail = [1, NH, S, DQ, DV, 1e-6, _lib.BF16, _lib.F32, _lib.GATE_SIG if sig else _lib.GATE_EXP, normalize]
     if noalloc:
         _lib.check(lib.mlstm_hip_chunkwise_fw_noalloc(*head, *tail, current_stream_ptr(dev)), "fw_noalloc")
     else:
@@ -39,6 +39,16 @@ def _forward(S, DQ, DV, *, in_place, keep=0, path=0, NH=2, sig=False, noalloc=Fa
 def test_short_sequences(S, DQ, DV, sig, noalloc):
     got = _forward(S, DQ, DV, in_place=True, sig=sig, noalloc=noalloc, seed=S)
     ref = _forward(S, DQ, DV, in_place=False, sig=sig, keep=1, seed=S)
+    for name, a, b in zip(("H", "C", "n", "m"), got, ref):
+        assert torch.equal(a, b), name
+
+
+# the path of one kernel, whose workgroups of a head all read n0; and n that the operator leaves as it is: the same bits
+@pytest.mark.parametrize("path,sig,normalize", [("fused", False, 1), ("fused", True, 0), ("auto", True, 0), ("split", False, 1)])
+def test_named_paths(path, sig, normalize):
+    from mlstm_kernels_amd import _lib
+
+    got, ref = (_forward(700, 128, 256, in_place=p, path=_lib.path_code(path), sig=sig, normalize=normalize, NH=3) for p in (True, False))
     for name, a, b in zip(("H", "C", "n", "m"), got, ref):
         assert torch.equal(a, b), name
 
