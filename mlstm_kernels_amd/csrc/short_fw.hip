@@ -4,8 +4,8 @@
 //   P[t][j] = (q_t . k_j) / sqrt(DHQK) * exp(u_t - w_j + G)
 //   C_c     = gbar_c C_{c-1} + sum_{j in c} abar_j k_j v_j^T,   n_c = gbar_c n_{c-1} + sum_{j in c} abar_j k_j
 //
-// with the gate vectors of gates.hip (G: the decay of the chunks between those of j and t; cs_t: bbar_t / sqrt(DHQK) and the
-// decay of the chunks in front of t's).  Where the whole sequence is one
+// with the gate vectors of gates.hip (G: the decay of the chunks between those of j and t; cs_t: bbar_t / sqrt(DHQK), C0 decayed
+// over the chunks in front of t's).  Where the whole sequence is one
 // group of source chunks no chunk state is needed: H takes all keys as score blocks, and the last state is one product over all
 // positions.  Neither waits for the other, so ONE launch holds the workgroups of both:
 //   * H: 64 positions x CW value columns of a (batch, head).  Its eight waves take tiles of 16 keys in turn, two at a time, fetch
@@ -30,14 +30,14 @@ constexpr int kShortThreads = 512;
 
 template <int DQ, int CW, bool INIT>
 struct ShortLds {
-  // H: [Q rows, then (INIT: behind them) slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs]
+  // H: [Q rows, then (INIT: behind them) slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs, decay]
   static constexpr int QS = DQ + 8, VS = CW + 32;
   static constexpr int NBT = INIT ? 2 : 4;  // slabs of V at a time
   static constexpr int kFront = INIT ? 64 * QS + NBT * 64 * VS : (64 * QS > NBT * 64 * VS ? 64 * QS : NBT * 64 * VS);
   static constexpr int RT = DQ % 128 == 0 ? 128 : 64, WT = CW;  // state tile
   static constexpr int XS = RT + 32, YS = WT + 32;
   static size_t bytes(int nt, bool with_c) {
-    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 9 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 64) * 4 : 0);
+    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 9 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 65) * 4 : 0);
     // C: [K slab | head of V | remainder of V | abar | abar as an operand]
     const size_t c = (size_t)64 * (XS + 2 * YS) * 2 + kShortMax * 4 + kShortMax * 3 * 2;
     return with_c && c > h ? c : h;
@@ -64,7 +64,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   float* const rows = wv + kShortMax;  // [8 waves][64], INIT: q . n0 [64]
   float* const inv = rows + 9 * 64;
   float* const nv = inv + 64;    // INIT: n0
-  float* const csv = nv + DQ;    // INIT: cs_t
+  float* const csv = nv + DQ;    // INIT: cs_t, decay of the initial state up to this chunk
   const size_t Sp = (size_t)NC * kChunk, gofs = (size_t)bh * Sp;
   const uint16_t* const Qg = a.Q + (size_t)bh * S * DQ;
   const uint16_t* const Kg = a.K + (size_t)bh * S * DQ;
@@ -112,11 +112,12 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   wv[tid] = w_own;
   if constexpr (INIT) {
     if (tid < DQ) nv[tid] = a.use_nrow ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
-    if (tid < 64) {
+    if (tid < 64) csv[tid] = a.g.bbar[gofs + t0 + tid] * a.qk_scale;
+    if (tid == 64) {
       float gsum = 0.f;
       for (int y = 0; y < c; ++y) gsum += a.g.graw[(size_t)bh * NC + y];
       const float* const mst = a.g.mstates + (size_t)bh * (NC + 1);
-      csv[tid] = a.g.bbar[gofs + t0 + tid] * a.qk_scale * (c > 0 ? __expf(gsum + mst[0] - mst[c]) : 1.f);
+      csv[64] = c > 0 ? __expf(gsum + mst[0] - mst[c]) : 1.f;
     }
   }
   __syncthreads();
@@ -129,7 +130,11 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
       vr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
     }
 
+  // The state takes its decay up to this chunk in fp32, in front of its rounding: one beyond the range of float16 that has decayed
+  // into it is finite where it is seen there.
+  float pre = 1.f;
   if constexpr (INIT) {
+    pre = csv[64];
     // q_t . n0, eight threads per position
     const int t = tid >> 3, part = tid & 7;
     float dot = 0.f;
@@ -142,7 +147,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     dot += __shfl_xor(dot, 1);
     dot += __shfl_xor(dot, 2);
     dot += __shfl_xor(dot, 4);
-    if (part == 0) rows[8 * 64 + t] = csv[t] * dot;
+    if (part == 0) rows[8 * 64 + t] = csv[t] * pre * dot;
   }
   // ---- scores of this wave's tiles, gated into P
   {
@@ -264,7 +269,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
 #pragma unroll
       for (int y = 0; y < VV; ++y) {
         const int idx = tid + y * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
-        const f32x4 lo = cr[s & 1][y][0], hi = cr[s & 1][y][1];
+        const f32x4 lo = cr[s & 1][y][0] * pre, hi = cr[s & 1][y][1] * pre;
         *(uint4*)(slab + row * VS + u * 8) = make_uint4(pack2<F16>(lo[0], lo[1]), pack2<F16>(lo[2], lo[3]), pack2<F16>(hi[0], hi[1]), pack2<F16>(hi[2], hi[3]));
       }
       __syncthreads();

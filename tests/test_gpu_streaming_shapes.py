@@ -250,6 +250,22 @@ def test_short_prompts_in_used_memory(S, DQ, DV):
         assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("S,DQ,DV", [(256, 64, 64), (317, 256, 512), (512, 128, 192)])
+def test_short_prompts_from_a_large_state(S, DQ, DV):
+    """float16 from a state beyond its range: finite, and as exact as from a small one, in the chunks where it has decayed."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    q, k, v, i, f = make_qkvif(1, 2, S, DQ, DV, seed=S, dtype=torch.float16, f_offset=3.0)
+    g = torch.Generator().manual_seed(S)
+    st = [1e5 * torch.randn(1, 2, DQ, DV, generator=g), 1e5 * torch.randn(1, 2, DQ, generator=g), torch.zeros(1, 2, 1)]
+    with torch.no_grad():
+        H, last = mlstm_chunkwise__hip_xl_chunk(*(t.cuda() for t in (q, k, v, i, f, *st)), return_last_states=True,
+                                                any_sequence_length=True)
+    ref = O.chunkwise_fw(*(t.double() for t in (q, k, v, i, f)), *(t.double() for t in st), chunk_size=S)
+    assert rel_norm(H[:, :, 128:], ref["H"][:, :, 128:]) <= 1.5e-3  # an eighth of bf16's 6e-3 (three bits more), doubled
+    assert rel_norm(last[0], ref["C_last"]) <= 5e-5 and rel_norm(last[1], ref["n_last"]) <= 5e-6
+
+
 # Up to 128 positions many heads take scan + H as well: the most heads that the short kernel takes, and one more.
 @pytest.mark.parametrize("S,DQ,DV,init,most", [(128, 256, 512, False, 112), (65, 256, 512, True, 56), (64, 256, 512, True, 384),
                                                (100, 128, 256, False, 768), (128, 64, 192, True, 1024)])
