@@ -214,22 +214,23 @@ __global__ __launch_bounds__(768) void stream_hv_kernel(ParHvArgs a, int n_items
       const uint32_t permo = (pc >> 1) * 32 + 8 * (pc & 1);
       const uint32_t klim = (uint32_t)(S - 1) * (DHQK * 2) + pc * 16;  // this thread's piece of the last row
       {
-        // ---- resident rows in four steps (for the consumers' epilogue of the previous item, and a step count per item that is
-        // a multiple of three): 32, 32, none and 64 rows.  (The step without rows stores what its registers held where the rows of
-        // the last one go.  Four steps of 32 rows, or 32, 32, 32 and the rest in a whole slab, measure the same.)
+        // ---- resident rows, 32 per step (half-size slabs: four steps for the consumers' epilogue of the previous
+        // item, and a step count per item that is a multiple of three).  In 32, 32, none and 64 rows, H of 32 heads of 16384
+        // positions took 445 us instead of 439, of 128 heads of 1024 112 instead of 109.5.
         const char* const base = Xn_b + (size_t)it.bh * S * DHQK * 2;
         const uint32_t g0 = ((uint32_t)(it.c * kChunk) + row) * (DHQK * 2) + pc * 16;
         const uint32_t d0 = row * (QS * 2) + permo;
         HV_PROC(0, 4, base, g0, 8 * DHQK * 2, klim, d0, gown)
         HV_PROC(1, 4, base, g0 + 32 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 32 * QS * 2, gown)
-        HV_PROC(2, 0, base, g0, 0, klim, (d0 + 64 * QS * 2) | 1u << 23, gown)
-        HV_PROC(0, 8, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 64 * QS * 2, gown)
+        HV_PROC(2, 4, base, g0 + 64 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 64 * QS * 2, gown)
+        HV_PROC(0, 4, base, g0 + 96 * DHQK * 2, 8 * DHQK * 2, klim, d0 + 96 * QS * 2, gown)
       }
       {
         // ---- state fragments: slab si holds contraction steps 2 si, 2 si + 1 of the sixteen 32-column blocks.  Without a
-        // state the first two only (a state of another chunk, which nobody looks at): one step the consumers need for the
-        // denominators, one that makes the number of steps a multiple of three.  (Two steps and then threes, so that the
-        // loads behind every register set are as many whether the loop runs or not: the compiler's waits stay partial.)
+        // state the first two only: one step the consumers need for the denominators, one that makes the number of steps a
+        // multiple of three.  They fetch from the item's own slot, which is in bounds but was not written: what they put into
+        // the ring is arbitrary and must not be multiplied.  (A form without the loop, for launches with few such items, was no
+        // faster: 8 heads of 10000 positions with it and without it 87 us, 32 heads of 16384 439.)
         const char* const base = St_b + ((size_t)it.bh * NCS + it.slot) * (size_t)(DHHV / 32) * ND * 1024;
         const uint32_t f0 = pl >> 6;  // fragment of the first piece inside the slab: block f0 / 2, contraction step f0 % 2
         const uint32_t g0 = (((uint32_t)it.ch * (CW / 32) + (f0 >> 1)) * ND + (f0 & 1)) * 1024 + (pl & 63) * 16;
