@@ -53,6 +53,7 @@ class mLSTMBackend(nn.Module):
     """Wraps the mLSTM kernels behind one ``forward(q, k, v, i, f, ...)`` for training and inference."""
 
     config_class = mLSTMBackendConfig
+    _native_step = None  # (here as well: modules pickled before there was one have none of their own)
 
     def __init__(self, config: mLSTMBackendConfig):
         super().__init__()
@@ -75,7 +76,6 @@ class mLSTMBackend(nn.Module):
         )
         # One token from given states goes to the native step without the layers in between (sequence adapter, partials, step
         # function): a call of one sequence, whose kernel takes 6.6 us, 10.9 -> 9.4 us.  None: another step kernel or state type
-        self._native_step = None
         if self.step_kernel_fn is mlstm_recurrent_step__hip and state_dtype in _STATE_CODES:
             self._native_step = (None, None, None, config.eps, _STATE_CODES[state_dtype])
         train_fn = partial(

@@ -209,6 +209,21 @@ def test_arbitrary_sequence_length_wrapper_hands_whole_sequence_to_a_capable_ker
     torch.testing.assert_close(C, C_r, rtol=1e-9, atol=1e-9)
 
 
+def test_backend_module_pickled_without_a_native_step():
+    """A whole module saved before single tokens had a way of their own has no such attribute: they take the general one."""
+    q, k, v, i, f = make_qkvif(1, 2, 1, 32, 32, seed=3, dtype=torch.float32)
+    backend = mLSTMBackend(mLSTMBackendConfig(chunkwise_kernel="chunkwise--native_custbw", sequence_kernel="native_sequence__native",
+                                              step_kernel="native", chunk_size=32, mode="inference", autocast_kernel_dtype="float32"))
+    H, st = backend(q, k, v, i, f)
+    old = backend.__dict__.copy()
+    old.pop("_native_step", None)
+    restored = mLSTMBackend.__new__(mLSTMBackend)
+    restored.__setstate__(old)
+    got, ref = restored(q, k, v, i, f, *st), backend(q, k, v, i, f, *st)
+    for a, b in zip((got[0], *got[1]), (ref[0], *ref[1])):
+        assert torch.equal(a, b)
+
+
 def test_backend_inference_mode_threads_states():
     q, k, v, i, f = make_qkvif(1, 2, 100, 32, 32, seed=3, dtype=torch.float32)
     backend = mLSTMBackend(mLSTMBackendConfig(chunkwise_kernel="chunkwise--native_custbw", sequence_kernel="native_sequence__native",
