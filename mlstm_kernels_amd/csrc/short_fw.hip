@@ -20,7 +20,9 @@
 //     head and a 16-bit remainder, two products per block, as in the scan.
 // What bounds it: latency, four trips to memory or LDS in a row and the matrix work of one workgroup.  The streaming kernels
 // take this in three launches (gates, a scan of up to four chunks that run twice, H from the chunk states), each with most of
-// the chip idle.
+// the chip idle.  us for all launches, streaming kernels / gates and this, the same rows again and again: 8 heads of 256/512, 128
+// positions 27.5 / 11.8, 317 36.5 / 16.8, 512 36.5 / 27.9, 317 from a state 37.3 / 20.4; 16 heads of 128/256, 317 33.2 / 14.9.
+// Rows that no cache holds: 28.7 / 13.4, 39.3 / 19.0, 39.0 / 30.7; 36.2 / 18.0.
 #include "common.h"
 #include "kernels.h"
 
@@ -523,13 +525,18 @@ const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
 }
 template <int DQ, int CW, int NSL>
 const char* launch_short_c(const ShortFwArgs& a, int BH, hipStream_t stream) {
-  if (a.init != nullptr)
-    return a.f16 ? launch_short_t<DQ, CW, NSL, true, true>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, true>(a, BH, stream);
+  if (a.init != nullptr) {
+    // (the Q rows of 512 beside the V slabs and more than five score tiles do not fit the LDS: no instance)
+    if constexpr (DQ == 512 && NSL > 5) return "short_fw: too long for one CU's LDS";
+    else return a.f16 ? launch_short_t<DQ, CW, NSL, true, true>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, true>(a, BH, stream);
+  }
   return a.f16 ? launch_short_t<DQ, CW, NSL, true, false>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, false>(a, BH, stream);
 }
 template <int DQ, int CW>
 const char* launch_short_s(const ShortFwArgs& a, int BH, hipStream_t stream) {
-  // (registers and requests for as many slabs as there are, in three steps)
+  // Registers and requests for as many slabs as there are, in three steps.  us, 8 heads of 256/512, gates and this / eight slabs
+  // always / an instance for every number: 128 positions 11.8 / 12.9 / 11.8, 192 13.6 / 14.1 / 13.3, 317 16.8 / 17.4 / 17.0, 321 19.1 /
+  // 19.1 / 18.3, 448 25.7 / 25.7 / 25.6; 16 heads of 128/256: 128 9.9 / 11.4 / 10.0, 129 12.4 / 13.1 / 11.9, 384 16.9 / 16.9 / 16.5.
   if (a.S <= 128) return launch_short_c<DQ, CW, 2>(a, BH, stream);
   return a.S <= 320 ? launch_short_c<DQ, CW, 5>(a, BH, stream) : launch_short_c<DQ, CW, 8>(a, BH, stream);
 }
