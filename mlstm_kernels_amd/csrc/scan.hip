@@ -735,8 +735,9 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 // and overlap; four waves per SIMD instead of two.
 //
 // The workgroups are persistent (MANY; a launch of no more jobs than fit the chip keeps the plain form, whose loop has no
-// cursors): one workgroup fills a CU, and a tile of eight chunks spent a third of its time on filling the pipeline and on
-// its last stores with the CU otherwise idle.  Now the next tile's rows are on their way meanwhile.  Without a last state the
+// cursors).  As many run as fit by LDS, one per CU (tiles of 64 x 64: two); with more than kScanRounds jobs for each the grid
+// has more workgroups than are resident, each of which ends after its share.  Where one fills a CU, a tile of eight chunks spent
+// a third of its time on filling the pipeline and on its last stores with the CU otherwise idle.  Now the next tile's rows are on their way meanwhile.  Without a last state the
 // chunks behind the last kept boundary (in front of the first one) are not run: only n, for its own tiles, is wanted there.
 // Both together, us for a forward and backward call: 128 heads of 1024, 256/512, with layer norm 729 -> 665, 64 heads of 1000
 // 330 -> 302, 128 heads of 2048, 128/256 500 -> 487; 128 heads of 2048 with the last state, forward 418 -> 416.
