@@ -288,6 +288,20 @@ def test_short_prompts_of_many_heads(S, DQ, DV, init, most, more):
     assert ("short_fw" in _lib.profile_read()) == (more == 0)
 
 
+def _fill_free_memory_with_nan(sizes):
+    """What the allocator hands out next is full of NaN: blocks of up to 1 MiB, which have a pool of their own, and larger ones.
+    Checked for blocks of `sizes` bytes."""
+    torch.cuda.empty_cache()
+    nan = lambda n_bytes: torch.full((n_bytes // 4,), float("nan"), device="cuda")
+    full = [nan(1 << 30)] + [nan(1 << 20) for _ in range(64)]
+    # and the gaps between blocks in use
+    full += [nan(b["size"]) for seg in torch.cuda.memory_snapshot() for b in seg["blocks"] if b["state"] == "inactive"]
+    del full
+    probes = [torch.empty(n // 4, device="cuda") for n in sizes]
+    for t in probes:
+        assert bool(t.isnan().all())
+
+
 # States that are known to be zero are neither written nor multiplied: the same bits as with zeros handed over, whatever the
 # workspace holds (it is taken from memory full of NaN), for one window, several, and a ragged last one of either length.
 @pytest.mark.parametrize("DQ,DV,path", [(256, 512, "auto"), (256, 512, "stream"), (256, 512, "split"), (64, 64, "auto"), (128, 256, "auto"),
@@ -295,10 +309,12 @@ def test_short_prompts_of_many_heads(S, DQ, DV, init, most, more):
 @pytest.mark.parametrize("NH,S", [(1, 64), (2, 256), (3, 384), (2, 600), (96, 700), (40, 1300)])
 @pytest.mark.parametrize("stride,sig,dtype", [(2, False, torch.bfloat16), (2, True, torch.float16), (3, False, torch.bfloat16)], ids=str)
 def test_zero_states_that_are_left_out(DQ, DV, path, NH, S, stride, sig, dtype):
+    from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
 
     if path == "stream":
         S = (S + 127) // 128 * 128
+    lib, code = _lib.get_lib(), _lib.path_code(path)
     op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
     q, k, v, i, f = (t.cuda() for t in make_qkvif(1, NH, S, DQ, DV, seed=S, dtype=dtype, f_offset=3.0))
     dH = torch.randn(1, NH, S, DV, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
@@ -307,9 +323,8 @@ def test_zero_states_that_are_left_out(DQ, DV, path, NH, S, stride, sig, dtype):
     for init, d_last in ((None, False), (zeros, True)):
         leaves = [t.clone().requires_grad_(True) for t in (q, k, v, i, f)]
         st = dict(zip(("c_initial", "n_initial", "m_initial"), init)) if init else {}
-        torch.cuda.empty_cache()
-        full = torch.full((1 << 28,), float("nan"), device="cuda")
-        del full
+        _fill_free_memory_with_nan([lib.mlstm_hip_chunkwise_fw_workspace_bytes(1, NH, S, DQ, DV, 1, code, stride),
+                                    lib.mlstm_hip_chunkwise_bw_workspace_bytes(1, NH, S, DQ, DV, stride)])
         H, last = op(*leaves, **st, return_last_states=True, any_sequence_length=True, kernel_path=path, chunk_size_intra=128 * stride)
         if d_last:
             grads = torch.autograd.grad((H, last[0]), leaves, (dH, torch.zeros_like(last[0])))
