@@ -157,6 +157,8 @@ size_t mlstm_hip_chunkwise_fw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   c_last, n_last, m_last may be c0, n0, m0 themselves (states updated in place; any other overlap is undefined).  Such a call
  *   does not take the kernel for short sequences and does not cut its scan into segments: within the tolerance of the 16-bit
  *   operands, but not bit for bit, what separate buffers give.
+ *   With MLSTM_PATH_AUTO the kernel for short sequences serves calls without keep_for_backward only: up to 512 positions H with
+ *   and without it agree within the tolerance of the 16-bit operands, but not bit for bit.  With a named path they are the same.
  *   H serves the state scan as scratch before it is written (dV likewise in the backward).
  *   With c_last given, the state scan carries the gated values as a 16-bit head plus a 16-bit remainder in every
  *   chunk that still weighs at least 2^-8 in the last state, so c_last is accurate to ~1e-5 relative; with c_last

@@ -237,8 +237,8 @@ def mlstm_chunkwise__hip_xl_chunk(
     ``any_sequence_length=True`` (not in the reference) skips the reference's shape rules: the kernels mask a ragged
     tail themselves, so every S >= 1 is one call.  ``kernel_path`` ("auto", "split", "stream", "fused"; not in the
     reference) selects the kernels of the chunk-parallel passes; with "auto" the number of heads in the batch has a part in
-    the choice, so that the last bits of a sequence's results may depend on what it is batched with, which they do not with
-    the others.  ``chunk_size_intra`` (reference keyword) sets the distance between
+    the choice, so that the last bits of a sequence's results may depend on what it is batched with, and up to 512 positions on whether
+    a gradient is wanted (under ``no_grad`` one kernel takes H and the last state), which they do not with the others.  ``chunk_size_intra`` (reference keyword) sets the distance between
     kept chunk states; ``recompute_states_in_bw=True`` (reference keyword) keeps none of them between forward and
     backward.  ``head_norm`` ("none", "layer", "rms"; not in the reference's operator) fuses the multi-head
     norm that follows the cell in the xLSTM block -- the reference's ``apply_normalize(norm_specifier, x, eps)``,

@@ -291,6 +291,24 @@ def test_short_prompts_are_as_exact_as_scan_and_h(S, DQ, DV, init, dtype):
         assert a <= max(1.05 * b, 2 ** -22)  # (states: below it, what the last rounding to 32 bits leaves)
 
 
+# Without a gradient "auto" takes H of a short sequence from another kernel: each is within 2.5e-3 of 64 bits (above), so they are
+# within the sum of it of each other; with the path named the bits are the same.
+@pytest.mark.parametrize("S,DQ,DV", [(65, 64, 64), (317, 256, 512), (512, 128, 256)])
+@pytest.mark.parametrize("path", ["auto", "split"])
+@pytest.mark.parametrize("last", [False, True])
+def test_forward_with_and_without_a_gradient(S, DQ, DV, path, last):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    x = [t.cuda().requires_grad_(True) for t in make_qkvif(1, 4, S, DQ, DV, seed=S, f_offset=3.0)]
+    out = []
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            r = mlstm_chunkwise__hip_xl_chunk(*x, return_last_states=last, any_sequence_length=True, kernel_path=path)
+        out.append([t.detach() for t in ((r[0], *r[1]) if last else (r,))])
+    for a, b, tol in zip(*out, (5e-3, 1e-5, 1e-6, 0.0)):
+        assert torch.equal(a, b) if path == "split" else rel_norm(a, b) <= tol
+
+
 # Up to 128 positions many heads take scan + H as well: the most heads that the short kernel takes, and one more.
 @pytest.mark.parametrize("S,DQ,DV,init,most", [(128, 256, 512, False, 112), (65, 256, 512, True, 56), (64, 256, 512, True, 384),
                                                (100, 128, 256, False, 768), (128, 64, 192, True, 1024)])
