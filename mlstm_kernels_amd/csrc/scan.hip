@@ -492,14 +492,25 @@ struct ScanJob {
 
 // Job of workgroup `vid` in round `round`.  Consecutive workgroups of an XCD take consecutive jobs: all tiles of one (batch,
 // head), which share its K / V rows in the L2.  The assignment rotates by one column of tiles per round, so that the first
-// column's tiles, which carry n and may run a chunk more, do not all fall to the same workgroups.
+// column's tiles, which carry n and may run a chunk more, do not all fall to the same workgroups.  A last round with jobs for some
+// of the workgroups only gives every XCD an eighth of them: as they come they would all lie on the first ones (576 tiles of 64 x 64,
+// 2048 positions, 54.9 -> 51.9 us without the last state).
 template <int RT, int WT, bool REP, bool SEG>
 __device__ __forceinline__ ScanJob scan_decode(const ScanArgs& a, int round, int vid, int lane) {
   ScanJob job = {0, 0, 0, 0, 0, 0, 0, 0};
   const int G = (int)gridDim.x, nx = a.DHQK / RT, ny = a.DHHV / WT;
-  const int rot = (int)((vid + (unsigned)round * nx) % (unsigned)G);
-  const long long idx = (long long)round * G + rot;
-  if (idx >= a.n_jobs) return job;
+  const long long left = a.n_jobs - (long long)round * G;  // jobs of this round and the later ones
+  long long idx = (long long)round * G;
+  if (left < G && G % 8 == 0) {
+    // the last round, with jobs for some of the workgroups only: an eighth of them for each XCD
+    const int per = G / 8, x = vid / per, l = (int)((vid % per + (unsigned)round * nx) % (unsigned)per);
+    const int lo = x * (int)left / 8, hi = (x + 1) * (int)left / 8;
+    if (l >= hi - lo) return job;
+    idx += lo + l;
+  } else {
+    idx += (vid + (unsigned)round * nx) % (unsigned)G;
+    if (idx >= a.n_jobs) return job;
+  }
   job.bx = (int)idx % nx;
   job.by = ((int)idx / nx) % ny;
   const int z = (int)idx / (nx * ny);
@@ -787,15 +798,22 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     const int c_base = a.backward ? NC - 1 : 0, c_step = a.backward ? -1 : 1;
     const int xrow = tid / XU, yrow = tid / YU;  // first row of this thread inside a chunk; further rows XRG / YRG apart
     const int xcol = (tid % XU) * 8, ycol = (tid % YU) * 8;
+    // byte offsets of the first row inside a chunk of the operands
+    const uint32_t xofs = (uint32_t)(xrow * DHQK + xcol) * 2, yofs = (uint32_t)(yrow * DHHV + ycol) * 2;
     // LDS store offsets of the first row (elements); the rows of a thread are a multiple of 4 apart: same swizzle
     const int xst = xrow * RT + (((tid % XU) ^ scan_swz<XU>(xrow)) << 3);
     const int yst = yrow * WT + (((tid % YU) ^ scan_swz<YU>(yrow)) << 3);
 
+    // (Scalar bases and 32-bit offsets inside a chunk: with a 64-bit product for every row, and with the bases worked out from the
+    // job's indexes in every run, the producers' instructions were what a narrow tile took.  256/320, 16 heads of 512 / of 2048 with
+    // the last state: 14.2 -> 13.1, 30.4 -> 28.1 us; 40 heads of 256/512, 512 positions, backward 23.3 -> 22.3.)
     // The runs of all jobs of this workgroup form one sequence, and the producers work ahead of it without regard to where a
     // job ends: run P + 3 is requested and run P + 1 staged while run P is multiplied, the scales of the chunk three ahead
     // are requested.  Two cursors walk the jobs, one over runs and one over chunks; past the last job they stay where they
     // are (the requests are unconditional: a conditional one makes the compiler keep the registers in scratch memory).
     int r_rd = -1, r_p = -1, r_bh = job0.bh, r_bx = job0.bx, r_by = job0.by, r_par = 0;  // run cursor
+    const uint16_t* r_x = a.X + (size_t)r_bh * S * DHQK + r_bx * RT;
+    const uint16_t* r_y = a.Y + (size_t)r_bh * S * DHHV + r_by * WT;
     ScanRuns<REP> rr;
     rr.set(job0.it_lo, job0.it_hi, job0.it_rep);
     int k_rd = -1, k_bh = job0.bh, k_by = job0.by, k_it = job0.it_lo - 1, k_hi = job0.it_hi;  // chunk cursor
@@ -819,6 +837,8 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
         r_by = __builtin_amdgcn_readfirstlane(jobs[r_rd].by);
         rr.set(lo, hi, rep);
         r_p = 0;
+        r_x = a.X + (size_t)r_bh * S * DHQK + r_bx * RT;
+        r_y = a.Y + (size_t)r_bh * S * DHHV + r_by * WT;
       }
       const bool last = rr.last(r_p);
       const int m = 1 | (rr.rest(r_p) ? 2 : 0) | (last ? 4 : 0) | (r_par << 3);
@@ -856,11 +876,11 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     int s_lim = 0;       // rows of the chunk that lie inside the sequence
     bool s_n = false;    // whether the chunk's tile carries n
     auto load_scales = [&](bool there) {  // of the chunk cursor's chunk
-      const int c = c_base + max(k_it, 0) * c_step;
-      const size_t o = (size_t)k_bh * Sp + c * kChunk + srow;
-      s_raw = a.scale_a[o];
-      s_nrm = nrow_or_dummy[o];
-      s_g = a.gbar[(size_t)k_bh * NC + c + opaque(0)];
+      const int c = __builtin_amdgcn_readfirstlane(c_base + max(k_it, 0) * c_step);
+      const size_t o = (size_t)k_bh * NC + c;
+      s_raw = (a.scale_a + o * kChunk)[(uint32_t)srow];
+      s_nrm = (nrow_or_dummy + o * kChunk)[(uint32_t)srow];
+      s_g = (a.gbar + o)[(uint32_t)opaque(0)];
       s_lim = there ? S - c * kChunk : 0;
       s_n = there && a.nstates != nullptr && k_by == 0;
     };
@@ -878,8 +898,9 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     // (position 8b + e of a chunk, part r, at [b][r][e]); K^T times it gives sum_j abar_j k_j in three partial columns
     // whose sum carries 24 bits of every abar_j.  Written two chunks before the chunk is multiplied, three slots.
     auto write_tables = [&](int chunk) {
-      const float sn = scale_value();
-      if (tid < kChunk) {
+      // (two waves have all rows: the others leave the division of the backward out)
+      if (NTP == kChunk || wave < kChunk / 64) {
+        const float sn = scale_value();
         scl[(chunk & 1) * kChunk + srow] = sn;
         if (tid == 0) gl[chunk & 3] = s_g;
         if (s_n) {
@@ -901,18 +922,15 @@ __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel
     // The prefetch only LOADS: any arithmetic on a loaded value here would make the wave wait for the whole batch.
 #define MLSTM_SCAN_PREFETCH(SET)                                                                                 \
   {                                                                                                              \
-    const int t0_ = (c_base + rr.it(max(r_p, 0)) * c_step) * kChunk;                                                \
-    const uint16_t* const Xg = a.X + (size_t)r_bh * S * DHQK + r_bx * RT + xcol;                               \
-    const uint16_t* const Yg = a.Y + (size_t)r_bh * S * DHHV + r_by * WT + ycol;                               \
-    _Pragma("unroll") for (int v = 0; v < XV; ++v) {                                                             \
-      /* rows past the end re-read the last row; their scale is 0 */                                             \
-      const int t = min(t0_ + xrow + v * XRG, S - 1);                                                            \
-      xr##SET[v] = *(const u32x4*)(Xg + (size_t)t * DHQK);                                                       \
-    }                                                                                                            \
-    _Pragma("unroll") for (int v = 0; v < YV; ++v) {                                                             \
-      const int t = min(t0_ + yrow + v * YRG, S - 1);                                                            \
-      yr##SET[v] = *(const u32x4*)(Yg + (size_t)t * DHHV);                                                       \
-    }                                                                                                            \
+    const int t0_ = __builtin_amdgcn_readfirstlane((c_base + rr.it(max(r_p, 0)) * c_step) * kChunk);             \
+    const int last_ = min(kChunk - 1, S - 1 - t0_); /* rows past the end re-read the last row; their scale is 0 */ \
+    const char* const xb_ = (const char*)(r_x + (size_t)t0_ * DHQK);                                             \
+    const char* const yb_ = (const char*)(r_y + (size_t)t0_ * DHHV);                                             \
+    const uint32_t xl_ = (uint32_t)(last_ * DHQK + xcol) * 2, yl_ = (uint32_t)(last_ * DHHV + ycol) * 2;         \
+    _Pragma("unroll") for (int v = 0; v < XV; ++v)                                                               \
+      xr##SET[v] = *(const u32x4*)(xb_ + min(xofs + (uint32_t)(v * XRG * 2) * (uint32_t)DHQK, xl_));              \
+    _Pragma("unroll") for (int v = 0; v < YV; ++v)                                                               \
+      yr##SET[v] = *(const u32x4*)(yb_ + min(yofs + (uint32_t)(v * YRG * 2) * (uint32_t)DHHV, yl_));              \
   }
     // registers -> LDS buffer SET (Y rows scaled in fp32, then rounded; second runs: the remainder of that rounding)
 #define MLSTM_SCAN_STAGE(SET, meta_)                                                                             \
@@ -1034,7 +1052,14 @@ static const char* launch_scan_roles_f(ScanArgs a, int BH, hipStream_t stream) {
   if (cus <= 0) return "scan: cannot read the number of compute units";
   a.n_jobs = (int)n_jobs;
   const int fit = cus * (int)(160 * 1024 / scan_roles_smem(RT, WT));
-  if (a.n_jobs <= fit) return launch_scan_roles_m<RT, WT, F16, REP, SEG, false>(a, a.n_jobs, 1, stream);
+  // Few tiles more than fit: where a tile is smaller than 128 x 128 a workgroup for each, which start as others end, is the faster
+  // form (fixed shares make the last of them late); not with one tile a head.  Us, persistent / a workgroup each, with the last
+  // state, without, backward: 256/320, 32 heads (1.25 tiles for each that fits) of 512 24.2 14.3 16.8 / 22.0 12.0 17.1, of 2048
+  // 52.4 41.6 41.4 / 50.0 37.1 41.2; 64/384, 112 heads (1.3) of 2048 70.8 58.7 66.6 / 66.5 56.6 67.8; 192/192, 64 heads (1.1) of 2048
+  // 68.6 53.8 51.6 / 63.9 49.5 49.7; but 128/192, 168 heads (2.0) of 2048 71.1 60.2 62.1 / 72.5 62.7 65.0 and 64/64, 640 heads (1.25)
+  // of 2048 96.1 84.5 83.1 / 104.6 89.7 88.1.
+  const bool few = (RT < 128 || WT < 128) && a.n_jobs > BH && 5ll * a.n_jobs < 7ll * fit;
+  if (a.n_jobs <= fit || (!SEG && few)) return launch_scan_roles_m<RT, WT, F16, REP, SEG, false>(a, a.n_jobs, 1, stream);
   if constexpr (SEG) {
     return "scan: more segments than the chip holds";
   } else {

@@ -154,7 +154,10 @@ def test_named_paths_do_not_depend_on_the_batch(path, S, DQ, DV):
 # chunks behind the last kept state are not run, with and without a last state, with strides that divide the chunks and not.
 # With the path named a head's bits do not depend on how the tiles fall to the workgroups.
 @pytest.mark.parametrize("DQ,DV,BH,S", [(256, 512, 33, 129), (256, 512, 80, 640), (64, 64, 514, 385), (128, 64, 300, 257), (64, 128, 300, 640),
-                                        (64, 64, 16500, 130)])
+                                        (64, 64, 16500, 130),
+                                        # tiles smaller than 128 x 128 around the line below which each has a workgroup of its own
+                                        (256, 320, 26, 385), (256, 320, 35, 640), (256, 320, 36, 257), (192, 192, 57, 257), (192, 192, 80, 640),
+                                        (64, 384, 119, 129), (64, 384, 120, 385)])
 @pytest.mark.parametrize("last,stride,init", [(False, 1, False), (False, 2, True), (False, 3, False), (True, 2, False), (True, 3, True)])
 def test_state_tiles_on_persistent_workgroups(DQ, DV, BH, S, last, stride, init):
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
