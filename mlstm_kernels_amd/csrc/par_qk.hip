@@ -74,6 +74,8 @@ __device__ __forceinline__ void par_qk_body(const ParQkArgs& a, const BlockId bl
   const int n0 = 64 * nh;
   const int stride = a.stride;
   const int slot = c / stride;
+  // (an initial state that is zero has no fragments; the gradient after the last chunk always has them where this kernel runs)
+  const bool no_state = IS_DQ && slot == 0 && __builtin_amdgcn_readfirstlane(*a.g.zero_c) != 0;
   // source chunks of the score blocks: dQ c0 .. c, dK c .. c1; the own chunk is handled first, together with the state
   const int sc_lo = IS_DQ ? slot * stride : c;
   const int sc_hi = IS_DQ ? c : min(slot * stride + stride - 1, NC - 1);
@@ -179,21 +181,23 @@ __device__ __forceinline__ void par_qk_body(const ParQkArgs& a, const BlockId bl
     constexpr int CV = NDT * 64 / NTH;      // state-fragment vectors per thread per slab
     // The state fragments come in slabs of 32 value columns, two slabs in flight in registers.
     u32x4 cregA[CV], cregB[CV];
+    // through a buffer descriptor: of no bytes where the state is known to be zero, so that the loads give zeros and nothing is selected
+    // behind them (16 selects a slab were 3 % of the kernel: 256/320, 32 heads of 400 positions 29.6 -> 30.4 us, now 28.9; 512/448 61.2
+    // -> 63.0 -> 61.3)
+    const auto st_buf = __builtin_amdgcn_make_buffer_rsrc((void*)st, 0, no_state ? 0 : (int)(NW * ND * 1024), 0x00020000);
 #define MLSTM_LOAD_C(slab_, creg)                                                                                    \
   {                                                                                                                  \
+    const int o_ = tid * 16 + ((slab_) * (int)ND + d_tile / 16) * 1024;                                              \
     _Pragma("unroll") for (int v = 0; v < CV; ++v)                                                                   \
-        creg[v] = st[((size_t)(slab_) * ND + d_tile / 16) * 64 + tid + v * NTH];                                     \
+        creg[v] = __builtin_amdgcn_raw_buffer_load_b128(st_buf, o_ + v * NTH * 16, 0, 0);                            \
   }
-    // (an initial state that is zero has no fragments; the gradient after the last chunk always has them where this kernel runs)
-    const bool no_state = IS_DQ && slot == 0 && *a.g.zero_c != 0;
     // lanes 32..63 of every state fragment are stored 4 slots off so that the two lane halves a transposing read
     // touches together fall on different LDS banks
 #define MLSTM_STORE_C(creg)                                                                                          \
   {                                                                                                                  \
     _Pragma("unroll") for (int v = 0; v < CV; ++v) {                                                                 \
       const int idx = tid + v * NTH;                                                                                 \
-      const u32x4 none = {0u, 0u, 0u, 0u};                                                                           \
-      ((u32x4*)Cf)[idx ^ (((idx >> 5) & 1) << 2)] = no_state ? none : creg[v];                                       \
+      ((u32x4*)Cf)[idx ^ (((idx >> 5) & 1) << 2)] = creg[v];                                                         \
     }                                                                                                                \
   }
     // transposing read of the staged fragments: lane i16 of a 16-lane block addresses value column
