@@ -182,8 +182,8 @@ __device__ __forceinline__ void par_qk_body(const ParQkArgs& a, const BlockId bl
     // The state fragments come in slabs of 32 value columns, two slabs in flight in registers.
     u32x4 cregA[CV], cregB[CV];
     // through a buffer descriptor: of no bytes where the state is known to be zero, so that the loads give zeros and nothing is selected
-    // behind them (16 selects a slab were 3 % of the kernel: 256/320, 32 heads of 400 positions 29.6 -> 30.4 us, now 28.9; 512/448 61.2
-    // -> 63.0 -> 61.3)
+    // behind them (16 selects a slab were 3 % of the kernel: 256/320, 32 heads of 400 positions 29.6 -> 30.4 us, now 29.7; 512/448 61.1
+    // -> 63.0 -> 61.0)
     const auto st_buf = __builtin_amdgcn_make_buffer_rsrc((void*)st, 0, no_state ? 0 : (int)(NW * ND * 1024), 0x00020000);
 #define MLSTM_LOAD_C(slab_, creg)                                                                                    \
   {                                                                                                                  \
