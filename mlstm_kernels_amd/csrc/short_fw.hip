@@ -559,7 +559,8 @@ const char* launch_short_d(const ShortFwArgs& a, int BH, hipStream_t stream) {
 //    115; 512/1024, 4 heads, B=24 165 / 135, B=32 145 / 162; 64/64, 8 heads, B=128 63 / 38; with a state 128/256 B=24 88 / 81, B=32
 //    97 / 107, 256/256 B=24 72 / 69, B=32 85 / 92.  7 where the other side is the streaming H / dV kernel: 256/512, 8 heads, B=8 35 /
 //    30, B=12 41 / 41, B=16 48.5 / 51, B=64 157 / 207; with a state B=4 34 / 24, B=8 49 / 48, B=12 59 / 67.
-//    Up to 64 positions without a state there is no line (256/512 B=64 138 / 116, 512/1024 B=32 142 / 105, 256/256 B=128 174 / 125);
+//    Up to 64 positions without a state there is no line (256/512 B=64 138 / 116, 512/1024 B=32 142 / 105, 256/256 B=128 174 / 125;
+//    1024 heads of 64 positions with all launches, groups of 64 columns: 64/192 127 / 49, 512/448 1105 / 615, 64/960 477 / 247);
 //    with one, 24 (256/256 B=128 269 / 240, 128/256 B=64 164 / 125) and 18 with the streaming kernel (256/512 B=48 170 / 168, B=64
 //    213 / 222).
 bool short_fw_preferred(const ShortFwArgs& a, int BH) {
