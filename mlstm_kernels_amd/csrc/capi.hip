@@ -328,6 +328,35 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     }
   }
 
+  if (path == MLSTM_PATH_AUTO && !in_place && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr)) {
+    mlstm::ChainHvArgs ca;
+    memset(&ca, 0, sizeof(ca));
+    ca.Q = (const uint16_t*)q; ca.K = (const uint16_t*)k; ca.V = (const uint16_t*)v;
+    ca.g = ws.g;
+    ca.init = c0;
+    ca.n_init = n0;
+    ca.states = keep_for_backward ? ws.cstates : nullptr;
+    ca.Out = (uint16_t*)H;
+    ca.nrow_out = ws.nrow;
+    ca.n_out = n_out; ca.m_out = m_out;
+    ca.final_out = c_last;
+    ca.n_final = track_n ? n_last : nullptr;
+    ca.S = S; ca.NC = NC; ca.DHQK = DHQK; ca.DHHV = DHHV;
+    ca.qk_scale = 1.0f / sqrtf((float)DHQK); ca.eps = eps;
+    ca.sig_gate = sig;
+    ca.use_nrow = track_n;
+    ca.stride = stride;
+    ca.f16 = f16;
+    ca.skip_zero = !has_c0;  // (both dQ / dK kernels know, from g.zero_c)
+    if (mlstm::chain_hv_preferred(ca, BH)) {
+      {
+        ProfileScope ps("chain_h", st);
+        if (const char* e = mlstm::launch_chain_hv(ca, BH, /*is_dv=*/false, st)) return fail(e);
+      }
+      return check_launch("chain_hv forward");
+    }
+  }
+
   mlstm::ParHvArgs pa;
   memset(&pa, 0, sizeof(pa));
   pa.Q = (const uint16_t*)q; pa.K = (const uint16_t*)k; pa.V = (const uint16_t*)v;
@@ -517,6 +546,24 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
   // dQ and dK in one launch: the workgroups of a chunk run side by side and share the Q, K, V and dH rows they stream
   pq.states = ws.cstates; pq.Out = (uint16_t*)dQ; pq.rowdot = bws.qdq;
   pq.states2 = bws.dcstates; pq.Out2 = (uint16_t*)dK; pq.rowdot2 = bws.kdk;
+  const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float);
+  const bool in_place = overlap(dC_last, c_bytes, dC0, c_bytes);
+  mlstm::ChainHvArgs ca;
+  memset(&ca, 0, sizeof(ca));
+  ca.Q = (const uint16_t*)q; ca.K = (const uint16_t*)k; ca.V = (const uint16_t*)v; ca.dH = (const uint16_t*)dH;
+  ca.g = ws.g;
+  ca.init = dC_last;
+  ca.nrow = ws.nrow;
+  ca.states = bws.dcstates;
+  ca.Out = (uint16_t*)dV;
+  ca.final_out = dC0;
+  ca.S = S; ca.NC = NC; ca.DHQK = DHQK; ca.DHHV = DHHV;
+  ca.qk_scale = qk_scale; ca.eps = eps;
+  ca.sig_gate = sig; ca.use_nrow = use_nrow;
+  ca.stride = stride;
+  ca.f16 = f16;
+  ca.skip_zero = dC_last == nullptr && choose_window_qk(path, pq, BH);
+  const bool use_chain = path == MLSTM_PATH_AUTO && mlstm::chain_hv_preferred(ca, BH);
   if (use_fused(path, DHQK, DHHV)) {
     if (f16) return fail("mlstm_hip_chunkwise_bw: the fused kernel path multiplies bf16 operands only");
     mlstm::FusedHvArgs fa;
@@ -537,6 +584,12 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
       if (const char* e = mlstm::launch_fused_hv(fa, BH, /*is_dv=*/true, st)) return fail(e);
     }
     if (check_launch("fused_hv dV")) return 1;
+  } else if (use_chain) {
+    {
+      ProfileScope ps("chain_dv", st);
+      if (const char* e = mlstm::launch_chain_hv(ca, BH, /*is_dv=*/true, st)) return fail(e);
+    }
+    if (check_launch("chain_hv dV")) return 1;
   } else {
     mlstm::ParHvArgs pv;
     memset(&pv, 0, sizeof(pv));
@@ -566,8 +619,7 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
     sa.skip_zero = choose_hv(path, pv, BH) != kHvTiled && choose_window_qk(path, pq, BH);
     sa.backward = 1;
     // as in the forward; dV is written after the scan
-    const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float);
-    sa.seg = path == MLSTM_PATH_AUTO && !overlap(dC_last, c_bytes, dC0, c_bytes) ? (float*)dV : nullptr;
+    sa.seg = path == MLSTM_PATH_AUTO && !in_place ? (float*)dV : nullptr;
     sa.seg_bytes = (size_t)BH * S * DHHV * 2;
     sa.stride = stride;
     sa.f16 = f16;

@@ -133,6 +133,29 @@ struct FusedHvArgs {
   int stride;               // a chunk state is emitted every `stride` chunks
 };
 
+// State recurrence and output in one launch (chain_hv.hip)
+struct ChainHvArgs {
+  const uint16_t *Q, *K, *V, *dH;  // forward uses Q,K,V; dV uses Q,K,dH
+  GateBufs g;
+  const float* init;        // (B,NH,DHQK,DHHV) fp32 initial state (forward: C0, dV: dC_last) or nullptr (zeros)
+  const float* n_init;      // forward: (B,NH,DHQK) or nullptr
+  const float* nrow;        // dV: row normaliser of the forward pass
+  uint16_t* states;         // state fragments [BH][ceil(NC/stride)][DHHV/32][DHQK/16][64][8] or nullptr (not kept)
+  uint16_t* Out;            // (B,NH,S,DHHV): H or dV
+  float* nrow_out;          // forward: row normaliser (workspace [BH][Sp])
+  float* n_out;             // forward, optional (B,NH,S)
+  float* m_out;             // forward, optional (B,NH,S)
+  float* final_out;         // (B,NH,DHQK,DHHV) fp32 or nullptr: C_last (forward) / dC0 (dV)
+  float* n_final;           // forward: (B,NH,DHQK) or nullptr
+  int S, NC, DHQK, DHHV;
+  float qk_scale, eps;
+  int sig_gate;
+  int use_nrow;             // 0 only for the un-normalised sigmoid-gate variant (n is then not tracked)
+  int stride;               // a chunk state is kept every `stride` chunks
+  int f16;
+  int skip_zero;            // the first kept state is zero and its readers know
+};
+
 constexpr int kShortMax = 512;  // longest sequence of the short forward
 struct ShortFwArgs {
   const uint16_t *Q, *K, *V;
@@ -211,6 +234,8 @@ const char* launch_window_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t
 bool short_fw_preferred(const ShortFwArgs& a, int BH);
 const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream);
 const char* launch_head_norm_bw(const HeadNormBwArgs& a, hipStream_t stream);
+bool chain_hv_preferred(const ChainHvArgs& a, int BH);
+const char* launch_chain_hv(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 bool fused_hv_supported(int DHQK, int DHHV);
 const char* launch_fused_hv(const FusedHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 const char* launch_par_qk_pair(const ParQkArgs& a, int BH, hipStream_t stream);

@@ -1,0 +1,122 @@
+"""The chain kernels (state recurrence and H / dV in one launch) where they can go wrong: lengths around steps of 64 positions,
+chunks of 128 and windows of 256, each width of a workgroup and head dimension, every option of the operators, against the fp64
+oracle on the first and the last (batch, head) pair.  Tolerances are norm-relative as for the other kernels of these outputs: H
+6e-3, gradients 8e-3 (float16: a quarter), gate gradients 5e-2 of their scale, states 1e-3."""
+import ctypes
+
+import pytest
+import torch
+
+import oracle as O
+from helpers import rel_norm
+
+pytestmark = pytest.mark.gpu
+
+
+def _names():
+    from mlstm_kernels_amd import _lib
+
+    lib, out, i = _lib.get_lib(), set(), 0
+    while True:
+        name, ms, n = ctypes.create_string_buffer(64), ctypes.c_float(), ctypes.c_int()
+        if i >= lib.mlstm_hip_profile_read(i, name, 64, ctypes.byref(ms), ctypes.byref(n)):
+            return out
+        out.add(name.value.decode())
+        i += 1
+
+
+def _heads(DV, width):
+    """Heads for one workgroup of `width` value columns on (almost) every CU."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return cus // (DV // width)
+
+
+def _run(BH, S, DQ, DV, *, sig=False, normalize=True, init=False, last=False, dtype=torch.bfloat16, stride=2, f_offset=3.0, seed=0,
+         recompute=False):
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    print(f"{BH} x {S} {DQ}/{DV} sig={sig} normalize={normalize} init={init} last={last} {dtype} stride={stride}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    q, k, v, dH = (rn(1, BH, S, x).to(dtype) for x in (DQ, DQ, DV, DV))
+    i, f = rn(1, BH, S), f_offset + rn(1, BH, S)
+    c0 = n0 = m0 = dC = None
+    if init:
+        c0, n0, m0 = 0.1 * rn(1, BH, DQ, DV), 0.1 * rn(1, BH, DQ), 0.3 * rn(1, BH, 1)
+    if last:
+        dC = 0.1 * rn(1, BH, DQ, DV)
+    leaves = [t.requires_grad_(True) for t in (q, k, v, i, f)] + ([c0.requires_grad_(True)] if init else [])
+    kw = dict(c_initial=c0, n_initial=n0, return_last_states=last, any_sequence_length=True, chunk_size_intra=128 * stride,
+              recompute_states_in_bw=recompute)
+    lib = _lib.get_lib()
+    _names()
+    lib.mlstm_hip_profile_enable(1)
+    try:
+        if sig:
+            out = mlstm_siging_chunkwise__hip_xl_chunk(*leaves[:5], normalize=normalize, **kw)
+        else:
+            out = mlstm_chunkwise__hip_xl_chunk(*leaves[:5], m_initial=m0, **kw)
+        H, states = (out[0], out[1]) if last else (out, ())
+        grads = torch.autograd.grad([H] + ([states[0]] if last else []), leaves, [dH] + ([dC] if last else []))
+        torch.cuda.synchronize()
+    finally:
+        lib.mlstm_hip_profile_enable(0)
+    assert {"chain_h", "chain_dv"} <= _names()   # the kernels that this is about
+    tol = 0.25 if dtype == torch.float16 else 1.0
+    L = next(x for x in (64, 32, 16, 8, 4, 2, 1) if S % x == 0)
+    for h in (0, BH - 1):
+        d = lambda t: None if t is None else t.detach()[:, h:h + 1].double().cpu()
+        args = (d(q), d(k), d(v), d(i), d(f))
+        m0d = None if sig else d(m0)
+        o = dict(chunk_size=L, siging=sig, normalize=normalize)
+        fw = O.chunkwise_fw(*args, d(c0), d(n0), m0d, **o)
+        bw = O.chunkwise_bw(*args, d(dH), d(c0), d(n0), m0d, d(dC), **o)
+        assert rel_norm(d(H), fw["H"]) <= 6e-3 * tol
+        for name, x, ref in zip(("dQ", "dK", "dV", "dI", "dF", "dC0"), grads, bw):
+            if name in ("dI", "dF"):
+                assert float((d(x) - ref).abs().max()) <= 5e-2 * float(ref.abs().max()), name
+            else:
+                assert rel_norm(d(x), ref) <= 8e-3 * tol, name
+        if last:
+            assert rel_norm(d(states[0]), fw["C_last"]) <= 1e-3
+            if normalize:
+                assert rel_norm(d(states[1]), fw["n_last"]) <= 1e-3
+
+
+@pytest.mark.parametrize("DQ,DV,width", [(64, 128, 128), (64, 256, 256), (128, 128, 128), (128, 256, 256), (256, 256, 256), (256, 512, 256),
+                                         (256, 128, 128), (128, 384, 128)])
+@pytest.mark.parametrize("S", [257, 320, 321, 383, 450])
+def test_lengths(DQ, DV, width, S):
+    _run(_heads(DV, width), S, DQ, DV, seed=S)
+
+
+@pytest.mark.parametrize("DQ,DV,width", [(128, 128, 128), (256, 256, 256)])
+@pytest.mark.parametrize("S", [384, 449])
+@pytest.mark.parametrize("opt", [dict(init=True, last=True), dict(sig=True, init=True, last=True), dict(sig=True, normalize=False, init=True, last=True),
+                                 dict(dtype=torch.float16, init=True, last=True), dict(stride=1, last=True), dict(stride=3, init=True),
+                                 dict(f_offset=-4.0, last=True), dict(f_offset=9.0, init=True, last=True), dict(f_offset=9.0, dtype=torch.float16),
+                                 dict(recompute=True, init=True)],
+                         ids=["states", "sig", "sig-raw", "fp16", "stride1", "stride3", "forget", "keep", "fp16-keep", "recompute"])
+def test_options(DQ, DV, width, S, opt):
+    _run(_heads(DV, width), S, DQ, DV, seed=S + 1, **opt)
+
+
+def test_closed_gates():
+    """A forget gate that forgets everything (decay zero) and an input gate that stays shut for several steps."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    BH, S, DQ, DV = _heads(256, 256), 400, 128, 256
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    q, k, v = (rn(1, BH, S, x).bfloat16() for x in (DQ, DQ, DV))
+    i, f = rn(1, BH, S), 3 + rn(1, BH, S)
+    f[:, :, 130] = -200.0
+    i[:, :, 200:330] = -float("inf")
+    H, (C, n, m) = mlstm_chunkwise__hip_xl_chunk(q, k, v, i, f, return_last_states=True, any_sequence_length=True)
+    for h in (0, BH - 1):
+        d = lambda t: t[:, h:h + 1].double().cpu()
+        # (the recurrence itself: an infinite gate is a weight of zero there)
+        ref, (Cr, nr, mr) = O.recurrent_sequence(d(q), d(k), d(v), d(i), d(f), torch.zeros(1, 1, DQ, DV, dtype=torch.float64),
+                                                 torch.zeros(1, 1, DQ, dtype=torch.float64), torch.zeros(1, 1, 1, dtype=torch.float64))
+        assert rel_norm(d(H), ref) <= 6e-3 and rel_norm(d(C), Cr) <= 1e-3 and rel_norm(d(n), nr) <= 1e-3
