@@ -249,14 +249,41 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   if (workspace_bytes < ws.bytes) return failw("workspace too small");
   const int NC = (S + 127) / 128, BH = B * NH;
   const int sig = gate == MLSTM_GATE_SIG;
-  {
-    ProfileScope ps("gates", st);
-    if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, !has_c0, st)) return fail(e);
-  }
-  if (check_launch("gates")) return 1;
-
   const size_t c_bytes = (size_t)BH * DHQK * DHHV * sizeof(float), n_bytes = (size_t)BH * DHQK * sizeof(float);
   const bool track_n = !(sig && !normalize);  // the un-normalised sigmoid-gate variant leaves n untouched
+  // States updated where they lie: the short kernel's workgroups of H read all of the initial state while others of the same
+  // launch write the last one.  Scan + H take these calls: a state tile is read and written by the same waves, and H reads the
+  // kept chunk states only.
+  const bool in_place = overlap(c0, c_bytes, c_last, c_bytes) || overlap(n0, n_bytes, n_last, n_bytes) ||
+                        overlap(c0, c_bytes, n_last, n_bytes) || overlap(n0, n_bytes, c_last, c_bytes);
+  mlstm::ShortFwArgs sf;
+  memset(&sf, 0, sizeof(sf));
+  sf.Q = (const uint16_t*)q; sf.K = (const uint16_t*)k; sf.V = (const uint16_t*)v;
+  sf.g = ws.g;
+  sf.ig = i; sf.fg = f;
+  sf.m0 = m0;
+  sf.m_last = m_last;
+  sf.Out = (uint16_t*)H;
+  sf.n_out = n_out; sf.m_out = m_out;
+  sf.init = c0;
+  sf.n_init = n0;
+  sf.final_out = c_last;
+  sf.n_final = track_n ? n_last : nullptr;
+  sf.S = S; sf.NC = NC; sf.DHQK = DHQK; sf.DHHV = DHHV;
+  sf.qk_scale = 1.0f / sqrtf((float)DHQK); sf.eps = eps;
+  sf.sig_gate = sig;
+  sf.use_nrow = track_n;
+  sf.f16 = f16; sf.dtype_gates = dtype_gates;
+  const bool use_short = path == MLSTM_PATH_AUTO && !keep_for_backward && !in_place && head_norm == MLSTM_NORM_NONE &&
+                         (n_last == nullptr || c_last != nullptr) && mlstm::short_fw_preferred(sf, BH);
+  sf.own_gates = use_short && mlstm::short_fw_own_gates(sf, BH);
+  if (!sf.own_gates) {
+    {
+      ProfileScope ps("gates", st);
+      if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, !has_c0, st)) return fail(e);
+    }
+    if (check_launch("gates")) return 1;
+  }
   if (!track_n && n_last != nullptr && n_last != n0) {
     if (n0 != nullptr) {
       if (hipMemcpyAsync(n_last, n0, n_bytes, hipMemcpyDeviceToDevice, st) != hipSuccess)
@@ -297,35 +324,18 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     return check_launch("fused_hv forward");
   }
 
-  // States updated where they lie: the short kernel's workgroups of H read all of the initial state while others of the same
-  // launch write the last one.  Scan + H take these calls: a state tile is read and written by the same waves, and H reads the
-  // kept chunk states only.
-  const bool in_place = overlap(c0, c_bytes, c_last, c_bytes) || overlap(n0, n_bytes, n_last, n_bytes) ||
-                        overlap(c0, c_bytes, n_last, n_bytes) || overlap(n0, n_bytes, c_last, c_bytes);
-  if (path == MLSTM_PATH_AUTO && !keep_for_backward && !in_place && head_norm == MLSTM_NORM_NONE &&
-      (n_last == nullptr || c_last != nullptr)) {
-    mlstm::ShortFwArgs fa;
-    memset(&fa, 0, sizeof(fa));
-    fa.Q = (const uint16_t*)q; fa.K = (const uint16_t*)k; fa.V = (const uint16_t*)v;
-    fa.g = ws.g;
-    fa.Out = (uint16_t*)H;
-    fa.n_out = n_out; fa.m_out = m_out;
-    fa.init = c0;
-    fa.n_init = n0;
-    fa.final_out = c_last;
-    fa.n_final = track_n ? n_last : nullptr;
-    fa.S = S; fa.NC = NC; fa.DHQK = DHQK; fa.DHHV = DHHV;
-    fa.qk_scale = 1.0f / sqrtf((float)DHQK); fa.eps = eps;
-    fa.sig_gate = sig;
-    fa.use_nrow = track_n;
-    fa.f16 = f16;
-    if (mlstm::short_fw_preferred(fa, BH)) {
-      {
-        ProfileScope ps("short_fw", st);
-        if (const char* e = mlstm::launch_short_fw(fa, BH, st)) return fail(e);
-      }
-      return check_launch("short_fw");
+  if (use_short) {
+    if (sf.own_gates && overlap(m0, (size_t)BH * sizeof(float), m_last, (size_t)BH * sizeof(float))) {
+      // every workgroup of a head reads m0 and one writes m_last: read from a copy, in a part of the workspace that this path does not use
+      if (hipMemcpyAsync(ws.g.mstates, m0, (size_t)BH * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess)
+        return failw("copying m0 failed");
+      sf.m0 = ws.g.mstates;
     }
+    {
+      ProfileScope ps("short_fw", st);
+      if (const char* e = mlstm::launch_short_fw(sf, BH, st)) return fail(e);
+    }
+    return check_launch("short_fw");
   }
 
   if (path == MLSTM_PATH_AUTO && !in_place && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr)) {

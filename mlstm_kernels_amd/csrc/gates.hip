@@ -23,74 +23,14 @@
 // over ALL chunks of its head with one wave (the recurrence is associative and only NC scalars long, so every
 // workgroup of a head repeats it rather than waiting for a neighbour) and finishes its own chunks elementwise.
 #include "common.h"
+#include "gate_scan.h"
 #include "kernels.h"
 
 namespace mlstm {
 
 constexpr int kGateThreads = 1024;
 
-template <typename Op>
-__device__ __forceinline__ float wave_incl_scan(float x, Op op, float identity) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float y = __shfl_up(x, o);
-    x = lane >= o ? op(y, x) : x;
-  }
-  (void)identity;
-  return x;
-}
-template <typename Op>
-__device__ __forceinline__ float wave_rev_incl_scan(float x, Op op) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float y = __shfl_down(x, o);
-    x = lane + o < 64 ? op(y, x) : x;
-  }
-  return x;
-}
-
 constexpr int kGateChunks = kGateThreads / kWave;  // chunks per workgroup: one wave each
-
-// Within-chunk scans of one chunk by one wave, two positions per lane.
-struct ChunkScan {
-  float b[2], a[2], cm[2], w[2];  // b; a; b + cummax(it - b); b - it
-  float g, amax;                  // of the whole chunk
-};
-__device__ __forceinline__ ChunkScan scan_chunk(const void* ig, const void* fg, int bh, int c, int lane, int S,
-                                                int dtype_gates, int sig_gate) {
-  const float NEG_INF = -__builtin_inff();
-  auto add = [](float a, float b) { return a + b; };
-  auto mx = [](float a, float b) { return fmaxf(a, b); };
-  const int t0 = c * kChunk + 2 * lane;
-  float lf[2], it[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int t = t0 + e;
-    if (t < S) {
-      const size_t o = (size_t)bh * S + t;
-      lf[e] = log_sigmoid(load_scalar(fg, o, dtype_gates));
-      const float iv = load_scalar(ig, o, dtype_gates);
-      it[e] = sig_gate ? log_sigmoid(iv) : iv;
-    } else {
-      lf[e] = 0.f;
-      it[e] = NEG_INF;
-    }
-  }
-  const float pair = lf[0] + lf[1];
-  const float incl = wave_incl_scan(pair, add, 0.f);
-  const float b1 = incl, b0 = (incl - pair) + lf[0];
-  const float rincl = wave_rev_incl_scan(pair, add);
-  const float suf1 = rincl - pair, suf0 = suf1 + lf[1];
-  const float a0 = suf0 + it[0], a1 = suf1 + it[1];
-  const float x0 = it[0] - b0, x1 = it[1] - b1;
-  const float pm = wave_incl_scan(fmaxf(x0, x1), mx, NEG_INF);
-  float pm_excl = __shfl_up(pm, 1);
-  if (lane == 0) pm_excl = NEG_INF;
-  const float cm0 = fmaxf(pm_excl, x0), cm1 = pm;
-  return {{b0, b1}, {a0, a1}, {b0 + cm0, b1 + cm1}, {b0 - it[0], b1 - it[1]}, __shfl(incl, 63), wave_max(fmaxf(a0, a1))};
-}
 
 __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
     const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb, int S, int NC,
@@ -104,7 +44,7 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
   const int c = blockIdx.x * kGateChunks + wave;
   if (c >= NC) return;
   const size_t o = bh * ((size_t)NC * kChunk) + c * kChunk + 2 * lane;
-  const ChunkScan x = scan_chunk(ig, fg, bh, c, lane, S, dtype_gates, sig_gate);
+  const ChunkScan x = scan_chunk(load_gates(ig, fg, bh, c, lane, S, dtype_gates), c, lane, S, dtype_gates, sig_gate);
   *(float2*)(gb.u + o) = make_float2(x.b[0], x.b[1]);  // b, a and b + cummax(it - b) for the moment
   *(float2*)(gb.mcomb + o) = make_float2(x.cm[0], x.cm[1]);
   *(float2*)(gb.abar + o) = make_float2(x.a[0], x.a[1]);
@@ -127,7 +67,7 @@ __global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;  // one wave per chunk
   const float NEG_INF = -__builtin_inff();
   const float m_init = !sig_gate && m0 != nullptr ? m0[bh] : 0.f;
-  const ChunkScan x = scan_chunk(ig, fg, bh, c, lane, S, dtype_gates, sig_gate);
+  const ChunkScan x = scan_chunk(load_gates(ig, fg, bh, c, lane, S, dtype_gates), c, lane, S, dtype_gates, sig_gate);
   if (lane == 0) {
     gs[c] = x.g;
     as[c] = x.amax;
@@ -326,7 +266,7 @@ __global__ __launch_bounds__(kGateThreads) void gate_grads_kernel(GateGradArgs a
   }
   const float pair = d[0] + d[1];
   auto add = [](float x, float y) { return x + y; };
-  const float rincl = wave_rev_incl_scan(pair, add);  // sum over lanes >= lane
+  const float rincl = wave_rev_incl_scan(pair, add, 0.f);  // sum over lanes >= lane
   if (lane == 0) wtot[wave] = rincl;
   __syncthreads();
   for (int w = wave + 1; w < kGateThreads / kWave; ++w) after += wtot[w];

@@ -159,7 +159,11 @@ struct ChainHvArgs {
 constexpr int kShortMax = 512;  // longest sequence of the short forward
 struct ShortFwArgs {
   const uint16_t *Q, *K, *V;
+  int own_gates;            // the workgroups scan the gates themselves; otherwise the vectors of the pre-pass are in g
   GateBufs g;
+  const void *ig, *fg;      // own gates: (B,NH,S) pre-activations
+  const float* m0;          // own gates: (B,NH) or nullptr (zeros)
+  float* m_last;            // own gates: (B,NH) or nullptr; not m0
   uint16_t* Out;            // (B,NH,S,DHHV)
   float* n_out;             // optional (B,NH,S)
   float* m_out;             // optional (B,NH,S)
@@ -170,7 +174,7 @@ struct ShortFwArgs {
   int S, NC, DHQK, DHHV;
   float qk_scale, eps;
   int sig_gate, use_nrow;
-  int f16;
+  int f16, dtype_gates;
 };
 
 struct ParQkArgs {
@@ -232,6 +236,7 @@ bool window_hv_preferred(const ParHvArgs& a, int BH);  // supported, and faster 
 const char* launch_window_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 // forward without backward of a short sequence: H and the last state in one launch
 bool short_fw_preferred(const ShortFwArgs& a, int BH);
+bool short_fw_own_gates(const ShortFwArgs& a, int BH);
 const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream);
 const char* launch_head_norm_bw(const HeadNormBwArgs& a, hipStream_t stream);
 bool chain_hv_preferred(const ChainHvArgs& a, int BH);

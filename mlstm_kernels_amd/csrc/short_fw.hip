@@ -4,7 +4,7 @@
 //   P[t][j] = (q_t . k_j) / sqrt(DHQK) * exp(u_t - w_j + G)
 //   C_c     = gbar_c C_{c-1} + sum_{j in c} abar_j k_j v_j^T,   n_c = gbar_c n_{c-1} + sum_{j in c} abar_j k_j
 //
-// with the gate vectors of gates.hip (G: the decay of the chunks between those of j and t; cs_t: bbar_t / sqrt(DHQK), C0 decayed
+// with the gate vectors of gates.hip, which few workgroups make themselves (short_fw_own_gates; G: the decay of the chunks between those of j and t; cs_t: bbar_t / sqrt(DHQK), C0 decayed
 // over the chunks in front of t's).  Where the whole sequence is one
 // group of source chunks no chunk state is needed: H takes all keys as score blocks, and the last state is one product over all
 // positions.  Neither waits for the other, so ONE launch holds the workgroups of both:
@@ -22,8 +22,9 @@
 // take this in three launches (gates, a scan of up to four chunks that run twice, H from the chunk states), each with most of
 // the chip idle.  us for all launches, streaming kernels / gates and this, the same rows again and again: 8 heads of 256/512, 128
 // positions 27.5 / 11.8, 317 36.5 / 16.8, 512 36.5 / 27.9, 317 from a state 37.3 / 20.4; 16 heads of 128/256, 317 33.2 / 14.9.
-// Rows that no cache holds: 28.7 / 13.4, 39.3 / 19.0, 39.0 / 30.7; 36.2 / 18.0.
+// Rows that no cache holds: 28.7 / 13.4, 39.3 / 19.0, 39.0 / 30.7; 36.2 / 18.0.  (The gates in a launch of their own in all of these.)
 #include "common.h"
+#include "gate_scan.h"
 #include "kernels.h"
 
 namespace mlstm {
@@ -32,21 +33,23 @@ constexpr int kShortThreads = 512;
 
 template <int DQ, int CW, bool INIT>
 struct ShortLds {
-  // H: [Q rows, then (INIT: behind them) slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | INIT: n0, cs, decay]
+  // H: [Q rows, then (INIT: behind them) slabs of V | P | w | row sums, INIT: q . n0 | 1 / normaliser | OWN: b,
+  // b + cummax(it - b) of the positions, decay and largest weight of every chunk | INIT: n0, cs, decay]
   static constexpr int QS = DQ + 8, VS = CW + 32;
   static constexpr int NBT = INIT ? 2 : 4;  // slabs of V at a time
   static constexpr int kFront = INIT ? 64 * QS + NBT * 64 * VS : (64 * QS > NBT * 64 * VS ? 64 * QS : NBT * 64 * VS);
   static constexpr int RT = DQ % 128 == 0 ? 128 : 64, WT = CW;  // state tile
   static constexpr int XS = RT + 32, YS = WT + 32;
   static size_t bytes(int nt, bool with_c) {
-    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 9 * 64 * 4 + 64 * 4 + (INIT ? (DQ + 65) * 4 : 0);
-    // C: [K slab | head of V | remainder of V | abar | abar as an operand]
-    const size_t c = (size_t)64 * (XS + 2 * YS) * 2 + kShortMax * 4 + kShortMax * 3 * 2;
+    const size_t h = (size_t)kFront * 2 + (size_t)64 * (64 * nt + 8) * 2 + kShortMax * 4 + 9 * 64 * 4 + 3 * 64 * 4 + 8 * 4 + (INIT ? (DQ + 65) * 4 : 0);
+    // C: [K slab | head of V | remainder of V | abar | abar as an operand | OWN: decay, largest weight of every chunk]
+    const size_t c = (size_t)64 * (XS + 2 * YS) * 2 + kShortMax * 4 + kShortMax * 3 * 2 + 8 * 4;
     return with_c && c > h ? c : h;
   }
 };
 
-template <int DQ, int CW, int NSL, bool F16, bool INIT>
+// OWN: the workgroup scans the gates of its head (its waves a chunk each, while the rows are on their way).
+template <int DQ, int CW, int NSL, bool F16, bool INIT, bool OWN>
 __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned char* smem) {
   using L = ShortLds<DQ, CW, INIT>;
   constexpr int QS = L::QS, VS = L::VS;
@@ -65,7 +68,9 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   float* const wv = (float*)(Ps + 64 * PSS);
   float* const rows = wv + kShortMax;  // [8 waves][64], INIT: q . n0 [64]
   float* const inv = rows + 9 * 64;
-  float* const nv = inv + 64;    // INIT: n0
+  float* const bv = inv + 64;    // OWN: [2][64]
+  float* const gch = bv + 128;   // OWN: [2][4]
+  float* const nv = gch + 8;     // INIT: n0
   float* const csv = nv + DQ;    // INIT: cs_t, decay of the initial state up to this chunk
   const size_t Sp = (size_t)NC * kChunk, gofs = (size_t)bh * Sp;
   const uint16_t* const Qg = a.Q + (size_t)bh * S * DQ;
@@ -74,23 +79,29 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   const int n_kt = min(4 * tq + 4, (S + 15) / 16);  // tiles of 16 keys
   const int n_sl = tq + 1;                          // slabs of 64 keys
 
-  // ---- everything this workgroup needs is requested here
+  // ---- everything this workgroup needs is requested here, the gates of a chunk by each wave first
+  const int gc = min(wave, NC - 1);
+  RawGates raw;
+  if constexpr (OWN) raw = load_gates(a.ig, a.fg, bh, gc, lane, S, a.dtype_gates);
   u32x4 qr[QV];
 #pragma unroll
   for (int x = 0; x < QV; ++x) {
     const int idx = tid + x * kShortThreads, row = idx / (DQ / 8), u = idx % (DQ / 8);
     qr[x] = *(const u32x4*)(Qg + (size_t)min(t0 + row, S - 1) * DQ + u * 8);
   }
-  // (the gate vectors cover whole chunks: positions past the end have w = infinity, a factor of zero)
-  const float w_own = a.g.w[gofs + min(tid, (int)Sp - 1)];
   const int l16 = lane & 15, lq = lane >> 4;
-  float un[4];
+  // (the gate vectors cover whole chunks: positions past the end have w = infinity, a factor of zero)
+  float w_own = 0.f, mc = 0.f, m_init = 0.f, un[4], gr[kShortMax / kChunk];
+  if constexpr (OWN) {
+    if (!a.sig_gate && a.m0 != nullptr) m_init = a.m0[bh];
+  } else {
+    w_own = a.g.w[gofs + min(tid, (int)Sp - 1)];
 #pragma unroll
-  for (int tc = 0; tc < 4; ++tc) un[tc] = a.g.u[gofs + t0 + 16 * tc + l16];
-  const float mc = a.g.mcomb[gofs + t0 + (tid & 63)];
-  float gr[kShortMax / kChunk];
+    for (int tc = 0; tc < 4; ++tc) un[tc] = a.g.u[gofs + t0 + 16 * tc + l16];
+    mc = a.g.mcomb[gofs + t0 + (tid & 63)];
 #pragma unroll
-  for (int y = 0; y < kShortMax / kChunk; ++y) gr[y] = a.g.graw[(size_t)bh * NC + min(y, NC - 1)];
+    for (int y = 0; y < kShortMax / kChunk; ++y) gr[y] = a.g.graw[(size_t)bh * NC + min(y, NC - 1)];
+  }
   __syncthreads();
   // unit x of a wave: tiles wave + 16 y and wave + 16 y + 8 (y = x / NGK), operands NF (x % NGK) .. of their rows
   Frag k0[2][NF], k1[2][NF];
@@ -106,20 +117,33 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   };
   fetch(k0, 0);
 
+  if constexpr (OWN) {  // the scans of a chunk by each wave, while the rows are on their way
+    const ChunkScan cs = scan_chunk(raw, gc, lane, S, a.dtype_gates, a.sig_gate);
+    if (wave < NC) {
+      *(float2*)(wv + kChunk * wave + 2 * lane) = make_float2(cs.w[0], cs.w[1]);
+      if (wave == c && lane / 32 == tq % 2) {
+        *(float2*)(bv + 2 * r) = make_float2(cs.b[0], cs.b[1]);
+        *(float2*)(bv + 64 + 2 * r) = make_float2(cs.cm[0], cs.cm[1]);
+      }
+      if (lane == 0) gch[wave] = cs.g, gch[4 + wave] = cs.amax;
+    }
+  }
 #pragma unroll
   for (int x = 0; x < QV; ++x) {
     const int idx = tid + x * kShortThreads, row = idx / (DQ / 8), u = idx % (DQ / 8);
     *(u32x4*)(Qs + row * QS + u * 8) = qr[x];
   }
-  wv[tid] = w_own;
+  if constexpr (!OWN) wv[tid] = w_own;
   if constexpr (INIT) {
     if (tid < DQ) nv[tid] = a.use_nrow ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
-    if (tid < 64) csv[tid] = a.g.bbar[gofs + t0 + tid] * a.qk_scale;
-    if (tid == 64) {
-      float gsum = 0.f;
-      for (int y = 0; y < c; ++y) gsum += a.g.graw[(size_t)bh * NC + y];
-      const float* const mst = a.g.mstates + (size_t)bh * (NC + 1);
-      csv[64] = c > 0 ? __expf(gsum + mst[0] - mst[c]) : 1.f;
+    if constexpr (!OWN) {
+      if (tid < 64) csv[tid] = a.g.bbar[gofs + t0 + tid] * a.qk_scale;
+      if (tid == 64) {
+        float gsum = 0.f;
+        for (int y = 0; y < c; ++y) gsum += a.g.graw[(size_t)bh * NC + y];
+        const float* const mst = a.g.mstates + (size_t)bh * (NC + 1);
+        csv[64] = c > 0 ? __expf(gsum + mst[0] - mst[c]) : 1.f;
+      }
     }
   }
   __syncthreads();
@@ -132,11 +156,32 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
       vr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
     }
 
+  float mp = 0.f;  // OWN: m before this chunk
+  auto m_at = [&](int t) { return a.sig_gate ? 0.f : fmaxf(bv[t] + mp, bv[64 + t]); };
+  if constexpr (OWN) {
+#pragma unroll
+    for (int y = 0; y < kShortMax / kChunk; ++y) gr[y] = gch[y];  // (those of chunks past the end are not used)
+    if (!a.sig_gate) mp = m_before(c, m_init, gch, gch + 4);
+#pragma unroll
+    for (int tc = 0; tc < 4; ++tc) un[tc] = bv[16 * tc + l16] - m_at(16 * tc + l16);
+    mc = m_at(lane);
+    if (a.m_last != nullptr && g == 0 && tq == nt - 1 && tid == 0) a.m_last[bh] = a.sig_gate ? 0.f : fmaxf(mp + gch[c], gch[4 + c]);
+  }
+
   // The state takes its decay up to this chunk in fp32, in front of its rounding: one beyond the range of float16 that has decayed
   // into it is finite where it is seen there.
   float pre = 1.f;
   if constexpr (INIT) {
-    pre = csv[64];
+    auto cs_at = [&](int t) { return OWN ? expf(bv[t] + mp - m_at(t)) * a.qk_scale : csv[t]; };
+    if constexpr (OWN) {
+      float gsum = 0.f;
+#pragma unroll
+      for (int y = 0; y < kShortMax / kChunk; ++y) gsum += y < c ? gr[y] : 0.f;
+      if (c > 0) pre = __expf(gsum + (a.sig_gate ? 0.f : m_before(0, m_init, gch, gch + 4)) - mp);
+      if (tid < 64) csv[tid] = cs_at(tid);
+    } else {
+      pre = csv[64];
+    }
     // q_t . n0, eight threads per position
     const int t = tid >> 3, part = tid & 7;
     float dot = 0.f;
@@ -149,7 +194,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
     dot += __shfl_xor(dot, 1);
     dot += __shfl_xor(dot, 2);
     dot += __shfl_xor(dot, 4);
-    if (part == 0) rows[8 * 64 + t] = csv[t] * pre * dot;
+    if (part == 0) rows[8 * 64 + t] = cs_at(t) * pre * dot;
   }
   // ---- scores of this wave's tiles, gated into P
   {
@@ -332,7 +377,7 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
   }
 }
 
-template <int DQ, int CW, int NSL, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT, bool OWN>
 __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned char* smem) {
   using L = ShortLds<DQ, CW, INIT>;
   constexpr int RT = L::RT, WT = L::WT, XS = L::XS, YS = L::YS;
@@ -350,27 +395,35 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
   uint16_t* const Yl = Yh + 64 * YS;
   float* const wt = (float*)(Yl + 64 * YS);
   uint16_t* const nB = (uint16_t*)(wt + kShortMax);  // [position / 8][3][8]
-  const size_t Sp = (size_t)NC * kChunk;
+  float* const gch = (float*)(nB + kShortMax * 3);   // OWN: [2][4]
   const uint16_t* const Kg = a.K + (size_t)bh * S * DQ + bx * RT;
   const uint16_t* const Vg = a.V + (size_t)bh * S * DHHV + by * WT;
   const int n_sl = (S + 63) / 64;
-  {
-    // (the decay of later chunks is left to the sums: the largest weight of a chunk is one, and one times v has no remainder)
-    const float ab = a.g.abar[(size_t)bh * Sp + min(tid, (int)Sp - 1)];
-    const float w = tid < S ? ab : 0.f;
-    wt[tid] = w;
+  auto weight = [&](int t, float w) {
+    wt[t] = w;
     // n as in the scan: the weights, split exactly into three 16-bit parts, are three columns of one more operand
-    uint16_t* const dst = nB + (tid >> 3) * 24 + (tid & 7);
+    uint16_t* const dst = nB + (t >> 3) * 24 + (t & 7);
     const uint16_t p0 = f32_to_elem<F16>(w);
     const float r1 = w - elem_to_f32<F16>(p0);
     const uint16_t p1 = f32_to_elem<F16>(r1);
     dst[0] = p0;
     dst[8] = p1;
     dst[16] = f32_to_elem<F16>(r1 - elem_to_f32<F16>(p1));
-  }
+  };
+  // (the decay of later chunks is left to the sums: the largest weight of a chunk is one, and one times v has no remainder)
   float gb[kShortMax / kChunk];
+  const int gc = min(wave, NC - 1);
+  RawGates raw;
+  float m_init = 0.f;
+  if constexpr (OWN) {
+    raw = load_gates(a.ig, a.fg, bh, gc, lane, S, a.dtype_gates);
+    if (!a.sig_gate && a.m0 != nullptr) m_init = a.m0[bh];
+  } else {
+    const float ab = a.g.abar[(size_t)bh * NC * kChunk + min(tid, NC * kChunk - 1)];
+    weight(tid, tid < S ? ab : 0.f);
 #pragma unroll
-  for (int y = 0; y < kShortMax / kChunk; ++y) gb[y] = a.g.gbar[(size_t)bh * NC + min(y, NC - 1)];
+    for (int y = 0; y < kShortMax / kChunk; ++y) gb[y] = a.g.gbar[(size_t)bh * NC + min(y, NC - 1)];
+  }
   u32x4 xr[NSL][XV], yr[NSL][YV];
 #pragma unroll
   for (int s = 0; s < NSL; ++s) {
@@ -383,6 +436,27 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
     for (int x = 0; x < YV; ++x) {
       const int idx = tid + x * kShortThreads, row = idx / (WT / 8), u = idx % (WT / 8);
       yr[s][x] = *(const u32x4*)(Vg + (size_t)min(64 * s + row, S - 1) * DHHV + u * 8);
+    }
+  }
+  if constexpr (OWN) {  // the scans of a chunk by each wave, while the rows are on their way
+    const ChunkScan cs = scan_chunk(raw, gc, lane, S, a.dtype_gates, a.sig_gate);
+    if (lane == 0 && wave < NC) gch[wave] = cs.g, gch[4 + wave] = cs.amax;
+    __syncthreads();
+#pragma unroll
+    for (int y = 0; y < kShortMax / kChunk; ++y) {
+      gb[y] = 1.f;
+      if (y < NC) {
+        const float mp = a.sig_gate ? 0.f : m_before(y, m_init, gch, gch + 4);
+        const float mn = a.sig_gate ? 0.f : fmaxf(mp + gch[y], gch[4 + y]);
+        gb[y] = expf(gch[y] + mp - mn);
+        if (wave == y) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int t = kChunk * y + 2 * lane + e;
+            weight(t, t < S ? expf(cs.a[e] - mn) : 0.f);
+          }
+        }
+      }
     }
   }
   const int rb = wave % NRB, cb0 = wave / NRB * NBW;
@@ -495,7 +569,7 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
 
 }  // namespace
 
-template <int DQ, int CW, int NSL, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT, bool OWN>
 __global__ __launch_bounds__(kShortThreads) void short_fw_kernel(ShortFwArgs a, int n_h, int n_c) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   // consecutive items (of one head) share an XCD and the head's rows in its L2
@@ -504,12 +578,12 @@ __global__ __launch_bounds__(kShortThreads) void short_fw_kernel(ShortFwArgs a, 
   if (!is_h) b -= n_h;
   const int n = is_h ? n_h : n_c;
   if (n_h % 8 == 0 && n % 8 == 0) b = (b % 8) * (n / 8) + b / 8;
-  if (is_h) short_h<DQ, CW, NSL, F16, INIT>(a, b, smem_raw);
-  else short_c<DQ, CW, NSL, F16, INIT>(a, b, smem_raw);
+  if (is_h) short_h<DQ, CW, NSL, F16, INIT, OWN>(a, b, smem_raw);
+  else short_c<DQ, CW, NSL, F16, INIT, OWN>(a, b, smem_raw);
 }
 
 namespace {
-template <int DQ, int CW, int NSL, bool F16, bool INIT>
+template <int DQ, int CW, int NSL, bool F16, bool INIT, bool OWN>
 const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
   using L = ShortLds<DQ, CW, INIT>;
   const int nt = (a.S + 63) / 64;
@@ -519,18 +593,22 @@ const char* launch_short_t(const ShortFwArgs& a, int BH, hipStream_t stream) {
   const size_t smem = L::bytes(nt, n_c > 0);
   if (smem > 160 * 1024) return "short_fw: too long for one CU's LDS";
   static LdsLimit lds;
-  if (!lds.allow((const void*)short_fw_kernel<DQ, CW, NSL, F16, INIT>, smem)) return "short_fw: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((short_fw_kernel<DQ, CW, NSL, F16, INIT>), dim3((unsigned)(n_h + n_c)), dim3(kShortThreads), smem, stream, a, (int)n_h, (int)n_c);
+  if (!lds.allow((const void*)short_fw_kernel<DQ, CW, NSL, F16, INIT, OWN>, smem)) return "short_fw: cannot raise the dynamic LDS limit";
+  hipLaunchKernelGGL((short_fw_kernel<DQ, CW, NSL, F16, INIT, OWN>), dim3((unsigned)(n_h + n_c)), dim3(kShortThreads), smem, stream, a, (int)n_h, (int)n_c);
   return nullptr;
+}
+template <int DQ, int CW, int NSL, bool F16, bool INIT>
+const char* launch_short_g(const ShortFwArgs& a, int BH, hipStream_t stream) {
+  return a.own_gates ? launch_short_t<DQ, CW, NSL, F16, INIT, true>(a, BH, stream) : launch_short_t<DQ, CW, NSL, F16, INIT, false>(a, BH, stream);
 }
 template <int DQ, int CW, int NSL>
 const char* launch_short_c(const ShortFwArgs& a, int BH, hipStream_t stream) {
   if (a.init != nullptr) {
     // (the Q rows of 512 beside the V slabs and more than five score tiles do not fit the LDS: no instance)
     if constexpr (DQ == 512 && NSL > 5) return "short_fw: too long for one CU's LDS";
-    else return a.f16 ? launch_short_t<DQ, CW, NSL, true, true>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, true>(a, BH, stream);
+    else return a.f16 ? launch_short_g<DQ, CW, NSL, true, true>(a, BH, stream) : launch_short_g<DQ, CW, NSL, false, true>(a, BH, stream);
   }
-  return a.f16 ? launch_short_t<DQ, CW, NSL, true, false>(a, BH, stream) : launch_short_t<DQ, CW, NSL, false, false>(a, BH, stream);
+  return a.f16 ? launch_short_g<DQ, CW, NSL, true, false>(a, BH, stream) : launch_short_g<DQ, CW, NSL, false, false>(a, BH, stream);
 }
 template <int DQ, int CW>
 const char* launch_short_s(const ShortFwArgs& a, int BH, hipStream_t stream) {
@@ -576,6 +654,17 @@ bool short_fw_preferred(const ShortFwArgs& a, int BH) {
   cost = cost * (a.DHQK < 256 ? a.DHQK : 256) / (wide ? 256 : 512);
   const bool streaming = a.DHQK == 256 && a.DHHV % 512 == 0;
   return cost <= (nt == 1 ? (streaming ? 18ll : 24ll) : (streaming ? 7ll : 12ll)) * device_cu_count();
+}
+
+// Whether its workgroups scan the gates themselves: each repeats the scans of its head, about a microsecond while its rows are on
+// their way, and the launch in front (4 us) is left out.  The line is at three workgroups a CU.  us, with the pre-pass / without, bf16:
+// 8 heads of 256/512, 64 positions 14.0 / 11.0 (of which the host takes all), 317 17.5 / 13.5, 512 28.5 / 26.4, 317 from a state
+// 20.6 / 16.4; 16 heads of 317 26.0 / 24.0 (1.75 workgroups a CU), 32 of 64 15.1 / 13.8 (1.5), 128 heads of 128/256 of 100 positions 22.1 /
+// 21.8 (3.0), 32 of 317 42.1 / 41.9 (3.5), 64 of 200 55.4 / 58.0 (6.0), 512 of 64 124.7 / 153.3 (24).
+bool short_fw_own_gates(const ShortFwArgs& a, int BH) {
+  const long long cw = a.DHHV % 128 == 0 ? 128 : 64, rt = a.DHQK % 128 == 0 ? 128 : 64;
+  const long long tiles = (a.S + 63) / 64 + (a.final_out == nullptr ? 0 : a.DHQK / rt);
+  return BH * tiles * (a.DHHV / cw) <= 3ll * device_cu_count();
 }
 
 const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream) {

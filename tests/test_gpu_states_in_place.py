@@ -43,6 +43,14 @@ def test_short_sequences(S, DQ, DV, sig, noalloc):
         assert torch.equal(a, b), name
 
 
+# m alone in place: the workgroups of the short kernel all read m0 and one writes m_last
+@pytest.mark.parametrize("S", [50, 300, 512])
+def test_short_sequences_stabiliser_only(S):
+    got, ref = (_forward(S, 128, 128, in_place=p, seed=S, share="m") for p in (True, False))
+    for name, a, b in zip(("H", "C", "n", "m"), got, ref):
+        assert torch.equal(a, b), name
+
+
 # the path of one kernel, whose workgroups of a head all read n0; and n that the operator leaves as it is: the same bits
 @pytest.mark.parametrize("path,sig,normalize", [("fused", False, 1), ("fused", True, 0), ("auto", True, 0), ("split", False, 1)])
 def test_named_paths(path, sig, normalize):

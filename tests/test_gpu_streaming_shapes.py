@@ -312,6 +312,61 @@ def test_forward_with_and_without_a_gradient(S, DQ, DV, path, last):
         assert torch.equal(a, b) if path == "split" else rel_norm(a, b) <= tol
 
 
+# The short kernel scans the gates itself: 16-bit gates are the same numbers as those of 32 bits, so every bit is the same.  Gates in
+# memory that is aligned to one element only.
+@pytest.mark.parametrize("S", [1, 127, 128, 129, 257, 385, 512])
+@pytest.mark.parametrize("gates", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sig", [False, True])
+def test_short_prompts_gate_types(S, gates, sig):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(1, 3, S, 64, 128, seed=S, f_offset=3.0))
+    i, f = i.to(gates), f.to(gates)
+    moved = [torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape) for t in (i, f)]
+    out = []
+    for x in ((i.float(), f.float()), (i, f), moved):
+        with torch.no_grad():
+            H, state = op(q, k, v, *x, return_last_states=True, any_sequence_length=True)
+        out.append((H, *state[:2], *([] if sig else state[2:])))
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert torch.equal(a, b)
+
+
+# Few workgroups scan the gates themselves, many take them from the pre-pass: the same numbers, so that a head's bits do not depend on
+# how many there are (the rule is at three workgroups a CU: more than 768 for all heads here, fewer for two of them).
+@pytest.mark.parametrize("S,DQ,DV,NH", [(17, 64, 128, 512), (64, 128, 192, 300), (65, 64, 64, 300), (128, 256, 64, 260), (129, 64, 64, 400),
+                                        (200, 128, 256, 128), (320, 64, 64, 160)])
+@pytest.mark.parametrize("opt", [dict(), dict(init=True), dict(sig=True, init=True), dict(dtype=torch.float16)], ids=str)
+def test_short_prompts_gates_of_the_pre_pass(S, DQ, DV, NH, opt):
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    init, sig, dtype = opt.get("init", False), opt.get("sig", False), opt.get("dtype", torch.bfloat16)
+    if init:
+        NH = {200: 80, 320: 112, 129: 272}.get(S, NH)  # (as many as take one launch from a state)
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *d: torch.randn(1, NH, *d, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), 3 + rn(S)]
+    state = [rn(DQ, DV), rn(DQ), None if sig else rn(1)] if init else [None] * 3
+    _lib.profile_read()
+    _lib.profile_enable(True)
+    try:
+        with torch.no_grad():
+            H, last = op(*x, *state, return_last_states=True, any_sequence_length=True)
+    finally:
+        _lib.profile_enable(False)
+    if S != 320 or not init:
+        assert {"gates", "short_fw"} <= set(_lib.profile_read())
+    cut = lambda t: None if t is None else t[:, NH - 2:].contiguous()
+    with torch.no_grad():
+        H2, last2 = op(*(cut(t) for t in x), *(cut(t) for t in state), return_last_states=True, any_sequence_length=True)
+    for a, b in zip((H, *last), (H2, *last2)):
+        assert torch.equal(cut(a), b)
+
+
 # Up to 128 positions many heads take scan + H as well: the most heads that the short kernel takes, and one more.
 @pytest.mark.parametrize("S,DQ,DV,init,most", [(128, 256, 512, False, 112), (65, 256, 512, True, 56), (64, 256, 512, True, 384),
                                                (100, 128, 256, False, 768), (128, 64, 192, True, 1024)])
