@@ -138,6 +138,19 @@ __device__ __forceinline__ float log_sigmoid(float x) {
   return fminf(x, 0.f) - log1pf(expf(-fabsf(x)));
 }
 
+// To memory at once, through the caches of the device (a store of device scope; the L2 line stays readable and is clean).  base, bytes:
+// the buffer, the same for all lanes.
+__device__ __forceinline__ void store_write_through(void* base, uint32_t bytes, uint32_t ofs, u32x4 x) {
+  __builtin_amdgcn_raw_buffer_store_b128(x, __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000), ofs, 0, 16);
+}
+__device__ __forceinline__ void store_write_through(void* base, uint32_t bytes, uint32_t ofs, uint32_t x) {
+  __builtin_amdgcn_raw_buffer_store_b32(x, __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000), ofs, 0, 16);
+}
+template <typename T>  // (4 or 8 bytes)
+__device__ __forceinline__ void store_write_through(T* dst, T x) {
+  __hip_atomic_store(dst, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // dtype: 0 float32, 1 bfloat16, 2 float16
 __device__ __forceinline__ float load_scalar(const void* p, size_t idx, int dtype) {
   if (dtype == 0) return ((const float*)p)[idx];

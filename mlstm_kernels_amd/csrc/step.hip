@@ -41,29 +41,35 @@ __device__ __forceinline__ StatePiece<SBF> load_piece(const void* base, size_t e
   }
   return p;
 }
-template <int SBF, bool NT>
-__device__ __forceinline__ void store_piece(void* base, size_t elem, const StatePiece<SBF>& p) {
+// How a state is stored.  Plain: it stays in the L2s, which hand what they still hold to memory when the launch ends and the next one
+// waits.  Write-through (device scope): on its way to memory at once, the lines stay readable.  Non-temporal: past the caches.
+enum StoreMode { kPlain, kNonTemporal, kWriteThrough };
+template <int MODE>
+__device__ __forceinline__ void store16(void* head, uint32_t head_bytes, size_t ofs, u32x4 raw) {
+  if constexpr (MODE == kNonTemporal) __builtin_nontemporal_store(raw, (u32x4*)((char*)head + ofs));
+  else if constexpr (MODE == kWriteThrough) store_write_through(head, head_bytes, (uint32_t)ofs, raw);
+  else *(u32x4*)((char*)head + ofs) = raw;
+}
+// (head: the state of the (batch, head), the same for all lanes)
+template <int SBF, int MODE>
+__device__ __forceinline__ void store_piece(void* head, uint32_t head_bytes, size_t elem, const StatePiece<SBF>& p) {
   if constexpr (SBF != 0) {
     const u32x4 raw = {pack_state2(p.x[0], p.x[1], SBF), pack_state2(p.x[2], p.x[3], SBF), pack_state2(p.x[4], p.x[5], SBF),
                        pack_state2(p.x[6], p.x[7], SBF)};
-    u32x4* dst = (u32x4*)((uint16_t*)base + elem);
-    if (NT) __builtin_nontemporal_store(raw, dst);
-    else *dst = raw;
+    store16<MODE>(head, head_bytes, elem * 2, raw);
   } else {
-    const f32x4 raw = {p.x[0], p.x[1], p.x[2], p.x[3]};
-    f32x4* dst = (f32x4*)((float*)base + elem);
-    if (NT) __builtin_nontemporal_store(raw, dst);
-    else *dst = raw;
+    store16<MODE>(head, head_bytes, elem * 4, u32x4{__float_as_uint(p.x[0]), __float_as_uint(p.x[1]), __float_as_uint(p.x[2]), __float_as_uint(p.x[3])});
   }
 }
 
-template <int COLS, int TY, int UNROLL, bool NONTEMPORAL, int SBF>
+template <int COLS, int TY, int UNROLL, int MODE, int SBF>
 __global__ __launch_bounds__((COLS / StatePiece<SBF>::N) * TY) void step_kernel(
     const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     const void* __restrict__ ig, const void* __restrict__ fg,
     const void* c_in, const void* n_in, const void* m_in,
     void* __restrict__ h, void* c_out, void* n_out, void* m_out,
     int DHQK, int DHHV, float eps, int dtype_qkv, int dtype_gates) {
+  constexpr bool NONTEMPORAL = MODE == kNonTemporal;
   constexpr int VPL = StatePiece<SBF>::N;   // state columns per lane
   constexpr int TX = COLS / VPL;
   constexpr int NTH = TX * TY;
@@ -85,6 +91,8 @@ __global__ __launch_bounds__((COLS / StatePiece<SBF>::N) * TY) void step_kernel(
   const int col = col0 + VPL * tx;
   const bool col_ok = col < DHHV;  // DHHV % VPL == 0 is checked on the host
   const size_t cbase = (size_t)bh * DHQK * DHHV + col;
+  void* const c_head = (char*)c_out + (size_t)bh * DHQK * DHHV * (SBF ? 2 : 4);
+  const uint32_t c_bytes = (uint32_t)DHQK * DHHV * (SBF ? 2 : 4);  // (write-through: below 2^32 by the rule of launch_step)
   const bool have_first = !NONTEMPORAL && col_ok && ty + (UNROLL - 1) * TY < DHQK;
   StatePiece<SBF> cfirst[UNROLL];
 #pragma unroll
@@ -169,7 +177,7 @@ __global__ __launch_bounds__((COLS / StatePiece<SBF>::N) * TY) void step_kernel(
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const int rr = r + u * TY;
-        store_piece<SBF, false>(c_out, cbase + (size_t)rr * DHHV, update(cfirst[u], rr));
+        store_piece<SBF, MODE>(c_head, c_bytes, (size_t)rr * DHHV + col, update(cfirst[u], rr));
       }
       r += UNROLL * TY;
     }
@@ -180,12 +188,12 @@ __global__ __launch_bounds__((COLS / StatePiece<SBF>::N) * TY) void step_kernel(
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const int rr = r + u * TY;
-        store_piece<SBF, NONTEMPORAL>(c_out, cbase + (size_t)rr * DHHV, update(c[u], rr));
+        store_piece<SBF, MODE>(c_head, c_bytes, (size_t)rr * DHHV + col, update(c[u], rr));
       }
     }
     for (; r < DHQK; r += TY) {
       const StatePiece<SBF> c = load_piece<SBF, false>(c_in, cbase + (size_t)r * DHHV);
-      store_piece<SBF, false>(c_out, cbase + (size_t)r * DHHV, update(c, r));
+      store_piece<SBF, NONTEMPORAL ? kPlain : MODE>(c_head, c_bytes, (size_t)r * DHHV + col, update(c, r));
     }
   }
 #pragma unroll
@@ -203,7 +211,7 @@ __global__ __launch_bounds__((COLS / StatePiece<SBF>::N) * TY) void step_kernel(
   }
 }
 
-template <int COLS, int TY, int UNROLL, bool NONTEMPORAL, int SBF>
+template <int COLS, int TY, int UNROLL, int MODE, int SBF>
 static const char* launch_step_t(const void* q, const void* k, const void* v, const void* i, const void* f,
                                  const void* c_in, const void* n_in, const void* m_in, void* h, void* c_out,
                                  void* n_out, void* m_out, int B, int NH, int DHQK, int DHHV, float eps,
@@ -211,7 +219,7 @@ static const char* launch_step_t(const void* q, const void* k, const void* v, co
   const size_t smem = (size_t)(2 * DHQK + TY * COLS) * sizeof(float);
   if (smem > 64 * 1024) return "mlstm_hip_step: DHQK too large for the LDS staging";
   dim3 grid((DHHV + COLS - 1) / COLS, B * NH);
-  hipLaunchKernelGGL((step_kernel<COLS, TY, UNROLL, NONTEMPORAL, SBF>), grid, dim3((COLS / StatePiece<SBF>::N) * TY), smem,
+  hipLaunchKernelGGL((step_kernel<COLS, TY, UNROLL, MODE, SBF>), grid, dim3((COLS / StatePiece<SBF>::N) * TY), smem,
                      stream, q, k, v, i, f, c_in, n_in, m_in, h, c_out, n_out, m_out, DHQK, DHHV, eps, dtype_qkv,
                      dtype_gates);
   return nullptr;
@@ -242,9 +250,28 @@ const char* launch_step(const void* q, const void* k, const void* v, const void*
     if (dtype_state == 2) return launch_step_t<COLS_, TY_, UN_, NT_, 2>(MLSTM_STEP_ARGS);               \
     return launch_step_t<COLS_, TY_, UN_, NT_, 0>(MLSTM_STEP_ARGS);                                      \
   }
-  if (DHHV % 256 == 0 && stream_past_cache) MLSTM_STEP_PICK(256, 8, 16, true)
-  if (stream_past_cache) MLSTM_STEP_PICK(128, 8, 8, true)
-  MLSTM_STEP_PICK(128, 16, 16, false)
+  if (DHHV % 256 == 0 && stream_past_cache) MLSTM_STEP_PICK(256, 8, 16, kNonTemporal)
+  if (stream_past_cache) MLSTM_STEP_PICK(128, 8, 8, kNonTemporal)
+  // Below it, the first batch is as many rows as every row group has, up to 16: what is left over is read one row after the other.
+  // us, 16 rows at a time / so (128/256 heads, inputs and state new to the caches): 16 x 16 heads 13.9 / 13.3, 64 x 16 60.2 / 53.3, 100 x 16
+  // 100.5 / 86.3, with 16-bit states 64 x 16 42.5 / 29.7; 64/64, 512 x 4 26.5 / 20.7.
+  // Write-through where many workgroups of up to 64 KB follow one another on a CU, and the memory-side cache holds the old state beside
+  // the new one: us, plain / write-through, the state of one call the next one's input: 128/256, 32 x 16 heads (64 MB) 24.4 / 22.9;
+  // 64/128, 128 x 8 (32 MB) 17.1 / 15.1, 400 x 8 42.0 / 37.9; 16-bit states, 256/512 32 x 8 (64 MB) 28.9 / 27.6, 128/256 64 x 16 26.7 / 24.2.
+  // Where a single round of workgroups fills the chip the stores wait for it: with 32 MB or less (128/256, 16 x 16, in place 10.1 / 12.4),
+  // 12 MB where a workgroup has 32 KB (64/128, 32 x 8 5.8 / 6.3), and with slices of 128 KB (256/512, 16 x 8 20.6 / 23.0).  With more than
+  // the cache holds it is memory either way (128/256, 64 x 16, other states in between 53.3 / 57.3).
+  const size_t slice_bytes = (size_t)128 * (DHQK < 256 ? DHQK : 256) * (sbf ? 2 : 4);
+  const bool through = slice_bytes <= 65536 && state_bytes > ((size_t)(slice_bytes <= 32768 ? 12 : 32) << 20) && state_bytes <= ((size_t)112 << 20);
+#define MLSTM_STEP_ROWS(MODE_)                                       \
+  {                                                                  \
+    if (DHQK >= 256) MLSTM_STEP_PICK(128, 16, 16, MODE_)             \
+    if (DHQK >= 128) MLSTM_STEP_PICK(128, 16, 8, MODE_)              \
+    MLSTM_STEP_PICK(128, 16, 4, MODE_)                               \
+  }
+  if (through) MLSTM_STEP_ROWS(kWriteThrough)
+  MLSTM_STEP_ROWS(kPlain)
+#undef MLSTM_STEP_ROWS
 #undef MLSTM_STEP_PICK
 #undef MLSTM_STEP_ARGS
 }
