@@ -96,8 +96,8 @@ __device__ __forceinline__ float lane_value(float x, int l) { return __int_as_fl
 }  // namespace
 
 // F16: q, k, v and h are float16 instead of bfloat16; SDT: state type (0 fp32, 1 bf16, 2 fp16); MODE: 1 up to 16
-// tokens, 2 up to 32, 3 more (several blocks).  rows: tokens of the largest block
-template <bool F16, int SDT, int MODE>
+// tokens, 2 up to 32, 3 more (several blocks); THROUGH: the state is written through the caches.  rows: tokens of the largest block
+template <bool F16, int SDT, int MODE, bool THROUGH>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void step_block_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const void* __restrict__ ig,
     const void* __restrict__ fg, const void* c_in, const void* n_in, const void* m_in, uint16_t* __restrict__ h, void* c_out,
@@ -496,31 +496,49 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const size_t o = c_base + (size_t)(32 * b + 8 * (i / 4) + (i % 4)) * DHHV;
-      if constexpr (SDT == 0) *(float2*)((float*)c_out + o + c_lane) = make_float2(C[b][0][i], C[b][1][i]);
-      else *(uint32_t*)((uint16_t*)c_out + o + c_lane) = pack_state2(C[b][0][i], C[b][1][i], SDT);
+      if constexpr (SDT == 0) {
+        float* const dst = (float*)c_out + o + c_lane;
+        if constexpr (THROUGH) store_write_through((uint64_t*)dst, (uint64_t)__float_as_uint(C[b][1][i]) << 32 | __float_as_uint(C[b][0][i]));
+        else *(float2*)dst = make_float2(C[b][0][i], C[b][1][i]);
+      } else {
+        uint32_t* const dst = (uint32_t*)((uint16_t*)c_out + o + c_lane);
+        if constexpr (THROUGH) store_write_through(dst, pack_state2(C[b][0][i], C[b][1][i], SDT));
+        else *dst = pack_state2(C[b][0][i], C[b][1][i], SDT);
+      }
     }
   if (id.x == 0 && cg == 0) store_state_scalar(n_out, (size_t)bh * DHQK + row0 + lane, SDT, nreg);
   if (id.x == 0 && tid == 0) store_state_scalar(m_out, bh, SDT, m);
   if (!MULTI && whole) finish(0, nb0);
 }
 
-template <bool F16, int SDT, int MODE>
+template <bool F16, int SDT, int MODE, bool THROUGH>
 static const char* launch_step_block_t(const StepBlockArgs& a, hipStream_t stream) {
   const int RG = a.DHQK / 64, CG = a.DHHV % 128 == 0 && RG <= 2 ? 2 : 1, nw = RG * CG;
   const int rows = a.T < kBlk ? a.T : kBlk;
   const int wave_bytes = kBlk * kRowS * 2 > rows * kOutS * 4 ? kBlk * kRowS * 2 : rows * kOutS * 4;
   const size_t smem = (size_t)(kBlk * kDS + 2 * kBlk + nw * (kBlk + 64) + 8) * 4 + (size_t)CG * kBlk * kRowS * 2 + (size_t)nw * wave_bytes;
   static LdsLimit lds;
-  if (!lds.allow((const void*)step_block_kernel<F16, SDT, MODE>, smem)) return "step_block: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((step_block_kernel<F16, SDT, MODE>), dim3(a.DHHV / (64 * CG), a.BH), dim3(64 * nw), smem, stream,
+  if (!lds.allow((const void*)step_block_kernel<F16, SDT, MODE, THROUGH>, smem)) return "step_block: cannot raise the dynamic LDS limit";
+  hipLaunchKernelGGL((step_block_kernel<F16, SDT, MODE, THROUGH>), dim3(a.DHHV / (64 * CG), a.BH), dim3(64 * nw), smem, stream,
                      (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v, a.i, a.f, a.c_in, a.n_in, a.m_in,
                      (uint16_t*)a.h, a.c_out, a.n_out, a.m_out, a.T, a.DHQK, a.DHHV, a.eps, a.dtype_gates, rows);
   return nullptr;
 }
+// All of the state is written at the very end, and what then lies in the L2s goes to memory while the next launch waits for it: a
+// state of up to 96 MB, which the memory-side cache holds beside the old one, is written through them instead.  us, plain /
+// write-through, other states in between and the state of one call the next one's input: 256/512, 8 heads, 16 tokens B=4 12.5 11.9 /
+// 11.3 11.5, B=8 17.4 17.4 / 15.5 15.4, B=16 32.8 31.1 / 29.0 27.1, B=24 (96 MB) 46.9 43.0 / 47.4 39.6, B=32 60.0 61.2 / 62.9 61.3; 64 tokens
+// B=16 65.1 59.0 / 62.2 57.1; 16 heads of 128/256, B=32 34.9 33.1 / 33.3 29.2; 64/128, 4 tokens B=64 13.4 12.9 / 11.5 11.2.  (Non-temporal
+// stores gain the same, B=16 28.2, but the next call then reads from memory: 33.2 instead of 27.1.)
+template <bool F16, int SDT, int MODE>
+static const char* launch_step_block_w(const StepBlockArgs& a, hipStream_t stream) {
+  const bool through = (size_t)a.BH * a.DHQK * a.DHHV * (SDT == 0 ? 4 : 2) <= ((size_t)96 << 20);
+  return through ? launch_step_block_t<F16, SDT, MODE, true>(a, stream) : launch_step_block_t<F16, SDT, MODE, false>(a, stream);
+}
 template <bool F16, int MODE>
 static const char* launch_step_block_s(const StepBlockArgs& a, hipStream_t stream) {
-  if (a.dtype_state == 0) return launch_step_block_t<F16, 0, MODE>(a, stream);
-  return a.dtype_state == 1 ? launch_step_block_t<F16, 1, MODE>(a, stream) : launch_step_block_t<F16, 2, MODE>(a, stream);
+  if (a.dtype_state == 0) return launch_step_block_w<F16, 0, MODE>(a, stream);
+  return a.dtype_state == 1 ? launch_step_block_w<F16, 1, MODE>(a, stream) : launch_step_block_w<F16, 2, MODE>(a, stream);
 }
 
 // 16-bit q, k, v and head dimensions that fill the waves' 64 x 64 parts, a power of two of them so that the rows of v deal
