@@ -48,7 +48,11 @@ struct ShortLds {
   }
 };
 
-// OWN: the workgroup scans the gates of its head (its waves a chunk each, while the rows are on their way).
+// OWN: few workgroups.  Each scans the gates of its head (its waves a chunk each, while the rows are on their way), and H and the last
+// state are written through the caches: what lies in the L2s at the end goes to memory while the next launch waits for it.  us, plain /
+// write-through: 8 heads of 256/512, 317 positions 13.5 / 12.9, 512 26.4 / 25.5; 32 heads of 64 13.7 / 12.2; 4 heads of 512/1024, 300 23.8 /
+// 22.8.  (With more it gains as much up to some 100 MB, but for 384 heads of 64 positions from a state, 192 MB of it, 169.2 / 171.2; chosen
+// in the kernel it costs 512 heads of 64 124 / 133.)
 template <int DQ, int CW, int NSL, bool F16, bool INIT, bool OWN>
 __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned char* smem) {
   using L = ShortLds<DQ, CW, INIT>;
@@ -373,7 +377,11 @@ __device__ __forceinline__ void short_h(const ShortFwArgs& a, int item, unsigned
 #pragma unroll
   for (int x = 0; x < VV; ++x) {
     const int idx = tid + x * kShortThreads, row = idx / (CW / 8), u = idx % (CW / 8);
-    if (t0 + row < S) *(u32x4*)(Og + (size_t)row * DHHV + u * 8) = *(const u32x4*)(Os + row * OS + u * 8);
+    if (t0 + row < S) {
+      const u32x4 x4 = *(const u32x4*)(Os + row * OS + u * 8);
+      if constexpr (OWN) store_write_through(Og, 64 * (uint32_t)DHHV * 2, (row * (uint32_t)DHHV + u * 8) * 2, x4);
+      else *(u32x4*)(Og + (size_t)row * DHHV + u * 8) = x4;
+    }
   }
 }
 
@@ -554,7 +562,12 @@ __device__ __forceinline__ void short_c(const ShortFwArgs& a, int item, unsigned
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int d = bx * RT + 32 * rb + 8 * (i / 4) + 4 * h + (i % 4);
-        a.final_out[((size_t)bh * DQ + d) * DHHV + by * WT + 32 * (cb0 + b) + r] = acc[b][i] + rest[b][i];
+        const float x = acc[b][i] + rest[b][i];
+        if constexpr (OWN) {
+          store_write_through(a.final_out + (size_t)bh * DQ * DHHV, DQ * (uint32_t)DHHV * 4, (uint32_t)(d * DHHV + by * WT + 32 * (cb0 + b) + r) * 4, __float_as_uint(x));
+        } else {
+          a.final_out[((size_t)bh * DQ + d) * DHHV + by * WT + 32 * (cb0 + b) + r] = x;
+        }
       }
   }
   if (with_n) {
