@@ -22,7 +22,7 @@
 // chunks twice, once with the heads and once with the remainders.  Same tiling, same arithmetic, same results.
 //
 // A scan of few (batch, head) pairs has too few state tiles to fill the chip and walks the sequence chunk by chunk at
-// 1.9 us, whatever the memory could deliver.  It is cut into segments of the sequence that run side by side: a first
+// 1.6 to 1.9 us, whatever the memory could deliver.  It is cut into segments of the sequence that run side by side: a first
 // launch accumulates every segment but the last from zero, a second one runs all segments from the state before them,
 // which is the decayed sum of the first launch's results (the decay factors depend on the gates only).
 //
@@ -1100,18 +1100,32 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
   if (a.skip_zero && a.init == nullptr && a.final_out == nullptr && a.nstates == nullptr && a.end_c == 0) return nullptr;
   const bool r128 = a.DHQK % 128 == 0;
   bool w128 = a.DHHV % 128 == 0;
-  // Segments (see the top of the file): as many as fit the chip beside each other, at most eight, of eight chunks or more;
-  // with fewer than three the second reading of the sequence costs what the segments gain.  Their states go through the
-  // caller's scratch (an output that is written later), which has to hold them.  B = 1, NH = 8, S = 10000, 256/512: one
-  // scan 151 us in one piece, 45 + 57 us in four.
+  // Segments (see the top of the file): the number of them, of those that fit the chip beside each other, that the two launches
+  // take the least time with.  Their states go through the caller's scratch (an output that is written later), which has to
+  // hold them.  Fixed time, time for a chunk of a segment and for a segment in front, from sweeps of 1 to 16 segments, and 10 %
+  // for what they leave out.  us, one scan in one piece / in the segments that this takes: 4 heads of 64/64, 2000 positions 37.0 / 30.5,
+  // 4000 62.3 / 34.5, 10000 135.6 / 42; 32 heads of 64/128, 4000 62.4 / 43.3; 16 heads of 128/256, 4000 50.0 / 47.1; 8 heads of 256/512,
+  // 10000 130.9 / 102.4, but 4000 50.1 / 53.4 (tiles of half the width in one piece).  With a backward the launches of a short call are what
+  // its host takes the longest for (4 heads of 64/64, 2048 positions, forward and backward 102 / 107): 8 us have to be gained there.
   {
     const int tiles = (a.DHQK / (r128 ? 128 : 64)) * (a.DHHV / (w128 ? 128 : 64));
+    const bool wide = r128 && w128;
     const int fit = device_cu_count() / (BH * tiles);
-    const int nseg = fit < 8 ? fit : 8;
-    const size_t need = (size_t)BH * (nseg - 1) * ((size_t)a.DHQK * a.DHHV + a.DHQK) * sizeof(float);
-    if (nseg >= 3 && a.NC >= 8 * nseg && a.seg != nullptr && need <= a.seg_bytes) {
-      a.seg_len = (a.NC + nseg - 1) / nseg;
-      a.nseg = (a.NC + a.seg_len - 1) / a.seg_len;
+    const bool halves = wide && 2ll * BH * tiles <= device_cu_count();  // (see below)
+    const float one_piece = wide ? (halves ? 4.f + 1.6f * a.NC : 12.f + 1.9f * a.NC) : 12.f + 1.57f * a.NC;
+    float best = a.with_backward ? fminf(0.9f * one_piece, one_piece - 8.f) : 0.9f * one_piece;
+    int len = 0;
+    for (int n = 2; n <= (wide ? 8 : 16) && n <= fit && a.seg != nullptr; ++n) {
+      const int l = (a.NC + n - 1) / n;
+      const float t = wide ? 16.f + 4.f * l + 1.2f * n : 20.f + 2.8f * l + 0.55f * n;
+      if (t < best && (size_t)BH * (n - 1) * ((size_t)a.DHQK * a.DHHV + a.DHQK) * sizeof(float) <= a.seg_bytes) {
+        best = t;
+        len = l;
+      }
+    }
+    if (len > 0) {
+      a.seg_len = len;
+      a.nseg = (a.NC + len - 1) / len;
     }
   }
   // Tiles of half the width where those of both halves still have a CU each: the walk over the chunks is what the launch

@@ -82,6 +82,14 @@ def test_segmented_scan(B, NH, S, DQ, DV, opt, f_offset):
     _run(S, DQ, DV, B=B, NH=NH, seed=S, f_offset=f_offset, **opt)
 
 
+# segments of two to six chunks, up to sixteen of them, the last one shorter than the others
+@pytest.mark.parametrize("NH,S,DQ,DV,opt", [(4, 20 * 128 - 3, 64, 64, dict()), (1, 32 * 128 + 1, 64, 128, dict(init=True)), (2, 33 * 128, 128, 128, dict(sig=True)),
+                                            (1, 41 * 128 + 5, 128, 64, dict(init=True, dtype=torch.float16)), (3, 24 * 128, 64, 192, dict(init=True, sig=True))])
+@pytest.mark.parametrize("f_offset", [3.0, 9.0])
+def test_short_segments(NH, S, DQ, DV, opt, f_offset):
+    _run(S, DQ, DV, NH=NH, seed=S, f_offset=f_offset, **opt)
+
+
 @pytest.mark.parametrize("NH,S,DQ,DV", [(1, 8200, 128, 128), (2, 8192, 256, 512), (8, 4100, 256, 512)])
 @pytest.mark.parametrize("path", ["auto", "split"])
 def test_segmented_scan_is_recomputed_in_segments(NH, S, DQ, DV, path):
