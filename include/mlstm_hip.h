@@ -256,6 +256,16 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
                            int dtype_qkv, int dtype_gates, int gate, int normalize, int path, int state_stride,
                            void* stream);
 
+/* The same with dI, dF in dtype_gate_grads (MLSTM_F32, MLSTM_BF16 or MLSTM_F16), rounded once from the fp32 sums. */
+int mlstm_hip_chunkwise_bw_typed(const void* q, const void* k, const void* v, const void* i, const void* f,
+                                 const void* dH, const float* dC_last,
+                                 void* dQ, void* dK, void* dV, void* dI, void* dF, float* dC0,
+                                 const void* fw_workspace, size_t fw_workspace_bytes,
+                                 void* bw_workspace, size_t bw_workspace_bytes,
+                                 int B, int NH, int S, int DHQK, int DHHV, float eps,
+                                 int dtype_qkv, int dtype_gates, int dtype_gate_grads, int gate, int normalize, int path,
+                                 int state_stride, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -36,6 +36,7 @@ _SIGNATURES = {
     "mlstm_hip_chunkwise_fw_noalloc": (_i, [_vp] * 14 + [_i] * 5 + [_f] + [_i] * 4 + [_vp]),
     "mlstm_hip_chunkwise_bw_workspace_bytes": (_sz, [_i] * 6),
     "mlstm_hip_chunkwise_bw": (_i, [_vp] * 14 + [_sz, _vp, _sz] + [_i] * 5 + [_f] + [_i] * 6 + [_vp]),
+    "mlstm_hip_chunkwise_bw_typed": (_i, [_vp] * 14 + [_sz, _vp, _sz] + [_i] * 5 + [_f] + [_i] * 7 + [_vp]),
 }
 
 

@@ -523,6 +523,17 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
                            size_t bw_workspace_bytes, int B, int NH, int S, int DHQK, int DHHV, float eps,
                            int dtype_qkv, int dtype_gates, int gate, int normalize, int path, int state_stride,
                            void* stream) {
+  return mlstm_hip_chunkwise_bw_typed(q, k, v, i, f, dH, dC_last, dQ, dK, dV, dI, dF, dC0, fw_workspace, fw_workspace_bytes, bw_workspace,
+                                      bw_workspace_bytes, B, NH, S, DHQK, DHHV, eps, dtype_qkv, dtype_gates, MLSTM_F32, gate, normalize,
+                                      path, state_stride, stream);
+}
+
+int mlstm_hip_chunkwise_bw_typed(const void* q, const void* k, const void* v, const void* i, const void* f, const void* dH,
+                                 const float* dC_last, void* dQ, void* dK, void* dV, void* dI, void* dF, float* dC0,
+                                 const void* fw_workspace, size_t fw_workspace_bytes, void* bw_workspace,
+                                 size_t bw_workspace_bytes, int B, int NH, int S, int DHQK, int DHHV, float eps,
+                                 int dtype_qkv, int dtype_gates, int dtype_gate_grads, int gate, int normalize, int path,
+                                 int state_stride, void* stream) {
   if (!q || !k || !v || !i || !f || !dH || !dQ || !dK || !dV || !dI || !dF || !fw_workspace || !bw_workspace)
     return fail("mlstm_hip_chunkwise_bw: null pointer argument");
   if (const char* e = check_dims(B, NH, S, DHQK, DHHV)) return fail(e);
@@ -530,6 +541,7 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
   if (dtype_qkv != MLSTM_BF16 && dtype_qkv != MLSTM_F16) return fail("mlstm_hip_chunkwise_bw: q/k/v/dH must be bf16 or fp16");
   if (dtype_gates != MLSTM_F32 && dtype_gates != MLSTM_BF16 && dtype_gates != MLSTM_F16)
     return fail("mlstm_hip_chunkwise_bw: unsupported gate dtype");
+  if (!valid_dtype(dtype_gate_grads)) return fail("mlstm_hip_chunkwise_bw: unsupported dtype of the gate gradients");
   const int f16 = dtype_qkv == MLSTM_F16;
   if (gate != MLSTM_GATE_EXP && gate != MLSTM_GATE_SIG) return fail("mlstm_hip_chunkwise_bw: unknown gate code");
   const int stride = resolve_stride(state_stride);
@@ -658,7 +670,7 @@ int mlstm_hip_chunkwise_bw(const void* q, const void* k, const void* v, const vo
   memset(&ga, 0, sizeof(ga));
   ga.i = i; ga.f = f; ga.qdq = bws.qdq; ga.kdk = bws.kdk; ga.dI = dI; ga.dF = dF;
   ga.ntiles = tiles;
-  ga.S = S; ga.NC = NC; ga.dtype_gates = dtype_gates; ga.sig_gate = sig;
+  ga.S = S; ga.NC = NC; ga.dtype_gates = dtype_gates; ga.sig_gate = sig; ga.dtype_grads = dtype_gate_grads;
   {
     ProfileScope ps("gate_grads", st);
     if (const char* e = mlstm::launch_gate_grads(ga, BH, st)) return fail(e);

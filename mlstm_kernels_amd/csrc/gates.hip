@@ -278,10 +278,10 @@ __global__ __launch_bounds__(kGateThreads) void gate_grads_kernel(GateGradArgs a
     if (t0 + e < S) {
       const size_t o = (size_t)bh * S + t0 + e;
       const float fv = load_scalar(a.f, o, a.dtype_gates);
-      a.dF[o] = suf[e] * (1.f / (1.f + expf(fv)));  // sigmoid(-f)
+      store_state_scalar(a.dF, o, a.dtype_grads, suf[e] * (1.f / (1.f + expf(fv))));  // sigmoid(-f)
       float di = kd[e];
       if (a.sig_gate) di *= 1.f / (1.f + expf(load_scalar(a.i, o, a.dtype_gates)));
-      a.dI[o] = di;
+      store_state_scalar(a.dI, o, a.dtype_grads, di);
     }
   }
 }

@@ -355,17 +355,20 @@ class ChunkwiseFunction : public torch::autograd::Function<ChunkwiseFunction> {
     Tensor dCl;
     if (grads.size() > 1 && grads[1].defined()) dCl = as_dense(grads[1], at::kFloat);
     const Tensor dQ = empty(q.sizes(), kd, dev), dK = empty(k.sizes(), kd, dev);
-    const Tensor dI = empty({B, NH, S}, at::kFloat, dev), dF = empty({B, NH, S}, at::kFloat, dev);
+    // (gradients of 16-bit gates are rounded where they are summed; gates of two types are left to the conversions below)
+    const at::ScalarType gd = cfg->it == cfg->ft && dtype_code(cfg->it) >= 0 ? cfg->it : at::kFloat;
+    const Tensor dI = empty({B, NH, S}, gd, dev), dF = empty({B, NH, S}, gd, dev);
     Tensor dC0;
     if (cfg->has_c0) dC0 = empty({B, NH, DQ, DV}, at::kFloat, dev);
-    check_rc(mlstm_hip_chunkwise_bw(ptr(q), ptr(k), ptr(v), ptr(i), ptr(f), ptr(dH), fptr(dCl), ptr(dQ), ptr(dK), ptr(dV),
-                                    fptr(dI), fptr(dF), fptr(dC0), ptr(ws), (size_t)ws.numel(), ptr(bws), bw_bytes, B, NH, S,
-                                    DQ, DV, (float)cfg->eps, dtype_code(kd), dtype_code(i.scalar_type()),
-                                    cfg->siging ? MLSTM_GATE_SIG : MLSTM_GATE_EXP, cfg->normalize, cfg->path, cfg->stride, stream),
+    check_rc(mlstm_hip_chunkwise_bw_typed(ptr(q), ptr(k), ptr(v), ptr(i), ptr(f), ptr(dH), fptr(dCl), ptr(dQ), ptr(dK), ptr(dV),
+                                          ptr(dI), ptr(dF), fptr(dC0), ptr(ws), (size_t)ws.numel(), ptr(bws), bw_bytes, B, NH, S,
+                                          DQ, DV, (float)cfg->eps, dtype_code(kd), dtype_code(i.scalar_type()), dtype_code(gd),
+                                          cfg->siging ? MLSTM_GATE_SIG : MLSTM_GATE_EXP, cfg->normalize, cfg->path, cfg->stride,
+                                          stream),
              "mlstm_hip_chunkwise_bw");
     Tensor dn0, dm0;
-    if (cfg->has_n0) dn0 = at::zeros({B, NH, DQ}, dI.options());
-    if (cfg->has_m0) dm0 = at::zeros({B, NH, 1}, dI.options());
+    if (cfg->has_n0) dn0 = at::zeros({B, NH, DQ}, at::TensorOptions().dtype(at::kFloat).device(dev));
+    if (cfg->has_m0) dm0 = at::zeros({B, NH, 1}, at::TensorOptions().dtype(at::kFloat).device(dev));
     return {dQ.to(cfg->qt), dK.to(cfg->kt), dV.to(cfg->vt), dI.to(cfg->it), dF.to(cfg->ft),
             dC0.defined() ? dC0.to(cfg->c0t) : dC0, dn0, dm0, Tensor()};
   }

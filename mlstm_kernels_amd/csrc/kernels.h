@@ -200,8 +200,9 @@ struct GateGradArgs {
   const void *i, *f;        // gate pre-activations (B,NH,S)
   const float *qdq, *kdk;   // [ntiles][BH][Sp]: one slot per head-dimension tile of the dQ/dK kernel
   int ntiles;
-  float *dI, *dF;           // (B,NH,S) fp32
+  void *dI, *dF;            // (B,NH,S)
   int S, NC, dtype_gates, sig_gate;
+  int dtype_grads;          // of dI and dF: 0 fp32, 1 bf16, 2 fp16
 };
 
 const char* launch_step(const void* q, const void* k, const void* v, const void* i, const void* f,

@@ -479,3 +479,23 @@ def test_padding_adapter_without_padding(S, chunk):
                               padded, dH)
     for name, x, y in zip(("dQ", "dK", "dV", "dI", "dF"), grads, ref):
         assert rel_norm(x, y[:, :, :S]) <= 2e-3, name
+
+
+@pytest.mark.parametrize("S", [1, 127, 2049])
+@pytest.mark.parametrize("gates", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sig", [False, True])
+def test_gradients_of_16_bit_gates(S, gates, sig):
+    """dI and dF leave the kernel in the gates' type: those of the same gates in 32 bits, rounded once."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    q, k, v, i, f = (t.cuda() for t in make_qkvif(1, 2, S, 64, 64, seed=S, f_offset=3.0))
+    dH = torch.randn(v.shape, generator=torch.Generator().manual_seed(2)).bfloat16().cuda()
+    grads = []
+    for gi, gf in ((torch.float32, torch.float32), (gates, gates), (gates, torch.float32)):
+        leaves = [t.detach().clone().requires_grad_(True) for t in (q, k, v, i.to(gates).to(gi), f.to(gates).to(gf))]
+        grads.append(torch.autograd.grad(op(*leaves, any_sequence_length=True), leaves, dH))
+        assert grads[-1][3].dtype == gi and grads[-1][4].dtype == gf
+    for other in grads[1:]:
+        for a, b in zip(grads[0], other):
+            assert torch.equal(a.to(b.dtype), b)
