@@ -5,28 +5,42 @@
 
 namespace mlstm {
 
-// Inclusive scan over the 64 lanes by cross-lane moves of the vector unit (inside rows of 16 lanes, then row totals): a shuffle through
-// LDS takes ten times as long, and a chunk needs over twenty one after the other (8 heads of 317 positions of 256/512, short_fw with its
-// own gates: 14.05 us by shuffles, 13.5 so; 512 heads of 64 162.8, 153.3).  `outside`: what a lane without a source sees (nothing is done there: op(outside, x) = x).
-template <typename Op>
-__device__ __forceinline__ float wave_incl_scan(float x, Op op, float outside) {
-#define MLSTM_DPP_STEP(ctrl, rows)                                                                                                 \
-  {                                                                                                                                \
-    const float y = __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(outside), __float_as_uint(x), ctrl, rows, 0xf, false)); \
-    x = op(y, x);                                                                                                                  \
+// Scans over the 64 lanes by cross-lane moves of the vector unit where it has them: a shuffle through LDS takes ten times as long, and a
+// chunk needs over twenty scan steps one after the other (8 heads of 317 positions of 256/512, short_fw with its own gates: 14.05 us by
+// shuffles, 13.5 with the sums in another order).
+__device__ __forceinline__ float lane_up(float x, float first) {  // of the lane before
+  return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(first), __float_as_uint(x), 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
+// Inclusive sums.  Step o adds the sum of the o lanes before to that of the last o: the order of the sums is that of six shuffles.
+__device__ __forceinline__ float wave_incl_sum(float x) {
+  float y = lane_up(x, 0.f);
+  x = y + x;
+  y = lane_up(lane_up(x, 0.f), 0.f);
+  x = y + x;
+  y = lane_up(lane_up(lane_up(lane_up(x, 0.f), 0.f), 0.f), 0.f);
+  x = y + x;
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1) {
+    y = __shfl_up(x, o);
+    x = (int)(threadIdx.x & 63) >= o ? y + x : x;
   }
-  MLSTM_DPP_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8
-  MLSTM_DPP_STEP(0x112, 0xf)
-  MLSTM_DPP_STEP(0x114, 0xf)
-  MLSTM_DPP_STEP(0x118, 0xf)
-  MLSTM_DPP_STEP(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
-  MLSTM_DPP_STEP(0x143, 0xc)  // row_bcast:31 into rows 2 and 3
-#undef MLSTM_DPP_STEP
   return x;
 }
-template <typename Op>
-__device__ __forceinline__ float wave_rev_incl_scan(float x, Op op, float outside) {  // over the lanes from this one on
-  return __shfl_xor(wave_incl_scan(__shfl_xor(x, 63), op, outside), 63);
+__device__ __forceinline__ float wave_rev_incl_sum(float x) {  // over the lanes from this one on
+  return __shfl_xor(wave_incl_sum(__shfl_xor(x, 63)), 63);
+}
+// Inclusive maxima (in any order the same): inside rows of 16 lanes, then row by row.
+__device__ __forceinline__ float wave_incl_max(float x) {
+#define MLSTM_DPP_MAX(ctrl, rows)                                                                                                  \
+  x = fmaxf(__uint_as_float(__builtin_amdgcn_update_dpp(0xff800000u, __float_as_uint(x), ctrl, rows, 0xf, false)), x);
+  MLSTM_DPP_MAX(0x111, 0xf)  // row_shr:1, 2, 4, 8
+  MLSTM_DPP_MAX(0x112, 0xf)
+  MLSTM_DPP_MAX(0x114, 0xf)
+  MLSTM_DPP_MAX(0x118, 0xf)
+  MLSTM_DPP_MAX(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
+  MLSTM_DPP_MAX(0x143, 0xc)  // row_bcast:31 into rows 2 and 3
+#undef MLSTM_DPP_MAX
+  return x;
 }
 __device__ __forceinline__ float last_lane(float x) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63)); }
 
@@ -61,8 +75,6 @@ struct ChunkScan {
 };
 __device__ __forceinline__ ChunkScan scan_chunk(const RawGates& raw, int c, int lane, int S, int dtype_gates, int sig_gate) {
   const float NEG_INF = -__builtin_inff();
-  auto add = [](float a, float b) { return a + b; };
-  auto mx = [](float a, float b) { return fmaxf(a, b); };
   const int t0 = c * kChunk + 2 * lane;
   float lf[2], it[2];
 #pragma unroll
@@ -73,17 +85,16 @@ __device__ __forceinline__ ChunkScan scan_chunk(const RawGates& raw, int c, int 
     it[e] = !in ? NEG_INF : sig_gate ? log_sigmoid(iv) : iv;
   }
   const float pair = lf[0] + lf[1];
-  const float incl = wave_incl_scan(pair, add, 0.f);
+  const float incl = wave_incl_sum(pair);
   const float b1 = incl, b0 = (incl - pair) + lf[0];
-  const float rincl = wave_rev_incl_scan(pair, add, 0.f);
+  const float rincl = wave_rev_incl_sum(pair);
   const float suf1 = rincl - pair, suf0 = suf1 + lf[1];
   const float a0 = suf0 + it[0], a1 = suf1 + it[1];
   const float x0 = it[0] - b0, x1 = it[1] - b1;
-  const float pm = wave_incl_scan(fmaxf(x0, x1), mx, NEG_INF);
-  float pm_excl = __shfl_up(pm, 1);
-  if (lane == 0) pm_excl = NEG_INF;
+  const float pm = wave_incl_max(fmaxf(x0, x1));
+  const float pm_excl = lane_up(pm, NEG_INF);
   const float cm0 = fmaxf(pm_excl, x0), cm1 = pm;
-  return {{b0, b1}, {a0, a1}, {b0 + cm0, b1 + cm1}, {b0 - it[0], b1 - it[1]}, last_lane(incl), last_lane(wave_incl_scan(fmaxf(a0, a1), mx, NEG_INF))};
+  return {{b0, b1}, {a0, a1}, {b0 + cm0, b1 + cm1}, {b0 - it[0], b1 - it[1]}, last_lane(incl), last_lane(wave_incl_max(fmaxf(a0, a1)))};
 }
 
 // m before chunk c < 4 of a head (the recurrence m_c = max(g_c + m_{c-1}, amax_c) with its sums in the order of the pre-pass)

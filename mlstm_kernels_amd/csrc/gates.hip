@@ -265,8 +265,7 @@ __global__ __launch_bounds__(kGateThreads) void gate_grads_kernel(GateGradArgs a
     d[e] = t0 + e < S ? diff(t0 + e) : 0.f;
   }
   const float pair = d[0] + d[1];
-  auto add = [](float x, float y) { return x + y; };
-  const float rincl = wave_rev_incl_scan(pair, add, 0.f);  // sum over lanes >= lane
+  const float rincl = wave_rev_incl_sum(pair);  // sum over lanes >= lane
   if (lane == 0) wtot[wave] = rincl;
   __syncthreads();
   for (int w = wave + 1; w < kGateThreads / kWave; ++w) after += wtot[w];
