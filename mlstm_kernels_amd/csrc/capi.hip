@@ -404,6 +404,7 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   sa.eps = eps;
   sa.backward = 0;
   sa.with_backward = keep_for_backward;
+  sa.by_batch = path == MLSTM_PATH_AUTO;
   sa.stride = stride;
   sa.f16 = f16;
   sa.skip_zero = choose_hv(path, pa, BH) != kHvTiled;  // (in the backward both dQ / dK kernels know, from g.zero_c)
@@ -485,6 +486,7 @@ int mlstm_hip_chunkwise_recompute_states_scratch(const void* k, const void* v, c
   sa.qk_scale = 1.0f / sqrtf((float)DHQK);
   sa.backward = 0;
   sa.with_backward = 1;
+  sa.by_batch = scratch != nullptr;
   sa.stride = stride;
   sa.f16 = dtype_qkv == MLSTM_F16;
   sa.seg = (float*)scratch;
@@ -642,6 +644,7 @@ int mlstm_hip_chunkwise_bw_typed(const void* q, const void* k, const void* v, co
     sa.qk_scale = qk_scale; sa.eps = eps;
     sa.skip_zero = choose_hv(path, pv, BH) != kHvTiled && choose_window_qk(path, pq, BH);
     sa.backward = sa.with_backward = 1;
+    sa.by_batch = path == MLSTM_PATH_AUTO;
     // as in the forward; dV is written after the scan
     sa.seg = path == MLSTM_PATH_AUTO && !in_place ? (float*)dV : nullptr;
     sa.seg_bytes = (size_t)BH * S * DHHV * 2;

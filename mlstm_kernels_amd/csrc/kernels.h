@@ -76,6 +76,8 @@ struct ScanArgs {
   int end_c, end_n;       // chunks run for the state (in scan order) and for n
   int part;               // 0 whole sequence; 1 / 2 the two launches of a forward scan that returns the last state
   int n_bh;               // batch * heads
+  int by_batch;           // the kernels may be chosen by the number of heads (a path that the caller names: not)
+  int repeat_all;         // (launch_scan) late chunks always run twice
   int with_backward;      // this is a call with a backward, or the backward
   int nseg, seg_len;      // segments of the sequence, chunks in each (the last one may be shorter)
   int seg_phase;          // 0 one piece; 1 every segment but the last from zero, 2 all segments from their states

@@ -77,9 +77,8 @@ __device__ __forceinline__ int first_remainder_chunk(const float* gbar_bh, int N
 // Whether the chunks that carry the remainder run twice in scan_roles_kernel (once with the 16-bit heads, once with the
 // remainders) or go to scan_kernel in a launch of its own.  A second run costs a chunk's time again (2.3 us at B = 4,
 // S = 16384, against 3.6 us for both operands at once in scan_kernel), the launch and its tail a fixed 12 us per round
-// of workgroups: worth it while the late chunks are at most a quarter of all, and for sequences of four chunks at most.
-constexpr int kScanShort = 4;
-__device__ __forceinline__ bool scan_repeats_late(int NC, int c_lo) { return NC <= kScanShort || 4 * (NC - c_lo) <= NC; }
+// of workgroups.  repeat_all: they always do (launch_scan has the rule); otherwise where they are at most a quarter of all.
+__device__ __forceinline__ bool scan_repeats_late(const ScanArgs& a, int c_lo) { return a.repeat_all || 4 * (a.NC - c_lo) <= a.NC; }
 
 #define SCAN_WPE(HILO_, WCOLS_) ((WCOLS_) == 64 && (HILO_) ? 1 : 2)
 // WCOLS = value columns per wave (64 or 32): with 32 a 128 x 128 tile takes eight waves, two per SIMD, each with
@@ -139,7 +138,7 @@ __global__ __launch_bounds__(64 * (RT / 64) * (WT / WCOLS))
   int c_lo = 0;
   if constexpr (HILO) {
     if (!a.backward) c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)bh * NC, NC, lane);
-    if (a.part == 2 && scan_repeats_late(NC, c_lo)) return;  // the first launch ran everything
+    if (a.part == 2 && scan_repeats_late(a, c_lo)) return;  // the first launch ran everything
   }
 
   f32x16 acc[2][NBW];
@@ -523,7 +522,7 @@ __device__ __forceinline__ ScanJob scan_decode(const ScanArgs& a, int round, int
   int n_all = a.nstates != nullptr && job.by == 0 ? a.end_n : a.end_c, c_lo = a.NC;
   if (REP) {
     c_lo = a.all_remainder ? 0 : first_remainder_chunk(a.gbar + (size_t)job.bh * a.NC, a.NC, lane);
-    if (!scan_repeats_late(a.NC, c_lo)) n_all = c_lo;
+    if (!scan_repeats_late(a, c_lo)) n_all = c_lo;
   }
   job.it_lo = SEG ? job.seg * a.seg_len : 0;
   job.it_hi = max(SEG ? min(job.it_lo + a.seg_len, n_all) : n_all, job.it_lo);
@@ -1115,7 +1114,7 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
     const float one_piece = wide ? (halves ? 4.f + 1.6f * a.NC : 12.f + 1.9f * a.NC) : 12.f + 1.57f * a.NC;
     float best = a.with_backward ? fminf(0.9f * one_piece, one_piece - 8.f) : 0.9f * one_piece;
     int len = 0;
-    for (int n = 2; n <= (wide ? 8 : 16) && n <= fit && a.seg != nullptr; ++n) {
+    for (int n = 2; n <= (wide ? 8 : 16) && n <= fit && a.by_batch; ++n) {
       const int l = (a.NC + n - 1) / n;
       const float t = wide ? 16.f + 4.f * l + 1.2f * n : 20.f + 2.8f * l + 0.55f * n;
       if (t < best && (size_t)BH * (n - 1) * ((size_t)a.DHQK * a.DHHV + a.DHQK) * sizeof(float) <= a.seg_bytes) {
@@ -1123,10 +1122,19 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
         len = l;
       }
     }
-    if (len > 0) {
+    if (len > 0 && a.seg != nullptr) {
       a.seg_len = len;
       a.nseg = (a.NC + len - 1) / len;
     }
+    // Late chunks in a second run whatever their number: sequences of four chunks, and where the kernels may be chosen by the heads
+    // of the call and the scan is in one piece (a call whose states are written in place, which alone keeps it from segments, has
+    // the bits of the other kernel in many late chunks, as a named path has) up to 24 chunks, or any number of them
+    // while the tiles do not fill the chip; not with the sigmoid gate and tiles that do, where all chunks are late.  us for a
+    // forward with the last state, a launch more / so, the last chunk late / all of them: 256/512, 8 heads of 700 49.3 52.2 / 39.5
+    // 44.4, of 2000 56.4 82.6 / 54.0 70.2, 64 of 1000 117.5 149.9 / 112.4 132.3, 96 of 3000 448 558 / 446 547; 64/64, 4 heads of 1000
+    // 37.2 50.3 / 35.7 45.4; but 96 of 8000 all late 1386 / 1414, and sigmoid gate, 64 of 4000 473 / 487.
+    const bool fills = (long long)BH * tiles >= device_cu_count();
+    a.repeat_all = a.NC <= 4 || (a.by_batch && len == 0 && (!fills || (a.NC <= 24 && !a.all_remainder)));
   }
   // Tiles of half the width where those of both halves still have a CU each: the walk over the chunks is what the launch
   // takes then, and half the columns make a chunk a quarter shorter (256/512, us, 128 / 64 columns: 8 heads of 317 positions
@@ -1152,14 +1160,14 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
     // Forward that returns the last state: the chunks whose rounding no longer shows in it need no remainder operand.
     // Where the rest are few they run twice in the same kernel; otherwise it leaves its state in final_out / n_final and
     // the kernel with both operands continues from there.  The number is known on the device only (it follows from the
-    // decay factors): the second launch is made in any case and ends at once where it has nothing to do, except for short
-    // sequences, which do not need it, and for the sigmoid gate, where all chunks carry the remainder.
+    // decay factors): the second launch is made in any case and ends at once where it has nothing to do, except where late
+    // chunks always run twice, and for the sigmoid gate, where all chunks carry the remainder.
     if (a.final_out == nullptr || a.backward) return "scan: the remainder split serves the forward last state only";
     const bool two = a.nstates == nullptr || a.n_final != nullptr;  // n needs its hand-over buffer too
-    if (a.NC <= kScanShort || (two && !a.all_remainder)) {
+    if (a.repeat_all || (two && !a.all_remainder)) {
       a.part = 1;
       if (const char* e = roles()) return e;
-      if (a.NC <= kScanShort) return nullptr;
+      if (a.repeat_all) return nullptr;
       a.part = 2;
     }
     if (r128 && w128) return launch_scan_t<128, 128, true>(a, BH, stream);
