@@ -255,6 +255,8 @@ const char* launch_step(const void* q, const void* k, const void* v, const void*
   // Below it, the first batch is as many rows as every row group has, up to 16: what is left over is read one row after the other.
   // us, 16 rows at a time / so (128/256 heads, inputs and state new to the caches): 16 x 16 heads 13.9 / 13.3, 64 x 16 60.2 / 53.3, 100 x 16
   // 100.5 / 86.3, with 16-bit states 64 x 16 42.5 / 29.7; 64/64, 512 x 4 26.5 / 20.7.
+  // Heads of 64 rows and columns: slices of 64, half the lanes of one of 128 have nothing to do (64/64, 4 heads, 128 / 64 columns: B=200
+  // 10.5 / 9.1, of which the host takes all, B=400 16.1 / 11.0, B=512 19.8 / 12.5, 16-bit states 14.1 / 9.1).
   // Write-through where many workgroups of up to 64 KB follow one another on a CU, and the memory-side cache holds the old state beside
   // the new one: us, plain / write-through, the state of one call the next one's input: 128/256, 32 x 16 heads (64 MB) 24.4 / 22.9;
   // 64/128, 128 x 8 (32 MB) 17.1 / 15.1, 400 x 8 42.0 / 37.9; 16-bit states, 256/512 32 x 8 (64 MB) 28.9 / 27.6, 128/256 64 x 16 26.7 / 24.2.
@@ -265,6 +267,7 @@ const char* launch_step(const void* q, const void* k, const void* v, const void*
   const bool through = slice_bytes <= 65536 && state_bytes > ((size_t)(slice_bytes <= 32768 ? 12 : 32) << 20) && state_bytes <= ((size_t)112 << 20);
 #define MLSTM_STEP_ROWS(MODE_)                                       \
   {                                                                  \
+    if (DHHV <= 64 && DHQK < 128) MLSTM_STEP_PICK(64, 16, 4, MODE_)  \
     if (DHQK >= 256) MLSTM_STEP_PICK(128, 16, 16, MODE_)             \
     if (DHQK >= 128) MLSTM_STEP_PICK(128, 16, 8, MODE_)              \
     MLSTM_STEP_PICK(128, 16, 4, MODE_)                               \

@@ -18,7 +18,8 @@ def _inputs(n, T, DQ, DV, sdt, seed):
 # (rows, columns, state type, MiB of state: on either side of 12, 32, 112 and 320)
 @pytest.mark.parametrize("DQ,DV,sdt,mib", [(64, 128, _F32, 11), (64, 128, _F32, 20), (64, 128, _F32, 120), (48, 132, _F32, 20), (65, 64, _F32, 40),
                                            (127, 256, _F32, 40), (128, 256, _F32, 40), (129, 260, _F32, 40), (255, 64, _BF16, 40),
-                                           (256, 512, _BF16, 40), (256, 512, _F32, 40), (100, 72, _BF16, 20), (128, 256, _F32, 330)])
+                                           (256, 512, _BF16, 40), (256, 512, _F32, 40), (100, 72, _BF16, 20), (128, 256, _F32, 330),
+                                           (64, 64, _F32, 5), (64, 64, _F32, 20), (33, 40, _BF16, 20), (127, 64, _F32, 20)])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_step(DQ, DV, sdt, mib, in_place):
     from mlstm_kernels_amd.torch.recurrent import mlstm_recurrent_step__hip_fw
