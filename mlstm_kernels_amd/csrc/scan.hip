@@ -1132,7 +1132,8 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
     // of all segments in one piece.  (Not the segments of more than eight narrow tiles up to 33 chunks: a call whose states are written
     // in place, which alone keeps it from segments, has the bits of one that is not at those lengths, and then only the other kernel
     // has them where many chunks are late.  There the empty segments in front cost what they do: 32 heads of 64/64, 2000 positions, one piece
-    // and its second launch / segments, last chunk late 56.6 / 49.3, all late 81.2 / 87.6; 12 of 4000 85.8 / 56.9, 133 / 141.)  us for a forward with the last state, a launch more / so, the last chunk late / all of them: 256/512,
+    // and its second launch / segments, last chunk late 56.6 / 49.3, all late 81.2 / 87.6; 12 of 4000 85.8 / 56.9, 133 / 141.)
+    // us for a forward with the last state, a launch more / so, the last chunk late / all of them: 256/512,
     // 8 heads of 700 49.3 52.2 / 39.5 44.4, of 2000 56.4 82.6 / 54.0 70.2, of 10000 201 370 / 199 257, 64 of 1000 117.5 149.9 / 112.4 132.3, 96 of
     // 3000 448 558 / 446 547; 64/64, 4 heads of 1000 37.2 50.3 / 35.7 45.4, of 10000 63.3 282 / 60.1 71.3; 16 of 128/256, 4000 81.0 149 / 78.7 86.7; but 96
     // of 8000 all late 1386 / 1414, and sigmoid gate, 64 of 4000 473 / 487.
