@@ -63,7 +63,10 @@ const char* mlstm_hip_last_error(void);
  *   MLSTM_PATH_AUTO  : the fastest one for the shape as measured on MI355X: the streaming H / dV kernels where the
  *                      conditions of MLSTM_PATH_STREAM hold; at state_stride 2 the kernels over windows of two chunks
  *                      that share a kept state (H / dV of the other shapes, dQ / dK of all) where the launch has enough
- *                      windows for them; the kernels of MLSTM_PATH_SPLIT for everything else.  The number of windows
+ *                      windows for them; where the heads fill the chip a chain kernel, which makes the state recurrence and H / dV
+ *                      in one launch (more than 256 positions, DHQK 64, 128 or 256; no head norm; forward: not with states updated
+ *                      in place); a forward without a backward of a short sequence in one launch; the kernels of
+ *                      MLSTM_PATH_SPLIT for everything else.  The number of windows
  *                      and heads (batch included) has a part in the choice, and so has the number of CUs: the last bits
  *                      of a sequence's results may depend on what it is batched with.  With the other paths they do not.
  *   MLSTM_PATH_SPLIT : state scan + chunk-parallel kernel over materialised chunk states
@@ -185,14 +188,15 @@ int mlstm_hip_chunkwise_fw(const void* q, const void* k, const void* v, const vo
  * of a full-size workspace and calls mlstm_hip_chunkwise_recompute_states, which runs the forward state scan again
  * and writes the chunk states behind them (k, v, c0, dtype_qkv, state_stride as in the forward call; c0 NULL = zero
  * initial state).  The workspace is then what mlstm_hip_chunkwise_bw expects.  The recomputed states equal the
- * forward's bit for bit when the forward returned no last state (c_last NULL); a forward that returned it carried a
+ * forward's bit for bit when the forward returned no last state (c_last NULL); a scan that returned it carried a
  * remainder of the value operand in its late chunks, and the recomputed states of those chunks differ from the
  * forward's by one 16-bit rounding of that operand.
  * A forward with MLSTM_PATH_AUTO cuts its scan into segments where few heads meet a long sequence, and keeps their fp32
- * states in H meanwhile.  For equal bits its recomputation takes a scratch buffer of H's size
+ * states in H meanwhile; where many heads do it takes the chain kernel (see MLSTM_PATH_AUTO), which carries the remainder always, and
+ * notes that in the workspace.  For equal bits its recomputation takes a scratch buffer of H's size
  * (mlstm_hip_chunkwise_recompute_states_scratch; the dV that the backward writes next serves), that of a forward with
- * another path takes none (scratch NULL, or the first form).  Without the scratch the scan runs in one piece, and the fp32
- * states in front of the rounding differ in the order of a sum.
+ * another path takes none (scratch NULL, or the first form).  Without the scratch the scan runs, in one piece: the fp32
+ * states in front of the rounding differ in the order of a sum, from the chain kernel's by the remainder.
  */
 size_t mlstm_hip_chunkwise_fw_saved_bytes(int B, int NH, int S, int DHQK, int DHHV);
 int mlstm_hip_chunkwise_recompute_states(const void* k, const void* v, const float* c0,

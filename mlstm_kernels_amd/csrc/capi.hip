@@ -274,13 +274,33 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   sf.sig_gate = sig;
   sf.use_nrow = track_n;
   sf.f16 = f16; sf.dtype_gates = dtype_gates;
-  const bool use_short = path == MLSTM_PATH_AUTO && !keep_for_backward && !in_place && head_norm == MLSTM_NORM_NONE &&
-                         (n_last == nullptr || c_last != nullptr) && mlstm::short_fw_preferred(sf, BH);
+  const bool one_launch = path == MLSTM_PATH_AUTO && !in_place && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr);
+  const bool use_short = one_launch && !keep_for_backward && mlstm::short_fw_preferred(sf, BH);
   sf.own_gates = use_short && mlstm::short_fw_own_gates(sf, BH);
+  mlstm::ChainHvArgs ca;
+  memset(&ca, 0, sizeof(ca));
+  ca.Q = (const uint16_t*)q; ca.K = (const uint16_t*)k; ca.V = (const uint16_t*)v;
+  ca.g = ws.g;
+  ca.init = c0;
+  ca.n_init = n0;
+  ca.states = keep_for_backward ? ws.cstates : nullptr;
+  ca.Out = (uint16_t*)H;
+  ca.nrow_out = ws.nrow;
+  ca.n_out = n_out; ca.m_out = m_out;
+  ca.final_out = c_last;
+  ca.n_final = track_n ? n_last : nullptr;
+  ca.S = S; ca.NC = NC; ca.DHQK = DHQK; ca.DHHV = DHHV;
+  ca.qk_scale = 1.0f / sqrtf((float)DHQK); ca.eps = eps;
+  ca.sig_gate = sig;
+  ca.use_nrow = track_n;
+  ca.stride = stride;
+  ca.f16 = f16;
+  ca.skip_zero = !has_c0;  // (both dQ / dK kernels know, from g.zero_c)
+  const bool use_chain = one_launch && !use_short && mlstm::chain_hv_preferred(ca, BH);
   if (!sf.own_gates) {
     {
       ProfileScope ps("gates", st);
-      if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, !has_c0, st)) return fail(e);
+      if (const char* e = mlstm::launch_gates(i, f, m0, ws.g, m_last, B, NH, S, dtype_gates, sig, !has_c0, use_chain, st)) return fail(e);
     }
     if (check_launch("gates")) return 1;
   }
@@ -338,33 +358,12 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
     return check_launch("short_fw");
   }
 
-  if (path == MLSTM_PATH_AUTO && !in_place && head_norm == MLSTM_NORM_NONE && (n_last == nullptr || c_last != nullptr)) {
-    mlstm::ChainHvArgs ca;
-    memset(&ca, 0, sizeof(ca));
-    ca.Q = (const uint16_t*)q; ca.K = (const uint16_t*)k; ca.V = (const uint16_t*)v;
-    ca.g = ws.g;
-    ca.init = c0;
-    ca.n_init = n0;
-    ca.states = keep_for_backward ? ws.cstates : nullptr;
-    ca.Out = (uint16_t*)H;
-    ca.nrow_out = ws.nrow;
-    ca.n_out = n_out; ca.m_out = m_out;
-    ca.final_out = c_last;
-    ca.n_final = track_n ? n_last : nullptr;
-    ca.S = S; ca.NC = NC; ca.DHQK = DHQK; ca.DHHV = DHHV;
-    ca.qk_scale = 1.0f / sqrtf((float)DHQK); ca.eps = eps;
-    ca.sig_gate = sig;
-    ca.use_nrow = track_n;
-    ca.stride = stride;
-    ca.f16 = f16;
-    ca.skip_zero = !has_c0;  // (both dQ / dK kernels know, from g.zero_c)
-    if (mlstm::chain_hv_preferred(ca, BH)) {
-      {
-        ProfileScope ps("chain_h", st);
-        if (const char* e = mlstm::launch_chain_hv(ca, BH, /*is_dv=*/false, st)) return fail(e);
-      }
-      return check_launch("chain_hv forward");
+  if (use_chain) {
+    {
+      ProfileScope ps("chain_h", st);
+      if (const char* e = mlstm::launch_chain_hv(ca, BH, /*is_dv=*/false, st)) return fail(e);
     }
+    return check_launch("chain_hv forward");
   }
 
   mlstm::ParHvArgs pa;
@@ -473,8 +472,30 @@ int mlstm_hip_chunkwise_recompute_states_scratch(const void* k, const void* v, c
   mlstm::FwWorkspace ws = mlstm::carve_fw_workspace(workspace, B, NH, S, DHQK, DHHV, true, stride);
   if (workspace_bytes < ws.bytes) return fail("mlstm_hip_chunkwise_recompute_states: workspace too small");
   hipStream_t st = (hipStream_t)stream;
+  // What the forward ran is in its workspace.  Where the shape leaves the choice to a flag on the device both kernels are launched,
+  // and one of them ends at once.
+  mlstm::ChainHvArgs ca;
+  memset(&ca, 0, sizeof(ca));
+  ca.K = (const uint16_t*)k; ca.V = (const uint16_t*)v;
+  ca.g = ws.g;
+  ca.init = c0;
+  ca.states = ws.cstates;
+  ca.S = S; ca.NC = (S + 127) / 128; ca.DHQK = DHQK; ca.DHHV = DHHV;
+  ca.qk_scale = 1.0f / sqrtf((float)DHQK);
+  ca.stride = stride;
+  ca.f16 = dtype_qkv == MLSTM_F16;
+  ca.skip_zero = c0 == nullptr;
+  const bool may_chain = scratch != nullptr && mlstm::chain_hv_preferred(ca, B * NH);
+  if (may_chain) {
+    {
+      ProfileScope ps("chain_states", st);
+      if (const char* e = mlstm::launch_chain_states(ca, B * NH, st)) return fail(e);
+    }
+    if (check_launch("chain_states")) return 1;
+  }
   mlstm::ScanArgs sa;
   memset(&sa, 0, sizeof(sa));
+  if (may_chain) sa.unless = ws.g.chained;
   sa.X = (const uint16_t*)k;
   sa.Y = (const uint16_t*)v;
   sa.scale_a = ws.g.abar;

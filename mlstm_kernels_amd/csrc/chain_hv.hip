@@ -148,8 +148,18 @@ __device__ __forceinline__ int unit_ofs(int u0, int u, int sw) {
 template <bool TIGHT>
 __device__ __forceinline__ int lane_of(int lane) { return TIGHT ? opaque(lane) : lane; }
 
-template <int DQ, int W, bool IS_DV, bool F16>
+// What a launch makes.  kKeptStates: the forward's kept states and nothing else, for a backward that has them recomputed: the same
+// arithmetic in the same order, hence the same bits, which the scan, rounding the scaled value rows once, does not have.  us, the whole
+// forward / the scan / this: 128 heads of 256/512, 2048 positions 341 / 154 / 174, 1024 147 / 70 / 74; 256 heads of 1024, 128/256 102 / 48 /
+// 50, 64/128 62 / 20 / 28.  (The scan's launch, which then ends at once, 6 us.)
+enum Kind { kForward, kBackward, kKeptStates };
+
+template <int DQ, int W, int KIND, bool F16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void chain_hv_kernel(ChainHvArgs a) {
+  constexpr bool IS_DV = KIND == kBackward, ROWS = KIND != kKeptStates;  // ROWS: H or dV is made
+  if constexpr (!ROWS) {
+    if (__builtin_amdgcn_readfirstlane(*a.g.chained) == 0) return;  // the forward's states came from the scan
+  }
   using L = ChainLds<DQ, W>;
   constexpr int G = L::G, DS = L::DS;
   constexpr int NDT = DQ / 32 / DS;         // 32-row state tiles of a wave
@@ -174,7 +184,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int S = a.S, NC = a.NC, DHHV = a.DHHV;
   const size_t Sp = (size_t)NC * kChunk;
   const int NS = (S + kStep - 1) / kStep;
-  const bool do_n = !IS_DV && a.use_nrow;
+  const int n_run = ROWS ? NS : 2 * ((NC - 1) / a.stride * a.stride) + 1;  // steps: up to the last kept state
+  const bool do_n = KIND == kForward && a.use_nrow;
   const u32x4 Xn_d = row_desc((IS_DV ? a.K : a.Q) + (size_t)bh * S * DQ, (uint32_t)S * DQ * 2);
   const u32x4 Xo_d = row_desc((IS_DV ? a.Q : a.K) + (size_t)bh * S * DQ, (uint32_t)S * DQ * 2);
   const u32x4 Xw_d = row_desc((IS_DV ? a.dH : a.V) + (size_t)bh * S * DHHV + w_tile, ((uint32_t)S * DHHV - w_tile) * 2);
@@ -262,7 +273,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto load_n = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xn_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
   auto load_o = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xo_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
   auto load_w = [&](int s) { DmaTile<W * 2>::load(Xw_d, w_off + (uint32_t)s * (kStep * 2) * (uint32_t)DHHV, DHHV * 2, lds0 + L::kV, wave); };
-  load_n(s_first, o_n);
+  if constexpr (ROWS) load_n(s_first, o_n);
   load_o(s_first, o_o);
   load_w(s_first);
   float gs = 0.f;
@@ -270,7 +281,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     gs = gates_load(s_first);
     dma_wait();
     gates_store(s_first, gs);
-    if (NS > 1) gs = gates_load(s_first + s_inc);
+    if (n_run > 1) gs = gates_load(s_first + s_inc);
   }
   dma_wait();
 
@@ -285,13 +296,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float log2_qk = __log2f(a.qk_scale);
   const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
 
-  for (int it = 0; it < NS; ++it) {
+  for (int it = 0; it < n_run; ++it) {
     const int s = s_first + it * s_inc, t0 = s * kStep;
     const int c = s >> 1;
-    const bool more = it + 1 < NS;
+    const bool more = it + 1 < n_run;
     const float* const v = vec + (s & 1) * 320;
     __syncthreads();  // ---- the tiles and vectors of this step are in LDS, the free tile is nobody's
-    if (more) load_n(s + s_inc, o_f);
+    if (more) {
+      if constexpr (ROWS) load_n(s + s_inc, o_f);
+      else load_o(s + s_inc, o_f);
+    }
     const uint16_t* const Xn = (const uint16_t*)(smem + o_n);
     const uint16_t* const Xo = (const uint16_t*)(smem + o_o);
 
@@ -310,10 +324,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     if (more && wave == 6) {
       gates_store(s + s_inc, gs);
-      if (it + 2 < NS) gs = gates_load(s + 2 * s_inc);
+      if (it + 2 < n_run) gs = gates_load(s + 2 * s_inc);
     }
     // ---- scores: P (other index, position), gated, rounded, to LDS as operand fragments
-    if (sc_cnt > 0) {
+    if (ROWS && sc_cnt > 0) {
       const int ln = lane_of<kTight>(lane);
       const int m16 = ln & 15, qq = ln >> 4;
       const int o16a = IS_DV ? 3 - sc_o : sc_o, o16b = IS_DV ? 2 - sc_o : sc_o + 1;
@@ -390,7 +404,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ---- q . n in float32, a quarter of the head dimension by each of the waves with few or no scores (lane = position; the parts
     // of n would be denormal float16 values)
-    if (!IS_DV && F16 && wave >= 4) {
+    if (KIND == kForward && F16 && wave >= 4) {
       const int ln = lane_of<kTight>(lane);
       const float* nw = nv + (wave - 4) * (DQ / 4);
       const uint16_t* qr = Xn + ln * DQ;
@@ -425,55 +439,57 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ---- product with the state: out[k] = position tile (DS == 1: k, else the wave's own one first)
     f32x16 out[2];
+    if constexpr (ROWS) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) out[k][i] = 0.f;
-    {
-      const int ln = lane_of<kTight>(lane);
-      const int rr = ln & 31, hh = ln >> 5;
-      // a wave's rows start at unit 4 tg0: an even number of 16-unit blocks, or (few head dimensions) an XOR on the unit
-      constexpr int UB = DQ * 2 == 128 ? 8 : 16;
-      const int u0 = 4 * tg0;
-      const uint16_t* x0 = Xn + (32 * (DS == 1 ? 0 : dq) + rr) * DQ + (u0 / UB) * (UB * 8);
-      const uint16_t* x1 = Xn + (32 * (DS == 1 ? 1 : 1 - dq) + rr) * DQ + (u0 / UB) * (UB * 8);
-      const int sw = swz<DQ * 2>(rr) ^ (u0 % UB);
-      Frag f[2][2][2];
-      auto fetch = [&](int dt) {
+        for (int i = 0; i < 16; ++i) out[k][i] = 0.f;
+      {
+        const int ln = lane_of<kTight>(lane);
+        const int rr = ln & 31, hh = ln >> 5;
+        // a wave's rows start at unit 4 tg0: an even number of 16-unit blocks, or (few head dimensions) an XOR on the unit
+        constexpr int UB = DQ * 2 == 128 ? 8 : 16;
+        const int u0 = 4 * tg0;
+        const uint16_t* x0 = Xn + (32 * (DS == 1 ? 0 : dq) + rr) * DQ + (u0 / UB) * (UB * 8);
+        const uint16_t* x1 = Xn + (32 * (DS == 1 ? 1 : 1 - dq) + rr) * DQ + (u0 / UB) * (UB * 8);
+        const int sw = swz<DQ * 2>(rr) ^ (u0 % UB);
+        Frag f[2][2][2];
+        auto fetch = [&](int dt) {
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const int o = unit_ofs<DQ * 2>(4 * dt, 2 * hf + hh, sw);
-          f[dt & 1][hf][0].u = *(const uint4*)(x0 + o);
-          f[dt & 1][hf][1].u = *(const uint4*)(x1 + o);
+          for (int hf = 0; hf < 2; ++hf) {
+            const int o = unit_ofs<DQ * 2>(4 * dt, 2 * hf + hh, sw);
+            f[dt & 1][hf][0].u = *(const uint4*)(x0 + o);
+            f[dt & 1][hf][1].u = *(const uint4*)(x1 + o);
+          }
+        };
+        Frag A[2];
+        auto round = [&](int i) {
+#pragma unroll
+          for (int p = 0; p < 4; ++p) A[i & 1].w[p] = pack2<F16>(acc[i >> 1][8 * (i & 1) + 2 * p], acc[i >> 1][8 * (i & 1) + 2 * p + 1]);
+        };
+        fetch(0);
+        round(0);
+        fence();
+#pragma unroll
+        for (int i = 0; i < 2 * NDT; ++i) {
+          if (i % 2 == 0 && i / 2 + 1 < NDT) fetch(i / 2 + 1);
+          mfma32<F16>(out[0], A[i & 1], f[(i >> 1) & 1][i & 1][0]);
+          mfma32<F16>(out[1], A[i & 1], f[(i >> 1) & 1][i & 1][1]);
+          if (i + 1 < 2 * NDT) round(i + 1);
         }
-      };
-      Frag A[2];
-      auto round = [&](int i) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) A[i & 1].w[p] = pack2<F16>(acc[i >> 1][8 * (i & 1) + 2 * p], acc[i >> 1][8 * (i & 1) + 2 * p + 1]);
-      };
-      fetch(0);
-      round(0);
-      fence();
-#pragma unroll
-      for (int i = 0; i < 2 * NDT; ++i) {
-        if (i % 2 == 0 && i / 2 + 1 < NDT) fetch(i / 2 + 1);
-        mfma32<F16>(out[0], A[i & 1], f[(i >> 1) & 1][i & 1][0]);
-        mfma32<F16>(out[1], A[i & 1], f[(i >> 1) & 1][i & 1][1]);
-        if (i + 1 < 2 * NDT) round(i + 1);
+        for (int i = 0; i < 4 * NDT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
+        fence();
       }
+      if constexpr (DS == 2) {  // the other half of the sum over the head dimension belongs to the partner wave
+        float4* ex = (float4*)(smem + L::kEx + wave * 4096) + lane;
 #pragma unroll
-      for (int i = 0; i < 4 * NDT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        for (int k = 0; k < 4; ++k) ex[64 * k] = make_float4(out[1][4 * k], out[1][4 * k + 1], out[1][4 * k + 2], out[1][4 * k + 3]);
       }
-      fence();
-    }
-    if constexpr (DS == 2) {  // the other half of the sum over the head dimension belongs to the partner wave
-      float4* ex = (float4*)(smem + L::kEx + wave * 4096) + lane;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) ex[64 * k] = make_float4(out[1][4 * k], out[1][4 * k + 1], out[1][4 * k + 2], out[1][4 * k + 3]);
     }
     // ---- kept state: before every stride-th chunk (forward), after the last chunk of every group (dV)
     if (a.states != nullptr) {
@@ -499,113 +515,115 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     __syncthreads();  // ---- scores, partial sums; the output-side rows and the value rows have been read
-    float4 ex[4];
-    if constexpr (DS == 2) {
-      const float4* src = (const float4*)(smem + L::kEx + (wave ^ G) * 4096) + lane_of<kTight>(lane);
+    if constexpr (ROWS) {
+      float4 ex[4];
+      if constexpr (DS == 2) {
+        const float4* src = (const float4*)(smem + L::kEx + (wave ^ G) * 4096) + lane_of<kTight>(lane);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) ex[k] = src[64 * k];
-    }
-    // denominators (lane = position)
-    float cs = v[192 + lane], ivl = 1.f;
-    {
-      const float mc = IS_DV ? 0.f : v[256 + lane];
-      float d[12];
-      if (!IS_DV) {
-#pragma unroll
-        for (int x = 0; x < 8; ++x) d[x] = rs[64 * x + lane];
-#pragma unroll
-        for (int x = 0; x < (F16 ? 4 : 1); ++x) d[8 + x] = qn[64 * x + lane];
+        for (int k = 0; k < 4; ++k) ex[k] = src[64 * k];
       }
-      if (!IS_DV) {
-        float nmax = 1.f;
-        if (do_n) {
-          const float q = F16 ? (d[8] + d[9]) + (d[10] + d[11]) : d[8];
-          const float sum = cs * q + (((d[0] + d[1]) + (d[2] + d[3])) + ((d[4] + d[5]) + (d[6] + d[7])));
-          nmax = fmaxf(fabsf(sum), a.sig_gate ? 1.f : __expf(-mc));
-          ivl = 1.f / (nmax + a.eps);
+      // denominators (lane = position)
+      float cs = v[192 + lane], ivl = 1.f;
+      {
+        const float mc = IS_DV ? 0.f : v[256 + lane];
+        float d[12];
+        if (!IS_DV) {
+#pragma unroll
+          for (int x = 0; x < 8; ++x) d[x] = rs[64 * x + lane];
+#pragma unroll
+          for (int x = 0; x < (F16 ? 4 : 1); ++x) d[8 + x] = qn[64 * x + lane];
         }
-        if (blk.x == 0 && wave == 7) {
-          a.nrow_out[bh * Sp + t0 + lane] = nmax;
-          // the second half of the last chunk, if no step covers it
-          if (s == NS - 1 && (s & 1) == 0) a.nrow_out[bh * Sp + t0 + kStep + lane] = 1.f;
-          if (t0 + lane < S) {
-            if (a.n_out != nullptr) a.n_out[(size_t)bh * S + t0 + lane] = nmax;
-            if (a.m_out != nullptr) a.m_out[(size_t)bh * S + t0 + lane] = mc;
+        if (!IS_DV) {
+          float nmax = 1.f;
+          if (do_n) {
+            const float q = F16 ? (d[8] + d[9]) + (d[10] + d[11]) : d[8];
+            const float sum = cs * q + (((d[0] + d[1]) + (d[2] + d[3])) + ((d[4] + d[5]) + (d[6] + d[7])));
+            nmax = fmaxf(fabsf(sum), a.sig_gate ? 1.f : __expf(-mc));
+            ivl = 1.f / (nmax + a.eps);
           }
-        }
-      }
-    }
-    // from lane = position to lane = position of the wave's tiles, in both halves of the wave
-    float csk[NO], iv[NO];
-    {
-      const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(cs), __float_as_uint(cs), false, false);
-      const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(ivl), __float_as_uint(ivl), false, false);
-#pragma unroll
-      for (int k = 0; k < NO; ++k) {
-        csk[k] = __uint_as_float(DS == 1 ? x[k] : (dq ? x[1] : x[0]));
-        iv[k] = __uint_as_float(DS == 1 ? y[k] : (dq ? y[1] : y[0]));
-      }
-    }
-    if constexpr (DS == 2) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        out[0][4 * k] += ex[k].x; out[0][4 * k + 1] += ex[k].y; out[0][4 * k + 2] += ex[k].z; out[0][4 * k + 3] += ex[k].w;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NO; ++k)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) out[k][i] *= csk[k];
-    // ---- product inside the step
-    {
-      const uint4* pf = (const uint4*)(smem + L::kP) + lane_of<kTight>(lane);
-      if constexpr (DS == 1) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-          for (int ks = 0; ks < 4; ++ks) {
-            if (IS_DV ? ks < 2 * k : ks >= 2 * (k + 1)) continue;
-            Frag b;
-            b.u = pf[(ks + 2 * k) * 64];
-            mfma32<F16>(out[k], vf[ks], b);
-          }
-      } else {
-#pragma unroll
-        for (int x = 0; x < 2; ++x)  // the diagonal block, then the other one where there is one
-          if (x == 0 || dq == (IS_DV ? 0 : 1))
-#pragma unroll
-            for (int y = 0; y < 2; ++y) {
-              Frag b;
-              b.u = pf[(2 * (x ^ dq) + y + 2 * dq) * 64];
-              mfma32<F16>(out[0], vf[2 * x + y], b);
+          if (blk.x == 0 && wave == 7) {
+            a.nrow_out[bh * Sp + t0 + lane] = nmax;
+            // the second half of the last chunk, if no step covers it
+            if (s == NS - 1 && (s & 1) == 0) a.nrow_out[bh * Sp + t0 + kStep + lane] = 1.f;
+            if (t0 + lane < S) {
+              if (a.n_out != nullptr) a.n_out[(size_t)bh * S + t0 + lane] = nmax;
+              if (a.m_out != nullptr) a.m_out[(size_t)bh * S + t0 + lane] = mc;
             }
+          }
+        }
       }
-    }
-    if (more) load_o(s + s_inc, o_n);
-    // ---- output rows: lane (h, r) holds columns 8 x + 4 h + 0 .. 3 of position r; first the halves of the wave trade, so that it
-    // holds eight neighbouring ones, then its rows of 16 lanes, so that four lanes hold the 32 columns of a position
-    {
-      uint16_t* const orow = a.Out + ((size_t)bh * S + t0) * DHHV + w_tile + 32 * g + 8 * h + (lane & 16);
+      // from lane = position to lane = position of the wave's tiles, in both halves of the wave
+      float csk[NO], iv[NO];
+      {
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(cs), __float_as_uint(cs), false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(ivl), __float_as_uint(ivl), false, false);
 #pragma unroll
-      for (int k = 0; k < NO; ++k) {
-        uint32_t w[8], o[2][4];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) w[x] = pack2<F16>(out[k][2 * x] * iv[k], out[k][2 * x + 1] * iv[k]);
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          const auto p = __builtin_amdgcn_permlane32_swap(w[4 * x], w[4 * x + 2], false, false);
-          const auto q = __builtin_amdgcn_permlane32_swap(w[4 * x + 1], w[4 * x + 3], false, false);
-          o[x][0] = p[0]; o[x][1] = q[0]; o[x][2] = p[1]; o[x][3] = q[1];
+        for (int k = 0; k < NO; ++k) {
+          csk[k] = __uint_as_float(DS == 1 ? x[k] : (dq ? x[1] : x[0]));
+          iv[k] = __uint_as_float(DS == 1 ? y[k] : (dq ? y[1] : y[0]));
         }
+      }
+      if constexpr (DS == 2) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const auto p = __builtin_amdgcn_permlane16_swap(o[0][x], o[1][x], false, false);
-          o[0][x] = p[0]; o[1][x] = p[1];
+        for (int k = 0; k < 4; ++k) {
+          out[0][4 * k] += ex[k].x; out[0][4 * k + 1] += ex[k].y; out[0][4 * k + 2] += ex[k].z; out[0][4 * k + 3] += ex[k].w;
         }
+      }
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          const int n = 32 * (DS == 1 ? k : dq) + 16 * x + (lane & 15);
-          if (t0 + n < S) *(u32x4*)(orow + (size_t)n * DHHV) = u32x4{o[x][0], o[x][1], o[x][2], o[x][3]};
+      for (int k = 0; k < NO; ++k)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) out[k][i] *= csk[k];
+      // ---- product inside the step
+      {
+        const uint4* pf = (const uint4*)(smem + L::kP) + lane_of<kTight>(lane);
+        if constexpr (DS == 1) {
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+              if (IS_DV ? ks < 2 * k : ks >= 2 * (k + 1)) continue;
+              Frag b;
+              b.u = pf[(ks + 2 * k) * 64];
+              mfma32<F16>(out[k], vf[ks], b);
+            }
+        } else {
+#pragma unroll
+          for (int x = 0; x < 2; ++x)  // the diagonal block, then the other one where there is one
+            if (x == 0 || dq == (IS_DV ? 0 : 1))
+#pragma unroll
+              for (int y = 0; y < 2; ++y) {
+                Frag b;
+                b.u = pf[(2 * (x ^ dq) + y + 2 * dq) * 64];
+                mfma32<F16>(out[0], vf[2 * x + y], b);
+              }
+        }
+      }
+      if (more) load_o(s + s_inc, o_n);
+      // ---- output rows: lane (h, r) holds columns 8 x + 4 h + 0 .. 3 of position r; first the halves of the wave trade, so that it
+      // holds eight neighbouring ones, then its rows of 16 lanes, so that four lanes hold the 32 columns of a position
+      {
+        uint16_t* const orow = a.Out + ((size_t)bh * S + t0) * DHHV + w_tile + 32 * g + 8 * h + (lane & 16);
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+          uint32_t w[8], o[2][4];
+#pragma unroll
+          for (int x = 0; x < 8; ++x) w[x] = pack2<F16>(out[k][2 * x] * iv[k], out[k][2 * x + 1] * iv[k]);
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const auto p = __builtin_amdgcn_permlane32_swap(w[4 * x], w[4 * x + 2], false, false);
+            const auto q = __builtin_amdgcn_permlane32_swap(w[4 * x + 1], w[4 * x + 3], false, false);
+            o[x][0] = p[0]; o[x][1] = q[0]; o[x][2] = p[1]; o[x][3] = q[1];
+          }
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const auto p = __builtin_amdgcn_permlane16_swap(o[0][x], o[1][x], false, false);
+            o[0][x] = p[0]; o[1][x] = p[1];
+          }
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const int n = 32 * (DS == 1 ? k : dq) + 16 * x + (lane & 15);
+            if (t0 + n < S) *(u32x4*)(orow + (size_t)n * DHHV) = u32x4{o[x][0], o[x][1], o[x][2], o[x][3]};
+          }
         }
       }
     }
@@ -613,6 +631,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float gdec = gdl[2 * (s & 1)];  // 1 where the decay is left in sigma
     // ---- state update, the scaled value rows as a 16-bit head and remainder; wave w takes rows 32 w .. of the normaliser state
     {
+      constexpr bool N = KIND == kForward;  // (nothing reads n behind the other two)
       const int ln = lane_of<kTight>(lane);
       const int i16 = ln & 15, kr = i16 >> 2;
       const int gp = ((i16 & 1) << 1) | ((i16 >> 1) & 1);  // the two middle groups of four rows trade places
@@ -632,8 +651,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // Operands are read kAhead state tiles ahead; the scaled value rows of the next 16 positions are made, a quarter at a time,
       // between the matrix instructions of these.
       constexpr int NT = 4 * NDT, kAhead = 3;
-      constexpr int kReads = 2 + ((IS_DV ? 2 : 4) + NDT - 1) / NDT;
-      constexpr int kValu = ((IS_DV ? 40 : 56) + 2 * NDT - 1) / (2 * NDT);
+      constexpr int kReads = 2 + ((N ? 4 : 2) + NDT - 1) / NDT;
+      constexpr int kValu = ((N ? 56 : 40) + 2 * NDT - 1) / (2 * NDT);
       Frag A[4], xn, vh[2], vl[2];
       float4 u0, u1;
       auto row0 = [&](int j) { return (j < 2 ? kb0 : kb1) + 16 * (j & 1); };
@@ -644,7 +663,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       auto weights = [&](int j) {
         u0 = *(const float4*)(us + row0(j));
         u1 = *(const float4*)(us + row0(j) + 4);
-        if (!IS_DV) xn = tr_frag(nlo + row0(j) * DQ, nhi + row0(j) * DQ);
+        if (N) xn = tr_frag(nlo + row0(j) * DQ, nhi + row0(j) * DQ);
       };
       auto scale = [&](int j, int p) {
         const float x = p == 0 ? u0.x : p == 1 ? u0.z : p == 2 ? u1.x : u1.z, y = p == 0 ? u0.y : p == 1 ? u0.w : p == 2 ? u1.y : u1.w;
@@ -653,7 +672,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if constexpr (F16) asm("" : "+v"(e0), "+v"(e1));
         vh[j & 1].w[p] = pack2<F16>(e0, e1);
         vl[j & 1].w[p] = pack2<F16>(e0 - lo2<F16>(vh[j & 1].w[p]), e1 - hi2<F16>(vh[j & 1].w[p]));
-        if (!IS_DV) {
+        if (N) {
           nsum = __builtin_fmaf(lo2<F16>(xn.w[p]), x, nsum);
           nsum = __builtin_fmaf(hi2<F16>(xn.w[p]), y, nsum);
         }
@@ -693,7 +712,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
       }
       fence();
-      if (!IS_DV) {
+      if (N) {
         nsum += __shfl_xor(nsum, 32);
         const int d = 32 * ntile + (ln & 31);
         const float nn = gdec * nv[d] + nsum;
@@ -705,7 +724,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     dma_wait();
     const uint32_t x = o_o;
-    o_o = o_n;
+    o_o = ROWS ? o_n : o_f;
     o_n = o_f;
     o_f = x;
   }
@@ -726,19 +745,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 namespace {
-template <int DQ, int W, bool IS_DV, bool F16>
+template <int DQ, int W, int KIND, bool F16>
 const char* launch_t(const ChainHvArgs& a, int BH, hipStream_t stream) {
   static LdsLimit lds;
   constexpr int smem = ChainLds<DQ, W>::kBytes;
   static_assert(smem <= 160 * 1024, "LDS of a CU");
-  if (!lds.allow((const void*)chain_hv_kernel<DQ, W, IS_DV, F16>, smem)) return "chain_hv: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((chain_hv_kernel<DQ, W, IS_DV, F16>), dim3(a.DHHV / W, BH), dim3(512), smem, stream, a);
+  if (!lds.allow((const void*)chain_hv_kernel<DQ, W, KIND, F16>, smem)) return "chain_hv: cannot raise the dynamic LDS limit";
+  hipLaunchKernelGGL((chain_hv_kernel<DQ, W, KIND, F16>), dim3(a.DHHV / W, BH), dim3(512), smem, stream, a);
   return nullptr;
 }
+template <int DQ, int W, int KIND>
+const char* launch_f(const ChainHvArgs& a, int BH, hipStream_t stream) {
+  return a.f16 ? launch_t<DQ, W, KIND, true>(a, BH, stream) : launch_t<DQ, W, KIND, false>(a, BH, stream);
+}
 template <int DQ, int W>
-const char* launch_w(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
-  if (is_dv) return a.f16 ? launch_t<DQ, W, true, true>(a, BH, stream) : launch_t<DQ, W, true, false>(a, BH, stream);
-  return a.f16 ? launch_t<DQ, W, false, true>(a, BH, stream) : launch_t<DQ, W, false, false>(a, BH, stream);
+const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream) {
+  if (kind == kBackward) return launch_f<DQ, W, kBackward>(a, BH, stream);
+  return kind == kForward ? launch_f<DQ, W, kForward>(a, BH, stream) : launch_f<DQ, W, kKeptStates>(a, BH, stream);
 }
 // Value columns of a workgroup, 0: another kernel is the better one.
 //  * One workgroup takes a CU and the launch as long as its rounds: the last one has to be nearly full.  256 columns are the more
@@ -770,17 +793,21 @@ int columns(const ChainHvArgs& a, int BH) {
 
 bool chain_hv_preferred(const ChainHvArgs& a, int BH) { return columns(a, BH) != 0; }
 
-const char* launch_chain_hv(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
+static const char* launch(const ChainHvArgs& a, int BH, int kind, hipStream_t stream) {
   if (a.stride < 1 || a.stride > kMaxStateStride) return "chain_hv: state stride out of range";
   switch (columns(a, BH) * 1000 + a.DHQK) {
-    case 256256: return launch_w<256, 256>(a, BH, is_dv, stream);
-    case 256128: return launch_w<128, 256>(a, BH, is_dv, stream);
-    case 256064: return launch_w<64, 256>(a, BH, is_dv, stream);
-    case 128256: return launch_w<256, 128>(a, BH, is_dv, stream);
-    case 128128: return launch_w<128, 128>(a, BH, is_dv, stream);
-    case 128064: return launch_w<64, 128>(a, BH, is_dv, stream);
+    case 256256: return launch_w<256, 256>(a, BH, kind, stream);
+    case 256128: return launch_w<128, 256>(a, BH, kind, stream);
+    case 256064: return launch_w<64, 256>(a, BH, kind, stream);
+    case 128256: return launch_w<256, 128>(a, BH, kind, stream);
+    case 128128: return launch_w<128, 128>(a, BH, kind, stream);
+    case 128064: return launch_w<64, 128>(a, BH, kind, stream);
     default: return "chain_hv: unsupported shape";
   }
 }
+const char* launch_chain_hv(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
+  return launch(a, BH, is_dv ? kBackward : kForward, stream);
+}
+const char* launch_chain_states(const ChainHvArgs& a, int BH, hipStream_t stream) { return launch(a, BH, kKeptStates, stream); }
 
 }  // namespace mlstm

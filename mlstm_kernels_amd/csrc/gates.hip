@@ -34,9 +34,9 @@ constexpr int kGateChunks = kGateThreads / kWave;  // chunks per workgroup: one 
 
 __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
     const void* __restrict__ ig, const void* __restrict__ fg, const float* __restrict__ m0, GateBufs gb, int S, int NC,
-    int dtype_gates, int sig_gate, int zero_c) {
+    int dtype_gates, int sig_gate, int zero_c, int chained) {
   const int bh = blockIdx.y;
-  if (bh == 0 && blockIdx.x == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
+  if (bh == 0 && blockIdx.x == 0 && threadIdx.x == 0) *gb.zero_c = zero_c, *gb.chained = chained;
   // m before the first chunk, for all workgroups of gates_finish_kernel: one of them writes m_last, which may be m0
   if (blockIdx.x == 0 && threadIdx.x == 0)
     gb.mstates[(size_t)bh * (NC + 1)] = !sig_gate && m0 != nullptr ? fmaxf(m0[bh], -__builtin_inff()) : 0.f;
@@ -60,10 +60,10 @@ __global__ __launch_bounds__(kGateThreads) void gates_scan_kernel(
 // gates_finish_kernel).
 __global__ __launch_bounds__(kGateThreads) void gates_whole_kernel(
     const void* __restrict__ ig, const void* __restrict__ fg, const float* m0, GateBufs gb, float* m_last, int S, int NC,
-    int dtype_gates, int sig_gate, int zero_c) {
+    int dtype_gates, int sig_gate, int zero_c, int chained) {
   __shared__ float gs[kGateChunks], as[kGateChunks];
   const int bh = blockIdx.y;
-  if (bh == 0 && threadIdx.x == 0) *gb.zero_c = zero_c;
+  if (bh == 0 && threadIdx.x == 0) *gb.zero_c = zero_c, *gb.chained = chained;
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;  // one wave per chunk
   const float NEG_INF = -__builtin_inff();
   const float m_init = !sig_gate && m0 != nullptr ? m0[bh] : 0.f;
@@ -204,15 +204,15 @@ __global__ __launch_bounds__(kGateThreads) void gates_finish_kernel(GateBufs gb,
 }
 
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
-                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, hipStream_t stream) {
+                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, int chained, hipStream_t stream) {
   const int NC = (S + kChunk - 1) / kChunk;
   if (NC <= kGateChunks) {
     hipLaunchKernelGGL(gates_whole_kernel, dim3(1, B * NH), dim3(kWave * NC), 0, stream, i, f, m0, gb, m_last, S, NC, dtype_gates,
-                       sig_gate, zero_c);
+                       sig_gate, zero_c, chained);
     return nullptr;
   }
   const dim3 grid((NC + kGateChunks - 1) / kGateChunks, B * NH);
-  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, m0, gb, S, NC, dtype_gates, sig_gate, zero_c);
+  hipLaunchKernelGGL(gates_scan_kernel, grid, dim3(kGateThreads), 0, stream, i, f, m0, gb, S, NC, dtype_gates, sig_gate, zero_c, chained);
   hipLaunchKernelGGL(gates_finish_kernel, grid, dim3(kGateThreads), 0, stream, gb, m_last, NC, sig_gate);
   return nullptr;
 }

@@ -77,6 +77,7 @@ struct ScanArgs {
   int part;               // 0 whole sequence; 1 / 2 the two launches of a forward scan that returns the last state
   int n_bh;               // batch * heads
   int by_batch;           // the kernels may be chosen by the number of heads (a path that the caller names: not)
+  const int* unless;      // device flag, nullptr: none; set: nothing is to be done (whole sequence without the last state only)
   int repeat_all;         // (launch_scan) late chunks always run twice
   int with_backward;      // this is a call with a backward, or the backward
   int nseg, seg_len;      // segments of the sequence, chunks in each (the last one may be shorter)
@@ -226,7 +227,7 @@ struct StepBlockArgs {
 bool step_block_supported(int DHQK, int DHHV, int dtype_qkv);
 const char* launch_step_block(const StepBlockArgs& a, hipStream_t stream);
 const char* launch_gates(const void* i, const void* f, const float* m0, const GateBufs& gb, float* m_last,
-                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, hipStream_t stream);
+                         int B, int NH, int S, int dtype_gates, int sig_gate, int zero_c, int chained, hipStream_t stream);
 const char* launch_scan(const ScanArgs& a, int BH, bool hilo, hipStream_t stream);
 const char* launch_par_hv(const ParHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 bool par_hv_head_norm_supported(int DHHV);
@@ -245,6 +246,7 @@ const char* launch_short_fw(const ShortFwArgs& a, int BH, hipStream_t stream);
 const char* launch_head_norm_bw(const HeadNormBwArgs& a, hipStream_t stream);
 bool chain_hv_preferred(const ChainHvArgs& a, int BH);
 const char* launch_chain_hv(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream);
+const char* launch_chain_states(const ChainHvArgs& a, int BH, hipStream_t stream);  // kept states only, if g.chained is set
 bool fused_hv_supported(int DHQK, int DHHV);
 const char* launch_fused_hv(const FusedHvArgs& a, int BH, bool is_dv, hipStream_t stream);
 const char* launch_par_qk_pair(const ParQkArgs& a, int BH, hipStream_t stream);

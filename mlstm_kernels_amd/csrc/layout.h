@@ -5,6 +5,7 @@
 //   per chunk      gbar, amax, graw            3 x fp32 [B*NH][NC]
 //   whole call     zero_c                      one int: the state before the first chunk is zero (its slot among the
 //                                              chunk states is then not written)
+//                  chained                     one int: the chunk states are those of the chain kernel, not of the scan
 //   stabiliser     mstates                     fp32 [B*NH][NC+1]   (index c = value before chunk c)
 //   normaliser     nstates                     fp32 [B*NH][NC][3][DHQK] (n before chunk c, as three partial vectors
 //                                              to be added up: the scan accumulates them on the matrix cores)
@@ -29,6 +30,7 @@ constexpr int kMaxStateStride = 8;  // chunk states are kept every 1 .. 8 chunks
 struct GateBufs {
   float *u, *w, *abar, *bbar, *mcomb, *gbar, *amax, *mstates;
   int* zero_c;  // whether the initial state is zero: the backward is not told, and its kernels leave out what it gives
+  int* chained;  // whether the chain kernel made the chunk states: a recomputation runs what the forward ran
   float* graw;  // per chunk: sum of logsig(f) over the chunk (input of the scan over chunks that yields gbar)
 };
 
@@ -71,7 +73,8 @@ inline FwWorkspace carve_fw_workspace(void* base, int B, int NH, int S, int DHQK
   w.g.amax = (float*)take(BH * NC * 4);
   w.g.mstates = (float*)take(BH * (NC + 1) * 4);
   w.g.graw = (float*)take(BH * NC * 4);
-  w.g.zero_c = (int*)take(4);
+  w.g.zero_c = (int*)take(8);
+  w.g.chained = w.g.zero_c + 1;
   w.nstates = (float*)take(BH * NC * 3 * DHQK * 4);
   w.nrow = (float*)take(BH * Sp * 4);
   w.cstates = with_states ? (uint16_t*)take(BH * NCS * (size_t)DHQK * DHHV * 2) : nullptr;

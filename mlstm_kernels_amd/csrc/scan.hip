@@ -753,6 +753,9 @@ __device__ __forceinline__ void scan_consumer(const ScanArgs& a, const uint16_t*
 // 330 -> 302, 128 heads of 2048, 128/256 500 -> 487; 128 heads of 2048 with the last state, forward 418 -> 416.
 template <int RT, int WT, bool F16, bool REP, bool SEG, bool MANY>
 __global__ __launch_bounds__(128 * (RT / 64) * (WT / 32)) void scan_roles_kernel(ScanArgs a, int n_rounds) {
+  if constexpr (!REP) {
+    if (a.unless != nullptr && __builtin_amdgcn_readfirstlane(*a.unless) != 0) return;
+  }
   constexpr int WC = WT / 32;
   constexpr int NWC = (RT / 64) * WC;     // consumer waves (and as many producer waves)
   constexpr int NTP = 64 * NWC;           // producer threads

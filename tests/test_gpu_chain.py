@@ -120,3 +120,41 @@ def test_closed_gates():
         ref, (Cr, nr, mr) = O.recurrent_sequence(d(q), d(k), d(v), d(i), d(f), torch.zeros(1, 1, DQ, DV, dtype=torch.float64),
                                                  torch.zeros(1, 1, DQ, dtype=torch.float64), torch.zeros(1, 1, 1, dtype=torch.float64))
         assert rel_norm(d(H), ref) <= 6e-3 and rel_norm(d(C), Cr) <= 1e-3 and rel_norm(d(n), nr) <= 1e-3
+
+
+@pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 700), (64, 256, 256, 300), (128, 128, 128, 1025), (128, 256, 256, 641), (256, 128, 128, 512),
+                                           (256, 512, 256, 600)])
+@pytest.mark.parametrize("opt", [dict(), dict(stride=1, f_offset=9.0), dict(stride=3, init=True, last=True), dict(dtype=torch.float16, f_offset=9.0),
+                                 dict(sig=True, normalize=False, init=True), dict(norm="layer")], ids=str)
+def test_recomputed_states_are_the_kept_ones(DQ, DV, width, S, opt):
+    """recompute_states_in_bw: the gradients are bit for bit those of the kept states, whichever kernel made them (a head norm keeps
+    the forward from this one)."""
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    BH, dtype, init, norm = _heads(DV, width), opt.get("dtype", torch.bfloat16), opt.get("init", False), opt.get("norm", "none")
+    print(f"{BH} x {S} {DQ}/{DV} {opt}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), opt.get("f_offset", 3.0) + rn(S)]
+    dH, state = rn(S, DV).to(dtype), (rn(DQ, DV), rn(DQ), rn(1)) if init else (None, None, None)
+    grads, names = [], []
+    for recompute in (False, True):
+        leaves = [t.clone().requires_grad_(True) for t in x]
+        kw = dict(c_initial=state[0], n_initial=state[1], return_last_states=opt.get("last", False), any_sequence_length=True,
+                  chunk_size_intra=128 * opt.get("stride", 2), recompute_states_in_bw=recompute, head_norm=norm)
+        _lib.profile_read()
+        _lib.profile_enable(True)
+        try:
+            if opt.get("sig"):
+                out = mlstm_siging_chunkwise__hip_xl_chunk(*leaves, normalize=opt.get("normalize", True), **kw)
+            else:
+                out = mlstm_chunkwise__hip_xl_chunk(*leaves, m_initial=state[2], **kw)
+            H = out[0] if opt.get("last") else out
+            grads.append((H.detach(), *torch.autograd.grad(H, leaves, dH)))
+        finally:
+            _lib.profile_enable(False)
+        names.append(set(_lib.profile_read()))
+    assert ("chain_h" in names[0]) == (norm == "none") and "scan_fw_recompute" in names[1]
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
