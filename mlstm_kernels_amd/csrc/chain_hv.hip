@@ -20,8 +20,9 @@
 //   * The value rows are scaled in fp32 and enter the state as a 16-bit head and remainder: the state is rounded every 64 positions
 //     for the product with it, and that alone is what it loses.  Errors against 64 bits, scan + H / dV here before and now: H 2.353e-3 /
 //     2.360e-3, dQ 2.330e-3 / 2.323e-3, dK 2.324e-3 / 2.317e-3, dF 4.9e-3 / 3.9e-3, C 1.99e-6 / 1.98e-6 (128 heads of 256/512, bf16).
-//   * The decay of the state is left in a factor (sigma) until it reaches 2^-24, then multiplied in; weights take the factor.
-//     float16 operands have no room for that and take the decay in every step.
+//   * The state takes its decay in every step.  Left in a factor until that reaches 2^-24, with weights that take it, the registers hold
+//     up to 2^24 times the state, which overflows with rows of 2^103 and above; and it gains nothing (us, forward, backward, so / now: 128
+//     heads of 256/512, 2048 positions 331 303 / 334 306, 256 heads of 1024, 128/256 103 97 / 102 96, 128/128 75 70 / 74 69, 64/128 61 60 / 59 60).
 // What bounds it: issue.  A step of 256 / 256 columns is 150 matrix and 900 vector instructions for the two waves of a SIMD, which
 // overlap only where they are interleaved (a matrix instruction hides about six of its wave: the schedules below); matrix pipes 42 %,
 // LDS 30 %, HBM half of what it gives.  us, forward / backward, scan + H (dV) and this: 256/512, 128 heads of 2048 with the last
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* const raw = vec + 640;                 // [5][64]
   float* const rs = raw + 320;                  // [8][64] row sums of P: two waves a position, four lanes each
   float* const qn = rs + 512;                   // [4][64] shares of q . n (bfloat16: one)
-  float* const gdl = qn + 256;                  // [2][2] factor on the state in a step, sigma before it; sigma after the last
+  float* const gdl = qn + 256;                  // [2] decay of the state in a step
   float* const nv = gdl + 8;                    // [DQ] normaliser state
   uint16_t* const npt = (uint16_t*)(nv + DQ);   // [3][DQ] the same as three 16-bit parts (bfloat16)
 
@@ -235,7 +236,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     return *p;
   };
   // ... and what they become: weights relative to the middle of the chunk, whose stabiliser is the combined one of position 63
-  float sigma = 1.f;
   auto gates_store = [&](int s, float gs) {
     const int ln = opaque(lane), c = s >> 1, odd = s & 1;
     const bool single = S - c * kChunk <= kStep;
@@ -244,28 +244,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float gu = raw[ln], gw = raw[64 + ln], gx = raw[256 + ln];
     const float A = odd || single ? raw[128 + ln] : expf(u63 - gw);  // weight of k v^T in the state after the step
     const float B = odd ? expf(gu - u63) : raw[192 + ln];            // weight of the state before the step
-    const float before = sigma, after = before * (odd ? expf(gg - u63 - gm) : gg);
-    const bool last = IS_DV ? s < 4 : s >= NS - 4;
-    const float mult = last || after < (F16 ? 1.f : 0x1p-24f) ? after : 1.f;
-    sigma = mult == after ? 1.f : after;
-    const float inv = 1.f / sigma;
     float* v = vec + (s & 1) * 320 + ln;
     v[0] = gu;
     v[64] = gw;
     if (IS_DV) {
       const float rho = in ? (a.use_nrow ? 1.f / (gx + a.eps) : 1.f) : 0.f;
-      v[128] = in ? B * a.qk_scale * rho * inv : 0.f;
-      v[192] = A * before;
+      v[128] = in ? B * a.qk_scale * rho : 0.f;
+      v[192] = A;
       v[256] = rho;
     } else {
-      v[128] = in ? A * inv : 0.f;
-      v[192] = B * a.qk_scale * before;
+      v[128] = in ? A : 0.f;
+      v[192] = B * a.qk_scale;
       v[256] = gx;
     }
-    if (ln == 0) {
-      gdl[2 * (s & 1)] = mult;
-      gdl[2 * (s & 1) + 1] = before;
-    }
+    if (ln == 0) gdl[s & 1] = odd ? expf(gg - u63 - gm) : gg;
   };
 
   const int s_first = IS_DV ? NS - 1 : 0, s_inc = IS_DV ? -1 : 1;
@@ -496,7 +488,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const bool chunk_start = IS_DV ? (s & 1) != 0 || s == NS - 1 : (s & 1) == 0;
       const bool keep = chunk_start && (IS_DV ? c == NC - 1 || (c + 1) % a.stride == 0 : c % a.stride == 0);
       if (keep && !(it == 0 && a.skip_zero)) {
-        const float sg = gdl[2 * (s & 1) + 1];
         u32x4* dst = (u32x4*)a.states + (((size_t)bh * NCS + c / a.stride) * (size_t)(DHHV / 32) + (w_tile >> 5) + g) * ND * 64 +
                      (size_t)tg0 * 128 + lane;
 #pragma unroll
@@ -505,7 +496,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           for (int hf = 0; hf < 2; ++hf) {
             uint32_t w[4];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) w[p] = pack2<F16>(acc[dt][8 * hf + 2 * p] * sg, acc[dt][8 * hf + 2 * p + 1] * sg);
+            for (int p = 0; p < 4; ++p) {
+              float e0 = acc[dt][8 * hf + 2 * p], e1 = acc[dt][8 * hf + 2 * p + 1];
+              asm("" : "+v"(e0), "+v"(e1));  // rounded once more: kept from the product they cost its registers (a quarter of the time)
+              w[p] = pack2<F16>(e0, e1);
+            }
             // rows 8 h + e -> rows 8 (e / 4) + 4 h + e % 4: the halves of the wave trade the middle groups of four
             const auto x = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
             const auto y = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
@@ -628,7 +623,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     if (more) load_w(s + s_inc);
-    const float gdec = gdl[2 * (s & 1)];  // 1 where the decay is left in sigma
+    const float gdec = gdl[s & 1];
     // ---- state update, the scaled value rows as a 16-bit head and remainder; wave w takes rows 32 w .. of the normaliser state
     {
       constexpr bool N = KIND == kForward;  // (nothing reads n behind the other two)
@@ -680,12 +675,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       weights(0);
 #pragma unroll
       for (int i = 0; i < kAhead; ++i) fetch(i);
-      if (__builtin_amdgcn_readfirstlane(__float_as_uint(gdec)) != 0x3f800000u) {
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
+      for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) acc[dt][i] *= gdec;
-      }
+        for (int i = 0; i < 16; ++i) acc[dt][i] *= gdec;
 #pragma unroll
       for (int p = 0; p < 4; ++p) scale(0, p);
       weights(1);
@@ -729,18 +722,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     o_f = x;
   }
 
-  if (wave == 6 && lane == 0) gdl[4] = sigma;
   __syncthreads();
-  const float sg = gdl[4];
   if (a.final_out != nullptr) {
     float* dst = a.final_out + ((size_t)bh * DQ + 32 * tg0 + 8 * h) * DHHV + w_tile + 32 * g + r;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dst[(size_t)(32 * dt + 16 * (i / 8) + i % 8) * DHHV] = acc[dt][i] * sg;
+      for (int i = 0; i < 16; ++i) dst[(size_t)(32 * dt + 16 * (i / 8) + i % 8) * DHHV] = acc[dt][i];
   }
   if (do_n && a.n_final != nullptr && blk.x == 0) {
-    for (int d = tid; d < DQ; d += 512) a.n_final[(size_t)bh * DQ + d] = nv[d] * sg;
+    for (int d = tid; d < DQ; d += 512) a.n_final[(size_t)bh * DQ + d] = nv[d];
   }
 }
 

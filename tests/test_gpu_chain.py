@@ -158,3 +158,31 @@ def test_recomputed_states_are_the_kept_ones(DQ, DV, width, S, opt):
     assert ("chain_h" in names[0]) == (norm == "none") and "scan_fw_recompute" in names[1]
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 700), (64, 256, 256, 1500), (128, 128, 128, 1500), (128, 256, 256, 700), (256, 128, 128, 700),
+                                           (256, 512, 256, 1500)])
+@pytest.mark.parametrize("name,power", [("v", 104), ("dH", 104), ("v", -80), ("dH", -80)])
+def test_range_of_values(DQ, DV, width, S, name, power):
+    """What is linear in v or dH scales with a power of two exactly, also where the state is within a few powers of two of the largest
+    float32 value: nothing that the kernels hold is larger than the state."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    BH = _heads(DV, width)
+    print(f"{BH} x {S} {DQ}/{DV} {name} {power}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).bfloat16(), rn(S, DQ).bfloat16(), rn(S, DV).bfloat16(), rn(S), 3 + rn(S)]
+    dH, state = rn(S, DV).bfloat16(), (rn(DQ, DV), rn(DQ), rn(1))
+    scale = 2.0 ** power
+    out = []
+    for factor in (1.0, scale):
+        y = [t * factor if j == 2 and name == "v" else t for j, t in enumerate(x)]
+        c0 = state[0] * factor if name == "v" else state[0]
+        leaves = [t.clone().requires_grad_(True) for t in y]
+        H, (C, n, m) = mlstm_chunkwise__hip_xl_chunk(*leaves, c0, *state[1:], return_last_states=True, any_sequence_length=True)
+        out.append((H.detach(), C.detach(), *torch.autograd.grad(H, leaves, dH * factor if name == "dH" else dH)))
+    linear = (True, True, True, True, False, True, True) if name == "v" else (False, False) + (True,) * 5
+    for what, a, b, lin in zip(("H", "C", "dQ", "dK", "dV", "dI", "dF"), *out, linear):
+        assert bool(torch.isfinite(b).all()), what
+        assert torch.equal(a * scale if lin else a, b), what
