@@ -759,6 +759,8 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //    efficient form (256/512, 96 heads of 1024, 192 workgroups: 170 us against 140 for scan + H; 128 heads 170 / 207: the line is at
 //    85 %); with 128 the state's rows are shared by two waves that both scale the value rows, and what is gained is less (128/256,
 //    128 heads 158 / 146, at 112 heads 138 / 146).  At 256/512 they gain nothing (64 heads of 1000: 102 / 101).
+//  * Rows move to LDS in pieces of 16 bytes without registers in between, which asks for addresses that are multiples of 16; the
+//    other kernels read theirs with ordinary loads, which do not.
 //  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 124 / 148, backward
 //    93 / 137); at 320 128 heads take 74 / 50 and 68 / 47.
 //  * Where the streaming kernels are the alternative, calls of more than 2^18 token-heads stay with them: at these sizes every
@@ -769,6 +771,8 @@ int columns(const ChainHvArgs& a, int BH) {
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return 0;
   if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return 0;  // 32-bit offsets in a head
   if (a.S <= 2 * kChunk) return 0;
+  // (dV reads no V, the kept states no Q)
+  if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V)) % 16 != 0) return 0;
   if (a.DHQK == 256 && a.DHHV % 512 == 0 && (long long)BH * a.S > kMostRows) return 0;
   const int cus = device_cu_count();
   if (cus <= 0) return 0;

@@ -674,7 +674,9 @@ bool short_fw_preferred(const ShortFwArgs& a, int BH) {
 // 8 heads of 256/512, 64 positions 14.0 / 11.0 (of which the host takes all), 317 17.5 / 13.5, 512 28.5 / 26.4, 317 from a state
 // 20.6 / 16.4; 16 heads of 317 26.0 / 24.0 (1.75 workgroups a CU), 32 of 64 15.1 / 13.8 (1.5), 128 heads of 128/256 of 100 positions 22.1 /
 // 21.8 (3.0), 32 of 317 42.1 / 41.9 (3.5), 64 of 200 55.4 / 58.0 (6.0), 512 of 64 124.7 / 153.3 (24).
+// (H goes out in write-through stores of 16 bytes, which take addresses that are multiples of 16.)
 bool short_fw_own_gates(const ShortFwArgs& a, int BH) {
+  if ((uintptr_t)a.Out % 16 != 0) return false;
   const long long cw = a.DHHV % 128 == 0 ? 128 : 64, rt = a.DHQK % 128 == 0 ? 128 : 64;
   const long long tiles = (a.S + 63) / 64 + (a.final_out == nullptr ? 0 : a.DHQK / rt);
   return BH * tiles * (a.DHHV / cw) <= 3ll * device_cu_count();

@@ -264,7 +264,8 @@ const char* launch_step(const void* q, const void* k, const void* v, const void*
   // 12 MB where a workgroup has 32 KB (64/128, 32 x 8 5.8 / 6.3), and with slices of 128 KB (256/512, 16 x 8 20.6 / 23.0).  With more than
   // the cache holds it is memory either way (128/256, 64 x 16, other states in between 53.3 / 57.3).
   const size_t slice_bytes = (size_t)128 * (DHQK < 256 ? DHQK : 256) * (sbf ? 2 : 4);
-  const bool through = slice_bytes <= 65536 && state_bytes > ((size_t)(slice_bytes <= 32768 ? 12 : 32) << 20) && state_bytes <= ((size_t)112 << 20);
+  // (Stores of 16 bytes: at multiples of 16 only.)
+  const bool through = (uintptr_t)c_out % 16 == 0 && slice_bytes <= 65536 && state_bytes > ((size_t)(slice_bytes <= 32768 ? 12 : 32) << 20) && state_bytes <= ((size_t)112 << 20);
 #define MLSTM_STEP_ROWS(MODE_)                                       \
   {                                                                  \
     if (DHHV <= 64 && DHQK < 128) MLSTM_STEP_PICK(64, 16, 4, MODE_)  \
