@@ -1114,7 +1114,7 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
     const bool wide = r128 && w128;
     const int fit = device_cu_count() / (BH * tiles);
     const bool halves = wide && 2ll * BH * tiles <= device_cu_count();  // (see below)
-    const float one_piece = wide ? (halves ? 4.f + 1.6f * a.NC : 12.f + 1.9f * a.NC) : 12.f + 1.57f * a.NC;
+    const float one_piece = wide ? (halves ? 4.f + 1.6f * a.NC : 12.f + 1.9f * a.NC) : 12.f + (r128 ? 1.4f : 1.57f) * a.NC;
     float best = a.with_backward ? fminf(0.9f * one_piece, one_piece - 8.f) : 0.9f * one_piece;
     int len = 0;
     for (int n = 2; n <= (wide ? 8 : 16) && n <= fit && a.by_batch; ++n) {
@@ -1130,18 +1130,19 @@ const char* launch_scan(const ScanArgs& a_in, int BH, bool hilo, hipStream_t str
       a.nseg = (a.NC + len - 1) / len;
     }
     // Late chunks in a second run whatever their number: sequences of four chunks; where the kernels may be chosen by the heads
-    // of the call, a scan in one piece up to 24 chunks, or of any number while the tiles do not fill the chip (not with the
-    // sigmoid gate, where all chunks are late, and tiles that do), and one in segments, whose other kernel would walk the late chunks
-    // of all segments in one piece.  (Not the segments of more than eight narrow tiles up to 33 chunks: a call whose states are written
-    // in place, which alone keeps it from segments, has the bits of one that is not at those lengths, and then only the other kernel
-    // has them where many chunks are late.  There the empty segments in front cost what they do: 32 heads of 64/64, 2000 positions, one piece
-    // and its second launch / segments, last chunk late 56.6 / 49.3, all late 81.2 / 87.6; 12 of 4000 85.8 / 56.9, 133 / 141.)
-    // us for a forward with the last state, a launch more / so, the last chunk late / all of them: 256/512,
-    // 8 heads of 700 49.3 52.2 / 39.5 44.4, of 2000 56.4 82.6 / 54.0 70.2, of 10000 201 370 / 199 257, 64 of 1000 117.5 149.9 / 112.4 132.3, 96 of
-    // 3000 448 558 / 446 547; 64/64, 4 heads of 1000 37.2 50.3 / 35.7 45.4, of 10000 63.3 282 / 60.1 71.3; 16 of 128/256, 4000 81.0 149 / 78.7 86.7; but 96
-    // of 8000 all late 1386 / 1414, and sigmoid gate, 64 of 4000 473 / 487.
+    // of the call, all in segments, whose other kernel would walk the late chunks of all segments in one piece; a scan in one piece up
+    // to 24 chunks, or of any number while the tiles do not fill the chip; with the sigmoid gate, where all chunks are late, while they do not
+    // and the rows that run twice are few.
+    // us for a forward with the last state, a launch more / so, the last chunk late / all of them: in one piece, 256/512, 8 heads of 700
+    // 49.3 52.2 / 39.5 44.4, of 2000 56.4 82.6 / 54.0 70.2, 64 of 1000 117.5 149.9 / 112.4 132.3, 96 of 3000 448 558 / 446 547, but 96 of 8000 all
+    // late 1386 / 1414; 64/64, 4 heads of 1000 37.2 50.3 / 35.7 45.4.  In segments, 256/512, 8 heads of 10000 201 370 / 199 257; 16 of
+    // 128/256, 4000 81.0 149 / 78.7 86.7; 64/64, 4 heads of 10000 63.3 282 / 60.1 71.3, 12 of 4000 56.9 141 / 54.2 57.1, 32 of 2000 49.3 87.6 / 46.4
+    // 48.7; 64/128, 64 of 4000 124 183 / 121 144; 128/64, 32 of 3000 74.5 121 / 72.3 75.3 (these three in one piece and a launch more 81 to 186 with
+    // all late).  Sigmoid gate in one piece: 128/128, 40 heads of 2000 87.0 / 83.3, 256/512, 8 of 2600 98.7 / 91.5, 256/256, 24 of 2600 136.7 /
+    // 134.8, but 256/512, 24 of 1100 68.9 / 70.7, 256/256, 40 of 1100 66.8 / 68.6, 128/256, 64 of 2000 105.1 / 109.4, 256/512, 64 of 4000 473 / 487.
     const bool fills = (long long)BH * tiles >= device_cu_count();
-    const bool one_launch = len == 0 ? !fills || (a.NC <= 24 && !a.all_remainder) : a.seg != nullptr && (wide || a.NC > 33 || BH * tiles <= 8);
+    const bool rows = wide && (long long)BH * (a.DHQK + a.DHHV) >= 48ll * device_cu_count();
+    const bool one_launch = len > 0 ? a.seg != nullptr : a.all_remainder ? !fills && !rows : !fills || a.NC <= 24;
     a.repeat_all = a.NC <= 4 || (a.by_batch && one_launch);
   }
   // Tiles of half the width where those of both halves still have a CU each: the walk over the chunks is what the launch

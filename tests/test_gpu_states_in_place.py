@@ -61,11 +61,12 @@ def test_named_paths(path, sig, normalize):
         assert torch.equal(a, b), name
 
 
-# a head's gates in several workgroups, all of which need the first m, and scan + H (not in segments) either way: the same bits
+# a head's gates in several workgroups, all of which need the first m, and scan + H (with so many heads not in segments) either way:
+# the same bits
 @pytest.mark.parametrize("S", [2048, 2049, 4100])
-@pytest.mark.parametrize("DQ,DV", [(64, 64), (256, 512)])
-def test_gates_of_several_workgroups(S, DQ, DV):
-    got, ref = (_forward(S, DQ, DV, in_place=p, NH=12, seed=S, f_offset=12.0) for p in (True, False))
+@pytest.mark.parametrize("DQ,DV,NH", [(64, 64, 140), (256, 512, 20)])
+def test_gates_of_several_workgroups(S, DQ, DV, NH):
+    got, ref = (_forward(S, DQ, DV, in_place=p, NH=NH, seed=S, f_offset=12.0) for p in (True, False))
     for name, a, b in zip(("H", "C", "n", "m"), got, ref):
         assert torch.equal(a, b), name
 
@@ -73,7 +74,7 @@ def test_gates_of_several_workgroups(S, DQ, DV):
 # Few heads and a long sequence: the scan in segments, which all read the initial state, is not taken in place.  The states are
 # those of the scan in one piece (which a named path takes), H that of separate buffers but for the order of a sum in fp32.  Gates
 # near one: the initial state still weighs at the end.
-@pytest.mark.parametrize("S,DQ,DV,NH", [(8192, 128, 128, 2), (8200, 256, 512, 1)])
+@pytest.mark.parametrize("S,DQ,DV,NH", [(8192, 128, 128, 2), (8200, 256, 512, 1), (2048, 64, 64, 12), (4100, 64, 64, 12), (2049, 128, 64, 32)])
 @pytest.mark.parametrize("sig", [False, True])
 def test_long_sequences_of_few_heads(S, DQ, DV, NH, sig):
     kw = dict(NH=NH, sig=sig, seed=S, f_offset=12.0, share="Cn")
