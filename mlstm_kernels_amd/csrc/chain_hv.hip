@@ -763,17 +763,15 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //    other kernels read theirs with ordinary loads, which do not.
 //  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 124 / 148, backward
 //    93 / 137); at 320 128 heads take 74 / 50 and 68 / 47.
-//  * Where the streaming kernels are the alternative, calls of more than 2^18 token-heads stay with them: at these sizes every
-//    element of the results is held to an emulation that rounds where THOSE kernels round (the state every 256 positions, this one
-//    every 64: the same error by norm, in other elements).  This one would be the faster one there as well.
-constexpr long long kMostRows = 1 << 18;
+//  * Longer sequences and several rounds are no other matter.  256/512, a forward with the last state and forward and backward, with the
+//    scan and the streaming kernels / so: 128 heads of 2049 positions 464 / 308 and 1287 / 1087, of 8192 1535 / 1150 and 4496 / 3953,
+//    512 of 1024 800 / 618 and 2037 / 1918; 1024 of 512 841 / 660 and 1786 / 1813, the one size where they are level with a backward.
 int columns(const ChainHvArgs& a, int BH) {
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return 0;
   if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return 0;  // 32-bit offsets in a head
   if (a.S <= 2 * kChunk) return 0;
   // (dV reads no V, the kept states no Q)
   if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V)) % 16 != 0) return 0;
-  if (a.DHQK == 256 && a.DHHV % 512 == 0 && (long long)BH * a.S > kMostRows) return 0;
   const int cus = device_cu_count();
   if (cus <= 0) return 0;
   auto full = [&](int w, int pct) {

@@ -12,7 +12,11 @@ rows whose terms nearly cancel is then shown to be the operand format, not the k
 Grouping of the products (what decides which values get rounded): the state recurrences run in chunks of 128
 positions; outputs are formed per window of `stride` chunks from the state kept at the window's boundary and the
 score blocks of the whole window (stride 1: the plain chunkwise form).  The sequence length must be a multiple of the
-window.  The training call is emulated (no last state returned: the forward scan rounds its value operand once)."""
+window.  The training call is emulated (no last state returned: the forward scan rounds its value operand once).
+
+The chain kernel (`chain`), which makes the state recurrence and H / dV in one launch, runs the recurrences in steps of 64
+positions and forms H and dV per step from the state at its boundary; its scaled value rows enter the state as a 16-bit head and a
+16-bit remainder.  dQ and dK come from the kept states and windows as above."""
 from __future__ import annotations
 
 import torch
@@ -30,9 +34,13 @@ def rounder(dtype):
     return lambda x: x.to(dtype).to(torch.float64)
 
 
-def _scan_gates(i, f, siging):
-    """Per 128-chunk gate quantities (oracle/mlstm_ref.py::_chunk_gates): b inclusive cumsum of logsig(f), g its last
-    entry, a = g - b + itilde."""
+def _value_rows(rnd, chain):
+    return (lambda x: rnd(x) + rnd(x - rnd(x))) if chain else rnd
+
+
+def _scan_gates(i, f, siging, L0=L0):
+    """Per chunk (128 positions, or a step of the chain kernel) gate quantities (oracle/mlstm_ref.py::_chunk_gates): b inclusive
+    cumsum of logsig(f), g its last entry, a = g - b + itilde."""
     B, NH, S = i.shape
     NC = S // L0
     lf = F.logsigmoid(f).reshape(B, NH, NC, L0)
@@ -43,7 +51,7 @@ def _scan_gates(i, f, siging):
 
 
 def chunkwise_fw_rounded(q, k, v, i, f, c_initial=None, n_initial=None, m_initial=None, stride=1, eps=1e-6,
-                         siging=False, normalize=True, rnd=_identity, nmax_given=None):
+                         siging=False, normalize=True, rnd=_identity, nmax_given=None, chain=False):
     """Forward.  Returns H (rounded like the kernel's output), nmax (B,NH,S), the per-chunk states (unrounded fp64
     accumulators) C_all (B,NH,NC+1,DQK,DHV), n_all, m_all, the per-position combined stabiliser m_comb, nmax_own (the
     emulation's own row normalisers) and den_abs, the sum of the magnitudes of the terms of every denominator.  `nmax_given` (B,NH,S): row normalisers to divide by
@@ -52,13 +60,16 @@ def chunkwise_fw_rounded(q, k, v, i, f, c_initial=None, n_initial=None, m_initia
     comparison of the outputs is about the matrix arithmetic alone)."""
     B, NH, S, DQK = q.shape
     DHV = v.shape[-1]
-    W = L0 * stride
-    assert S % W == 0, "the emulation needs a sequence length that is a multiple of the window"
+    assert S % (128 * stride) == 0, "the emulation needs a sequence length that is a multiple of the window"
+    L0 = 64 if chain else 128
+    W = L0 if chain else L0 * stride
     NC = S // L0
+    rnd_v = _value_rows(rnd, chain)
     s = DQK ** -0.5
     dt = torch.float64
-    lf, it, b, g, a = _scan_gates(i, f, siging)
-    # ---- state scan in chunks of 128 (native/fw.py:88-121): the value operand is scaled in fp32 and rounded once
+    lf, it, b, g, a = _scan_gates(i, f, siging, L0)
+    # ---- state scan in chunks of 128 (native/fw.py:88-121): the value operand is scaled in fp32 and rounded once (chain: in steps,
+    # head and remainder)
     C = torch.zeros(B, NH, DQK, DHV, dtype=dt) if c_initial is None else c_initial.to(dt)
     n = torch.zeros(B, NH, DQK, dtype=dt) if n_initial is None else n_initial.to(dt)
     m = torch.zeros(B, NH, dtype=dt) if (m_initial is None or siging) else m_initial.to(dt).reshape(B, NH)
@@ -69,7 +80,7 @@ def chunkwise_fw_rounded(q, k, v, i, f, c_initial=None, n_initial=None, m_initia
         m_next = torch.zeros_like(m) if siging else torch.maximum(g[:, :, c] + m, a[:, :, c].max(-1).values)
         abar = torch.exp(a[:, :, c] - m_next[..., None])
         gbar = torch.exp(g[:, :, c] + m - m_next)
-        C = gbar[..., None, None] * C + k[:, :, sl].transpose(-1, -2) @ rnd(v[:, :, sl] * abar[..., None])
+        C = gbar[..., None, None] * C + k[:, :, sl].transpose(-1, -2) @ rnd_v(v[:, :, sl] * abar[..., None])
         if track_n:
             n = gbar[..., None] * n + (k[:, :, sl] * abar[..., None]).sum(-2)
         m = m_next
@@ -83,7 +94,7 @@ def chunkwise_fw_rounded(q, k, v, i, f, c_initial=None, n_initial=None, m_initia
     lfw, itw = lf.reshape(B, NH, S // W, W), it.reshape(B, NH, S // W, W)
     for w in range(S // W):
         sl = slice(w * W, (w + 1) * W)
-        c0 = w * stride
+        c0 = w * W // L0
         qc, kc, vc = q[:, :, sl], k[:, :, sl], v[:, :, sl]
         bw_ = lfw[:, :, w].cumsum(-1)
         logD = (bw_[..., :, None] - bw_[..., None, :]).masked_fill(~causal, float("-inf")) + itw[:, :, w][..., None, :]
@@ -110,21 +121,23 @@ def chunkwise_fw_rounded(q, k, v, i, f, c_initial=None, n_initial=None, m_initia
 
 
 def chunkwise_bw_rounded(q, k, v, i, f, dH, c_initial=None, n_initial=None, m_initial=None, stride=1, eps=1e-6,
-                         siging=False, normalize=True, rnd=_identity, nmax_given=None):
+                         siging=False, normalize=True, rnd=_identity, nmax_given=None, chain=False):
     """Backward (native/bw.py:67-198): returns dQ, dK, dV rounded like the kernels' outputs."""
     B, NH, S, DQK = q.shape
-    W = L0 * stride
+    L0 = 64 if chain else 128
+    W = 128 * stride
     NC = S // L0
     s = DQK ** -0.5
+    rnd_v = _value_rows(rnd, chain)
     fw = chunkwise_fw_rounded(q, k, v, i, f, c_initial, n_initial, m_initial, stride, eps, siging, normalize, rnd,
-                              nmax_given)
+                              nmax_given, chain)
     C_all, m_all = fw["C_all"], fw["m_all"]
     track_n = not (siging and not normalize)
     rho = 1.0 / (fw["nmax"] + eps) if track_n else torch.ones_like(fw["nmax"])
-    lf, it, b, g, a = _scan_gates(i, f, siging)
+    lf, it, b, g, a = _scan_gates(i, f, siging, L0)
     m_comb128 = fw["m_comb"].reshape(B, NH, NC, L0)
-    # ---- dC scan in chunks of 128 (bw.py:67-98): the dH rows are scaled in fp32 and rounded once; dC_all[c] is the
-    # gradient of the state after chunk c-1 (= before chunk c)
+    # ---- dC scan in chunks of 128 (bw.py:67-98): the dH rows are scaled in fp32 and rounded once (chain: as in the forward); dC_all[c]
+    # is the gradient of the state after chunk c-1 (= before chunk c)
     dC = torch.zeros_like(C_all[0])
     dC_all = [None] * (NC + 1)
     dC_all[NC] = dC
@@ -133,27 +146,32 @@ def chunkwise_bw_rounded(q, k, v, i, f, dH, c_initial=None, n_initial=None, m_in
         bbar = torch.exp(b[:, :, c] + m_all[c][..., None] - m_comb128[:, :, c])
         gbar = torch.exp(g[:, :, c] + m_all[c] - m_all[c + 1])
         sc = bbar * s * rho[:, :, sl]
-        dC = gbar[..., None, None] * dC + q[:, :, sl].transpose(-1, -2) @ rnd(dH[:, :, sl] * sc[..., None])
+        dC = gbar[..., None, None] * dC + q[:, :, sl].transpose(-1, -2) @ rnd_v(dH[:, :, sl] * sc[..., None])
         dC_all[c] = dC
     # ---- gradients per window (bw.py:153-198)
     dQ, dK, dV = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    causal = torch.ones(W, W, dtype=torch.bool).tril()
-    lfw, itw = lf.reshape(B, NH, S // W, W), it.reshape(B, NH, S // W, W)
-    for w in range(S // W):
+
+    def window(w, W):  # what a window of W positions has in common: its positions, states, decays and weights
         sl = slice(w * W, (w + 1) * W)
-        c0, c1 = w * stride, (w + 1) * stride
-        qc, kc, vc, dhc, rc = q[:, :, sl], k[:, :, sl], v[:, :, sl], dH[:, :, sl], rho[:, :, sl]
-        bw_ = lfw[:, :, w].cumsum(-1)
-        gw = bw_[..., -1]
-        logD = (bw_[..., :, None] - bw_[..., None, :]).masked_fill(~causal, float("-inf")) + itw[:, :, w][..., None, :]
+        c0, c1 = w * W // L0, (w + 1) * W // L0
+        bw_, it_ = lf.reshape(B, NH, S // W, W)[:, :, w].cumsum(-1), it.reshape(B, NH, S // W, W)[:, :, w]
+        causal = torch.ones(W, W, dtype=torch.bool).tril()
+        logD = (bw_[..., :, None] - bw_[..., None, :]).masked_fill(~causal, float("-inf")) + it_[..., None, :]
         m_comb = fw["m_comb"][:, :, sl]
         D = torch.exp(logD - m_comb[..., None])
         bbar = torch.exp(bw_ + m_all[c0][..., None] - m_comb)
-        abar = torch.exp((gw[..., None] - bw_) + itw[:, :, w] - m_all[c1][..., None])
-        Pv = rnd((qc @ kc.transpose(-1, -2)) * s * D * rc[..., None])      # score block of the dV kernel (rho folded in)
+        abar = torch.exp((bw_[..., -1:] - bw_) + it_ - m_all[c1][..., None])
+        return sl, D, bbar, abar, rnd(C_all[c0]), rnd(dC_all[c1])
+
+    WV = L0 if chain else W
+    for w in range(S // WV):
+        sl, D, _, abar, _, dCn = window(w, WV)
+        Pv = rnd((q[:, :, sl] @ k[:, :, sl].transpose(-1, -2)) * s * D * rho[:, :, sl][..., None])  # score block of dV (rho folded in)
+        dV[:, :, sl] = rnd(Pv.transpose(-1, -2) @ dH[:, :, sl] + (k[:, :, sl] @ dCn) * abar[..., None])
+    for w in range(S // W):
+        sl, D, bbar, abar, Cp, dCn = window(w, W)
+        qc, kc, vc, dhc, rc = q[:, :, sl], k[:, :, sl], v[:, :, sl], dH[:, :, sl], rho[:, :, sl]
         dS = rnd((dhc @ vc.transpose(-1, -2)) * s * D * rc[..., None])     # score block of the dQ/dK kernel
-        dCn, Cp = rnd(dC_all[c1]), rnd(C_all[c0])
-        dV[:, :, sl] = rnd(Pv.transpose(-1, -2) @ dhc + (kc @ dCn) * abar[..., None])
         dK[:, :, sl] = rnd(dS.transpose(-1, -2) @ qc + (vc @ dCn.transpose(-1, -2)) * abar[..., None])
         dQ[:, :, sl] = rnd(dS @ kc + (dhc @ Cp.transpose(-1, -2)) * (bbar * s * rc)[..., None])
     return dQ, dK, dV

@@ -186,3 +186,51 @@ def test_range_of_values(DQ, DV, width, S, name, power):
     for what, a, b, lin in zip(("H", "C", "dQ", "dK", "dV", "dI", "dF"), *out, linear):
         assert bool(torch.isfinite(b).all()), what
         assert torch.equal(a * scale if lin else a, b), what
+
+
+@pytest.mark.parametrize("DQ,DV,width", [(64, 128, 128), (64, 256, 256), (128, 128, 128), (128, 256, 256), (256, 128, 128), (256, 512, 256)])
+@pytest.mark.parametrize("opt", [dict(S=512), dict(S=1024), dict(S=768, stride=1, init=True), dict(S=512, sig=True, init=True),
+                                 dict(S=512, sig=True, normalize=False), dict(S=768, stride=3, dtype=torch.float16)], ids=str)
+def test_every_element_within_tolerance_of_the_rounding_emulation(DQ, DV, width, opt):
+    """H, dQ, dK, dV against the fp64 emulation that rounds what the kernels round, in steps of 64 positions (tests/rounding_emulation.py): every
+    element inside |x - ref| <= 2e-2 + 2e-2 |ref|.  The row normalisers are held to fp32 summation accuracy first and then handed to it."""
+    import rounding_emulation as R
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import hip_xl_chunk as X
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    BH, S, stride, dtype = _heads(DV, width), opt["S"], opt.get("stride", 2), opt.get("dtype", torch.bfloat16)
+    sig, normalize, init = opt.get("sig", False), opt.get("normalize", True), opt.get("init", False)
+    print(f"{BH} x {S} {DQ}/{DV} {opt}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S + DQ)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), opt.get("f_offset", 3.0) + rn(S)]
+    dH, st = rn(S, DV).to(dtype), (0.1 * rn(DQ, DV), 0.1 * rn(DQ), torch.zeros(1, BH, 1, device="cuda")) if init else (None,) * 3
+    leaves = [t.clone().requires_grad_(True) for t in x]
+    kw = dict(c_initial=st[0], n_initial=st[1], chunk_size_intra=128 * stride)
+    _names()
+    _lib.profile_enable(True)
+    try:
+        H = mlstm_siging_chunkwise__hip_xl_chunk(*leaves, normalize=normalize, **kw) if sig else mlstm_chunkwise__hip_xl_chunk(*leaves, m_initial=st[2], **kw)
+        got = (H, *torch.autograd.grad(H, leaves[:3], dH))
+    finally:
+        _lib.profile_enable(False)
+    assert {"chain_h", "chain_dv"} <= _names()
+    track_n = not (sig and not normalize)
+    _, qb, kb, vb, ib, fb, c0f, n0f, m0f = X._prep_inputs(*x, *st, sig)
+    n_kernel = torch.empty(1, BH, S, device="cuda")
+    X._fw_launch(qb, kb, vb, ib, fb, c0f, n0f, m0f, 1e-6, sig, normalize, False, False, _lib.PATH_AUTO, stride, n_out=n_kernel)
+    for h in (0, BH - 1):
+        d = lambda t: None if t is None else t.detach()[:, h:h + 1].double().cpu()
+        args, first = [d(t) for t in x], [d(t) for t in st]
+        ekw = dict(stride=stride, siging=sig, normalize=normalize, rnd=R.rounder(dtype), chain=True)
+        own = R.chunkwise_fw_rounded(*args, *first, **ekw)
+        nk = d(n_kernel) if track_n else None
+        if track_n:  # a sum of up to 64 + DHQK fp32 terms, and the state's own of up to S
+            assert float(((nk - own["nmax_own"]).abs() - (2e-6 * own["den_abs"] + 1e-6 * own["nmax_own"])).max()) <= 0
+        ref = (R.chunkwise_fw_rounded(*args, *first, nmax_given=nk, **ekw)["H"],
+               *R.chunkwise_bw_rounded(*args, d(dH), *first, nmax_given=nk, **ekw))
+        for name, a, b in zip(("H", "dQ", "dK", "dV"), got, ref):
+            worst = float(((d(a) - b).abs() / (2e-2 + 2e-2 * b.abs())).max())
+            print(f"  {name} head {h}: {worst:.2f} x the bound", flush=True)
+            assert worst <= 1, (name, h, worst)

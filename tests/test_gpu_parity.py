@@ -669,7 +669,8 @@ def test_chunkwise_every_element_within_tolerance_of_the_rounding_emulation(kw, 
     |x - ref| <= 2e-2 + 2e-2 |ref|, no allowance.  The elements that miss this bound against the exact oracle in the
     other tests are therefore the 16-bit operand format's, not the kernels'.  The row normalisers are held to fp32
     summation accuracy first (a denominator whose terms nearly cancel cannot be more accurate than that in fp32, and
-    the whole row scales with it), then handed to the emulation.  Split and stream paths, every state stride."""
+    the whole row scales with it), then handed to the emulation, which groups the products like the kernels that ran.  Split and
+    stream paths, every state stride, and the library's choice."""
     import rounding_emulation as R
 
     if kernel_variant.startswith("fused"):
@@ -692,11 +693,21 @@ def test_chunkwise_every_element_within_tolerance_of_the_rounding_emulation(kw, 
         c0, n0, m0 = 0.1 * rn(B, NH, DQK, DHV), 0.1 * rn(B, NH, DQK), torch.zeros(B, NH, 1, device=DEV)
     leaves = [t.clone().requires_grad_(True) for t in (q, k, v, i, f)]
     okw = dict(c_initial=c0, n_initial=n0, m_initial=m0, return_last_states=False, chunk_size=128)
-    H = sig_op(*leaves, normalize=normalize, **okw) if siging else exp_op(*leaves, **okw)
-    H.backward(dH)
-    # the kernels' own row normalisers (vecN_out of the reference's forward), from one more forward launch
     from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.chunkwise import hip_xl_chunk as X
+
+    _lib.profile_read()
+    _lib.profile_enable(True)
+    try:
+        H = sig_op(*leaves, normalize=normalize, **okw) if siging else exp_op(*leaves, **okw)
+        H.backward(dH)
+    finally:
+        _lib.profile_enable(False)
+    # many heads on the path of the library's choice: the chain kernel groups the products in steps of 64 positions
+    kernels = {"chain_h", "chain_dv"} & set(_lib.profile_read())
+    assert len(kernels) != 1 and not (kernels and not kernel_variant.startswith("auto"))
+    chain = bool(kernels)
+    # the kernels' own row normalisers (vecN_out of the reference's forward), from one more forward launch
 
     track_n = not (siging and not normalize)
     _, qb, kb, vb, ib, fb, c0f, n0f, m0f = X._prep_inputs(q, k, v, i, f, c0, n0, m0, siging)
@@ -709,7 +720,7 @@ def test_chunkwise_every_element_within_tolerance_of_the_rounding_emulation(kw, 
     for (b, h) in pairs:
         sl = lambda t: None if t is None else d64(t[b:b + 1, h:h + 1])
         args = (sl(q), sl(k), sl(v), sl(i), sl(f))
-        ekw = dict(stride=stride, siging=siging, normalize=normalize, rnd=rnd)
+        ekw = dict(stride=stride, siging=siging, normalize=normalize, rnd=rnd, chain=chain)
         nk = None
         if track_n:
             # a denominator is a sum of up to 128 * stride + DHQK fp32 terms: the kernel's and the emulation's agree to

@@ -280,7 +280,8 @@ def test_head_normalize_matches_library_routine_and_autograd(spec):
 @pytest.mark.parametrize("stride", [1, 2, 4])
 @pytest.mark.parametrize("siging,normalize,init", [(False, True, False), (False, True, True), (True, True, True),
                                                    (True, False, False)])
-def test_rounding_emulation_without_rounding_is_the_oracle(stride, siging, normalize, init):
+@pytest.mark.parametrize("chain", [False, True])
+def test_rounding_emulation_without_rounding_is_the_oracle(stride, siging, normalize, init, chain):
     """tests/rounding_emulation.py restates the chunkwise forward and backward with explicit rounding points and its
     own grouping (scans in chunks of 128, outputs per window of `stride` chunks).  With the identity as rounding
     function it must reproduce the oracle's H, row normaliser, dQ, dK and dV to fp64 accuracy."""
@@ -297,8 +298,8 @@ def test_rounding_emulation_without_rounding_is_the_oracle(stride, siging, norma
         m0 = torch.zeros(1, 2, 1, dtype=torch.float64)
     fw = O.chunkwise_fw(q, k, v, i, f, c0, n0, m0, chunk_size=64, siging=siging, normalize=normalize)
     bw = O.chunkwise_bw(q, k, v, i, f, dH, c0, n0, m0, chunk_size=64, siging=siging, normalize=normalize)
-    em = R.chunkwise_fw_rounded(q, k, v, i, f, c0, n0, m0, stride=stride, siging=siging, normalize=normalize)
-    dQ, dK, dV = R.chunkwise_bw_rounded(q, k, v, i, f, dH, c0, n0, m0, stride=stride, siging=siging, normalize=normalize)
+    em = R.chunkwise_fw_rounded(q, k, v, i, f, c0, n0, m0, stride=stride, siging=siging, normalize=normalize, chain=chain)
+    dQ, dK, dV = R.chunkwise_bw_rounded(q, k, v, i, f, dH, c0, n0, m0, stride=stride, siging=siging, normalize=normalize, chain=chain)
     assert torch.allclose(em["H"], fw["H"], rtol=1e-9, atol=1e-10)
     assert torch.allclose(em["nmax"], fw["n_out"], rtol=1e-9, atol=1e-12)
     for name, x, r in zip(["dQ", "dK", "dV"], [dQ, dK, dV], bw[:3]):
