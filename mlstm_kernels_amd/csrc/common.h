@@ -127,11 +127,6 @@ __device__ __forceinline__ float wave_sum(float x) {
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
   return x;
 }
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
-  return x;
-}
 
 __device__ __forceinline__ float log_sigmoid(float x) {
   // log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|))

@@ -262,16 +262,24 @@ const char* launch_step(const void* q, const void* k, const void* v, const void*
   // 64/128, 128 x 8 (32 MB) 17.1 / 15.1, 400 x 8 42.0 / 37.9; 16-bit states, 256/512 32 x 8 (64 MB) 28.9 / 27.6, 128/256 64 x 16 26.7 / 24.2.
   // Where a single round of workgroups fills the chip the stores wait for it: with 32 MB or less (128/256, 16 x 16, in place 10.1 / 12.4),
   // 12 MB where a workgroup has 32 KB (64/128, 32 x 8 5.8 / 6.3), and with slices of 128 KB (256/512, 16 x 8 20.6 / 23.0).  With more than
-  // the cache holds it is memory either way (128/256, 64 x 16, other states in between 53.3 / 57.3).
-  const size_t slice_bytes = (size_t)128 * (DHQK < 256 ? DHQK : 256) * (sbf ? 2 : 4);
+  // the cache holds it is memory either way (128/256, 64 x 16, other states in between 53.3 / 57.3).  16-bit states of more rows gain as
+  // well (512/1024, 40 MB 21.8 / 21.1, 96 MB 41.8 / 40.6).  Slices of 64 columns from 20 MB on (64/64, 16 MB 7.7 / 7.8, 24 MB 11.2 / 10.0; 100/64 8.2 /
+  // 8.8, 11.5 / 11.1), 16-bit states from 12 (64/64, 8 MB 6.3 / 6.8, 16 MB 9.4 / 8.8).
+  const bool narrow = DHHV <= 64 && DHQK < 128;
+  const size_t slice_bytes = (size_t)128 * DHQK * (sbf ? 2 : 4);
+  const size_t least = narrow ? (sbf ? 12 : 20) : slice_bytes <= 32768 ? 12 : 32;  // MB
   // (Stores of 16 bytes: at multiples of 16 only.)
-  const bool through = (uintptr_t)c_out % 16 == 0 && slice_bytes <= 65536 && state_bytes > ((size_t)(slice_bytes <= 32768 ? 12 : 32) << 20) && state_bytes <= ((size_t)112 << 20);
+  const bool through = (uintptr_t)c_out % 16 == 0 && (sbf || slice_bytes <= 65536) && state_bytes > least << 20 && state_bytes <= (size_t)112 << 20;
 #define MLSTM_STEP_ROWS(MODE_)                                       \
   {                                                                  \
-    if (DHHV <= 64 && DHQK < 128) MLSTM_STEP_PICK(64, 16, 4, MODE_)  \
-    if (DHQK >= 256) MLSTM_STEP_PICK(128, 16, 16, MODE_)             \
+    if (narrow) MLSTM_STEP_PICK(64, 16, 4, MODE_)                    \
     if (DHQK >= 128) MLSTM_STEP_PICK(128, 16, 8, MODE_)              \
     MLSTM_STEP_PICK(128, 16, 4, MODE_)                               \
+  }
+  if (DHQK >= 256) {
+    if (through && dtype_state == 1) return launch_step_t<128, 16, 16, kWriteThrough, 1>(MLSTM_STEP_ARGS);
+    if (through) return launch_step_t<128, 16, 16, kWriteThrough, 2>(MLSTM_STEP_ARGS);  // (no float32 state)
+    MLSTM_STEP_PICK(128, 16, 16, kPlain)
   }
   if (through) MLSTM_STEP_ROWS(kWriteThrough)
   MLSTM_STEP_ROWS(kPlain)

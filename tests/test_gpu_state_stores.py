@@ -1,7 +1,10 @@
 """The recurrent kernels' ways of reading and storing the state, chosen by its size: a head's results are the same bits whatever it is
-batched with.  Heads of rows and columns that leave row groups, lanes and the first batch of rows unfilled."""
+batched with, but for the order of the sum in h beyond 320 MiB, where the rows are dealt to other groups.  Heads of rows and columns
+that leave row groups, lanes and the first batch of rows unfilled."""
 import pytest
 import torch
+
+import oracle as O
 
 pytestmark = pytest.mark.gpu
 _F32, _BF16 = torch.float32, torch.bfloat16
@@ -15,11 +18,12 @@ def _inputs(n, T, DQ, DV, sdt, seed):
     return x, [rn(1, DQ, DV).to(sdt), rn(1, DQ).to(sdt), rn(1, 1).to(sdt)]
 
 
-# (rows, columns, state type, MiB of state: on either side of 12, 32, 112 and 320)
+# (rows, columns, state type, MiB of state: on either side of 12, 20, 32, 112 and 320)
 @pytest.mark.parametrize("DQ,DV,sdt,mib", [(64, 128, _F32, 11), (64, 128, _F32, 20), (64, 128, _F32, 120), (48, 132, _F32, 20), (65, 64, _F32, 40),
                                            (127, 256, _F32, 40), (128, 256, _F32, 40), (129, 260, _F32, 40), (255, 64, _BF16, 40),
                                            (256, 512, _BF16, 40), (256, 512, _F32, 40), (100, 72, _BF16, 20), (128, 256, _F32, 330),
-                                           (64, 64, _F32, 5), (64, 64, _F32, 20), (33, 40, _BF16, 20), (127, 64, _F32, 20)])
+                                           (64, 64, _F32, 5), (64, 64, _F32, 20), (64, 64, _F32, 24), (33, 40, _BF16, 20), (127, 64, _F32, 24),
+                                           (512, 64, _BF16, 40)])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_step(DQ, DV, sdt, mib, in_place):
     from mlstm_kernels_amd.torch.recurrent import mlstm_recurrent_step__hip_fw
@@ -29,19 +33,21 @@ def test_step(DQ, DV, sdt, mib, in_place):
     x, (c, nn, m) = _inputs(n, None, DQ, DV, sdt, DQ)
     some = [0, 1, n - 2, n - 1]
     h1, (c1, n1, m1) = mlstm_recurrent_step__hip_fw(c[some], nn[some], m[some], *(t[some] for t in x), dtype_state=sdt)
+    d = lambda t: t[some].double()
+    ref = O.recurrent_step(*(d(t) for t in x), d(c), d(nn), d(m))  # (in front of the call, which may write over c)
     kw = dict(matC_new=c, vecN_new=torch.empty_like(nn), scaM_new=torch.empty_like(m)) if in_place else {}
     h, (c2, n2, m2) = mlstm_recurrent_step__hip_fw(c, nn, m, *x, dtype_state=sdt, **kw)
-    for a, b in ((h, h1), (c2, c1), (n2, n1), (m2, m1)):
+    for a, b in ((c2, c1), (n2, n1), (m2, m1)):
         assert torch.equal(a[some], b)
-    # the recurrence in 64 bits, of the state that came out (the states went in as they are read)
-    if not in_place:
-        d = lambda t: t[some].double()
-        lf = torch.nn.functional.logsigmoid(d(x[4]))
-        m_new = torch.maximum(lf + d(m), d(x[3]))
-        fa, ia = torch.exp(lf + d(m) - m_new), torch.exp(d(x[3]) - m_new)
-        ref = fa[..., None] * d(c) + ia[..., None] * d(x[1])[..., None] * d(x[2])[:, :, None, :]
-        tol = 1e-6 if sdt == _F32 else 2 ** -8  # (16 bits: half a unit in the last place of each value)
-        assert float(((d(c2) - ref).norm() / ref.norm())) <= tol
+    if mib <= 320:
+        assert torch.equal(h[some], h1)
+    else:  # a sum in another order may be rounded to the other bfloat16 neighbour
+        assert bool(((h[some].double() - h1.double()).abs() <= 2 ** -7 * h1.double().abs() + 1e-5 * float(h1.double().abs().max())).all())
+    # the recurrence in 64 bits.  h is rounded to bfloat16, a 16-bit state to 16 bits: half a unit in the last place of each value
+    ref_h, ref_states = ref
+    assert float((h[some].double() - ref_h).norm() / ref_h.norm()) <= 2 ** -8
+    for a, b in zip((c2, n2, m2), ref_states):
+        assert float((a[some].double() - b).norm() / b.norm()) <= (1e-6 if sdt == _F32 else 2 ** -8)
 
 
 # (on either side of 96 MiB of state)
