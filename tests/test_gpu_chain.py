@@ -1,6 +1,6 @@
 """The chain kernels (state recurrence and H / dV in one launch) where they can go wrong: lengths around steps of 64 positions,
-chunks of 128 and windows of 256, each width of a workgroup and head dimension, every option of the operators, against the fp64
-oracle on the first and the last (batch, head) pair.  Tolerances are norm-relative as for the other kernels of these outputs: H
+chunks of 128 and windows of 256 and long ones, each width of a workgroup and head dimension, every option of the operators, one and
+several rounds of workgroups, against the fp64 oracle on the first and the last (batch, head) pair.  Tolerances are norm-relative as for the other kernels of these outputs: H
 6e-3, gradients 8e-3 (float16: a quarter), gate gradients 5e-2 of their scale, states 1e-3."""
 import ctypes
 
@@ -91,7 +91,7 @@ def test_lengths(DQ, DV, width, S):
     _run(_heads(DV, width), S, DQ, DV, seed=S)
 
 
-@pytest.mark.parametrize("DQ,DV,width", [(128, 128, 128), (256, 256, 256)])
+@pytest.mark.parametrize("DQ,DV,width", [(64, 128, 128), (64, 256, 256), (128, 128, 128), (128, 256, 256), (256, 128, 128), (256, 256, 256)])
 @pytest.mark.parametrize("S", [384, 449])
 @pytest.mark.parametrize("opt", [dict(init=True, last=True), dict(sig=True, init=True, last=True), dict(sig=True, normalize=False, init=True, last=True),
                                  dict(dtype=torch.float16, init=True, last=True), dict(stride=1, last=True), dict(stride=3, init=True),
@@ -100,6 +100,57 @@ def test_lengths(DQ, DV, width, S):
                          ids=["states", "sig", "sig-raw", "fp16", "stride1", "stride3", "forget", "keep", "fp16-keep", "recompute"])
 def test_options(DQ, DV, width, S, opt):
     _run(_heads(DV, width), S, DQ, DV, seed=S + 1, **opt)
+
+
+# many steps: decays that add up, sums over a long walk; forget gates that forget, that mostly keep and that keep nearly all
+@pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 2048), (64, 256, 256, 2111), (128, 128, 128, 4100), (128, 256, 256, 2017), (256, 128, 128, 2050),
+                                           (256, 512, 256, 2200)])
+@pytest.mark.parametrize("opt", [dict(f_offset=0.0, last=True), dict(f_offset=3.0, init=True, last=True), dict(f_offset=9.0, last=True),
+                                 dict(f_offset=3.0, dtype=torch.float16, last=True), dict(f_offset=9.0, dtype=torch.float16), dict(sig=True, last=True)],
+                         ids=str)
+def test_long(DQ, DV, width, S, opt):
+    _run(_heads(DV, width), S, DQ, DV, seed=S, **opt)
+
+
+# two rounds of workgroups (the last head is in the second one), and a first round that is all there is, not quite full
+@pytest.mark.parametrize("DQ,DV,width,share", [(128, 256, 256, 2.0), (256, 512, 256, 1.95), (64, 128, 128, 2.0), (128, 256, 256, 0.9)])
+def test_rounds(DQ, DV, width, share):
+    _run(int(_heads(DV, width) * share), 330, DQ, DV, seed=7, last=True)
+
+
+@pytest.mark.parametrize("DQ,DV,width", [(64, 128, 128), (64, 256, 256), (128, 128, 128), (128, 256, 256), (256, 128, 128), (256, 512, 256)])
+@pytest.mark.parametrize("S", [513, 1100, 2048])
+@pytest.mark.parametrize("dtype,init", [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float16, False)], ids=str)
+def test_without_kept_states(DQ, DV, width, S, dtype, init):
+    """A forward without a backward keeps no states; H and the last states are the bits of one that does."""
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    BH = _heads(DV, width)
+    print(f"{BH} x {S} {DQ}/{DV} {dtype} init={init}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), 3 + rn(S)]
+    st = (0.1 * rn(DQ, DV), 0.1 * rn(DQ), 0.3 * rn(1)) if init else (None,) * 3
+    out = []
+    for grad in (False, True):
+        leaves = [t.clone().requires_grad_(grad) for t in x]
+        _names()
+        _lib.profile_enable(True)
+        try:
+            H, last = mlstm_chunkwise__hip_xl_chunk(*leaves, *st, return_last_states=True, any_sequence_length=True)
+        finally:
+            _lib.profile_enable(False)
+        assert "chain_h" in _names()
+        out.append([t.detach() for t in (H, *last)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    L = next(y for y in (64, 32, 16, 8, 4, 2, 1) if S % y == 0)
+    for h in (0, BH - 1):
+        d = lambda t: None if t is None else t.detach()[:, h:h + 1].double().cpu()
+        fw = O.chunkwise_fw(*(d(t) for t in x), *(d(t) for t in st), chunk_size=L)
+        assert rel_norm(d(out[0][0]), fw["H"]) <= 6e-3 * (0.25 if dtype == torch.float16 else 1.0)
+        assert rel_norm(d(out[0][1]), fw["C_last"]) <= 1e-3 and rel_norm(d(out[0][2]), fw["n_last"]) <= 1e-3
 
 
 def test_closed_gates():
@@ -113,7 +164,15 @@ def test_closed_gates():
     i, f = rn(1, BH, S), 3 + rn(1, BH, S)
     f[:, :, 130] = -200.0
     i[:, :, 200:330] = -float("inf")
-    H, (C, n, m) = mlstm_chunkwise__hip_xl_chunk(q, k, v, i, f, return_last_states=True, any_sequence_length=True)
+    from mlstm_kernels_amd import _lib
+
+    _names()
+    _lib.profile_enable(True)
+    try:
+        H, (C, n, m) = mlstm_chunkwise__hip_xl_chunk(q, k, v, i, f, return_last_states=True, any_sequence_length=True)
+    finally:
+        _lib.profile_enable(False)
+    assert "chain_h" in _names()
     for h in (0, BH - 1):
         d = lambda t: t[:, h:h + 1].double().cpu()
         # (the recurrence itself: an infinite gate is a weight of zero there)

@@ -353,7 +353,9 @@ def test_short_prompts_gates_of_the_pre_pass(S, DQ, DV, NH, opt):
 
     init, sig, dtype = opt.get("init", False), opt.get("sig", False), opt.get("dtype", torch.bfloat16)
     if init:
-        NH = {200: 80, 320: 112, 129: 272}.get(S, NH)  # (as many as take one launch from a state)
+        if S == 320:
+            pytest.skip("from a state so many heads do not take the short kernel")
+        NH = {200: 80, 129: 272}.get(S, NH)  # (as many as take one launch from a state)
     op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
     g = torch.Generator(device="cuda").manual_seed(S)
     rn = lambda *d: torch.randn(1, NH, *d, device="cuda", generator=g)
@@ -366,8 +368,7 @@ def test_short_prompts_gates_of_the_pre_pass(S, DQ, DV, NH, opt):
             H, last = op(*x, *state, return_last_states=True, any_sequence_length=True)
     finally:
         _lib.profile_enable(False)
-    if S != 320 or not init:
-        assert {"gates", "short_fw"} <= set(_lib.profile_read())
+    assert {"gates", "short_fw"} <= set(_lib.profile_read())
     cut = lambda t: None if t is None else t[:, NH - 2:].contiguous()
     with torch.no_grad():
         H2, last2 = op(*(cut(t) for t in x), *(cut(t) for t in state), return_last_states=True, any_sequence_length=True)
