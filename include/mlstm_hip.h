@@ -157,16 +157,17 @@ size_t mlstm_hip_chunkwise_fw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   c0,n0,m0: initial states or NULL (all three NULL together; m0 ignored for the sig gate).
  *   H (B,NH,S,DHHV) in dtype_qkv.  n_out, m_out: optional fp32 (B,NH,S) per-row normaliser max(|den|,floor)
  *   and stabiliser (NULL to skip).  c_last,n_last,m_last: optional fp32 last states (NULL to skip).
- *   c_last, n_last, m_last may be c0, n0, m0 themselves (states updated in place; any other overlap is undefined).  Such a call
- *   does not take the kernel for short sequences and does not cut its scan into segments: within the tolerance of the 16-bit
- *   operands, but not bit for bit, what separate buffers give.
+ *   c_last, n_last, m_last may be c0, n0, m0 themselves (states updated in place; any other overlap is undefined).  With C or n in place
+ *   a call takes neither the kernel for short sequences nor the chain kernel and does not cut its scan into segments: within the
+ *   tolerance of the 16-bit operands, but not bit for bit, what separate buffers give.  (m alone in place changes nothing.)
  *   With MLSTM_PATH_AUTO the kernel for short sequences serves calls without keep_for_backward only: up to 512 positions H with
  *   and without it agree within the tolerance of the 16-bit operands, but not bit for bit.  With a named path they are the same.
  *   H serves the state scan as scratch before it is written (dV likewise in the backward).
  *   With c_last given, the state scan carries the gated values as a 16-bit head plus a 16-bit remainder in every
  *   chunk that still weighs at least 2^-8 in the last state, so c_last is accurate to ~1e-5 relative; with c_last
  *   NULL it rounds them once (as the replaced kernels do), which is up to a fifth faster and changes H only within
- *   the tolerance of its 16-bit operands.
+ *   the tolerance of its 16-bit operands.  The chain kernel carries the remainder in every step either way.
+ *   q, k, v (and dH in the backward) may begin at any element; the chain kernel takes those at multiples of 16 bytes.
  *   MLSTM_PATH_FUSED takes bf16 only.
  *   normalize applies to the sig gate only (0: H is the bare numerator).
  */

@@ -528,9 +528,9 @@ static const char* launch_step_block_t(const StepBlockArgs& a, hipStream_t strea
 // state of up to 96 MB, which the memory-side cache holds beside the old one, is written through them instead.  us, plain /
 // write-through, other states in between and the state of one call the next one's input: 256/512, 8 heads, 16 tokens B=4 12.5 11.9 /
 // 11.3 11.5, B=8 17.4 17.4 / 15.5 15.4, B=16 32.8 31.1 / 29.0 27.1, B=24 (96 MB) 46.9 43.0 / 47.4 39.6, B=32 60.0 61.2 / 62.9 61.3; 64 tokens
-// B=16 65.1 59.0 / 62.2 57.1; 16 heads of 128/256, B=32 34.9 33.1 / 33.3 29.2; 64/128, 4 tokens B=64 13.4 12.9 / 11.5 11.2.  (Non-temporal
-// stores gain the same, B=16 28.2, but the next call then reads from memory: 33.2 instead of 27.1.  At multiples of 8 bytes only: two
-// columns in one atomic store.)
+// B=16 65.1 59.0 / 62.2 57.1; 16 heads of 128/256, B=32 34.9 33.1 / 33.3 29.2; 64/128, 4 tokens B=64 13.4 12.9 / 11.5 11.2.  It gains nothing
+// where the same call is repeated on the same state (16 tokens B=16 34.6 / 34.5).  (Non-temporal stores gain the same, B=16 28.2, but the
+// next call then reads from memory: 33.2 instead of 27.1.  At multiples of 8 bytes only: two columns in one atomic store.)
 template <bool F16, int SDT, int MODE>
 static const char* launch_step_block_w(const StepBlockArgs& a, hipStream_t stream) {
   const bool through = (uintptr_t)a.c_out % 8 == 0 && (size_t)a.BH * a.DHQK * a.DHHV * (SDT == 0 ? 4 : 2) <= ((size_t)96 << 20);

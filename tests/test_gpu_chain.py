@@ -293,3 +293,33 @@ def test_every_element_within_tolerance_of_the_rounding_emulation(DQ, DV, width,
             worst = float(((d(a) - b).abs() / (2e-2 + 2e-2 * b.abs())).max())
             print(f"  {name} head {h}: {worst:.2f} x the bound", flush=True)
             assert worst <= 1, (name, h, worst)
+
+
+@pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 1000), (128, 256, 256, 1024), (256, 512, 256, 1024)])
+@pytest.mark.parametrize("opt", [dict(f_offset=0.0), dict(), dict(f_offset=9.0), dict(sig=True), dict(f_offset=9.0, dtype=torch.float16)], ids=str)
+def test_as_exact_as_scan_and_h(DQ, DV, width, S, opt):
+    """Distance from 64 bits by norm, over eight heads, against that of the scan and the kernels over chunks ("split")."""
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    BH, dtype, sig = _heads(DV, width), opt.get("dtype", torch.bfloat16), opt.get("sig", False)
+    print(f"{BH} x {S} {DQ}/{DV} {opt}", flush=True)
+    op = mlstm_siging_chunkwise__hip_xl_chunk if sig else mlstm_chunkwise__hip_xl_chunk
+    g = torch.Generator(device="cuda").manual_seed(S + DQ)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), opt.get("f_offset", 3.0) + rn(S)]
+    dH, heads = rn(S, DV).to(dtype), list(range(0, BH, BH // 8))
+    d = lambda t: t.detach()[:, heads].double().cpu()
+    L = next(y for y in (64, 32, 16, 8) if S % y == 0)
+    fw = O.chunkwise_fw(*(d(t) for t in x), chunk_size=L, siging=sig)
+    bw = O.chunkwise_bw(*(d(t) for t in x), d(dH), chunk_size=L, siging=sig)
+    err = []
+    for path in ("auto", "split"):
+        leaves = [t.clone().requires_grad_(True) for t in x]
+        H, last = op(*leaves, return_last_states=True, any_sequence_length=True, kernel_path=path)
+        grads = torch.autograd.grad(H, leaves[:3], dH)
+        err.append([rel_norm(d(a), b) for a, b in zip((H, *grads, *last[:2]), (fw["H"], *bw[:3], fw["C_last"], fw["n_last"]))])
+    print(err, flush=True)
+    for a, b in zip(err[0][:4], err[1][:4]):
+        assert a <= 1.02 * b
+    for a, b in zip(err[0][4:], err[1][4:]):
+        assert a <= max(1.05 * b, 2 ** -20)  # (fp32 sums of up to S terms, in another order)
