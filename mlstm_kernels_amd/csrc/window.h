@@ -26,9 +26,20 @@ constexpr int kWinSlot = 32768;          // bytes per ring slot (the largest sla
 constexpr int kWinPOfs = 2 * kWinSlot;   // P behind the two slots: 36 blocks of 32 x 32 (2 KB each, 64-byte rows, swizzled)
 constexpr int kWinPBytes = 36 * 2048;
 
-// 16-byte-unit swizzle of tiles with 64-byte rows (operand rows of 32 columns, blocks of P): eight consecutive rows read
-// at one unit, and the 4 rows x 2 units patch of a transposing read, both fall on distinct LDS banks
-__device__ __forceinline__ int win_f64(int row) { return (((row >> 1) & 1) << 1) | ((row >> 2) & 1); }
+// Swizzles of 16-byte units.  LDS has 64 banks of 4 bytes and serves a 16-byte read in groups of 16 lanes, 0-3 12-15 20-27 and
+// 4-11 16-19 28-31 (and the same of lanes 32-63), an 8-byte one, transposing or not, in groups of 32.
+// Tiles with 64-byte rows (operand rows of 32 columns, blocks of P), four rows to a line of banks: of 32 rows read at one unit a group
+// has four of every residue mod 4, whose numbers / 4 differ mod 4; the 4 rows x 4 units patch of a transposing read is a line.
+__device__ __forceinline__ int win_f64(int row) { return (row >> 2) & 3; }
+// Tiles with rows of RB = 128, 256 or 512 bytes: a transposing read takes 4 neighbouring units of 4 consecutive rows, and a read of 8
+// bytes of one unit 32 rows.  (512: 8 rows further on, which is where the next piece of a thread goes, it is the same again.)
+// Against swizzles for groups of 8 and 16 neighbouring lanes, which two lanes of every group shared a bank with (us, before / after):
+// dQ / dK of 256/512, 32 heads of 16384 770 / 757, 128 of 1024 183 / 179.
+template <int RB>
+__device__ __forceinline__ int win_zsw(int row) {
+  if (RB == 128) return (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
+  return ((row & 3) << 2) | (RB == 256 ? (row >> 2) & 3 : ((row >> 2) & 1) << 1);
+}
 
 // The blocks (tb, jb) of the lower triangle that a consumer wave computes: three blocks of row ta (keys ja, ja + 1, ja + 2)
 // and up to two of row tc (keys jc, jc + 1).  With at most two rows per wave and the split between them fixed, the

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
           const uint32_t vrow = pl / UPR, vun = pl % UPR;
           const uint32_t vp = (uint32_t)DHHV * 2, vcol = (uint32_t)cg * (CW * 2) + vun * 16;
           const uint32_t vlim = (uint32_t)(S - 1) * vp + vcol, vstep = (256 / UPR) * vp;
-          const uint32_t vd = (vrow * UPR + (vun ^ (2 * (vrow & 3)))) * 16;
+          const uint32_t vd = (vrow * UPR + (vun ^ (uint32_t)win_zsw<CW * 2>((int)vrow))) * 16;
           const uint32_t vg = (t0 + vrow) * vp + vcol;
           for (int z = 0; z < NVS; z += 2) {
             const uint32_t g0 = vg + (uint32_t)(z * VROWS) * vp, g1 = vg + (uint32_t)((z + 1) * VROWS) * vp;
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(768) void window_hv_kernel(ParHvArgs a, int n_items
                 for (int half = 0; half < 2; ++half) {
                   const int row = 32 * zh + 16 * kk + krow + 4 * half;
                   const int un = 8 * ci + 4 * mb + zun;
-                  A[mb].d[half] = lds_read_tr16(Zs + row * (CW * 2) + ((un ^ (2 * (row & 3))) * 16) + zin);
+                  A[mb].d[half] = lds_read_tr16(Zs + row * (CW * 2) + ((un ^ win_zsw<CW * 2>(row)) * 16) + zin);
                 }
 #pragma unroll
               for (int nb = 0; nb < NNB; ++nb) {

@@ -172,14 +172,15 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
       const uint32_t xg = (t0 + xrow) * (uint32_t)(DHHV * 2) + xun * 16;
       const uint32_t xstep = 64 * (uint32_t)DHHV * 2;
       const uint32_t xlim = (uint32_t)(S - 1) * (uint32_t)(DHHV * 2) + xun * 16;  // this thread's unit of the last row
-      // state fragments of 32 value columns: DT / 16 KB contiguous in memory; lanes 32..63 of every fragment are stored 4
-      // slots off so that the two lane halves a transposing read touches together fall on different LDS banks
-      const uint32_t cdu = pl ^ (((pl >> 5) & 1) << 2);
+      // state fragments of 32 value columns: DT / 16 KB contiguous in memory; lanes 32..63 of every fragment are stored 4 slots off
+      // and every second fragment 8, so that the two lane halves of two fragments that a transposing read touches together fall
+      // on different LDS banks
+      const uint32_t cdu = pl ^ (((pl >> 5) & 1) << 2) ^ (((pl >> 6) & 1) << 3);
       // ZROWS rows x DT head-dim entries: piece (row, unit) = (pl / UPR + 256 / UPR i, pl % UPR)
       constexpr int UPR = DT / 8;  // 16-byte units per row of a tile
       const uint32_t zpitch = (uint32_t)DHQK * 2;
       const uint32_t zrow = pl / UPR, zun = pl % UPR;
-      const uint32_t zdu = zrow * UPR + (zun ^ (2 * (zrow & 3)));
+      const uint32_t zdu = zrow * UPR + (zun ^ (uint32_t)win_zsw<DT * 2>((int)zrow));
       const uint32_t zg0 = (t0 + zrow) * zpitch + zun * 16;
       const uint32_t zlim0 = (uint32_t)(S - 1) * zpitch + zun * 16;
       const uint32_t zstep = (256 / UPR) * zpitch;
@@ -443,7 +444,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
 #pragma unroll
               for (int half = 0; half < 2; ++half) {
                 const int wr = wrow + 4 * half;
-                const int slot_l = (32 * h_src + wr) ^ (h_src << 2);
+                const int slot_l = (32 * h_src + wr) ^ (h_src << 2) ^ (q16 << 3);
                 A[mb].d[half] = lds_read_tr16(Cf + ((size_t)ds_l * 64 + slot_l) * 16 + 8 * a_src);
               }
             }
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
                 for (int half = 0; half < 2; ++half) {
                   const int row = 32 * zh + 16 * kk + krow + 4 * half;
                   const int un = 8 * di + 4 * mb + zun;
-                  A[mb].d[half] = lds_read_tr16(Zs + row * (DT * 2) + ((un ^ (2 * (row & 3))) * 16) + zin);
+                  A[mb].d[half] = lds_read_tr16(Zs + row * (DT * 2) + ((un ^ win_zsw<DT * 2>(row)) * 16) + zin);
                 }
 #pragma unroll
               for (int nb = 0; nb < NNB; ++nb) {
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(768) void window_qk_kernel(ParQkArgs a, int n_items
           {
             const int row = 32 * pg + r;
             const unsigned char* const xrow = Xs + row * (DT * 2) + 8 * h;
-            const int sw = 2 * (row & 3);
+            const int sw = win_zsw<DT * 2>(row);
             float part = 0.f;
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb)
