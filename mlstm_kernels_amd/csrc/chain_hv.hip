@@ -13,8 +13,13 @@
 //     partial products of a position then meet in LDS.  A state tile of 32 x 32 is at once the accumulator of the update and, rounded,
 //     the operand of the product with the state: its rows are taken in the order in which a lane's registers are eight neighbouring
 //     ones (the transposing reads of K trade two groups of four), so that it never passes through LDS.
-//   * Rows come straight into LDS, swizzled, one step ahead: the output-side rows of the next step into a free tile at the start of
-//     a step, the other rows and the value rows where the present ones have been read.  Two barriers a step.
+//   * Rows come straight into LDS, swizzled, one step ahead.  Where two sets of tiles fit (64 and 128 state rows) all of them are
+//     requested in the first half of a step; with 256 the output-side rows go to a free tile, the other rows and the value rows, in the
+//     second half, where the present ones have been read.  Two barriers a step.
+//   * What goes through the memory path in the second half, requests and rows of the output, goes out between the matrix instructions of
+//     the update: in front of it the waves stood there (256/256 columns, of 15.9 thousand cycles a step 3.0 were the slower waves' wait;
+//     now 13.6), and a step ends when its requests are there, not when its output is written.  us, before / after: 128 heads of
+//     256/512, 2048 positions with the last state 277 / 257, dV of 1024 135 / 127; 128/256, 128 heads of 2048, 129 / 121 and 121 / 107.
 //   * Scores: 10 live tiles of 16 x 16, two a wave, gated in fp32 and written to LDS as operand fragments; q . n on the way as one more
 //     operand (three 16-bit parts of n, exactly).
 //   * The value rows are scaled in fp32 and enter the state as a 16-bit head and remainder: the state is rounded every 64 positions
@@ -100,9 +105,11 @@ struct DmaTile {
     }
   }
 };
+// (the wave's last N vector-memory instructions may still be on their way)
+template <int N = 0>
 __device__ __forceinline__ void dma_wait() {
   asm volatile("" : : : "memory");
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __builtin_amdgcn_s_waitcnt(0x0f70 | N);  // vmcnt(N), N < 16
   asm volatile("" : : : "memory");
 }
 // 64 consecutive fp32 values to LDS, one per lane
@@ -126,15 +133,19 @@ __device__ __forceinline__ Frag tr_frag(const uint16_t* lo, const uint16_t* hi) 
 
 }  // namespace
 
-template <int DQ, int W>
+template <int DQ, int W, bool F16>
 struct ChainLds {  // bytes
   static constexpr int G = W / 32, DS = 8 / G;
   static constexpr int TQ = kStep * DQ * 2, TV = kStep * W * 2, PB = 6144;
   static constexpr int EX = DS == 2 ? 8 * 4096 : 0;
-  static constexpr int kV = 3 * TQ, kP = kV + TV, kEx = kP + PB, kVec = kEx + EX;
-  // [2][5][64] weights, [5][64] gate vectors as they arrive, [8][64] row sums, [4][64] q . n, n as [DQ] fp32 and [3][NP] 16-bit parts, decay
+  // Two sets of tiles where they fit (DQ 64 and 128): everything of the next step is requested at the start of this one.
+  static constexpr bool kAhead = 4 * TQ + 2 * TV + PB + EX + 12288 <= 160 * 1024;
+  static constexpr int kV = (kAhead ? 4 : 3) * TQ, kP = kV + (kAhead ? 2 : 1) * TV, kEx = kP + PB, kVec = kEx + EX;
+  // [2][5][64] weights, [2][5][64] gate vectors as they arrive, [8][64] row sums, [4 or 1][64] q . n, decay, n as [DQ] fp32 and (bfloat16)
+  // [3][NP] 16-bit parts
   static constexpr int NP = DQ + 16;  // (32 bytes apart: the three rows of a fragment on distinct banks)
-  static constexpr int kBytes = kVec + (640 + 320 + 768 + 8) * 4 + DQ * 4 + 3 * NP * 2;
+  static constexpr int QN = F16 ? 256 : 64;
+  static constexpr int kBytes = kVec + (640 + 640 + 512 + QN + 8 + DQ) * 4 + (F16 ? 0 : 3 * NP * 2);
 };
 
 // x = sum of three bfloat16 values, exactly (a float32 has 24 significant bits)
@@ -170,7 +181,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (!ROWS) {
     if (__builtin_amdgcn_readfirstlane(*a.g.chained) == 0) return;  // the forward's states came from the scan
   }
-  using L = ChainLds<DQ, W>;
+  using L = ChainLds<DQ, W, F16>;
   constexpr int G = L::G, DS = L::DS;
   constexpr int NDT = DQ / 32 / DS;         // 32-row state tiles of a wave
   constexpr int NO = DS == 1 ? 2 : 1;       // position tiles of 32 whose output a wave finishes
@@ -179,10 +190,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   static_assert(G * DS == 8 && NDT >= 1 && DS <= 2, "eight waves");
   extern __shared__ __align__(16) unsigned char smem[];
   float* const vec = (float*)(smem + L::kVec);  // [2][5][64]: u (t), w (j), us, csc, aux
-  float* const raw = vec + 640;                 // [5][64]
-  float* const rs = raw + 320;                  // [8][64] row sums of P: two waves a position, four lanes each
+  float* const raw = vec + 640;                 // [2][5][64]
+  float* const rs = raw + 640;                  // [8][64] row sums of P: two waves a position, four lanes each
   float* const qn = rs + 512;                   // [4][64] shares of q . n (bfloat16: one)
-  float* const gdl = qn + 256;                  // [2] decay of the state in a step
+  float* const gdl = qn + L::QN;                // [2] decay of the state in a step
   float* const nv = gdl + 8;                    // [DQ] normaliser state
   uint16_t* const npt = (uint16_t*)(nv + DQ);   // [3][NP] the same as three 16-bit parts (bfloat16)
 
@@ -202,6 +213,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t q_off = DmaTile<DQ * 2>::offset(wave, lane, DQ * 2);
   const uint32_t w_off = DmaTile<W * 2>::offset(wave, lane, DHHV * 2);
   const uint32_t lds0 = lds_addr(smem);
+  // rows past the end of the sequence fall outside
+  const auto out_d = __builtin_amdgcn_make_buffer_rsrc(a.Out + (size_t)bh * S * DHHV, 0, (uint32_t)S * DHHV * 2, 0x00020000);
 
   // ---- state: tile dt holds rows 32 (dq NDT + dt) .. +31 in the order 16 (i / 8) + 8 h + i % 8 (register i), column 32 g + r
   f32x16 acc[NDT];
@@ -222,16 +235,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (tid < DQ) {
     const float x = do_n && a.n_init != nullptr ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
     nv[tid] = x;
-    split3(x, npt + tid, L::NP);
+    if constexpr (!F16) split3(x, npt + tid, L::NP);
   }
   rs[tid] = 0.f;
   for (int x = tid; x < L::PB / 16; x += 512) ((uint4*)(smem + L::kP))[x] = make_uint4(0, 0, 0, 0);
 
-  // gate vectors of step s, by one wave: requested ...
+  // gate vectors of step s, by wave 5 or 6 (which have no scores; in turn): requested ...
   auto gates_load = [&](int s) -> float {
     const int ln = opaque(lane), c = s >> 1;
     const uint32_t o = (uint32_t)s * (kStep * 4) + ln * 4;
-    const uint32_t dst = lds0 + L::kVec + 640 * 4;
+    const uint32_t dst = lds0 + L::kVec + 640 * 4 + (s & 1) * 1280;
     dma_vec(a.g.u + bh * Sp, o, dst);
     dma_vec(a.g.w + bh * Sp, o, dst + 256);
     dma_vec(a.g.abar + bh * Sp, o, dst + 512);
@@ -250,9 +263,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool single = S - c * kChunk <= kStep;
     const bool in = s * kStep + ln < S;
     const float u63 = __shfl(gs, 0), gg = __shfl(gs, 1), gm = __shfl(gs, 2);
-    const float gu = raw[ln], gw = raw[64 + ln], gx = raw[256 + ln];
-    const float A = odd || single ? raw[128 + ln] : expf(u63 - gw);  // weight of k v^T in the state after the step
-    const float B = odd ? expf(gu - u63) : raw[192 + ln];            // weight of the state before the step
+    const float* const raw_s = raw + (s & 1) * 320;
+    const float gu = raw_s[ln], gw = raw_s[64 + ln], gx = raw_s[256 + ln];
+    const float A = odd || single ? raw_s[128 + ln] : expf(u63 - gw);  // weight of k v^T in the state after the step
+    const float B = odd ? expf(gu - u63) : raw_s[192 + ln];            // weight of the state before the step
     float* v = vec + (s & 1) * 320 + ln;
     v[0] = gu;
     v[64] = gw;
@@ -273,18 +287,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint32_t o_n = 0, o_o = L::TQ, o_f = 2 * L::TQ;  // LDS offsets of the tiles: output-side rows, other rows, free
   auto load_n = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xn_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
   auto load_o = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xo_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
-  auto load_w = [&](int s) { DmaTile<W * 2>::load(Xw_d, w_off + (uint32_t)s * (kStep * 2) * (uint32_t)DHHV, DHHV * 2, lds0 + L::kV, wave); };
+  uint32_t o_w = L::kV;                            // ... and value rows
+  auto load_w = [&](int s, uint32_t o) { DmaTile<W * 2>::load(Xw_d, w_off + (uint32_t)s * (kStep * 2) * (uint32_t)DHHV, DHHV * 2, lds0 + o, wave); };
   if constexpr (ROWS) load_n(s_first, o_n);
   load_o(s_first, o_o);
-  load_w(s_first);
+  load_w(s_first, o_w);
   float gs = 0.f;
-  if (wave == 6) {
+  if (wave == 5 + (s_first & 1)) {
     gs = gates_load(s_first);
-    dma_wait();
+    dma_wait<>();
     gates_store(s_first, gs);
-    if (n_run > 1) gs = gates_load(s_first + s_inc);
   }
-  dma_wait();
+  if (wave == 6 - (s_first & 1) && n_run > 1) gs = gates_load(s_first + s_inc);
+  dma_wait<>();
 
   // score tiles (16 x 16) of a wave: position block n16 and two neighbouring blocks of the other index, from ob on (mirrored for dV)
   // wave            0  1  2  3  4  5  6  7
@@ -304,31 +319,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float* const v = vec + (s & 1) * 320;
     __syncthreads();  // ---- the tiles and vectors of this step are in LDS, the free tile is nobody's
     if (more) {
-      if constexpr (ROWS) load_n(s + s_inc, o_f);
-      else load_o(s + s_inc, o_f);
+      if constexpr (L::kAhead) {
+        if constexpr (ROWS) load_n(s + s_inc, it & 1 ? 0 : 2 * L::TQ);
+      } else {
+        if constexpr (ROWS) load_n(s + s_inc, o_f);
+        else load_o(s + s_inc, o_f);
+      }
     }
     const uint16_t* const Xn = (const uint16_t*)(smem + o_n);
     const uint16_t* const Xo = (const uint16_t*)(smem + o_o);
 
-    // ---- value rows: transposed fragments, lane = column 32 g + r, eight positions (DS == 2: those of the own position tile first)
-    Frag vf[4];
-    {
-      const int ln = lane_of<kTight>(lane);
-      const int i16 = ln & 15, kr = i16 >> 2;
-      const int unit = 4 * g + 2 * ((ln >> 4) & 1) + ((i16 & 3) >> 1), sub = 4 * (i16 & 1), row = 8 * (ln >> 5) + kr;
-      const uint16_t* base = (const uint16_t*)(smem + L::kV) + row * W + sub;
-      const uint16_t* lo = base + ((unit ^ swz<W * 2>(row)) << 3);
-      const uint16_t* hi = base + 4 * W + ((unit ^ swz<W * 2>(row + 4)) << 3);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) vf[j] = tr_frag(lo + (j < 2 ? kb0 : kb1) * W + (j & 1) * 16 * W, hi + (j < 2 ? kb0 : kb1) * W + (j & 1) * 16 * W);
-    }
-
-    if (more && wave == 6) {
-      gates_store(s + s_inc, gs);
+    if (wave == 6 - (s & 1)) {
+      if (more) gates_store(s + s_inc, gs);
+    } else if (wave == 5 + (s & 1)) {
       if (it + 2 < n_run) gs = gates_load(s + 2 * s_inc);
     }
     // ---- scores: P (other index, position), gated, rounded, to LDS as operand fragments
-    if (ROWS && sc_cnt > 0) {
+    auto scores = [&]() __attribute__((always_inline)) {
+    if (sc_cnt > 0) {
       const int ln = lane_of<kTight>(lane);
       const int m16 = ln & 15, qq = ln >> 4;
       const int o16a = IS_DV ? 3 - sc_o : sc_o, o16b = IS_DV ? 2 - sc_o : sc_o + 1;
@@ -437,10 +445,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
       qn[(wave - 4) * 64 + ln] = dot[0] + dot[1];
     }
+    };
 
     // ---- product with the state: out[k] = position tile (DS == 1: k, else the wave's own one first)
     f32x16 out[2];
-    if constexpr (ROWS) {
+    auto product = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int k = 0; k < 2; ++k)
 #pragma unroll
@@ -491,6 +500,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int k = 0; k < 4; ++k) ex[64 * k] = make_float4(out[1][4 * k], out[1][4 * k + 1], out[1][4 * k + 2], out[1][4 * k + 3]);
       }
+    };
+    if constexpr (ROWS) scores();
+    if (L::kAhead && more) {
+      load_o(s + s_inc, (it & 1 ? 0 : 2 * L::TQ) + L::TQ);
+      load_w(s + s_inc, it & 1 ? L::kV : L::kV + L::TV);
+    }
+    if constexpr (ROWS) product();
+    // ---- value rows: transposed fragments, lane = column 32 g + r, eight positions (DS == 2: those of the own position tile first)
+    Frag vf[4];
+    {
+      const int ln = lane_of<kTight>(lane);
+      const int i16 = ln & 15, kr = i16 >> 2;
+      const int unit = 4 * g + 2 * ((ln >> 4) & 1) + ((i16 & 3) >> 1), sub = 4 * (i16 & 1), row = 8 * (ln >> 5) + kr;
+      const uint16_t* base = (const uint16_t*)(smem + o_w) + row * W + sub;
+      const uint16_t* lo = base + ((unit ^ swz<W * 2>(row)) << 3);
+      const uint16_t* hi = base + 4 * W + ((unit ^ swz<W * 2>(row + 4)) << 3);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vf[j] = tr_frag(lo + (j < 2 ? kb0 : kb1) * W + (j & 1) * 16 * W, hi + (j < 2 ? kb0 : kb1) * W + (j & 1) * 16 * W);
     }
     // ---- kept state: before every stride-th chunk (forward), after the last chunk of every group (dV)
     if (a.states != nullptr) {
@@ -519,6 +546,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     __syncthreads();  // ---- scores, partial sums; the output-side rows and the value rows have been read
+    u32x4 orow[2 * NO];
     if constexpr (ROWS) {
       float4 ex[4];
       if constexpr (DS == 2) {
@@ -602,36 +630,42 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
               }
         }
       }
-      if (more) load_o(s + s_inc, o_n);
       // ---- output rows: lane (h, r) holds columns 8 x + 4 h + 0 .. 3 of position r; first the halves of the wave trade, so that it
       // holds eight neighbouring ones, then its rows of 16 lanes, so that four lanes hold the 32 columns of a position
-      {
-        uint16_t* const orow = a.Out + ((size_t)bh * S + t0) * DHHV + w_tile + 32 * g + 8 * h + (lane & 16);
 #pragma unroll
-        for (int k = 0; k < NO; ++k) {
-          uint32_t w[8], o[2][4];
+      for (int k = 0; k < NO; ++k) {
+        uint32_t w[8], o[2][4];
 #pragma unroll
-          for (int x = 0; x < 8; ++x) w[x] = pack2<F16>(out[k][2 * x] * iv[k], out[k][2 * x + 1] * iv[k]);
+        for (int x = 0; x < 8; ++x) w[x] = pack2<F16>(out[k][2 * x] * iv[k], out[k][2 * x + 1] * iv[k]);
 #pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            const auto p = __builtin_amdgcn_permlane32_swap(w[4 * x], w[4 * x + 2], false, false);
-            const auto q = __builtin_amdgcn_permlane32_swap(w[4 * x + 1], w[4 * x + 3], false, false);
-            o[x][0] = p[0]; o[x][1] = q[0]; o[x][2] = p[1]; o[x][3] = q[1];
-          }
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const auto p = __builtin_amdgcn_permlane16_swap(o[0][x], o[1][x], false, false);
-            o[0][x] = p[0]; o[1][x] = p[1];
-          }
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            const int n = 32 * (DS == 1 ? k : dq) + 16 * x + (lane & 15);
-            if (t0 + n < S) *(u32x4*)(orow + (size_t)n * DHHV) = u32x4{o[x][0], o[x][1], o[x][2], o[x][3]};
-          }
+        for (int x = 0; x < 2; ++x) {
+          const auto p = __builtin_amdgcn_permlane32_swap(w[4 * x], w[4 * x + 2], false, false);
+          const auto q = __builtin_amdgcn_permlane32_swap(w[4 * x + 1], w[4 * x + 3], false, false);
+          o[x][0] = p[0]; o[x][1] = q[0]; o[x][2] = p[1]; o[x][3] = q[1];
         }
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const auto p = __builtin_amdgcn_permlane16_swap(o[0][x], o[1][x], false, false);
+          o[0][x] = p[0]; o[1][x] = p[1];
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x) orow[2 * k + x] = u32x4{o[x][0], o[x][1], o[x][2], o[x][3]};
       }
     }
-    if (more) load_w(s + s_inc);
+    // what goes out during the update (it is what the memory path takes a while for: in front of it the waves stood there)
+    auto memory = [&](int i) {
+      if constexpr (!L::kAhead) {
+        if (i == 0 && ROWS && more) load_o(s + s_inc, o_n);
+        if (i == 1 && more) load_w(s + s_inc, o_w);
+        i -= 2;
+      }
+      if constexpr (ROWS) {
+        if (i >= 0 && i < 2 * NO) {
+          const int n = 32 * (DS == 1 ? i >> 1 : dq) + 16 * (i & 1) + (lane & 15);
+          __builtin_amdgcn_raw_buffer_store_b128(orow[i], out_d, (uint32_t)(t0 + n) * (uint32_t)(DHHV * 2) + (uint32_t)(w_tile + 32 * g + 8 * h + (lane & 16)) * 2, 0, 0);
+        }
+      }
+    };
     const float gdec = gdl[s & 1];
     // ---- state update, the scaled value rows as a 16-bit head and remainder; wave w takes rows 32 w .. of the normaliser state
     {
@@ -692,28 +726,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int p = 0; p < 4; ++p) scale(0, p);
       weights(1);
       fence();
+      constexpr int NM = L::kAhead ? 2 * NO : 2 * NO + 2;          // memory instructions (or groups of them) to go out
+      constexpr int kSeg = NT >= 4 * NM ? NT / 8 : (NT >= NM ? NT / NM : 1);  // state tiles between two of them
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const int j = i / NDT, d = i % NDT;
-        if (i + kAhead < NT) fetch(i + kAhead);
-        mfma32<F16>(acc[d], A[i & 3], vh[j & 1]);
-        mfma32<F16>(acc[d], A[i & 3], vl[j & 1]);
-        if (j < 3) {
+      for (int i0 = 0; i0 < NT; i0 += kSeg) {
+        memory(i0 / kSeg);
+        fence();
 #pragma unroll
-          for (int p = 4 * d / NDT; p < 4 * (d + 1) / NDT; ++p) scale(j + 1, p);
+        for (int i = i0; i < i0 + kSeg; ++i) {
+          const int j = i / NDT, d = i % NDT;
+          if (i + kAhead < NT) fetch(i + kAhead);
+          mfma32<F16>(acc[d], A[i & 3], vh[j & 1]);
+          mfma32<F16>(acc[d], A[i & 3], vl[j & 1]);
+          if (j < 3) {
+#pragma unroll
+            for (int p = 4 * d / NDT; p < 4 * (d + 1) / NDT; ++p) scale(j + 1, p);
+          }
+          if (d == NDT - 1 && j < 2) weights(j + 2);
         }
-        if (d == NDT - 1 && j < 2) weights(j + 2);
-      }
-      // a matrix instruction hides about six others of its wave
+        // a matrix instruction hides about six others of its wave
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+        for (int i = i0; i < i0 + kSeg; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+        }
+        fence();
       }
-      fence();
       if (N) {
         nsum += __shfl_xor(nsum, 32);
         const int d = 32 * ntile + (ln & 31);
@@ -724,11 +765,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       }
     }
-    dma_wait();
-    const uint32_t x = o_o;
-    o_o = ROWS ? o_n : o_f;
-    o_n = o_f;
-    o_f = x;
+    // (the rows of the next step were requested before the rows of this one went out)
+    dma_wait<ROWS ? 2 * NO : 0>();
+    asm volatile("" : "+v"(gs));  // has arrived with them; where it is used the compiler would wait for the rows requested by then
+    if constexpr (L::kAhead) {
+      o_n = it & 1 ? 0 : 2 * L::TQ;
+      o_o = o_n + L::TQ;
+      o_w = it & 1 ? L::kV : L::kV + L::TV;
+    } else {
+      const uint32_t x = o_o;
+      o_o = ROWS ? o_n : o_f;
+      o_n = o_f;
+      o_f = x;
+    }
   }
 
   __syncthreads();
@@ -748,7 +797,7 @@ namespace {
 template <int DQ, int W, int KIND, bool F16>
 const char* launch_t(const ChainHvArgs& a, int BH, hipStream_t stream) {
   static LdsLimit lds;
-  constexpr int smem = ChainLds<DQ, W>::kBytes;
+  constexpr int smem = ChainLds<DQ, W, F16>::kBytes;
   static_assert(smem <= 160 * 1024, "LDS of a CU");
   if (!lds.allow((const void*)chain_hv_kernel<DQ, W, KIND, F16>, smem)) return "chain_hv: cannot raise the dynamic LDS limit";
   hipLaunchKernelGGL((chain_hv_kernel<DQ, W, KIND, F16>), dim3(a.DHHV / W, BH), dim3(512), smem, stream, a);
