@@ -104,12 +104,41 @@ def test_options(DQ, DV, width, S, opt):
 
 # many steps: decays that add up, sums over a long walk; forget gates that forget, that mostly keep and that keep nearly all
 @pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 2048), (64, 256, 256, 2111), (128, 128, 128, 4100), (128, 256, 256, 2017), (256, 128, 128, 2050),
-                                           (256, 512, 256, 2200)])
+                                           (256, 512, 256, 2200), (256, 512, 128, 1600)])
 @pytest.mark.parametrize("opt", [dict(f_offset=0.0, last=True), dict(f_offset=3.0, init=True, last=True), dict(f_offset=9.0, last=True),
                                  dict(f_offset=3.0, dtype=torch.float16, last=True), dict(f_offset=9.0, dtype=torch.float16), dict(sig=True, last=True)],
                          ids=str)
 def test_long(DQ, DV, width, S, opt):
     _run(_heads(DV, width), S, DQ, DV, seed=S, **opt)
+
+
+@pytest.mark.parametrize("S", [257, 321, 1000, 1024])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_halves_of_wide_heads(S, dtype):
+    """Half of the heads that fill the chip with 256 columns a workgroup: 128, where no state is kept or there are thirteen chunks."""
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    BH, DQ, DV = _heads(512, 128), 256, 512
+    print(f"{BH} x {S} {DQ}/{DV} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(dtype), rn(S, DQ).to(dtype), rn(S, DV).to(dtype), rn(S), 3 + rn(S)]
+    st = [0.1 * rn(DQ, DV), 0.1 * rn(DQ), 0.3 * rn(1)]
+    _names()
+    _lib.profile_enable(True)
+    try:
+        H, last = mlstm_chunkwise__hip_xl_chunk(*x, c_initial=st[0], n_initial=st[1], m_initial=st[2], return_last_states=True, any_sequence_length=True)
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    assert "chain_h" in _names()
+    L = next(y for y in (64, 32, 16, 8, 4, 2, 1) if S % y == 0)
+    for h in (0, BH - 1):
+        d = lambda t: t[:, h:h + 1].double().cpu()
+        fw = O.chunkwise_fw(*map(d, x), *map(d, st), chunk_size=L)
+        assert rel_norm(d(H), fw["H"]) <= 6e-3 * (0.25 if dtype == torch.float16 else 1.0)
+        assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3 and rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
 
 
 # two rounds of workgroups (the last head is in the second one), and a first round that is all there is, not quite full
