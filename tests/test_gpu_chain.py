@@ -141,6 +141,48 @@ def test_halves_of_wide_heads(S, dtype):
         assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3 and rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
 
 
+# Few heads: segments of the sequence side by side.  Both widths, one slot and the most between segments, a last segment that is a chunk, a
+# part of one or whole, more segments than fit the scratch, heads that leave CUs over.
+@pytest.mark.parametrize("BH,S,DQ,DV", [(1, 16384, 128, 256), (2, 8300, 256, 512), (8, 5000, 256, 512), (8, 10000, 256, 512), (40, 8060, 256, 512),
+                                        (100, 3968, 128, 256), (4, 4428, 128, 256), (24, 3528, 128, 128), (3, 16384, 64, 128), (12, 6016, 64, 256),
+                                        (7, 10185, 256, 256), (9, 6003, 128, 384)])
+@pytest.mark.parametrize("opt", [dict(), dict(f_offset=9.0, init=True), dict(f_offset=0.0, last=False), dict(sig=True, init=True), dict(sig=True, normalize=False, init=True),
+                                 dict(dtype=torch.float16, f_offset=9.0)], ids=["", "keep", "forget", "sig", "sig-raw", "fp16-keep"])
+def test_segments(BH, S, DQ, DV, opt):
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
+
+    o = dict(dict(f_offset=3.0, init=False, last=True, sig=False, normalize=True, dtype=torch.bfloat16), **opt)
+    print(f"{BH} x {S} {DQ}/{DV} {opt}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, BH, *s, device="cuda", generator=g)
+    x = [rn(S, DQ).to(o["dtype"]), rn(S, DQ).to(o["dtype"]), rn(S, DV).to(o["dtype"]), rn(S), o["f_offset"] + rn(S)]
+    c0, n0, m0 = (0.1 * rn(DQ, DV), 0.1 * rn(DQ), None if o["sig"] else 0.3 * rn(1)) if o["init"] else (None, None, None)
+    kw = dict(c_initial=c0, n_initial=n0, return_last_states=o["last"], any_sequence_length=True)
+    _names()
+    _lib.profile_enable(True)
+    try:
+        with torch.no_grad():
+            if o["sig"]:
+                out = mlstm_siging_chunkwise__hip_xl_chunk(*x, normalize=o["normalize"], **kw)
+            else:
+                out = mlstm_chunkwise__hip_xl_chunk(*x, m_initial=m0, **kw)
+        torch.cuda.synchronize()
+    finally:
+        _lib.profile_enable(False)
+    assert "chain_h" in _names()
+    H, last = out if o["last"] else (out, None)
+    L = max(y for y in range(1, 257) if S % y == 0)  # (the oracle's chunks)
+    for h in {0, BH - 1}:
+        d = lambda t: None if t is None else t[:, h:h + 1].double().cpu()
+        fw = O.chunkwise_fw(*map(d, x), d(c0), d(n0), d(m0), chunk_size=L, siging=o["sig"], normalize=o["normalize"])
+        assert rel_norm(d(H), fw["H"]) <= 6e-3 * (0.25 if o["dtype"] == torch.float16 else 1.0)
+        if last is not None:
+            assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3
+            if o["normalize"]:
+                assert rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
+
+
 # two rounds of workgroups (the last head is in the second one), and a first round that is all there is, not quite full
 @pytest.mark.parametrize("DQ,DV,width,share", [(128, 256, 256, 2.0), (256, 512, 256, 1.95), (64, 128, 128, 2.0), (128, 256, 256, 0.9)])
 def test_rounds(DQ, DV, width, share):
