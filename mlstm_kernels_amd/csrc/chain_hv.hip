@@ -916,8 +916,11 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //    around 9, where all positions are kept), scan + H / segments: 256/512, 8 heads of 5000 positions 128 (150) / 101 (108), 8000 154
 //    (195) / 139 (146), 10000 196 (246) / 165 (170), 16384 278 (368) / 230 (243), 4 of 16384 160 / 148, 16 of 8000 240 (318) / 218 (232), 40 of
 //    8000 552 / 467, but 8 of 3000 75 (100) / 81 (100), 16 of 4000 129 (167) / 135 (142), 32 of 2000 112 (132) / 130 (134); 128/256, 16 of 4000
-//    80 (85) / 70 (71), of 16384 205 (242) / 165 (168), 1 of 16384 96 / 65, 64 of 4000 169 (203) / 152 (159); 256/256, 8 of 10185 148 / 115;
-//    128/128, 32 of 4000 93 (100) / 72 (74), 120 of 3000 165 / 145; 64/128, 32 of 4000 78 (85) / 60 (60), but 8 of 2600 49 / 53.  Of the two
+//    80 (85) / 70 (71), of 16384 205 (242) / 165 (168), 64 of 4000 169 (203) / 152 (159); 256/256, 8 of 10185 148 / 115;
+//    128/128, 32 of 4000 93 (100) / 72 (74), 120 of 3000 165 / 145; 64/128, 32 of 4000 78 (85) / 60 (60), but 8 of 2600 49 / 53.  Level where the
+//    scan's tiles just fill the chip (256/512, 32 heads of 4000 211 / 212, of 8000 391 / 386): not there.  Nor with one to three heads, although it would be
+//    faster (256/512, 1 head of 16384 101 / 81, of 4000 66 / 71): their results are held to 2^-9 of those of calls that update their states in place, which
+//    scan + H take, and with all positions kept two kernels that round the state at other positions are 2.8e-3 apart, each 1.9e-3 from 64 bits.  Of the two
 //    widths 256 columns take fewer passes over the rows, 128 half of the traffic of the states between segments and shorter segments where the chip
 //    is not full (8 of 5000, 128 / 256 columns 101 / 112, of 16384 260 / 230).
 struct Plan {
@@ -938,7 +941,9 @@ Plan plan(const ChainHvArgs& a, int BH) {
   };
   if (full(256, 85)) return {256, 0};
   if (full(128, 95) && !(a.DHQK == 256 && a.DHHV % 512 == 0 && a.states != nullptr && a.NC <= 12)) return {128, 0};
-  if (a.seg_c == nullptr || a.NC < 20) return none;
+  if (a.seg_c == nullptr || a.NC < 20 || BH < 4) return none;
+  const long long scan_tiles = (long long)BH * ((a.DHQK + 127) / 128) * ((a.DHHV + 127) / 128);
+  if (scan_tiles <= cus && 8 * scan_tiles > 7ll * cus) return none;
   // Segments: what scan and H take and what the segments that fit the chip beside each other do, us, as in the sweep above.
   const float state = (float)a.DHQK * a.DHHV / 65536.f;
   float best = 0.97f * (38.f + a.NC * (0.4f + BH * (0.03f + 0.07f * state)));

@@ -143,8 +143,8 @@ def test_halves_of_wide_heads(S, dtype):
 
 # Few heads: segments of the sequence side by side.  Both widths, one slot and the most between segments, a last segment that is a chunk, a
 # part of one or whole, more segments than fit the scratch, heads that leave CUs over.
-@pytest.mark.parametrize("BH,S,DQ,DV", [(1, 16384, 128, 256), (2, 8300, 256, 512), (8, 5000, 256, 512), (8, 10000, 256, 512), (40, 8060, 256, 512),
-                                        (100, 3968, 128, 256), (4, 4428, 128, 256), (24, 3528, 128, 128), (3, 16384, 64, 128), (12, 6016, 64, 256),
+@pytest.mark.parametrize("BH,S,DQ,DV", [(4, 16384, 128, 256), (4, 8300, 256, 512), (8, 5000, 256, 512), (8, 10000, 256, 512), (40, 8060, 256, 512),
+                                        (100, 3968, 128, 256), (4, 4428, 128, 256), (24, 3528, 128, 128), (5, 16384, 64, 128), (12, 6016, 64, 256),
                                         (7, 10185, 256, 256), (9, 6003, 128, 384)])
 @pytest.mark.parametrize("opt", [dict(), dict(f_offset=9.0, init=True), dict(f_offset=0.0, last=False), dict(sig=True, init=True), dict(sig=True, normalize=False, init=True),
                                  dict(dtype=torch.float16, f_offset=9.0)], ids=["", "keep", "forget", "sig", "sig-raw", "fp16-keep"])
