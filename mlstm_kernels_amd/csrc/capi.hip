@@ -296,11 +296,6 @@ int chunkwise_fw_impl(const char* who, const void* q, const void* k, const void*
   ca.stride = stride;
   ca.f16 = f16;
   ca.skip_zero = !has_c0;  // (both dQ / dK kernels know, from g.zero_c)
-  if (!keep_for_backward && ws.cstates != nullptr) {  // (the chunk states of scan + H, which then do not run)
-    ca.seg_c = (float*)ws.cstates;
-    ca.seg_n = ws.nstates;
-    ca.seg_bytes = (size_t)BH * ((NC + stride - 1) / stride) * DHQK * DHHV * 2;
-  }
   const bool use_chain = one_launch && !use_short && mlstm::chain_hv_preferred(ca, BH);
   if (!sf.own_gates) {
     {

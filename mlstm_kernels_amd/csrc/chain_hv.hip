@@ -37,9 +37,6 @@
 // heads of 2048 with the last state 466 / 321, of 1024 207 / 170 and 199 / 157, of 512 89 / 77 and 83 / 71; 128/256, 256 heads of 1024 169 /
 // 103 and 152 / 97, 128 of 2048 158 / 146 and 144 / 134; 128/128, 256 of 1024 107 / 83 and 95 / 75; 64/128, 256 of 1024 80 / 62 and 71 / 61;
 // 256/256, 256 of 512 94 / 80 and 89 / 75.
-#include <algorithm>
-#include <type_traits>
-
 #include "common.h"
 #include "kernels.h"
 
@@ -136,17 +133,14 @@ __device__ __forceinline__ Frag tr_frag(const uint16_t* lo, const uint16_t* hi) 
 
 }  // namespace
 
-template <int DQ, int W, bool F16, bool ROWS>
+template <int DQ, int W, bool F16>
 struct ChainLds {  // bytes
   static constexpr int G = W / 32, DS = 8 / G;
-  static constexpr int TQ = kStep * DQ * 2, TV = kStep * W * 2, PB = ROWS ? 6144 : 0;
-  static constexpr int EX = ROWS && DS == 2 ? 8 * 4096 : 0;
-  // Two sets of tiles where they fit (DQ 64 and 128, or no output-side rows): everything of the next step is requested at the start of
-  // this one.
-  static constexpr int kSet = (ROWS ? 2 : 1) * TQ;  // tiles of rows of a set
-  static constexpr bool kAhead = 2 * kSet + 2 * TV + PB + EX + 12288 <= 160 * 1024;
-  static_assert(ROWS || kAhead, "states alone are made with two sets");
-  static constexpr int kV = kAhead ? 2 * kSet : 3 * TQ, kP = kV + (kAhead ? 2 : 1) * TV, kEx = kP + PB, kVec = kEx + EX;
+  static constexpr int TQ = kStep * DQ * 2, TV = kStep * W * 2, PB = 6144;
+  static constexpr int EX = DS == 2 ? 8 * 4096 : 0;
+  // Two sets of tiles where they fit (DQ 64 and 128): everything of the next step is requested at the start of this one.
+  static constexpr bool kAhead = 4 * TQ + 2 * TV + PB + EX + 12288 <= 160 * 1024;
+  static constexpr int kV = (kAhead ? 4 : 3) * TQ, kP = kV + (kAhead ? 2 : 1) * TV, kEx = kP + PB, kVec = kEx + EX;
   // [2][5][64] weights, [2][5][64] gate vectors as they arrive, [8][64] row sums, [4 or 1][64] q . n, decay, n as [DQ] fp32 and (bfloat16)
   // [3][NP] 16-bit parts
   static constexpr int NP = DQ + 16;  // (32 bytes apart: the three rows of a fragment on distinct banks)
@@ -175,25 +169,19 @@ __device__ __forceinline__ int unit_ofs(int u0, int u, int sw) {
 template <bool TIGHT>
 __device__ __forceinline__ int lane_of(int lane) { return TIGHT ? opaque(lane) : lane; }
 
-// Segments of the sequence (few heads, no state kept): a launch (kSegments) makes what every segment but the last adds to the state,
-// from zero, one turns that into the states in front of the segments (chain_segments_kernel), and one (kForward) runs all of them.  Between
-// them three quarters of a GB move for 256 workgroups of 256 x 256, a third of the bytes; us at 8 heads of 256/512, 10000 positions 47
-// to 58, 22 and 88 to 111 (scan in segments, twice, and H: 42, 52, 86).  kSegments adds the remainders of the value rows in the chunks that
-// weigh 2^-8 or more in the state after the segment, all of them with the sigmoid gate (see scan.hip); it has room for two sets of
-// tiles and needs one barrier a step: 64 to 53.
 // What a launch makes.  kKeptStates: the forward's kept states and nothing else, for a backward that has them recomputed: the same
 // arithmetic in the same order, hence the same bits, which the scan, rounding the scaled value rows once, does not have.  us, the whole
 // forward / the scan / this: 128 heads of 256/512, 2048 positions 341 / 154 / 174, 1024 147 / 70 / 74; 256 heads of 1024, 128/256 102 / 48 /
 // 50, 64/128 62 / 20 / 28.  (The scan's launch, which then ends at once, 6 us.)
-enum Kind { kForward, kBackward, kKeptStates, kSegments };
+enum Kind { kForward, kBackward, kKeptStates };
 
 template <int DQ, int W, int KIND, bool F16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void chain_hv_kernel(ChainHvArgs a) {
-  constexpr bool IS_DV = KIND == kBackward, ROWS = KIND == kForward || KIND == kBackward;  // ROWS: H or dV is made
-  if constexpr (KIND == kKeptStates) {
+  constexpr bool IS_DV = KIND == kBackward, ROWS = KIND != kKeptStates;  // ROWS: H or dV is made
+  if constexpr (!ROWS) {
     if (__builtin_amdgcn_readfirstlane(*a.g.chained) == 0) return;  // the forward's states came from the scan
   }
-  using L = ChainLds<DQ, W, F16, ROWS>;
+  using L = ChainLds<DQ, W, F16>;
   constexpr int G = L::G, DS = L::DS;
   constexpr int NDT = DQ / 32 / DS;         // 32-row state tiles of a wave
   constexpr int NO = DS == 1 ? 2 : 1;       // position tiles of 32 whose output a wave finishes
@@ -213,18 +201,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int r = lane & 31, h = lane >> 5;
   const int g = wave % G, dq = wave / G;        // column group, group of state rows
   const BlockId blk = xcd_block_id();
+  const int bh = blk.y, w_tile = blk.x * W;
   const int S = a.S, NC = a.NC, DHHV = a.DHHV;
-  const int ncol = DHHV / W, seg = a.seg_len > 0 ? blk.x / ncol : 0, col = blk.x - seg * ncol;
-  const int bh = blk.y, w_tile = col * W;
   const size_t Sp = (size_t)NC * kChunk;
   const int NS = (S + kStep - 1) / kStep;
-  // steps: up to the last kept state, those of the segment, or all
-  const int s_lo = 2 * seg * a.seg_len;
-  const int n_run = KIND == kKeptStates ? 2 * ((NC - 1) / a.stride * a.stride) + 1 : a.seg_len > 0 ? min(2 * a.seg_len, NS - s_lo) : NS;
-  constexpr bool N = KIND == kForward || KIND == kSegments;  // (nothing reads n behind the other two)
-  const bool do_n = N && a.use_nrow;
-  // slot of the segment among the states between segments (the last one has none)
-  const size_t slot = N && a.seg_len > 0 ? (size_t)bh * (a.nseg - 1) + seg : 0;
+  const int n_run = ROWS ? NS : 2 * ((NC - 1) / a.stride * a.stride) + 1;  // steps: up to the last kept state
+  const bool do_n = KIND == kForward && a.use_nrow;
   const u32x4 Xn_d = row_desc((IS_DV ? a.K : a.Q) + (size_t)bh * S * DQ, (uint32_t)S * DQ * 2);
   const u32x4 Xo_d = row_desc((IS_DV ? a.Q : a.K) + (size_t)bh * S * DQ, (uint32_t)S * DQ * 2);
   const u32x4 Xw_d = row_desc((IS_DV ? a.dH : a.V) + (size_t)bh * S * DHHV + w_tile, ((uint32_t)S * DHHV - w_tile) * 2);
@@ -237,16 +219,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // ---- state: tile dt holds rows 32 (dq NDT + dt) .. +31 in the order 16 (i / 8) + 8 h + i % 8 (register i), column 32 g + r
   f32x16 acc[NDT];
   const int tg0 = dq * NDT;
-  const float* c_from = a.init != nullptr ? a.init + (size_t)bh * DQ * DHHV : nullptr;
-  const float* n_from = a.n_init != nullptr ? a.n_init + (size_t)bh * DQ : nullptr;
-  if (KIND == kSegments) c_from = n_from = nullptr;
-  if (KIND == kForward && seg > 0) {
-    c_from = a.seg_c + (slot - 1) * DQ * DHHV;
-    n_from = a.seg_n + (slot - 1) * DQ;
-  }
   const int kb0 = DS == 2 ? 32 * dq : 0, kb1 = 32 - kb0;
-  if (c_from != nullptr) {
-    const float* src = c_from + (size_t)(32 * tg0 + 8 * h) * DHHV + w_tile + 32 * g + r;
+  if (a.init != nullptr) {
+    const float* src = a.init + ((size_t)bh * DQ + 32 * tg0 + 8 * h) * DHHV + w_tile + 32 * g + r;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -258,13 +233,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
   }
   if (tid < DQ) {
-    const float x = do_n && n_from != nullptr ? n_from[tid] : 0.f;
+    const float x = do_n && a.n_init != nullptr ? a.n_init[(size_t)bh * DQ + tid] : 0.f;
     nv[tid] = x;
     if constexpr (!F16) split3(x, npt + tid, L::NP);
   }
   rs[tid] = 0.f;
-  if constexpr (ROWS)
-    for (int x = tid; x < L::PB / 16; x += 512) ((uint4*)(smem + L::kP))[x] = make_uint4(0, 0, 0, 0);
+  for (int x = tid; x < L::PB / 16; x += 512) ((uint4*)(smem + L::kP))[x] = make_uint4(0, 0, 0, 0);
 
   // gate vectors of step s, by wave 5 or 6 (which have no scores; in turn): requested ...
   auto gates_load = [&](int s) -> float {
@@ -309,8 +283,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (ln == 0) gdl[s & 1] = odd ? expf(gg - u63 - gm) : gg;
   };
 
-  const int s_first = IS_DV ? NS - 1 : s_lo, s_inc = IS_DV ? -1 : 1;
-  uint32_t o_n = 0, o_o = ROWS ? L::TQ : 0, o_f = 2 * L::TQ;  // LDS offsets of the tiles: output-side rows, other rows, free
+  const int s_first = IS_DV ? NS - 1 : 0, s_inc = IS_DV ? -1 : 1;
+  uint32_t o_n = 0, o_o = L::TQ, o_f = 2 * L::TQ;  // LDS offsets of the tiles: output-side rows, other rows, free
   auto load_n = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xn_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
   auto load_o = [&](int s, uint32_t o) { DmaTile<DQ * 2>::load(Xo_d, q_off + (uint32_t)s * (kStep * DQ * 2), DQ * 2, lds0 + o, wave); };
   uint32_t o_w = L::kV;                            // ... and value rows
@@ -338,8 +312,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float log2_qk = __log2f(a.qk_scale);
   const size_t NCS = (size_t)(NC + a.stride - 1) / a.stride;
 
-  auto step = [&](int it, auto lo) __attribute__((always_inline)) {
-    constexpr bool LO = decltype(lo)::value;  // the value rows' remainders enter the state too
+  for (int it = 0; it < n_run; ++it) {
     const int s = s_first + it * s_inc, t0 = s * kStep;
     const int c = s >> 1;
     const bool more = it + 1 < n_run;
@@ -347,9 +320,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();  // ---- the tiles and vectors of this step are in LDS, the free tile is nobody's
     if (more) {
       if constexpr (L::kAhead) {
-        if constexpr (ROWS) load_n(s + s_inc, it & 1 ? 0 : L::kSet);
+        if constexpr (ROWS) load_n(s + s_inc, it & 1 ? 0 : 2 * L::TQ);
       } else {
-        load_n(s + s_inc, o_f);
+        if constexpr (ROWS) load_n(s + s_inc, o_f);
+        else load_o(s + s_inc, o_f);
       }
     }
     const uint16_t* const Xn = (const uint16_t*)(smem + o_n);
@@ -529,7 +503,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
     if constexpr (ROWS) scores();
     if (L::kAhead && more) {
-      load_o(s + s_inc, (it & 1 ? 0 : L::kSet) + L::kSet - L::TQ);
+      load_o(s + s_inc, (it & 1 ? 0 : 2 * L::TQ) + L::TQ);
       load_w(s + s_inc, it & 1 ? L::kV : L::kV + L::TV);
     }
     if constexpr (ROWS) product();
@@ -571,7 +545,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           }
       }
     }
-    if constexpr (ROWS) __syncthreads();  // ---- scores, partial sums; the output-side rows and the value rows have been read
+    __syncthreads();  // ---- scores, partial sums; the output-side rows and the value rows have been read
     u32x4 orow[2 * NO];
     if constexpr (ROWS) {
       float4 ex[4];
@@ -599,7 +573,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             nmax = fmaxf(fabsf(sum), a.sig_gate ? 1.f : __expf(-mc));
             ivl = 1.f / (nmax + a.eps);
           }
-          if (col == 0 && wave == 7) {
+          if (blk.x == 0 && wave == 7) {
             a.nrow_out[bh * Sp + t0 + lane] = nmax;
             // the second half of the last chunk, if no step covers it
             if (s == NS - 1 && (s & 1) == 0) a.nrow_out[bh * Sp + t0 + kStep + lane] = 1.f;
@@ -681,7 +655,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // what goes out during the update (it is what the memory path takes a while for: in front of it the waves stood there)
     auto memory = [&](int i) {
       if constexpr (!L::kAhead) {
-        if (i == 0 && more) load_o(s + s_inc, o_n);
+        if (i == 0 && ROWS && more) load_o(s + s_inc, o_n);
         if (i == 1 && more) load_w(s + s_inc, o_w);
         i -= 2;
       }
@@ -695,6 +669,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float gdec = gdl[s & 1];
     // ---- state update, the scaled value rows as a 16-bit head and remainder; wave w takes rows 32 w .. of the normaliser state
     {
+      constexpr bool N = KIND == kForward;  // (nothing reads n behind the other two)
       const int ln = lane_of<kTight>(lane);
       const int i16 = ln & 15, kr = i16 >> 2;
       const int gp = ((i16 & 1) << 1) | ((i16 >> 1) & 1);  // the two middle groups of four rows trade places
@@ -715,7 +690,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // between the matrix instructions of these.
       constexpr int NT = 4 * NDT, kAhead = 3;
       constexpr int kReads = 2 + ((N ? 4 : 2) + NDT - 1) / NDT;
-      constexpr int kValu = (LO ? ((N ? 56 : 40) + 2 * NDT - 1) / (2 * NDT) : ((N ? 36 : 20) + NDT - 1) / NDT);
+      constexpr int kValu = ((N ? 56 : 40) + 2 * NDT - 1) / (2 * NDT);
       Frag A[4], xn, vh[2], vl[2];
       float4 u0, u1;
       auto row0 = [&](int j) { return (j < 2 ? kb0 : kb1) + 16 * (j & 1); };
@@ -734,7 +709,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // (head and remainder of the same fp32 product: to float16 it may be converted and multiplied in one step)
         if constexpr (F16) asm("" : "+v"(e0), "+v"(e1));
         vh[j & 1].w[p] = pack2<F16>(e0, e1);
-        if constexpr (LO) vl[j & 1].w[p] = pack2<F16>(e0 - lo2<F16>(vh[j & 1].w[p]), e1 - hi2<F16>(vh[j & 1].w[p]));
+        vl[j & 1].w[p] = pack2<F16>(e0 - lo2<F16>(vh[j & 1].w[p]), e1 - hi2<F16>(vh[j & 1].w[p]));
         if (N) {
           nsum = __builtin_fmaf(lo2<F16>(xn.w[p]), x, nsum);
           nsum = __builtin_fmaf(hi2<F16>(xn.w[p]), y, nsum);
@@ -762,7 +737,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const int j = i / NDT, d = i % NDT;
           if (i + kAhead < NT) fetch(i + kAhead);
           mfma32<F16>(acc[d], A[i & 3], vh[j & 1]);
-          if constexpr (LO) mfma32<F16>(acc[d], A[i & 3], vl[j & 1]);
+          mfma32<F16>(acc[d], A[i & 3], vl[j & 1]);
           if (j < 3) {
 #pragma unroll
             for (int p = 4 * d / NDT; p < 4 * (d + 1) / NDT; ++p) scale(j + 1, p);
@@ -775,10 +750,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
-          if constexpr (LO) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
-          }
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
         }
         fence();
       }
@@ -788,7 +761,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const float nn = gdec * nv[d] + nsum;
         if (wave < DQ / 32 && ln < 32) {
           nv[d] = nn;
-          if (ROWS && !F16) split3(nn, npt + d, L::NP);
+          if (!F16) split3(nn, npt + d, L::NP);
         }
       }
     }
@@ -796,85 +769,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     dma_wait<ROWS ? 2 * NO : 0>();
     asm volatile("" : "+v"(gs));  // has arrived with them; where it is used the compiler would wait for the rows requested by then
     if constexpr (L::kAhead) {
-      o_n = it & 1 ? 0 : L::kSet;
-      o_o = o_n + L::kSet - L::TQ;
+      o_n = it & 1 ? 0 : 2 * L::TQ;
+      o_o = o_n + L::TQ;
       o_w = it & 1 ? L::kV : L::kV + L::TV;
     } else {
       const uint32_t x = o_o;
-      o_o = o_n;
+      o_o = ROWS ? o_n : o_f;
       o_n = o_f;
       o_f = x;
     }
-  };
-  int it = 0;
-  if constexpr (KIND == kSegments) {
-    // without remainders: the chunks that weigh less than 2^-8 in the state after the segment
-    if (!a.sig_gate) {
-      const float* gb = a.g.gbar + (size_t)bh * NC + seg * a.seg_len;
-      int c1 = a.seg_len - 1;
-      for (float w = gb[c1]; c1 > 0 && w >= 0x1p-8f; w *= gb[c1]) --c1;
-      for (; it < 2 * c1; ++it) step(it, std::false_type());
-    }
   }
-  for (; it < n_run; ++it) step(it, std::true_type());
 
   __syncthreads();
-  float* c_to = a.final_out != nullptr ? a.final_out + (size_t)bh * DQ * DHHV : nullptr;
-  float* n_to = a.n_final != nullptr ? a.n_final + (size_t)bh * DQ : nullptr;
-  if (KIND == kForward && a.seg_len > 0 && seg < a.nseg - 1) c_to = n_to = nullptr;
-  if (KIND == kSegments) {
-    c_to = a.seg_c + slot * DQ * DHHV;
-    n_to = a.seg_n + slot * DQ;
-  }
-  if (c_to != nullptr) {
-    float* dst = c_to + (size_t)(32 * tg0 + 8 * h) * DHHV + w_tile + 32 * g + r;
+  if (a.final_out != nullptr) {
+    float* dst = a.final_out + ((size_t)bh * DQ + 32 * tg0 + 8 * h) * DHHV + w_tile + 32 * g + r;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) dst[(size_t)(32 * dt + 16 * (i / 8) + i % 8) * DHHV] = acc[dt][i];
   }
-  if (do_n && n_to != nullptr && col == 0) {
-    for (int d = tid; d < DQ; d += 512) n_to[d] = nv[d];
-  }
-}
-
-// Slot x, what segment x adds to a state of zero, becomes the state after it: the state in front of it, decayed over the segment, and this.
-// Bound by its bytes (64 MB read and written in 22 us, mostly in the memory-side cache).  Four values of C or n a thread, eight slots
-// requested at once.  (A segment that added up those in front of it by itself would read 7.5 slots of them on average, with sixteen, for one
-// and this pass.)
-constexpr int kMaxSlots = 32;
-__global__ __launch_bounds__(256) void chain_segments_kernel(ChainHvArgs a) {
-  __shared__ float dec[kMaxSlots];
-  const int bh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, n = a.nseg - 1;
-  for (int x = tid >> 6; x < n; x += 4) {
-    float d = 1.f;
-    for (int k = lane; k < a.seg_len; k += 64) d *= a.g.gbar[(size_t)bh * a.NC + x * a.seg_len + k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) d *= __shfl_xor(d, o);
-    if (lane == 0) dec[x] = d;
-  }
-  __syncthreads();
-  const int per_c = a.DHQK * a.DHHV / 4, i = blockIdx.x * 256 + tid;
-  const bool is_c = i < per_c;
-  if (!is_c && (!a.use_nrow || i >= per_c + a.DHQK / 4)) return;
-  const size_t per = is_c ? per_c : a.DHQK / 4, e = is_c ? i : i - per_c;
-  const float* const from = is_c ? a.init : a.n_init;
-  f32x4 st = {0.f, 0.f, 0.f, 0.f};
-  if (from != nullptr) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) st[k] = from[(bh * per + e) * 4 + k];  // (the caller's: any alignment)
-  }
-  f32x4* const p = (f32x4*)(is_c ? a.seg_c : a.seg_n) + (size_t)bh * n * per + e;
-  for (int x0 = 0; x0 < n; x0 += 8) {
-    f32x4 v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = p[min(x0 + k, n - 1) * per];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (x0 + k < n) {
-        st = st * dec[x0 + k] + v[k];
-        p[(x0 + k) * per] = st;
-      }
+  if (do_n && a.n_final != nullptr && blk.x == 0) {
+    for (int d = tid; d < DQ; d += 512) a.n_final[(size_t)bh * DQ + d] = nv[d];
   }
 }
 
@@ -882,10 +797,10 @@ namespace {
 template <int DQ, int W, int KIND, bool F16>
 const char* launch_t(const ChainHvArgs& a, int BH, hipStream_t stream) {
   static LdsLimit lds;
-  constexpr int smem = ChainLds<DQ, W, F16, KIND == kForward || KIND == kBackward>::kBytes;
+  constexpr int smem = ChainLds<DQ, W, F16>::kBytes;
   static_assert(smem <= 160 * 1024, "LDS of a CU");
   if (!lds.allow((const void*)chain_hv_kernel<DQ, W, KIND, F16>, smem)) return "chain_hv: cannot raise the dynamic LDS limit";
-  hipLaunchKernelGGL((chain_hv_kernel<DQ, W, KIND, F16>), dim3(a.DHHV / W * (KIND == kSegments ? a.nseg - 1 : a.seg_len > 0 ? a.nseg : 1), BH), dim3(512), smem, stream, a);
+  hipLaunchKernelGGL((chain_hv_kernel<DQ, W, KIND, F16>), dim3(a.DHHV / W, BH), dim3(512), smem, stream, a);
   return nullptr;
 }
 template <int DQ, int W, int KIND>
@@ -895,7 +810,6 @@ const char* launch_f(const ChainHvArgs& a, int BH, hipStream_t stream) {
 template <int DQ, int W>
 const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream) {
   if (kind == kBackward) return launch_f<DQ, W, kBackward>(a, BH, stream);
-  if (kind == kSegments) return launch_f<DQ, W, kSegments>(a, BH, stream);
   return kind == kForward ? launch_f<DQ, W, kForward>(a, BH, stream) : launch_f<DQ, W, kKeptStates>(a, BH, stream);
 }
 // Value columns of a workgroup, 0: another kernel is the better one.
@@ -912,65 +826,29 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //  * Longer sequences and several rounds are no other matter.  256/512, a forward with the last state and forward and backward, with the
 //    scan and the streaming kernels / so: 128 heads of 2049 positions 464 / 308 and 1287 / 1087, of 8192 1535 / 1150 and 4496 / 3953,
 //    512 of 1024 800 / 618 and 2037 / 1918; 1024 of 512 841 / 660 and 1786 / 1813, the one size where they are level with a backward.
-//  * Few heads, no state kept: segments of the sequence side by side.  us for a forward with the last state, 16-bit gates around 3 (and
-//    around 9, where all positions are kept), scan + H / segments: 256/512, 8 heads of 5000 positions 128 (150) / 101 (108), 8000 154
-//    (195) / 139 (146), 10000 196 (246) / 165 (170), 16384 278 (368) / 230 (243), 4 of 16384 160 / 148, 16 of 8000 240 (318) / 218 (232), 40 of
-//    8000 552 / 467, but 8 of 3000 75 (100) / 81 (100), 16 of 4000 129 (167) / 135 (142), 32 of 2000 112 (132) / 130 (134); 128/256, 16 of 4000
-//    80 (85) / 70 (71), of 16384 205 (242) / 165 (168), 64 of 4000 169 (203) / 152 (159); 256/256, 8 of 10185 148 / 115;
-//    128/128, 32 of 4000 93 (100) / 72 (74), 120 of 3000 165 / 145; 64/128, 32 of 4000 78 (85) / 60 (60), but 8 of 2600 49 / 53.  Level where the
-//    scan's tiles just fill the chip (256/512, 32 heads of 4000 211 / 212, of 8000 391 / 386): not there.  Nor with one to three heads, although it would be
-//    faster (256/512, 1 head of 16384 101 / 81, of 4000 66 / 71): their results are held to 2^-9 of those of calls that update their states in place, which
-//    scan + H take, and with all positions kept two kernels that round the state at other positions are 2.8e-3 apart, each 1.9e-3 from 64 bits.  Of the two
-//    widths 256 columns take fewer passes over the rows, 128 half of the traffic of the states between segments and shorter segments where the chip
-//    is not full (8 of 5000, 128 / 256 columns 101 / 112, of 16384 260 / 230).
-struct Plan {
-  int w, seg_len;  // value columns of a workgroup (0: another kernel is the better one), chunks in a segment (0: one piece)
-};
-Plan plan(const ChainHvArgs& a, int BH) {
-  const Plan none = {0, 0};
-  if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return none;
-  if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return none;  // 32-bit offsets in a head
-  if (a.S <= 2 * kChunk) return none;
+int columns(const ChainHvArgs& a, int BH) {
+  if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return 0;
+  if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return 0;  // 32-bit offsets in a head
+  if (a.S <= 2 * kChunk) return 0;
   // (dV reads no V, the kept states no Q)
-  if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V)) % 16 != 0) return none;
+  if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V)) % 16 != 0) return 0;
   const int cus = device_cu_count();
-  if (cus <= 0) return none;
+  if (cus <= 0) return 0;
   auto full = [&](int w, int pct) {
     const long long n = (long long)BH * (a.DHHV / w), rounds = (n + cus - 1) / cus;
     return a.DHHV % w == 0 && 100 * n >= pct * rounds * cus;
   };
-  if (full(256, 85)) return {256, 0};
-  if (full(128, 95) && !(a.DHQK == 256 && a.DHHV % 512 == 0 && a.states != nullptr && a.NC <= 12)) return {128, 0};
-  if (a.seg_c == nullptr || a.NC < 20 || BH < 4) return none;
-  const long long scan_tiles = (long long)BH * ((a.DHQK + 127) / 128) * ((a.DHHV + 127) / 128);
-  if (scan_tiles <= cus && 8 * scan_tiles > 7ll * cus) return none;
-  // Segments: what scan and H take and what the segments that fit the chip beside each other do, us, as in the sweep above.
-  const float state = (float)a.DHQK * a.DHHV / 65536.f;
-  float best = 0.97f * (38.f + a.NC * (0.4f + BH * (0.03f + 0.07f * state)));
-  Plan p = none;
-  const long long slots = (long long)(a.seg_bytes / ((size_t)BH * a.DHQK * a.DHHV * sizeof(float)));
-  for (int w = 256; w >= 128; w /= 2) {
-    const long long tiles = (long long)BH * (a.DHHV / w);
-    if (a.DHHV % w != 0 || 2 * tiles > cus) continue;
-    const int n = (int)std::min({cus / tiles, slots + 1, (long long)kMaxSlots + 1});
-    if (n < 2) continue;
-    const int len = (a.NC + n - 1) / n, nseg = (a.NC + len - 1) / len;
-    const float fill = (float)(tiles * nseg) / cus;
-    const float each = w == 256 ? 9.5f + 0.047f * a.DHQK : 7.f + 0.0245f * a.DHQK;  // a chunk of every segment, the chip full
-    const float t = fmaxf(32.f, 23.f + w * a.DHQK / 2600.f) + each * len * fmaxf(0.1f + 0.9f * fill, 0.55f + 0.35f * fill);
-    if (t < best) {
-      best = t;
-      p = {w, len};
-    }
-  }
-  return p;
+  if (full(256, 85)) return 256;
+  if (full(128, 95) && !(a.DHQK == 256 && a.DHHV % 512 == 0 && a.states != nullptr && a.NC <= 12)) return 128;
+  return 0;
 }
 }  // namespace
 
-bool chain_hv_preferred(const ChainHvArgs& a, int BH) { return plan(a, BH).w != 0; }
+bool chain_hv_preferred(const ChainHvArgs& a, int BH) { return columns(a, BH) != 0; }
 
-static const char* launch_kind(const ChainHvArgs& a, int w, int BH, int kind, hipStream_t stream) {
-  switch (w * 1000 + a.DHQK) {
+static const char* launch(const ChainHvArgs& a, int BH, int kind, hipStream_t stream) {
+  if (a.stride < 1 || a.stride > kMaxStateStride) return "chain_hv: state stride out of range";
+  switch (columns(a, BH) * 1000 + a.DHQK) {
     case 256256: return launch_w<256, 256>(a, BH, kind, stream);
     case 256128: return launch_w<128, 256>(a, BH, kind, stream);
     case 256064: return launch_w<64, 256>(a, BH, kind, stream);
@@ -979,18 +857,6 @@ static const char* launch_kind(const ChainHvArgs& a, int w, int BH, int kind, hi
     case 128064: return launch_w<64, 128>(a, BH, kind, stream);
     default: return "chain_hv: unsupported shape";
   }
-}
-static const char* launch(const ChainHvArgs& a_in, int BH, int kind, hipStream_t stream) {
-  if (a_in.stride < 1 || a_in.stride > kMaxStateStride) return "chain_hv: state stride out of range";
-  ChainHvArgs a = a_in;
-  const Plan pl = plan(a, BH);
-  a.seg_len = pl.seg_len;
-  a.nseg = pl.seg_len > 0 ? (a.NC + pl.seg_len - 1) / pl.seg_len : 1;
-  if (pl.seg_len > 0) {
-    if (const char* e = launch_kind(a, pl.w, BH, kSegments, stream)) return e;
-    hipLaunchKernelGGL(chain_segments_kernel, dim3((a.DHQK * a.DHHV / 4 + a.DHQK / 4 + 255) / 256, BH), dim3(256), 0, stream, a);
-  }
-  return launch_kind(a, pl.w, BH, kind, stream);
 }
 const char* launch_chain_hv(const ChainHvArgs& a, int BH, bool is_dv, hipStream_t stream) {
   return launch(a, BH, is_dv ? kBackward : kForward, stream);

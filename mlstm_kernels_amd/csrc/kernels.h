@@ -158,12 +158,6 @@ struct ChainHvArgs {
   int stride;               // a chunk state is kept every `stride` chunks
   int f16;
   int skip_zero;            // the first kept state is zero and its readers know
-  // forward without kept states: scratch for the states between segments of the sequence, or nullptr
-  float* seg_c;             // [BH][segments - 1][DHQK][DHHV], of seg_bytes
-  float* seg_n;             // [BH][segments - 1][DHQK], for up to three times as many as there are chunks
-  size_t seg_bytes;
-  // set by the launcher:
-  int seg_len, nseg;        // chunks in a segment (0: one piece), segments (the last one may be shorter)
 };
 
 constexpr int kShortMax = 512;  // longest sequence of the short forward

@@ -141,14 +141,14 @@ def test_halves_of_wide_heads(S, dtype):
         assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3 and rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
 
 
-# Few heads: segments of the sequence side by side.  Both widths, one slot and the most between segments, a last segment that is a chunk, a
-# part of one or whole, more segments than fit the scratch, heads that leave CUs over.
+# Few heads and a long prompt, whose heads leave the chain kernel most of the chip: it is not taken, whether states are kept or not.  The last
+# states are held to the 1e-5 of a scan that carries the remainder of the value operand where it weighs.
 @pytest.mark.parametrize("BH,S,DQ,DV", [(4, 16384, 128, 256), (4, 8300, 256, 512), (8, 5000, 256, 512), (8, 10000, 256, 512), (40, 8060, 256, 512),
                                         (100, 3968, 128, 256), (4, 4428, 128, 256), (24, 3528, 128, 128), (5, 16384, 64, 128), (12, 6016, 64, 256),
                                         (7, 10185, 256, 256), (9, 6003, 128, 384)])
 @pytest.mark.parametrize("opt", [dict(), dict(f_offset=9.0, init=True), dict(f_offset=0.0, last=False), dict(sig=True, init=True), dict(sig=True, normalize=False, init=True),
                                  dict(dtype=torch.float16, f_offset=9.0)], ids=["", "keep", "forget", "sig", "sig-raw", "fp16-keep"])
-def test_segments(BH, S, DQ, DV, opt):
+def test_long_prompts_of_few_heads(BH, S, DQ, DV, opt):
     from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
 
@@ -170,7 +170,7 @@ def test_segments(BH, S, DQ, DV, opt):
         torch.cuda.synchronize()
     finally:
         _lib.profile_enable(False)
-    assert "chain_h" in _names()
+    assert "chain_h" not in _names()
     H, last = out if o["last"] else (out, None)
     L = max(y for y in range(1, 257) if S % y == 0)  # (the oracle's chunks)
     for h in {0, BH - 1}:
@@ -178,9 +178,9 @@ def test_segments(BH, S, DQ, DV, opt):
         fw = O.chunkwise_fw(*map(d, x), d(c0), d(n0), d(m0), chunk_size=L, siging=o["sig"], normalize=o["normalize"])
         assert rel_norm(d(H), fw["H"]) <= 6e-3 * (0.25 if o["dtype"] == torch.float16 else 1.0)
         if last is not None:
-            assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3
+            assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-5
             if o["normalize"]:
-                assert rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
+                assert rel_norm(d(last[1]), fw["n_last"]) <= 1e-5
 
 
 # two rounds of workgroups (the last head is in the second one), and a first round that is all there is, not quite full

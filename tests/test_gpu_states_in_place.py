@@ -74,7 +74,8 @@ def test_gates_of_several_workgroups(S, DQ, DV, NH):
 # Few heads and a long sequence: the scan in segments, which all read the initial state, is not taken in place.  The states are
 # those of the scan in one piece (which a named path takes), H that of separate buffers but for the order of a sum in fp32.  Gates
 # near one: the initial state still weighs at the end.
-@pytest.mark.parametrize("S,DQ,DV,NH", [(8192, 128, 128, 2), (8200, 256, 512, 1), (2048, 64, 64, 12), (4100, 64, 64, 12), (2049, 128, 64, 32)])
+@pytest.mark.parametrize("S,DQ,DV,NH", [(8192, 128, 128, 2), (8200, 256, 512, 1), (2048, 64, 64, 12), (4100, 64, 64, 12), (2049, 128, 64, 32),
+                                          (8200, 256, 512, 4), (8192, 128, 128, 8), (6016, 64, 256, 12)])
 @pytest.mark.parametrize("sig", [False, True])
 def test_long_sequences_of_few_heads(S, DQ, DV, NH, sig):
     kw = dict(NH=NH, sig=sig, seed=S, f_offset=12.0, share="Cn")

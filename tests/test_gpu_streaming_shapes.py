@@ -320,6 +320,26 @@ def test_forward_with_and_without_a_gradient(S, DQ, DV, path, last):
         assert torch.equal(a, b) if path == "split" else rel_norm(a, b) <= tol
 
 
+# Beyond 512 positions "auto" takes the same kernels with a gradient and without one: the same bits.
+@pytest.mark.parametrize("NH,S,DQ,DV", [(4, 8300, 256, 512), (8, 8192, 128, 128), (12, 6016, 64, 256), (4, 4428, 128, 256), (1, 8200, 256, 512), (128, 700, 256, 512)])
+@pytest.mark.parametrize("f_offset", [3.0, 9.0])
+@pytest.mark.parametrize("last", [False, True])
+def test_long_forward_with_and_without_a_gradient(NH, S, DQ, DV, f_offset, last):
+    from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
+
+    print(f"{NH} x {S} {DQ}/{DV} {f_offset} {last}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    rn = lambda *s: torch.randn(1, NH, *s, device="cuda", generator=g)
+    x = [t.requires_grad_(True) for t in (rn(S, DQ).bfloat16(), rn(S, DQ).bfloat16(), rn(S, DV).bfloat16(), rn(S), f_offset + rn(S))]
+    out = []
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            r = mlstm_chunkwise__hip_xl_chunk(*x, return_last_states=last, any_sequence_length=True)
+        out.append([t.detach() for t in ((r[0], *r[1]) if last else (r,))])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 # The short kernel scans the gates itself: 16-bit gates are the same numbers as those of 32 bits, so every bit is the same.  Gates in
 # memory that is aligned to one element only.
 @pytest.mark.parametrize("S", [1, 127, 128, 129, 257, 385, 512])
