@@ -816,9 +816,11 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //  * One workgroup takes a CU and the launch as long as its rounds: the last one has to be nearly full.  256 columns are the more
 //    efficient form (256/512, 96 heads of 1024, 192 workgroups: 158 us against 140 for scan + H; 128 heads 160 / 207: the line is at
 //    85 %); with 128 the state's rows are shared by two waves that both scale the value rows, and what is gained is less (128/256,
-//    128 heads 158 / 146, at 112 heads 138 / 146).  256/512, 64 heads, scan + stream_hv / so: forward with the last state, 320
-//    positions 57 / 40, 512 65 / 53, 768 97 / 72, 1000 106 / 90, 2000 211 / 184; forward and backward, 512 151 / 155, 1000 292 / 294, 1024
-//    299 / 300, 1280 420 / 394, 1536 463 / 456, 2048 599 / 574, 4096 1171 / 1136: with kept states from thirteen chunks on.
+//    128 heads 158 / 146, at 112 heads 138 / 146).  Not for half of the heads of 256/512, which would be
+//    faster (64 heads, scan + stream_hv / so: forward with the last state, 512 positions 63 / 49, 1000 107 / 89, 2000 201 / 169; forward and
+//    backward, 512 151 / 155, 1000 292 / 294, 2048 599 / 574): H is a little further from 64 bits than theirs (errors times 1e-3, gates around 3, 6, 9: 1000
+//    positions 2.357 2.343 2.353 / 2.365 2.372 2.367, 2000 2.355 2.411 2.365 / 2.363 2.379 2.375), and where only a forward without a gradient gains it
+//    would not have the bits of one with a gradient.
 //  * Rows move to LDS in pieces of 16 bytes without registers in between, which asks for addresses that are multiples of 16; the
 //    other kernels read theirs with ordinary loads, which do not.
 //  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 124 / 148, backward
@@ -839,7 +841,7 @@ int columns(const ChainHvArgs& a, int BH) {
     return a.DHHV % w == 0 && 100 * n >= pct * rounds * cus;
   };
   if (full(256, 85)) return 256;
-  if (full(128, 95) && !(a.DHQK == 256 && a.DHHV % 512 == 0 && a.states != nullptr && a.NC <= 12)) return 128;
+  if (full(128, 95) && !(a.DHQK == 256 && a.DHHV % 512 == 0)) return 128;
   return 0;
 }
 }  // namespace

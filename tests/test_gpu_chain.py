@@ -104,7 +104,7 @@ def test_options(DQ, DV, width, S, opt):
 
 # many steps: decays that add up, sums over a long walk; forget gates that forget, that mostly keep and that keep nearly all
 @pytest.mark.parametrize("DQ,DV,width,S", [(64, 128, 128, 2048), (64, 256, 256, 2111), (128, 128, 128, 4100), (128, 256, 256, 2017), (256, 128, 128, 2050),
-                                           (256, 512, 256, 2200), (256, 512, 128, 1600)])
+                                           (256, 512, 256, 2200), (256, 256, 128, 1600)])
 @pytest.mark.parametrize("opt", [dict(f_offset=0.0, last=True), dict(f_offset=3.0, init=True, last=True), dict(f_offset=9.0, last=True),
                                  dict(f_offset=3.0, dtype=torch.float16, last=True), dict(f_offset=9.0, dtype=torch.float16), dict(sig=True, last=True)],
                          ids=str)
@@ -112,10 +112,10 @@ def test_long(DQ, DV, width, S, opt):
     _run(_heads(DV, width), S, DQ, DV, seed=S, **opt)
 
 
-@pytest.mark.parametrize("S", [257, 321, 1000, 1024])
+@pytest.mark.parametrize("S", [257, 321, 1000, 1024, 1700])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
 def test_halves_of_wide_heads(S, dtype):
-    """Half of the heads that fill the chip with 256 columns a workgroup: 128, where no state is kept or there are thirteen chunks."""
+    """Half of the heads that fill the chip with 256 columns a workgroup: the scan and the streaming kernel, whether states are kept or not."""
     from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk
 
@@ -132,13 +132,13 @@ def test_halves_of_wide_heads(S, dtype):
         torch.cuda.synchronize()
     finally:
         _lib.profile_enable(False)
-    assert "chain_h" in _names()
+    assert "chain_h" not in _names()
     L = next(y for y in (64, 32, 16, 8, 4, 2, 1) if S % y == 0)
     for h in (0, BH - 1):
         d = lambda t: t[:, h:h + 1].double().cpu()
         fw = O.chunkwise_fw(*map(d, x), *map(d, st), chunk_size=L)
         assert rel_norm(d(H), fw["H"]) <= 6e-3 * (0.25 if dtype == torch.float16 else 1.0)
-        assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-3 and rel_norm(d(last[1]), fw["n_last"]) <= 1e-3
+        assert rel_norm(d(last[0]), fw["C_last"]) <= 1e-5 and rel_norm(d(last[1]), fw["n_last"]) <= 1e-5
 
 
 # Few heads and a long prompt, whose heads leave the chain kernel most of the chip: it is not taken, whether states are kept or not.  The last

@@ -321,7 +321,8 @@ def test_forward_with_and_without_a_gradient(S, DQ, DV, path, last):
 
 
 # Beyond 512 positions "auto" takes the same kernels with a gradient and without one: the same bits.
-@pytest.mark.parametrize("NH,S,DQ,DV", [(4, 8300, 256, 512), (8, 8192, 128, 128), (12, 6016, 64, 256), (4, 4428, 128, 256), (1, 8200, 256, 512), (128, 700, 256, 512)])
+@pytest.mark.parametrize("NH,S,DQ,DV", [(4, 8300, 256, 512), (8, 8192, 128, 128), (12, 6016, 64, 256), (4, 4428, 128, 256), (1, 8200, 256, 512), (128, 700, 256, 512),
+                                          (64, 513, 256, 512), (64, 700, 256, 512), (64, 1300, 256, 512), (64, 1700, 256, 512)])
 @pytest.mark.parametrize("f_offset", [3.0, 9.0])
 @pytest.mark.parametrize("last", [False, True])
 def test_long_forward_with_and_without_a_gradient(NH, S, DQ, DV, f_offset, last):
