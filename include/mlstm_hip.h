@@ -167,7 +167,8 @@ size_t mlstm_hip_chunkwise_fw_workspace_bytes(int B, int NH, int S, int DHQK, in
  *   chunk that still weighs at least 2^-8 in the last state, so c_last is accurate to ~1e-5 relative; with c_last
  *   NULL it rounds them once (as the replaced kernels do), which is up to a fifth faster and changes H only within
  *   the tolerance of its 16-bit operands.  The chain kernel carries the remainder in every step either way.
- *   q, k, v (and dH in the backward) may begin at any element; the chain kernel takes those at multiples of 16 bytes.
+ *   q, k, v and H (and dH and dV in the backward) may begin at any element; the chain kernel takes calls with all of them at multiples of
+ *   16 bytes.
  *   MLSTM_PATH_FUSED takes bf16 only.
  *   normalize applies to the sig gate only (0: H is the bare numerator).
  */

@@ -821,8 +821,9 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //    backward, 512 151 / 155, 1000 292 / 294, 2048 599 / 574): H is a little further from 64 bits than theirs (errors times 1e-3, gates around 3, 6, 9: 1000
 //    positions 2.357 2.343 2.353 / 2.365 2.372 2.367, 2000 2.355 2.411 2.365 / 2.363 2.379 2.375), and where only a forward without a gradient gains it
 //    would not have the bits of one with a gradient.
-//  * Rows move to LDS in pieces of 16 bytes without registers in between, which asks for addresses that are multiples of 16; the
-//    other kernels read theirs with ordinary loads, which do not.
+//  * Rows move to LDS in pieces of 16 bytes without registers in between, and rows of the output leave through a buffer descriptor, 16
+//    bytes a lane: both ask for addresses that are multiples of 16; the other kernels read and write theirs with ordinary instructions,
+//    which do not.
 //  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 124 / 148, backward
 //    93 / 137); at 320 128 heads take 74 / 50 and 68 / 47.
 //  * Longer sequences and several rounds are no other matter.  256/512, a forward with the last state and forward and backward, with the
@@ -832,8 +833,8 @@ int columns(const ChainHvArgs& a, int BH) {
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return 0;
   if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return 0;  // 32-bit offsets in a head
   if (a.S <= 2 * kChunk) return 0;
-  // (dV reads no V, the kept states no Q)
-  if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V)) % 16 != 0) return 0;
+  // (dV reads no V; the kept states read no Q and write no rows)
+  if (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)(a.dH != nullptr ? a.dH : a.V) | (uintptr_t)a.Out) % 16 != 0) return 0;
   const int cus = device_cu_count();
   if (cus <= 0) return 0;
   auto full = [&](int w, int pct) {

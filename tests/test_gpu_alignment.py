@@ -45,6 +45,58 @@ def test_rows(DQ, DV, width, moved, recompute):
         assert rel_norm(b, a) <= (8e-3 if name[1:] in ("I", "F") else 6e-3) * 2 ** 0.5, name
 
 
+# H and dV of a C caller in memory that is aligned to one element: the other kernels, and nothing beside the rows is written
+@pytest.mark.parametrize("DQ,DV,width", [(64, 128, 128), (128, 256, 256), (256, 512, 256)])
+@pytest.mark.parametrize("moved", ["H", "dV"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_output_rows(DQ, DV, width, moved, dtype):
+    from mlstm_kernels_amd import _lib
+    from mlstm_kernels_amd.torch.utils import current_stream_ptr, ptr
+
+    lib, dev = _lib.get_lib(), torch.device("cuda")
+    S, BH = 330, torch.cuda.get_device_properties(0).multi_processor_count // (DV // width)
+    print(f"{BH} x {S} {DQ}/{DV} {moved} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(DQ)
+    rn = lambda *s: torch.randn(1, BH, *s, device=dev, generator=g)
+    q, k, v, dH = (rn(S, d).to(dtype) for d in (DQ, DQ, DV, DV))
+    i, f = rn(S), 3 + rn(S)
+    code = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    nf = lib.mlstm_hip_chunkwise_fw_workspace_bytes(1, BH, S, DQ, DV, 1, _lib.PATH_AUTO, 0)
+    nb = lib.mlstm_hip_chunkwise_bw_workspace_bytes(1, BH, S, DQ, DV, 0)
+
+    def output(odd):  # a buffer of ones and the rows in it
+        buf = torch.ones(v.numel() + 16, dtype=dtype, device=dev)
+        return buf, buf[1 if odd else 8:][:v.numel()].view(v.shape)
+
+    out = []
+    for which in ("", moved):
+        (bh, H), (bv, dV) = output(which == "H"), output(which == "dV")
+        assert (H.data_ptr() % 16 == 0) == (which != "H") and (dV.data_ptr() % 16 == 0) == (which != "dV")
+        ws, bws = (torch.empty(n, dtype=torch.uint8, device=dev) for n in (nf, nb))
+        dQ, dK, dI, dF = torch.empty_like(q), torch.empty_like(k), torch.empty_like(i), torch.empty_like(f)
+        _lib.profile_read()
+        _lib.profile_enable(True)
+        try:
+            _lib.check(lib.mlstm_hip_chunkwise_fw(*[ptr(t) for t in (q, k, v, i, f)], None, None, None, ptr(H), *[None] * 5, ptr(ws), nf, 1,
+                                                  1, BH, S, DQ, DV, 1e-6, code, _lib.F32, _lib.GATE_EXP, 1, _lib.PATH_AUTO, 0, _lib.NORM_NONE,
+                                                  1e-6, None, None, current_stream_ptr(dev)), "forward")
+            _lib.check(lib.mlstm_hip_chunkwise_bw(*[ptr(t) for t in (q, k, v, i, f, dH)], None, *[ptr(t) for t in (dQ, dK, dV, dI, dF)], None,
+                                                  ptr(ws), nf, ptr(bws), nb, 1, BH, S, DQ, DV, 1e-6, code, _lib.F32, _lib.GATE_EXP, 1,
+                                                  _lib.PATH_AUTO, 0, current_stream_ptr(dev)), "backward")
+            torch.cuda.synchronize()
+        finally:
+            _lib.profile_enable(False)
+        names = set(_lib.profile_read())
+        assert ("chain_h" in names) == (which != "H") and ("chain_dv" in names) == (which != "dV")
+        for buf, rows in ((bh, H), (bv, dV)):
+            first = (rows.data_ptr() - buf.data_ptr()) // buf.element_size()
+            assert bool((buf[:first] == 1).all()) and bool((buf[first + rows.numel():] == 1).all())
+        out.append((H, dV, dQ, dK))
+    tol = (0.25 if dtype == torch.float16 else 1.0) * 6e-3 * 2 ** 0.5  # (as above)
+    for name, a, b in zip(("H", "dV", "dQ", "dK"), *out):
+        assert rel_norm(b, a) <= tol, name
+
+
 # a state between 32 and 112 MiB, whose stores go through the caches where they can
 @pytest.mark.parametrize("in_place", [False, True])
 def test_step_state(in_place):
