@@ -17,9 +17,9 @@
 //     requested in the first half of a step; with 256 the output-side rows go to a free tile, the other rows and the value rows, in the
 //     second half, where the present ones have been read.  Two barriers a step.
 //   * What goes through the memory path in the second half, requests and rows of the output, goes out between the matrix instructions of
-//     the update: in front of it the waves stood there (256/256 columns, of 15.9 thousand cycles a step 3.0 were the slower waves' wait;
-//     now 13.6), and a step ends when its requests are there, not when its output is written.  us, before / after: 128 heads of
-//     256/512, 2048 positions with the last state 277 / 257, dV of 1024 135 / 127; 128/256, 128 heads of 2048, 129 / 121 and 121 / 107.
+//     the update: in front of it the waves stood there, and a step ends when its requests are there, not when its output is written.
+//     With that, the two sets and the swizzles below, before / after: a step of 256/256 columns 15.9 / 14.1 thousand cycles; us, 128 heads of
+//     256/512, 2048 positions with the last state 276 / 260, dV of 1024 133 / 126; 128/256, 128 heads of 2048, 131 / 126 and 123 / 107.
 //   * Scores: 10 live tiles of 16 x 16, two a wave, gated in fp32 and written to LDS as operand fragments; q . n on the way as one more
 //     operand (three 16-bit parts of n, exactly).
 //   * The value rows are scaled in fp32 and enter the state as a 16-bit head and remainder: the state is rounded every 64 positions
@@ -29,14 +29,14 @@
 //     2.371, dV 2.363 / 2.366.  (Rows right behind a step's boundary take most of H from the rounded state; where a normaliser nearly
 //     cancels that weighs more: the 99th percentile of the rows is 2 % higher.)
 //   * The state takes its decay in every step.  Left in a factor until that reaches 2^-24, with weights that take it, the registers hold
-//     up to 2^24 times the state, which overflows with rows of 2^103 and above; and it gains nothing (us, forward, backward, so / now: 128
-//     heads of 256/512, 2048 positions 331 303 / 334 306, 256 heads of 1024, 128/256 103 97 / 102 96, 128/128 75 70 / 74 69, 64/128 61 60 / 59 60).
-// What bounds it: issue.  A step of 256 / 256 columns is 120 matrix and 800 vector instructions a wave, two waves a SIMD, which
-// overlap only where they are interleaved (a matrix instruction hides about six of its wave: the schedules below); matrix pipes 45 %
-// busy (128 columns: 24 %), LDS 32 %, memory 3.2 TB/s, every row read once.  us, forward / backward, scan + H (dV) and this: 256/512, 128
-// heads of 2048 with the last state 466 / 321, of 1024 207 / 170 and 199 / 157, of 512 89 / 77 and 83 / 71; 128/256, 256 heads of 1024 169 /
-// 103 and 152 / 97, 128 of 2048 158 / 146 and 144 / 134; 128/128, 256 of 1024 107 / 83 and 95 / 75; 64/128, 256 of 1024 80 / 62 and 71 / 61;
-// 256/256, 256 of 512 94 / 80 and 89 / 75.
+//     up to 2^24 times the state, which overflows with rows of 2^103 and above; and it gained nothing (us, an earlier form of the kernel, forward,
+//     backward, so / with the decay: 128 heads of 256/512, 2048 positions 331 303 / 334 306, 256 heads of 1024, 128/256 103 97 / 102 96, 128/128 75 70 / 74 69, 64/128 61 60 / 59 60).
+// What bounds it: issue.  A step of 256 / 256 columns is 120 matrix and 807 vector instructions a wave, two waves a SIMD, which
+// overlap only where they are interleaved (a matrix instruction hides about six of its wave: the schedules below); matrix pipes 50 %
+// busy (128 columns: 26 and 29 %), LDS 29 %, 1 to 2 % of that conflicts (20 and 15 % with swizzles for other groups of lanes); 3.4 TB/s,
+// every row read once.  us, forward / backward, scan + H (dV) and this: 256/512, 128 heads of 2048 with the last state 377 / 258, of 1024
+// 174 / 131 and 167 / 121, of 512 88 / 70 and 80 / 62; 128/256, 256 heads of 1024 141 / 92 and 122 / 90, 128 of 2048 145 / 123 and 129 /
+// 105; 128/128, 256 of 1024 102 / 68 and 88 / 59; 64/128, 256 of 1024 81 / 57 and 69 / 47; 256/256, 256 of 512 99 / 75 and 85 / 69.
 #include "common.h"
 #include "kernels.h"
 
@@ -171,8 +171,8 @@ __device__ __forceinline__ int lane_of(int lane) { return TIGHT ? opaque(lane) :
 
 // What a launch makes.  kKeptStates: the forward's kept states and nothing else, for a backward that has them recomputed: the same
 // arithmetic in the same order, hence the same bits, which the scan, rounding the scaled value rows once, does not have.  us, the whole
-// forward / the scan / this: 128 heads of 256/512, 2048 positions 341 / 154 / 174, 1024 147 / 70 / 74; 256 heads of 1024, 128/256 102 / 48 /
-// 50, 64/128 62 / 20 / 28.  (The scan's launch, which then ends at once, 6 us.)
+// forward / the scan / this: 128 heads of 256/512, 2048 positions 272 / 139 / 152, 1024 131 / 69 / 70; 256 heads of 1024, 128/256 93 / 51 /
+// 53, 64/128 58 / 27 / 25.  (The scan's launch, which then ends at once, 6 us.)
 enum Kind { kForward, kBackward, kKeptStates };
 
 template <int DQ, int W, int KIND, bool F16>
@@ -814,9 +814,10 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 }
 // Value columns of a workgroup, 0: another kernel is the better one.
 //  * One workgroup takes a CU and the launch as long as its rounds: the last one has to be nearly full.  256 columns are the more
-//    efficient form (256/512, 96 heads of 1024, 192 workgroups: 158 us against 140 for scan + H; 128 heads 160 / 207: the line is at
-//    85 %); with 128 the state's rows are shared by two waves that both scale the value rows, and what is gained is less (128/256,
-//    128 heads 158 / 146, at 112 heads 138 / 146).  Not for half of the heads of 256/512, which would be
+//    efficient form; with 128 the state's rows are shared by two waves that both scale the value rows, and what is gained is less.  The
+//    lines, 85 and 95 %, lie between 96 and 128 heads of 256/512 (192 and 256 workgroups of 256) and between 112 and 128 of 128/256 (of 128),
+//    where an earlier form of this kernel crossed scan + H.  The present one is past it at 75 and 87 % (scan + H / so: 96 heads of 1024
+//    135 / 112, dV 129 / 104, 128 175 / 131; 128/256, 112 heads of 2048 136 / 115, dV 122 / 99): they could lie lower.  Not for half of the heads of 256/512, which would be
 //    faster (64 heads, scan + stream_hv / so: forward with the last state, 512 positions 63 / 49, 1000 107 / 89, 2000 201 / 169; forward and
 //    backward, 512 151 / 155, 1000 292 / 294, 2048 599 / 574): H is a little further from 64 bits than theirs (errors times 1e-3, gates around 3, 6, 9: 1000
 //    positions 2.357 2.343 2.353 / 2.365 2.372 2.367, 2000 2.355 2.411 2.365 / 2.363 2.379 2.375), and where only a forward without a gradient gains it
@@ -824,11 +825,11 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 //  * Rows move to LDS in pieces of 16 bytes without registers in between, and rows of the output leave through a buffer descriptor, 16
 //    bytes a lane: both ask for addresses that are multiples of 16; the other kernels read and write theirs with ordinary instructions,
 //    which do not.
-//  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 124 / 148, backward
-//    93 / 137); at 320 128 heads take 74 / 50 and 68 / 47.
+//  * Up to 256 positions the other kernels need no state at all and are faster (256/512, 512 heads of 256: forward 117 / 136, backward
+//    87 / 126); at 320 128 heads take 75 / 47 and 65 / 43.
 //  * Longer sequences and several rounds are no other matter.  256/512, a forward with the last state and forward and backward, with the
-//    scan and the streaming kernels / so: 128 heads of 2049 positions 464 / 308 and 1287 / 1087, of 8192 1535 / 1150 and 4496 / 3953,
-//    512 of 1024 800 / 618 and 2037 / 1918; 1024 of 512 841 / 660 and 1786 / 1813, the one size where they are level with a backward.
+//    scan and the streaming kernels / so: 128 heads of 2049 positions 444 / 279 and 1233 / 996, of 8192 1479 / 1047 and 4318 / 3671,
+//    512 of 1024 779 / 557 and 1994 / 1797, 1024 of 512 816 / 602 and 1726 / 1678.
 int columns(const ChainHvArgs& a, int BH) {
   if (a.DHQK != 64 && a.DHQK != 128 && a.DHQK != 256) return 0;
   if (((size_t)a.S + kStep) * (size_t)(a.DHHV > a.DHQK ? a.DHHV : a.DHQK) * 2 >= ((size_t)1 << 32)) return 0;  // 32-bit offsets in a head

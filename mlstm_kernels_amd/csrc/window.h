@@ -34,9 +34,9 @@ __device__ __forceinline__ int win_f64(int row) { return (row >> 2) & 3; }
 // Tiles with rows of RB = 128, 256 or 512 bytes: a transposing read takes 4 neighbouring units of 4 consecutive rows, and a read of 8
 // bytes of one unit 32 rows.  (512: 8 rows further on, which is where the next piece of a thread goes, it is the same again.)
 // Against swizzles for groups of 8 and 16 neighbouring lanes, which two lanes of every group shared a bank with (us, before / after):
-// dQ / dK of 256/512, 32 heads of 16384 770 / 757, 128 of 1024 183 / 179.  Rows of 128 bytes keep theirs, with
-// which the patch falls on distinct banks too: one that also spreads the 8-byte reads measured slower, for a reason not found (forward and
-// backward, with that / this: 64/64, 24 heads of 9984 239 / 235, 32 of 4096 148 / 145; 128/256, 32 of 8192 546 / 539).
+// dQ / dK of 256/512, 32 heads of 16384 759 / 747, 128 of 1024 188 / 185; conflicts 0.40 / 0.12 of the LDS cycles.  Rows of 128 bytes
+// keep theirs, with which the patch falls on distinct banks too: one that also spreads the 8-byte reads measured slower, for a reason not
+// found (forward and backward, with that / this: 64/64, 24 heads of 9984 239 / 235, 32 of 4096 148 / 145; 128/256, 32 of 8192 546 / 539).
 template <int RB>
 __device__ __forceinline__ int win_zsw(int row) {
   if (RB == 128) return 2 * (row & 3);
