@@ -28,9 +28,10 @@
 //     2.374 / 2.368, gates around 9 2.680 / 2.376, 2.629 / 2.328, 2.690 / 2.324, 2.739 / 2.384; 256 heads of 128/128, gates around 3, H 2.362 /
 //     2.371, dV 2.363 / 2.366.  (Rows right behind a step's boundary take most of H from the rounded state; where a normaliser nearly
 //     cancels that weighs more: the 99th percentile of the rows is 2 % higher.)
-//   * The state takes its decay in every step.  Left in a factor until that reaches 2^-24, with weights that take it, the registers hold
-//     up to 2^24 times the state, which overflows with rows of 2^103 and above; and it gained nothing (us, an earlier form of the kernel, forward,
-//     backward, so / with the decay: 128 heads of 256/512, 2048 positions 331 303 / 334 306, 256 heads of 1024, 128/256 103 97 / 102 96, 128/128 75 70 / 74 69, 64/128 61 60 / 59 60).
+//   * The state takes its decay in every step.  Left in a factor until that reaches 2^-24, with weights that take it, the registers
+//     hold up to 2^24 times the state, which overflows with rows of 2^103 and above; and it gained nothing (us, an earlier form of the
+//     kernel, forward, backward, so / with the decay: 128 heads of 256/512, 2048 positions 331 303 / 334 306, 256 heads of 1024,
+//     128/256 103 97 / 102 96, 128/128 75 70 / 74 69, 64/128 61 60 / 59 60).
 // What bounds it: issue.  A step of 256 / 256 columns is 120 matrix and 807 vector instructions a wave, two waves a SIMD, which
 // overlap only where they are interleaved (a matrix instruction hides about six of its wave: the schedules below); matrix pipes 50 %
 // busy (128 columns: 26 and 29 %), LDS 29 %, 1 to 2 % of that conflicts (20 and 15 % with swizzles for other groups of lanes); 3.4 TB/s,
@@ -815,13 +816,13 @@ const char* launch_w(const ChainHvArgs& a, int BH, int kind, hipStream_t stream)
 // Value columns of a workgroup, 0: another kernel is the better one.
 //  * One workgroup takes a CU and the launch as long as its rounds: the last one has to be nearly full.  256 columns are the more
 //    efficient form; with 128 the state's rows are shared by two waves that both scale the value rows, and what is gained is less.  The
-//    lines, 85 and 95 %, lie between 96 and 128 heads of 256/512 (192 and 256 workgroups of 256) and between 112 and 128 of 128/256 (of 128),
-//    where an earlier form of this kernel crossed scan + H.  The present one is past it at 75 and 87 % (scan + H / so: 96 heads of 1024
-//    135 / 112, dV 129 / 104, 128 175 / 131; 128/256, 112 heads of 2048 136 / 115, dV 122 / 99): they could lie lower.  Not for half of the heads of 256/512, which would be
-//    faster (64 heads, scan + stream_hv / so: forward with the last state, 512 positions 63 / 49, 1000 107 / 89, 2000 201 / 169; forward and
-//    backward, 512 151 / 155, 1000 292 / 294, 2048 599 / 574): H is a little further from 64 bits than theirs (errors times 1e-3, gates around 3, 6, 9: 1000
-//    positions 2.357 2.343 2.353 / 2.365 2.372 2.367, 2000 2.355 2.411 2.365 / 2.363 2.379 2.375), and where only a forward without a gradient gains it
-//    would not have the bits of one with a gradient.
+//    lines, 85 and 95 %, lie between 96 and 128 heads of 256/512 (192 and 256 workgroups of 256) and between 112 and 128 of 128/256 (of
+//    128), where an earlier form of this kernel crossed scan + H.  The present one is past it at 75 and 87 % (scan + H / so: 96 heads of
+//    1024 135 / 112, dV 129 / 104, 128 175 / 131; 128/256, 112 heads of 2048 136 / 115, dV 122 / 99): they could lie lower.  Not for half
+//    of the heads of 256/512, which would be faster (64 heads, scan + stream_hv / so: forward with the last state, 512 positions 63 / 49,
+//    1000 107 / 89, 2000 201 / 169; forward and backward, 512 151 / 155, 1000 292 / 294, 2048 599 / 574): H is a little further from 64
+//    bits than theirs (errors times 1e-3, gates around 3, 6, 9: 1000 positions 2.357 2.343 2.353 / 2.365 2.372 2.367, 2000 2.355 2.411
+//    2.365 / 2.363 2.379 2.375), and where only a forward without a gradient gains it would not have the bits of one with a gradient.
 //  * Rows move to LDS in pieces of 16 bytes without registers in between, and rows of the output leave through a buffer descriptor, 16
 //    bytes a lane: both ask for addresses that are multiples of 16; the other kernels read and write theirs with ordinary instructions,
 //    which do not.

@@ -142,12 +142,14 @@ def test_halves_of_wide_heads(S, dtype):
 
 
 # Few heads and a long prompt, whose heads leave the chain kernel most of the chip: it is not taken, whether states are kept or not.  The last
-# states are held to the 1e-5 of a scan that carries the remainder of the value operand where it weighs.
+# states are held to the 1e-5 of a scan that carries the remainder of the value operand in the chunks that weigh 2^-8 or more: what the others lose
+# is up to 2^-9 of them, 2^-17 = 7.6e-6 of the state (gates around 6: it is a part of the chunks of every segment).
 @pytest.mark.parametrize("BH,S,DQ,DV", [(4, 16384, 128, 256), (4, 8300, 256, 512), (8, 5000, 256, 512), (8, 10000, 256, 512), (40, 8060, 256, 512),
                                         (100, 3968, 128, 256), (4, 4428, 128, 256), (24, 3528, 128, 128), (5, 16384, 64, 128), (12, 6016, 64, 256),
                                         (7, 10185, 256, 256), (9, 6003, 128, 384)])
-@pytest.mark.parametrize("opt", [dict(), dict(f_offset=9.0, init=True), dict(f_offset=0.0, last=False), dict(sig=True, init=True), dict(sig=True, normalize=False, init=True),
-                                 dict(dtype=torch.float16, f_offset=9.0)], ids=["", "keep", "forget", "sig", "sig-raw", "fp16-keep"])
+@pytest.mark.parametrize("opt", [dict(), dict(f_offset=6.0, init=True), dict(f_offset=9.0, init=True), dict(f_offset=0.0, last=False), dict(sig=True, init=True),
+                                 dict(sig=True, normalize=False, init=True), dict(dtype=torch.float16, f_offset=9.0)],
+                         ids=["", "half", "keep", "forget", "sig", "sig-raw", "fp16-keep"])
 def test_long_prompts_of_few_heads(BH, S, DQ, DV, opt):
     from mlstm_kernels_amd import _lib
     from mlstm_kernels_amd.torch.chunkwise import mlstm_chunkwise__hip_xl_chunk, mlstm_siging_chunkwise__hip_xl_chunk
